@@ -1,135 +1,222 @@
-// C[M,N] = A[M,K] * W[N,K]^T (+ bias), everything float, plain fused multiply-adds: the matrix
-// product of the 32-bit path.  No matrix-core instruction is used here on purpose.
-#include "common.h"
+// C[M,N] = A[M,K] * W[N,K]^T (+ bias), everything float: the matrix products of the 32-bit path.
+//
+// The float matrix instructions (v_mfma_f32_32x32x2_f32, v_mfma_f32_16x16x4_f32) multiply 32-bit operands and add to 32-bit
+// sums, rounding as a multiply-add does: nothing is narrower than with vector instructions, and a compute unit does 256
+// operations a clock where vector multiply-adds do 128.  Three kernels:
+//   more than 16 rows   tiles through LDS, K cut over workgroups where the tiles alone would leave compute units idle
+//   up to 16 rows       one pass over the weights, sixteen weight rows a workgroup whose waves share K
+//   K no multiple of 4 (or unaligned rows), up to 16 rows    plain multiply-adds, an element a load
+#include "splitk_reduce.h"
 
-#define TM 64
-#define TN 64
-#define TK 16
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+__device__ __forceinline__ float silu_f32(float g) { return g / (1.0f + expf(-g)); }
+
+// ---------------------------------------------------------------------------------------------------- many rows
+// A workgroup of four waves makes a BM x BN tile, each wave a quarter of it in blocks of 32 x 32.  K goes in steps of 32
+// floats: a row of a step is eight pieces of sixteen bytes, which lie in LDS XOR-swizzled by the row, so that the 32 rows a
+// fragment read takes at one place of the step fall into all banks.  A lane of the lower half of a wave reads k..k+3 of its
+// row, one of the upper half k+4..k+7: the sums run over the same k in both operands, whatever their order, so one sixteen
+// byte read feeds four matrix instructions.  The next step's rows are on their way to registers while the current one is
+// multiplied; two buffers in LDS, one barrier a step.
+// Bound by the matrix cores: 128 x 128 x 32 are 4,096 clocks of them against 32 KB fetched and 128 KB read from LDS.
+// blockIdx.x runs over tiles so that the workgroups of one chiplet (every eighth) share strips of weight rows.
+// (1,280 rows at 0.5B sizes: gate/up, 9,728 columns over 896, 890 us with vector multiply-adds, 217 with this = 110 TFLOP/s; a
+// layer's four products 1,503 and 423 us.)
+template <int BM, int BN>
 __global__ void __launch_bounds__(256)
-gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
-  __shared__ float a_s[TK][TM + 1];
-  __shared__ float w_s[TK][TN + 1];
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;  // 16 x 16 threads, 4 x 4 outputs each
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += TK) {
-    for (int idx = threadIdx.x; idx < TM * TK; idx += 256) {
-      const int r = idx / TK, c = idx % TK;
-      const int m = m0 + r, k = k0 + c;
-      a_s[c][r] = (m < M && k < K) ? A[(size_t)m * lda + k] : 0.f;
-      const int n = n0 + r;
-      w_s[c][r] = (n < N && k < K) ? W[(size_t)n * K + k] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < TK; ++kk) {
-      float a[4], w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { a[i] = a_s[kk][ty * 4 + i]; w[i] = w_s[kk][tx * 4 + i]; }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n < N) C[(size_t)m * ldc + n] = acc[i][j] + (bias ? bias[n] : 0.f);
-    }
-  }
-}
+gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int vec, int k_part, int m_tiles,
+                     int n_tiles, float* __restrict__ partial) {
+  constexpr int TK = 32, QM = BM / 64, QN = BN / 64;       // blocks of 32 x 32 a wave holds each way
+  constexpr int PA = BM / 32, PW = BN / 32;                // rows a thread brings of each operand
+  __shared__ __attribute__((aligned(16))) float a_s[2][BM * TK];
+  __shared__ __attribute__((aligned(16))) float w_s[2][BN * TK];
+  const int total = m_tiles * n_tiles, per_chiplet = (total + 7) / 8;
+  const int tile = (blockIdx.x % 8) * per_chiplet + blockIdx.x / 8;
+  if (tile >= total) return;
+  const int m0 = tile % m_tiles * BM, n0 = tile / m_tiles * BN;
+  const int k_begin = blockIdx.y * k_part, k_end = min(K, k_begin + k_part);
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int row_in = threadIdx.x >> 3, piece = threadIdx.x & 7;       // 32 rows of eight pieces at a time
+  f32x4 a_next[PA], w_next[PW];
 
-// Many rows: tiles of 128 x 128 with 8 x 8 outputs a thread (two 4 x 4 quarters each way, so that LDS is read
-// sixteen bytes at a time), K in steps of 16; the next step's tiles are on their way from memory while the
-// current one is multiplied.  Plain multiply-adds as everywhere in this file.
-#define BTM 128
-#define BTN 128
-#define BTK 16
-
-__global__ void __launch_bounds__(256)
-gemm_f32_big_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                    float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
-  __shared__ __attribute__((aligned(16))) float a_s[BTK][BTM + 4];
-  __shared__ __attribute__((aligned(16))) float w_s[BTK][BTN + 4];
-  const int m0 = blockIdx.y * BTM, n0 = blockIdx.x * BTN;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  // Each thread brings in two rows x four consecutive k of A and of W per step: row = id / 4 (+ 64), k = (id % 4) * 4.
-  const int lr = threadIdx.x / 4, lk = (threadIdx.x % 4) * 4;
-  const bool vec = (K % 4 == 0) && (lda % 4 == 0) && (((uintptr_t)A | (uintptr_t)W) % 16 == 0);
-  float acc[8][8] = {};
-  float4 a_next[2], w_next[2];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int m = m0 + lr + 64 * h, n = n0 + lr + 64 * h, k = k0 + lk;
-      float4 av = make_float4(0.f, 0.f, 0.f, 0.f), wv = av;
-      if (vec && k + 3 < K) {
-        if (m < M) av = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
-        if (n < N) wv = *reinterpret_cast<const float4*>(W + (size_t)n * K + k);
+  auto piece_of = [&](const float* base, int row, int rows, int stride, int k) -> f32x4 {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (row < rows) {
+      const float* p = base + (size_t)row * stride + k;
+      if (vec && k + 3 < k_end) {
+        v = *reinterpret_cast<const f32x4*>(p);
       } else {
-        float at[4] = {0.f, 0.f, 0.f, 0.f}, wt[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (m < M && k + i < K) at[i] = A[(size_t)m * lda + k + i];
-          if (n < N && k + i < K) wt[i] = W[(size_t)n * K + k + i];
-        }
-        av = make_float4(at[0], at[1], at[2], at[3]);
-        wv = make_float4(wt[0], wt[1], wt[2], wt[3]);
+        for (int i = 0; i < 4; ++i)
+          if (k + i < k_end) v[i] = p[i];
       }
-      a_next[h] = av;
-      w_next[h] = wv;
     }
+    return v;
   };
-  auto stash = [&]() {
+  auto fetch = [&](int k0) {
+    const int k = k0 + piece * 4;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int r = lr + 64 * h;
-      a_s[lk][r] = a_next[h].x; a_s[lk + 1][r] = a_next[h].y; a_s[lk + 2][r] = a_next[h].z; a_s[lk + 3][r] = a_next[h].w;
-      w_s[lk][r] = w_next[h].x; w_s[lk + 1][r] = w_next[h].y; w_s[lk + 2][r] = w_next[h].z; w_s[lk + 3][r] = w_next[h].w;
-    }
+    for (int i = 0; i < PA; ++i) a_next[i] = piece_of(A, m0 + row_in + 32 * i, M, lda, k);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) w_next[i] = piece_of(W, n0 + row_in + 32 * i, N, K, k);
   };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += BTK) {
-    stash();
+  auto put = [&](int buffer) {
+    const int at = row_in * TK + ((piece ^ (row_in & 7)) << 2);       // (rows 32 apart are swizzled alike)
+#pragma unroll
+    for (int i = 0; i < PA; ++i) *reinterpret_cast<f32x4*>(&a_s[buffer][at + 32 * TK * i]) = a_next[i];
+#pragma unroll
+    for (int i = 0; i < PW; ++i) *reinterpret_cast<f32x4*>(&w_s[buffer][at + 32 * TK * i]) = w_next[i];
+  };
+
+  f32x16 acc[QM][QN];
+#pragma unroll
+  for (int i = 0; i < QM; ++i)
+#pragma unroll
+    for (int j = 0; j < QN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+  const int r = lane & 31, half = lane >> 5;
+
+  fetch(k_begin);
+  put(0);
+  int buffer = 0;
+  for (int k0 = k_begin; k0 < k_end; k0 += TK, buffer ^= 1) {
     __syncthreads();
-    if (k0 + BTK < K) fetch(k0 + BTK);
+    const bool more = k0 + TK < k_end;
+    if (more) fetch(k0 + TK);
 #pragma unroll
-    for (int kk = 0; kk < BTK; ++kk) {
-      float a[8], w[8];
-      const float4 a0 = *reinterpret_cast<const float4*>(&a_s[kk][ty * 4]);
-      const float4 a1 = *reinterpret_cast<const float4*>(&a_s[kk][64 + ty * 4]);
-      const float4 w0 = *reinterpret_cast<const float4*>(&w_s[kk][tx * 4]);
-      const float4 w1 = *reinterpret_cast<const float4*>(&w_s[kk][64 + tx * 4]);
-      a[0] = a0.x; a[1] = a0.y; a[2] = a0.z; a[3] = a0.w; a[4] = a1.x; a[5] = a1.y; a[6] = a1.z; a[7] = a1.w;
-      w[0] = w0.x; w[1] = w0.y; w[2] = w0.z; w[3] = w0.w; w[4] = w1.x; w[5] = w1.y; w[6] = w1.z; w[7] = w1.w;
+    for (int s = 0; s < TK / 8; ++s) {
+      const int at = r * TK + (((2 * s + half) ^ (r & 7)) << 2);
+      f32x4 a[QM], w[QN];
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < QM; ++i) a[i] = *reinterpret_cast<const f32x4*>(&a_s[buffer][(wm + 32 * i) * TK + at]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
+      for (int j = 0; j < QN; ++j) w[j] = *reinterpret_cast<const f32x4*>(&w_s[buffer][(wn + 32 * j) * TK + at]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < QM; ++i)
+#pragma unroll
+          for (int j = 0; j < QN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[j][e], a[i][e], acc[i][j], 0, 0, 0);
     }
-    __syncthreads();
+    if (more) put(buffer ^ 1);        // (its readers passed the barrier above)
   }
+  // Weight rows are the instruction's rows: element e of a lane is column 8 (e / 4) + 4 half + e % 4 of row r of A.
+  float* dst = partial ? partial + (size_t)blockIdx.y * M * N : C;
+  const int stride = partial ? N : ldc;
+  const bool quads = N % 4 == 0 && stride % 4 == 0 && ((uintptr_t)dst & 15) == 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + (i < 4 ? ty * 4 + i : 64 + ty * 4 + i - 4);
+  for (int i = 0; i < QM; ++i) {
+    const int m = m0 + wm + 32 * i + r;
     if (m >= M) continue;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int n = n0 + (j < 4 ? tx * 4 + j : 64 + tx * 4 + j - 4);
-      if (n < N) C[(size_t)m * ldc + n] = acc[i][j] + (bias ? bias[n] : 0.f);
-    }
+    for (int j = 0; j < QN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + wn + 32 * j + 8 * q + 4 * half;
+        f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        float* out = dst + (size_t)m * stride + n;
+        if (quads && n < N) {
+          if (bias && !partial) { v[0] += bias[n]; v[1] += bias[n + 1]; v[2] += bias[n + 2]; v[3] += bias[n + 3]; }
+          *reinterpret_cast<f32x4*>(out) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) out[e] = v[e] + (bias && !partial ? bias[n + e] : 0.f);
+        }
+      }
   }
 }
 
-// Few rows (M <= 16): the product is one pass over the weights, so a wave takes four weight rows and walks K
-// with sixteen bytes per lane, every row of A against them; the sums are added up over the wave at the end.
-// Plain multiply-adds here as well.
+// ----------------------------------------------------------------------------------------------------- few rows
+// Up to sixteen rows: sixteen weight rows a workgroup (GATED: eight rows of the first half of W and the eight as far into
+// its second half, whose results meet in silu(first) * second), eight waves that take units of 32 floats of K in turn.
+// Lane (row, g) reads the sixteen bytes g and g + 4 of a weight row's 128 byte line and the same of row `row` of A; the
+// matrix instruction's sum runs over the four g.  Four sums a lane (one for each float of a piece) keep the chains of
+// additions short; they and the eight waves' come together through LDS.  Bound by the weights' trip from memory: a wave
+// asks for its first two pairs of units at once and for the next pair before it multiplies the current one.
+// (Four rows at 0.5B sizes, the four products of a layer: 54 us with a wave on four weight rows and the gate's kernel, 41 with
+// this: gate/up with its gate 12.6, 896 columns over 4,864 8.5 in eight parts of K and 18.8 in one.)
+template <bool GATED>
+__global__ void __launch_bounds__(512)
+gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int units_part,
+                     float* __restrict__ partial) {
+  constexpr int WAVES = 8, PAIR = 2;
+  __shared__ float sums[WAVES][16][17];
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int row = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * (GATED ? 8 : 16), half = N / 2;
+  const int n = GATED ? (row < 8 ? min(n0 + row, half - 1) : half + min(n0 + row - 8, half - 1)) : min(n0 + row, N - 1);
+  const int units = (K + 31) / 32;
+  const int u_begin = blockIdx.y * units_part, u_end = min(units, u_begin + units_part);
+  const float* w_row = W + (size_t)n * K;
+  const float* a_row = A + (size_t)min(row, M - 1) * lda;
+  f32x4 w[2][PAIR][2], a[2][PAIR][2];
+  auto ask = [&](int slot, int u0) {
+#pragma unroll
+    for (int p = 0; p < PAIR; ++p)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        // (K is a multiple of four: a piece is inside a row or past its end, where the row's first piece is read and
+        // multiplied by zeros.)
+        const int u = u0 + p * WAVES, k = u * 32 + 16 * h + 4 * g;
+        const bool in = u < u_end && k < K;
+        w[slot][p][h] = *reinterpret_cast<const f32x4*>(w_row + (in ? k : 0));
+        a[slot][p][h] = *reinterpret_cast<const f32x4*>(a_row + (in ? k : 0));
+      }
+  };
+  f32x4 acc[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int first = u_begin + wave;
+  ask(0, first);
+  for (int u0 = first; u0 < u_end; u0 += 2 * PAIR * WAVES) {
+#pragma unroll
+    for (int slot = 0; slot < 2; ++slot) {
+      const int now = u0 + slot * PAIR * WAVES;
+      ask(slot ^ 1, now + PAIR * WAVES);
+#pragma unroll
+      for (int p = 0; p < PAIR; ++p)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int u = now + p * WAVES;
+          const bool in = u < u_end && u * 32 + 16 * h + 4 * g < K;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            // (Both operands: the first piece of a row may hold an infinity, whose product with zero is no number.)
+            const float wv = in ? w[slot][p][h][e] : 0.f, av = in ? a[slot][p][h][e] : 0.f;
+            acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, av, acc[e], 0, 0, 0);
+          }
+        }
+    }
+  }
+  // A lane holds weight rows 4 g .. 4 g + 3 of A's row `row`.
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sums[wave][row][4 * g + j] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
+  __syncthreads();
+  const int m = threadIdx.x >> 4, at = threadIdx.x & 15;
+  if (m >= M) return;                                      // (threads from the sixteenth row on leave here too)
+  auto total = [&](int place) {
+    float t = 0.f;
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) t += sums[v][m][place];
+    return t;
+  };
+  if (GATED) {
+    if (at < 8 && n0 + at < half) C[(size_t)m * ldc + n0 + at] = silu_f32(total(at)) * total(at + 8);
+  } else if (n0 + at < N) {
+    if (partial) partial[((size_t)blockIdx.y * M + m) * N + n0 + at] = total(at);
+    else C[(size_t)m * ldc + n0 + at] = total(at) + (bias ? bias[n0 + at] : 0.f);
+  }
+}
+
+// Up to sixteen rows whose pieces of sixteen bytes do not lie on sixteen bytes: a wave takes four weight rows and walks K
+// an element a lane.
 template <int MR>
 __global__ void __launch_bounds__(256)
 gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
@@ -145,33 +232,16 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
   const float* w[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) w[r] = W + (size_t)min(n0 + r, N - 1) * K;
-  const bool vec = (K % 4 == 0) && (lda % 4 == 0) && (((uintptr_t)A | (uintptr_t)W) % 16 == 0);
-  if (vec) {
-    for (int k = lane * 4; k < K; k += WAVE * 4) {
-      float4 wv[4];
+  for (int k = lane; k < K; k += WAVE) {
+    float wv[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) wv[r] = *reinterpret_cast<const float4*>(w[r] + k);
+    for (int r = 0; r < 4; ++r) wv[r] = w[r][k];
 #pragma unroll
-      for (int m = 0; m < MR; ++m) {
-        if (m >= M) break;
-        const float4 a = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
+    for (int m = 0; m < MR; ++m) {
+      if (m >= M) break;
+      const float a = A[(size_t)m * lda + k];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc[r][m] = fmaf(a.x, wv[r].x, fmaf(a.y, wv[r].y, fmaf(a.z, wv[r].z, fmaf(a.w, wv[r].w, acc[r][m]))));
-      }
-    }
-  } else {
-    for (int k = lane; k < K; k += WAVE) {
-      float wv[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) wv[r] = w[r][k];
-#pragma unroll
-      for (int m = 0; m < MR; ++m) {
-        if (m >= M) break;
-        const float a = A[(size_t)m * lda + k];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r][m] = fmaf(a, wv[r], acc[r][m]);
-      }
+      for (int r = 0; r < 4; ++r) acc[r][m] = fmaf(a, wv[r], acc[r][m]);
     }
   }
 #pragma unroll
@@ -183,25 +253,91 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
     }
 }
 
-extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void* C, int M, int N, int K,
-                           int lda, int ldc, hipStream_t stream) {
-  if (M <= 0 || N <= 0) return 0;
+static bool sixteen_bytes(const void* A, const void* W, int M, int K, int lda) {
+  return K % 4 == 0 && (M <= 1 || lda % 4 == 0) && (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
+}
+
+// Which kernel and into how many parts of K (a power of two at most 8): `tile` 16 (few rows), 64 or 128, 0 (an element a
+// load).  Few rows: parts until there are workgroups for every compute unit, each of eight units of 32 at least, and only
+// where the next kernel adds them (`pending`): a reduction of its own costs as much as it saves.  Many rows: the estimate is
+// rounds of workgroups over the compute units, a round as long as its tile's multiplications at what the two tiles reach
+// (128 x 128: 110 of the 157 TFLOP/s there are, 64 x 64: 88), plus the parts' trip to memory and, where nobody else adds
+// them, a further launch.
+static void f32_choice(int M, int N, int K, bool aligned, bool pending, int* tile, int* parts) {
+  const int units = compute_units();
+  *tile = 0;
+  *parts = 1;
   if (M <= 16) {
+    if (!aligned) return;
+    *tile = 16;
+    if (pending && N % 4 == 0)
+      while (*parts < 8 && (N + 15) / 16 * *parts < units && K / 32 / (2 * *parts) >= 8) *parts *= 2;
+    return;
+  }
+  double best = 1e30;
+  for (int t = 64; t <= 128; t *= 2)
+    for (int p = 1; p <= 8; p *= 2) {
+      if (p > 1 && (N % 4 || K / p < 128)) continue;
+      const double tiles = (double)((M + t - 1) / t) * ((N + t - 1) / t) * p;
+      const double flops = 2.0 * t * t * ((K + p - 1) / p), rate = (t == 128 ? 110e6 : 88e6) / units;   // a unit's, per us
+      const double rounds = tiles <= units ? 1.0 : (double)(long)((tiles + units - 1) / units);
+      double cost = rounds * flops / rate + 3.0;
+      if (p > 1) cost += (double)M * N * 4 * p * 2 / 4e6 + (pending ? 0.0 : 4.0);
+      if (cost < best) { best = cost; *tile = t; *parts = p; }
+    }
+}
+
+// The parts of K a product is cut into where `pending` says that whoever takes it adds them; 1: it is not.
+extern "C" int ta_gemm_f32_parts(const void* A, const void* W, int M, int N, int K, int lda, int pending) {
+  if (M <= 0 || N <= 0 || K <= 0) return 1;
+  int tile, parts;
+  f32_choice(M, N, K, sixteen_bytes(A, W, M, K, lda), pending != 0, &tile, &parts);
+  return parts_of_k(K, parts, 32);
+}
+
+// partial: float [ta_gemm_f32_parts][M][N] where that is more than 1, else null.  C null: the parts are left there.
+extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void* C, int M, int N, int K,
+                           int lda, int ldc, void* partial, int pending, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  const bool aligned = sixteen_bytes(A, W, M, K, lda);
+  int tile = 0, parts = 1;
+  f32_choice(M, N, K, aligned, pending != 0, &tile, &parts);
+  parts = parts_of_k(K, parts, 32);
+  if ((parts > 1) != (partial != nullptr) || (!C && parts == 1)) return -1;
+  const float *a = (const float*)A, *w = (const float*)W, *b = (const float*)bias;
+  float *c = (float*)C, *slabs = (float*)partial;
+  const int k_part = parts > 1 ? ((K + parts - 1) / parts + 31) / 32 * 32 : K;
+  if (tile == 16) {
+    gemm_f32_rows_kernel<false><<<dim3((N + 15) / 16, parts), 512, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc,
+                                                                               (k_part + 31) / 32, slabs);
+  } else if (tile) {
+    const int m_tiles = (M + tile - 1) / tile, n_tiles = (N + tile - 1) / tile;
+    dim3 grid((m_tiles * n_tiles + 7) / 8 * 8, parts);
+    if (tile == 128)
+      gemm_f32_tile_kernel<128, 128><<<grid, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, aligned, k_part, m_tiles,
+                                                               n_tiles, slabs);
+    else
+      gemm_f32_tile_kernel<64, 64><<<grid, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, aligned, k_part, m_tiles,
+                                                             n_tiles, slabs);
+  } else {
     const int blocks = (N + 15) / 16;
-#define GO(MR) gemv_f32_kernel<MR><<<blocks, 256, 0, stream>>>((const float*)A, (const float*)W, (const float*)bias, \
-                                                              (float*)C, M, N, K, lda, ldc)
+#define GO(MR) gemv_f32_kernel<MR><<<blocks, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc)
     if (M <= 1) GO(1); else if (M <= 2) GO(2); else if (M <= 4) GO(4); else if (M <= 8) GO(8); else GO(16);
 #undef GO
-    return LAUNCH_STATUS();
   }
-  if (M > 64 && N > 64) {
-    dim3 big((N + BTN - 1) / BTN, (M + BTM - 1) / BTM);
-    gemm_f32_big_kernel<<<big, 256, 0, stream>>>((const float*)A, (const float*)W, (const float*)bias, (float*)C,
-                                                 M, N, K, lda, ldc);
-    return LAUNCH_STATUS();
-  }
-  dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
-  gemm_f32_kernel<<<grid, 256, 0, stream>>>((const float*)A, (const float*)W, (const float*)bias, (float*)C,
-                                            M, N, K, lda, ldc);
+  int status = LAUNCH_STATUS();
+  if (status == 0 && parts > 1 && C) status = launch_splitk_reduce(slabs, bias, C, M, N, ldc, parts, DT_F32, stream);
+  return status;
+}
+
+// out[M, N/2] = silu(A W1^T) * (A W2^T), W = [W1; W2], for up to sixteen rows; -2 where the pieces are not aligned (the caller
+// then runs the product and the gate one after the other).
+extern "C" int ta_gemm_f32_silu_gate(const void* A, const void* W, void* out, int M, int N, int K, int lda, int ldc,
+                                     hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (N % 2 || K <= 0) return -1;
+  if (M > 16 || !sixteen_bytes(A, W, M, K, lda)) return -2;
+  gemm_f32_rows_kernel<true><<<(N / 2 + 7) / 8, 512, 0, stream>>>((const float*)A, (const float*)W, nullptr, (float*)out, M, N,
+                                                                  K, lda, ldc, (K + 31) / 32, nullptr);
   return LAUNCH_STATUS();
 }

@@ -148,7 +148,7 @@ class Ops:
         for name in ("ta_embedding", "ta_add_rmsnorm", "ta_silu_gate", "ta_rope_store",
                      "ta_paged_attention_generic", "ta_decode_attention_bf16", "ta_prefill_attention_bf16",
                      "ta_prefill_attention_shared_plan", "ta_prefill_attention_key_splits",
-                     "ta_gemm_f32", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
+                     "ta_gemm_f32", "ta_gemm_f32_parts", "ta_gemm_f32_silu_gate", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
                      "ta_gemm_skinny_bf16_splitk", "ta_gemm_skinny_qkv_rope", "ta_fused_norm_qkv_rope",
                      "ta_fused_norm_gated", "ta_fused_linear_residual", "ta_fused_qkv_rope", "ta_fused_gated",
                      "ta_splitk_reduce", "ta_splitk_add_rmsnorm", "ta_argmax", "ta_argmax_next_step", "ta_sample",
@@ -1365,7 +1365,7 @@ class Ops:
                pending: bool = False) -> "torch.Tensor | PendingSum":
         """out = x @ weight.T (+ bias).  x [M, K] (rows may be strided); weight [N, K]; bias float32 [N].
 
-        float32 operands run on plain multiply-adds; bfloat16 operands on the matrix cores with
+        float32 operands run on the matrix cores' 32-bit instructions; bfloat16 operands on theirs, with
         float accumulation and a bfloat16 or float32 result.  `pending=True` allows the result to come back
         as a `PendingSum` when K is cut over workgroups: whoever takes it next (the norm that follows) adds the
         parts in its own kernel and the addition's launch is saved.
@@ -1379,7 +1379,7 @@ class Ops:
         lda = x.stride(0) if m > 1 else k
         if out_dtype is None:
             out_dtype = x.dtype if out is None else out.dtype
-        pending = pending and out is None and x.dtype == torch.bfloat16
+        pending = pending and out is None
         if out is None and not pending:
             out = torch.empty((m, n), dtype=out_dtype, device=x.device)
         if out is not None:
@@ -1388,8 +1388,17 @@ class Ops:
             _need(bias.is_cuda and bias.dtype == torch.float32 and bias.numel() == n, "bias must be float32 [N]")
         if x.dtype == torch.float32:
             _need(out_dtype == torch.float32, "float32 products give float32")
-            status = self.lib.ta_gemm_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), m, n, k, lda, n,
-                                          self._stream())
+            # (The library cuts K over workgroups by its own rule and says into how many parts.)
+            parts = self.lib.ta_gemm_f32_parts(_ptr(x), _ptr(weight), m, n, k, lda, int(pending))
+            leave = pending and parts > 1
+            if out is None and not leave:
+                out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+            partial = torch.empty((parts, m, n), dtype=torch.float32, device=x.device) if parts > 1 else None
+            status = self.lib.ta_gemm_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(None if leave else out), m, n, k, lda, n,
+                                          _ptr(partial), int(pending), self._stream())
+            if leave:
+                self._check(status, "linear")
+                return PendingSum(self, partial, bias, out_dtype)
         else:
             _need(x.dtype == torch.bfloat16, "linear takes float32 or bfloat16")
             if k % 8 or lda % 8 or x.data_ptr() % 16:
@@ -1559,6 +1568,15 @@ class Ops:
         _need(tuple(out.shape) == (m, inner) and out.dtype == x.dtype and out.is_contiguous(), "gated output shape")
         if act is not None and not isinstance(act, str):
             return self.silu_gate(self.linear(x, weight), out, act=act)
+        if x.dtype == torch.float32 and act is None and 0 < m <= self.FUSED_ROWS:
+            _need(x.is_cuda and weight.is_cuda and x.dim() == 2 and x.shape[1] == weight.shape[1], "linear shapes do not fit")
+            _need(x.stride(1) == 1 and weight.is_contiguous() and weight.dtype == torch.float32, "linear operands")
+            k = x.shape[1]
+            status = self.lib.ta_gemm_f32_silu_gate(_ptr(x), _ptr(weight), _ptr(out), m, 2 * inner, k,
+                                                    x.stride(0) if m > 1 else k, inner, self._stream())
+            if status != -2:                  # -2: pieces of sixteen bytes that are not aligned
+                self._check(status, "linear_silu_gate")
+                return out
         if (x.dtype == torch.bfloat16 and m <= self.SKINNY_ROWS and x.shape[1] % 8 == 0 and (m == 1 or x.stride(0) % 8 == 0)
                 and not (self.use_library_gemm and m > self.FUSED_ROWS
                          and weight.shape[0] * weight.shape[1] >= self.GATED_LIBRARY_WEIGHT)):
