@@ -1,11 +1,13 @@
 """The 32-bit path's matrix-core kernels alone against plain references, at the edges of their tiles, units and parts."""
+import math
+
 import pytest
 import torch
 
 from tokenizer_amd.kernels import PendingSum
 
 from kernel_refs import PlainOps
-from test_kernels_gpu import linear_tol, rand
+from test_kernels_gpu import linear_tol, make_batch, make_paged_case, rand
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +66,49 @@ def test_gated_product_of_few_rows(ops, shape):
     bound = linear_tol(torch.float32, x, w)["atol"] * 2.2 * float(both.abs().max())
     torch.testing.assert_close(got.double(), want, rtol=2e-5, atol=bound)
 
+
+FORMS = [dict(), dict(window=37), dict(chunk=50), dict(slopes=True, sinks=True), dict(softcap=3.0, sinks=True),
+         dict(window=29, keep_first=21), dict(value_heads=1), dict(value_dim=40)]
+
+
+@pytest.mark.parametrize("geometry", [(6, 2, 64, 16), (20, 1, 16, 16), (4, 2, 100, 48), (2, 2, 256, 32)])
+@pytest.mark.parametrize("form", FORMS, ids=str)
+def test_attention(ops, ref, geometry, form, monkeypatch):
+    """Portions that start and end inside pages, tiles and blocks of keys, single tokens whose keys are cut over workgroups (also
+    into more parts than there are blocks), against the reference and, form by form, the generic kernel."""
+    n_q, n_kv, d, page_size = geometry
+    form = dict(form)
+    lengths, q_lens = [1, 300, 64, 17, 200, 33], [1, 5, 64, 1, 100, 2]
+    dv, n_v = form.get("value_dim", d), form.get("value_heads", n_kv)
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.float32, n_q, n_kv, d, page_size, lengths=lengths, q_lens=q_lens, seed=31)
+    if dv != d or n_v != n_kv:
+        written = torch.isfinite(v_pages[:, :1, :1]).expand(-1, n_v, dv, -1)
+        v_pages = torch.where(written, rand((v_pages.shape[0], n_v, dv, page_size), torch.float32, 68), float("nan"))
+    for name, seed in (("slopes", 69), ("sinks", 70)):
+        if form.get(name):
+            form[name] = rand((n_q,), torch.float32, seed, 0.1 if name == "slopes" else 2.0)
+    window = form.pop("window", None)
+    scale = 1.0 / math.sqrt(d)
+
+    def run(which, batch=None):
+        on = (lambda v: v.cpu() if isinstance(v, torch.Tensor) else v) if which is ref else (lambda v: v)
+        out = on(torch.full((qkv.shape[0], n_q * dv), float("nan"), device="cuda"))
+        which.paged_attention(*map(on, (qkv, out, k_pages, v_pages, positions, entry_of_token, table)), n_q, n_kv, d, window, scale,
+                              max_position=max(lengths) - 1, **({"batch": batch} if batch else {}),
+                              **{name: on(value) for name, value in form.items()})
+        return out.cuda()
+
+    want = run(ref)
+    # (Scores of about 1 from sums of d products, weighted sums of at most 300 values of about 1.)
+    close = dict(rtol=2e-5, atol=4e-6)
+    batch = make_batch(lengths, q_lens)
+    assert ops.use_fast_attention
+    torch.testing.assert_close(run(ops, batch), want, **close)
+    torch.testing.assert_close(run(ops), want, **close)
+    monkeypatch.setattr(ops, "min_split_keys_f32", 16)
+    torch.testing.assert_close(run(ops), want, **close)
+    monkeypatch.setattr(ops, "target_workgroups", 1)
+    torch.testing.assert_close(run(ops), want, **close)
+    monkeypatch.setattr(ops, "use_fast_attention", False)
+    torch.testing.assert_close(run(ops), want, **close)

@@ -148,7 +148,7 @@ class Ops:
         for name in ("ta_embedding", "ta_add_rmsnorm", "ta_silu_gate", "ta_rope_store",
                      "ta_paged_attention_generic", "ta_decode_attention_bf16", "ta_prefill_attention_bf16",
                      "ta_prefill_attention_shared_plan", "ta_prefill_attention_key_splits",
-                     "ta_gemm_f32", "ta_gemm_f32_parts", "ta_gemm_f32_silu_gate", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
+                     "ta_gemm_f32", "ta_gemm_f32_parts", "ta_gemm_f32_silu_gate", "ta_paged_attention_f32", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
                      "ta_gemm_skinny_bf16_splitk", "ta_gemm_skinny_qkv_rope", "ta_fused_norm_qkv_rope",
                      "ta_fused_norm_gated", "ta_fused_linear_residual", "ta_fused_qkv_rope", "ta_fused_gated",
                      "ta_splitk_reduce", "ta_splitk_add_rmsnorm", "ta_argmax", "ta_argmax_next_step", "ta_sample",
@@ -1229,6 +1229,10 @@ class Ops:
             if batch.decode_rows.numel():
                 self._decode_attention(*args, rows=batch.decode_rows, **extras)
             return out
+        if qkv.dtype == torch.float32 and self.use_fast_attention and self._attention_f32(
+                qkv, out, k_pages, v_pages, positions, entry_of_token, block_table, n_q, n_kv, head_dim, value_dim, page_size,
+                window, scale, max_position, batch, chunk, slopes, sinks, keep_first, value_heads, softcap):
+            return out
         self._check(self.lib.ta_paged_attention_generic(
             _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(k_pages), _ptr(v_pages), _ptr(positions),
             _ptr(entry_of_token), _ptr(block_table), block_table.shape[1], n_tokens, n_q, n_kv, head_dim,
@@ -1237,6 +1241,39 @@ class Ops:
             ctypes.c_float(softcap or 0.0), self._stream()), "paged_attention")
         return out
 
+    def _attention_f32(self, qkv, out, k_pages, v_pages, positions, entry_of_token, block_table, n_q, n_kv, head_dim, value_dim,
+                       page_size, window, scale, max_position, batch, chunk, slopes, sinks, keep_first, value_heads, softcap) -> bool:
+        """Attention in 32 bits on the matrix cores' float instructions: the portions' tiles of sixteen tokens, and single
+        tokens with the key range cut over workgroups.  False for a form that stays with the generic kernel."""
+        tiles = batch.q_tiles.shape[0] if batch is not None else 0
+        _need(not tiles or (batch.n_tokens == qkv.shape[0] and batch.cu_q.numel() == block_table.shape[0] + 1),
+              "the batch description does not belong to these tokens")
+        single = qkv.shape[0] if batch is None or tiles == 0 else batch.decode_rows.numel()
+        rows = batch.decode_rows if tiles and single else None
+        max_keys = (block_table.shape[1] * page_size) if max_position is None else max_position + 1
+        max_keys = -(-max_keys // self.PLAN_KEYS) * self.PLAN_KEYS          # (as for the bfloat16 kernels)
+        for reach in (window, chunk):
+            max_keys = max_keys if reach is None else min(max_keys, reach + keep_first + 32)
+        head_blocks = -(-(n_q // n_kv) // 16)
+        per_item = max(1, self.target_workgroups // max(1, single * n_kv * head_blocks))
+        splits = max(1, min(per_item, -(-max_keys // self.min_split_keys_f32)))
+        part_o = part_ml = None
+        if single and splits > 1:
+            part_o = torch.empty((single, n_q, splits, value_dim), dtype=torch.float32, device=qkv.device)
+            part_ml = torch.empty((single, n_q, splits, 2), dtype=torch.float32, device=qkv.device)
+        status = self.lib.ta_paged_attention_f32(
+            _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(k_pages), _ptr(v_pages), _ptr(batch.q_tiles if tiles else None), tiles,
+            _ptr(batch.cu_q if tiles else None), _ptr(batch.first_position if tiles else None), _ptr(rows), single,
+            _ptr(positions), _ptr(entry_of_token), _ptr(block_table), block_table.shape[1], n_q, n_kv, head_dim, value_dim,
+            page_size, -1 if window is None else int(window), ctypes.c_float(scale), 0 if chunk is None else int(chunk),
+            _ptr(slopes), _ptr(sinks), keep_first, value_heads, ctypes.c_float(softcap or 0.0), splits, _ptr(part_o),
+            _ptr(part_ml), self._stream())
+        if status == -2:
+            return False
+        self._check(status, "paged_attention")
+        return True
+
+    min_split_keys_f32 = 64       # the 32-bit kernel's parts of the keys for single tokens (a block of 16 for each of four waves)
     DECODE_HEAD_DIMS = (16, 32, 48, 64, 80, 96, 112, 128, 160, 192, 224, 256)
     use_tied_values = True        # whether tied keys and values that both have pages are read once (tests compare the two)
     use_fast_attention = True     # tests switch it off to reach the generic kernel in bfloat16
