@@ -438,6 +438,134 @@ norm_side_norm_vec_kernel(float* __restrict__ residual, const T* __restrict__ de
   }
 }
 
+// The same for few rows (no more than compute units) and token inputs of up to sixteen numbers, bfloat16: sixteen waves a
+// workgroup, so that everything a row needs of both small matrices is asked for at once, beside the row itself, and a row is
+// one trip to memory.  Wave j holds row j of the gate's matrix (its dot product is a wave's own), a thread the projection's
+// rows of its two elements of each run of 2,048.  Bound by the trip and the four sums over the workgroup behind it.
+// (1 to 64 rows of 1,536: 12.1 us in the kernel above, 7.0 here; of 896 9.8 and 6.8, of 3,584 18.8 and 9.6.  With more rows a workgroup would read both
+// matrices for each of them, or hold them and take row after row: 2,048 rows of 896 24.6 us above, 34.9 so.)
+#define NA_WIDE 1024
+template <int RUNS>
+__global__ void __launch_bounds__(NA_WIDE)
+norm_side_norm_held_kernel(float* __restrict__ residual, const bf16_t* __restrict__ delta, const float* __restrict__ post_weight,
+                           float post_eps, const bf16_t* __restrict__ gate, const bf16_t* __restrict__ proj, int proj_stride,
+                           const float* __restrict__ side_norm, float side_eps, const bf16_t* __restrict__ table, int table_width,
+                           const int* __restrict__ token_ids, int offset, int dim, const float* __restrict__ weight, float eps,
+                           bf16_t* __restrict__ out, const int* __restrict__ rows, int hidden, int store_residual) {
+  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float x_s[RUNS * 2048];
+  __shared__ float g_s[16];
+  const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+  const bool two = dim > 8;
+  const int r = rows ? rows[blockIdx.x] : blockIdx.x;
+  float* res = residual + (size_t)r * hidden;
+  float2 x[RUNS];
+  uint32_t d[RUNS];
+  float e = 0.f;
+  if (threadIdx.x < dim) e = ld(table + (size_t)token_ids[r] * table_width + offset + threadIdx.x);
+#pragma unroll
+  for (int c = 0; c < RUNS; ++c) {
+    const int h = min(c * 2048 + (int)threadIdx.x * 2, hidden - 2);
+    x[c] = *reinterpret_cast<const float2*>(res + h);
+    d[c] = delta ? *reinterpret_cast<const uint32_t*>(delta + (size_t)r * hidden + h) : 0u;
+  }
+  uint4 gate_row[RUNS * 4], proj_row[RUNS][2][2];
+#pragma unroll
+  for (int c = 0; c < RUNS * 4; ++c) {                       // eight elements a lane and run of 512
+    const int at = min(c * 512 + lane * 8, hidden - 8);
+    gate_row[c] = *reinterpret_cast<const uint4*>(gate + (size_t)min(wave, dim - 1) * hidden + at);
+  }
+  float2 behind[RUNS], tail[RUNS], next[RUNS];
+#pragma unroll
+  for (int c = 0; c < RUNS; ++c) {
+    const int h = min(c * 2048 + (int)threadIdx.x * 2, hidden - 2);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        proj_row[c][q][p] = *reinterpret_cast<const uint4*>(proj + (size_t)(h + q) * proj_stride + (p && two ? 8 : 0));
+    behind[c] = delta && post_weight ? *reinterpret_cast<const float2*>(post_weight + h) : make_float2(1.f, 1.f);
+    tail[c] = *reinterpret_cast<const float2*>(side_norm + h);
+    next[c] = weight ? *reinterpret_cast<const float2*>(weight + h) : make_float2(1.f, 1.f);
+  }
+  auto low = [](uint32_t w) { return __uint_as_float(w << 16); };
+  auto high = [](uint32_t w) { return __uint_as_float(w & 0xffff0000u); };
+  float sq = 0.f, inv = 1.f;
+#pragma unroll
+  for (int c = 0; c < RUNS; ++c) {
+    const float a = low(d[c]), b = high(d[c]);
+    if (c * 2048 + (int)threadIdx.x * 2 < hidden) sq += a * a + b * b;
+  }
+  if (delta && post_weight) inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)hidden + post_eps);
+#pragma unroll
+  for (int c = 0; c < RUNS; ++c) {
+    const int h = c * 2048 + (int)threadIdx.x * 2;
+    x[c].x += low(d[c]) * inv * behind[c].x;
+    x[c].y += high(d[c]) * inv * behind[c].y;
+    if (h < hidden) *reinterpret_cast<float2*>(x_s + h) = x[c];
+  }
+  __syncthreads();
+  float z = 0.f;
+  if (wave < dim) {
+#pragma unroll
+    for (int c = 0; c < RUNS * 4; ++c) {
+      const int at = c * 512 + lane * 8;
+      if (at >= hidden) break;
+      const float4 a = *reinterpret_cast<const float4*>(x_s + at), b = *reinterpret_cast<const float4*>(x_s + at + 4);
+      const uint4 w = gate_row[c];
+      z = fmaf(low(w.x), a.x, fmaf(high(w.x), a.y, fmaf(low(w.y), a.z, fmaf(high(w.y), a.w, z))));
+      z = fmaf(low(w.z), b.x, fmaf(high(w.z), b.y, fmaf(low(w.w), b.z, fmaf(high(w.w), b.w, z))));
+    }
+    z = wave_sum(z);
+    if (lane == 0) g_s[wave] = z;
+  }
+  __syncthreads();
+  if (threadIdx.x < 16) g_s[threadIdx.x] = threadIdx.x < dim ? na_gelu_tanh(g_s[threadIdx.x]) * e : 0.f;
+  __syncthreads();
+  float g[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) g[k] = g_s[k];
+  float2 y[RUNS];
+  sq = 0.f;
+#pragma unroll
+  for (int c = 0; c < RUNS; ++c) {
+    float s[2] = {0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        if (p && !two) continue;
+        const uint32_t w[4] = {proj_row[c][q][p].x, proj_row[c][q][p].y, proj_row[c][q][p].z, proj_row[c][q][p].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[q] = fmaf(high(w[k]), g[8 * p + 2 * k + 1], fmaf(low(w[k]), g[8 * p + 2 * k], s[q]));
+      }
+    y[c] = make_float2(s[0], s[1]);
+    if (c * 2048 + (int)threadIdx.x * 2 < hidden) sq += s[0] * s[0] + s[1] * s[1];
+  }
+  const float inv_y = 1.0f / sqrtf(block_sum(sq, scratch) / (float)hidden + side_eps);
+  sq = 0.f;
+#pragma unroll
+  for (int c = 0; c < RUNS; ++c) {
+    const int h = c * 2048 + (int)threadIdx.x * 2;
+    x[c].x += y[c].x * inv_y * tail[c].x;
+    x[c].y += y[c].y * inv_y * tail[c].y;
+    if (h < hidden) {
+      if (store_residual) *reinterpret_cast<float2*>(res + h) = x[c];
+      sq += x[c].x * x[c].x + x[c].y * x[c].y;
+    }
+  }
+  inv = 1.f;
+  if (weight) inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)hidden + eps);
+  bf16_t* dst = out + (size_t)blockIdx.x * hidden;
+#pragma unroll
+  for (int c = 0; c < RUNS; ++c) {
+    const int h = c * 2048 + (int)threadIdx.x * 2;
+    if (h >= hidden) continue;
+    *reinterpret_cast<uint32_t*>(dst + h) = (uint32_t)float_to_bf16_bits(x[c].x * inv * next[c].x) |
+                                            ((uint32_t)float_to_bf16_bits(x[c].y * inv * next[c].y) << 16);
+  }
+}
+
 // dtype: of delta, gate, proj, table and out.  Returns -2 for sizes the fused kernel does not take (rows longer than
 // a workgroup holds, a wider token input): the caller then runs the steps one by one.
 extern "C" int ta_norm_side_norm(void* residual, const void* delta, const void* post_weight, float post_eps, const void* gate,
@@ -457,6 +585,16 @@ extern "C" int ta_norm_side_norm(void* residual, const void* delta, const void* 
         (float*)residual, (const TT*)delta, (const float*)post_weight, post_eps, (const TT*)gate, (const TT*)proj,      \
         proj_stride, (const float*)side_norm, side_eps, (const TT*)table, table_width, (const int*)token_ids, offset,   \
         dim, (const float*)weight, eps, (TT*)out, (const int*)rows, hidden, store_residual)
+    if (dtype != DT_F32 && dim <= 16 && n_rows <= compute_units()) {
+#define HELD_SIDE(RR)                                                                                                  \
+      norm_side_norm_held_kernel<RR><<<n_rows, NA_WIDE, 0, stream>>>(                                                  \
+          (float*)residual, (const bf16_t*)delta, (const float*)post_weight, post_eps, (const bf16_t*)gate,            \
+          (const bf16_t*)proj, proj_stride, (const float*)side_norm, side_eps, (const bf16_t*)table, table_width,      \
+          (const int*)token_ids, offset, dim, (const float*)weight, eps, (bf16_t*)out, (const int*)rows, hidden, store_residual)
+      if (hidden <= 2048) HELD_SIDE(1); else HELD_SIDE(2);
+#undef HELD_SIDE
+      return LAUNCH_STATUS();
+    }
     if (dtype == DT_F32) { if (hidden <= 1024) SIDE(float, 1); else if (hidden <= 2048) SIDE(float, 2); else SIDE(float, 4); }
     else { if (hidden <= 1024) SIDE(bf16_t, 1); else if (hidden <= 2048) SIDE(bf16_t, 2); else SIDE(bf16_t, 4); }
 #undef SIDE
