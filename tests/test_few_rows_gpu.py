@@ -17,6 +17,39 @@ def rounded(t):
     return t.to(torch.bfloat16).to(torch.float64)
 
 
+# Inner widths with a block of sixteen columns left over, a shared expert wider than four others (four parts), narrower than one
+# (one part), and whose last part of K is empty (a part of 64 for 72 columns in two); one row and sixteen, one expert and all of them.
+@pytest.mark.parametrize("width,inner,shared,experts,top,rows", [(64, 24, 104, 8, 2, 1), (1032, 40, 8, 3, 1, 16), (72, 1032, 1040, 4, 4, 5),
+                                                                 (896, 64, 72, 8, 3, 16), (1536, 72, 200, 1, 1, 3)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_chosen_experts_beside_one_that_all_rows_use(ops, width, inner, shared, experts, top, rows, weighted):
+    gen = torch.Generator().manual_seed(width + rows)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, dtype=torch.float64)
+    sizes = [inner] * experts + [shared]
+    first = [rounded(rand(2, n, width) / width ** 0.5 * 2) for n in sizes]
+    second = [rounded(rand(width, n) / n ** 0.5) for n in sizes]
+    x = rounded(rand(rows, width))
+    chosen = torch.stack([torch.randperm(experts, generator=gen)[:top] for _ in range(rows)]).to(torch.int32)
+    weights = (0.2 + torch.rand(rows, top, generator=gen)).float()
+    share = (0.2 + torch.rand(rows, generator=gen)).float() if weighted else None
+    for e in range(experts):                                  # an expert nobody chose is not read
+        if not bool((chosen == e).any()):
+            first[e], second[e] = torch.full_like(first[e], float("nan")), torch.full_like(second[e], float("nan"))
+    on = lambda t: t.to(torch.bfloat16).cuda().contiguous()
+    parts = ops.experts_few(on(x), chosen.cuda(), weights.cuda(), experts, on(torch.cat([m.reshape(-1, width) for m in first])), True,
+                            inner, on(torch.cat(second, dim=1)), shared=shared, shared_weight=None if share is None else share.cuda())
+    expert = lambda t, e: second[e] @ (plain.silu(first[e][0] @ x[t]) * (first[e][1] @ x[t]))
+    want = torch.zeros(rows, width, dtype=torch.float64)
+    for t in range(rows):
+        want[t] = sum(float(weights[t, k]) * expert(t, int(chosen[t, k])) for k in range(top))
+        want[t] += (1.0 if share is None else float(share[t])) * expert(t, experts)
+    # Gate, up and their product are rounded to bfloat16 (2^-9 each), so a result is off by less than four such roundings of sums
+    # whose terms are as large as the largest result.
+    got = parts.resolve().double().cpu()
+    assert parts.partial.shape[0] == top + min(4, -(-shared // inner))
+    assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("width", [8, 520, 2048, 2056, 4096])
 @pytest.mark.parametrize("dim", [8, 16])
 @pytest.mark.parametrize("rows", [1, 256])

@@ -3,7 +3,9 @@
 // the second product, whose results lie pick by pick (slab k holds every row's k-th pick), for whoever adds them up.
 // bfloat16 operands, float sums on the matrix cores (16x16x32), computed transposed, C^T = W x^T, as the weight-streaming
 // product does: sixteen weight rows are the M side, up to sixteen (row, pick) pairs of the expert the N side, the waves of a
-// workgroup take turns of 64 elements of K and add up through LDS.
+// workgroup take turns of 64 elements of K and add up through LDS.  An expert that every row uses besides (of an inner width of
+// its own) is one further expert in both grids, whose pairs are the rows; its K in the second product is cut into parts about
+// as long as the others', each a slab of its own.
 #include "common.h"
 
 typedef __bf16 ef_bf16x8 __attribute__((ext_vector_type(8)));
@@ -35,6 +37,9 @@ __device__ __forceinline__ int ef_pairs_of(const int* __restrict__ chosen, int n
   }
   return __builtin_amdgcn_readfirstlane(count);
 }
+
+// The expert that all rows use: `inner` 0 says that there is none.  Its matrices stand behind the others'; weights null: 1.
+struct EfShared { int inner; const float* weights; bf16_t* act; int parts; };
 
 // acc[h] += sixteen rows of matrix h (row `wrow` + h * second of W, K elements `ldw` apart) times the lane's row of x, over this
 // wave's turns of K.
@@ -74,19 +79,32 @@ template <int NW, int HALVES>
 __global__ void __launch_bounds__(NW * WAVE)
 experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __restrict__ chosen, const float* __restrict__ weights,
                       int n_pairs, int top, const bf16_t* __restrict__ W, int inner, int hidden, bf16_t* __restrict__ act,
-                      int weigh_input) {
+                      int weigh_input, EfShared every) {
   HELD(x, x_stride, chosen, weights, n_pairs, top, W, inner, hidden, act, weigh_input);
   __shared__ int list[EF_MAX_PAIRS];
   __shared__ float red[NW][HALVES * 4][WAVE];
-  const int expert = blockIdx.y, n0 = blockIdx.x * 16;
-  const int count = ef_pairs_of(chosen, n_pairs, expert, list);
-  if (count == 0) return;                                    // nobody's expert: the same for the whole workgroup
+  // (The shared expert's workgroups, the ones with the most rows, come first.)
+  const bool shared = every.inner > 0 && blockIdx.y == 0;
+  const int expert = blockIdx.y - (every.inner > 0 ? 1 : 0), n0 = blockIdx.x * 16;
+  const bf16_t* first = W + (size_t)(shared ? gridDim.y - 1 : expert) * HALVES * inner * hidden;
+  int count;
+  if (shared) {                                              // its pairs are the rows
+    count = n_pairs / top;
+    inner = every.inner;
+    top = 1;
+    weights = every.weights;
+    act = every.act;
+    for (int i = threadIdx.x; i < count; i += NW * WAVE) list[i] = i;
+  } else {
+    count = ef_pairs_of(chosen, n_pairs, expert, list);
+  }
+  if (count == 0 || n0 >= inner) return;                     // nobody's expert, or past its width: the same for the whole workgroup
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = wave_index(), col = lane & 15, g = lane >> 4;
   const bf16_t* w_at[HALVES];
 #pragma unroll
   for (int h = 0; h < HALVES; ++h)
-    w_at[h] = W + ((size_t)expert * HALVES * inner + (size_t)h * inner + min(n0 + col, inner - 1)) * hidden + 8 * g;
+    w_at[h] = first + ((size_t)h * inner + min(n0 + col, inner - 1)) * hidden + 8 * g;
   for (int p0 = 0; p0 < count; p0 += 16) {
     const bool ok = p0 + col < count;
     const bf16_t* x_at = x + (size_t)(list[min(p0 + col, count - 1)] / top) * x_stride + 8 * g;
@@ -114,7 +132,7 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
         v[h] = bf16_bits_to_float(float_to_bf16_bits(v[h]));
       }
       const int p = list[p0 + c];
-      const float wgt = weights[p];
+      const float wgt = weights ? weights[p] : 1.f;
       float value;
       if constexpr (HALVES == 2) {
         const float before = weigh_input ? wgt : 1.f, z = before * v[0];
@@ -134,19 +152,35 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
 template <int NW>
 __global__ void __launch_bounds__(NW * WAVE)
 experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ chosen, int n_pairs, int top, int n_rows,
-                        const bf16_t* __restrict__ W, int ldw, int inner, int hidden, float* __restrict__ out) {
+                        const bf16_t* __restrict__ W, int ldw, int inner, int hidden, float* __restrict__ out, EfShared every) {
   HELD(act, chosen, n_pairs, top, n_rows, W, ldw, inner, hidden, out);
   __shared__ int list[EF_MAX_PAIRS];
   __shared__ float red[NW][4][WAVE];
-  const int expert = blockIdx.y, n0 = blockIdx.x * 16;
-  const int count = ef_pairs_of(chosen, n_pairs, expert, list);
+  const int part = blockIdx.y;                               // below every.parts: a part of the shared expert's K
+  const bool shared = part < every.parts;
+  const int expert = part - every.parts, n0 = blockIdx.x * 16;
+  const bf16_t* columns = W + (size_t)(shared ? (int)gridDim.y - every.parts : expert) * inner;
+  int count, stride = inner, slab = 0;
+  if (shared) {
+    const int length = ((every.inner + every.parts - 1) / every.parts + 63) / 64 * 64, begin = part * length;
+    count = n_rows;
+    stride = every.inner;
+    inner = min(length, every.inner - begin);                // (nothing of it: the slab is zeros)
+    columns += begin;
+    act = every.act + begin;
+    slab = top + part;
+    top = 1;
+    for (int i = threadIdx.x; i < count; i += NW * WAVE) list[i] = i;
+  } else {
+    count = ef_pairs_of(chosen, n_pairs, expert, list);
+  }
   if (count == 0) return;
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = wave_index(), col = lane & 15, g = lane >> 4;
-  const bf16_t* const w_at[1] = {W + (size_t)min(n0 + col, hidden - 1) * ldw + (size_t)expert * inner + 8 * g};
+  const bf16_t* const w_at[1] = {columns + (size_t)min(n0 + col, hidden - 1) * ldw + 8 * g};
   for (int p0 = 0; p0 < count; p0 += 16) {
     const bool ok = p0 + col < count;
-    const bf16_t* x_at = act + (size_t)list[min(p0 + col, count - 1)] * inner + 8 * g;
+    const bf16_t* x_at = act + (size_t)list[min(p0 + col, count - 1)] * stride + 8 * g;
     ef_floatx4 acc[1] = {(ef_floatx4){0.f, 0.f, 0.f, 0.f}};
     ef_walk<NW, 1>(w_at, x_at, ok, inner, g, wave, acc);
 #pragma unroll
@@ -159,29 +193,41 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
 #pragma unroll
       for (int w = 0; w < NW; ++w) v += red[w][r & 3][(r >> 2) * 16 + c];
       const int p = list[p0 + c];
-      out[((size_t)(p % top) * n_rows + p / top) * hidden + n0 + r] = v;
+      out[((size_t)(slab + p % top) * n_rows + p / top) * hidden + n0 + r] = v;
     }
     __syncthreads();
   }
 }
 
+// The parts the shared expert's second product is left in (slabs behind the picks').
+extern "C" int ta_experts_few_shared_parts(int inner, int shared) {
+  if (shared <= 0 || inner <= 0) return 0;
+  const int parts = (shared + inner - 1) / inner;
+  return parts < 4 ? parts : 4;
+}
+
 // Returns -2 for sizes the kernels do not take.  halves: 2 = gate and up rows (silu), 1 = up rows alone (squared ReLU).
+// shared: the inner width of the expert all rows use (0: there is none), whose matrices stand behind the others' in w_first and
+// w_second; shared_weights float [n_rows] or null; act_shared [n_rows, shared].
 extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, const void* weights, int n_rows, int top,
                               int n_experts, const void* w_first, int halves, int inner, int hidden, int weigh_input, void* act,
-                              const void* w_second, int ldw, void* out, hipStream_t stream) {
+                              const void* w_second, int ldw, void* out, int shared, const void* shared_weights, void* act_shared,
+                              hipStream_t stream) {
   if (n_rows <= 0) return 0;
   const long pairs = (long)n_rows * top;
-  if (top <= 0 || n_experts <= 0 || n_experts > 65535 || inner <= 0 || hidden <= 0 || (halves != 1 && halves != 2) ||
-      ldw < n_experts * inner || x_stride < hidden)
+  if (top <= 0 || n_experts <= 0 || n_experts > 65000 || inner <= 0 || hidden <= 0 || (halves != 1 && halves != 2) ||
+      ldw < n_experts * inner + shared || x_stride < hidden || shared < 0 || (shared > 0 && (!act_shared || weigh_input)))
     return -1;
-  if (pairs > EF_MAX_PAIRS || inner % 8 || hidden % 8 || ldw % 8 || x_stride % 8 ||
-      (((uintptr_t)x | (uintptr_t)w_first | (uintptr_t)w_second | (uintptr_t)act) & 15))
+  if (pairs > EF_MAX_PAIRS || inner % 8 || hidden % 8 || ldw % 8 || x_stride % 8 || shared % 8 ||
+      (((uintptr_t)x | (uintptr_t)w_first | (uintptr_t)w_second | (uintptr_t)act | (uintptr_t)act_shared) & 15))
     return -2;
-  const dim3 up((inner + 15) / 16, n_experts), down((hidden + 15) / 16, n_experts);
+  const EfShared every = {shared, (const float*)shared_weights, (bf16_t*)act_shared, ta_experts_few_shared_parts(inner, shared)};
+  const dim3 up(((inner > shared ? inner : shared) + 15) / 16, n_experts + (shared > 0)),
+      down((hidden + 15) / 16, n_experts + every.parts);
 #define UP(NW, HH) experts_few_up_kernel<NW, HH><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
-    (const float*)weights, (int)pairs, top, (const bf16_t*)w_first, inner, hidden, (bf16_t*)act, weigh_input)
+    (const float*)weights, (int)pairs, top, (const bf16_t*)w_first, inner, hidden, (bf16_t*)act, weigh_input, every)
 #define DOWN(NW) experts_few_down_kernel<NW><<<down, NW * WAVE, 0, stream>>>((const bf16_t*)act, (const int*)chosen, (int)pairs, top, \
-    n_rows, (const bf16_t*)w_second, ldw, inner, hidden, (float*)out)
+    n_rows, (const bf16_t*)w_second, ldw, inner, hidden, (float*)out, every)
   if (halves == 2) { if (hidden <= 1024) UP(4, 2); else UP(8, 2); }
   else { if (hidden <= 1024) UP(4, 1); else UP(8, 1); }
   int status = LAUNCH_STATUS();

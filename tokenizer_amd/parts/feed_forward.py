@@ -131,7 +131,8 @@ class RoutedExperts(FeedForward):
     experts a token chose and into zero for the others (the shared expert counts as chosen with weight 1), and the
     second product then adds the chosen experts' outputs up in its own sum.  That multiplies every token with every
     expert, which is right while the weights bound the step and nearly every expert is somebody's.  Steps of fewer
-    rows (`FEW_ROWS`, `FEW_AN_EXPERT`; bfloat16, no shared expert) read the chosen experts alone (`ops.experts_few`).  Steps
+    rows (`FEW_ROWS`, `FEW_AN_EXPERT`, beside a shared expert `FEW_ROWS_SHARED`; bfloat16) read the chosen experts, and the
+    shared one, alone (`ops.experts_few`).  Steps
     with `GROUPED_FROM` or more (token, expert) pairs, or `GROUPED_ROWS` or more rows, in bfloat16 sort the pairs by expert on
     the device into tiles of rows that belong to one expert each, multiply every tile with its expert's matrices alone, and add a token's experts
     up at the end (the shared expert runs as a dense one).  Either way the routing stays on the device, so the step's
@@ -165,6 +166,11 @@ class RoutedExperts(FeedForward):
     # 350 | 304, 32 rows 333 | 356; width 1,536, 4 of 64 of 768: 1 row 136 | 42, 8 rows 144 | 79, 64 rows 155 | 141.
     FEW_ROWS = 16
     FEW_AN_EXPERT = 4
+    # With a shared expert (every row's, so read by every block of sixteen rows) up to sixteen rows at any size.  Measured alike:
+    # width 896, 2 of 8 of 1,216 and a shared one of 2,432: 1 row 30 | 20, 16 rows 37 | 31, 64 rows 46 | 52; width 1,536, 2 of 8 of
+    # 2,240 and 4,480: 3 rows 60 | 50, 16 rows 81 | 68, 24 rows 68 | 76; width 3,584, 2 of 8 of 9,472 and 4,736: 1 row 338 | 129,
+    # 16 rows 415 | 352, 24 rows 351 | 386.
+    FEW_ROWS_SHARED = 16
 
     def __init__(self, spec: FeedForwardSpec, tensors: dict[str, torch.Tensor], runtime: Runtime):
         if (spec.activation, spec.gated) not in (("silu", True), ("relu2", False)):
@@ -271,10 +277,11 @@ class RoutedExperts(FeedForward):
         if (self.groupable and (x.shape[0] * self.top_k >= self.GROUPED_FROM or x.shape[0] >= self.GROUPED_ROWS)
                 and hasattr(ops, "grouped_linear")):
             return self._sorted(x, chosen, weights, shared_weight)
-        if (not self.shared and x.shape[0] <= max(self.FEW_ROWS, self.FEW_AN_EXPERT * self.n_experts // self.top_k)
-                and hasattr(ops, "experts_few")):
+        few = self.FEW_ROWS_SHARED if self.shared else max(self.FEW_ROWS, self.FEW_AN_EXPERT * self.n_experts // self.top_k)
+        if x.shape[0] <= few and hasattr(ops, "experts_few"):
             parts = ops.experts_few(x, chosen, weights, self.n_experts, self.w_gate_up, self.gated, self.inner, self.w_down,
-                                    weigh_input=self.weigh_input)
+                                    weigh_input=self.weigh_input,
+                                    **({"shared": self.shared, "shared_weight": shared_weight} if self.shared else {}))
             if parts is not None:
                 return parts if pending else parts.resolve()
         gate_up = ops.linear(x, self.w_gate_up)
