@@ -76,3 +76,32 @@ def test_norm_with_the_token_input_of_few_rows(ops, width, dim, rows):
             assert float((stream.double().cpu() - stored).abs().max()) <= 1e-4 * float(stored.abs().max())
             rows_want = want if picked is None else want[[rows - 1, 0]]
             assert float((out.double().cpu() - rows_want).abs().max()) <= 2 ** -8 * float(rows_want.abs().max()) + 1e-4
+
+
+# K of one, two, three and four steps of 32 (rounds of three, and what is left of one) and of no whole step; columns of one strip, one
+# past it, no multiple of four; an expert nobody chose, one with a single pair, one with several tiles.
+@pytest.mark.parametrize("k", [32, 64, 96, 160, 136])
+@pytest.mark.parametrize("n_out", [256, 257, 90, 520])
+@pytest.mark.parametrize("bm", [64, 128])
+def test_sorted_products_in_either_kernel(ops, k, n_out, bm):
+    gen = torch.Generator().manual_seed(k + n_out)
+    experts, rows, ldw = 4, 150, k + 24
+    rand = lambda *shape: rounded(torch.randn(*shape, generator=gen, dtype=torch.float64))
+    chosen = torch.where(torch.arange(rows) < 149, torch.tensor(2), torch.tensor(0)).to(torch.int32)[:, None]
+    chosen[:5] = 3
+    x, w = rand(rows, k), rand(experts, n_out, k) / k ** 0.5
+    w = rounded(w)
+    joined = torch.full((experts * n_out, ldw), float("nan"), dtype=torch.bfloat16)        # columns behind K are not read
+    joined[:, :k] = w.reshape(-1, k).to(torch.bfloat16)
+    slot_of, row_of, tile_expert = ops.expert_slots(chosen.cuda(), experts, bm)
+    on = lambda t: t.to(torch.bfloat16).cuda().contiguous()
+    want = torch.stack([w[int(chosen[t, 0])] @ x[t] for t in range(rows)])
+    slots = slot_of.cpu().long()
+    by_slot = torch.zeros(row_of.numel(), k, dtype=torch.float64)
+    by_slot[slots] = x
+    for expected in (1, 100_000):                             # (many tiles to come: the wide kernel, where K goes in whole steps)
+        for dtype in (torch.float32, torch.bfloat16):
+            for rows_of, source in ((row_of, x), (None, by_slot)):
+                got = ops.grouped_linear(on(source), rows_of, tile_expert, bm, joined.cuda(), n_out * ldw, n_out, k, dtype, expected=expected)
+                error = (got.double().cpu()[slots] - want).abs().max() / want.abs().max()
+                assert float(error) <= (2e-6 * k ** 0.5 if dtype == torch.float32 else 2 ** -8)

@@ -167,7 +167,7 @@ class Ops:
             getattr(self.lib, name).restype = ctypes.c_int
         self.lib.ta_grouped_gemm_bf16.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                                   ctypes.c_int, ctypes.c_void_p, ctypes.c_long, ctypes.c_int, ctypes.c_void_p,
-                                                  ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+                                                  ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
         self.lib.ta_library_gemm_bf16.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 5 + [
             ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_void_p]
         self._workspaces: dict[int, torch.Tensor] = {}
@@ -945,10 +945,12 @@ class Ops:
         return slot_of, row_of, tile_expert
 
     def grouped_linear(self, x: torch.Tensor, row_of: torch.Tensor | None, tile_expert: torch.Tensor, bm: int,
-                       weight: torch.Tensor, expert_stride: int, n_out: int, k: int, out_dtype: torch.dtype) -> torch.Tensor:
+                       weight: torch.Tensor, expert_stride: int, n_out: int, k: int, out_dtype: torch.dtype,
+                       expected: int | None = None) -> torch.Tensor:
         """out[slot] = x[row_of[slot]] (or x[slot] without `row_of`) @ W_e.T for every slot of every tile, W_e the
         [n_out, k] block of `weight` (contiguous [rows, ldw]) that starts `expert_stride` elements times the tile's
-        expert into it.  bfloat16 operands, float32 sums; out [tiles * bm, n_out] bfloat16 or float32."""
+        expert into it.  bfloat16 operands, float32 sums; out [tiles * bm, n_out] bfloat16 or float32.  `expected`: about how
+        many of the tiles will have slots (the choice of kernel goes by it)."""
         _dev(x, row_of, tile_expert, weight)
         tiles = tile_expert.numel()
         _need(x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.stride(1) == 1 and weight.is_contiguous(),
@@ -960,7 +962,8 @@ class Ops:
         out = torch.empty((tiles * bm, n_out), dtype=out_dtype, device=x.device)
         self._check(self.lib.ta_grouped_gemm_bf16(_ptr(x), x.stride(0), _ptr(row_of), _ptr(tile_expert), tiles, bm, _ptr(weight),
                                                   int(expert_stride), weight.shape[1], _ptr(out), n_out, n_out, k,
-                                                  _code(out_dtype), self._stream()), "grouped_linear")
+                                                  _code(out_dtype), tiles if expected is None else int(expected), self._stream()),
+                    "grouped_linear")
         return out
 
     def expert_combine(self, rows: torch.Tensor, slot_of: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None,

@@ -299,10 +299,17 @@ class RoutedExperts(FeedForward):
         """Tiles of rows that belong to one expert each: gate/up, the activation, down, then a token's experts added up."""
         ops = self.runtime.ops
         hidden, inner = x.shape[1], self.inner
-        bm = 128 if x.shape[0] * self.top_k >= 2048 * max(1, self.n_experts // 8) else 64
-        slot_of, row_of, tile_expert = ops.expert_slots(chosen, self.n_experts, bm)
         wide = (2 if self.gated else 1) * inner          # an expert's rows of the joined first matrix
-        gate_up = ops.grouped_linear(x, row_of, tile_expert, bm, self.w_gate_up, wide * hidden, wide, hidden, torch.bfloat16)
+        # Tiles of 128 slots where an expert has some 256 pairs, or fewer but more than 64 while such tiles still give every
+        # compute unit three workgroups of 256 columns.  (Both products, us, tiles of 64 | 128: width 3,584, 8 experts of 9,472, 100
+        # pairs an expert 483 | 447, 167 pairs 677 | 577; width 1,536, experts of 4,480, 167 pairs 162 | 183, 250 pairs 195 | 189.)
+        pairs = x.shape[0] * self.top_k
+        tiles = lambda height: pairs // height + self.n_experts // 2       # about as many as will have slots
+        bm = 128 if (pairs >= 2048 * max(1, self.n_experts // 8)
+                     or (pairs > 64 * self.n_experts and tiles(128) * -(-wide // 256) >= 700)) else 64
+        slot_of, row_of, tile_expert = ops.expert_slots(chosen, self.n_experts, bm)
+        gate_up = ops.grouped_linear(x, row_of, tile_expert, bm, self.w_gate_up, wide * hidden, wide, hidden, torch.bfloat16,
+                                     expected=tiles(bm))
         act = torch.empty((gate_up.shape[0], inner), dtype=x.dtype, device=x.device)
         if self.weigh_input:
             ops.expert_gate_slots(gate_up, slot_of, weights, act)
@@ -310,7 +317,8 @@ class RoutedExperts(FeedForward):
             ops.silu_gate(gate_up, act)
         else:
             ops.relu2(gate_up, act)
-        rows = ops.grouped_linear(act, None, tile_expert, bm, self.w_down, inner, hidden, inner, torch.float32)
+        rows = ops.grouped_linear(act, None, tile_expert, bm, self.w_down, inner, hidden, inner, torch.float32,
+                                  expected=tiles(bm))
         shared = None
         if self.shared:
             shared = ops.linear(ops.linear_silu_gate(x, self.w_shared_gate_up), self.w_shared_down)
