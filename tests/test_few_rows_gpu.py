@@ -105,3 +105,30 @@ def test_sorted_products_in_either_kernel(ops, k, n_out, bm):
                 got = ops.grouped_linear(on(source), rows_of, tile_expert, bm, joined.cuda(), n_out * ldw, n_out, k, dtype, expected=expected)
                 error = (got.double().cpu()[slots] - want).abs().max() / want.abs().max()
                 assert float(error) <= (2e-6 * k ** 0.5 if dtype == torch.float32 else 2 ** -8)
+
+
+# Rows of one piece a lane, of two and an incomplete one, the longest; fewer experts than waves, one more, many; more rows than compute
+# units (four waves a row).
+@pytest.mark.parametrize("width,experts,top,rows", [(8, 3, 2, 1), (512, 8, 2, 5), (1032, 9, 4, 3), (4096, 17, 1, 2), (896, 8, 2, 300),
+                                                    (2056, 64, 6, 7)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_routers_of_few_rows(ops, width, experts, top, rows, dtype):
+    width = min(width, 2048) if dtype == torch.float32 else width         # (the longest rows the kernels take, in bytes)
+    gen = torch.Generator().manual_seed(width + experts)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).to(dtype)
+    x, router = rand(rows, width), rand(experts, width)
+    logits = x.double() @ router.double().t()
+    chosen = torch.empty((rows, top), dtype=torch.int32, device="cuda")
+    weights = torch.empty((rows, top), dtype=torch.float32, device="cuda")
+    assert ops.route_rows(x.cuda(), router.cuda(), chosen, weights)
+    best = torch.topk(logits, top, dim=-1)
+    assert torch.equal(chosen.cpu().long(), best.indices)
+    # (Logits of about sqrt(width) from float sums of `width` products.)
+    torch.testing.assert_close(weights.double().cpu(), torch.softmax(best.values, -1), rtol=3e-6 * width, atol=1e-6)
+    gate = torch.empty(rows, dtype=torch.float32, device="cuda")
+    both = torch.cat([router, rand(1, width)])
+    assert ops.route_rows_scores(x.cuda(), both.cuda(), None, experts, 0, 0, chosen, weights, softmax=True, group_max=False, gate=gate)
+    assert torch.equal(chosen.cpu().long(), best.indices)
+    picked = torch.softmax(logits, -1).gather(1, best.indices)
+    torch.testing.assert_close(weights.double().cpu(), picked / (picked.sum(-1, keepdim=True) + 1e-20), rtol=3e-6 * width, atol=1e-6)
+    torch.testing.assert_close(gate.double().cpu(), torch.sigmoid(x.double() @ both[-1].double()), rtol=3e-6 * width, atol=1e-6)

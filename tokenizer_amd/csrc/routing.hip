@@ -74,43 +74,49 @@ template <> struct RtVec<float> {
   }
 };
 
+// The float sums of a row with router rows wave, wave + WAVES, ... below `count`, handed to `put(row, sum)` in every lane: a lane
+// keeps its PIECES pieces of sixteen bytes of the row.  Few rows (AHEAD): the first router row's pieces are asked for beside them, so
+// a wave with one row to do makes one trip to memory; many rows hide the trips of one behind the others', and a wave that holds
+// half as many registers leaves room for more of them.  (Pieces past the rows' end are the row's last ones again, replaced by zeros.)
+template <typename T, int PIECES, int WAVES, bool AHEAD, typename Put>
+__device__ __forceinline__ void rt_row_sums(const T* __restrict__ row, const T* __restrict__ router, int hidden, int count, Put put) {
+  constexpr int N = RtVec<T>::N;
+  const int lane = threadIdx.x & (WAVE - 1), wave = wave_index();
+  if (wave >= count) return;
+  float xv[PIECES][N], wv[PIECES][N];
+  auto ask = [&](const T* from, float (&v)[PIECES][N]) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) RtVec<T>::load(from + min((p * WAVE + lane) * N, hidden - N), v[p]);
+  };
+  ask(row, xv);
+  if (AHEAD) ask(router + (size_t)wave * hidden, wv);
+  for (int e = wave; e < count; e += WAVES) {
+    float sum = 0.f;
+    if (!AHEAD) ask(router + (size_t)e * hidden, wv);
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const bool in = (p * WAVE + lane) * N < hidden;
+#pragma unroll
+      for (int k = 0; k < N; ++k) sum = fmaf(in ? wv[p][k] : 0.f, in ? xv[p][k] : 0.f, sum);
+    }
+    if (AHEAD && e + WAVES < count) ask(router + (size_t)(e + WAVES) * hidden, wv);
+    put(e, wave_sum(sum));
+  }
+}
+
 // The router's product and the choice in one kernel, a workgroup a token: x [n_tokens, hidden] (row stride lda) and
-// router [n_experts, hidden] of type T in pieces of sixteen bytes; wave w forms the logits of experts w, w + 4, ... as
-// float sums (a lane keeps its pieces of the row), wave 0 then picks as route_top_kernel does.
-template <typename T>
-__global__ void __launch_bounds__(256)
+// router [n_experts, hidden] of type T in pieces of sixteen bytes; wave w forms the logits of experts w, w + WAVES, ... as
+// float sums, wave 0 then picks as route_top_kernel does.  (Three rows of 1,536 and 8 experts: 5.5 us with four waves and loads
+// behind branches, 4.4 with a wave an expert.)
+template <typename T, int PIECES, int WAVES>
+__global__ void __launch_bounds__(WAVES * WAVE)
 route_rows_kernel(const T* __restrict__ x, int lda, const T* __restrict__ router, int hidden, int n_experts, int top,
                   int* __restrict__ chosen, float* __restrict__ weights) {
-  constexpr int N = RtVec<T>::N;
   __shared__ float logit_s[RT_MAX_EXPERTS];
   const int t = blockIdx.x;
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-  const T* row = x + (size_t)t * lda;
-  float xv[RT_ROW_PIECES][N];
-#pragma unroll
-  for (int p = 0; p < RT_ROW_PIECES; ++p) {
-    const int at = (p * WAVE + lane) * N;
-    if (at < hidden) RtVec<T>::load(row + at, xv[p]);
-    else
-#pragma unroll
-      for (int k = 0; k < N; ++k) xv[p][k] = 0.f;
-  }
-  for (int e = wave; e < n_experts; e += 256 / WAVE) {
-    const T* w = router + (size_t)e * hidden;
-    float sum = 0.f;
-#pragma unroll
-    for (int p = 0; p < RT_ROW_PIECES; ++p) {
-      const int at = (p * WAVE + lane) * N;
-      if (at < hidden) {
-        float wv[N];
-        RtVec<T>::load(w + at, wv);
-#pragma unroll
-        for (int k = 0; k < N; ++k) sum = fmaf(wv[k], xv[p][k], sum);
-      }
-    }
-    sum = wave_sum(sum);
-    if (lane == 0) logit_s[e] = sum;
-  }
+  rt_row_sums<T, PIECES, WAVES, WAVES == 8>(x + (size_t)t * lda, router, hidden, n_experts,
+                                [&](int e, float sum) { if (lane == 0) logit_s[e] = sum; });
   __syncthreads();
   if (wave != 0) return;
   float top_value = 0.f, total = 0.f, mine = 0.f, last_value = INFINITY;
@@ -307,6 +313,16 @@ extern "C" int ta_route_top(const void* logits, int n_tokens, int n_experts, int
   return LAUNCH_STATUS();
 }
 
+// GO(type, pieces a lane keeps of a row, waves) for these rows: eight while there are no more rows than compute units, else four
+// (2,048 rows of 1,536: 14.5 us with eight, 8.4 with four).
+#define RT_PIECES(GO, TT, WW) do { const int pieces = (hidden + WAVE * piece - 1) / (WAVE * piece);                         \
+    if (pieces <= 1) GO(TT, 1, WW); else if (pieces <= 2) GO(TT, 2, WW); else if (pieces <= 4) GO(TT, 4, WW);               \
+    else GO(TT, 8, WW); } while (0)
+#define RT_INSTANCES(GO, count) do { const bool wide = n_tokens <= compute_units();                       \
+  if (dtype == DT_F32) { if (wide) RT_PIECES(GO, float, 8); else RT_PIECES(GO, float, 4); }                                  \
+  else { if (wide) RT_PIECES(GO, bf16_t, 8); else RT_PIECES(GO, bf16_t, 4); } } while (0);
+
+
 // Returns -2 for sizes the fused kernel does not take (the caller then forms the logits with a product of its own).
 extern "C" int ta_route_rows(const void* x, int lda, const void* router, int n_tokens, int hidden, int n_experts, int top,
                              void* chosen, void* weights, int dtype, hipStream_t stream) {
@@ -316,12 +332,10 @@ extern "C" int ta_route_rows(const void* x, int lda, const void* router, int n_t
   if (n_experts > RT_MAX_EXPERTS || hidden % piece || lda % piece || hidden > WAVE * RT_ROW_PIECES * piece ||
       (((uintptr_t)x | (uintptr_t)router) & 15))
     return -2;
-  if (dtype == DT_F32)
-    route_rows_kernel<float><<<n_tokens, 256, 0, stream>>>((const float*)x, lda, (const float*)router, hidden, n_experts, top,
-                                                           (int*)chosen, (float*)weights);
-  else
-    route_rows_kernel<bf16_t><<<n_tokens, 256, 0, stream>>>((const bf16_t*)x, lda, (const bf16_t*)router, hidden, n_experts,
-                                                            top, (int*)chosen, (float*)weights);
+#define ROUTE(TT, PP, WW) route_rows_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, 0, stream>>>((const TT*)x, lda, (const TT*)router, \
+    hidden, n_experts, top, (int*)chosen, (float*)weights)
+  RT_INSTANCES(ROUTE, n_experts)
+#undef ROUTE
   return LAUNCH_STATUS();
 }
 
@@ -529,65 +543,41 @@ route_scores_kernel(const float* __restrict__ logits, int stride, const float* _
 }
 
 // The router's product and the choice in one kernel, a token a workgroup (few rows: a decode step): as route_rows_kernel
-// forms the logits (float sums of the row with each expert's router row, the row kept in registers), then all four
-// waves choose together and the first stores.
-template <typename T>
-__global__ void __launch_bounds__(256)
+// forms the logits (float sums of the row with each expert's router row, the row kept in registers), then all
+// waves choose together and the first stores.  (Three rows of 896 and 8 experts in 4 groups: 6.8 us with four waves and loads
+// behind branches, 5.7 with a wave an expert.)
+template <typename T, int PIECES, int WAVES>
+__global__ void __launch_bounds__(WAVES * WAVE)
 route_rows_sigmoid_kernel(const T* __restrict__ x, int lda, const T* __restrict__ router, const float* __restrict__ correction,
                           int hidden, int n_experts, int n_groups, int keep, int top, int* __restrict__ chosen,
                           float* __restrict__ weights, int softmax = 0, int group_max = 0, float* __restrict__ gate = nullptr,
                           int raw = 0) {
-  constexpr int N = RtVec<T>::N;
   extern __shared__ float rs_scratch[];
   float* choice = rs_scratch;
   float* score = choice + n_experts;
   float* worth = score + n_experts;
   const int t = blockIdx.x;
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-  const T* row = x + (size_t)t * lda;
-  float xv[RT_ROW_PIECES][N];
-#pragma unroll
-  for (int p = 0; p < RT_ROW_PIECES; ++p) {
-    const int at = (p * WAVE + lane) * N;
-    if (at < hidden) RtVec<T>::load(row + at, xv[p]);
-    else
-#pragma unroll
-      for (int k = 0; k < N; ++k) xv[p][k] = 0.f;
-  }
   // (With a gate, the router has one row more: the gate's, behind the experts'.)
-  for (int e = wave; e < n_experts + (gate ? 1 : 0); e += 256 / WAVE) {
-    const T* w = router + (size_t)e * hidden;
-    float sum = 0.f;
-#pragma unroll
-    for (int p = 0; p < RT_ROW_PIECES; ++p) {
-      const int at = (p * WAVE + lane) * N;
-      if (at < hidden) {
-        float wv[N];
-        RtVec<T>::load(w + at, wv);
-#pragma unroll
-        for (int k = 0; k < N; ++k) sum = fmaf(wv[k], xv[p][k], sum);
-      }
+  rt_row_sums<T, PIECES, WAVES, WAVES == 8>(x + (size_t)t * lda, router, hidden, n_experts + (gate ? 1 : 0), [&](int e, float sum) {
+    if (lane != 0) return;
+    if (e == n_experts) {
+      gate[t] = 1.0f / (1.0f + expf(-sum));
+    } else if (softmax) {
+      score[e] = sum;                                        // the logit, until all of them are there
+    } else {
+      const float s = 1.0f / (1.0f + expf(-sum));
+      score[e] = s;
+      choice[e] = correction ? s + correction[e] : (n_groups > 0 ? s : sum);
     }
-    sum = wave_sum(sum);
-    if (lane == 0) {
-      if (e == n_experts) {
-        gate[t] = 1.0f / (1.0f + expf(-sum));
-      } else if (softmax) {
-        score[e] = sum;                                      // the logit, until all of them are there
-      } else {
-        const float s = 1.0f / (1.0f + expf(-sum));
-        score[e] = s;
-        choice[e] = correction ? s + correction[e] : (n_groups > 0 ? s : sum);
-      }
-    }
-  }
+  });
   __syncthreads();
   if (softmax) {                                             // every thread sums the few logits up for itself
     float top_logit = -INFINITY, total = 0.f;
     for (int e = 0; e < n_experts; ++e) top_logit = fmaxf(top_logit, score[e]);
     for (int e = 0; e < n_experts; ++e) total += expf(score[e] - top_logit);
     __syncthreads();
-    for (int e = threadIdx.x; e < n_experts; e += 256) {
+    for (int e = threadIdx.x; e < n_experts; e += WAVES * WAVE) {
       const float z = score[e], s = expf(z - top_logit) / total;
       score[e] = s;
       choice[e] = correction ? s + correction[e] : (n_groups > 0 ? s : z);
@@ -701,14 +691,11 @@ extern "C" int ta_route_rows_scores(const void* x, int lda, const void* router, 
       (((uintptr_t)x | (uintptr_t)router) & 15))
     return -2;
   const size_t lds = (size_t)(2 * n_experts + n_groups) * sizeof(float);
-  if (dtype == DT_F32)
-    route_rows_sigmoid_kernel<float><<<n_tokens, 256, lds, stream>>>((const float*)x, lda, (const float*)router,
-        (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights, softmax, group_max,
-        (float*)gate, raw);
-  else
-    route_rows_sigmoid_kernel<bf16_t><<<n_tokens, 256, lds, stream>>>((const bf16_t*)x, lda, (const bf16_t*)router,
-        (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights, softmax, group_max,
-        (float*)gate, raw);
+#define ROUTE(TT, PP, WW) route_rows_sigmoid_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, lds, stream>>>((const TT*)x, lda, \
+    (const TT*)router, (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights, softmax, \
+    group_max, (float*)gate, raw)
+  RT_INSTANCES(ROUTE, n_experts + (gate ? 1 : 0))
+#undef ROUTE
   return LAUNCH_STATUS();
 }
 
@@ -724,12 +711,10 @@ extern "C" int ta_route_rows_sigmoid(const void* x, int lda, const void* router,
       (((uintptr_t)x | (uintptr_t)router) & 15))
     return -2;
   const size_t lds = (size_t)(2 * n_experts + n_groups) * sizeof(float);
-  if (dtype == DT_F32)
-    route_rows_sigmoid_kernel<float><<<n_tokens, 256, lds, stream>>>((const float*)x, lda, (const float*)router,
-        (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights);
-  else
-    route_rows_sigmoid_kernel<bf16_t><<<n_tokens, 256, lds, stream>>>((const bf16_t*)x, lda, (const bf16_t*)router,
-        (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights);
+#define ROUTE(TT, PP, WW) route_rows_sigmoid_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, lds, stream>>>((const TT*)x, lda, \
+    (const TT*)router, (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights)
+  RT_INSTANCES(ROUTE, n_experts)
+#undef ROUTE
   return LAUNCH_STATUS();
 }
 
