@@ -132,3 +132,22 @@ def test_routers_of_few_rows(ops, width, experts, top, rows, dtype):
     picked = torch.softmax(logits, -1).gather(1, best.indices)
     torch.testing.assert_close(weights.double().cpu(), picked / (picked.sum(-1, keepdim=True) + 1e-20), rtol=3e-6 * width, atol=1e-6)
     torch.testing.assert_close(gate.double().cpu(), torch.sigmoid(x.double() @ both[-1].double()), rtol=3e-6 * width, atol=1e-6)
+
+
+@pytest.mark.parametrize("width", [4, 1028, 4096])
+@pytest.mark.parametrize("count,normed", [(0, True), (0, False), (2, False), (3, False)])
+def test_terms_onto_the_stream_without_terms_or_norm(ops, width, count, normed):
+    rows = 5
+    gen = torch.Generator().manual_seed(width + count)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, dtype=torch.float64)
+    stream, weight = rand(rows, width).float(), rand(width).float()
+    terms = [(rounded(rand(rows, width)), 0.5 + k, rand(width).float()) for k in range(count)]
+    want = stream.double() + sum((f * s.double() * t for t, f, s in terms), torch.zeros(rows, width, dtype=torch.float64))
+    wide = torch.full((rows, 2 * width), 7.0, dtype=torch.bfloat16, device="cuda")        # the result is a half of wider rows
+    residual = stream.cuda()
+    ops.add_terms_rmsnorm(residual, [(t.to(torch.bfloat16).cuda(), f, s.cuda()) for t, f, s in terms], weight.cuda() if normed else None,
+                          1e-5, wide[:, :width], store_residual=True)
+    torch.testing.assert_close(residual.double().cpu(), want, rtol=1e-6, atol=1e-6)
+    result = plain.weighted_norm(want, weight.double(), 1e-5) if normed else want
+    torch.testing.assert_close(wide[:, :width].double().cpu(), result, rtol=2 ** -8, atol=1e-6)
+    assert bool((wide[:, width:] == 7.0).all())
