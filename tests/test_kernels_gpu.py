@@ -463,6 +463,25 @@ def test_decode_attention_long_contexts_and_many_splits(ops, ref, window, target
         torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
 
 
+@pytest.mark.parametrize("n_q,n_kv,d,items,longest,window", [
+    (16, 16, 64, 9, 1000, None), (16, 16, 64, 9, 513, 200), (8, 8, 128, 17, 480, None), (32, 16, 32, 33, 1024, None),
+    (24, 8, 128, 130, 300, None), (24, 8, 64, 130, 97, 33), (16, 16, 64, 33, 1500, None), (4, 1, 256, 5, 700, None),
+    (2, 2, 256, 3, 600, 129), (14, 2, 64, 7, 2100, None)])
+def test_decode_attention_of_many_rows_and_few_parts(ops, ref, n_q, n_kv, d, items, longest, window):
+    # Rows whose keys stay in one part (workgroups of many waves where they are few), parts dealt to the workgroups from another
+    # start for every row, contexts of one key to the longest.  (The tolerance of the comparisons above: probabilities and
+    # results in bfloat16.)
+    lengths = [longest] + [1 + (i * 131) % longest for i in range(items - 1)]
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.bfloat16, n_q, n_kv, d, 16, lengths=lengths, q_lens=[1] * items, seed=17)
+    out_a = torch.full((items, n_q * d), float("nan"), dtype=torch.bfloat16).cuda()
+    out_b = torch.empty_like(out_a)
+    ops.paged_attention(qkv, out_a, k_pages, v_pages, positions, entry_of_token, table, n_q, n_kv, d, window, d ** -0.5,
+                        max_position=longest - 1)
+    ref.paged_attention(qkv, out_b, k_pages, v_pages, positions, entry_of_token, table, n_q, n_kv, d, window, d ** -0.5)
+    torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
+
+
 @pytest.mark.parametrize("attention_mode", ATTENTION_MODES, indirect=True)
 def test_paged_attention_finds_one_far_key(ops, attention_mode):
     dtype = attention_mode

@@ -57,9 +57,13 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   float (*acc_s)[D][17] = reinterpret_cast<float (*)[D][17]>(shared_s);
   __shared__ float m_s[DEC_WAVES][16], l_s[DEC_WAVES][16];
 
-  const int split = blockIdx.x;
   const int group = n_q / n_kv;
   const int head_blocks = (group + 15) / 16;
+  // Chiplets get every eighth workgroup, compute units every so manieth of those: with the parts counted alike for every row,
+  // one of them could get all rows' last parts, which short contexts leave empty.  So a row's count starts anywhere (the
+  // multiplicative hash of the row's number), the same place for all its parts.
+  const uint32_t turn = ((blockIdx.y + n_kv * head_blocks * blockIdx.z) * 2654435761u) >> 16;
+  const int split = (int)((blockIdx.x + turn) % (uint32_t)splits);
   const int kvh = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
   const int item = blockIdx.z;
   const int t = rows ? scalar_int(rows + item) : item;      // the same for every lane
@@ -415,16 +419,25 @@ static int launch_decode(const void* q, int q_stride, void* out, const void* k_p
                          float softcap, int tied, hipStream_t stream) {
   const int group = n_q / n_kv;
   dim3 grid(splits, n_kv * ((group + 15) / 16), n_items);
-  constexpr int NW = D > 128 ? 2 : 4;   // keeps the merge buffer within 64 KB of LDS
-#define GO(AHEAD, EE, TT) decode_attention_kernel<D, NW, AHEAD, EE, TT><<<grid, NW * WAVE, 0, stream>>>( \
+  constexpr int NW = D > 128 ? 2 : 4, WIDE = D <= 64 ? 16 : D <= 128 ? 8 : 4;
+#define GO(WAVES, AHEAD, EE, TT) decode_attention_kernel<D, WAVES, AHEAD, EE, TT><<<grid, WAVES * WAVE, 0, stream>>>( \
       (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_pages, (const bf16_t*)vt_pages, (const int*)rows, \
       (const int*)positions, (const int*)entry_of_token, (const int*)block_table, table_stride, (float*)part_o, \
       (float*)part_ml, n_q, n_kv, page_size, window, scale, split_keys, splits, chunk, (const float*)slopes, \
       (const float*)sinks, keep_first, kept_splits, n_v, softcap)
   const bool few = split_keys <= 32 * NW * 8;              // up to eight blocks a wave
-  if (chunk > 0 || slopes || kept_splits > 0 || softcap > 0.f || (n_v > 0 && n_v < n_kv)) { if (!vt_pages) return -1; if (few) GO(true, true, false); else GO(false, true, false); }
-  else if (tied || !vt_pages) { if (few) GO(true, false, true); else GO(false, false, true); }
-  else if (few) GO(true, false, false); else GO(false, false, false);
+  // Workgroups of sixteen (eight, four) waves where they are few and each has many keys: the keys are on their way at once, and
+  // a range of up to 1,024 is left in one part with nothing to merge.  64 tokens, 2 kv heads, 1,000 keys: head size 64 11.8 us
+  // in parts of four waves with their merge, 10.0 so; 128 20.4 and 17.7; one token, 256 15.6 (two waves) and 13.0.
+  // A chip that is full anyway is better off with four waves (1,024 workgroups of 500 keys, size 64: 22.7 us, 28.5 with sixteen).
+  const bool wide = split_keys >= (D > 128 ? 128 : 288) && split_keys <= 2048 &&
+                    (long)splits * n_kv * ((group + 15) / 16) * n_items < 512;
+  const bool extra = chunk > 0 || slopes || kept_splits > 0 || softcap > 0.f || (n_v > 0 && n_v < n_kv);
+  if (extra && !vt_pages) return -1;
+  if (extra) { if (wide) GO(WIDE, true, true, false); else if (few) GO(NW, true, true, false); else GO(NW, false, true, false); }
+  else if (tied || !vt_pages) { if (few) GO(NW, true, false, true); else GO(NW, false, false, true); }
+  else if (wide) GO(WIDE, true, false, false);
+  else if (few) GO(NW, true, false, false); else GO(NW, false, false, false);
 #undef GO
   int status = LAUNCH_STATUS();
   if (status == 0 && splits > 1) {

@@ -1315,10 +1315,22 @@ class Ops:
         if chunk is not None:
             max_keys = min(max_keys, chunk + 32)
         head_blocks = -(-(n_q // n_kv) // 16)
-        per_split = max(1, self.target_workgroups // max(1, n_items * n_kv * head_blocks))
+        rows_of_keys = n_items * n_kv * head_blocks
+        # (Two parts a row would be the whole grid in one go; with three the compute units that got short rows take more.)
+        per_split = max(3 if rows_of_keys < self.target_workgroups else 1, self.target_workgroups // max(1, rows_of_keys))
         split_keys = max(self.min_split_keys, -(-max_keys // per_split))
+        if rows_of_keys >= self.target_workgroups or (2 * rows_of_keys >= self.target_workgroups and max_keys <= 1024):
+            # Two workgroups a compute unit and more without a cut: a merge would cost more than parts could give (head size
+            # 64, 512 rows of 1,000 keys 26.7 us in two parts, 22.8 in one; 1,024 of 1,500 94.5 with an empty part, 72.6 without).
+            split_keys = max(split_keys, max_keys + 31)
+        elif 8 * rows_of_keys >= self.target_workgroups and max_keys <= 1024 and not tied_values and v_pages is not None:
+            # Half a chip's worth of rows: a workgroup of many waves for each, cut only to give every compute unit one (128
+            # rows of 500 keys of size 64 8.9 -> 6.7 us, of 128 14.3 -> 10.1; a single row of 2,000 keys among short ones would
+            # take 23 us instead of 16, so longer ranges stay cut; tied values have workgroups of four waves only).
+            split_keys = max(split_keys, 512, -(-4 * rows_of_keys * max_keys // self.target_workgroups))
         split_keys = -(-split_keys // 32) * 32
-        splits = max(1, -(-(max_keys + 31) // split_keys))
+        # (A window's or run's first key may lie within its block of 32; without either the first key is key 0.)
+        splits = max(1, -(-(max_keys + (0 if window is None and chunk is None else 31)) // split_keys))
         kept_splits = -(-int(keep_first) // split_keys) if keep_first and window is not None else 0
         splits += kept_splits
         part_o = part_ml = None
