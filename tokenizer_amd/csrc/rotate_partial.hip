@@ -14,8 +14,12 @@
 // in float; coordinates from rot on pass.  slots (or null): page * page_size + offset of each token, negative =
 // nothing is stored.  Key pages [n_pages, n_k, page_size, d]; value pages transposed inside a page,
 // [n_pages, n_v, dv, page_size].
-template <typename T>
-__global__ void __launch_bounds__(RP_THREADS)
+// THREADS: a loop below is a trip to memory a turn, and while tokens are no more than compute units a workgroup has one to
+// itself: 1,024 threads then go through a row of 896 to 4,096 elements in a turn or a few, 256 otherwise.
+// (28 / 4 heads of 64, both norms, half a head turning: three tokens 7.2 -> 5.4 us; 16 / 16 of 128 12.4 -> 6.9; 300 tokens of the
+// latter 14.6 either way, and 1,024 threads would leave a compute unit two tokens at a time.)
+template <typename T, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 norm_rotate_store_kernel(T* __restrict__ qkv, int row_stride, const float* __restrict__ bias,
                          const int* __restrict__ positions, const float* __restrict__ rates, int rot,
                          const int* __restrict__ slots, T* __restrict__ k_pages, T* __restrict__ v_pages,
@@ -30,7 +34,7 @@ norm_rotate_store_kernel(T* __restrict__ qkv, int row_stride, const float* __res
   const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
   if (half > 0) {
     const float position = (float)positions[t];
-    for (int i = threadIdx.x; i < half; i += RP_THREADS) {
+    for (int i = threadIdx.x; i < half; i += THREADS) {
       float s, c;
       sincosf(position * rates[i], &s, &c);
       cos_s[i] = c;
@@ -40,7 +44,7 @@ norm_rotate_store_kernel(T* __restrict__ qkv, int row_stride, const float* __res
   float inv_q = 1.f, inv_k = 1.f;
   if (q_norm) {
     float sq = 0.f;
-    for (int i = threadIdx.x; i < q_size; i += RP_THREADS) {
+    for (int i = threadIdx.x; i < q_size; i += THREADS) {
       const float v = ld(row + i) + (bias ? bias[i] : 0.f);
       sq += v * v;
     }
@@ -48,7 +52,7 @@ norm_rotate_store_kernel(T* __restrict__ qkv, int row_stride, const float* __res
   }
   if (k_norm && k_size > 0) {
     float sq = 0.f;
-    for (int i = threadIdx.x; i < k_size; i += RP_THREADS) {
+    for (int i = threadIdx.x; i < k_size; i += THREADS) {
       const float v = ld(row + q_size + i) + (bias ? bias[q_size + i] : 0.f);
       sq += v * v;
     }
@@ -57,7 +61,7 @@ norm_rotate_store_kernel(T* __restrict__ qkv, int row_stride, const float* __res
   __syncthreads();
   const bool changes = bias || q_norm || k_norm;
   // The pairs that turn.
-  for (int idx = threadIdx.x; idx < (n_q + n_k) * half; idx += RP_THREADS) {
+  for (int idx = threadIdx.x; idx < (n_q + n_k) * half; idx += THREADS) {
     const int head = idx / half, i = idx - head * half;
     const int at = head * d + i, with = at + half;
     float a = ld(row + at), b = ld(row + with);
@@ -77,7 +81,7 @@ norm_rotate_store_kernel(T* __restrict__ qkv, int row_stride, const float* __res
   }
   // The coordinates that pass.
   const int rest = d - rot;
-  for (int idx = threadIdx.x; idx < (n_q + n_k) * rest; idx += RP_THREADS) {
+  for (int idx = threadIdx.x; idx < (n_q + n_k) * rest; idx += THREADS) {
     const int head = idx / rest, i = rot + (idx - head * rest);
     const int at = head * d + i;
     float a = ld(row + at);
@@ -93,7 +97,7 @@ norm_rotate_store_kernel(T* __restrict__ qkv, int row_stride, const float* __res
   }
   // Values.
   const int v_at = q_size + k_size;
-  for (int idx = threadIdx.x; idx < n_v * dv; idx += RP_THREADS) {
+  for (int idx = threadIdx.x; idx < n_v * dv; idx += THREADS) {
     float a = ld(row + v_at + idx);
     if (bias) { a += bias[v_at + idx]; st(row + v_at + idx, a); }
     if (slot >= 0) {
@@ -110,14 +114,13 @@ extern "C" int ta_norm_rotate_store(void* qkv, int row_stride, const void* bias,
   if (n_tokens <= 0) return 0;
   if (rot < 0 || rot % 2 || rot > d || rot / 2 > RP_MAX_HALF || d <= 0 || dv <= 0 || n_q < 0 || n_k < 0 || n_v < 0) return -1;
   if (rot > 0 && !rates) return -1;
-  if (dtype == DT_F32)
-    norm_rotate_store_kernel<float><<<n_tokens, RP_THREADS, 0, stream>>>(
-        (float*)qkv, row_stride, (const float*)bias, (const int*)positions, (const float*)rates, rot, (const int*)slots,
-        (float*)k_pages, (float*)v_pages, n_q, n_k, n_v, d, dv, page_size, (const float*)q_norm, (const float*)k_norm, eps);
-  else
-    norm_rotate_store_kernel<bf16_t><<<n_tokens, RP_THREADS, 0, stream>>>(
-        (bf16_t*)qkv, row_stride, (const float*)bias, (const int*)positions, (const float*)rates, rot, (const int*)slots,
-        (bf16_t*)k_pages, (bf16_t*)v_pages, n_q, n_k, n_v, d, dv, page_size, (const float*)q_norm, (const float*)k_norm, eps);
+#define GO(T, THREADS) norm_rotate_store_kernel<T, THREADS><<<n_tokens, THREADS, 0, stream>>>( \
+      (T*)qkv, row_stride, (const float*)bias, (const int*)positions, (const float*)rates, rot, (const int*)slots, \
+      (T*)k_pages, (T*)v_pages, n_q, n_k, n_v, d, dv, page_size, (const float*)q_norm, (const float*)k_norm, eps)
+  const bool few = n_tokens <= compute_units();
+  if (dtype == DT_F32) { if (few) GO(float, 1024); else GO(float, 256); }
+  else { if (few) GO(bf16_t, 1024); else GO(bf16_t, 256); }
+#undef GO
   return LAUNCH_STATUS();
 }
 
