@@ -112,3 +112,34 @@ def test_attention(ops, ref, geometry, form, monkeypatch):
     torch.testing.assert_close(run(ops), want, **close)
     monkeypatch.setattr(ops, "use_fast_attention", False)
     torch.testing.assert_close(run(ops), want, **close)
+
+
+@pytest.mark.parametrize("geometry", [(6, 2, 64, 16), (20, 1, 16, 16), (2, 2, 256, 32)])
+@pytest.mark.parametrize("form", [dict(), dict(window=29), dict(chunk=50), dict(window=29, keep_first=21)], ids=str)
+def test_attention_keeps_an_infinite_value_to_the_queries_that_see_its_key(ops, ref, geometry, form):
+    """Values that are infinite or no number at keys that some queries of a tile see and others do not (later tokens of the
+    tile, keys that have just left the window or lie in front of the run), and at ones just outside a single token's reach."""
+    n_q, n_kv, d, page_size = geometry
+    lengths, q_lens = [300, 64, 90], [100, 1, 21]
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.float32, n_q, n_kv, d, page_size, lengths=lengths, q_lens=q_lens, seed=32)
+    infinity, nothing = float("inf"), float("nan")
+    for entry, key, coordinate, value in ((0, 205, 3, infinity), (0, 250, 4, nothing), (0, 268, 5, -infinity), (0, 180, 6, infinity),
+                                          (0, 5, 7, infinity), (1, 25, 2, nothing), (1, 33, 1, infinity), (1, 49, 5, -infinity),
+                                          (2, 40, 9, infinity), (2, 89, 10, nothing)):
+        v_pages[int(table[entry, key // page_size]), n_kv - 1, coordinate, key % page_size] = value
+
+    def run(which, batch=None):
+        on = (lambda t: t.cpu()) if which is ref else (lambda t: t)
+        out = on(torch.full((qkv.shape[0], n_q * d), 7.0, device="cuda"))
+        which.paged_attention(*map(on, (qkv, out, k_pages, v_pages, positions, entry_of_token, table)), n_q, n_kv, d,
+                              form.get("window"), 1.0 / math.sqrt(d), max_position=max(lengths) - 1,
+                              **({"batch": batch} if batch else {}), **{name: v for name, v in form.items() if name != "window"})
+        return out.cuda()
+
+    want = run(ref)
+    clean = torch.isfinite(want)
+    assert 0 < int((~clean).sum()) < want.numel() // 2
+    for got in (run(ops, make_batch(lengths, q_lens)), run(ops)):
+        assert torch.equal(torch.isfinite(got), clean)
+        torch.testing.assert_close(got, want, rtol=2e-5, atol=4e-6, equal_nan=True)

@@ -63,7 +63,7 @@ attention_f32_kernel(F32Args p) {
     int lo = p.window >= 0 && at > p.window ? at - p.window : 0;
     return p.chunk > 0 ? max(lo, at / p.chunk * p.chunk) : lo;
   };
-  const int lo = low_of(pos), lo_block = low_of(first_pos) / 16;
+  const int lo = low_of(pos), lo_first = low_of(first_pos), lo_last = low_of(last_pos), lo_block = lo_first / 16;
   // Blocks of sixteen keys in the order they are walked: the kept first ones, then from the first any query sees.
   const int kept = min((min(p.keep_first, last_pos + 1) + 15) / 16, lo_block);
   const int blocks = kept + last_pos / 16 - lo_block + 1;
@@ -103,15 +103,22 @@ attention_f32_kernel(F32Args p) {
   const float slope = p.slopes ? p.slopes[head] : 0.f;
   if (begin + wave < end) ask(begin + wave);
   for (int index = begin + wave; index < end; index += F32_WAVES) {
-    const int key0 = first_key(index) + 4 * g;
+    const int block0 = first_key(index), key0 = block0 + 4 * g;
 #pragma unroll
     for (int i = 0; i < S; ++i) { k[i] = k_next[i]; v[i] = v_next[i]; }
-    if (key0 - 4 * g + 15 > last_pos) {
-      // Keys behind the last one are slots that nobody wrote: whatever they hold must not meet a weight, be it zero.
+    // Keys that some query of the workgroup does not see: a value must not meet their weight, be it zero, if it is no number
+    // or infinite.
+    const bool partly = block0 + 15 > first_pos || (block0 < lo_last && block0 + 15 >= p.keep_first);
+    if (partly) {
+      // Of keys that none sees (behind the last query, where nobody may have written, or between the kept first keys and the
+      // window) nothing is used.
 #pragma unroll
-      for (int i = 0; i < S; ++i)
+      for (int j = 0; j < 4; ++j) {
+        const int key = key0 + j;
+        const bool used = key <= last_pos && (key >= lo_first || key < p.keep_first);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[i][j] = key0 + j > last_pos ? 0.f : v[i][j];
+        for (int i = 0; i < S; ++i) v[i][j] = used ? v[i][j] : 0.f;
+      }
     }
     ask(index + F32_WAVES);
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;              // two chains of sums
@@ -145,6 +152,33 @@ attention_f32_kernel(F32Args p) {
     m = m_new;
 #pragma unroll
     for (int i = 0; i < S; ++i) acc[i] *= keep;
+    if (!SINGLE && partly) {
+      float extremes = 0.f;                                // no number if one of the values is none, or infinite
+#pragma unroll
+      for (int i = 0; i < S; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) extremes = fmaf(v[i][j], 0.f, extremes);
+      if (__ballot(extremes != 0.f)) {
+        // Such a value goes to the queries that see its key and to no other: the block's products one key after the other.
+        // Lane (c, g) holds the sums of coordinates 4 g .. 4 g + 3 of each sixteen for query c.
+        for (int from = 0; from < 4; ++from)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int key = block0 + 4 * from + j;
+            const float weight = __shfl(score[j], 16 * from + c, WAVE);
+            const bool seen = key <= pos && (key >= lo || key < p.keep_first);
+#pragma unroll
+            for (int i = 0; i < S; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float value = __shfl(v[i][j], 16 * from + 4 * g + e, WAVE);
+                if (seen) acc[i][e] = fmaf(value, weight, acc[i][e]);
+              }
+          }
+#pragma unroll
+        for (int i = 0; i < S; ++i) v[i] = f32x4{0.f, 0.f, 0.f, 0.f};      // (all of it is in the sums)
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
