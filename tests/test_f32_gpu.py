@@ -55,6 +55,14 @@ def test_a_product_of_infinities_keeps_them_to_their_row(ops):
     assert torch.isfinite(got[[0, 2, 3]]).all() and not torch.isfinite(got[1]).any()
 
 
+@pytest.mark.parametrize("rows", [1, 3, 16, 17, 70])
+def test_a_product_over_nothing_is_its_bias(ops, rows):
+    x, w, bias = rand((rows, 0), torch.float32, 71), rand((20, 0), torch.float32, 72), rand((20,), torch.float32, 73)
+    for pending in (False, True):
+        assert torch.equal(ops.linear(x, w, bias, pending=pending), bias.expand(rows, 20))
+        assert torch.equal(ops.linear(x, w, pending=pending), torch.zeros(rows, 20, device="cuda"))
+
+
 @pytest.mark.parametrize("shape", [(1, 8, 4), (4, 4864, 896), (16, 100, 260), (9, 33, 64), (5, 24, 30)])
 def test_gated_product_of_few_rows(ops, shape):
     m, inner, k = shape

@@ -253,8 +253,9 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
     }
 }
 
+// (Rows without elements have no piece that could be read: they go to the kernels that walk K an element at a time.)
 static bool sixteen_bytes(const void* A, const void* W, int M, int K, int lda) {
-  return K % 4 == 0 && (M <= 1 || lda % 4 == 0) && (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
+  return K > 0 && K % 4 == 0 && (M <= 1 || lda % 4 == 0) && (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
 }
 
 // Which kernel and into how many parts of K (a power of two at most 8): `tile` 16 (few rows), 64 or 128, 0 (an element a
