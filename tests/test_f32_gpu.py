@@ -75,6 +75,12 @@ def test_gated_product_of_few_rows(ops, shape):
     torch.testing.assert_close(got.double(), want, rtol=2e-5, atol=bound)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17])
+def test_gated_product_over_nothing_is_zero(ops, rows):
+    x, w = rand((rows, 0), torch.float32, 74), rand((24, 0), torch.float32, 75)
+    assert torch.equal(ops.linear_silu_gate(x, w), torch.zeros(rows, 12, device="cuda"))
+
+
 FORMS = [dict(), dict(window=37), dict(chunk=50), dict(slopes=True, sinks=True), dict(softcap=3.0, sinks=True),
          dict(window=29, keep_first=21), dict(value_heads=1), dict(value_dim=40)]
 

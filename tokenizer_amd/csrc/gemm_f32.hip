@@ -331,12 +331,12 @@ extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void*
   return status;
 }
 
-// out[M, N/2] = silu(A W1^T) * (A W2^T), W = [W1; W2], for up to sixteen rows; -2 where the pieces are not aligned (the caller
+// out[M, N/2] = silu(A W1^T) * (A W2^T), W = [W1; W2], for up to sixteen rows; -2 where the pieces are not aligned or K is 0 (the caller
 // then runs the product and the gate one after the other).
 extern "C" int ta_gemm_f32_silu_gate(const void* A, const void* W, void* out, int M, int N, int K, int lda, int ldc,
                                      hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (N % 2 || K <= 0) return -1;
+  if (N % 2) return -1;
   if (M > 16 || !sixteen_bytes(A, W, M, K, lda)) return -2;
   gemm_f32_rows_kernel<true><<<(N / 2 + 7) / 8, 512, 0, stream>>>((const float*)A, (const float*)W, nullptr, (float*)out, M, N,
                                                                   K, lda, ldc, (K + 31) / 32, nullptr);
