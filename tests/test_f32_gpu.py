@@ -4,7 +4,7 @@ import math
 import pytest
 import torch
 
-from tokenizer_amd.kernels import PendingSum
+from tokenizer_amd.kernels import KernelError, PendingSum
 
 from kernel_refs import PlainOps
 from test_kernels_gpu import linear_tol, make_batch, make_paged_case, rand
@@ -79,6 +79,13 @@ def test_gated_product_of_few_rows(ops, shape):
 def test_gated_product_over_nothing_is_zero(ops, rows):
     x, w = rand((rows, 0), torch.float32, 74), rand((24, 0), torch.float32, 75)
     assert torch.equal(ops.linear_silu_gate(x, w), torch.zeros(rows, 12, device="cuda"))
+
+
+@pytest.mark.parametrize("rows", [4, 20])
+def test_gated_product_refuses_a_result_on_the_host(ops, rows):
+    x, w = rand((rows, 64), torch.float32, 76), rand((24, 64), torch.float32, 77)
+    with pytest.raises(KernelError):
+        ops.linear_silu_gate(x, w, out=torch.empty(rows, 12))
 
 
 FORMS = [dict(), dict(window=37), dict(chunk=50), dict(slopes=True, sinks=True), dict(softcap=3.0, sinks=True),

@@ -1626,6 +1626,7 @@ class Ops:
         if out is None:
             out = torch.empty((m, inner), dtype=x.dtype, device=x.device)
         _need(tuple(out.shape) == (m, inner) and out.dtype == x.dtype and out.is_contiguous(), "gated output shape")
+        _need(out.is_cuda, "kernel operands must live on the GPU")
         if act is not None and not isinstance(act, str):
             return self.silu_gate(self.linear(x, weight), out, act=act)
         if x.dtype == torch.float32 and act is None and 0 < m <= self.FUSED_ROWS:
