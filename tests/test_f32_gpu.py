@@ -164,3 +164,20 @@ def test_attention_keeps_an_infinite_value_to_the_queries_that_see_its_key(ops, 
     for got in (run(ops, make_batch(lengths, q_lens)), run(ops)):
         assert torch.equal(torch.isfinite(got), clean)
         torch.testing.assert_close(got, want, rtol=2e-5, atol=4e-6, equal_nan=True)
+
+
+def test_attention_passes_over_a_description_of_other_tokens(ops, ref):
+    n_q, n_kv, d, page_size, lengths, q_lens = 6, 2, 64, 16, [1, 300, 64], [1, 100, 2]
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.float32, n_q, n_kv, d, page_size, lengths=lengths, q_lens=q_lens, seed=33)
+
+    def run(which, batch=None):
+        on = (lambda t: t.cpu()) if which is ref else (lambda t: t)
+        out = on(torch.full((qkv.shape[0], n_q * d), float("nan"), device="cuda"))
+        which.paged_attention(*map(on, (qkv, out, k_pages, v_pages, positions, entry_of_token, table)), n_q, n_kv, d, None,
+                              1.0 / math.sqrt(d), max_position=max(lengths) - 1, **({"batch": batch} if batch else {}))
+        return out.cuda()
+
+    want = run(ref)
+    for batch in (make_batch(lengths, [1, 101, 2]), make_batch(lengths + [30], [1, 98, 2, 2])):    # other tokens, other entries
+        torch.testing.assert_close(run(ops, batch), want, rtol=2e-5, atol=4e-6)

@@ -1257,9 +1257,9 @@ class Ops:
         """Attention in 32 bits on the matrix cores' float instructions: the portions' tiles of sixteen tokens, and single
         tokens with the key range cut over workgroups.  False for a form that stays with the generic kernel."""
         tiles = batch.q_tiles.shape[0] if batch is not None else 0
-        _need(not tiles or (batch.n_tokens == qkv.shape[0] and batch.cu_q.numel() == block_table.shape[0] + 1),
-              "the batch description does not belong to these tokens")
-        single = qkv.shape[0] if batch is None or tiles == 0 else batch.decode_rows.numel()
+        if tiles and (batch.n_tokens != qkv.shape[0] or batch.cu_q.numel() != block_table.shape[0] + 1):
+            tiles = 0              # (a description of other tokens says nothing about these: each is taken by itself)
+        single = batch.decode_rows.numel() if tiles else qkv.shape[0]
         rows = batch.decode_rows if tiles and single else None
         max_keys = (block_table.shape[1] * page_size) if max_position is None else max_position + 1
         max_keys = -(-max_keys // self.PLAN_KEYS) * self.PLAN_KEYS          # (as for the bfloat16 kernels)
