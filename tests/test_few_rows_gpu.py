@@ -134,6 +134,19 @@ def test_routers_of_few_rows(ops, width, experts, top, rows, dtype):
     torch.testing.assert_close(gate.double().cpu(), torch.sigmoid(x.double() @ both[-1].double()), rtol=3e-6 * width, atol=1e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_router_over_nothing_takes_the_first_experts_alike(ops, dtype):
+    x, router = torch.empty((1, 0), dtype=dtype, device="cuda"), torch.empty((11, 0), dtype=dtype, device="cuda")
+    chosen, weights = torch.empty((1, 3), dtype=torch.int32, device="cuda"), torch.empty((1, 3), device="cuda")
+    first = torch.arange(3, dtype=torch.int32, device="cuda")[None]
+    for route in (lambda: ops.route_rows(x, router, chosen, weights),
+                  lambda: ops.route_rows_scores(x, router, None, 11, 0, 0, chosen, weights, softmax=True),
+                  lambda: ops.route_rows_sigmoid(x, router, torch.zeros(11, device="cuda"), 0, 0, chosen, weights)):
+        chosen.fill_(-1)
+        assert route() and torch.equal(chosen, first)
+        torch.testing.assert_close(weights, torch.full_like(weights, 1 / 3), rtol=1e-6, atol=0)
+
+
 @pytest.mark.parametrize("width", [4, 1028, 4096])
 @pytest.mark.parametrize("count,normed", [(0, True), (0, False), (2, False), (3, False)])
 def test_terms_onto_the_stream_without_terms_or_norm(ops, width, count, normed):

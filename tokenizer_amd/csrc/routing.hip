@@ -83,6 +83,10 @@ __device__ __forceinline__ void rt_row_sums(const T* __restrict__ row, const T* 
   constexpr int N = RtVec<T>::N;
   const int lane = threadIdx.x & (WAVE - 1), wave = wave_index();
   if (wave >= count) return;
+  if (hidden <= 0) {                                         // rows without a piece that could be read
+    for (int e = wave; e < count; e += WAVES) put(e, 0.f);
+    return;
+  }
   float xv[PIECES][N], wv[PIECES][N];
   auto ask = [&](const T* from, float (&v)[PIECES][N]) {
 #pragma unroll
