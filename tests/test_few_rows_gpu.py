@@ -17,6 +17,10 @@ def rounded(t):
     return t.to(torch.bfloat16).to(torch.float64)
 
 
+def rand_bf16(shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16).cuda()
+
+
 # Inner widths with a block of sixteen columns left over, a shared expert wider than four others (four parts), narrower than one
 # (one part), and whose last part of K is empty (a part of 64 for 72 columns in two); one row and sixteen, one expert and all of them.
 @pytest.mark.parametrize("width,inner,shared,experts,top,rows", [(64, 24, 104, 8, 2, 1), (1032, 40, 8, 3, 1, 16), (72, 1032, 1040, 4, 4, 5),
@@ -105,6 +109,21 @@ def test_sorted_products_in_either_kernel(ops, k, n_out, bm):
                 got = ops.grouped_linear(on(source), rows_of, tile_expert, bm, joined.cuda(), n_out * ldw, n_out, k, dtype, expected=expected)
                 error = (got.double().cpu()[slots] - want).abs().max() / want.abs().max()
                 assert float(error) <= (2e-6 * k ** 0.5 if dtype == torch.float32 else 2 ** -8)
+
+
+@pytest.mark.parametrize("bm", [64, 128])
+def test_sorted_products_pass_over_tiles_without_slots_anywhere_in_the_list(ops, bm):
+    k, n_out, experts = 64, 256, 3
+    of_tile = [2, -1, 0, -1, -1, 1, -1]
+    x, w = rand_bf16((len(of_tile) * bm, k), 41), rand_bf16((experts * n_out, k), 42)
+    on_tiles = torch.tensor(of_tile, dtype=torch.int32, device="cuda")
+    for expected in (1, 100_000):                             # (the latter runs the wide kernel)
+        got = ops.grouped_linear(x, None, on_tiles, bm, w, n_out * k, n_out, k, torch.float32, expected=expected)
+        for tile, expert in enumerate(of_tile):
+            if expert >= 0:
+                at = slice(tile * bm, tile * bm + bm)
+                want = x[at].double() @ w[expert * n_out:(expert + 1) * n_out].double().t()
+                assert float((got[at].double() - want).abs().max()) <= 2e-6 * k ** 0.5 * float(want.abs().max())
 
 
 # Rows of one piece a lane, of two and an incomplete one, the longest; fewer experts than waves, one more, many; more rows than compute

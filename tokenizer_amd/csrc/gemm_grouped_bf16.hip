@@ -175,7 +175,7 @@ grouped_gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
 // rows of 64 bytes keep their four pieces XOR-swizzled by the row (no bank is asked twice by the eight lanes that a read or
 // a write serves at a time); the fragments of the next two blocks of slots are read while two are multiplied.
 // Rounds of three steps run without a branch, so that the compiler counts the loads under way and waits for the oldest alone.
-// Workgroups run over the tiles that have slots alone, in groups of sixteen tiles times all columns; the chiplets (every eighth
+// Workgroups run over the tiles up to the last that has slots, in groups of sixteen tiles times all columns; the chiplets (every eighth
 // workgroup) get equal runs of that order, so what is under way on one chiplet at a time are sixteen tiles of slots times a few
 // strips of columns, and its L2 serves an operand's row several times for one trip from memory.
 // Bound by LDS and the vector memory pipe together (12 KB of fragments and 6 KB of rows a wave for 512 clocks of matrix work).
@@ -191,17 +191,21 @@ grouped_gemm_wide_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
   __shared__ __attribute__((aligned(16))) uint16_t a_s[2][BM * BK];
   __shared__ __attribute__((aligned(16))) uint16_t w_s[2][BN * BK];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(), r = lane & 15, g = lane >> 4;
-  // The tiles that have slots lead the list.
+  // The list up to its last tile with slots.
   int used = 0;
-  for (int base = 0; base < n_tiles; base += WAVE)
-    used += __popcll(__ballot(base + lane < n_tiles && tile_expert[min(base + lane, n_tiles - 1)] >= 0));
+  for (int base = 0; base < n_tiles; base += WAVE) {
+    const unsigned long long has = __ballot(base + lane < n_tiles && tile_expert[min(base + lane, n_tiles - 1)] >= 0);
+    if (has) used = base + WAVE - __clzll(has);
+  }
   used = __builtin_amdgcn_readfirstlane(used);
   const int strips = (N + BN - 1) / BN, total = used * strips, per_chiplet = (total + 7) / 8;
   const int turn = (int)(blockIdx.x >> 3), place = (int)(blockIdx.x & 7) * per_chiplet + turn;
   if (turn >= per_chiplet || place >= total) return;
   const int first = place / (GROUP * strips) * GROUP, high = min(GROUP, used - first), inside = place - first * strips;
   const int tile = first + inside % high, m0 = tile * BM, n0 = inside / high * BN;
-  const bf16_t* We = W + (size_t)scalar_int(tile_expert + tile) * expert_stride;
+  const int expert = scalar_int(tile_expert + tile);
+  if (expert < 0) return;                                   // (a tile without slots among the others)
+  const bf16_t* We = W + (size_t)expert * expert_stride;
   // A thread brings pieces of sixteen bytes of rows tid / 4, 64 further, ...: four neighbours a row's 64 bytes.  Places are
   // 32-bit offsets from a pointer that is the same for the workgroup and moves along K.
   uint32_t a_at[PA], w_at[4];
