@@ -126,6 +126,20 @@ def test_sorted_products_pass_over_tiles_without_slots_anywhere_in_the_list(ops,
                 assert float((got[at].double() - want).abs().max()) <= 2e-6 * k ** 0.5 * float(want.abs().max())
 
 
+def test_sorted_products_take_rows_far_apart(ops):
+    """More than 2^31 elements from the first row to the last that a single tile names."""
+    k, n_out, bm, rows = 64, 256, 64, 2100
+    x = torch.empty((rows, (1 << 20) + 8), dtype=torch.bfloat16, device="cuda")
+    x[:, :k] = rand_bf16((rows, k), 43)
+    w = rand_bf16((n_out, k), 44)
+    row_of = (torch.arange(bm, dtype=torch.int32, device="cuda") * 33 + 5).contiguous()
+    want = x[row_of.long(), :k].double() @ w.double().t()
+    for expected in (1, 100_000):
+        got = ops.grouped_linear(x, row_of, torch.zeros(1, dtype=torch.int32, device="cuda"), bm, w, n_out * k, n_out, k, torch.float32,
+                                 expected=expected)
+        assert float((got.double() - want).abs().max()) <= 2e-6 * k ** 0.5 * float(want.abs().max())
+
+
 # Rows of one piece a lane, of two and an incomplete one, the longest; fewer experts than waves, one more, many; more rows than compute
 # units (four waves a row).
 @pytest.mark.parametrize("width,experts,top,rows", [(8, 3, 2, 1), (512, 8, 2, 5), (1032, 9, 4, 3), (4096, 17, 1, 2), (896, 8, 2, 300),

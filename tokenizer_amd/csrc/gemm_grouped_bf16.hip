@@ -332,8 +332,8 @@ extern "C" int ta_expert_slots(const void* chosen, int n_entries, int top, int n
 }
 
 // bm: 64 or 128 (the tile height the slots were made for).  C has n_tiles * bm rows.  expected: about how many of the tiles will
-// have slots (the launch's sizes do not depend on it).
-extern "C" int ta_grouped_gemm_bf16(const void* A, int lda, const void* row_of, const void* tile_expert, int n_tiles, int bm,
+// have slots (the launch's sizes do not depend on it).  rows: how many A has.
+extern "C" int ta_grouped_gemm_bf16(const void* A, int rows, int lda, const void* row_of, const void* tile_expert, int n_tiles, int bm,
                                     const void* W, long expert_stride, int ldw, void* C, int ldc, int N, int K,
                                     int out_dtype, int expected, hipStream_t stream) {
   if (n_tiles <= 0 || N <= 0) return 0;
@@ -351,7 +351,7 @@ extern "C" int ta_grouped_gemm_bf16(const void* A, int lda, const void* row_of, 
   // columns over 3,584 1,276 | 1,018, 24 480 | 434; 24 tiles x 3,584 columns over 9,472 243 | 298.
   const int units = compute_units(), strips = (N + 255) / 256, blocks = (strips * n_tiles + 7) / 8 * 8;
   auto rounds = [&](int width) { return (int)(((long)((N + width - 1) / width) * expected + units - 1) / units); };
-  const bool wide = K % 32 == 0 && (long)(N - 1) * ldw + K < (1l << 31) && (long)n_tiles * bm * lda < (1l << 31) &&
+  const bool wide = K % 32 == 0 && (long)(N - 1) * ldw + K < (1l << 31) && (long)rows * lda < (1l << 31) &&
                     rounds(256) * (bm == 128 ? 1.65 : 3.15) < rounds(bm);
   if (wide) {
     if (bm == 128) { if (out_dtype == DT_F32) WIDE(128, float); else WIDE(128, bf16_t); }

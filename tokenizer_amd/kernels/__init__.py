@@ -165,7 +165,7 @@ class Ops:
                      "ta_fused_qk_temper",
                      "ta_expert_gate_slots"):
             getattr(self.lib, name).restype = ctypes.c_int
-        self.lib.ta_grouped_gemm_bf16.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
+        self.lib.ta_grouped_gemm_bf16.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                                   ctypes.c_int, ctypes.c_void_p, ctypes.c_long, ctypes.c_int, ctypes.c_void_p,
                                                   ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
         self.lib.ta_library_gemm_bf16.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 5 + [
@@ -960,7 +960,7 @@ class Ops:
         _need(tile_expert.dtype == torch.int32 and k % 8 == 0 and x.stride(0) % 8 == 0 and weight.shape[1] % 8 == 0
               and expert_stride % 8 == 0, "K, strides and the experts' offsets in eights")
         out = torch.empty((tiles * bm, n_out), dtype=out_dtype, device=x.device)
-        self._check(self.lib.ta_grouped_gemm_bf16(_ptr(x), x.stride(0), _ptr(row_of), _ptr(tile_expert), tiles, bm, _ptr(weight),
+        self._check(self.lib.ta_grouped_gemm_bf16(_ptr(x), x.shape[0], x.stride(0), _ptr(row_of), _ptr(tile_expert), tiles, bm, _ptr(weight),
                                                   int(expert_stride), weight.shape[1], _ptr(out), n_out, n_out, k,
                                                   _code(out_dtype), tiles if expected is None else int(expected), self._stream()),
                     "grouped_linear")
