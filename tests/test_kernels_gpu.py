@@ -482,6 +482,24 @@ def test_decode_attention_of_many_rows_and_few_parts(ops, ref, n_q, n_kv, d, ite
     torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
 
 
+@pytest.mark.parametrize("parts", [3, 4, 6, 8, 12, 16, 17, 24])
+@pytest.mark.parametrize("n_kv,items", [(1, 3), (4, 75)])
+def test_decode_attention_deals_every_part_of_every_row_once(ops, monkeypatch, ref, parts, n_kv, items):
+    # Counts that share 1, 2, 4 and 8 with the chiplets, few rows and more than one round of the compute units.
+    longest, d = 1500, 64
+    lengths = [longest] + [1 + (i * 131) % longest for i in range(items - 1)]
+    monkeypatch.setattr(ops, "min_split_keys", 32)
+    monkeypatch.setattr(ops, "target_workgroups", parts * items * n_kv)
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.bfloat16, 2 * n_kv, n_kv, d, 16, lengths=lengths, q_lens=[1] * items, seed=18)
+    out_a = torch.full((items, 2 * n_kv * d), float("nan"), dtype=torch.bfloat16).cuda()
+    out_b = torch.empty_like(out_a)
+    ops.paged_attention(qkv, out_a, k_pages, v_pages, positions, entry_of_token, table, 2 * n_kv, n_kv, d, None, d ** -0.5,
+                        max_position=longest - 1)
+    ref.paged_attention(qkv, out_b, k_pages, v_pages, positions, entry_of_token, table, 2 * n_kv, n_kv, d, None, d ** -0.5)
+    torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
+
+
 @pytest.mark.parametrize("attention_mode", ATTENTION_MODES, indirect=True)
 def test_paged_attention_finds_one_far_key(ops, attention_mode):
     dtype = attention_mode

@@ -46,7 +46,7 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
                         int table_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
                         int n_q, int n_kv, int page_size, int window, float scale, int split_keys, int splits,
                         int chunk, const float* __restrict__ slopes, const float* __restrict__ sinks,
-                        int keep_first, int kept_splits, int n_v, float softcap) {
+                        int keep_first, int kept_splits, int n_v, float softcap, int units_log2) {
   constexpr int KS = (D + 31) / 32;   // 32-wide steps over the head size for Q K^T
   constexpr int DB = D / 16;          // 16-row blocks of O^T
   HELD(q, q_stride, out, k_pages, vt_pages, rows, positions, entry_of_token, block_table, table_stride, part_o, part_ml,
@@ -59,10 +59,15 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
 
   const int group = n_q / n_kv;
   const int head_blocks = (group + 15) / 16;
-  // Chiplets get every eighth workgroup, compute units every so manieth of those: with the parts counted alike for every row,
-  // one of them could get all rows' last parts, which short contexts leave empty.  So a row's count starts anywhere (the
-  // multiplicative hash of the row's number), the same place for all its parts.
-  const uint32_t turn = ((blockIdx.y + n_kv * head_blocks * blockIdx.z) * 2654435761u) >> 16;
+  // Chiplets get every eighth workgroup, and a chiplet's compute units take those in turn.  With an even count of parts the same
+  // parts of all rows would land on the same chiplets and units, and short contexts leave the last parts empty.  So a row's
+  // count starts one further for every eight workgroups in front of it, and once more for every round of the units; an odd count
+  // goes round by itself.  (16 rows of 16 kv heads of size 64, contexts spread up to 8,000, four parts, three draws: counted alike
+  // in all rows 66, 66 and 51 us, from a hash of the row 66, 67 and 41, so 62, 63 and 41; 32 such rows, three parts, four draws:
+  // hashed 112 to 116, so 101 to 112.)
+  const uint32_t row = blockIdx.y + gridDim.y * blockIdx.z;
+  const int even = __builtin_ctz((uint32_t)splits | 8u);   // log2 of the greatest common divisor of the parts and eight
+  const uint32_t turn = even ? (row >> (3 - even)) + ((row * (uint32_t)splits) >> units_log2) : 0u;
   const int split = (int)((blockIdx.x + turn) % (uint32_t)splits);
   const int kvh = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
   const int item = blockIdx.z;
@@ -419,12 +424,13 @@ static int launch_decode(const void* q, int q_stride, void* out, const void* k_p
                          float softcap, int tied, hipStream_t stream) {
   const int group = n_q / n_kv;
   dim3 grid(splits, n_kv * ((group + 15) / 16), n_items);
+  const int units_log2 = 31 - __builtin_clz((unsigned)compute_units());
   constexpr int NW = D > 128 ? 2 : 4, WIDE = D <= 64 ? 16 : D <= 128 ? 8 : 4;
 #define GO(WAVES, AHEAD, EE, TT) decode_attention_kernel<D, WAVES, AHEAD, EE, TT><<<grid, WAVES * WAVE, 0, stream>>>( \
       (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_pages, (const bf16_t*)vt_pages, (const int*)rows, \
       (const int*)positions, (const int*)entry_of_token, (const int*)block_table, table_stride, (float*)part_o, \
       (float*)part_ml, n_q, n_kv, page_size, window, scale, split_keys, splits, chunk, (const float*)slopes, \
-      (const float*)sinks, keep_first, kept_splits, n_v, softcap)
+      (const float*)sinks, keep_first, kept_splits, n_v, softcap, units_log2)
   const bool few = split_keys <= 32 * NW * 8;              // up to eight blocks a wave
   // Workgroups of sixteen (eight, four) waves where they are few and each has many keys: the keys are on their way at once, and
   // a range of up to 1,024 is left in one part with nothing to merge.  64 tokens, 2 kv heads, 1,000 keys: head size 64 11.8 us
