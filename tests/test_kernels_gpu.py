@@ -500,6 +500,25 @@ def test_decode_attention_deals_every_part_of_every_row_once(ops, monkeypatch, r
     torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
 
 
+@pytest.mark.parametrize("reach", [dict(window=0), dict(window=31), dict(window=32), dict(window=95), dict(window=96),
+                                   dict(window=480), dict(chunk=32), dict(chunk=97), dict(window=70, chunk=96)], ids=str)
+def test_decode_attention_behind_windows_and_runs_that_start_anywhere_in_a_block(ops, monkeypatch, ref, reach):
+    # Every place of the first key within its block of 32, keys in parts of one block: a part too few would lose the last keys.
+    n_q, n_kv, d, reach = 4, 2, 64, dict(reach)
+    lengths = list(range(450, 514))
+    monkeypatch.setattr(ops, "min_split_keys", 32)
+    monkeypatch.setattr(ops, "target_workgroups", 1 << 20)
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.bfloat16, n_q, n_kv, d, 16, lengths=lengths, q_lens=[1] * len(lengths), seed=19)
+    out_a = torch.full((len(lengths), n_q * d), float("nan"), dtype=torch.bfloat16).cuda()
+    out_b = torch.empty_like(out_a)
+    window = reach.pop("window", None)
+    ops.paged_attention(qkv, out_a, k_pages, v_pages, positions, entry_of_token, table, n_q, n_kv, d, window, d ** -0.5,
+                        max_position=max(lengths) - 1, **reach)
+    ref.paged_attention(qkv, out_b, k_pages, v_pages, positions, entry_of_token, table, n_q, n_kv, d, window, d ** -0.5, **reach)
+    torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
+
+
 @pytest.mark.parametrize("attention_mode", ATTENTION_MODES, indirect=True)
 def test_paged_attention_finds_one_far_key(ops, attention_mode):
     dtype = attention_mode
