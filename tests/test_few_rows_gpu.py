@@ -22,7 +22,8 @@ def rand_bf16(shape, seed):
 
 
 # Inner widths with a block of sixteen columns left over, a shared expert wider than four others (four parts), narrower than one
-# (one part), and whose last part of K is empty (a part of 64 for 72 columns in two); one row and sixteen, one expert and all of them.
+# (one part), with parts that whole turns of 64 leave no columns for (104 in four parts of 24 are two of 64) and a last part of eight
+# (72 in two); one row and sixteen, one expert and all of them.
 @pytest.mark.parametrize("width,inner,shared,experts,top,rows", [(64, 24, 104, 8, 2, 1), (1032, 40, 8, 3, 1, 16), (72, 1032, 1040, 4, 4, 5),
                                                                  (896, 64, 72, 8, 3, 16), (1536, 72, 200, 1, 1, 3)])
 @pytest.mark.parametrize("weighted", [False, True])
@@ -50,7 +51,9 @@ def test_chosen_experts_beside_one_that_all_rows_use(ops, width, inner, shared, 
     # Gate, up and their product are rounded to bfloat16 (2^-9 each), so a result is off by less than four such roundings of sums
     # whose terms are as large as the largest result.
     got = parts.resolve().double().cpu()
-    assert parts.partial.shape[0] == top + min(4, -(-shared // inner))
+    # (As many parts of the shared expert as the others are long, four at most, of whole turns of 64: none is empty.)
+    length = -(-(-(-shared // min(4, -(-shared // inner)))) // 64) * 64
+    assert parts.partial.shape[0] == top + -(-shared // length)
     assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max())
 
 

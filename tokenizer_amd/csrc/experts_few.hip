@@ -39,7 +39,7 @@ __device__ __forceinline__ int ef_pairs_of(const int* __restrict__ chosen, int n
 }
 
 // The expert that all rows use: `inner` 0 says that there is none.  Its matrices stand behind the others'; weights null: 1.
-struct EfShared { int inner; const float* weights; bf16_t* act; int parts; };
+struct EfShared { int inner; const float* weights; bf16_t* act; int parts, length; };   // K of `inner` in `parts` of `length`
 
 // acc[h] += sixteen rows of matrix h (row `wrow` + h * second of W, K elements `ldw` apart) times the lane's row of x, over this
 // wave's turns of K.
@@ -162,10 +162,10 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
   const bf16_t* columns = W + (size_t)(shared ? (int)gridDim.y - every.parts : expert) * inner;
   int count, stride = inner, slab = 0;
   if (shared) {
-    const int length = ((every.inner + every.parts - 1) / every.parts + 63) / 64 * 64, begin = part * length;
+    const int begin = part * every.length;
     count = n_rows;
     stride = every.inner;
-    inner = min(length, every.inner - begin);                // (nothing of it: the slab is zeros)
+    inner = min(every.length, every.inner - begin);
     columns += begin;
     act = every.act + begin;
     slab = top + part;
@@ -199,11 +199,19 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
   }
 }
 
-// The parts the shared expert's second product is left in (slabs behind the picks').
+// The shared expert's second product: K in parts about as long as the others' K, four at most, each of whole turns of 64 and none
+// without one.
+static int shared_part(int inner, int shared) {
+  const int parts = (shared + inner - 1) / inner;
+  const int most = parts < 4 ? parts : 4;
+  return ((shared + most - 1) / most + 63) / 64 * 64;
+}
+
+// The parts it is left in (slabs behind the picks').
 extern "C" int ta_experts_few_shared_parts(int inner, int shared) {
   if (shared <= 0 || inner <= 0) return 0;
-  const int parts = (shared + inner - 1) / inner;
-  return parts < 4 ? parts : 4;
+  const int length = shared_part(inner, shared);
+  return (shared + length - 1) / length;
 }
 
 // Returns -2 for sizes the kernels do not take.  halves: 2 = gate and up rows (silu), 1 = up rows alone (squared ReLU).
@@ -221,7 +229,8 @@ extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, c
   if (pairs > EF_MAX_PAIRS || inner % 8 || hidden % 8 || ldw % 8 || x_stride % 8 || shared % 8 ||
       (((uintptr_t)x | (uintptr_t)w_first | (uintptr_t)w_second | (uintptr_t)act | (uintptr_t)act_shared) & 15))
     return -2;
-  const EfShared every = {shared, (const float*)shared_weights, (bf16_t*)act_shared, ta_experts_few_shared_parts(inner, shared)};
+  const EfShared every = {shared, (const float*)shared_weights, (bf16_t*)act_shared, ta_experts_few_shared_parts(inner, shared),
+                          shared > 0 ? shared_part(inner, shared) : 0};
   const dim3 up(((inner > shared ? inner : shared) + 15) / 16, n_experts + (shared > 0)),
       down((hidden + 15) / 16, n_experts + every.parts);
 #define UP(NW, HH) experts_few_up_kernel<NW, HH><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
