@@ -90,7 +90,7 @@ def test_norm_with_the_token_input_of_few_rows(ops, width, dim, rows):
 @pytest.mark.parametrize("k", [32, 64, 96, 160, 136])
 @pytest.mark.parametrize("n_out", [256, 257, 90, 520])
 @pytest.mark.parametrize("bm", [64, 128])
-def test_sorted_products_in_either_kernel(ops, k, n_out, bm):
+def test_sorted_products_in_either_kernel(ops, k, n_out, bm, monkeypatch):
     gen = torch.Generator().manual_seed(k + n_out)
     experts, rows, ldw = 4, 150, k + 24
     rand = lambda *shape: rounded(torch.randn(*shape, generator=gen, dtype=torch.float64))
@@ -106,22 +106,44 @@ def test_sorted_products_in_either_kernel(ops, k, n_out, bm):
     slots = slot_of.cpu().long()
     by_slot = torch.zeros(row_of.numel(), k, dtype=torch.float64)
     by_slot[slots] = x
-    for expected in (1, 100_000):                             # (many tiles to come: the wide kernel, where K goes in whole steps)
+    for wide in (-1, 1):                                      # (the wide kernel where K goes in whole steps)
+        monkeypatch.setattr(ops, "grouped_wide", wide)
         for dtype in (torch.float32, torch.bfloat16):
             for rows_of, source in ((row_of, x), (None, by_slot)):
-                got = ops.grouped_linear(on(source), rows_of, tile_expert, bm, joined.cuda(), n_out * ldw, n_out, k, dtype, expected=expected)
+                got = ops.grouped_linear(on(source), rows_of, tile_expert, bm, joined.cuda(), n_out * ldw, n_out, k, dtype)
                 error = (got.double().cpu()[slots] - want).abs().max() / want.abs().max()
                 assert float(error) <= (2e-6 * k ** 0.5 if dtype == torch.float32 else 2 ** -8)
 
 
+# A list of more than 64 tiles, and sixteen tiles at a time with a few left over, over several strips of columns.
+@pytest.mark.parametrize("bm,rows", [(64, 900), (128, 2700)])
+def test_sorted_products_of_many_tiles_in_either_kernel(ops, bm, rows, monkeypatch):
+    experts, top, k, n_out = 45, 2, 96, 520
+    gen = torch.Generator().manual_seed(bm)
+    chosen = torch.stack([torch.randperm(experts - 2, generator=gen)[:top] for _ in range(rows)]).to(torch.int32).cuda()
+    x, w = rand_bf16((rows, k), 45), rand_bf16((experts * n_out, k), 46)
+    slot_of, row_of, on_tiles = ops.expert_slots(chosen, experts, bm)
+    used = int((on_tiles >= 0).sum())
+    assert on_tiles.numel() > 64 and used > 16 and used % 16
+    want = torch.empty((rows * top, n_out), dtype=torch.float64, device="cuda")
+    for e in range(experts):
+        at = (chosen.reshape(-1) == e).nonzero()[:, 0]
+        want[at] = x[at // top].double() @ w[e * n_out:(e + 1) * n_out].double().t()
+    for wide in (-1, 1):
+        monkeypatch.setattr(ops, "grouped_wide", wide)
+        got = ops.grouped_linear(x, row_of, on_tiles, bm, w, n_out * k, n_out, k, torch.float32)[slot_of.long()]
+        assert float((got.double() - want).abs().max()) <= 2e-6 * k ** 0.5 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("bm", [64, 128])
-def test_sorted_products_pass_over_tiles_without_slots_anywhere_in_the_list(ops, bm):
+def test_sorted_products_pass_over_tiles_without_slots_anywhere_in_the_list(ops, bm, monkeypatch):
     k, n_out, experts = 64, 256, 3
     of_tile = [2, -1, 0, -1, -1, 1, -1]
     x, w = rand_bf16((len(of_tile) * bm, k), 41), rand_bf16((experts * n_out, k), 42)
     on_tiles = torch.tensor(of_tile, dtype=torch.int32, device="cuda")
-    for expected in (1, 100_000):                             # (the latter runs the wide kernel)
-        got = ops.grouped_linear(x, None, on_tiles, bm, w, n_out * k, n_out, k, torch.float32, expected=expected)
+    for wide in (-1, 1):
+        monkeypatch.setattr(ops, "grouped_wide", wide)
+        got = ops.grouped_linear(x, None, on_tiles, bm, w, n_out * k, n_out, k, torch.float32)
         for tile, expert in enumerate(of_tile):
             if expert >= 0:
                 at = slice(tile * bm, tile * bm + bm)
@@ -129,7 +151,7 @@ def test_sorted_products_pass_over_tiles_without_slots_anywhere_in_the_list(ops,
                 assert float((got[at].double() - want).abs().max()) <= 2e-6 * k ** 0.5 * float(want.abs().max())
 
 
-def test_sorted_products_take_rows_far_apart(ops):
+def test_sorted_products_take_rows_far_apart(ops, monkeypatch):
     """More than 2^31 elements from the first row to the last that a single tile names."""
     k, n_out, bm, rows = 64, 256, 64, 2100
     x = torch.empty((rows, (1 << 20) + 8), dtype=torch.bfloat16, device="cuda")
@@ -137,9 +159,9 @@ def test_sorted_products_take_rows_far_apart(ops):
     w = rand_bf16((n_out, k), 44)
     row_of = (torch.arange(bm, dtype=torch.int32, device="cuda") * 33 + 5).contiguous()
     want = x[row_of.long(), :k].double() @ w.double().t()
-    for expected in (1, 100_000):
-        got = ops.grouped_linear(x, row_of, torch.zeros(1, dtype=torch.int32, device="cuda"), bm, w, n_out * k, n_out, k, torch.float32,
-                                 expected=expected)
+    for wide in (-1, 1):
+        monkeypatch.setattr(ops, "grouped_wide", wide)
+        got = ops.grouped_linear(x, row_of, torch.zeros(1, dtype=torch.int32, device="cuda"), bm, w, n_out * k, n_out, k, torch.float32)
         assert float((got.double() - want).abs().max()) <= 2e-6 * k ** 0.5 * float(want.abs().max())
 
 

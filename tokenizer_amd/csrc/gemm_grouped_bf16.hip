@@ -332,10 +332,11 @@ extern "C" int ta_expert_slots(const void* chosen, int n_entries, int top, int n
 }
 
 // bm: 64 or 128 (the tile height the slots were made for).  C has n_tiles * bm rows.  expected: about how many of the tiles will
-// have slots (the launch's sizes do not depend on it).  rows: how many A has.
+// have slots (the launch's sizes do not depend on it).  rows: how many A has.  choice: 1 = the wide kernel wherever it can, -1 = never,
+// 0 = where it is expected to be the faster one.
 extern "C" int ta_grouped_gemm_bf16(const void* A, int rows, int lda, const void* row_of, const void* tile_expert, int n_tiles, int bm,
                                     const void* W, long expert_stride, int ldw, void* C, int ldc, int N, int K,
-                                    int out_dtype, int expected, hipStream_t stream) {
+                                    int out_dtype, int expected, int choice, hipStream_t stream) {
   if (n_tiles <= 0 || N <= 0) return 0;
   if ((K & 7) || (lda & 7) || (ldw & 7) || (expert_stride & 7) || K < 8 || (((uintptr_t)A | (uintptr_t)W) & 15)) return -1;
   if (bm != 64 && bm != 128) return -1;
@@ -352,7 +353,7 @@ extern "C" int ta_grouped_gemm_bf16(const void* A, int rows, int lda, const void
   const int units = compute_units(), strips = (N + 255) / 256, blocks = (strips * n_tiles + 7) / 8 * 8;
   auto rounds = [&](int width) { return (int)(((long)((N + width - 1) / width) * expected + units - 1) / units); };
   const bool wide = K % 32 == 0 && (long)(N - 1) * ldw + K < (1l << 31) && (long)rows * lda < (1l << 31) &&
-                    rounds(256) * (bm == 128 ? 1.65 : 3.15) < rounds(bm);
+                    (choice > 0 || (choice == 0 && rounds(256) * (bm == 128 ? 1.65 : 3.15) < rounds(bm)));
   if (wide) {
     if (bm == 128) { if (out_dtype == DT_F32) WIDE(128, float); else WIDE(128, bf16_t); }
     else if (out_dtype == DT_F32) WIDE(64, float); else WIDE(64, bf16_t);

@@ -167,7 +167,8 @@ class Ops:
             getattr(self.lib, name).restype = ctypes.c_int
         self.lib.ta_grouped_gemm_bf16.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                                   ctypes.c_int, ctypes.c_void_p, ctypes.c_long, ctypes.c_int, ctypes.c_void_p,
-                                                  ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+                                                  ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                                  ctypes.c_void_p]
         self.lib.ta_library_gemm_bf16.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 5 + [
             ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_void_p]
         self._workspaces: dict[int, torch.Tensor] = {}
@@ -922,6 +923,8 @@ class Ops:
 
     # Routed feed-forwards over sorted tokens (bfloat16): tiles of `bm` slots that belong to one expert each.
     GROUPED_EXPERTS = 256
+    grouped_wide = 0          # the kernel with tiles of 256 columns: 1 = wherever it can (K in steps of 32), -1 = never, 0 = where
+    #                           the launcher expects it to be the faster one
 
     @staticmethod
     def grouped_tiles(n_entries: int, n_experts: int, bm: int) -> int:
@@ -962,7 +965,7 @@ class Ops:
         out = torch.empty((tiles * bm, n_out), dtype=out_dtype, device=x.device)
         self._check(self.lib.ta_grouped_gemm_bf16(_ptr(x), x.shape[0], x.stride(0), _ptr(row_of), _ptr(tile_expert), tiles, bm, _ptr(weight),
                                                   int(expert_stride), weight.shape[1], _ptr(out), n_out, n_out, k,
-                                                  _code(out_dtype), tiles if expected is None else int(expected), self._stream()),
+                                                  _code(out_dtype), tiles if expected is None else int(expected), self.grouped_wide, self._stream()),
                     "grouped_linear")
         return out
 
