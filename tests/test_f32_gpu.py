@@ -92,7 +92,8 @@ FORMS = [dict(), dict(window=37), dict(chunk=50), dict(slopes=True, sinks=True),
          dict(window=29, keep_first=21), dict(value_heads=1), dict(value_dim=40)]
 
 
-@pytest.mark.parametrize("geometry", [(6, 2, 64, 16), (20, 1, 16, 16), (4, 2, 100, 48), (2, 2, 256, 32)])
+@pytest.mark.parametrize("geometry", [(6, 2, 64, 16), (20, 1, 16, 16), (4, 2, 100, 48), (2, 2, 256, 32), (4, 2, 32, 16),
+                                      (6, 2, 96, 32), (4, 4, 192, 16)])
 @pytest.mark.parametrize("form", FORMS, ids=str)
 def test_attention(ops, ref, geometry, form, monkeypatch):
     """Portions that start and end inside pages, tiles and blocks of keys, single tokens whose keys are cut over workgroups (also
@@ -124,9 +125,11 @@ def test_attention(ops, ref, geometry, form, monkeypatch):
     # (Scores of about 1 from sums of d products, weighted sums of at most 300 values of about 1.)
     close = dict(rtol=2e-5, atol=4e-6)
     batch = make_batch(lengths, q_lens)
-    assert ops.use_fast_attention
+    tiled, ran = ops._attention_f32, []
+    monkeypatch.setattr(ops, "_attention_f32", lambda *args: ran.append(tiled(*args)) or ran[-1])
     torch.testing.assert_close(run(ops, batch), want, **close)
     torch.testing.assert_close(run(ops), want, **close)
+    assert ran == [True, True]                                # (not the generic kernel in its place)
     monkeypatch.setattr(ops, "min_split_keys_f32", 16)
     torch.testing.assert_close(run(ops), want, **close)
     monkeypatch.setattr(ops, "target_workgroups", 1)
@@ -164,6 +167,26 @@ def test_attention_keeps_an_infinite_value_to_the_queries_that_see_its_key(ops, 
     for got in (run(ops, make_batch(lengths, q_lens)), run(ops)):
         assert torch.equal(torch.isfinite(got), clean)
         torch.testing.assert_close(got, want, rtol=2e-5, atol=4e-6, equal_nan=True)
+
+
+@pytest.mark.parametrize("head_dim,page_size,tied", [(64, 16, True), (260, 16, False), (30, 16, False), (64, 24, False)])
+def test_attention_of_other_forms_stays_with_the_generic_kernel(ops, ref, head_dim, page_size, tied, monkeypatch):
+    n_q, n_kv, lengths, q_lens = 4, 2, [40, 1, 70], [9, 1, 1]
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.float32, n_q, n_kv, head_dim, page_size, lengths=lengths, q_lens=q_lens, seed=34)
+    tiled, ran = ops._attention_f32, []
+    monkeypatch.setattr(ops, "_attention_f32", lambda *args: ran.append(tiled(*args)) or ran[-1])
+
+    def run(which):
+        on = (lambda t: t.cpu()) if which is ref else (lambda t: t)
+        out = on(torch.full((qkv.shape[0], n_q * head_dim), float("nan"), device="cuda"))
+        which.paged_attention(on(qkv), out, on(k_pages), None if tied else on(v_pages), on(positions), on(entry_of_token), on(table),
+                              n_q, n_kv, head_dim, None, 1.0 / math.sqrt(head_dim), max_position=max(lengths) - 1,
+                              **({"tied_values": True} if tied else {}))
+        return out.cuda()
+
+    torch.testing.assert_close(run(ops), run(ref), rtol=2e-5, atol=4e-6)
+    assert ran == [False]
 
 
 def test_attention_passes_over_a_description_of_other_tokens(ops, ref):

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from kernel_refs import PlainOps
 from plain import dolidra_plain as plain
 
 pytestmark = pytest.mark.gpu
@@ -224,8 +225,8 @@ def test_terms_onto_the_stream_without_terms_or_norm(ops, width, count, normed):
     assert bool((wide[:, width:] == 7.0).all())
 
 
-# More tokens than compute units (256 threads a token) against the same tokens in calls of few (1,024): rows shorter than either
-# workgroup, a row that 1,024 threads go through in turns with a rest, a whole-head and a partial rotation.
+# More tokens than compute units (256 threads a token) and the same tokens in calls of few (1,024), each against the reference: rows
+# shorter than either workgroup, a row that 1,024 threads go through in turns with a rest, a whole-head and a partial rotation.
 @pytest.mark.parametrize("n_q,n_k,n_v,d,dims", [(2, 1, 1, 24, 8), (14, 2, 2, 64, 64), (16, 16, 8, 128, 32)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_norm_rotation_and_store_of_many_tokens_and_of_few(ops, n_q, n_k, n_v, d, dims, dtype):
@@ -235,18 +236,19 @@ def test_norm_rotation_and_store_of_many_tokens_and_of_few(ops, n_q, n_k, n_v, d
     positions = torch.randint(0, 4096, (count,), generator=gen, dtype=torch.int32).cuda()
     slots = torch.randperm(count, generator=gen).to(torch.int32).cuda()
     rates, wq, wk = torch.rand(dims // 2, generator=gen).cuda(), torch.rand(n_q * d, generator=gen).cuda(), torch.rand(n_k * d, generator=gen).cuda()
-    results = []
+    pages = lambda device: (torch.zeros(count // 16 + 1, n_k, 16, d, dtype=dtype, device=device),
+                            torch.zeros(count // 16 + 1, n_v, d, 16, dtype=dtype, device=device))
+    want = (rows.cpu(), *pages("cpu"))
+    PlainOps(torch.float64).norm_rotate_store(want[0], None, positions.cpu(), rates.cpu(), dims, slots.cpu(), *want[1:], n_q, n_k, n_v,
+                                              d, d, wq.cpu(), wk.cpu(), 1e-5)
+    # Both results are rounded to bfloat16, where sums that differ by float32 rounding can end as neighbours (2^-7 of the value
+    # apart at most); float32: sums of up to 2,048 squares.  Two terms of up to about 5 may cancel.
+    bound = 2.0 ** -7 if dtype == torch.bfloat16 else 2e-5
     for step in (count, 40):
-        held = rows.clone()
-        k_pages = torch.zeros(count // 16 + 1, n_k, 16, d, dtype=dtype, device="cuda")
-        v_pages = torch.zeros(count // 16 + 1, n_v, d, 16, dtype=dtype, device="cuda")
+        got = (rows.clone(), *pages("cuda"))
         for at in range(0, count, step):
             part = slice(at, at + step)
-            ops.norm_rotate_store(held[part], None, positions[part], rates, dims, slots[part], k_pages, v_pages, n_q, n_k, n_v, d, d,
+            ops.norm_rotate_store(got[0][part], None, positions[part], rates, dims, slots[part], *got[1:], n_q, n_k, n_v, d, d,
                                   wq, wk, 1e-5)
-        results.append((held, k_pages, v_pages))
-    # The sums of squares come in another order: float32 rounding of up to 2,048 terms on the norm, then at most a neighbour.
-    bound = 2.0 ** -7 if dtype == torch.bfloat16 else 2e-5
-    for many, few in zip(*results):
-        torch.testing.assert_close(many.float(), few.float(), rtol=bound, atol=1e-5)
-    assert float((results[0][0] - rows).abs().max()) > 0.1
+        for mine, right in zip(got, want):
+            torch.testing.assert_close(mine.cpu().float(), right.float(), rtol=bound, atol=1e-5)
