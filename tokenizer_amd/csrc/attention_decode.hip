@@ -433,9 +433,10 @@ static int launch_decode(const void* q, int q_stride, void* out, const void* k_p
       (const float*)sinks, keep_first, kept_splits, n_v, softcap, units_log2)
   const bool few = split_keys <= 32 * NW * 8;              // up to eight blocks a wave
   // Workgroups of sixteen (eight, four) waves where they are few and each has many keys: the keys are on their way at once, and
-  // a range of up to 1,024 is left in one part with nothing to merge.  64 tokens, 2 kv heads, 1,000 keys: head size 64 11.8 us
-  // in parts of four waves with their merge, 10.0 so; 128 20.4 and 17.7; one token, 256 15.6 (two waves) and 13.0.
-  // A chip that is full anyway is better off with four waves (1,024 workgroups of 500 keys, size 64: 22.7 us, 28.5 with sixteen).
+  // fewer parts do.  64 tokens, 2 kv heads, 1,000 keys, two parts and their merge: head size 64 12.3 us in nine parts of four
+  // waves, 10.5 so; 128 21.0 and 17.9; of 500 keys, in one part without a merge, 9.2 -> 7.1 and 14.6 -> 10.4; one token, 256, eight
+  // heads on one, 16.2 (two waves) and 13.5.  Many workgroups are better off with four waves (1,024 of 500 keys, size 64: 22.7 us,
+  // 28.5 with sixteen); 512 is a measured line, two for each of 256 compute units.
   const bool wide = split_keys >= (D > 128 ? 128 : 288) && split_keys <= 2048 &&
                     (long)splits * n_kv * ((group + 15) / 16) * n_items < 512;
   const bool extra = chunk > 0 || slopes || kept_splits > 0 || softcap > 0.f || (n_v > 0 && n_v < n_kv);

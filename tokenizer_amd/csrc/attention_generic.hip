@@ -1,6 +1,7 @@
 // Attention over paged keys and values, one block per (token, query head), any storage type.
-// Plain float arithmetic (no matrix cores): this is the kernel of the 32-bit path and the
-// yardstick for the faster bfloat16 kernels.  Softmax runs online in float.
+// Plain float arithmetic (no matrix cores): what the matrix-core kernels of either type have no instance for (other head sizes,
+// value heads of another size than the key heads', 32-bit values that are the keys), and their yardstick.  Softmax runs online in
+// float.
 #include "common.h"
 
 #define ATT_WAVES 4

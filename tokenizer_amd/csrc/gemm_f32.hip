@@ -20,10 +20,10 @@ __device__ __forceinline__ float silu_f32(float g) { return g / (1.0f + expf(-g)
 // row, one of the upper half k+4..k+7: the sums run over the same k in both operands, whatever their order, so one sixteen
 // byte read feeds four matrix instructions.  The next step's rows are on their way to registers while the current one is
 // multiplied; two buffers in LDS, one barrier a step.
-// Bound by the matrix cores: 128 x 128 x 32 are 4,096 clocks of them against 32 KB fetched and 128 KB read from LDS.
+// Bound by the matrix cores: 128 x 128 x 32 are 4,096 clocks of them against 32 KB fetched and 64 KB read from LDS.
 // blockIdx.x runs over tiles so that the workgroups of one chiplet (every eighth) share strips of weight rows.
-// (1,280 rows at 0.5B sizes: gate/up, 9,728 columns over 896, 890 us with vector multiply-adds, 217 with this = 110 TFLOP/s; a
-// layer's four products 1,503 and 423 us.)
+// (1,280 rows at 0.5B sizes, vector multiply-adds and this: gate/up, 9,728 columns over 896, 283 us = 79 TFLOP/s and 203 = 110; down,
+// 896 columns over 4,864 with K cut, 863 and 135; a layer's four products 1,480 and 415.)
 template <int BM, int BN>
 __global__ void __launch_bounds__(256)
 gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
@@ -262,8 +262,8 @@ static bool sixteen_bytes(const void* A, const void* W, int M, int K, int lda) {
 // load).  Few rows: parts until there are workgroups for every compute unit, each of eight units of 32 at least, and only
 // where the next kernel adds them (`pending`): a reduction of its own costs as much as it saves.  Many rows: the estimate is
 // rounds of workgroups over the compute units, a round as long as its tile's multiplications at what the two tiles reach
-// (128 x 128: 110 of the 157 TFLOP/s there are, 64 x 64: 88), plus the parts' trip to memory and, where nobody else adds
-// them, a further launch.
+// (128 x 128: 110 to 121 of the 157 TFLOP/s there are; 64 x 64: 99 to 102 in one part, 90 in two, counted as 88), plus the
+// parts' trip to memory and, where nobody else adds them, a further launch.
 static void f32_choice(int M, int N, int K, bool aligned, bool pending, int* tile, int* parts) {
   const int units = compute_units();
   *tile = 0;

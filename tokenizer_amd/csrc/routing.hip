@@ -322,10 +322,9 @@ extern "C" int ta_route_top(const void* logits, int n_tokens, int n_experts, int
 #define RT_PIECES(GO, TT, WW) do { const int pieces = (hidden + WAVE * piece - 1) / (WAVE * piece);                         \
     if (pieces <= 1) GO(TT, 1, WW); else if (pieces <= 2) GO(TT, 2, WW); else if (pieces <= 4) GO(TT, 4, WW);               \
     else GO(TT, 8, WW); } while (0)
-#define RT_INSTANCES(GO, count) do { const bool wide = n_tokens <= compute_units();                       \
+#define RT_INSTANCES(GO) do { const bool wide = n_tokens <= compute_units();                       \
   if (dtype == DT_F32) { if (wide) RT_PIECES(GO, float, 8); else RT_PIECES(GO, float, 4); }                                  \
-  else { if (wide) RT_PIECES(GO, bf16_t, 8); else RT_PIECES(GO, bf16_t, 4); } } while (0);
-
+  else { if (wide) RT_PIECES(GO, bf16_t, 8); else RT_PIECES(GO, bf16_t, 4); } } while (0)
 
 // Returns -2 for sizes the fused kernel does not take (the caller then forms the logits with a product of its own).
 extern "C" int ta_route_rows(const void* x, int lda, const void* router, int n_tokens, int hidden, int n_experts, int top,
@@ -338,7 +337,7 @@ extern "C" int ta_route_rows(const void* x, int lda, const void* router, int n_t
     return -2;
 #define ROUTE(TT, PP, WW) route_rows_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, 0, stream>>>((const TT*)x, lda, (const TT*)router, \
     hidden, n_experts, top, (int*)chosen, (float*)weights)
-  RT_INSTANCES(ROUTE, n_experts)
+  RT_INSTANCES(ROUTE);
 #undef ROUTE
   return LAUNCH_STATUS();
 }
@@ -698,7 +697,7 @@ extern "C" int ta_route_rows_scores(const void* x, int lda, const void* router, 
 #define ROUTE(TT, PP, WW) route_rows_sigmoid_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, lds, stream>>>((const TT*)x, lda, \
     (const TT*)router, (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights, softmax, \
     group_max, (float*)gate, raw)
-  RT_INSTANCES(ROUTE, n_experts + (gate ? 1 : 0))
+  RT_INSTANCES(ROUTE);
 #undef ROUTE
   return LAUNCH_STATUS();
 }
@@ -717,7 +716,7 @@ extern "C" int ta_route_rows_sigmoid(const void* x, int lda, const void* router,
   const size_t lds = (size_t)(2 * n_experts + n_groups) * sizeof(float);
 #define ROUTE(TT, PP, WW) route_rows_sigmoid_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, lds, stream>>>((const TT*)x, lda, \
     (const TT*)router, (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights)
-  RT_INSTANCES(ROUTE, n_experts)
+  RT_INSTANCES(ROUTE);
 #undef ROUTE
   return LAUNCH_STATUS();
 }

@@ -1164,7 +1164,7 @@ class Ops:
 
         `keep_first` n (with a window): keys at positions below n stay visible behind the window.  `value_heads`
         (a divisor of n_kv): the value pages hold so many heads, and key head g reads value head
-        g / (n_kv / value_heads).  Both run the generic kernel.
+        g / (n_kv / value_heads).
 
         Beyond the plain form: `value_dim` (value heads of dv elements; out is [T, n_q dv]), `chunk` (only keys
         of the query's own run of so many positions, counted from position 0), `slopes` (float32 [n_q]: head h's
@@ -1175,8 +1175,8 @@ class Ops:
         value pages [n_pages, n_kv, d, page_size];
         positions, entry_of_token int32 [T]; block_table int32 [E, P]; a token at position p sees keys
         max(0, p - window)..p.  `max_position` (host) lets the wrapper check that the table is wide enough.
-        `batch` (a StepContext of the same tokens) lets bfloat16 batches run the tiled kernel on prompt
-        portions and the split kernel on single tokens; without it every token goes through the latter.
+        `batch` (a StepContext of the same tokens) lets the tiled kernel run on prompt portions and the split
+        kernel on single tokens; without it every token goes through the latter.
         """
         _dev(qkv, out, k_pages, v_pages, positions, entry_of_token, block_table)
         n_tokens = qkv.shape[0]
@@ -1298,7 +1298,7 @@ class Ops:
     prefill_shared = 0            # the prompt kernel whose waves share a block of keys through LDS: 1 = wherever it has
     #                               an instance, -1 = never, 0 = where the launcher expects it to be the faster one
     prefill_key_splits = True     # whether the prompt kernel may cut a tile's keys over workgroups (tests switch it off)
-    target_workgroups = 1024      # what the split of the key range aims at
+    target_workgroups = 1024      # what the split of the key range aims at (as the lines drawn by it, measured on 256 compute units)
     min_split_keys = 128          # ... in parts of at least so many keys (a block of 32 for each of a workgroup's four waves)
     PLAN_KEYS = 512               # launch shapes depend on the context only through its multiple of this
 
@@ -1323,11 +1323,12 @@ class Ops:
         per_split = max(3 if rows_of_keys < self.target_workgroups else 1, self.target_workgroups // max(1, rows_of_keys))
         split_keys = max(self.min_split_keys, -(-max_keys // per_split))
         if rows_of_keys >= self.target_workgroups or (2 * rows_of_keys >= self.target_workgroups and max_keys <= 1024):
-            # Two workgroups a compute unit and more without a cut: a merge would cost more than parts could give (head size
-            # 64, 512 rows of 1,000 keys 26.7 us in two parts, 22.8 in one; 1,024 of 1,500 94.5 with an empty part, 72.6 without).
+            # Whole: a merge would cost more than parts could give (head size 64, 512 rows of 1,000 keys 26.7 us in two parts, 22.8
+            # in one, spread up to that 19.4 and 16.8; 1,024 of 1,500 94.5 with an empty part, 72.6 without).  One row of 1,000 among
+            # 511 of 100 is the price, 10.4 to 12.3 us in two parts and 13.6 in one: the lengths are not known here.
             split_keys = max(split_keys, max_keys + 31)
         elif 8 * rows_of_keys >= self.target_workgroups and max_keys <= 1024 and not tied_values and v_pages is not None:
-            # Half a chip's worth of rows: a workgroup of many waves for each, cut only to give every compute unit one (128
+            # From 128 rows on a workgroup of many waves for each, cut only while there would be fewer than 256 of them (128
             # rows of 500 keys of size 64 8.9 -> 6.7 us, of 128 14.3 -> 10.1; a single row of 2,000 keys among short ones would
             # take 23 us instead of 16, so longer ranges stay cut; tied values have workgroups of four waves only).
             split_keys = max(split_keys, 512, -(-4 * rows_of_keys * max_keys // self.target_workgroups))

@@ -300,9 +300,11 @@ class RoutedExperts(FeedForward):
         ops = self.runtime.ops
         hidden, inner = x.shape[1], self.inner
         wide = (2 if self.gated else 1) * inner          # an expert's rows of the joined first matrix
-        # Tiles of 128 slots where an expert has some 256 pairs, or fewer but more than 64 while such tiles still give every
-        # compute unit three workgroups of 256 columns.  (Both products, us, tiles of 64 | 128: width 3,584, 8 experts of 9,472, 100
-        # pairs an expert 483 | 447, 167 pairs 677 | 577; width 1,536, experts of 4,480, 167 pairs 162 | 183, 250 pairs 195 | 189.)
+        # Tiles of 128 slots where an expert has some 256 pairs, or fewer but more than 64 while such tiles still make many
+        # workgroups of 256 columns.  (Both products on 256 compute units, us, tiles of 64 | 128, with the workgroups of the latter's
+        # first product: width 3,584, 8 experts of 9,472, 100 pairs an expert 483 | 447, 740; 167 pairs 677 | 577, 1,036; width 1,536,
+        # experts of 4,480, 167 pairs 162 | 183, 490; 250 pairs 195 | 189, 665.  The line of 700 lies among those, at no multiple of
+        # the units.)
         pairs = x.shape[0] * self.top_k
         tiles = lambda height: pairs // height + self.n_experts // 2       # about as many as will have slots
         bm = 128 if (pairs >= 2048 * max(1, self.n_experts // 8)
