@@ -58,6 +58,21 @@ def test_chosen_experts_beside_one_that_all_rows_use(ops, width, inner, shared, 
     assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("gated,shared,weigh_input", [(True, 48, False), (True, 0, True), (False, 0, False)])
+def test_a_pick_that_weighs_nothing_adds_nothing(ops, gated, shared, weigh_input):
+    """Expert 1 overflows on every row and is chosen with a weight of zero: the rows are those of expert 0 (and the shared one)."""
+    width, inner, experts, rows, halves = 64, 32, 3, 4, 2 if gated else 1
+    first, second = rand_bf16((halves * (experts * inner + shared), width), 51) / 8, rand_bf16((width, experts * inner + shared), 52)
+    x = rand_bf16((rows, width), 53).abs()
+    first[halves * inner:2 * halves * inner] = 3e38
+    chosen = torch.tensor([[0, 1]] * rows, dtype=torch.int32, device="cuda")
+    weights = torch.tensor([[0.75, 0.0]] * rows, device="cuda")
+    run = lambda: ops.experts_few(x, chosen, weights, experts, first, gated, inner, second, weigh_input=weigh_input, shared=shared).resolve()
+    got = run()
+    first[halves * inner:2 * halves * inner] = 0.25
+    assert bool(torch.isfinite(got).all()) and torch.equal(got, run())
+
+
 @pytest.mark.parametrize("width", [8, 520, 2048, 2056, 4096])
 @pytest.mark.parametrize("dim", [8, 16])
 @pytest.mark.parametrize("rows", [1, 256])

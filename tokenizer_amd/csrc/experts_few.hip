@@ -141,6 +141,8 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
         const float z = fmaxf(v[0], 0.f);
         value = wgt * (z * z);
       }
+      // (A pick that weighs nothing adds nothing, whatever its expert makes of the row: as the form over all experts has it.)
+      if (!shared && wgt == 0.f) value = 0.f;
       st(act + (size_t)p * inner + n0 + r, value);
     }
     __syncthreads();                                         // the sums are read before the next sixteen pairs' are written
