@@ -23,9 +23,11 @@ def ref():
     return PlainOps(torch.float64)
 
 
-# Few rows: one and sixteen, K of one piece, of one unit and a piece, no multiple of four (the element form); many rows: around a
+# Few rows: one and sixteen, K of one piece, of one unit and a piece, no multiple of four (the element form); vector multiply-adds
+# of one, two, four and eight rows of long K, columns that are no multiple of a wave's four; many rows: around a
 # tile's 64 and 128, K of a step and a piece, of no multiple of four, N of one column past a tile, K cut over workgroups.
 @pytest.mark.parametrize("shape", [(1, 16, 4), (16, 17, 36), (3, 40, 33), (7, 896, 4864), (15, 1152, 896), (2, 50, 260),
+                                   (1, 899, 896), (2, 2049, 4100), (4, 50, 4096), (3, 2052, 4104), (6, 38, 16384), (8, 21, 16388),
                                    (17, 64, 32), (64, 65, 36), (65, 63, 30), (129, 257, 100), (128, 128, 4864), (300, 896, 4864),
                                    (1280, 132, 896), (513, 1000, 64)])
 def test_products(ops, ref, shape):
@@ -63,7 +65,8 @@ def test_a_product_over_nothing_is_its_bias(ops, rows):
         assert torch.equal(ops.linear(x, w, pending=pending), torch.zeros(rows, 20, device="cuda"))
 
 
-@pytest.mark.parametrize("shape", [(1, 8, 4), (4, 4864, 896), (16, 100, 260), (9, 33, 64), (5, 24, 30)])
+@pytest.mark.parametrize("shape", [(1, 8, 4), (4, 4864, 896), (16, 100, 260), (9, 33, 64), (5, 24, 30), (1, 4863, 896), (2, 33, 260),
+                                   (4, 19, 4096), (7, 22, 16384)])
 def test_gated_product_of_few_rows(ops, shape):
     m, inner, k = shape
     x, w = rand((m, k), torch.float32, 66), rand((2 * inner, k), torch.float32, 67, 0.1)

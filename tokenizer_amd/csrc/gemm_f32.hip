@@ -5,7 +5,8 @@
 // operations a clock where vector multiply-adds do 128.  Three kernels:
 //   more than 16 rows   tiles through LDS, K cut over workgroups where the tiles alone would leave compute units idle
 //   up to 16 rows       one pass over the weights, sixteen weight rows a workgroup whose waves share K
-//   K no multiple of 4 (or unaligned rows), up to 16 rows    plain multiply-adds, an element a load
+//   one or two rows (up to four of large matrices), and up to 16 whose pieces of sixteen bytes are not aligned    vector
+//                       multiply-adds, four weight rows a wave
 #include "splitk_reduce.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -215,15 +216,19 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
   }
 }
 
-// Up to sixteen rows whose pieces of sixteen bytes do not lie on sixteen bytes: a wave takes four weight rows and walks K
-// an element a lane.
-template <int MR>
+// One or two rows, four of large matrices, and up to sixteen whose pieces of sixteen bytes do not lie on sixteen bytes (VEC false):
+// a wave takes four weight rows (GATED: two of W's first half and the two as far into its second, whose results meet in
+// silu(first) * second) and walks K sixteen bytes or an element a lane, every row of A against them.  With so little work for a
+// weight the matrix instructions gain nothing, and this way more of the weights are on their way at once: 9,728 columns over
+// 896, one row 8.7 us, 11.8 with the kernel above; 3,584 over 3,584 10.9 and 17.5; 896 over 4,864 11.6 and 19.4 (where K is cut
+// and the next norm adds the parts, the two together 13.9 and 11.9).
+template <int MR, bool VEC, bool GATED>
 __global__ void __launch_bounds__(256)
 gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
                 float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n0 = (blockIdx.x * 4 + wave) * 4;               // this wave's four weight rows
-  if (n0 >= N) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = N / 2;
+  const int n0 = (blockIdx.x * 4 + wave) * (GATED ? 2 : 4);  // this wave's weight rows
+  if (n0 >= (GATED ? half : N)) return;
   float acc[4][MR];
 #pragma unroll
   for (int r = 0; r < 4; ++r)
@@ -231,26 +236,52 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
     for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
   const float* w[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) w[r] = W + (size_t)min(n0 + r, N - 1) * K;
-  for (int k = lane; k < K; k += WAVE) {
-    float wv[4];
+  for (int r = 0; r < 4; ++r)
+    w[r] = W + (size_t)(GATED ? (r < 2 ? 0 : half) + min(n0 + (r & 1), half - 1) : min(n0 + r, N - 1)) * K;
+  if constexpr (VEC) {
+    for (int k = lane * 4; k < K; k += WAVE * 4) {
+      float4 wv[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) wv[r] = w[r][k];
+      for (int r = 0; r < 4; ++r) wv[r] = *reinterpret_cast<const float4*>(w[r] + k);
 #pragma unroll
-    for (int m = 0; m < MR; ++m) {
-      if (m >= M) break;
-      const float a = A[(size_t)m * lda + k];
+      for (int m = 0; m < MR; ++m) {
+        if (m >= M) break;
+        const float4 a = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r][m] = fmaf(a, wv[r], acc[r][m]);
+        for (int r = 0; r < 4; ++r)
+          acc[r][m] = fmaf(a.x, wv[r].x, fmaf(a.y, wv[r].y, fmaf(a.z, wv[r].z, fmaf(a.w, wv[r].w, acc[r][m]))));
+      }
+    }
+  } else {
+    for (int k = lane; k < K; k += WAVE) {
+      float wv[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) wv[r] = w[r][k];
+#pragma unroll
+      for (int m = 0; m < MR; ++m) {
+        if (m >= M) break;
+        const float a = A[(size_t)m * lda + k];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r][m] = fmaf(a, wv[r], acc[r][m]);
+      }
     }
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int m = 0; m < MR; ++m) {
+    float total[4];
 #pragma unroll
-    for (int m = 0; m < MR; ++m) {
-      const float total = wave_sum(acc[r][m]);
-      if (lane == 0 && m < M && n0 + r < N) C[(size_t)m * ldc + n0 + r] = total + (bias ? bias[n0 + r] : 0.f);
+    for (int r = 0; r < 4; ++r) total[r] = wave_sum(acc[r][m]);
+    if (lane != 0 || m >= M) continue;
+    if constexpr (GATED) {
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+        if (n0 + r < half) C[(size_t)m * ldc + n0 + r] = silu_f32(total[r]) * total[r + 2];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (n0 + r < N) C[(size_t)m * ldc + n0 + r] = total[r] + (bias ? bias[n0 + r] : 0.f);
     }
+  }
 }
 
 // (Rows without elements have no piece that could be read: they go to the kernels that walk K an element at a time.)
@@ -258,8 +289,17 @@ static bool sixteen_bytes(const void* A, const void* W, int M, int K, int lda) {
   return K > 0 && K % 4 == 0 && (M <= 1 || lda % 4 == 0) && (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
 }
 
-// Which kernel and into how many parts of K (a power of two at most 8): `tile` 16 (few rows), 64 or 128, 0 (an element a
-// load).  Few rows: parts until there are workgroups for every compute unit, each of eight units of 32 at least, and only
+// Whether up to sixteen aligned rows go to the vector kernel.  (us, matrix instructions | vector: two rows of 1,536 columns over
+// 8,960 34.0 | 21.7, of 2,048 over 1,024 6.6 | 6.6; four of 17,920 over 1,536 33.7 | 24.4, of 896 over 4,864 20.0 | 18.5, of 2,048
+// over 1,536 9.5 | 10.0, of 896 over 896 6.1 | 7.9; eight of 3,584 over 18,944 96.9 | 92.0, of 1,536 over 8,960 36.6 | 38.9.  With
+// K cut for the next norm, both kernels: two rows of 896 over 4,864 12.2 | 15.9, one of 3,584 over 18,944 80.9 | 67.9.)
+static bool vector_rows(int M, int N, int K, bool pending) {
+  if (pending && N % 4 == 0 && K >= 4096 && N <= 2048) return false;
+  return M <= 2 || (M <= 4 && (K >= 4096 || (long)N * K >= (8l << 20))) || (M <= 8 && K >= 16384 && !pending);
+}
+
+// Which kernel and into how many parts of K (a power of two at most 8): `tile` 16 (few rows), 64 or 128, 0 (vector
+// multiply-adds).  Few rows: parts until there are workgroups for every compute unit, each of eight units of 32 at least, and only
 // where the next kernel adds them (`pending`): a reduction of its own costs as much as it saves.  Many rows: the estimate is
 // rounds of workgroups over the compute units, a round as long as its tile's multiplications at what the two tiles reach
 // (128 x 128: 110 to 121 of the 157 TFLOP/s there are; 64 x 64: 99 to 102 in one part, 90 in two, counted as 88), plus the
@@ -269,7 +309,7 @@ static void f32_choice(int M, int N, int K, bool aligned, bool pending, int* til
   *tile = 0;
   *parts = 1;
   if (M <= 16) {
-    if (!aligned) return;
+    if (!aligned || vector_rows(M, N, K, pending)) return;
     *tile = 16;
     if (pending && N % 4 == 0)
       while (*parts < 8 && (N + 15) / 16 * *parts < units && K / 32 / (2 * *parts) >= 8) *parts *= 2;
@@ -322,8 +362,10 @@ extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void*
                                                              n_tiles, slabs);
   } else {
     const int blocks = (N + 15) / 16;
-#define GO(MR) gemv_f32_kernel<MR><<<blocks, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc)
-    if (M <= 1) GO(1); else if (M <= 2) GO(2); else if (M <= 4) GO(4); else if (M <= 8) GO(8); else GO(16);
+#define GO(MR, VEC) gemv_f32_kernel<MR, VEC, false><<<blocks, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc)
+    if (aligned) { if (M <= 1) GO(1, true); else if (M <= 2) GO(2, true); else if (M <= 4) GO(4, true); else GO(8, true); }
+    else if (M <= 1) GO(1, false); else if (M <= 2) GO(2, false); else if (M <= 4) GO(4, false);
+    else if (M <= 8) GO(8, false); else GO(16, false);
 #undef GO
   }
   int status = LAUNCH_STATUS();
@@ -338,7 +380,12 @@ extern "C" int ta_gemm_f32_silu_gate(const void* A, const void* W, void* out, in
   if (M <= 0 || N <= 0) return 0;
   if (N % 2) return -1;
   if (M > 16 || !sixteen_bytes(A, W, M, K, lda)) return -2;
-  gemm_f32_rows_kernel<true><<<(N / 2 + 7) / 8, 512, 0, stream>>>((const float*)A, (const float*)W, nullptr, (float*)out, M, N,
-                                                                  K, lda, ldc, (K + 31) / 32, nullptr);
+  const float *a = (const float*)A, *w = (const float*)W;
+  const int blocks = (N / 2 + 7) / 8;
+#define GO(MR) gemv_f32_kernel<MR, true, true><<<blocks, 256, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc)
+  if (!vector_rows(M, N, K, false))
+    gemm_f32_rows_kernel<true><<<blocks, 512, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc, (K + 31) / 32, nullptr);
+  else if (M <= 1) GO(1); else if (M <= 2) GO(2); else if (M <= 4) GO(4); else GO(8);
+#undef GO
   return LAUNCH_STATUS();
 }
