@@ -96,7 +96,7 @@ FORMS = [dict(), dict(window=37), dict(chunk=50), dict(slopes=True, sinks=True),
 
 
 @pytest.mark.parametrize("geometry", [(6, 2, 64, 16), (20, 1, 16, 16), (4, 2, 100, 48), (2, 2, 256, 32), (4, 2, 32, 16),
-                                      (6, 2, 96, 32), (4, 4, 192, 16)])
+                                      (6, 2, 96, 32), (4, 4, 192, 16), (5, 1, 96, 16), (17, 1, 128, 16)])
 @pytest.mark.parametrize("form", FORMS, ids=str)
 def test_attention(ops, ref, geometry, form, monkeypatch):
     """Portions that start and end inside pages, tiles and blocks of keys, single tokens whose keys are cut over workgroups (also

@@ -6,8 +6,6 @@
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-#define F32_WAVES 4
-
 struct F32Args {
   const float* q; int q_stride; float* out; const float* k_pages; const float* v_pages;
   const int* tiles; const int* cu_q; const int* first_position; const int* rows; const int* positions;
@@ -16,8 +14,8 @@ struct F32Args {
 };
 
 // A workgroup takes sixteen queries that see the same pages: SINGLE, the heads of one key head of one token (and one part
-// of its keys); else sixteen tokens of a portion under one head.  Its four waves walk the blocks of sixteen keys in turn and
-// bring their softmax states together through LDS at the end.  With the queries as columns of S^T = K Q^T, lane (column c,
+// of its keys); else sixteen tokens of a portion under one head.  Its waves walk the blocks of sixteen keys in turn and
+// bring their softmax states together through LDS at the end (eight where a single token's keys are one part and few).  With the queries as columns of S^T = K Q^T, lane (column c,
 // g) gets the scores of keys 4 g .. 4 g + 3; summed over the keys in the order j, g those are, as they stand, the right
 // operand of O^T = V^T P^T, and the left one, keys 4 g .. 4 g + 3 of a row of V^T, is one load of sixteen bytes from the
 // value page.  No operand goes through LDS.  S: blocks of sixteen coordinates.  Bound by the matrix cores while the
@@ -25,11 +23,11 @@ struct F32Args {
 // block's keys and values are asked for before the current one is worked on.
 // (14 / 2 heads of 64, portions of 77 to 700 tokens, 1,273 in all: 315 us with a workgroup a token and head on vector
 // multiply-adds, 39 with this; four single tokens behind as many keys 28.6 and 6.7 + 3.6 for the merge.)
-template <int S, bool SINGLE>
-__global__ void __launch_bounds__(F32_WAVES * WAVE)
+template <int S, bool SINGLE, int WAVES>
+__global__ void __launch_bounds__(WAVES * WAVE)
 attention_f32_kernel(F32Args p) {
-  __shared__ float m_s[F32_WAVES][16], l_s[F32_WAVES][16];
-  __shared__ float acc_s[F32_WAVES][S * 16][17];
+  __shared__ float m_s[WAVES][16], l_s[WAVES][16];
+  __shared__ float acc_s[WAVES][S * 16][17];
   const int lane = threadIdx.x & 63, wave = wave_index(), c = lane & 15, g = lane >> 4;
   const int group = p.n_q / p.n_kv, head_blocks = (group + 15) / 16;
   int entry, kvh, head, row, pos, first_pos, last_pos;     // head, row, pos: this column's query
@@ -102,7 +100,7 @@ attention_f32_kernel(F32Args p) {
   float m = -INFINITY, l = 0.f;                            // of this column; l: this lane's keys only, until the end
   const float slope = p.slopes ? p.slopes[head] : 0.f;
   if (begin + wave < end) ask(begin + wave);
-  for (int index = begin + wave; index < end; index += F32_WAVES) {
+  for (int index = begin + wave; index < end; index += WAVES) {
     const int block0 = first_key(index), key0 = block0 + 4 * g;
 #pragma unroll
     for (int i = 0; i < S; ++i) { k[i] = k_next[i]; v[i] = v_next[i]; }
@@ -120,7 +118,7 @@ attention_f32_kernel(F32Args p) {
         for (int i = 0; i < S; ++i) v[i][j] = used ? v[i][j] : 0.f;
       }
     }
-    ask(index + F32_WAVES);
+    ask(index + WAVES);
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;              // two chains of sums
 #pragma unroll
     for (int i = 0; i < S; ++i) {
@@ -195,23 +193,23 @@ attention_f32_kernel(F32Args p) {
   // Each lane keeps its column; the workgroup's sixteen groups of sixteen lanes take the coordinates in turn.
   float big = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < F32_WAVES; ++w) big = fmaxf(big, m_s[w][c]);
+  for (int w = 0; w < WAVES; ++w) big = fmaxf(big, m_s[w][c]);
   // (A sink joins the first part's softmax.)
   const bool with_sink = p.sinks && (!SINGLE || blockIdx.x == 0);
   if (with_sink) big = fmaxf(big, p.sinks[head]);
   const float base = big == -INFINITY ? 0.f : big;
-  float weight[F32_WAVES], total = with_sink ? expf(p.sinks[head] - base) : 0.f;
+  float weight[WAVES], total = with_sink ? expf(p.sinks[head] - base) : 0.f;
 #pragma unroll
-  for (int w = 0; w < F32_WAVES; ++w) { weight[w] = expf(m_s[w][c] - base); total += l_s[w][c] * weight[w]; }
+  for (int w = 0; w < WAVES; ++w) { weight[w] = expf(m_s[w][c] - base); total += l_s[w][c] * weight[w]; }
   if (!valid) return;
   const bool whole = !SINGLE || p.splits == 1;
   const size_t item = SINGLE ? ((size_t)blockIdx.z * p.n_q + head) * p.splits + blockIdx.x : 0;
   float* dst = whole ? p.out + ((size_t)row * p.n_q + head) * p.dv : p.part_o + item * p.dv;
   const float inv = whole ? 1.0f / total : 1.0f;
-  for (int i = threadIdx.x >> 4; i < p.dv; i += F32_WAVES * 4) {
+  for (int i = threadIdx.x >> 4; i < p.dv; i += WAVES * 4) {
     float o = 0.f;
 #pragma unroll
-    for (int w = 0; w < F32_WAVES; ++w) o += acc_s[w][i][c] * weight[w];
+    for (int w = 0; w < WAVES; ++w) o += acc_s[w][i][c] * weight[w];
     dst[i] = o * inv;
   }
   if (!whole && threadIdx.x < 16) { p.part_ml[2 * item] = big; p.part_ml[2 * item + 1] = total; }
@@ -262,9 +260,13 @@ extern "C" int ta_paged_attention_f32(const void* q, int q_stride, void* out, co
                         (float*)part_o, (float*)part_ml};
   const int blocks = ((d > dv ? d : dv) + 15) / 16;
   const dim3 many(n_tiles, n_q), few(splits, n_kv * ((n_q / n_kv + 15) / 16), n_single);
+  // Single tokens whose keys are not cut: eight waves while workgroups are few (up to 512 keys, 128 rows of head size 64, 300 keys
+  // 11.4 -> 10.4 us; 512 rows 19.3 -> 23.3, so not there) and two of them fit a unit's registers (up to 128 coordinates).
+  const bool wide = splits == 1 && blocks <= 8 && (long)few.y * n_single <= 256;
 #define GO(SS) do {                                                                                                  \
-    if (n_tiles > 0) attention_f32_kernel<SS, false><<<many, F32_WAVES * WAVE, 0, stream>>>(args);                   \
-    if (n_single > 0) attention_f32_kernel<SS, true><<<few, F32_WAVES * WAVE, 0, stream>>>(args);                    \
+    if (n_tiles > 0) attention_f32_kernel<SS, false, 4><<<many, 4 * WAVE, 0, stream>>>(args);                        \
+    if (n_single > 0 && wide) attention_f32_kernel<SS, true, (SS <= 8 ? 8 : 4)><<<few, (SS <= 8 ? 8 : 4) * WAVE, 0, stream>>>(args); \
+    else if (n_single > 0) attention_f32_kernel<SS, true, 4><<<few, 4 * WAVE, 0, stream>>>(args);                    \
   } while (0)
   if (blocks <= 1) GO(1); else if (blocks <= 2) GO(2); else if (blocks <= 4) GO(4); else if (blocks <= 6) GO(6);
   else if (blocks <= 8) GO(8); else if (blocks <= 12) GO(12); else GO(16);

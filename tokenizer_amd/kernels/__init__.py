@@ -1269,8 +1269,17 @@ class Ops:
         for reach in (window, chunk):
             max_keys = max_keys if reach is None else min(max_keys, reach + keep_first + 32)
         head_blocks = -(-(n_q // n_kv) // 16)
-        per_item = max(1, self.target_workgroups // max(1, single * n_kv * head_blocks))
+        rows_of_keys, size = max(1, single * n_kv * head_blocks), max(head_dim, value_dim)
+        # (Beyond 128 coordinates a workgroup fills a compute unit's registers: 64 rows of head size 256 and 300 keys, aimed at 1,024
+        # workgroups 28.8 us, at 256 of them 26.1; 256 rows 72 and 37.)
+        per_item = max(1, (self.target_workgroups if size <= 128 else self.target_workgroups // 4) // rows_of_keys)
         splits = max(1, min(per_item, -(-max_keys // self.min_split_keys_f32)))
+        # Up to 512 keys whole from 128 rows on, and up to 256 at head sizes to 64: the merge, 3.6 us, and the parts that short
+        # contexts leave empty cost more.  (Head size 64, 128 rows of 24 | 300 | 500 keys in parts 13.0 | 15.2 | 17.2 us, whole
+        # 6.4 | 10.4 | 14.5, the generic kernel 8.6 | 25.5 | 34; 16 rows 8.8 | 9.1 | 9.4, 6.3 | 10.1 | 13.1, 7.6 | 16.4 | 18.8: parts,
+        # at the price of contexts of up to some 40 keys.)
+        if size <= 128 and ((max_keys <= 512 and rows_of_keys >= 128) or (max_keys <= 256 and size <= 64)):
+            splits = 1
         part_o = part_ml = None
         if single and splits > 1:
             part_o = torch.empty((single, n_q, splits, value_dim), dtype=torch.float32, device=qkv.device)
