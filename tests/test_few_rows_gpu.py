@@ -73,6 +73,28 @@ def test_a_pick_that_weighs_nothing_adds_nothing(ops, gated, shared, weigh_input
     assert bool(torch.isfinite(got).all()) and torch.equal(got, run())
 
 
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("width", [896, 1536])
+def test_chosen_experts_are_the_same_in_every_call(ops, gated, width):
+    """More workgroups than the device holds at once: a sum read before it is there would differ from call to call."""
+    inner, experts, top, rows, halves = 3648, 8, 2, 4, 2 if gated else 1
+    first, second = rand_bf16((halves * experts * inner, width), 61) / 32, rand_bf16((width, experts * inner), 62) / 64
+    x, weights = rand_bf16((rows, width), 63), (0.2 + torch.rand(rows, top, generator=torch.Generator().manual_seed(64))).cuda()
+    chosen = torch.tensor([[5, 4], [4, 3], [5, 2], [2, 1]], dtype=torch.int32, device="cuda")
+    run = lambda: ops.experts_few(x, chosen, weights, experts, first, gated, inner, second).partial
+    got = run()
+    for _ in range(24):
+        assert torch.equal(run(), got)
+    # Rounded to bfloat16: the first product's results, and what the second is handed (2^-9 each).
+    for t in range(rows):
+        for k in range(top):
+            e = int(chosen[t, k])
+            each = (first[e * halves * inner:(e + 1) * halves * inner].double() @ x[t].double()).bfloat16().double()
+            act = plain.silu(each[:inner]) * each[inner:] if gated else each.clamp(min=0) ** 2
+            want = second[:, e * inner:(e + 1) * inner].double() @ (float(weights[t, k]) * act).bfloat16().double()
+            assert float((got[k, t] - want).abs().max()) <= 2e-2 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("width", [8, 520, 2048, 2056, 4096])
 @pytest.mark.parametrize("dim", [8, 16])
 @pytest.mark.parametrize("rows", [1, 256])
