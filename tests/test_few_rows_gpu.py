@@ -95,6 +95,27 @@ def test_chosen_experts_are_the_same_in_every_call(ops, gated, width):
             assert float((got[k, t] - want).abs().max()) <= 2e-2 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("experts,shared,taken", [(65535, 0, True), (65534, 8, True), (65533, 264, False), (65535, 8, False)])
+def test_as_many_experts_as_a_grid_has_places_for(ops, experts, shared, taken):
+    """The last experts of a full grid; where the shared one's parts have no place left, the call is handed back, not refused."""
+    width = inner = 8
+    total = experts * inner + shared
+    first = torch.randn((2 * total, width), device="cuda", dtype=torch.float32).to(torch.bfloat16)
+    second = torch.randn((width, total), device="cuda", dtype=torch.float32).to(torch.bfloat16)
+    x = rand_bf16((2, width), 55)
+    chosen = torch.tensor([[0, experts - 1], [experts - 2, 31]], dtype=torch.int32, device="cuda")
+    weights = torch.tensor([[0.75, 0.5], [1.25, 0.25]], device="cuda")
+    parts = ops.experts_few(x, chosen, weights, experts, first, True, inner, second, shared=shared)
+    assert (parts is not None) == taken
+    if not taken:
+        return
+    expert = lambda t, at, n: second[:, at:at + n].double().cpu() @ (
+        plain.silu(first[2 * at:2 * at + n].double().cpu() @ x[t].double().cpu()) * (first[2 * at + n:2 * at + 2 * n].double().cpu() @ x[t].double().cpu()))
+    want = torch.stack([sum(float(weights[t, k]) * expert(t, int(chosen[t, k]) * inner, inner) for k in range(2))
+                        + (expert(t, experts * inner, shared) if shared else 0) for t in range(2)])
+    assert float((parts.resolve().double().cpu() - want).abs().max()) <= 2e-2 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("width", [8, 520, 2048, 2056, 4096])
 @pytest.mark.parametrize("dim", [8, 16])
 @pytest.mark.parametrize("rows", [1, 256])

@@ -230,7 +230,7 @@ extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, c
                               hipStream_t stream) {
   if (n_rows <= 0) return 0;
   const long pairs = (long)n_rows * top;
-  if (top <= 0 || n_experts <= 0 || n_experts > 65000 || inner <= 0 || hidden <= 0 || (halves != 1 && halves != 2) ||
+  if (top <= 0 || n_experts <= 0 || n_experts > 65535 || inner <= 0 || hidden <= 0 || (halves != 1 && halves != 2) ||
       ldw < n_experts * inner + shared || x_stride < hidden || shared < 0 || (shared > 0 && (!act_shared || weigh_input)))
     return -1;
   if (pairs > EF_MAX_PAIRS || inner % 8 || hidden % 8 || ldw % 8 || x_stride % 8 || shared % 8 ||
@@ -238,6 +238,7 @@ extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, c
     return -2;
   const EfShared every = {shared, (const float*)shared_weights, (bf16_t*)act_shared, ta_experts_few_shared_parts(inner, shared),
                           shared > 0 ? shared_part(inner, shared) : 0};
+  if (n_experts + every.parts > 65535) return -2;            // (a grid's second dimension)
   const dim3 up(((inner > shared ? inner : shared) + 15) / 16, n_experts + (shared > 0)),
       down((hidden + 15) / 16, n_experts + every.parts);
 #define UP(NW, HH) experts_few_up_kernel<NW, HH><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
