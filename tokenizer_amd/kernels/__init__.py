@@ -1328,7 +1328,10 @@ class Ops:
             max_keys = min(max_keys, chunk + 32)
         head_blocks = -(-(n_q // n_kv) // 16)
         rows_of_keys = n_items * n_kv * head_blocks
-        # (Two parts a row would be the whole grid in one go; with three the compute units that got short rows take more.)
+        # (Three parts at least: two a row are the whole grid in one go; with three the compute units that got short rows take more.  In
+        # one, two and three, us: 800 rows of head size 64, spread up to 8,000 keys 189, 179, 166; all of 4,000 159, 157, 153; one of 4,000
+        # among ones of 300 52, 34, 26; 360 rows (one part falls out as two) 39 and 43, 73 and 75, 30 and 23; 720 rows of size 128, spread
+        # up to 4,000 153, 159, 151, all of that 253, 263, 267, one long 73, 47, 37.)
         per_split = max(3 if rows_of_keys < self.target_workgroups else 1, self.target_workgroups // max(1, rows_of_keys))
         split_keys = max(self.min_split_keys, -(-max_keys // per_split))
         if rows_of_keys >= self.target_workgroups or (2 * rows_of_keys >= self.target_workgroups and max_keys <= 1024):
