@@ -44,9 +44,9 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
                         const int* __restrict__ rows, const int* __restrict__ positions,
                         const int* __restrict__ entry_of_token, const int* __restrict__ block_table,
                         int table_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
-                        int n_q, int n_kv, int page_size, int window, float scale, int split_keys, int splits,
+                        int n_q, int n_kv, int page_size, int window, float scale, int split_keys, int splits, int deal,
                         int chunk, const float* __restrict__ slopes, const float* __restrict__ sinks,
-                        int keep_first, int kept_splits, int n_v, float softcap, int units_log2) {
+                        int keep_first, int kept_splits, int n_v, float softcap) {
   constexpr int KS = (D + 31) / 32;   // 32-wide steps over the head size for Q K^T
   constexpr int DB = D / 16;          // 16-row blocks of O^T
   HELD(q, q_stride, out, k_pages, vt_pages, rows, positions, entry_of_token, block_table, table_stride, part_o, part_ml,
@@ -64,10 +64,10 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   // count starts one further for every eight workgroups in front of it, and once more for every round of the units; an odd count
   // goes round by itself.  (16 rows of 16 kv heads of size 64, contexts spread up to 8,000, four parts, three draws: counted alike
   // in all rows 66, 66 and 51 us, from a hash of the row 66, 67 and 41, so 62, 63 and 41; 32 such rows, three parts, four draws:
-  // hashed 112 to 116, so 101 to 112.)
-  const uint32_t row = blockIdx.y + gridDim.y * blockIdx.z;
-  const int even = __builtin_ctz((uint32_t)splits | 8u);   // log2 of the greatest common divisor of the parts and eight
-  const uint32_t turn = even ? (row >> (3 - even)) + ((row * (uint32_t)splits) >> units_log2) : 0u;
+  // hashed 112 to 116, so 101 to 112.)  `deal` holds the two shifts and stands beside `splits`, with which it is fetched: worked out
+  // here they took a branch and a further fetch at the head of the kernel, 0.2 to 0.4 % of a decode step at batch 8.
+  const uint32_t row = blockIdx.y + n_kv * head_blocks * blockIdx.z;
+  const uint32_t turn = (row >> (deal & 255)) + ((row * (uint32_t)splits) >> (deal >> 8));
   const int split = (int)((blockIdx.x + turn) % (uint32_t)splits);
   const int kvh = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
   const int item = blockIdx.z;
@@ -424,13 +424,16 @@ static int launch_decode(const void* q, int q_stride, void* out, const void* k_p
                          float softcap, int tied, hipStream_t stream) {
   const int group = n_q / n_kv;
   dim3 grid(splits, n_kv * ((group + 15) / 16), n_items);
-  const int units_log2 = 31 - __builtin_clz((unsigned)compute_units());
+  // The shifts by which a row's first part moves on with the rows in front of it (31: it does not): with an even count, by the log2
+  // of eight over what it shares with eight, and by that of the compute units.
+  const int even = __builtin_ctz((unsigned)splits | 8u);
+  const int deal = even ? (3 - even) | (31 - __builtin_clz((unsigned)compute_units())) << 8 : 31 | 31 << 8;
   constexpr int NW = D > 128 ? 2 : 4, WIDE = D <= 64 ? 16 : D <= 128 ? 8 : 4;
 #define GO(WAVES, AHEAD, EE, TT) decode_attention_kernel<D, WAVES, AHEAD, EE, TT><<<grid, WAVES * WAVE, 0, stream>>>( \
       (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_pages, (const bf16_t*)vt_pages, (const int*)rows, \
       (const int*)positions, (const int*)entry_of_token, (const int*)block_table, table_stride, (float*)part_o, \
-      (float*)part_ml, n_q, n_kv, page_size, window, scale, split_keys, splits, chunk, (const float*)slopes, \
-      (const float*)sinks, keep_first, kept_splits, n_v, softcap, units_log2)
+      (float*)part_ml, n_q, n_kv, page_size, window, scale, split_keys, splits, deal, chunk, (const float*)slopes, \
+      (const float*)sinks, keep_first, kept_splits, n_v, softcap)
   const bool few = split_keys <= 32 * NW * 8;              // up to eight blocks a wave
   // Workgroups of sixteen (eight, four) waves where they are few and each has many keys: the keys are on their way at once, and
   // fewer parts do.  64 tokens, 2 kv heads, 1,000 keys, two parts and their merge: head size 64 12.3 us in nine parts of four
