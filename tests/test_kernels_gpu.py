@@ -1154,3 +1154,26 @@ def test_read_stream_reads_every_word_once(ops):
         data = torch.randint(-2 ** 31, 2 ** 31 - 1, (words,), dtype=torch.int32, device="cuda")
         parts = ops.read_stream(data, workgroups).cpu().numpy().view(np.uint32)
         assert int(np.bitwise_xor.reduce(parts)) == int(np.bitwise_xor.reduce(data.cpu().numpy().view(np.uint32))), words
+
+
+@pytest.mark.parametrize("lengths", [[1307, 641], [40, 3, 90]])
+@pytest.mark.parametrize("n", [16, 40])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_selective_scan_is_the_same_in_every_call(ops, lengths, n, dtype):
+    """In chunks and whole, many turns of sixteen tokens: a row handed from one wave to another before it is written would differ
+    from call to call."""
+    gen, channels, tokens = torch.Generator().manual_seed(n), 896, sum(lengths)
+    rand = lambda *shape: torch.randn(*shape, generator=gen)
+    x, low, rows = (rand(tokens, width).to(dtype).cuda() for width in (channels, 2 * n + 8, 2 * channels))
+    pre, rate, skip = rand(tokens, channels).cuda(), -(0.5 + rand(channels, n).abs()).cuda(), rand(channels).cuda()
+    as_ints = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")
+    cu_q = as_ints([sum(lengths[:i]) for i in range(len(lengths) + 1)])
+    results = []
+    for _ in range(40):
+        state, out = torch.zeros(len(lengths), channels * n + 4, device="cuda"), torch.empty((tokens, channels), dtype=dtype, device="cuda")
+        ops.selective_scan(x, pre, rate, low, 8, 8 + n, skip, rows, channels, state, cu_q, as_ints([0] * len(lengths)),
+                           as_ints(list(range(len(lengths)))), out, channels, n)
+        results.append((out, state))
+    assert bool(torch.isfinite(results[0][0]).all())
+    for out, state in results[1:]:
+        assert torch.equal(out, results[0][0]) and torch.equal(state, results[0][1])

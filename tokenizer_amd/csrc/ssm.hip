@@ -174,6 +174,9 @@ selective_scan_kernel(const T* __restrict__ x, int x_stride, const float* __rest
 #undef SS_XOR8
       const float gate = s_z[part][mine];
       s_out[part][mine] = fmaf(skip, s_x[part][mine], y) * (gate / (1.0f + __expf(-gate)));
+      // The next turn's barrier must find this written.  (The compiler waits for it in front of the barrier behind the loop and not
+      // in front of the one at the loop's head: now and then another wave wrote out the row before.)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   }
   if (MODE != SS_LOCAL) {
