@@ -69,11 +69,6 @@ __device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES], con
         for (int h = 0; h < HALVES; ++h)
           acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[q][h][s], xf[q][s], acc[h], 0, 0, 0);
   }
-  // A matrix instruction's result may be read eight wait states behind it at the earliest.  The compiler leaves them out in front of
-  // the stores to LDS that follow where a kernel has one matrix (HALVES 1 of the first product: the store is the second
-  // instruction behind the last sum, and with many workgroups some stored a sum that was not there yet), so they are here, twice over.
-#pragma unroll
-  for (int h = 0; h < HALVES; ++h) asm volatile("s_nop 7\n\ts_nop 7" : "+v"(acc[h]));
 }
 
 // x [n_rows, x_stride]; chosen int [n_rows * top], weights float [n_rows * top]; expert e's first matrix starts at
@@ -117,6 +112,10 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) acc[h] = (ef_floatx4){0.f, 0.f, 0.f, 0.f};
     ef_walk<NW, HALVES>(w_at, x_at, ok, hidden, g, wave, acc);
+    // A matrix instruction's result may be read eight wait states behind it at the earliest.  The compiler leaves them out in front
+    // of the stores below where there is one matrix (the store is the second instruction behind the last sum; with many
+    // workgroups some stored a sum that was not there yet), so they are here, twice over; with two matrices it has them.
+    if constexpr (HALVES == 1) asm volatile("s_nop 7\n\ts_nop 7" : "+v"(acc[0]));
 #pragma unroll
     for (int h = 0; h < HALVES; ++h)
 #pragma unroll
