@@ -194,6 +194,32 @@ def test_sorted_products_of_many_tiles_in_either_kernel(ops, bm, rows, monkeypat
         assert float((got.double() - want).abs().max()) <= 2e-6 * k ** 0.5 * float(want.abs().max())
 
 
+# The ring kernel's tiles: K of one step and of every number of steps past the first round of two, three or four buffers, with and
+# without half a step behind them; columns of one tile, one past it, no multiple of four.
+@pytest.mark.parametrize("bm,width", [(64, 64), (64, 128), (64, 256), (128, 128), (128, 256)])
+@pytest.mark.parametrize("k", [64, 96, 128, 192, 224, 256, 320, 416, 448])
+def test_sorted_products_of_every_ring(ops, bm, width, k, monkeypatch):
+    experts, tiles, ldw = 2, 3, k + 24
+    x = rand_bf16((tiles * bm, k + 8), k)
+    x[:, k:] = float("nan")                                   # columns behind K are not read, on either side
+    on_tiles = torch.tensor([1, -1, 0], dtype=torch.int32, device="cuda")
+    row_of = torch.randperm(tiles * bm, generator=torch.Generator().manual_seed(k)).to(torch.int32).cuda()
+    row_of[5] = -1
+    for n_out in (width, width + 1, 90):
+        joined = torch.full((experts * n_out, ldw), float("nan"), dtype=torch.bfloat16, device="cuda")
+        joined[:, :k] = rand_bf16((experts * n_out, k), n_out)
+        monkeypatch.setattr(ops, "grouped_wide", width)
+        for dtype in (torch.float32, torch.bfloat16):
+            got = ops.grouped_linear(x, row_of, on_tiles, bm, joined, n_out * ldw, n_out, k, dtype)
+            for tile, expert in ((0, 1), (2, 0)):
+                at = torch.arange(tile * bm, tile * bm + bm, device="cuda")
+                at = at[row_of[at] >= 0]
+                want = x[row_of[at].long(), :k].double() @ joined[expert * n_out:(expert + 1) * n_out, :k].double().t()
+                # Float sums of K exact products: at most K / 2 roundings of 2^-24 of the largest partial sum, fewer in practice.
+                error = float((got[at].double() - want).abs().max() / want.abs().max())
+                assert error <= (2e-6 * k ** 0.5 if dtype == torch.float32 else 2 ** -8), (n_out, tile)
+
+
 @pytest.mark.parametrize("bm", [64, 128])
 def test_sorted_products_pass_over_tiles_without_slots_anywhere_in_the_list(ops, bm, monkeypatch):
     k, n_out, experts = 64, 256, 3

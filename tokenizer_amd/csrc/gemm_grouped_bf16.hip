@@ -3,7 +3,7 @@
 // (v_mfma_f32_32x32x16_bf16), staged through LDS as in gemm_bf16.hip; and the two small kernels around them: the one
 // that sorts a step's (token, chosen expert) pairs into such tiles, and the one that adds a token's experts up.
 #include "common.h"
-#include <type_traits>
+#include "tile_ring.h"
 
 typedef __bf16 gg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float gg_floatx16 __attribute__((ext_vector_type(16)));
@@ -170,27 +170,21 @@ grouped_gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
     }
 }
 
-// The same for tiles of BM slots and 256 columns, K in steps of 32 (a multiple of 32 here).  A wave owns 64 columns and all the
-// slots.  Three steps' rows are on their way to registers, the next step's lie in the other of two buffers in LDS, whose
-// rows of 64 bytes keep their four pieces XOR-swizzled by the row (no bank is asked twice by the eight lanes that a read or
-// a write serves at a time); the fragments of the next two blocks of slots are read while two are multiplied.
-// Rounds of three steps run without a branch, so that the compiler counts the loads under way and waits for the oldest alone.
+// The same for tiles of BM slots and BN columns with the inner loop of tile_ring.h (K a multiple of 32, from 64 on).
 // Workgroups run over the tiles up to the last that has slots, in groups of sixteen tiles times all columns; the chiplets (every eighth
 // workgroup) get equal runs of that order, so what is under way on one chiplet at a time are sixteen tiles of slots times a few
 // strips of columns, and its L2 serves an operand's row several times for one trip from memory.
-// Bound by LDS and the vector memory pipe together (12 KB of fragments and 6 KB of rows a wave for 512 clocks of matrix work).
-// (2,048 tokens, two of eight experts of 9,472 on a width of 3,584: both products 958 + 482 us in the kernel above, 739 + 394
-// here, 750 TFLOP/s.  The weights' fragments straight from memory, past LDS: 885 + 440, since neighbouring lanes then name
-// different rows and the pipe takes such loads lane by lane.)
-template <int BM, typename OutT, int AHEAD = 3>
-__global__ void __launch_bounds__(256, 2)
-grouped_gemm_wide_kernel(const bf16_t* __restrict__ A, int lda, const int* __restrict__ row_of,
+// Bound by the loads' way into LDS (128 x 256: 48 KB a step of 1,024 clocks of matrix work).  36 tiles of 128 slots over 3,584 x 18,944
+// and 9,472 x 3,584: 679 + 327 us, 921 and 955 TFLOP/s; 808 + 402 with rows that went through registers on their way to LDS (256 columns,
+// steps of 32), 1,094 + 500 in the kernel above.
+template <int BM, int BN, int STAGES, int WN_WAVES, typename OutT>
+__global__ void __launch_bounds__(128 * WN_WAVES)
+grouped_gemm_ring_kernel(const bf16_t* __restrict__ A, int lda, const int* __restrict__ row_of,
                          const int* __restrict__ tile_expert, int n_tiles, const bf16_t* __restrict__ W, long expert_stride,
                          int ldw, OutT* __restrict__ C, int ldc, int N, int K) {
-  constexpr int BN = 256, BK = 32, GROUP = 16, PA = BM / 64, BLOCKS = BM / 16;
-  __shared__ __attribute__((aligned(16))) uint16_t a_s[2][BM * BK];
-  __shared__ __attribute__((aligned(16))) uint16_t w_s[2][BN * BK];
-  const int tid = threadIdx.x, lane = tid & 63, wave = wave_index(), r = lane & 15, g = lane >> 4;
+  typedef RingTile<BM, BN, STAGES, 2, WN_WAVES> Ring;
+  constexpr int GROUP = 16;
+  const int lane = threadIdx.x & 63, wave = wave_index();
   // The list up to its last tile with slots.
   int used = 0;
   for (int base = 0; base < n_tiles; base += WAVE) {
@@ -205,92 +199,24 @@ grouped_gemm_wide_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
   const int tile = first + inside % high, m0 = tile * BM, n0 = inside / high * BN;
   const int expert = scalar_int(tile_expert + tile);
   if (expert < 0) return;                                   // (a tile without slots among the others)
-  const bf16_t* We = W + (size_t)expert * expert_stride;
-  // A thread brings pieces of sixteen bytes of rows tid / 4, 64 further, ...: four neighbours a row's 64 bytes.  Places are
-  // 32-bit offsets from a pointer that is the same for the workgroup and moves along K.
-  uint32_t a_at[PA], w_at[4];
+  uint32_t a_at[Ring::LA], w_at[Ring::LB];
 #pragma unroll
-  for (int i = 0; i < PA; ++i) {
-    const int slot = m0 + (tid >> 2) + 64 * i;
-    a_at[i] = ((uint32_t)(row_of ? max(row_of[slot], 0) : slot) * lda + (tid & 3) * 8) * 2;
+  for (int i = 0; i < Ring::LA; ++i) {
+    const int slot = m0 + Ring::load_row(wave, lane, Ring::LA, i);
+    a_at[i] = (uint32_t)(row_of ? max(row_of[slot], 0) : slot) * lda * 2 + Ring::piece_bytes(lane);
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) w_at[j] = ((uint32_t)min(n0 + (tid >> 2) + 64 * j, N - 1) * ldw + (tid & 3) * 8) * 2;
-  gg_floatx4 acc[BLOCKS][4];
+  for (int i = 0; i < Ring::LB; ++i)
+    w_at[i] = (uint32_t)min(n0 + Ring::load_row(wave, lane, Ring::LB, i), N - 1) * ldw * 2 + Ring::piece_bytes(lane);
+  ring_floatx4 acc[Ring::MI][Ring::NI];
+  Ring::run(A, a_at, W + (size_t)expert * expert_stride, w_at, K / 64, (K & 32) != 0, acc);
+  const int r = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int i = 0; i < BLOCKS; ++i)
+  for (int i = 0; i < Ring::MI; ++i) {
+    OutT* row = C + (size_t)(m0 + wave / WN_WAVES * Ring::WM + 16 * i + r) * ldc;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = gg_floatx4{0.f, 0.f, 0.f, 0.f};
-  word4 a_reg[AHEAD][PA], w_reg[AHEAD][4];
-  const int steps = K / BK;
-  typedef const char __attribute__((address_space(1)))* memory;
-  typedef const word4 __attribute__((address_space(1)))* pieces;
-  auto fetch = [&](int step, word4 (&a_now)[PA], word4 (&w_now)[4]) {
-    // (Past the last step it is asked for again: a valid place, never used.)
-    const size_t along = (size_t)min(step, steps - 1) * (2 * BK);
-    memory a_base = (memory)(uintptr_t)A + along, w_base = (memory)(uintptr_t)We + along;
-    asm("" : "+s"(a_base), "+s"(w_base));
-#pragma unroll
-    for (int i = 0; i < PA; ++i) a_now[i] = *(pieces)(a_base + a_at[i]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) w_now[j] = *(pieces)(w_base + w_at[j]);
-  };
-  const int put_at = (tid >> 2) * BK + ((tid & 3) ^ ((tid >> 3) & 3)) * 8;         // (rows 64 apart are swizzled alike)
-  auto stash = [&](int buf, const word4 (&a_now)[PA], const word4 (&w_now)[4]) {
-#pragma unroll
-    for (int i = 0; i < PA; ++i) *reinterpret_cast<word4*>(a_s[buf] + put_at + 64 * BK * i) = a_now[i];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<word4*>(w_s[buf] + put_at + 64 * BK * j) = w_now[j];
-  };
-#pragma unroll
-  for (int j = 0; j < AHEAD; ++j) fetch(j, a_reg[j], w_reg[j]);
-  stash(0, a_reg[0], w_reg[0]);
-  __syncthreads();
-  int buf = 0;
-  const int get_at = r * BK + (g ^ ((r >> 1) & 3)) * 8;
-  auto one = [&](int step, auto which) {
-    constexpr int j = decltype(which)::value, next = (j + 1) % AHEAD;
-    fetch(step + AHEAD, a_reg[j], w_reg[j]);
-    __builtin_amdgcn_sched_barrier(0);
-    stash(buf ^ 1, a_reg[next], w_reg[next]);                // (its readers passed the barrier of the step before)
-    gg_bf16x8 wf[4], af[2][2];
-    auto read = [&](int pair, gg_bf16x8 (&now)[2]) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        now[i] = *reinterpret_cast<const gg_bf16x8*>(a_s[buf] + (pair * 2 + i) * 16 * BK + get_at);
-    };
-#pragma unroll
-    for (int n = 0; n < 4; ++n) wf[n] = *reinterpret_cast<const gg_bf16x8*>(w_s[buf] + (wave * 64 + n * 16) * BK + get_at);
-    read(0, af[0]);
-#pragma unroll
-    for (int pair = 0; pair < BLOCKS / 2; ++pair) {
-      if (pair + 1 < BLOCKS / 2) read(pair + 1, af[(pair + 1) & 1]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-          acc[pair * 2 + i][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[n], af[pair & 1][i], acc[pair * 2 + i][n], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __syncthreads();
-    buf ^= 1;
-  };
-  static_assert(AHEAD == 3);
-  int step = 0;
-  for (; step + AHEAD <= steps; step += AHEAD) {
-    one(step, std::integral_constant<int, 0>{});
-    one(step + 1, std::integral_constant<int, 1>{});
-    one(step + 2, std::integral_constant<int, 2>{});
-  }
-  if (step < steps) one(step, std::integral_constant<int, 0>{});
-  if (step + 1 < steps) one(step + 1, std::integral_constant<int, 1>{});
-  // Weight rows are the instruction's rows: a lane holds columns 4 g .. 4 g + 3 of slot r of each block of sixteen.
-#pragma unroll
-  for (int i = 0; i < BLOCKS; ++i) {
-    OutT* row = C + (size_t)(m0 + 16 * i + r) * ldc;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + wave * 64 + 16 * j + 4 * g;
+    for (int j = 0; j < Ring::NI; ++j) {
+      const int n = n0 + wave % WN_WAVES * Ring::WN + 16 * j + 4 * g;
       if (n + 3 < N && (ldc & 3) == 0) gg_store4(row + n, acc[i][j]);
       else
 #pragma unroll
@@ -332,8 +258,9 @@ extern "C" int ta_expert_slots(const void* chosen, int n_entries, int top, int n
 }
 
 // bm: 64 or 128 (the tile height the slots were made for).  C has n_tiles * bm rows.  expected: about how many of the tiles will
-// have slots (the launch's sizes do not depend on it).  rows: how many A has.  choice: 1 = the wide kernel wherever it can, -1 = never,
-// 0 = where it is expected to be the faster one.
+// have slots (it only goes into the choice of kernel).  rows: how many A has.  choice: 0 = the expected fastest, -1 = the general kernel,
+// 64, 128 or 256 = the ring kernel with so many columns a tile wherever it can (64 columns: tiles of 64 slots; 128 in their place at
+// 128), 1 = with 256.
 extern "C" int ta_grouped_gemm_bf16(const void* A, int rows, int lda, const void* row_of, const void* tile_expert, int n_tiles, int bm,
                                     const void* W, long expert_stride, int ldw, void* C, int ldc, int N, int K,
                                     int out_dtype, int expected, int choice, hipStream_t stream) {
@@ -343,23 +270,33 @@ extern "C" int ta_grouped_gemm_bf16(const void* A, int rows, int lda, const void
 #define GO(BMV, BNV, BKV, TT)                                                                                          \
   grouped_gemm_bf16_kernel<BMV, BNV, BKV, TT><<<dim3((N + BNV - 1) / BNV, n_tiles), 256, 0, stream>>>(                 \
       (const bf16_t*)A, lda, (const int*)row_of, (const int*)tile_expert, (const bf16_t*)W, expert_stride, ldw, (TT*)C, ldc, N, K)
-#define WIDE(BMV, TT) grouped_gemm_wide_kernel<BMV, TT><<<blocks, 256, 0, stream>>>((const bf16_t*)A, lda, (const int*)row_of, \
-    (const int*)tile_expert, n_tiles, (const bf16_t*)W, expert_stride, ldw, (TT*)C, ldc, N, K)
-  // Which kernel: by the rounds of workgroups that each needs over the compute units, a round of wide tiles as long as 1.65 of
-  // 128 x 128 ones or 3.15 of 64 x 64 ones (for twice and four times the work).  Measured at 128 slots a tile, us, this | the wide
-  // one: 36 tiles x 18,944 columns over 3,584 958 | 739, 3,584 columns over 9,472 482 | 394, 8 tiles of those 178 | 207; 36 tiles x
-  // 4,480 columns over 1,536 114 | 100, 18 tiles 67 | 71; 36 tiles x 896 columns over 3,648 70 | 72.  At 64: 68 tiles x 18,944
-  // columns over 3,584 1,276 | 1,018, 24 480 | 434; 24 tiles x 3,584 columns over 9,472 243 | 298.
-  const int units = compute_units(), strips = (N + 255) / 256, blocks = (strips * n_tiles + 7) / 8 * 8;
-  auto rounds = [&](int width) { return (int)(((long)((N + width - 1) / width) * expected + units - 1) / units); };
-  const bool wide = K % 32 == 0 && (long)(N - 1) * ldw + K < (1l << 31) && (long)rows * lda < (1l << 31) &&
-                    (choice > 0 || (choice == 0 && rounds(256) * (bm == 128 ? 1.65 : 3.15) < rounds(bm)));
-  if (wide) {
-    if (bm == 128) { if (out_dtype == DT_F32) WIDE(128, float); else WIDE(128, bf16_t); }
-    else if (out_dtype == DT_F32) WIDE(64, float); else WIDE(64, bf16_t);
-  } else if (bm == 128) { if (out_dtype == DT_F32) GO(128, 128, 32, float); else GO(128, 128, 32, bf16_t); }
-  else if (out_dtype == DT_F32) GO(64, 64, 64, float); else GO(64, 64, 64, bf16_t);
-#undef WIDE
+#define RING(BMV, BNV, ST, WAVES, TT) grouped_gemm_ring_kernel<BMV, BNV, ST, WAVES, TT><<<blocks, 128 * WAVES, 0, stream>>>( \
+    (const bf16_t*)A, lda, (const int*)row_of, (const int*)tile_expert, n_tiles, (const bf16_t*)W, expert_stride, ldw, (TT*)C, ldc, N, K)
+  // Which width: 64 columns (tiles of 64 slots) where even those give no compute unit a second workgroup; else 256 where their
+  // rounds over the units, each 1.6 times as long, are fewer than those of 128.  Measured, us, 64 | 128 | 256 columns (and the general
+  // kernel).  64 slots a tile: 12 tiles x 896 columns over 3,648 23 | 32 | 50 (31), 24 tiles 37 | 31 | 47 (42), 40 tiles 48 | 45 | 47 (62);
+  // 12 tiles x 3,648 columns over 896 20 | 20 | 19 (20); 24 tiles x 3,584 columns over 9,472 261 | 215 | 243 (250), 68 tiles x 18,944
+  // columns over 3,584 1,178 | 955 | 908 (1,340).  128 slots, 128 | 256 columns: 36 tiles x 18,944 over 3,584 795 | 679 (1,129), 36 x
+  // 3,584 over 9,472 395 | 327 (502), 8 such tiles 132 | 171 (181); 36 x 896 over 3,648 42 | 58 (73); 18 x 4,480 over 1,536 61 | 62 (68).
+  // The general kernel is left with a K that is no multiple of 32, one of 32, and matrices past 32-bit places.
+  const bool ring = choice >= 0 && K % 32 == 0 && K >= 64 && (long)(N - 1) * ldw + K < (1l << 31) && (long)rows * lda < (1l << 31);
+  const int units = compute_units();
+  auto workgroups = [&](int width) { return (long)((N + width - 1) / width) * expected; };
+  auto rounds = [&](int width) { return (double)((workgroups(width) + units - 1) / units); };
+  const int width = choice > 0 ? (choice == 1 ? 256 : choice) : bm == 64 && workgroups(64) <= units ? 64 : rounds(256) * 1.6 < rounds(128) ? 256 : 128;
+  if (width != 64 && width != 128 && width != 256) return -1;
+  const int blocks = ((N + width - 1) / width * n_tiles + 7) / 8 * 8;
+  const bool f32 = out_dtype == DT_F32;
+  if (ring && bm == 128) {
+    if (width == 256) { if (f32) RING(128, 256, 3, 4, float); else RING(128, 256, 3, 4, bf16_t); }
+    else if (f32) RING(128, 128, 4, 4, float); else RING(128, 128, 4, 4, bf16_t);
+  } else if (ring) {
+    if (width == 256) { if (f32) RING(64, 256, 4, 4, float); else RING(64, 256, 4, 4, bf16_t); }
+    else if (width == 128) { if (f32) RING(64, 128, 3, 4, float); else RING(64, 128, 3, 4, bf16_t); }
+    else if (f32) RING(64, 64, 4, 2, float); else RING(64, 64, 4, 2, bf16_t);
+  } else if (bm == 128) { if (f32) GO(128, 128, 32, float); else GO(128, 128, 32, bf16_t); }
+  else if (f32) GO(64, 64, 64, float); else GO(64, 64, 64, bf16_t);
+#undef RING
 #undef GO
   return LAUNCH_STATUS();
 }

@@ -923,8 +923,8 @@ class Ops:
 
     # Routed feed-forwards over sorted tokens (bfloat16): tiles of `bm` slots that belong to one expert each.
     GROUPED_EXPERTS = 256
-    grouped_wide = 0          # the kernel with tiles of 256 columns: 1 = wherever it can (K in steps of 32), -1 = never, 0 = where
-    #                           the launcher expects it to be the faster one
+    grouped_wide = 0          # columns a tile: 64 (with tiles of 64 slots), 128 or 256 (or 1) = the ring kernel of that width wherever it
+    #                           can (K in steps of 32), -1 = the general kernel, 0 = what the launcher expects to be the fastest
 
     @staticmethod
     def grouped_tiles(n_entries: int, n_experts: int, bm: int) -> int:
