@@ -1,0 +1,130 @@
+"""Products of many rows in the ring kernel, tile by tile, against the same products in 64 bits."""
+import ctypes
+
+import pytest
+import torch
+
+from tokenizer_amd.kernels import PendingSum, _ptr, get_ops
+
+pytestmark = pytest.mark.gpu
+TILES = [(64, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 192), (256, 256)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    return get_ops()
+
+
+def rand(shape, seed, spread=1.0):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(shape, generator=gen, device="cuda") * spread).to(torch.bfloat16)
+
+
+def strided(rows, k, lda, seed):
+    x = torch.full((rows, lda), float("nan"), dtype=torch.bfloat16, device="cuda")      # columns behind K are not read
+    x[:, :k] = rand((rows, k), seed)
+    return x[:, :k]
+
+
+# Float sums of K exact products, of which each rounding takes 2^-24 of a partial sum: 2e-6 sqrt(K) of the largest result is some
+# eight times what is seen; a result rounded to bfloat16 is within 2^-8 of its own size.
+def close(got, want, k, rounded):
+    bound = 2e-6 * k ** 0.5 * float(want.abs().max()) + (2.0 ** -8 * want.abs() if rounded else 0.0)
+    return bool(((got.double() - want).abs() <= bound).all())
+
+
+# Rows and columns of one tile, one past it and a remainder; K of one step, of every number of steps past the buffers, of half a step more.
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("k", [64, 96, 192, 320, 352, 448])
+def test_plain_products_of_every_tile(ops, tile, k):
+    bm, bn = TILES[tile]
+    for m, n in ((bm, bn), (bm + 1, bn + 4), (65, 100)):
+        x, w = strided(m, k, k + 40, k + m), rand((n, k), k + n, 0.1)
+        bias = torch.randn(n, device="cuda")
+        want = x.double() @ w.double().t() + bias.double()
+        for dtype, code in ((torch.float32, 0), (torch.bfloat16, 1)):
+            out = torch.full((m, n + 12), float("nan"), dtype=dtype, device="cuda")
+            assert ops.lib.ta_gemm_ring(_ptr(x), _ptr(w), _ptr(bias), _ptr(out), None, m, n, k, k + 40, n + 12, 1, code, tile, ops._stream()) == 0
+            assert close(out[:, :n], want, k, dtype == torch.bfloat16) and bool(out[:, n:].isnan().all())
+
+
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("k,parts", [(576, 3), (1056, 4), (2080, 7), (544, 5)])     # (the last: a part of half a step)
+def test_products_in_parts_of_every_tile(ops, tile, k, parts):
+    m, n = TILES[tile][0] + 3, TILES[tile][1] + 8
+    x, w, bias = rand((m, k), 1), rand((n, k), 2, 0.1), torch.randn(n, device="cuda")
+    want = x.double() @ w.double().t()
+    partial = torch.full((parts, m, n), float("nan"), device="cuda")
+    assert ops.lib.ta_gemm_ring(_ptr(x), _ptr(w), None, None, _ptr(partial), m, n, k, k, n, parts, 1, tile, ops._stream()) == 0
+    assert close(partial.double().sum(0), want, k, False)
+    out = torch.empty((m, n), device="cuda")
+    assert ops.lib.ta_gemm_ring(_ptr(x), _ptr(w), _ptr(bias), _ptr(out), _ptr(partial), m, n, k, k, n, parts, 0, tile, ops._stream()) == 0
+    assert close(out, want + bias.double(), k, False)
+
+
+@pytest.mark.parametrize("tile", range(1, len(TILES)))
+@pytest.mark.parametrize("act", [None, "gelu_tanh", "relu", (1.702, 2.0, 1.0)])
+def test_gated_products_of_every_tile(ops, tile, act):
+    bm, bn = TILES[tile]
+    numbers = act if isinstance(act, tuple) else (0.0, 0.0, 0.0)
+    code = 4 if isinstance(act, tuple) else {None: 1, "gelu_tanh": 2, "relu": 3}[act]
+    for m, inner, k in ((bm, bn // 2, 64), (bm + 1, bn // 2 + 4, 352), (70, 52, 224)):
+        x, w = strided(m, k, k + 8, m), rand((2 * inner, k), inner, 0.2)
+        gate, up = (x.double() @ half.double().t() for half in (w[:inner], w[inner:]))
+        if act is None:
+            want = gate * torch.sigmoid(gate) * up
+        elif act == "gelu_tanh":
+            want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+        elif act == "relu":
+            want = torch.relu(gate) * up
+        else:
+            g = gate.clamp(max=act[1])
+            want = g * torch.sigmoid(act[0] * g) * (up.clamp(-act[1], act[1]) + act[2])
+        out = torch.full((m, inner), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert ops.lib.ta_gemm_ring_gated(_ptr(x), _ptr(w), _ptr(out), m, inner, k, k + 8, code, *map(ctypes.c_float, numbers), tile,
+                                          ops._stream()) == 0
+        # The activation in float: 2^-20 of the product of its factors, beside the rounding of the result.
+        slack = 2.0 ** -20 * float(gate.abs().max() * up.abs().max())
+        assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 4e-5 * float(want.abs().max()) + slack).all())
+
+
+# What goes to the ring kernel comes back as the general kernels give it: rows and sizes on either side of its lines, an activation of
+# each kind, infinities and NaN in a row, which stay in that row.
+@pytest.mark.parametrize("m,n,k", [(65, 96, 64), (300, 128, 2080), (1025, 64, 256), (70, 4100, 512), (33, 96, 64), (257, 8, 96)])
+def test_the_choice_of_kernel_does_not_change_the_product(ops, m, n, k, monkeypatch):
+    x, w, bias = rand((m, k), m), rand((n, k), n, 0.1), torch.randn(n, device="cuda")
+    x[1, 3], x[2, 5] = float("inf"), float("nan")
+    for act in (None, "gelu_tanh", "relu", (1.702, 2.0, 1.0)):
+        got = ops.linear_silu_gate(x, w, act=act)
+        with monkeypatch.context() as only:
+            only.setattr(ops, "use_ring", False)
+            want = ops.linear_silu_gate(x, w, act=act)
+        rest = torch.arange(m, device="cuda") > 2
+        # (There the sums are rounded to bfloat16 before the activation: 2^-8 of either factor.)
+        assert float((got[rest].double() - want[rest].double()).abs().max()) <= 4 * 2.0 ** -8 * float(want[rest].double().abs().max())
+        assert torch.equal(got[1:3].isfinite(), want[1:3].isfinite())
+    for pending in (False, True):
+        for dtype in (torch.bfloat16, torch.float32):
+            got = ops.linear(x, w, bias, out_dtype=dtype, pending=pending)
+            got = got.resolve() if isinstance(got, PendingSum) else got
+            with monkeypatch.context() as only:
+                only.setattr(ops, "use_ring", False)
+                want = ops.linear(x, w, bias, out_dtype=dtype)
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+            fine = want.isfinite()
+            limit = 2.0 ** -7 if dtype == torch.bfloat16 else 2e-6 * k ** 0.5
+            assert float((got[fine].double() - want[fine].double()).abs().max()) <= limit * float(want[fine].double().abs().max())
+
+
+def test_operands_that_are_refused(ops):
+    x, w, out = rand((80, 96), 1), rand((64, 96), 2), torch.empty((80, 64), dtype=torch.bfloat16, device="cuda")
+    call = lambda m, n, k, lda, ldc, parts=1, partial=None, xp=None: ops.lib.ta_gemm_ring(
+        xp or _ptr(x), _ptr(w), None, _ptr(out), partial, m, n, k, lda, ldc, parts, 1, -1, ops._stream())
+    assert call(80, 64, 32, 96, 64) == -2                     # less than a step of K
+    assert call(80, 64, 80, 96, 64) == -2                     # no whole half step
+    assert call(80, 62, 96, 96, 64) == -2                     # columns no multiple of four
+    assert call(80, 64, 96, 92, 64) == -2                     # rows not sixteen bytes apart
+    assert call(80, 64, 96, 96, 64, xp=ctypes.c_void_p(x.data_ptr() + 2)) == -2
+    assert call(80, 64, 96, 96, 64, parts=2) == -1            # parts without a place
+    assert call(80, 64, 96, 96, 64, parts=3, partial=_ptr(out)) == -1      # more parts than steps
+    assert call(0, 64, 96, 96, 64) == 0

@@ -1,0 +1,210 @@
+// Products of many bfloat16 rows with the inner loop of tile_ring.h, for what the vendor's library does not do or does slowly:
+// C = A W^T in parts of K for the norm that follows to add (few tiles, long K), and the gated product
+// act(A Wg^T) * (A Wu^T) in one kernel, gate and up sums meeting in a lane's registers.
+#include "common.h"
+#include "splitk_reduce.h"
+#include "tile_ring.h"
+
+enum { RING_PLAIN = 0, RING_SILU = 1, RING_GELU = 2, RING_RELU = 3, RING_CAPPED = 4 };
+
+template <int GATE>
+__device__ __forceinline__ float ring_gate(float z, float u, float alpha, float limit, float shift) {
+  if constexpr (GATE == RING_SILU) return z / (1.0f + __expf(-z)) * u;
+  else if constexpr (GATE == RING_RELU) return fmaxf(z, 0.f) * u;
+  else if constexpr (GATE == RING_CAPPED) {
+    const float g = fminf(z, limit);
+    return g / (1.0f + __expf(-alpha * g)) * (fminf(fmaxf(u, -limit), limit) + shift);
+  } else {
+    const float t = 0.7978845608028654f * (z + 0.044715f * z * z * z);
+    return 0.5f * z * (2.0f - 2.0f / (1.0f + __expf(2.0f * t))) * u;        // 1 + tanh(t)
+  }
+}
+
+__device__ __forceinline__ void ring_store4(float* p, const ring_floatx4& v) { *reinterpret_cast<ring_floatx4*>(p) = v; }
+__device__ __forceinline__ void ring_store4(bf16_t* p, const ring_floatx4& v) {
+  *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16),
+                                            (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16));
+}
+
+// C[M, N] = A[M, K] W[N, K]^T (+ bias), N a multiple of 4, K of 32.  `splits` parts of K, `k_chunk` (a multiple of 64) each: part s goes to
+// slab s of C (float [splits, M, N], ldc = N, no bias).  GATE: W holds `N` gate rows, then N up rows; C[M, N] is the gated result.  Weight
+// rows of a gated tile lie in LDS as sixteen gate rows, the sixteen up rows of the same columns, and so on.
+// Workgroups in groups of sixteen tiles of rows times all columns, equal runs of that order to the chiplets (every eighth workgroup).
+template <class Ring, int BM, int BN, int GATE, typename OutT>
+__global__ void __launch_bounds__(Ring::THREADS)
+gemm_ring_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ bias, OutT* __restrict__ C,
+                 int M, int N, int K, int lda, int ldc, int splits, int k_chunk, float alpha, float limit, float shift) {
+  constexpr int GROUP = 16, COLUMNS = GATE ? BN / 2 : BN;
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int tall = (M + BM - 1) / BM, strips = (N + COLUMNS - 1) / COLUMNS, total = tall * strips * splits, per_chiplet = (total + 7) / 8;
+  const int turn = (int)(blockIdx.x >> 3), place = (int)(blockIdx.x & 7) * per_chiplet + turn;
+  if (turn >= per_chiplet || place >= total) return;
+  const int split = place / (tall * strips), at = place - split * tall * strips;
+  const int first = at / (GROUP * strips) * GROUP, high = min(GROUP, tall - first), inside = at - first * strips;
+  const int m0 = (first + inside % high) * BM, n0 = inside / high * COLUMNS;
+  uint32_t a_at[Ring::LA], w_at[Ring::LB];
+#pragma unroll
+  for (int i = 0; i < Ring::LA; ++i)
+    a_at[i] = (uint32_t)min(m0 + Ring::load_row(wave, lane, Ring::LA, i), M - 1) * lda * 2 + Ring::piece_bytes(lane);
+#pragma unroll
+  for (int i = 0; i < Ring::LB; ++i) {
+    const int row = Ring::load_row(wave, lane, Ring::LB, i);
+    const int n = GATE ? min(n0 + (row >> 5) * 16 + (row & 15), N - 1) + (row & 16 ? N : 0) : min(n0 + row, N - 1);
+    w_at[i] = (uint32_t)n * K * 2 + Ring::piece_bytes(lane);
+  }
+  const int k_begin = split * k_chunk, k_here = min(K - k_begin, k_chunk);
+  ring_floatx4 acc[Ring::MI][Ring::NI];
+  Ring::run(A + k_begin, a_at, W + k_begin, w_at, k_here / 64, (k_here & 32) != 0, acc);
+  const int r = lane & 15, g = lane >> 4, wm = wave / Ring::ACROSS, wn = wave % Ring::ACROSS;
+  C += (size_t)split * M * ldc;
+#pragma unroll
+  for (int i = 0; i < Ring::MI; ++i) {
+    const int m = m0 + wm * Ring::WM + 16 * i + r;
+    if (m >= M) continue;
+    OutT* row = C + (size_t)m * ldc;
+    if constexpr (GATE != RING_PLAIN) {
+#pragma unroll
+      for (int j = 0; j < Ring::NI; j += 2) {
+        const int n = n0 + wn * (Ring::WN / 2) + 8 * j + 4 * g;
+        if (n >= N) continue;
+        ring_floatx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = ring_gate<GATE>(acc[i][j][e], acc[i][j + 1][e], alpha, limit, shift);
+        ring_store4(row + n, v);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < Ring::NI; ++j) {
+        const int n = n0 + wn * Ring::WN + 16 * j + 4 * g;
+        if (n >= N) continue;
+        ring_floatx4 v = acc[i][j];
+        if (bias)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += bias[n + e];
+        ring_store4(row + n, v);
+      }
+    }
+  }
+}
+
+// The tiles there are, and what a product costs with each, in microseconds on a device of 256 compute units:
+//   start + rounds * (fixed + steps * step), rounds of workgroups over the compute units, steps of 64 of K,
+// but no less than the weights' trip from memory, and on top the result's (parts are written, and read by whoever adds them).
+// Fitted to 5,700 timed products (17 to 4,096 rows, the Qwen2.5 models' matrices at 0.5B, 1.5B and 7B sizes, one to ten parts, plain and
+// gated, weights from memory); the tile and parts with the lowest cost are on average 3 % slower than the fastest of all, 30 % at worst
+// (long K, fewer than 100 rows).
+struct RingShape { int bm, bn; double start, fixed, step; };
+static const RingShape RING_SHAPES[] = {
+  {64, 64, 2.06, 0.58, 0.232}, {64, 128, 2.37, 0.62, 0.376}, {64, 256, 0.99, 3.08, 0.627}, {128, 128, 0.39, 3.73, 0.513},
+  {128, 256, 1.53, 4.57, 0.793}, {256, 128, 1.05, 5.31, 0.757}, {256, 192, 1.97, 4.86, 1.153}, {256, 256, 3.26, 6.01, 1.316}};
+enum { RING_SHAPE_COUNT = 8, RING_MOST_PARTS = 8 };
+
+struct RingPlan { int shape, parts; double cost; };
+
+// gated: N columns of the result, 2 N weight rows.  pending: parts are left for the caller to add.  least, most: how many parts.
+static RingPlan ring_plan(long M, long N, long K, bool gated, bool pending, int least, int most) {
+  const int units = compute_units();
+  RingPlan best = {gated ? 1 : 0, least, 1e30};
+  const double weights = 3.0 + (gated ? 2.0 : 1.0) * N * K * 2 / 5.2e6;
+  for (int shape = gated ? 1 : 0; shape < RING_SHAPE_COUNT; ++shape) {
+    const RingShape& t = RING_SHAPES[shape];
+    if (M <= t.bm / 2 && t.bm > 64) continue;
+    const long columns = gated ? t.bn / 2 : t.bn, tiles = (M + t.bm - 1) / t.bm * ((N + columns - 1) / columns);
+    for (int s = least; s <= most; ++s) {
+      if (s > 1 && least < most && (K / s < 256 || parts_of_k((int)K, s, 64) != s || (double)s * M * N > (1 << 25))) continue;
+      const double rounds = (double)((tiles * s + units - 1) / units), steps = (double)((K + s - 1) / s) / 64;
+      double cost = t.start + rounds * (t.fixed + steps * t.step);
+      if (cost < weights) cost = weights;
+      cost += s == 1 ? M * N * 2 / 8e6 : s * (double)M * N * 4 / 4e6 + (pending ? 0.0 : 4.0);
+      if (cost < best.cost) best = {shape, s, cost};
+    }
+  }
+  return best;
+}
+
+template <int BM, int BN, int STAGES, int WM_WAVES, int WN_WAVES, int GATE, typename OutT>
+static int launch_ring(const void* A, const void* W, const void* bias, void* C, int M, int N, int K, int lda, int ldc, int splits,
+                       int k_chunk, float alpha, float limit, float shift, hipStream_t stream) {
+  typedef RingTile<BM, BN, STAGES, WM_WAVES, WN_WAVES> Ring;
+  constexpr int COLUMNS = GATE ? BN / 2 : BN;
+  const long tiles = (long)((M + BM - 1) / BM) * ((N + COLUMNS - 1) / COLUMNS) * splits;
+  if (tiles > 0x7ffffff0L) return -1;
+  gemm_ring_kernel<Ring, BM, BN, GATE, OutT><<<(int)((tiles + 7) / 8 * 8), Ring::THREADS, 0, stream>>>(
+      (const bf16_t*)A, (const bf16_t*)W, (const float*)bias, (OutT*)C, M, N, K, lda, ldc, splits, k_chunk, alpha, limit, shift);
+  return LAUNCH_STATUS();
+}
+
+// Whether the kernels of this file take the operands.
+static bool ring_takes(const void* A, const void* W, const void* C, int M, long w_rows, int N, int K, int lda, int ldc) {
+  return K >= 64 && K % 32 == 0 && N % 4 == 0 && lda % 8 == 0 && ldc % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15) == 0 &&
+         (long)M * lda < (1l << 31) && w_rows * K < (1l << 31);
+}
+
+// How `ta_gemm_ring` cuts K: into how many parts.
+extern "C" int ta_gemm_ring_parts(int M, int N, int K, int pending) {
+  if (M <= 0 || N <= 0 || K < 64) return 1;
+  return ring_plan(M, N, K, false, pending != 0, 1, RING_MOST_PARTS).parts;
+}
+
+// out[M, N] = act(A Wg^T) * (A Wu^T), W = [Wg; Wu] of 2 N rows.  act: 1 silu, 2 gelu_tanh, 3 relu, 4 the capped gate of (alpha, limit, shift).
+// shape: a tile of RING_SHAPES, or -1 for the cheapest.  -2: not these operands.
+extern "C" int ta_gemm_ring_gated(const void* A, const void* W, void* out, int M, int N, int K, int lda, int act, float alpha, float limit,
+                                  float shift, int shape, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (!ring_takes(A, W, out, M, 2l * N, N, K, lda, N)) return -2;
+  if (shape < 0) shape = ring_plan(M, N, K, true, false, 1, 1).shape;
+#define GO(BM, BN, ST, WMW, WNW, ACT) launch_ring<BM, BN, ST, WMW, WNW, ACT, bf16_t>(A, W, nullptr, out, M, N, K, lda, N, 1, K, alpha, limit, shift, stream)
+#define SHAPES(ACT)                                         \
+  switch (shape) {                                          \
+    case 1: return GO(64, 128, 3, 2, 4, ACT);               \
+    case 2: return GO(64, 256, 4, 2, 4, ACT);               \
+    case 3: return GO(128, 128, 4, 2, 4, ACT);              \
+    case 4: return GO(128, 256, 3, 2, 4, ACT);              \
+    case 5: return GO(256, 128, 3, 4, 2, ACT);              \
+    case 6: return GO(256, 192, 2, 4, 2, ACT);              \
+    case 7: return GO(256, 256, 2, 2, 4, ACT);              \
+    default: return -1;                                     \
+  }
+  switch (act) {
+    case RING_SILU: SHAPES(RING_SILU)
+    case RING_GELU: SHAPES(RING_GELU)
+    case RING_RELU: SHAPES(RING_RELU)
+    case RING_CAPPED: SHAPES(RING_CAPPED)
+    default: return -1;
+  }
+#undef SHAPES
+#undef GO
+}
+
+// C[M, N] (rows ldc apart; bfloat16 or float) = A W^T + bias.  parts: what `ta_gemm_ring_parts` said; with more than one `partial` takes
+// them, float [parts, M, N], and C may be null: whoever comes next adds them (and the bias).  shape: a tile, or -1 for the cheapest with
+// these parts.  -2: not these operands.
+extern "C" int ta_gemm_ring(const void* A, const void* W, const void* bias, void* C, void* partial, int M, int N, int K, int lda, int ldc,
+                            int parts, int out_dtype, int shape, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (parts < 1 || (parts > 1 && !partial) || (parts == 1 && !C)) return -1;
+  if (!ring_takes(A, W, parts > 1 ? partial : C, M, N, N, K, lda, parts > 1 ? N : ldc) || (C && (ldc % 4 || (uintptr_t)C % 16))) return -2;
+  if (parts > 1 && parts_of_k(K, parts, 64) != parts) return -1;
+  if (shape < 0) shape = ring_plan(M, N, K, false, C == nullptr, parts, parts).shape;
+  const int chunk = parts == 1 ? K : ((K + parts - 1) / parts + 63) / 64 * 64;
+#define GO(BM, BN, ST, WMW, WNW)                                                                                                         \
+  {                                                                                                                                      \
+    int status = parts > 1 ? launch_ring<BM, BN, ST, WMW, WNW, 0, float>(A, W, nullptr, partial, M, N, K, lda, N, parts, chunk, 0, 0, 0, stream) \
+      : out_dtype == DT_F32 ? launch_ring<BM, BN, ST, WMW, WNW, 0, float>(A, W, bias, C, M, N, K, lda, ldc, 1, chunk, 0, 0, 0, stream)   \
+                            : launch_ring<BM, BN, ST, WMW, WNW, 0, bf16_t>(A, W, bias, C, M, N, K, lda, ldc, 1, chunk, 0, 0, 0, stream); \
+    if (status == 0 && parts > 1 && C) status = launch_splitk_reduce((const float*)partial, bias, C, M, N, ldc, parts, out_dtype, stream); \
+    return status;                                                                                                                       \
+  }
+  switch (shape) {
+    case 0: GO(64, 64, 4, 2, 2)
+    case 1: GO(64, 128, 3, 2, 4)
+    case 2: GO(64, 256, 4, 2, 4)
+    case 3: GO(128, 128, 4, 2, 4)
+    case 4: GO(128, 256, 3, 2, 4)
+    case 5: GO(256, 128, 3, 4, 2)
+    case 6: GO(256, 192, 2, 4, 2)
+    case 7: GO(256, 256, 2, 2, 4)
+    default: return -1;
+  }
+#undef GO
+}

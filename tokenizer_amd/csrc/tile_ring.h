@@ -45,7 +45,7 @@ __device__ __forceinline__ void ring_barrier() {
 // of row r of block i (row wm * WM + 16 i + r, column wn * WN + 16 j + 4 g).
 template <int BM, int BN, int STAGES, int WM_WAVES, int WN_WAVES>
 struct RingTile {
-  static constexpr int WAVES = WM_WAVES * WN_WAVES, THREADS = WAVES * WAVE, BK = 64, ROW = 128;
+  static constexpr int WAVES = WM_WAVES * WN_WAVES, ACROSS = WN_WAVES, THREADS = WAVES * WAVE, ROW = 128;
   static constexpr int WM = BM / WM_WAVES, WN = BN / WN_WAVES, MI = WM / 16, NI = WN / 16;
   static constexpr int LA = BM / 8 / WAVES, LB = BN / 8 / WAVES, LOADS = LA + LB, STAGE = (BM + BN) * ROW;
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0 && STAGES >= 2 && STAGES <= 4 && STAGES * STAGE <= 160 * 1024);
@@ -53,7 +53,7 @@ struct RingTile {
   static __device__ __forceinline__ int load_row(int wave, int lane, int loads, int i) { return (wave * loads + i) * 8 + (lane >> 3); }
   static __device__ __forceinline__ uint32_t piece_bytes(int lane) { return ((lane & 7) ^ (lane >> 3)) * 16; }
 
-  // A, W: where the tile's K starts; K of `steps` * 64 (at least one step) and, if `half`, 32 more.
+  // A, W: where the tile's K starts; K of `steps` * 64 and, if `half`, 32 more.
   static __device__ __forceinline__ void run(const void* A, const uint32_t (&a_at)[LA], const void* W, const uint32_t (&w_at)[LB],
                                              int steps, bool half, ring_floatx4 (&acc)[MI][NI]) {
     __shared__ __attribute__((aligned(1024))) char ring0[STAGE];

@@ -155,7 +155,7 @@ class Ops:
                      "ta_sample_workspace_words", "ta_library_gemm_bf16", "ta_compute_units", "ta_read_stream",
                      "ta_embedding_streams", "ta_streams_step", "ta_token_shift", "ta_mlstm_scan", "ta_mlstm_chunked", "ta_head_norm_gate",
                      "ta_capped_gate", "ta_norm_add_rmsnorm", "ta_norm_rotate_store", "ta_differential_heads",
-                     "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_expert_combine",
+                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_parts", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_expert_combine",
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
@@ -1488,6 +1488,21 @@ class Ops:
                 m, k = x.shape
                 lda = k
             _need(x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0, "operands must be 16-byte aligned")
+            if self._to_ring(m, n, k, lda, out_dtype, pending):
+                # The ring kernel says into how many parts it wants K cut; parts nobody may be left with it adds itself.
+                # (A recorded step's products of up to 256 rows and a K below 2,048 have always come back whole; 128 rows x 896 over 896
+                # and the norm 8.4 us so, 7.3 in three parts.)
+                leave = pending and not (self.capturing and m <= 256 and k < 2048)
+                parts = self.lib.ta_gemm_ring_parts(m, n, k, int(leave))
+                leave = leave and parts > 1
+                if out is None and not leave:
+                    out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+                partial = torch.empty((parts, m, n), dtype=torch.float32, device=x.device) if parts > 1 else None
+                status = self.lib.ta_gemm_ring(_ptr(x), _ptr(weight), _ptr(bias), _ptr(None if leave else out), _ptr(partial), m, n, k,
+                                               lda, n, parts, _code(out_dtype), -1, self._stream())
+                if status != -2:              # -2: not these operands after all (an output that is not aligned)
+                    self._check(status, "linear")
+                    return PendingSum(self, partial, bias, out_dtype) if leave else out
             streaming_splits = self._streaming_splits(m, n, k, pending)
             if streaming_splits > 1 and self.split_k_kind == "streaming":
                 # 17 to 64 rows, a long K and few output columns (the down projection of a decode batch): the
@@ -1560,6 +1575,25 @@ class Ops:
 
     use_split_k = True
     skinny_column_blocks = 0   # blocks of sixteen output columns per workgroup of the weight-streaming kernel: 0 = its choice
+
+    use_ring = True            # products of many rows in the ring kernel (gemm_ring_bf16.hip) where it is the faster one
+    RING_ROWS = 1024           # plain bfloat16 products: up to so many rows ...
+    RING_WEIGHT = 2 ** 23      # ... of matrices of up to so many elements, or with a K of four times the columns
+    RING_PENDING_ROWS = 4096   # products whose parts the next norm adds, and those with a float result
+
+    def _to_ring(self, m: int, n: int, k: int, lda: int, out_dtype: torch.dtype, pending: bool) -> bool:
+        """Whether a bfloat16 product of more than 64 rows goes to the ring kernel.  Against the library's timed choice, us (weights
+        from memory, library | ring, the norm that follows included where parts are left for it): 512 rows x 1,536 over 8,960
+        42.7 | 30.1, 256 x 3,584 over 18,944 120 | 55, 2,048 x 896 over 4,864 37.7 | 32.9, 4,096 x 1,536 over 1,536 39.5 | 39.4; plain:
+        512 x 1,152 over 896 8.5 | 6.0, 1,024 x 2,048 over 1,536 12.8 | 11.1, 512 x 1,536 over 8,960 38 | 29; and the other way
+        1,536 x 2,048 over 1,536 15.0 | 16.3, 2,048 x 1,152 over 896 10.8 | 11.6, 512 x 4,608 over 3,584 29 | 33, 3,072 x 896 over
+        4,864 36 | 40."""
+        if not (self.use_ring and m > self.SKINNY_ROWS and k >= 64 and k % 32 == 0 and n % 4 == 0
+                and m * lda < 2 ** 31 and n * k < 2 ** 31):
+            return False
+        if pending or out_dtype == torch.float32 or not self.use_library_gemm:
+            return m <= self.RING_PENDING_ROWS or not self.use_library_gemm
+        return m <= self.RING_ROWS and (n * k <= self.RING_WEIGHT or k >= 4 * n)
 
     def _k_splits(self, m: int, n: int, k: int, pending: bool = False) -> int:
         """Into how many parts the tiled kernel cuts K.  17 to 64 rows: more than one with a K so long, and so few
@@ -1644,6 +1678,18 @@ class Ops:
             out = torch.empty((m, inner), dtype=x.dtype, device=x.device)
         _need(tuple(out.shape) == (m, inner) and out.dtype == x.dtype and out.is_contiguous(), "gated output shape")
         _need(out.is_cuda, "kernel operands must live on the GPU")
+        if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and self._gated_to_ring(m, inner, x.shape[1]):
+            _need(x.is_cuda and weight.is_cuda and x.dim() == 2 and x.shape[1] == weight.shape[1], "linear shapes do not fit")
+            _need(x.stride(1) == 1 and weight.is_contiguous(), "linear operands must have contiguous rows")
+            alpha, limit, shift = act if isinstance(act, tuple) else (0.0, 0.0, 0.0)
+            _need(not isinstance(act, str) or act in ("gelu_tanh", "relu"), f"unknown gated activation {act!r}")
+            status = self.lib.ta_gemm_ring_gated(_ptr(x), _ptr(weight), _ptr(out), m, inner, x.shape[1], x.stride(0),
+                                                 4 if isinstance(act, tuple) else {None: 1, "gelu_tanh": 2, "relu": 3}[act],
+                                                 ctypes.c_float(alpha), ctypes.c_float(limit), ctypes.c_float(shift), -1,
+                                                 self._stream())
+            if status != -2:                  # -2: rows that are not aligned, matrices past 32-bit places
+                self._check(status, "linear_silu_gate")
+                return out
         if act is not None and not isinstance(act, str):
             return self.silu_gate(self.linear(x, weight), out, act=act)
         if x.dtype == torch.float32 and act is None and 0 < m <= self.FUSED_ROWS:
@@ -1669,6 +1715,20 @@ class Ops:
                                                      self._stream()), "linear_silu_gate")
             return out
         return self.silu_gate(self.linear(x, weight), out, act=act)
+
+    RING_GATED_WEIGHT = 2 ** 26    # joined gate and up elements from which ...
+    RING_GATED_ROWS = 640          # ... the library's product and the activation kernel take up to so many rows
+    RING_GATED_FROM = 32           # the rows from which the ring kernel takes the smaller ones
+
+    def _gated_to_ring(self, m: int, inner: int, k: int) -> bool:
+        """Whether a gated bfloat16 product goes to the ring kernel, sums and activation in one.  Us, product and activation before
+        (the weight-streaming kernel up to 64 rows, the library above) | ring: 64 rows, inner 4,864 over 896 12.6 | 10.9, 512 rows
+        23.1 | 18.1, 2,048 rows 59 | 51; 512 rows, 8,960 over 1,536 43 | 42, 2,048 rows 138 | 117; 2,048 rows, 18,944 over 3,584
+        557 | 449, 4,096 rows 934 | 908, but 64 rows 62 | 70, 192 rows 83 | 91, 512 rows 147 | 159 (256 rows 103 | 97): large weights
+        of few rows are a stream that tiles of 128 columns do not share evenly.  32 rows, 4,864 over 896: 10.1 | 9.9, 17 rows 8.9 | 9.8."""
+        if not (self.use_ring and m > self.RING_GATED_FROM and k >= 64 and k % 32 == 0 and inner % 4 == 0):
+            return False
+        return m > self.RING_GATED_ROWS or 2 * inner * k < self.RING_GATED_WEIGHT or not self.use_library_gemm
 
     # ------------------------------------------------------- fused decode products
     FUSED_ROWS = 16
