@@ -482,6 +482,23 @@ def test_decode_attention_of_many_rows_and_few_parts(ops, ref, n_q, n_kv, d, ite
     torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
 
 
+@pytest.mark.parametrize("n_q,n_kv,d,items,longest,reach", [
+    (14, 2, 64, 3, 512, {}), (14, 2, 64, 1, 24, {}), (8, 8, 96, 2, 511, {}), (12, 2, 128, 4, 500, {}), (4, 2, 64, 5, 1400, dict(window=400)),
+    (4, 2, 128, 5, 1400, dict(chunk=480)), (6, 2, 128, 3, 300, dict(softcap=20.0))], ids=str)
+def test_decode_attention_of_few_rows_keeps_short_ranges_whole(ops, ref, n_q, n_kv, d, items, longest, reach):
+    # One workgroup a row and key head over all its keys, the last block's end and both ends of a window inside a block.
+    lengths, reach = [longest] + [1 + (i * 131) % longest for i in range(items - 1)], dict(reach)
+    qkv, k_pages, v_pages, positions, entry_of_token, table = make_paged_case(
+        torch.bfloat16, n_q, n_kv, d, 16, lengths=lengths, q_lens=[1] * items, seed=21)
+    out_a = torch.full((items, n_q * d), float("nan"), dtype=torch.bfloat16).cuda()
+    out_b = torch.empty_like(out_a)
+    window = reach.pop("window", None)
+    ops.paged_attention(qkv, out_a, k_pages, v_pages, positions, entry_of_token, table, n_q, n_kv, d, window, d ** -0.5,
+                        max_position=longest - 1, **reach)
+    ref.paged_attention(qkv, out_b, k_pages, v_pages, positions, entry_of_token, table, n_q, n_kv, d, window, d ** -0.5, **reach)
+    torch.testing.assert_close(out_a.float(), out_b.float(), rtol=2e-2, atol=4e-3)
+
+
 @pytest.mark.parametrize("parts", [3, 4, 6, 8, 12, 16, 17, 24])
 @pytest.mark.parametrize("n_kv,items", [(1, 3), (4, 75)])
 def test_decode_attention_deals_every_part_of_every_row_once(ops, monkeypatch, ref, parts, n_kv, items):

@@ -1344,6 +1344,12 @@ class Ops:
             # rows of 500 keys of size 64 8.9 -> 6.7 us, of 128 14.3 -> 10.1; a single row of 2,000 keys among short ones would
             # take 23 us instead of 16, so longer ranges stay cut; tied values have workgroups of four waves only).
             split_keys = max(split_keys, 512, -(-4 * rows_of_keys * max_keys // self.target_workgroups))
+        elif max_keys <= 4 * self.min_split_keys and head_dim <= 128 and not keep_first and not tied_values and v_pages is not None:
+            # Fewer rows, up to 512 keys: whole too, a workgroup of many waves for each and no merge.  (One row in parts | whole, 24, 150,
+            # 300 and 500 keys of head size 64: 5.8 6.1 6.2 6.4 | 4.0 4.6 5.4 6.1 us; 96: 6.8 7.2 7.2 7.6 | 3.6 4.4 5.2 6.8; 128: 7.3 8.1 8.3
+            # 8.2 | 4.3 5.5 7.0 9.2, where a compute unit's intake of the last hundred keys costs what the merge did; 256: 11.1 12.8 12.9
+            # 13.0 | 6.7 10.0 13.1 18.1, so there in parts.  Of 513 to 1,024 keys, size 64, 600 and 1,000: 6.3 6.4 | 6.6 9.1.)
+            split_keys = max(split_keys, max_keys)
         split_keys = -(-split_keys // 32) * 32
         # (Reach enough for the block of 32 that a window's or run's first key lies in: `max_keys` has it in its 32 more.  Counted
         # twice, it was a part of its own for a few keys: 512 rows of head size 128 behind a window of 1,000 52.6 us, 48.8 without.)
