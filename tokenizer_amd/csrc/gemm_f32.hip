@@ -2,8 +2,9 @@
 //
 // The float matrix instructions (v_mfma_f32_32x32x2_f32, v_mfma_f32_16x16x4_f32) multiply 32-bit operands and add to 32-bit
 // sums, rounding as a multiply-add does: nothing is narrower than with vector instructions, and a compute unit does 256
-// operations a clock where vector multiply-adds do 128.  Three kernels:
-//   more than 16 rows   tiles through LDS, K cut over workgroups where the tiles alone would leave compute units idle
+// operations a clock where vector multiply-adds do 128.  The kernels:
+//   more than 16 rows   tiles through LDS, K cut over workgroups where the tiles alone would leave compute units idle; where pieces of
+//                       sixteen bytes are aligned on the bfloat16 instructions, every operand split into three numbers of theirs
 //   up to 16 rows       one pass over the weights, sixteen weight rows a workgroup whose waves share K
 //   one or two rows (up to four of large matrices), and up to 16 whose pieces of sixteen bytes are not aligned    vector
 //                       multiply-adds, four weight rows a wave
@@ -25,54 +26,61 @@ __device__ __forceinline__ float silu_f32(float g) { return g / (1.0f + expf(-g)
 // blockIdx.x runs over tiles so that the workgroups of one chiplet (every eighth) share strips of weight rows.
 // (1,280 rows at 0.5B sizes, vector multiply-adds and this: gate/up, 9,728 columns over 896, 283 us = 79 TFLOP/s and 203 = 110; down,
 // 896 columns over 4,864 with K cut, 863 and 135; a layer's four products 1,480 and 415.)
+// A tile's place in the launch: false where there is none.
+struct F32Tile { int m0, n0, k_begin, k_end; };
 template <int BM, int BN>
-__global__ void __launch_bounds__(256)
-gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int vec, int k_part, int m_tiles,
-                     int n_tiles, float* __restrict__ partial) {
-  constexpr int TK = 32, QM = BM / 64, QN = BN / 64;       // blocks of 32 x 32 a wave holds each way
-  constexpr int PA = BM / 32, PW = BN / 32;                // rows a thread brings of each operand
-  __shared__ __attribute__((aligned(16))) float a_s[2][BM * TK];
-  __shared__ __attribute__((aligned(16))) float w_s[2][BN * TK];
+__device__ __forceinline__ bool f32_tile_place(F32Tile& t, int K, int k_part, int m_tiles, int n_tiles) {
   const int total = m_tiles * n_tiles, per_chiplet = (total + 7) / 8;
   const int tile = (blockIdx.x % 8) * per_chiplet + blockIdx.x / 8;
-  if (tile >= total) return;
-  const int m0 = tile % m_tiles * BM, n0 = tile / m_tiles * BN;
-  const int k_begin = blockIdx.y * k_part, k_end = min(K, k_begin + k_part);
+  if (tile >= total) return false;
+  t.m0 = tile % m_tiles * BM;
+  t.n0 = tile / m_tiles * BN;
+  t.k_begin = blockIdx.y * k_part;
+  t.k_end = min(K, t.k_begin + k_part);
+  return true;
+}
+
+// Four floats of a row (zeros past the rows and past the part of K).
+__device__ __forceinline__ f32x4 f32_piece(const float* base, int row, int rows, int stride, int k, int k_end, int vec) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (row < rows) {
+    const float* p = base + (size_t)row * stride + k;
+    if (vec && k + 3 < k_end) {
+      v = *reinterpret_cast<const f32x4*>(p);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (k + i < k_end) v[i] = p[i];
+    }
+  }
+  return v;
+}
+
+// The sums of a tile; `lds` holds BUFFERS (BM + BN) rows of 32 floats (with one buffer a step has a barrier more).
+template <int BM, int BN, int BUFFERS>
+__device__ __forceinline__ void f32_tile_sums(const F32Tile& t, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K,
+                                              int lda, int vec, float (&lds)[BUFFERS * (BM + BN) * 32],
+                                              f32x16 (&acc)[BM / 64][BN / 64]) {
+  constexpr int TK = 32, QM = BM / 64, QN = BN / 64;       // blocks of 32 x 32 a wave holds each way
+  constexpr int PA = BM / 32, PW = BN / 32;                // rows a thread brings of each operand
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int row_in = threadIdx.x >> 3, piece = threadIdx.x & 7;       // 32 rows of eight pieces at a time
   f32x4 a_next[PA], w_next[PW];
-
-  auto piece_of = [&](const float* base, int row, int rows, int stride, int k) -> f32x4 {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (row < rows) {
-      const float* p = base + (size_t)row * stride + k;
-      if (vec && k + 3 < k_end) {
-        v = *reinterpret_cast<const f32x4*>(p);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (k + i < k_end) v[i] = p[i];
-      }
-    }
-    return v;
-  };
   auto fetch = [&](int k0) {
     const int k = k0 + piece * 4;
 #pragma unroll
-    for (int i = 0; i < PA; ++i) a_next[i] = piece_of(A, m0 + row_in + 32 * i, M, lda, k);
+    for (int i = 0; i < PA; ++i) a_next[i] = f32_piece(A, t.m0 + row_in + 32 * i, M, lda, k, t.k_end, vec);
 #pragma unroll
-    for (int i = 0; i < PW; ++i) w_next[i] = piece_of(W, n0 + row_in + 32 * i, N, K, k);
+    for (int i = 0; i < PW; ++i) w_next[i] = f32_piece(W, t.n0 + row_in + 32 * i, N, K, k, t.k_end, vec);
   };
   auto put = [&](int buffer) {
     const int at = row_in * TK + ((piece ^ (row_in & 7)) << 2);       // (rows 32 apart are swizzled alike)
 #pragma unroll
-    for (int i = 0; i < PA; ++i) *reinterpret_cast<f32x4*>(&a_s[buffer][at + 32 * TK * i]) = a_next[i];
+    for (int i = 0; i < PA; ++i) *reinterpret_cast<f32x4*>(&lds[buffer * (BM + BN) * TK + at + 32 * TK * i]) = a_next[i];
 #pragma unroll
-    for (int i = 0; i < PW; ++i) *reinterpret_cast<f32x4*>(&w_s[buffer][at + 32 * TK * i]) = w_next[i];
+    for (int i = 0; i < PW; ++i) *reinterpret_cast<f32x4*>(&lds[(buffer * (BM + BN) + BM) * TK + at + 32 * TK * i]) = w_next[i];
   };
 
-  f32x16 acc[QM][QN];
 #pragma unroll
   for (int i = 0; i < QM; ++i)
 #pragma unroll
@@ -82,21 +90,21 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, c
   const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
   const int r = lane & 31, half = lane >> 5;
 
-  fetch(k_begin);
+  fetch(t.k_begin);
   put(0);
   int buffer = 0;
-  for (int k0 = k_begin; k0 < k_end; k0 += TK, buffer ^= 1) {
+  for (int k0 = t.k_begin; k0 < t.k_end; k0 += TK, buffer ^= BUFFERS - 1) {
     __syncthreads();
-    const bool more = k0 + TK < k_end;
+    const bool more = k0 + TK < t.k_end;
     if (more) fetch(k0 + TK);
 #pragma unroll
     for (int s = 0; s < TK / 8; ++s) {
       const int at = r * TK + (((2 * s + half) ^ (r & 7)) << 2);
       f32x4 a[QM], w[QN];
 #pragma unroll
-      for (int i = 0; i < QM; ++i) a[i] = *reinterpret_cast<const f32x4*>(&a_s[buffer][(wm + 32 * i) * TK + at]);
+      for (int i = 0; i < QM; ++i) a[i] = *reinterpret_cast<const f32x4*>(&lds[(buffer * (BM + BN) + wm + 32 * i) * TK + at]);
 #pragma unroll
-      for (int j = 0; j < QN; ++j) w[j] = *reinterpret_cast<const f32x4*>(&w_s[buffer][(wn + 32 * j) * TK + at]);
+      for (int j = 0; j < QN; ++j) w[j] = *reinterpret_cast<const f32x4*>(&lds[(buffer * (BM + BN) + BM + wn + 32 * j) * TK + at]);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -104,9 +112,18 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 #pragma unroll
           for (int j = 0; j < QN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[j][e], a[i][e], acc[i][j], 0, 0, 0);
     }
-    if (more) put(buffer ^ 1);        // (its readers passed the barrier above)
+    if (BUFFERS == 1) __syncthreads();
+    if (more) put(buffer ^ (BUFFERS - 1));        // (its readers passed the barrier above)
   }
-  // Weight rows are the instruction's rows: element e of a lane is column 8 (e / 4) + 4 half + e % 4 of row r of A.
+}
+
+// Weight rows are the instruction's rows: element e of a lane is column 8 (e / 4) + 4 half + e % 4 of row r of A.
+template <int BM, int BN>
+__device__ __forceinline__ void f32_tile_store(const F32Tile& t, const float* __restrict__ bias, float* __restrict__ C, int M, int N, int ldc,
+                                               float* __restrict__ partial, const f32x16 (&acc)[BM / 64][BN / 64]) {
+  constexpr int QM = BM / 64, QN = BN / 64;
+  const int lane = threadIdx.x & 63, wave = wave_index(), r = lane & 31, half = lane >> 5;
+  const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2), m0 = t.m0, n0 = t.n0;
   float* dst = partial ? partial + (size_t)blockIdx.y * M * N : C;
   const int stride = partial ? N : ldc;
   const bool quads = N % 4 == 0 && stride % 4 == 0 && ((uintptr_t)dst & 15) == 0;
@@ -131,6 +148,151 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, c
         }
       }
   }
+}
+
+template <int BM, int BN>
+__global__ void __launch_bounds__(256)
+gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int vec, int k_part, int m_tiles,
+                     int n_tiles, float* __restrict__ partial) {
+  __shared__ __attribute__((aligned(16))) float lds[2 * (BM + BN) * 32];
+  F32Tile t;
+  if (!f32_tile_place<BM, BN>(t, K, k_part, m_tiles, n_tiles)) return;
+  f32x16 acc[BM / 64][BN / 64];
+  f32_tile_sums<BM, BN, 2>(t, A, W, M, N, K, lda, vec, lds, acc);
+  f32_tile_store<BM, BN>(t, bias, C, M, N, ldc, partial, acc);
+}
+
+// The same products on the bfloat16 instructions, sixteen times as fast as the float ones, without losing anything of the operands: a float
+// is the sum of three bfloat16 numbers (its nearest one, that of the rest, that of what then is left: 8 + 8 + 8 bits and the signs), and
+// of the nine products of two such sums the six largest are summed, smallest first (a1 b3, a3 b1, a2 b2, a1 b2, a2 b1, a1 b1); the
+// three left out are at most 2^-26 of |a b| each.  Products of bfloat16 numbers are exact, the sums are floats, and an instruction rounds
+// a sum of sixteen products where the float one rounds after two: against 64 bits the relative error (2-norm) is 2.1e-7 to 7.7e-7
+// over 17 to 2,048 rows and K of 896 to 4,864, 10 to 20 % below the float instructions' at every size measured.
+// A sum that is no finite number sends its workgroup back over the tile with the float instructions: infinities have no rest to
+// split off, and numbers past the largest bfloat16 none either.
+// The splitting is done once a tile and step, on the way from registers to LDS: three planes of rows of 64 bytes, whose four pieces are
+// XOR-swizzled by a quarter of the row (by half of it the reads run at 0.9 of LDS's rate, by the row itself at half).  One buffer: three workgroups share a compute unit, so that one splits while another multiplies.
+// AHEAD steps' rows are on their way to registers.  Bound by the matrix cores (1,536 clocks a step of 32 at 128 x 128, six times the work of a
+// bfloat16 product: 1,000 to 1,100 TFLOP/s of it) and, beside them, by the splitting's vector instructions (some 700); few tiles by a
+// step's chain of load, split, LDS and multiplication, 0.8 us.
+// (Float tiles | this, us: 1,280 rows of 9,728 columns over 896 208 | 130, of 896 over 4,864 129 | 80, of 1,152 over 896 37 | 25; 300 rows 69 | 52,
+// 45 | 31, 17.6 | 12.5; 64 rows of 151,936 over 896 218 | 155.)
+typedef __bf16 split_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 split_bf16x4 __attribute__((ext_vector_type(4)));
+template <int BM, int BN, int AHEAD>
+__global__ void __launch_bounds__(256, 3)
+gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+                      float* __restrict__ C, int M, int N, int K, int lda, int ldc, int k_part, int m_tiles, int n_tiles,
+                      float* __restrict__ partial) {
+  constexpr int TK = 32, ROW = 64, QM = BM / 64, QN = BN / 64, PA = BM / 32, PW = BN / 32, PLANE = (BM + BN) * ROW;
+  // (The planes; a buffer of float rows, where it comes to that.)
+  __shared__ __attribute__((aligned(16))) union { char planes[3 * PLANE]; float rows[(BM + BN) * 32]; } lds;
+  F32Tile t;
+  if (!f32_tile_place<BM, BN>(t, K, k_part, m_tiles, n_tiles)) return;
+  const int lane = threadIdx.x & 63, wave = wave_index(), r = lane & 31, half = lane >> 5;
+  const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+  const int row_in = threadIdx.x >> 3, piece = threadIdx.x & 7;
+  // Rows past the last read the last one (their results are not stored); pieces past the end of K read the part's first and are put
+  // down as zeros.  So every load is made, and the compiler can count them.
+  uint32_t a_at[PA], w_at[PW];
+#pragma unroll
+  for (int i = 0; i < PA; ++i) a_at[i] = ((uint32_t)min(t.m0 + row_in + 32 * i, M - 1) * lda + piece * 4) * 4;
+#pragma unroll
+  for (int i = 0; i < PW; ++i) w_at[i] = ((uint32_t)min(t.n0 + row_in + 32 * i, N - 1) * K + piece * 4) * 4;
+  f32x4 a_next[AHEAD][PA], w_next[AHEAD][PW];
+  typedef const char __attribute__((address_space(1)))* memory;
+  typedef const f32x4 __attribute__((address_space(1)))* pieces;
+  const int k_last = t.k_begin + (t.k_end - t.k_begin - 1) / TK * TK;
+  auto fetch = [&](int k_asked, f32x4 (&a_now)[PA], f32x4 (&w_now)[PW]) {
+    const int k0 = min(k_asked, k_last);                    // (past the end the last step again)
+    const uint32_t back = k0 + piece * 4 < t.k_end ? 0 : piece * 16;
+    memory a_base = (memory)(uintptr_t)(A + k0), w_base = (memory)(uintptr_t)(W + k0);
+    asm("" : "+s"(a_base), "+s"(w_base));
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      uint32_t at = a_at[i] - back;
+      asm("" : "+v"(at));
+      a_now[i] = *(pieces)(a_base + at);
+    }
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      uint32_t at = w_at[i] - back;
+      asm("" : "+v"(at));
+      w_now[i] = *(pieces)(w_base + at);
+    }
+  };
+  const int put_at = row_in * ROW + (((piece >> 1) ^ ((row_in >> 2) & 3)) << 4) + (piece & 1) * 8;   // (rows 32 apart are swizzled alike)
+  auto put = [&](const f32x4& v, int at) {
+    f32x4 rest = v;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      split_bf16x4 near;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) near[e] = (__bf16)rest[e];
+      *reinterpret_cast<split_bf16x4*>(lds.planes + p * PLANE + at) = near;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rest[e] -= (float)near[e];
+    }
+  };
+  f32x16 acc[QM][QN];
+#pragma unroll
+  for (int i = 0; i < QM; ++i)
+#pragma unroll
+    for (int j = 0; j < QN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  auto one = [&](int k0, f32x4 (&a_now)[PA], f32x4 (&w_now)[PW]) {
+    if (k0 + piece * 4 >= t.k_end) {
+#pragma unroll
+      for (int i = 0; i < PA; ++i) a_now[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < PW; ++i) w_now[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();                                        // (the step before has been read)
+#pragma unroll
+    for (int i = 0; i < PA; ++i) put(a_now[i], put_at + 32 * ROW * i);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) put(w_now[i], BM * ROW + put_at + 32 * ROW * i);
+    __syncthreads();
+    fetch(k0 + AHEAD * TK, a_now, w_now);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int at = r * ROW + (((2 * s + half) ^ ((r >> 2) & 3)) << 4);
+      split_bf16x8 a[3][QM], w[3][QN];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+#pragma unroll
+        for (int i = 0; i < QM; ++i) a[p][i] = *reinterpret_cast<const split_bf16x8*>(lds.planes + p * PLANE + (wm + 32 * i) * ROW + at);
+#pragma unroll
+        for (int j = 0; j < QN; ++j) w[p][j] = *reinterpret_cast<const split_bf16x8*>(lds.planes + p * PLANE + (BM + wn + 32 * j) * ROW + at);
+      }
+      constexpr int OF_A[6] = {0, 2, 1, 0, 1, 0}, OF_W[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int i = 0; i < QM; ++i)
+#pragma unroll
+          for (int j = 0; j < QN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[OF_W[p]][j], a[OF_A[p]][i], acc[i][j], 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) fetch(t.k_begin + j * TK, a_next[j], w_next[j]);
+  for (int k0 = t.k_begin; k0 < t.k_end; k0 += AHEAD * TK) {
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      if (k0 + j * TK < t.k_end) one(k0 + j * TK, a_next[j], w_next[j]);
+  }
+  int odd = 0;
+#pragma unroll
+  for (int i = 0; i < QM; ++i)
+#pragma unroll
+    for (int j = 0; j < QN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) odd |= !(fabsf(acc[i][j][e]) < INFINITY);
+  if (__syncthreads_or(odd)) f32_tile_sums<BM, BN, 1>(t, A, W, M, N, K, lda, 1, lds.rows, acc);
+  f32_tile_store<BM, BN>(t, bias, C, M, N, ldc, partial, acc);
 }
 
 // ----------------------------------------------------------------------------------------------------- few rows
@@ -298,12 +460,17 @@ static bool vector_rows(int M, int N, int K, bool pending) {
   return M <= 2 || (M <= 4 && (K >= 4096 || (long)N * K >= (8l << 20))) || (M <= 8 && K >= 16384 && !pending);
 }
 
-// Which kernel and into how many parts of K (a power of two at most 8): `tile` 16 (few rows), 64 or 128, 0 (vector
-// multiply-adds).  Few rows: parts until there are workgroups for every compute unit, each of eight units of 32 at least, and only
-// where the next kernel adds them (`pending`): a reduction of its own costs as much as it saves.  Many rows: the estimate is
-// rounds of workgroups over the compute units, a round as long as its tile's multiplications at what the two tiles reach
-// (128 x 128: 110 to 121 of the 157 TFLOP/s there are; 64 x 64: 99 to 102 in one part, 90 in two, counted as 88), plus the
-// parts' trip to memory and, where nobody else adds them, a further launch.
+// The split kernel's microseconds for tiles of 64 and 128: start, a workgroup's fixed ones, and those of a step of 32 with one, two and three
+// workgroups on a compute unit (each step 16 or 32 KB from memory, and no less than the weights' trip).  Fitted to 1,070 timed products (17
+// to 3,000 rows, matrices of the 0.5B and 1.5B models, one to eight parts); the choice is on average 1 % slower than the fastest, 17 % at worst.
+static const double SPLIT_64[] = {6.46, -2.10, 0.797, 1.048, 1.382}, SPLIT_128[] = {7.22, -1.00, 1.632, 2.475, 3.672};
+
+// Which kernel and into how many parts of K (at most 8): `tile` 16 (few rows), 64 or 128, 0 (vector
+// multiply-adds).  Few rows: a power of two, until there are workgroups for every compute unit, each of eight units of 32 at least, and only
+// where the next kernel adds them (`pending`): a reduction of its own costs as much as it saves.  Many rows: the estimate above where the
+// pieces are aligned; else rounds of workgroups over the compute units, a round as long as its tile's multiplications at what the
+// two float tiles reach (128 x 128: 110 to 121 of the 157 TFLOP/s there are; 64 x 64: 99 to 102 in one part, 90 in two, counted as 88); plus
+// the parts' trip to memory and, where nobody else adds them, a further launch.
 static void f32_choice(int M, int N, int K, bool aligned, bool pending, int* tile, int* parts) {
   const int units = compute_units();
   *tile = 0;
@@ -316,6 +483,20 @@ static void f32_choice(int M, int N, int K, bool aligned, bool pending, int* til
     return;
   }
   double best = 1e30;
+  if (aligned) {
+    for (int t = 64; t <= 128; t *= 2)
+      for (int p = 1; p <= 8; ++p) {
+        if (p > 1 && (N % 4 || K / p < 128 || parts_of_k(K, p, 32) != p)) continue;
+        const long tiles = (long)((M + t - 1) / t) * ((N + t - 1) / t) * p, load = (tiles + units - 1) / units;
+        const double steps = (double)(((K + p - 1) / p + 31) / 32), *c = t == 64 ? SPLIT_64 : SPLIT_128;
+        double cost = c[0] + (double)(load / 3) * (c[1] + steps * c[4]) + (load % 3 ? c[1] + steps * c[1 + load % 3] : 0.0);
+        const double weights = 3.0 + (double)N * K * 4 / 5.2e6;
+        if (cost < weights) cost = weights;
+        cost += p == 1 ? (double)M * N * 4 / 8e6 : (double)M * N * 4 * p / 4e6 + (pending ? 0.0 : 4.0);
+        if (cost < best) { best = cost; *tile = t; *parts = p; }
+      }
+    return;
+  }
   for (int t = 64; t <= 128; t *= 2)
     for (int p = 1; p <= 8; p *= 2) {
       if (p > 1 && (N % 4 || K / p < 128)) continue;
@@ -354,7 +535,12 @@ extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void*
   } else if (tile) {
     const int m_tiles = (M + tile - 1) / tile, n_tiles = (N + tile - 1) / tile;
     dim3 grid((m_tiles * n_tiles + 7) / 8 * 8, parts);
-    if (tile == 128)
+    const bool split = aligned && (long)M * lda < (1l << 30) && (long)N * K < (1l << 30);      // (32-bit places)
+    if (split && tile == 128)
+      gemm_f32_split_kernel<128, 128, 2><<<grid, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, k_part, m_tiles, n_tiles, slabs);
+    else if (split)
+      gemm_f32_split_kernel<64, 64, 3><<<grid, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, k_part, m_tiles, n_tiles, slabs);
+    else if (tile == 128)
       gemm_f32_tile_kernel<128, 128><<<grid, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, aligned, k_part, m_tiles,
                                                                n_tiles, slabs);
     else
