@@ -62,13 +62,14 @@ def test_products_in_parts_of_every_tile(ops, tile, k, parts):
     assert close(out, want + bias.double(), k, False)
 
 
-@pytest.mark.parametrize("tile", range(1, len(TILES)))
+# (The two after the tiles: large tiles in front, small ones behind, as many columns in either.)
+@pytest.mark.parametrize("tile", range(1, len(TILES) + 2))
 @pytest.mark.parametrize("act", [None, "gelu_tanh", "relu", (1.702, 2.0, 1.0)])
 def test_gated_products_of_every_tile(ops, tile, act):
-    bm, bn = TILES[tile]
+    bm, bn = (TILES + [(128, 256), (256, 256)])[tile]
     numbers = act if isinstance(act, tuple) else (0.0, 0.0, 0.0)
     code = 4 if isinstance(act, tuple) else {None: 1, "gelu_tanh": 2, "relu": 3}[act]
-    for m, inner, k in ((bm, bn // 2, 64), (bm + 1, bn // 2 + 4, 352), (70, 52, 224)):
+    for m, inner, k in ((bm, bn // 2, 64), (bm + 1, bn // 2 + 4, 352), (70, 52, 224), (bm + 70, 300, 192)):
         x, w = strided(m, k, k + 8, m), rand((2 * inner, k), inner, 0.2)
         gate, up = (x.double() @ half.double().t() for half in (w[:inner], w[inner:]))
         if act is None:

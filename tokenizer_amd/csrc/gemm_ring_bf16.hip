@@ -97,14 +97,14 @@ struct RingShape { int bm, bn; double start, fixed, step; };
 static const RingShape RING_SHAPES[] = {
   {64, 64, 2.06, 0.58, 0.232}, {64, 128, 2.37, 0.62, 0.376}, {64, 256, 0.99, 3.08, 0.627}, {128, 128, 0.39, 3.73, 0.513},
   {128, 256, 1.53, 4.57, 0.793}, {256, 128, 1.05, 5.31, 0.757}, {256, 192, 1.97, 4.86, 1.153}, {256, 256, 3.26, 6.01, 1.316}};
-enum { RING_SHAPE_COUNT = 8, RING_MOST_PARTS = 8 };
+enum { RING_SHAPE_COUNT = 8, RING_TAILED = 8, RING_MOST_PARTS = 8 };
 
-struct RingPlan { int shape, parts; double cost; };
+struct RingPlan { int shape, parts; double cost; int main_strips; };
 
 // gated: N columns of the result, 2 N weight rows.  pending: parts are left for the caller to add.  least, most: how many parts.
 static RingPlan ring_plan(long M, long N, long K, bool gated, bool pending, int least, int most) {
   const int units = compute_units();
-  RingPlan best = {gated ? 1 : 0, least, 1e30};
+  RingPlan best = {gated ? 1 : 0, least, 1e30, 0};
   const double weights = 3.0 + (gated ? 2.0 : 1.0) * N * K * 2 / 5.2e6;
   for (int shape = gated ? 1 : 0; shape < RING_SHAPE_COUNT; ++shape) {
     const RingShape& t = RING_SHAPES[shape];
@@ -116,10 +116,103 @@ static RingPlan ring_plan(long M, long N, long K, bool gated, bool pending, int 
       double cost = t.start + rounds * (t.fixed + steps * t.step);
       if (cost < weights) cost = weights;
       cost += s == 1 ? M * N * 2 / 8e6 : s * (double)M * N * 4 / 4e6 + (pending ? 0.0 : 4.0);
-      if (cost < best.cost) best = {shape, s, cost};
+      if (cost < best.cost) best = {shape, s, cost, 0};
     }
   }
+  // Whole rounds of 256 x 256 (128 x 256) tiles and the columns behind them in 128 x 128 (64 x 128) ones.
+  if (gated && least == 1)
+    for (int shape = 4; shape <= 7; shape += 3) {
+      const RingShape &t = RING_SHAPES[shape], &u = RING_SHAPES[shape == 7 ? 3 : 1];
+      const long tall = (M + t.bm - 1) / t.bm, strips = (N + 127) / 128, rounds = tall * strips / units, main = rounds * units / tall;
+      if (rounds < 1 || main < 1 || main >= strips) continue;
+      const long left = (M + u.bm - 1) / u.bm * ((N - main * 128 + 63) / 64);
+      const double steps = (double)K / 64;
+      double cost = t.start + rounds * (t.fixed + steps * t.step) + (double)((left + units - 1) / units) * (u.fixed + steps * u.step);
+      if (cost < weights) cost = weights;
+      cost += M * N * 2 / 8e6;
+      if (cost < best.cost) best = {RING_TAILED + (shape == 7), 1, cost, (int)main};
+    }
   return best;
+}
+
+// The gated product where rounds of large tiles would leave the last one mostly empty: `main_strips` strips of columns in the large tiles of
+// Main, the columns behind them in the smaller ones of Tail, which the compute units take up as they get through with the large ones.
+// Both use the same LDS: Main's stages have A and W in arrays of their own, Tail's lie in those.
+// (2,048 rows x 4,864 columns over 896: 256 + 192 tiles in 44.8 us, 408 of 256 x 192 in 50.9, 304 of 256 x 256 in 54.0; 8,960 over 1,536
+// 112, 119, 128; 512 rows x 18,944 over 3,584 136, 156 without.)
+template <class Tile, int BM, int BN, int GATE, class ASlot, class WSlot>
+__device__ __forceinline__ void gated_tile(ASlot a_slot, WSlot w_slot, int m0, int n0, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                           bf16_t* __restrict__ C, int M, int N, int K, int lda, float alpha, float limit, float shift) {
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  uint32_t a_at[Tile::LA], w_at[Tile::LB];
+#pragma unroll
+  for (int i = 0; i < Tile::LA; ++i)
+    a_at[i] = (uint32_t)min(m0 + Tile::load_row(wave, lane, Tile::LA, i), M - 1) * lda * 2 + Tile::piece_bytes(lane);
+#pragma unroll
+  for (int i = 0; i < Tile::LB; ++i) {
+    const int row = Tile::load_row(wave, lane, Tile::LB, i);
+    w_at[i] = (uint32_t)(min(n0 + (row >> 5) * 16 + (row & 15), N - 1) + (row & 16 ? N : 0)) * K * 2 + Tile::piece_bytes(lane);
+  }
+  ring_floatx4 acc[Tile::MI][Tile::NI];
+  Tile::run_in(a_slot, w_slot, A, a_at, W, w_at, K / 64, (K & 32) != 0, acc);
+  const int r = lane & 15, g = lane >> 4, wm = wave / Tile::ACROSS, wn = wave % Tile::ACROSS;
+#pragma unroll
+  for (int i = 0; i < Tile::MI; ++i) {
+    const int m = m0 + wm * Tile::WM + 16 * i + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < Tile::NI; j += 2) {
+      const int n = n0 + wn * (Tile::WN / 2) + 8 * j + 4 * g;
+      if (n >= N) continue;
+      ring_floatx4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = ring_gate<GATE>(acc[i][j][e], acc[i][j + 1][e], alpha, limit, shift);
+      ring_store4(C + (size_t)m * N + n, v);
+    }
+  }
+}
+
+// WIDE: 256 x 256 (two stages) and 128 x 128 (four); else 128 x 256 and 64 x 128 (three stages both).
+template <bool WIDE, int GATE>
+__global__ void __launch_bounds__(512)
+gemm_ring_tailed_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, bf16_t* __restrict__ C, int M, int N, int K, int lda,
+                        int main_strips, int main_blocks, float alpha, float limit, float shift) {
+  constexpr int BM = WIDE ? 256 : 128, TM = BM / 2, GROUP = 16;
+  __shared__ __attribute__((aligned(1024))) char wide0[32768];
+  __shared__ __attribute__((aligned(1024))) char wide1[32768];
+  __shared__ __attribute__((aligned(1024))) char wide2[32768];
+  __shared__ __attribute__((aligned(1024))) char more0[WIDE ? 32768 : 16384];
+  __shared__ __attribute__((aligned(1024))) char more1[WIDE ? 16 : 16384];
+  __shared__ __attribute__((aligned(1024))) char more2[WIDE ? 16 : 16384];
+  const bool main = (int)blockIdx.x < main_blocks;
+  const int columns = main ? 128 : 64, height = main ? BM : TM, block = main ? blockIdx.x : blockIdx.x - main_blocks;
+  const int from = main ? 0 : main_strips * 128;
+  const int tall = (M + height - 1) / height, strips = main ? main_strips : (N - from + columns - 1) / columns;
+  const int total = tall * strips, per_chiplet = (total + 7) / 8, turn = block >> 3, place = (block & 7) * per_chiplet + turn;
+  if (turn >= per_chiplet || place >= total) return;
+  const int first = place / (GROUP * strips) * GROUP, high = min(GROUP, tall - first), inside = place - first * strips;
+  const int m0 = (first + inside % high) * height, n0 = from + inside / high * columns;
+  if (main) {
+    auto a_slot = [&](auto which) -> ring_lds {
+      constexpr int j = decltype(which)::value % (WIDE ? 2 : 3);
+      if constexpr (WIDE) { if constexpr (j == 0) return (ring_lds)wide0; else return (ring_lds)wide1; }
+      else if constexpr (j == 0) return (ring_lds)more0; else if constexpr (j == 1) return (ring_lds)more1; else return (ring_lds)more2;
+    };
+    auto w_slot = [&](auto which) -> ring_lds {
+      constexpr int j = decltype(which)::value % (WIDE ? 2 : 3);
+      if constexpr (WIDE) { if constexpr (j == 0) return (ring_lds)wide2; else return (ring_lds)more0; }
+      else if constexpr (j == 0) return (ring_lds)wide0; else if constexpr (j == 1) return (ring_lds)wide1; else return (ring_lds)wide2;
+    };
+    gated_tile<RingTile<BM, 256, WIDE ? 2 : 3, 2, 4>, BM, 256, GATE>(a_slot, w_slot, m0, n0, A, W, C, M, N, K, lda, alpha, limit, shift);
+  } else {
+    auto a_slot = [&](auto which) -> ring_lds {
+      constexpr int j = decltype(which)::value % (WIDE ? 4 : 3);
+      if constexpr (j == 0) return (ring_lds)wide0; else if constexpr (j == 1) return (ring_lds)wide1;
+      else if constexpr (j == 2) return (ring_lds)wide2; else return (ring_lds)more0;
+    };
+    auto w_slot = [&](auto which) -> ring_lds { return a_slot(which) + TM * 128; };
+    gated_tile<RingTile<TM, 128, WIDE ? 4 : 3, 2, 4>, TM, 128, GATE>(a_slot, w_slot, m0, n0, A, W, C, M, N, K, lda, alpha, limit, shift);
+  }
 }
 
 template <int BM, int BN, int STAGES, int WM_WAVES, int WN_WAVES, int GATE, typename OutT>
@@ -131,6 +224,17 @@ static int launch_ring(const void* A, const void* W, const void* bias, void* C, 
   if (tiles > 0x7ffffff0L) return -1;
   gemm_ring_kernel<Ring, BM, BN, GATE, OutT><<<(int)((tiles + 7) / 8 * 8), Ring::THREADS, 0, stream>>>(
       (const bf16_t*)A, (const bf16_t*)W, (const float*)bias, (OutT*)C, M, N, K, lda, ldc, splits, k_chunk, alpha, limit, shift);
+  return LAUNCH_STATUS();
+}
+
+template <bool WIDE, int GATE>
+static int launch_tailed(const void* A, const void* W, void* out, int M, int N, int K, int lda, int main_strips, float alpha, float limit,
+                         float shift, hipStream_t stream) {
+  const long tall = (M + (WIDE ? 255 : 127)) / (WIDE ? 256 : 128), low = (M + (WIDE ? 127 : 63)) / (WIDE ? 128 : 64);
+  const long main = tall * main_strips, left = low * ((N - 128l * main_strips + 63) / 64), main_blocks = (main + 7) / 8 * 8;
+  if (main_strips < 0 || 128l * main_strips >= N || main_blocks + left > 0x7ffffff0L) return -1;
+  gemm_ring_tailed_kernel<WIDE, GATE><<<(int)(main_blocks + (left + 7) / 8 * 8), 512, 0, stream>>>(
+      (const bf16_t*)A, (const bf16_t*)W, (bf16_t*)out, M, N, K, lda, main_strips, (int)main_blocks, alpha, limit, shift);
   return LAUNCH_STATUS();
 }
 
@@ -147,12 +251,20 @@ extern "C" int ta_gemm_ring_parts(int M, int N, int K, int pending) {
 }
 
 // out[M, N] = act(A Wg^T) * (A Wu^T), W = [Wg; Wu] of 2 N rows.  act: 1 silu, 2 gelu_tanh, 3 relu, 4 the capped gate of (alpha, limit, shift).
-// shape: a tile of RING_SHAPES, or -1 for the cheapest.  -2: not these operands.
+// shape: a tile of RING_SHAPES, RING_TAILED for 128 x 256 and 64 x 128, + 1 for 256 x 256 and 128 x 128, or -1 for the cheapest.  -2: not these
+// operands.
 extern "C" int ta_gemm_ring_gated(const void* A, const void* W, void* out, int M, int N, int K, int lda, int act, float alpha, float limit,
                                   float shift, int shape, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (!ring_takes(A, W, out, M, 2l * N, N, K, lda, N)) return -2;
-  if (shape < 0) shape = ring_plan(M, N, K, true, false, 1, 1).shape;
+  int main_strips = 0;
+  if (shape < 0) {
+    const RingPlan best = ring_plan(M, N, K, true, false, 1, 1);
+    shape = best.shape;
+    main_strips = best.main_strips;
+  } else if (shape >= RING_TAILED) {                        // (asked for: half of the columns in large tiles)
+    main_strips = (N + 127) / 256;
+  }
 #define GO(BM, BN, ST, WMW, WNW, ACT) launch_ring<BM, BN, ST, WMW, WNW, ACT, bf16_t>(A, W, nullptr, out, M, N, K, lda, N, 1, K, alpha, limit, shift, stream)
 #define SHAPES(ACT)                                         \
   switch (shape) {                                          \
@@ -163,6 +275,8 @@ extern "C" int ta_gemm_ring_gated(const void* A, const void* W, void* out, int M
     case 5: return GO(256, 128, 3, 4, 2, ACT);              \
     case 6: return GO(256, 192, 2, 4, 2, ACT);              \
     case 7: return GO(256, 256, 2, 2, 4, ACT);              \
+    case RING_TAILED: return launch_tailed<false, ACT>(A, W, out, M, N, K, lda, main_strips, alpha, limit, shift, stream);      \
+    case RING_TAILED + 1: return launch_tailed<true, ACT>(A, W, out, M, N, K, lda, main_strips, alpha, limit, shift, stream);   \
     default: return -1;                                     \
   }
   switch (act) {

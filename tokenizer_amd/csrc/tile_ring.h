@@ -67,11 +67,19 @@ struct RingTile {
       else if constexpr (j == 2) return (ring_lds)ring2;
       else return (ring_lds)ring3;
     };
+    run_in(slot, [&](auto which) -> ring_lds { return slot(which) + BM * ROW; }, A, a_at, W, w_at, steps, half, acc);
+  }
+
+  // The same in buffers of the caller's: `a_slot(j)`, `w_slot(j)` (j an integral constant, to be taken modulo STAGES) give the places of
+  // BM and BN rows, in arrays of their own for every j.
+  template <class ASlot, class WSlot>
+  static __device__ __forceinline__ void run_in(ASlot a_slot, WSlot w_slot, const void* A, const uint32_t (&a_at)[LA], const void* W,
+                                                const uint32_t (&w_at)[LB], int steps, bool half, ring_floatx4 (&acc)[MI][NI]) {
     const int lane = threadIdx.x & 63, wave = wave_index(), r = lane & 15, g = lane >> 4;
     const int wm = wave / WN_WAVES, wn = wave % WN_WAVES;
     // `keep`: the bits of a place that count.  A step past the last one asks for the first piece again and again: one line, so
     // that the loads under way stay countable and cost next to nothing.
-    auto bring = [&](ring_lds to, ring_memory a, ring_memory w, uint32_t keep, uint32_t back) {
+    auto bring = [&](ring_lds to_a, ring_lds to_w, ring_memory a, ring_memory w, uint32_t keep, uint32_t back) {
       asm("" : "+s"(a), "+s"(w));
       uint32_t av[LA], wv[LB];
 #pragma unroll
@@ -81,22 +89,22 @@ struct RingTile {
 #pragma unroll
       for (int i = 0; i < LA; ++i)
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a + av[i]),
-                                         (__attribute__((address_space(3))) void*)(to + (wave * LA + i) * 1024), 16, 0, 0);
+                                         (__attribute__((address_space(3))) void*)(to_a + (wave * LA + i) * 1024), 16, 0, 0);
 #pragma unroll
       for (int i = 0; i < LB; ++i)
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(w + wv[i]),
-                                         (__attribute__((address_space(3))) void*)(to + BM * ROW + (wave * LB + i) * 1024), 16, 0, 0);
+                                         (__attribute__((address_space(3))) void*)(to_w + (wave * LB + i) * 1024), 16, 0, 0);
     };
     auto fetch = [&](int step, auto which) {
       const bool past = step >= steps;
       const size_t along = past ? 0 : (size_t)step * ROW;
-      bring(slot(which), (ring_memory)(uintptr_t)A + along, (ring_memory)(uintptr_t)W + along, past ? 0u : ~0u, 0u);
+      bring(a_slot(which), w_slot(which), (ring_memory)(uintptr_t)A + along, (ring_memory)(uintptr_t)W + along, past ? 0u : ~0u, 0u);
     };
     uint32_t a_get[2], w_get[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       a_get[ks] = (wm * WM + r) * ROW + (((ks * 4 + g) ^ (r & 7)) * 16);
-      w_get[ks] = BM * ROW + (wn * WN + r) * ROW + (((ks * 4 + g) ^ (r & 7)) * 16);
+      w_get[ks] = (wn * WN + r) * ROW + (((ks * 4 + g) ^ (r & 7)) * 16);
     }
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -105,7 +113,7 @@ struct RingTile {
     ring_bf16x8 af[2][MI], wf[2][NI];
     auto read = [&](auto which, auto half_step) {
       constexpr int ks = decltype(half_step)::value;
-      const ring_lds from_a = slot(which) + a_get[ks], from_w = slot(which) + w_get[ks];
+      const ring_lds from_a = a_slot(which) + a_get[ks], from_w = w_slot(which) + w_get[ks];
 #pragma unroll
       for (int j = 0; j < NI; ++j) wf[ks][j] = *(const ring_bf16x8 __attribute__((address_space(3)))*)(from_w + j * 16 * ROW);
 #pragma unroll
@@ -161,7 +169,7 @@ struct RingTile {
       ring_barrier();
       const size_t along = (size_t)steps * ROW;
       const uint32_t back = (((lane & 7) ^ (lane >> 3)) & 4) * 16;
-      bring(slot(first), (ring_memory)(uintptr_t)A + along, (ring_memory)(uintptr_t)W + along, ~0u, back);
+      bring(a_slot(first), w_slot(first), (ring_memory)(uintptr_t)A + along, (ring_memory)(uintptr_t)W + along, ~0u, back);
       ring_wait<0>();
       ring_barrier();
       read(first, first);

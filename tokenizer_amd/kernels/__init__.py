@@ -1723,15 +1723,15 @@ class Ops:
         return self.silu_gate(self.linear(x, weight), out, act=act)
 
     RING_GATED_WEIGHT = 2 ** 26    # joined gate and up elements from which ...
-    RING_GATED_ROWS = 640          # ... the library's product and the activation kernel take up to so many rows
+    RING_GATED_ROWS = 224          # ... the library's product and the activation kernel take up to so many rows
     RING_GATED_FROM = 32           # the rows from which the ring kernel takes the smaller ones
 
     def _gated_to_ring(self, m: int, inner: int, k: int) -> bool:
         """Whether a gated bfloat16 product goes to the ring kernel, sums and activation in one.  Us, product and activation before
         (the weight-streaming kernel up to 64 rows, the library above) | ring: 64 rows, inner 4,864 over 896 12.6 | 10.9, 512 rows
-        23.1 | 18.1, 2,048 rows 59 | 51; 512 rows, 8,960 over 1,536 43 | 42, 2,048 rows 138 | 117; 2,048 rows, 18,944 over 3,584
-        557 | 449, 4,096 rows 934 | 908, but 64 rows 62 | 70, 192 rows 83 | 91, 512 rows 147 | 159 (256 rows 103 | 97): large weights
-        of few rows are a stream that tiles of 128 columns do not share evenly.  32 rows, 4,864 over 896: 10.1 | 9.9, 17 rows 8.9 | 9.8."""
+        23.1 | 18.1, 2,048 rows 59 | 45; 512 rows, 8,960 over 1,536 43 | 42, 2,048 rows 138 | 112; 300 rows, 18,944 over 3,584 120 | 108,
+        512 rows 149 | 136, 2,048 rows 557 | 468, 4,096 rows 934 | 899, but 64 rows 62 | 70, 192 rows 83 | 91: large weights of few rows
+        are a stream that tiles of 128 columns do not share evenly.  32 rows, 4,864 over 896: 10.1 | 9.9, 17 rows 8.9 | 9.8."""
         if not (self.use_ring and m > self.RING_GATED_FROM and k >= 64 and k % 32 == 0 and inner % 4 == 0):
             return False
         return m > self.RING_GATED_ROWS or 2 * inner * k < self.RING_GATED_WEIGHT or not self.use_library_gemm
