@@ -61,3 +61,13 @@ def test_split_products_repeat_bit_for_bit(ops):
     first = ops.linear(x, w)
     for _ in range(5):
         assert torch.equal(ops.linear(x, w), first)
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 96, 200), (260, 1152, 896)])
+def test_split_products_of_a_row_do_not_hang_on_other_rows(ops, m, n, k):
+    x, w = rand((m, k), 7), rand((n, k), 8)
+    alone = ops.linear(x, w)
+    x[m - 1], x[20, 3] = float("nan"), float("inf")
+    beside = ops.linear(x, w)
+    rest = [t for t in range(m) if t not in (20, m - 1)]
+    assert torch.equal(beside[rest], alone[rest]) and not beside[m - 1].isfinite().any() and not beside[20].isfinite().any()

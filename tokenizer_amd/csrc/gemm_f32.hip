@@ -169,8 +169,8 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 // three left out are at most 2^-26 of |a b| each.  Products of bfloat16 numbers are exact, the sums are floats, and an instruction rounds
 // a sum of sixteen products where the float one rounds after two: against 64 bits the relative error (2-norm) is 2.1e-7 to 7.7e-7
 // over 17 to 2,048 rows and K of 896 to 4,864, 10 to 20 % below the float instructions' at every size measured.
-// A sum that is no finite number sends its workgroup back over the tile with the float instructions: infinities have no rest to
-// split off, and numbers past the largest bfloat16 none either.
+// A sum that is no finite number sends its workgroup back over the tile with the float instructions, whose result takes its place:
+// infinities have no rest to split off, and numbers past the largest bfloat16 none either.
 // The splitting is done once a tile and step, on the way from registers to LDS: three planes of rows of 64 bytes, whose four pieces are
 // XOR-swizzled by a quarter of the row (by half of it the reads run at 0.9 of LDS's rate, by the row itself at half).  One buffer: three workgroups share a compute unit, so that one splits while another multiplies.
 // AHEAD steps' rows are on their way to registers.  Bound by the matrix cores (1,536 clocks a step of 32 at 128 x 128, six times the work of a
@@ -284,15 +284,31 @@ gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, 
     for (int j = 0; j < AHEAD; ++j)
       if (k0 + j * TK < t.k_end) one(k0 + j * TK, a_next[j], w_next[j]);
   }
-  int odd = 0;
+  // Only the sums that are no finite numbers are replaced, so that a row's result does not hang on what other rows of its tile hold
+  // (rows that only fill a batch up may hold anything).
+  uint64_t odd = 0;
 #pragma unroll
   for (int i = 0; i < QM; ++i)
 #pragma unroll
     for (int j = 0; j < QN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) odd |= !(fabsf(acc[i][j][e]) < INFINITY);
-  if (__syncthreads_or(odd)) f32_tile_sums<BM, BN, 1>(t, A, W, M, N, K, lda, 1, lds.rows, acc);
+      for (int e = 0; e < 16; ++e)
+        if (!(fabsf(acc[i][j][e]) < INFINITY)) odd |= 1ull << ((i * QN + j) * 16 + e);
   f32_tile_store<BM, BN>(t, bias, C, M, N, ldc, partial, acc);
+  if (!__syncthreads_or(odd != 0)) return;
+  f32_tile_sums<BM, BN, 1>(t, A, W, M, N, K, lda, 1, lds.rows, acc);
+  float* dst = partial ? partial + (size_t)blockIdx.y * M * N : C;
+  const int stride = partial ? N : ldc;
+#pragma unroll
+  for (int i = 0; i < QM; ++i)
+#pragma unroll
+    for (int j = 0; j < QN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = t.m0 + wm + 32 * i + r, n = t.n0 + wn + 32 * j + 8 * (e >> 2) + 4 * half + (e & 3);
+        if ((odd >> ((i * QN + j) * 16 + e) & 1) && m < M && n < N)
+          dst[(size_t)m * stride + n] = acc[i][j][e] + (bias && !partial ? bias[n] : 0.f);
+      }
 }
 
 // ----------------------------------------------------------------------------------------------------- few rows
