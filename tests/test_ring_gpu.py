@@ -89,6 +89,59 @@ def test_gated_products_of_every_tile(ops, tile, act):
         assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 4e-5 * float(want.abs().max()) + slack).all())
 
 
+# Heads of one pair of blocks, of two and of three, more columns than a tile and fewer; tokens that are stored nowhere, pages in any order.
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("n_q,n_kv,d,page_size", [(3, 1, 64, 16), (5, 2, 32, 16), (2, 1, 96, 32), (4, 2, 128, 16)])
+def test_projections_with_rotation_and_store_of_every_tile(ops, tile, n_q, n_kv, d, page_size):
+    m, k, n = TILES[tile][0] + 5, 96 + 64 * (tile % 3), (n_q + 2 * n_kv) * d
+    x, w, bias = strided(m, k, k + 8, tile), rand((n, k), d, 0.1), torch.randn(n, device="cuda")
+    gen = torch.Generator().manual_seed(d)
+    positions = torch.randint(0, 500, (m,), generator=gen).int().cuda()
+    table = torch.randn((500, d), device="cuda")
+    pages = (m + page_size - 1) // page_size + 1
+    slots = torch.randperm(pages * page_size, generator=gen)[:m].int().cuda()
+    slots[3] = -1
+    for use_bias, turn, store in ((True, True, True), (False, True, True), (True, False, True), (True, True, False)):
+        out = x.double() @ w.double().t() + (bias.double() if use_bias else 0.0)
+        heads = out.view(m, n_q + 2 * n_kv, d).clone()
+        if turn:
+            cos, sin = (t[:, None] for t in table.double()[positions.long()].split(d // 2, 1))
+            u, v = heads[:, :n_q + n_kv, :d // 2].clone(), heads[:, :n_q + n_kv, d // 2:].clone()
+            heads[:, :n_q + n_kv] = torch.cat([u * cos - v * sin, v * cos + u * sin], -1)
+        keys = torch.zeros((pages, n_kv, page_size, d), dtype=torch.float64, device="cuda")
+        values = torch.zeros((pages, n_kv, d, page_size), dtype=torch.float64, device="cuda")
+        if store:
+            for t in torch.nonzero(slots >= 0)[:, 0].tolist():
+                page, off = divmod(int(slots[t]), page_size)
+                keys[page, :, off], values[page, :, :, off] = heads[t, n_q:n_q + n_kv], heads[t, n_q + n_kv:]
+        q = torch.full((m, n_q * d), float("nan"), dtype=torch.bfloat16, device="cuda")
+        k_pages, v_pages = keys.to(torch.bfloat16) * 0, values.to(torch.bfloat16) * 0
+        at = lambda t, given=True: _ptr(t if given else None)
+        assert ops.lib.ta_gemm_ring_qkv(_ptr(x), k + 8, _ptr(w), at(bias, use_bias), _ptr(q), _ptr(positions), at(table, turn), at(slots, store),
+                                        _ptr(k_pages), _ptr(v_pages), m, k, n_q, n_kv, d, page_size, tile, ops._stream()) == 0
+        # Float throughout, one rounding of the result: 2^-8 of itself, and of the float sums what a turn by these angles leaves.
+        slack = 8 * 2e-6 * k ** 0.5 * float(out.abs().max())
+        for got, want in ((q, heads[:, :n_q].reshape(m, -1)), (k_pages, keys), (v_pages, values)):
+            assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + slack).all())
+
+
+# Through the entry point: a width that the ring kernel does not take comes back from the two kernels before it, keys and values stored alike.
+@pytest.mark.parametrize("width", [96, 104])
+def test_projection_of_many_rows_whatever_the_width(ops, width):
+    m, n_q, n_kv, d = 70, 2, 1, 32
+    n = (n_q + 2 * n_kv) * d
+    x, w, bias = rand((m, width), 1), rand((n, width), 2, 0.1), torch.randn(n, device="cuda")
+    positions, slots = (torch.arange(m, dtype=torch.int32, device="cuda") for _ in range(2))
+    table = torch.randn((m, d), device="cuda")
+    k_pages, v_pages = (torch.zeros(shape, dtype=torch.bfloat16, device="cuda") for shape in ((5, n_kv, 16, d), (5, n_kv, d, 16)))
+    got = ops.fused_norm_qkv_rope(x, None, 0.0, w, bias, positions, table, slots, k_pages, v_pages, n_q, n_kv, d)[:, :n_q * d]
+    qkv = ops.linear(x, w, bias)
+    keys, values = torch.zeros_like(k_pages), torch.zeros_like(v_pages)
+    ops.rope_store(qkv, None, positions, table, slots, keys, values, n_q, n_kv, d)
+    for a, b in ((got, qkv[:, :n_q * d]), (k_pages, keys), (v_pages, values)):
+        assert float((a.float() - b.float()).abs().max()) <= 3 * 2.0 ** -8 * float(b.float().abs().max())
+
+
 # What goes to the ring kernel comes back as the general kernels give it: rows and sizes on either side of its lines, an activation of
 # each kind, infinities and NaN in a row, which stay in that row.
 @pytest.mark.parametrize("m,n,k", [(65, 96, 64), (300, 128, 2080), (1025, 64, 256), (70, 4100, 512), (33, 96, 64), (257, 8, 96)])

@@ -155,7 +155,7 @@ class Ops:
                      "ta_sample_workspace_words", "ta_library_gemm_bf16", "ta_compute_units", "ta_read_stream",
                      "ta_embedding_streams", "ta_streams_step", "ta_token_shift", "ta_mlstm_scan", "ta_mlstm_chunked", "ta_head_norm_gate",
                      "ta_capped_gate", "ta_norm_add_rmsnorm", "ta_norm_rotate_store", "ta_differential_heads",
-                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_parts", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_expert_combine",
+                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_expert_combine",
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
@@ -1498,7 +1498,7 @@ class Ops:
                 # The ring kernel says into how many parts it wants K cut; parts nobody may be left with it adds itself.
                 # (A recorded step's products of up to 256 rows and a K below 2,048 have always come back whole; 128 rows x 896 over 896
                 # and the norm 8.4 us so, 7.3 in three parts.)
-                leave = pending and not (self.capturing and m <= 256 and k < 2048)
+                leave = pending and not (m <= 256 and k < 2048 and (self.capturing or m * n * k >= self.EAGER_LIBRARY_WORK))
                 parts = self.lib.ta_gemm_ring_parts(m, n, k, int(leave))
                 leave = leave and parts > 1
                 if out is None and not leave:
@@ -1762,7 +1762,8 @@ class Ops:
     def fused_norm_qkv_rope(self, residual, norm_weight, eps, weight, bias, positions, cos_sin, slots,
                             k_pages, v_pages, n_q: int, n_kv: int, head_dim: int) -> torch.Tensor:
         """q, k, v = rmsnorm(residual) @ weight.T + bias; q and k rotated; k and v stored into their pages
-        (when `slots` is given); returns q [M, n_q * d] in bfloat16.  residual float32 [M, K]; or, with
+        (when `slots` is given); returns q [M, n_q * d] in bfloat16 (more than 64 rows that the ring kernel does not take: q, k
+        and v side by side, the query heads first).  residual float32 [M, K]; or, with
         `norm_weight` None, `residual` holds the normalised rows in bfloat16 already."""
         _dev(norm_weight, weight, bias, positions, cos_sin, slots, k_pages, v_pages)
         _need(residual.is_cuda and residual.dim() == 2, "the rows must live on the GPU")
@@ -1776,7 +1777,7 @@ class Ops:
         _need(weight.dtype == torch.bfloat16 and tuple(weight.shape) == ((n_q + 2 * n_kv) * head_dim, k),
               "the joined q/k/v matrix has the wrong shape")
         _need(k % 8 == 0 and head_dim % 32 == 0
-              and (m <= self.FUSED_ROWS or (norm_weight is None and m <= self.SKINNY_ROWS)),
+              and (m <= self.FUSED_ROWS or norm_weight is None),
               "sizes the fused projection does not take")
         _need(positions.dtype == torch.int32 and positions.numel() == m, "positions must be int32 [M]")
         if bias is not None:
@@ -1792,7 +1793,15 @@ class Ops:
         tail = (_ptr(weight), _ptr(bias), _ptr(q), _ptr(positions), _ptr(cos_sin), _ptr(slots),
                 _ptr(k_pages if slots is not None else None), _ptr(v_pages if slots is not None else None),
                 m, k, n_q, n_kv, head_dim, page_size, self.fused_rows, self.fused_waves, self._stream())
-        if m > self.FUSED_ROWS:
+        if m > self.SKINNY_ROWS:
+            # More than 64 rows: the ring kernel with the same epilogue.
+            status = self.lib.ta_gemm_ring_qkv(_ptr(residual), residual.stride(0), *tail[:-3], -1, self._stream())
+            if status == -2:                  # rows of no half steps of K, matrices past 32-bit places, a bias that is not aligned
+                qkv = self.linear(residual, weight, bias)
+                self.rope_store(qkv, None, positions, cos_sin, slots, k_pages if slots is not None else None,
+                                v_pages if slots is not None else None, n_q, n_kv, head_dim)
+                return qkv
+        elif m > self.FUSED_ROWS:
             # 17 to 64 rows: the weight-streaming kernel with the same epilogue.
             status = self.lib.ta_gemm_skinny_qkv_rope(_ptr(residual), residual.stride(0), *tail[:-3], self._stream())
         elif norm_weight is None:
@@ -1832,9 +1841,16 @@ class Ops:
         """Whether `fused_norm_qkv_rope` should take this many normalised bfloat16 rows: 17 to 64 go through the
         weight-streaming kernel, which then needs no rotation kernel after it.  That pays while the matrix is
         small (measured: 0.5B and 1.5B sizes); a big one is better off with the library's product and the
-        rotation kernel."""
-        return (self.use_fused_decode and dtype == torch.bfloat16 and self.FUSED_ROWS < rows <= self.SKINNY_ROWS
-                and weight_elements <= self.ROPE_STORE_WEIGHT)
+        rotation kernel.  More rows go to the ring kernel.  (Product and rotation | ring, us: 1,152 columns over 896, 65 rows
+        9.4 | 6.7, 512 10.2 | 7.1, 2,048 18.0 | 14.8, 4,096 22.8 | 24.0; 2,048 over 1,536 10.8 | 8.1, 13.6 | 9.2, 26.6 | 20.3, 40.7 | 35.3;
+        4,608 over 3,584, 65 rows 22.4 | 18.2, 128 22.8 | 21.1, 300 28.6 | 29.4, 1,024 51.7 | 54.9, 4,096 140 | 164.)"""
+        if dtype != torch.bfloat16 or not self.use_fused_decode:
+            return False
+        if rows > self.SKINNY_ROWS:
+            return self.use_ring and rows <= (self.RING_QKV_ROWS if weight_elements <= self.RING_WEIGHT else 2 * self.SKINNY_ROWS)
+        return self.FUSED_ROWS < rows and weight_elements <= self.ROPE_STORE_WEIGHT
+
+    RING_QKV_ROWS = 3072
 
     def fused_norm_gated(self, residual, norm_weight, eps, weight, act: torch.Tensor | None = None) -> torch.Tensor:
         """silu(x @ Wg.T) * (x @ Wu.T) with x = rmsnorm(residual), weight = [Wg; Wu]; bfloat16 [M, I].  With

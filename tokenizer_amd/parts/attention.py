@@ -331,7 +331,7 @@ class GQAttention(Mixer):
         elif even and not self.plain and _can_fuse(ops, x, self.runtime.dtype) and x.shape[1] % 8 == 0:
             behind = self.position.epilogue()       # up to sixteen normalised rows: the fused decode projection
         if behind is not None:
-            # A few dozen rows: bias, rotation and the cache write ride in the projection's epilogue.
+            # A few dozen rows and many: bias, rotation and the cache write ride in the projection's epilogue.
             qkv = ops.fused_norm_qkv_rope(x, None, 0.0, self.w_qkv, self.b_qkv, ctx.positions, behind.cos_sin,
                                           ctx.slots[cache.group] if cache.writes else None, cache.k_pages,
                                           cache.v_pages, self.n_q, self.n_kv, self.d)
