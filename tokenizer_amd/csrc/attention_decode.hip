@@ -337,10 +337,13 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
 }
 
 // out[t, head, :] = sum_s part_o[s] * exp(m_s - M) / sum_s l_s * exp(m_s - M).  One wave per (item, head).
-// Sixteen lanes share a split's 64 elements (a float4 each), the four groups of sixteen take every fourth
-// split, and all of a lane's loads are requested before the first is used: the kernel is one trip to memory.
+// LANES (16, 32 or 64: those of head sizes to 64, 128 and 256) lanes share a split's elements (a float4 each), the groups of so many
+// take every 64 / LANES-th split, and all of a lane's loads are requested before the first is used: the kernel is one trip to memory.
+// (With sixteen lanes for every head size longer heads were two to four trips.  Attention and merge, eight rows of 1,000
+// keys: 12 heads of 128 9.1 -> 8.5 us, eight of 256 13.8 -> 11.8.)
 // A separate kernel on purpose: a last-arrival merge inside the first kernel needs device-wide fences,
 // which flush the L2 of every XCD and cost more than this launch.
+template <int LANES>
 __global__ void __launch_bounds__(WAVE)
 decode_attention_merge(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                        const int* __restrict__ rows, bf16_t* __restrict__ out, int n_q, int d, int splits,
@@ -358,19 +361,20 @@ decode_attention_merge(const float* __restrict__ part_o, const float* __restrict
     t = row0 + token;
   }
   const size_t base = ((size_t)item * n_q + head) * splits;
-  const int lane = threadIdx.x, part = lane & 15, grp = lane >> 4;
+  constexpr int GROUPS = WAVE / LANES;
+  const int lane = threadIdx.x, part = lane % LANES, grp = lane / LANES;
   const float2* ml = reinterpret_cast<const float2*>(part_ml) + base;
-  constexpr int HELD = 8;                                    // splits a lane holds at once: 32 per round
-  for (int e0 = 0; e0 < d; e0 += 64) {
+  constexpr int HELD = LANES == 16 ? 8 : 16;                 // splits a lane holds at once: 32 or 16 a round
+  for (int e0 = 0; e0 < d; e0 += 4 * LANES) {
     const int e = e0 + 4 * part;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
     float big = -INFINITY, denom = 0.f;
-    for (int s0 = 0; s0 < splits; s0 += 4 * HELD) {
+    for (int s0 = 0; s0 < splits; s0 += GROUPS * HELD) {
       float4 v[HELD];
       float2 stat[HELD];
 #pragma unroll
       for (int j = 0; j < HELD; ++j) {
-        const int s = s0 + 4 * j + grp;
+        const int s = s0 + GROUPS * j + grp;
         v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
         stat[j] = make_float2(-INFINITY, 0.f);
         if (s < splits) {
@@ -392,14 +396,15 @@ decode_attention_merge(const float* __restrict__ part_o, const float* __restrict
         denom += stat[j].y * w;
       }
     }
-    // The four lane groups hold sums over different splits under different maxima: bring them together.
-    float all_big = fmaxf(big, __shfl_xor(big, 16, WAVE));
-    all_big = fmaxf(all_big, __shfl_xor(all_big, 32, WAVE));
+    // The lane groups hold sums over different splits under different maxima: bring them together.
+    float all_big = big;
+#pragma unroll
+    for (int shift = LANES; shift < WAVE; shift *= 2) all_big = fmaxf(all_big, __shfl_xor(all_big, shift, WAVE));
     const float w = (big == -INFINITY) ? 0.f : __expf(big - all_big);
     o.x *= w; o.y *= w; o.z *= w; o.w *= w;
     denom *= w;
 #pragma unroll
-    for (int shift = 16; shift <= 32; shift *= 2) {
+    for (int shift = LANES; shift < WAVE; shift *= 2) {
       o.x += __shfl_xor(o.x, shift, WAVE); o.y += __shfl_xor(o.y, shift, WAVE);
       o.z += __shfl_xor(o.z, shift, WAVE); o.w += __shfl_xor(o.w, shift, WAVE);
       denom += __shfl_xor(denom, shift, WAVE);
@@ -451,8 +456,8 @@ static int launch_decode(const void* q, int q_stride, void* out, const void* k_p
 #undef GO
   int status = LAUNCH_STATUS();
   if (status == 0 && splits > 1) {
-    decode_attention_merge<<<n_items * n_q, 64, 0, stream>>>((const float*)part_o, (const float*)part_ml,
-                                                             (const int*)rows, (bf16_t*)out, n_q, D, splits,
+    decode_attention_merge<D <= 64 ? 16 : D <= 128 ? 32 : 64><<<n_items * n_q, 64, 0, stream>>>(
+                                                             (const float*)part_o, (const float*)part_ml, (const int*)rows, (bf16_t*)out, n_q, D, splits,
                                                              nullptr, nullptr);
     status = LAUNCH_STATUS();
   }
@@ -465,9 +470,10 @@ extern "C" int ta_attention_merge_tiles(const void* part_o, const void* part_ml,
                                         const void* cu_q, void* out, int n_q, int d, int splits, hipStream_t stream) {
   if (n_tiles <= 0) return 0;
   if ((long)n_tiles * 16 * n_q > 0x7fffffffL || d % 4 || splits < 1) return -1;
-  decode_attention_merge<<<n_tiles * 16 * n_q, 64, 0, stream>>>((const float*)part_o, (const float*)part_ml, nullptr,
-                                                                (bf16_t*)out, n_q, d, splits, (const int*)tiles,
-                                                                (const int*)cu_q);
+#define GO(LANES) decode_attention_merge<LANES><<<n_tiles * 16 * n_q, 64, 0, stream>>>((const float*)part_o, (const float*)part_ml, nullptr, \
+      (bf16_t*)out, n_q, d, splits, (const int*)tiles, (const int*)cu_q)
+  if (d <= 64) GO(16); else if (d <= 128) GO(32); else GO(64);
+#undef GO
   return LAUNCH_STATUS();
 }
 
