@@ -1498,7 +1498,7 @@ class Ops:
                 # The ring kernel says into how many parts it wants K cut; parts nobody may be left with it adds itself.
                 # (A recorded step's products of up to 256 rows and a K below 2,048 have always come back whole; 128 rows x 896 over 896
                 # and the norm 8.4 us so, 7.3 in three parts.)
-                leave = pending and not (m <= 256 and k < 2048 and (self.capturing or m * n * k >= self.EAGER_LIBRARY_WORK))
+                leave = pending and not (self.SKINNY_ROWS < m <= 256 and k < 2048 and (self.capturing or m * n * k >= self.EAGER_LIBRARY_WORK))
                 parts = self.lib.ta_gemm_ring_parts(m, n, k, int(leave))
                 leave = leave and parts > 1
                 if out is None and not leave:
@@ -1588,15 +1588,22 @@ class Ops:
     RING_PENDING_ROWS = 4096   # products whose parts the next norm adds, and those with a float result
 
     def _to_ring(self, m: int, n: int, k: int, lda: int, out_dtype: torch.dtype, pending: bool) -> bool:
-        """Whether a bfloat16 product of more than 64 rows goes to the ring kernel.  Against the library's timed choice, us (weights
+        """Whether a bfloat16 product goes to the ring kernel.  More than 64 rows against the library's timed choice, us (weights
         from memory, library | ring, the norm that follows included where parts are left for it): 512 rows x 1,536 over 8,960
         42.7 | 30.1, 256 x 3,584 over 18,944 120 | 55, 2,048 x 896 over 4,864 37.7 | 32.9, 4,096 x 1,536 over 1,536 39.5 | 39.4; plain:
         512 x 1,152 over 896 8.5 | 6.0, 1,024 x 2,048 over 1,536 12.8 | 11.1, 512 x 1,536 over 8,960 38 | 29; and the other way
         1,536 x 2,048 over 1,536 15.0 | 16.3, 2,048 x 1,152 over 896 10.8 | 11.6, 512 x 4,608 over 3,584 29 | 33, 3,072 x 896 over
-        4,864 36 | 40."""
-        if not (self.use_ring and m > self.SKINNY_ROWS and k >= 64 and k % 32 == 0 and n % 4 == 0
-                and m * lda < 2 ** 31 and n * k < 2 ** 31):
+        4,864 36 | 40.  Of 17 to 64 rows those whose parts are left (the weight-streaming and the tiled kernel | ring, with the norm:
+        17 and 64 rows x 896 over 4,864 9.3 | 7.7 and 11.7 | 8.6, x 3,584 over 18,944 39.5 | 33.4 and 47.4 | 36.0, but x 896 over 896
+        6.4 | 6.7 and 7.1 | 7.1), and the vocabulary's projection of any number (weight-streaming kernel up to 16 rows, tiled above | ring:
+        151,936 over 896, 1, 8, 16, 64 rows 51.7 | 52.0, 55.4 | 52.7, 60.8 | 53.0, 78 | 65; over 1,536 87.1 | 85.0, 90.4 | 87.3, 101 | 90,
+        118 | 109; over 3,584 197 | 192, 196 | 190, 211 | 193, 248 | 218)."""
+        if not (self.use_ring and k >= 64 and k % 32 == 0 and n % 4 == 0 and m * lda < 2 ** 31 and n * k < 2 ** 31):
             return False
+        if m <= self.SKINNY_ROWS:
+            if out_dtype == torch.float32 and n >= self.WIDE_OUTPUT:
+                return k >= 1536 or m > 4
+            return pending and m > self.FUSED_ROWS and n * k >= 2 ** 20
         if pending or out_dtype == torch.float32 or not self.use_library_gemm:
             return m <= self.RING_PENDING_ROWS or not self.use_library_gemm
         return m <= self.RING_ROWS and (n * k <= self.RING_WEIGHT or k >= 4 * n)
