@@ -1583,8 +1583,8 @@ class Ops:
     skinny_column_blocks = 0   # blocks of sixteen output columns per workgroup of the weight-streaming kernel: 0 = its choice
 
     use_ring = True            # products of many rows in the ring kernel (gemm_ring_bf16.hip) where it is the faster one
-    RING_ROWS = 1024           # plain bfloat16 products: up to so many rows ...
-    RING_WEIGHT = 2 ** 23      # ... of matrices of up to so many elements, or with a K of four times the columns
+    RING_ROWS = 1024           # plain bfloat16 products: up to so many rows (twice as many of narrow results) ...
+    RING_WEIGHT = 2 ** 23      # ... of matrices of up to so many elements, or with a long K (see `_to_ring`)
     RING_PENDING_ROWS = 4096   # products whose parts the next norm adds, and those with a float result
 
     def _to_ring(self, m: int, n: int, k: int, lda: int, out_dtype: torch.dtype, pending: bool) -> bool:
@@ -1606,7 +1606,12 @@ class Ops:
             return pending and m > self.FUSED_ROWS and n * k >= 2 ** 20
         if pending or out_dtype == torch.float32 or not self.use_library_gemm:
             return m <= self.RING_PENDING_ROWS or not self.use_library_gemm
-        return m <= self.RING_ROWS and (n * k <= self.RING_WEIGHT or k >= 4 * n)
+        # Plain ones, us, library | ring.  Narrow results: 2,048 rows x 896 over 2,432 17.9 | 15.6, x 1,536 over 4,480 39.3 | 37.3, over 8,960
+        # 75.6 | 65.2 (1,600 rows, which no tile divides, 15.3 | 15.2, 33.3 | 36.2, 65.2 | 60.3), 2,600 rows 19.0 | 21.2, 44.9 | 39.4, 86 | 82.
+        # Wider ones with a long K: 400 rows x 3,584 over 7,168 47.8 | 38.1, 800 54.2 | 58.8, 1,600 rows over 18,944 233 | 217, 2,048 236 | 248.
+        if n <= 1536:
+            return m <= 2 * self.RING_ROWS
+        return m <= self.RING_ROWS and n * k <= self.RING_WEIGHT or k >= 2 * n and m <= 640 or k >= 4 * n and m <= 1700
 
     def _k_splits(self, m: int, n: int, k: int, pending: bool = False) -> int:
         """Into how many parts the tiled kernel cuts K.  17 to 64 rows: more than one with a K so long, and so few
