@@ -182,3 +182,46 @@ def test_operands_that_are_refused(ops):
     assert call(80, 64, 96, 96, 64, parts=2) == -1            # parts without a place
     assert call(80, 64, 96, 96, 64, parts=3, partial=_ptr(out)) == -1      # more parts than steps
     assert call(0, 64, 96, 96, 64) == 0
+
+
+# The first product of a routed layer with its activation, in every tile: against 64 bits, an expert without a pair, one with several tiles,
+# slots that only fill a tile up, columns past a tile and no multiple of four, widths with half a step.
+@pytest.mark.parametrize("bm,width", [(64, 64), (64, 128), (64, 256), (128, 128), (128, 256)])
+@pytest.mark.parametrize("act", ["silu", "weighed", "relu2"])
+@pytest.mark.parametrize("inner,k", [(64, 64), (132, 96), (90, 224)])
+def test_sorted_products_with_their_activation(ops, bm, width, act, inner, k, monkeypatch):
+    experts, top, rows = 5, 2, 2 * bm + 9
+    gen = torch.Generator().manual_seed(inner + k)
+    first = torch.where(torch.arange(rows) < rows - 4, 2, 4)
+    chosen = torch.stack([first, (first + 1 + torch.arange(rows) % 2) % 4], 1).to(torch.int32)
+    chosen[3, 1] = -1                                         # a pair that is passed over
+    wide = (1 if act == "relu2" else 2) * inner
+    x, w = rand((rows, k + 8), k), rand((experts * wide, k + 16), inner, 0.2)
+    x[:, k:], w[:, k:] = float("nan"), float("nan")             # columns behind K are not read
+    weights = torch.rand((rows, top), generator=gen).cuda() + 0.5
+    slot_of, row_of, tile_expert = ops.expert_slots(chosen.cuda(), experts, bm)
+    monkeypatch.setattr(ops, "grouped_wide", width)
+    out = ops.grouped_act(x, row_of, tile_expert, bm, w, wide * (k + 16), inner, k, act, slot_of, weights)
+    slots = slot_of.cpu().view(rows, top)
+    for e in range(experts):
+        t, p = (chosen == e).nonzero(as_tuple=True)
+        if not len(t):
+            continue
+        z = x[t.cuda(), :k].double() @ w[e * wide:(e + 1) * wide, :k].double().t()
+        if act == "relu2":
+            want, parts = torch.relu(z) ** 2, float(z.abs().max()) ** 2
+        else:
+            a = weights[t.cuda(), p.cuda()].double()[:, None] if act == "weighed" else 1.0
+            gate, up = a * z[:, :inner], a * z[:, inner:]
+            want, parts = gate * torch.sigmoid(gate) * up, float(gate.abs().max() * up.abs().max())
+        got = out[slots[t, p].long().cuda()].double()
+        # Float sums and activation (2^-19 of the product of its factors), one rounding of the result.
+        assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -19 * parts + 4e-5 * float(want.abs().max())).all()), e
+
+
+def test_sorted_products_with_activation_leave_other_operands_to_the_two_kernels(ops, monkeypatch):
+    x, w = rand((64, 104), 1), rand((128, 104), 2)
+    tile_expert, row_of = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.arange(64, dtype=torch.int32, device="cuda")
+    assert ops.grouped_act(x, row_of, tile_expert, 64, w, 128 * 104, 64, 104, "silu") is None
+    monkeypatch.setattr(ops, "grouped_wide", -1)
+    assert ops.grouped_act(x, row_of, tile_expert, 64, w, 128 * 104, 64, 96, "silu") is None

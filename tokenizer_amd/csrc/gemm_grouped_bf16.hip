@@ -177,13 +177,21 @@ grouped_gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
 // Bound by the loads' way into LDS (128 x 256: 48 KB a step of 1,024 clocks of matrix work).  36 tiles of 128 slots over 3,584 x 18,944
 // and 9,472 x 3,584: 679 + 327 us, 921 and 955 TFLOP/s; 808 + 402 with rows that went through registers on their way to LDS (256 columns,
 // steps of 32), 1,094 + 500 in the kernel above.
-template <int BM, int BN, int STAGES, int WN_WAVES, typename OutT>
+// ACT: what becomes of the sums before they are stored.  GROUPED_SILU: an expert's W has N gate rows, then N up rows, and C[slot, :N] =
+// silu(gate) * up; GROUPED_WEIGHED: silu(w gate) * (w up), w = weights[p] of the pair p with slot_of[p] = slot, one of the `top` of the
+// slot's token; GROUPED_RELU2: max(z, 0)^2.  Gate and up rows lie in LDS sixteen by sixteen, so that a lane has both sums of a column.
+// (Two of eight experts of 9,472 on a width of 3,584, 2,048 tokens: product and activation 654 + 46 us, as one 640; whole passes of
+// that design 26.3 -> 25.5 ms.)
+enum { GROUPED_PLAIN = 0, GROUPED_SILU = 1, GROUPED_WEIGHED = 2, GROUPED_RELU2 = 3 };
+template <int BM, int BN, int STAGES, int WN_WAVES, int ACT, typename OutT>
 __global__ void __launch_bounds__(128 * WN_WAVES)
 grouped_gemm_ring_kernel(const bf16_t* __restrict__ A, int lda, const int* __restrict__ row_of,
                          const int* __restrict__ tile_expert, int n_tiles, const bf16_t* __restrict__ W, long expert_stride,
-                         int ldw, OutT* __restrict__ C, int ldc, int N, int K) {
+                         int ldw, OutT* __restrict__ C, int ldc, int N, int K, const int* __restrict__ slot_of,
+                         const float* __restrict__ weights, int top) {
   typedef RingTile<BM, BN, STAGES, 2, WN_WAVES> Ring;
-  constexpr int GROUP = 16;
+  constexpr bool GATED = ACT == GROUPED_SILU || ACT == GROUPED_WEIGHED;
+  constexpr int GROUP = 16, COLUMNS = GATED ? BN / 2 : BN;
   const int lane = threadIdx.x & 63, wave = wave_index();
   // The list up to its last tile with slots.
   int used = 0;
@@ -192,11 +200,11 @@ grouped_gemm_ring_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
     if (has) used = base + WAVE - __clzll(has);
   }
   used = __builtin_amdgcn_readfirstlane(used);
-  const int strips = (N + BN - 1) / BN, total = used * strips, per_chiplet = (total + 7) / 8;
+  const int strips = (N + COLUMNS - 1) / COLUMNS, total = used * strips, per_chiplet = (total + 7) / 8;
   const int turn = (int)(blockIdx.x >> 3), place = (int)(blockIdx.x & 7) * per_chiplet + turn;
   if (turn >= per_chiplet || place >= total) return;
   const int first = place / (GROUP * strips) * GROUP, high = min(GROUP, used - first), inside = place - first * strips;
-  const int tile = first + inside % high, m0 = tile * BM, n0 = inside / high * BN;
+  const int tile = first + inside % high, m0 = tile * BM, n0 = inside / high * COLUMNS;
   const int expert = scalar_int(tile_expert + tile);
   if (expert < 0) return;                                   // (a tile without slots among the others)
   uint32_t a_at[Ring::LA], w_at[Ring::LB];
@@ -206,22 +214,46 @@ grouped_gemm_ring_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
     a_at[i] = (uint32_t)(row_of ? max(row_of[slot], 0) : slot) * lda * 2 + Ring::piece_bytes(lane);
   }
 #pragma unroll
-  for (int i = 0; i < Ring::LB; ++i)
-    w_at[i] = (uint32_t)min(n0 + Ring::load_row(wave, lane, Ring::LB, i), N - 1) * ldw * 2 + Ring::piece_bytes(lane);
+  for (int i = 0; i < Ring::LB; ++i) {
+    const int row = Ring::load_row(wave, lane, Ring::LB, i);
+    const int n = GATED ? min(n0 + (row >> 5) * 16 + (row & 15), N - 1) + (row & 16 ? N : 0) : min(n0 + row, N - 1);
+    w_at[i] = (uint32_t)n * ldw * 2 + Ring::piece_bytes(lane);
+  }
+  const int r = lane & 15, g = lane >> 4;
+  float weight[Ring::MI];
+  if constexpr (ACT == GROUPED_WEIGHED) {
+#pragma unroll
+    for (int i = 0; i < Ring::MI; ++i) {
+      const int slot = m0 + wave / WN_WAVES * Ring::WM + 16 * i + r, token = row_of[slot];
+      weight[i] = 0.f;                                      // (a slot that only fills the tile up)
+      if (token >= 0)
+        for (int k = 0; k < top; ++k)
+          if (slot_of[token * top + k] == slot) weight[i] = weights[token * top + k];
+    }
+  }
   ring_floatx4 acc[Ring::MI][Ring::NI];
   Ring::run(A, a_at, W + (size_t)expert * expert_stride, w_at, K / 64, (K & 32) != 0, acc);
-  const int r = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int i = 0; i < Ring::MI; ++i) {
     OutT* row = C + (size_t)(m0 + wave / WN_WAVES * Ring::WM + 16 * i + r) * ldc;
 #pragma unroll
-    for (int j = 0; j < Ring::NI; ++j) {
-      const int n = n0 + wave % WN_WAVES * Ring::WN + 16 * j + 4 * g;
-      if (n + 3 < N && (ldc & 3) == 0) gg_store4(row + n, acc[i][j]);
+    for (int j = 0; j < Ring::NI; j += GATED ? 2 : 1) {
+      const int n = n0 + (GATED ? wave % WN_WAVES * (Ring::WN / 2) + 8 * j : wave % WN_WAVES * Ring::WN + 16 * j) + 4 * g;
+      ring_floatx4 v = acc[i][j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (ACT == GROUPED_SILU) v[e] = v[e] / (1.0f + __expf(-v[e])) * acc[i][j + 1][e];
+        if constexpr (ACT == GROUPED_WEIGHED) {
+          const float z = weight[i] * v[e];
+          v[e] = z / (1.0f + __expf(-z)) * (weight[i] * acc[i][j + 1][e]);
+        }
+        if constexpr (ACT == GROUPED_RELU2) { const float z = fmaxf(v[e], 0.f); v[e] = z * z; }
+      }
+      if (n + 3 < N && (ldc & 3) == 0) gg_store4(row + n, v);
       else
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (n + e < N) gg_store(row + n + e, acc[i][j][e]);
+          if (n + e < N) gg_store(row + n + e, v[e]);
     }
   }
 }
@@ -257,6 +289,21 @@ extern "C" int ta_expert_slots(const void* chosen, int n_entries, int top, int n
   return LAUNCH_STATUS();
 }
 
+// Which width: 64 columns (tiles of 64 slots) where even those give no compute unit a second workgroup; else 256 where their
+// rounds over the units, each 1.6 times as long, are fewer than those of 128.  Measured, us, 64 | 128 | 256 columns (and the general
+// kernel).  64 slots a tile: 12 tiles x 896 columns over 3,648 23 | 32 | 50 (31), 24 tiles 37 | 31 | 47 (42), 40 tiles 48 | 45 | 47 (62);
+// 12 tiles x 3,648 columns over 896 20 | 20 | 19 (20); 24 tiles x 3,584 columns over 9,472 261 | 215 | 243 (250), 68 tiles x 18,944
+// columns over 3,584 1,178 | 955 | 908 (1,340).  128 slots, 128 | 256 columns: 36 tiles x 18,944 over 3,584 795 | 679 (1,129), 36 x
+// 3,584 over 9,472 395 | 327 (502), 8 such tiles 132 | 171 (181); 36 x 896 over 3,648 42 | 58 (73); 18 x 4,480 over 1,536 61 | 62 (68).
+// The general kernel is left with a K that is no multiple of 32, one of 32, and matrices past 32-bit places.
+static int ring_width(int choice, int bm, int N, int expected) {
+  const int units = compute_units();
+  auto workgroups = [&](int width) { return (long)((N + width - 1) / width) * expected; };
+  auto rounds = [&](int width) { return (double)((workgroups(width) + units - 1) / units); };
+  if (choice > 0) return choice == 1 ? 256 : choice;
+  return bm == 64 && workgroups(64) <= units ? 64 : rounds(256) * 1.6 < rounds(128) ? 256 : 128;
+}
+
 // bm: 64 or 128 (the tile height the slots were made for).  C has n_tiles * bm rows.  expected: about how many of the tiles will
 // have slots (it only goes into the choice of kernel).  rows: how many A has.  choice: 0 = the expected fastest, -1 = the general kernel,
 // 64, 128 or 256 = the ring kernel with so many columns a tile wherever it can (64 columns: tiles of 64 slots; 128 in their place at
@@ -270,20 +317,11 @@ extern "C" int ta_grouped_gemm_bf16(const void* A, int rows, int lda, const void
 #define GO(BMV, BNV, BKV, TT)                                                                                          \
   grouped_gemm_bf16_kernel<BMV, BNV, BKV, TT><<<dim3((N + BNV - 1) / BNV, n_tiles), 256, 0, stream>>>(                 \
       (const bf16_t*)A, lda, (const int*)row_of, (const int*)tile_expert, (const bf16_t*)W, expert_stride, ldw, (TT*)C, ldc, N, K)
-#define RING(BMV, BNV, ST, WAVES, TT) grouped_gemm_ring_kernel<BMV, BNV, ST, WAVES, TT><<<blocks, 128 * WAVES, 0, stream>>>( \
-    (const bf16_t*)A, lda, (const int*)row_of, (const int*)tile_expert, n_tiles, (const bf16_t*)W, expert_stride, ldw, (TT*)C, ldc, N, K)
-  // Which width: 64 columns (tiles of 64 slots) where even those give no compute unit a second workgroup; else 256 where their
-  // rounds over the units, each 1.6 times as long, are fewer than those of 128.  Measured, us, 64 | 128 | 256 columns (and the general
-  // kernel).  64 slots a tile: 12 tiles x 896 columns over 3,648 23 | 32 | 50 (31), 24 tiles 37 | 31 | 47 (42), 40 tiles 48 | 45 | 47 (62);
-  // 12 tiles x 3,648 columns over 896 20 | 20 | 19 (20); 24 tiles x 3,584 columns over 9,472 261 | 215 | 243 (250), 68 tiles x 18,944
-  // columns over 3,584 1,178 | 955 | 908 (1,340).  128 slots, 128 | 256 columns: 36 tiles x 18,944 over 3,584 795 | 679 (1,129), 36 x
-  // 3,584 over 9,472 395 | 327 (502), 8 such tiles 132 | 171 (181); 36 x 896 over 3,648 42 | 58 (73); 18 x 4,480 over 1,536 61 | 62 (68).
-  // The general kernel is left with a K that is no multiple of 32, one of 32, and matrices past 32-bit places.
+#define RING(BMV, BNV, ST, WAVES, TT) grouped_gemm_ring_kernel<BMV, BNV, ST, WAVES, 0, TT><<<blocks, 128 * WAVES, 0, stream>>>( \
+    (const bf16_t*)A, lda, (const int*)row_of, (const int*)tile_expert, n_tiles, (const bf16_t*)W, expert_stride, ldw, (TT*)C, ldc, N, K, \
+    nullptr, nullptr, 0)
   const bool ring = choice >= 0 && K % 32 == 0 && K >= 64 && (long)(N - 1) * ldw + K < (1l << 31) && (long)rows * lda < (1l << 31);
-  const int units = compute_units();
-  auto workgroups = [&](int width) { return (long)((N + width - 1) / width) * expected; };
-  auto rounds = [&](int width) { return (double)((workgroups(width) + units - 1) / units); };
-  const int width = choice > 0 ? (choice == 1 ? 256 : choice) : bm == 64 && workgroups(64) <= units ? 64 : rounds(256) * 1.6 < rounds(128) ? 256 : 128;
+  const int width = ring_width(choice, bm, N, expected);
   if (width != 64 && width != 128 && width != 256) return -1;
   const int blocks = ((N + width - 1) / width * n_tiles + 7) / 8 * 8;
   const bool f32 = out_dtype == DT_F32;
@@ -315,5 +353,37 @@ extern "C" int ta_expert_combine(const void* rows, const void* slot_of, const vo
     expert_combine_kernel<bf16_t><<<blocks, 256, 0, stream>>>((const float*)rows, (const int*)slot_of, (const float*)weights,
                                                               top, (const bf16_t*)shared, (bf16_t*)out, hidden, total,
                                                               (const float*)shared_weight);
+  return LAUNCH_STATUS();
+}
+
+// The first product of a routed layer and its activation: C[slot, :inner] (bfloat16) = act over A's rows and the tile's expert, W_e as the
+// kernel's ACT says (1: [gate; up] rows, silu; 2: the same with weighted inputs, slot_of, weights [tokens, top] and row_of given; 3: inner rows,
+// max(z, 0)^2).  The other arguments as in `ta_grouped_gemm_bf16`.  -2: not these operands (the product and the activation one by one).
+extern "C" int ta_grouped_gemm_act(const void* A, int rows, int lda, const void* row_of, const void* tile_expert, int n_tiles, int bm,
+                                   const void* W, long expert_stride, int ldw, void* C, int inner, int K, int act, const void* slot_of,
+                                   const void* weights, int top, int expected, int choice, hipStream_t stream) {
+  if (n_tiles <= 0 || inner <= 0) return 0;
+  if (bm != 64 && bm != 128) return -1;
+  if (act < 1 || act > 3 || (act == GROUPED_WEIGHED && (!slot_of || !weights || !row_of || top <= 0))) return -1;
+  const long w_rows = (act == GROUPED_RELU2 ? 1l : 2l) * inner;
+  if (choice < 0 || (K & 31) || K < 64 || (lda & 7) || (ldw & 7) || (expert_stride & 7) || (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15) ||
+      (w_rows - 1) * ldw + K >= (1l << 31) || (long)rows * lda >= (1l << 31) || w_rows > 0x7fffffffL)
+    return -2;
+  const int width = ring_width(choice, bm, (int)w_rows, expected);
+  if (width != 64 && width != 128 && width != 256) return -1;
+  const int columns = act == GROUPED_RELU2 ? width : width / 2, blocks = ((inner + columns - 1) / columns * n_tiles + 7) / 8 * 8;
+#define RING(BMV, BNV, ST, WAVES, ACT) grouped_gemm_ring_kernel<BMV, BNV, ST, WAVES, ACT, bf16_t><<<blocks, 128 * WAVES, 0, stream>>>( \
+    (const bf16_t*)A, lda, (const int*)row_of, (const int*)tile_expert, n_tiles, (const bf16_t*)W, expert_stride, ldw, (bf16_t*)C, inner, \
+    inner, K, (const int*)slot_of, (const float*)weights, top)
+#define WIDTHS(ACT)                                                                                              \
+  {                                                                                                              \
+    if (bm == 128) { if (width == 256) RING(128, 256, 3, 4, ACT); else RING(128, 128, 4, 4, ACT); }              \
+    else if (width == 256) RING(64, 256, 4, 4, ACT);                                                             \
+    else if (width == 128) RING(64, 128, 3, 4, ACT);                                                             \
+    else RING(64, 64, 4, 2, ACT);                                                                                \
+  }
+  if (act == GROUPED_SILU) WIDTHS(GROUPED_SILU) else if (act == GROUPED_WEIGHED) WIDTHS(GROUPED_WEIGHED) else WIDTHS(GROUPED_RELU2)
+#undef WIDTHS
+#undef RING
   return LAUNCH_STATUS();
 }

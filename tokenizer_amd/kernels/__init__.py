@@ -155,7 +155,7 @@ class Ops:
                      "ta_sample_workspace_words", "ta_library_gemm_bf16", "ta_compute_units", "ta_read_stream",
                      "ta_embedding_streams", "ta_streams_step", "ta_token_shift", "ta_mlstm_scan", "ta_mlstm_chunked", "ta_head_norm_gate",
                      "ta_capped_gate", "ta_norm_add_rmsnorm", "ta_norm_rotate_store", "ta_differential_heads",
-                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_expert_combine",
+                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
@@ -169,6 +169,10 @@ class Ops:
                                                   ctypes.c_int, ctypes.c_void_p, ctypes.c_long, ctypes.c_int, ctypes.c_void_p,
                                                   ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                                   ctypes.c_void_p]
+        self.lib.ta_grouped_gemm_act.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
+                                                 ctypes.c_int, ctypes.c_void_p, ctypes.c_long, ctypes.c_int, ctypes.c_void_p,
+                                                 ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
+                                                 ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
         self.lib.ta_library_gemm_bf16.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 5 + [
             ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_void_p]
         self._workspaces: dict[int, torch.Tensor] = {}
@@ -967,6 +971,36 @@ class Ops:
                                                   int(expert_stride), weight.shape[1], _ptr(out), n_out, n_out, k,
                                                   _code(out_dtype), tiles if expected is None else int(expected), self.grouped_wide, self._stream()),
                     "grouped_linear")
+        return out
+
+    def grouped_act(self, x: torch.Tensor, row_of: torch.Tensor, tile_expert: torch.Tensor, bm: int, weight: torch.Tensor,
+                    expert_stride: int, inner: int, k: int, act: str, slot_of: torch.Tensor | None = None,
+                    weights: torch.Tensor | None = None, expected: int | None = None) -> torch.Tensor | None:
+        """The first product of a routed layer and its activation in one kernel: out [tiles * bm, inner] bfloat16.  W_e as in
+        `grouped_linear`, with `act` "silu" the gate rows, then as many up rows: silu(gate) * up; "weighed" the same of inputs
+        times the pair's weight (weights float32 [T, top], slot_of as `expert_slots` gave it): silu(w gate) * (w up); "relu2"
+        max(z, 0)^2.  The sums are not rounded in between.  None where the ring kernel does not take the operands."""
+        _dev(x, row_of, tile_expert, weight, slot_of, weights)
+        tiles = tile_expert.numel()
+        _need(x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.stride(1) == 1 and weight.is_contiguous(),
+              "bfloat16 operands with contiguous rows")
+        _need(x.shape[1] >= k and row_of.dtype == torch.int32 and row_of.numel() == tiles * bm and tile_expert.dtype == torch.int32,
+              "rows of x for every slot, row_of int32 [tiles bm]")
+        top = 0
+        if act == "weighed":
+            _need(weights.dtype == torch.float32 and weights.is_contiguous() and weights.dim() == 2 and slot_of.dtype == torch.int32
+                  and slot_of.numel() == weights.numel(), "slot_of int32 [T top], weights float32 [T, top]")
+            top = weights.shape[1]
+        if not self.use_ring or k % 8 or x.stride(0) % 8:
+            return None
+        out = torch.empty((tiles * bm, inner), dtype=torch.bfloat16, device=x.device)
+        status = self.lib.ta_grouped_gemm_act(
+            _ptr(x), x.shape[0], x.stride(0), _ptr(row_of), _ptr(tile_expert), tiles, bm, _ptr(weight), int(expert_stride),
+            weight.shape[1], _ptr(out), inner, k, {"silu": 1, "weighed": 2, "relu2": 3}[act], _ptr(slot_of), _ptr(weights), top,
+            tiles if expected is None else int(expected), self.grouped_wide, self._stream())
+        if status == -2:
+            return None
+        self._check(status, "grouped_act")
         return out
 
     def expert_combine(self, rows: torch.Tensor, slot_of: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None,

@@ -310,15 +310,21 @@ class RoutedExperts(FeedForward):
         bm = 128 if (pairs >= 2048 * max(1, self.n_experts // 8)
                      or (pairs > 64 * self.n_experts and tiles(128) * -(-wide // 256) >= 700)) else 64
         slot_of, row_of, tile_expert = ops.expert_slots(chosen, self.n_experts, bm)
-        gate_up = ops.grouped_linear(x, row_of, tile_expert, bm, self.w_gate_up, wide * hidden, wide, hidden, torch.bfloat16,
-                                     expected=tiles(bm))
-        act = torch.empty((gate_up.shape[0], inner), dtype=x.dtype, device=x.device)
-        if self.weigh_input:
-            ops.expert_gate_slots(gate_up, slot_of, weights, act)
-        elif self.gated:
-            ops.silu_gate(gate_up, act)
-        else:
-            ops.relu2(gate_up, act)
+        act = None
+        if hasattr(ops, "grouped_act"):                  # the first product with the activation behind it, where there is a kernel
+            kind = "weighed" if self.weigh_input else "silu" if self.gated else "relu2"
+            act = ops.grouped_act(x, row_of, tile_expert, bm, self.w_gate_up, wide * hidden, inner, hidden, kind,
+                                  slot_of, weights, expected=tiles(bm))
+        if act is None:
+            gate_up = ops.grouped_linear(x, row_of, tile_expert, bm, self.w_gate_up, wide * hidden, wide, hidden, torch.bfloat16,
+                                         expected=tiles(bm))
+            act = torch.empty((gate_up.shape[0], inner), dtype=x.dtype, device=x.device)
+            if self.weigh_input:
+                ops.expert_gate_slots(gate_up, slot_of, weights, act)
+            elif self.gated:
+                ops.silu_gate(gate_up, act)
+            else:
+                ops.relu2(gate_up, act)
         rows = ops.grouped_linear(act, None, tile_expert, bm, self.w_down, inner, hidden, inner, torch.float32,
                                   expected=tiles(bm))
         shared = None
