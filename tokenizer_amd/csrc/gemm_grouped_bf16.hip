@@ -180,7 +180,7 @@ grouped_gemm_bf16_kernel(const bf16_t* __restrict__ A, int lda, const int* __res
 // ACT: what becomes of the sums before they are stored.  GROUPED_SILU: an expert's W has N gate rows, then N up rows, and C[slot, :N] =
 // silu(gate) * up; GROUPED_WEIGHED: silu(w gate) * (w up), w = weights[p] of the pair p with slot_of[p] = slot, one of the `top` of the
 // slot's token; GROUPED_RELU2: max(z, 0)^2.  Gate and up rows lie in LDS sixteen by sixteen, so that a lane has both sums of a column.
-// (Two of eight experts of 9,472 on a width of 3,584, 2,048 tokens: product and activation 654 + 46 us, as one 640; whole passes of
+// (Two of eight experts of 9,472 on a width of 3,584, 2,048 tokens: product and activation 654 + 30 us, as one 649; whole passes of
 // that design 26.3 -> 25.5 ms.)
 enum { GROUPED_PLAIN = 0, GROUPED_SILU = 1, GROUPED_WEIGHED = 2, GROUPED_RELU2 = 3 };
 template <int BM, int BN, int STAGES, int WN_WAVES, int ACT, typename OutT>
