@@ -4,7 +4,7 @@ import ctypes
 import pytest
 import torch
 
-from tokenizer_amd.kernels import PendingSum, _ptr, get_ops
+from tokenizer_amd.kernels import KernelError, PendingSum, _ptr, get_ops
 
 pytestmark = pytest.mark.gpu
 TILES = [(64, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 192), (256, 256)]
@@ -225,3 +225,43 @@ def test_sorted_products_with_activation_leave_other_operands_to_the_two_kernels
     assert ops.grouped_act(x, row_of, tile_expert, 64, w, 128 * 104, 64, 104, "silu") is None
     monkeypatch.setattr(ops, "grouped_wide", -1)
     assert ops.grouped_act(x, row_of, tile_expert, 64, w, 128 * 104, 64, 96, "silu") is None
+
+
+# A product whose parts the grouped norms add themselves: rows of one piece a thread and of several, the last ones partly filled, a number of
+# parts that is no multiple of the four asked for at a time, rows picked out, and rows that only the general kernel takes (40 in 4 groups of
+# ten, 5,120).  float results: 2^-24 of the sums' size for each of the few dozen roundings; bfloat16 ones 2^-8 of their own size more.
+@pytest.mark.parametrize("hidden,post_groups,groups", [(1536, 2, 2), (1024, 1, 4), (1028, 257, 1), (2048, 8, 1), (4096, 2, 1024), (896, 2, 2),
+                                                       (40, 4, 4), (5120, 4, 2)])
+@pytest.mark.parametrize("parts", [1, 2, 4, 5, 11])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_grouped_norms_add_the_parts_of_a_product(ops, hidden, post_groups, groups, parts, dtype):
+    rows = 5
+    gen = torch.Generator(device="cuda").manual_seed(hidden + parts)
+    draw = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    stream, slabs = draw(rows, hidden), draw(parts, rows, hidden)
+    behind, weight = 1 + 0.3 * draw(hidden), 1 + 0.3 * draw(hidden)
+
+    def norm(v, w, count, eps):
+        runs = v.reshape(len(v), count, -1)
+        return (runs / (runs.square().mean(-1, keepdim=True) + eps).sqrt()).reshape(v.shape) * w.double()
+    pending = lambda: PendingSum(ops, slabs, None, dtype)
+    # (The general kernel takes the product as it comes without parts: added, and rounded to its own type.)
+    general = hidden % (4 * post_groups) or hidden % (4 * groups) or hidden > 4096
+    product = pending().resolve().double() if general else slabs.double().sum(0)
+    x = stream.double() + norm(product, behind, post_groups, 1e-5)
+    y = norm(x, weight, groups, 1e-3)
+    near = lambda got, want: bool(((got.double() - want).abs() <= 2e-6 * want.abs().max()
+                                   + (2.0 ** -8 * want.abs() if got.dtype == torch.bfloat16 else 0.0)).all())
+    args = dict(post_groups=post_groups, groups=groups)
+    kept, out = stream.clone(), torch.empty(rows, hidden, dtype=dtype, device="cuda")
+    ops.norm_add_rmsnorm(kept, pending(), behind, 1e-5, weight, 1e-3, out, **args)
+    assert near(kept, x) and near(out, y)
+    again, same = stream.clone(), torch.empty_like(out)
+    ops.norm_add_rmsnorm(again, pending(), behind, 1e-5, None, 0.0, same, **args)              # the sum itself
+    assert torch.equal(again, kept) and near(same, x)
+    pick = torch.tensor([4, 0], dtype=torch.int32, device="cuda")
+    again, some = stream.clone(), torch.empty(2, hidden, dtype=dtype, device="cuda")
+    ops.norm_add_rmsnorm(again, pending(), behind, 1e-5, weight, 1e-3, some, pick, store_residual=False, **args)
+    assert torch.equal(again, stream) and torch.equal(some, out[[4, 0]])
+    with pytest.raises(KernelError):                                                          # slabs of other rows
+        ops.norm_add_rmsnorm(kept[:3].contiguous(), pending(), behind, 1e-5, weight, 1e-3, out[:3], **args)

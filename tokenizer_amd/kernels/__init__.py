@@ -159,7 +159,7 @@ class Ops:
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
-                     "ta_rotation_table", "ta_head_norm_rotate_store", "ta_group_norm_add", "ta_relu_gate",
+                     "ta_rotation_table", "ta_head_norm_rotate_store", "ta_group_norm_add", "ta_group_norm_add_parts", "ta_relu_gate",
                      "ta_talking_attention_generic", "ta_talking_decode_bf16", "ta_talking_prefill_bf16",
                      "ta_talking_prefill_parts", "ta_retention_scan", "ta_retention_chunked", "ta_temper_store", "ta_add_slabs_rmsnorm", "ta_experts_few", "ta_experts_few_shared_parts",
                      "ta_fused_qk_temper",
@@ -650,8 +650,30 @@ class Ops:
         off; out = x / sqrt(mean(x^2) + eps) * weight, or x itself without `weight`.  `post_groups`, `groups`: the norm on
         delta (on x) is over so many equal runs of neighbours, each divided by its own root mean square.
 
-        residual float32 [T, H]; delta [T, H] float32 or bfloat16; weights float32 [H]; rows int32 or None; out
-        [rows, H] in delta's dtype or float32."""
+        residual float32 [T, H]; delta [T, H] float32 or bfloat16, or a product still in parts (`PendingSum`: norms over
+        groups add them in the same kernel); weights float32 [H]; rows int32 or None; out [rows, H] in delta's dtype or
+        float32."""
+        if isinstance(delta, PendingSum):
+            if (post_groups != 1 or groups != 1) and delta.bias is None:
+                n_rows, hidden = residual.shape[0] if rows is None else rows.numel(), residual.shape[1]
+                _dev(residual, delta.partial, post_weight, weight, out, rows)
+                _need(residual.dtype == torch.float32 and residual.is_contiguous(), "the residual stream is float32")
+                _need(tuple(out.shape) == (n_rows, hidden) and out.is_contiguous(), "norm output shape")
+                _need(delta.shape == tuple(residual.shape) and delta.partial.is_contiguous(), "delta must match the residual's shape")
+                _need(out.dtype in (delta.dtype, torch.float32), "out has delta's dtype or float32")
+                for vector in (post_weight, weight):
+                    _need(vector is None or (vector.dtype == torch.float32 and vector.numel() == hidden), "norm weights are float32 [H]")
+                _need(rows is None or (rows.dtype == torch.int32 and not store_residual), "a row subset (int32) never stores the residual")
+                _need(post_groups > 0 and groups > 0 and hidden % post_groups == 0 and hidden % groups == 0,
+                      "the groups are equal parts of the row")
+                status = self.lib.ta_group_norm_add_parts(
+                    _ptr(residual), _ptr(delta.partial), delta.partial.shape[0], residual.shape[0], _ptr(post_weight),
+                    ctypes.c_float(post_eps), post_groups, _ptr(weight), ctypes.c_float(eps), groups, _ptr(out), _ptr(rows), n_rows,
+                    hidden, int(store_residual), _code(out.dtype), self._stream())
+                if status != -2:              # -2: rows that only the general kernel takes
+                    self._check(status, "group_norm_add")
+                    return out
+            delta = delta.resolve()
         _dev(residual, delta, post_weight, weight, out, rows)
         hidden = residual.shape[1]
         n_rows = residual.shape[0] if rows is None else rows.numel()
@@ -1475,6 +1497,7 @@ class Ops:
     talking_workgroups = 512      # what the single tokens' split of the keys aims at
 
     # --------------------------------------------------------------------- linear
+    takes_pending_groups = True   # `norm_add_rmsnorm` over groups takes a product still in parts as its delta
     takes_pending = True      # `linear(pending=True)` and `add_rmsnorm` with a `PendingSum` exist here
 
     def linear(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,

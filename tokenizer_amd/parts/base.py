@@ -191,8 +191,9 @@ class Block:
 
 
 class NormedDelta:
-    """What a sub-layer that is normalised behind itself hands on: its output `rows` [T, H] (compute dtype) still to
-    be brought to unit RMS, scaled by `weight` (float32 [H]) and added to the stream.  A norm of the form
+    """What a sub-layer that is normalised behind itself hands on: its output `rows` [T, H] (compute dtype, or a product
+    still in parts, which the kernel library's `norm_add_rmsnorm` adds up) still to be brought to unit RMS, scaled by
+    `weight` (float32 [H]) and added to the stream.  A norm of the form
     x / sqrt(mean(x^2) + eps) * w takes it as its delta and does all of that in its own kernel
     (`ops.norm_add_rmsnorm`); for anyone else `resolve()` gives the sum's term as a float32 tensor.
 
@@ -218,7 +219,7 @@ class NormedDelta:
     def resolve(self) -> torch.Tensor:
         if self.side is not None:
             raise ValueError("a term with an addition behind it that reads the stream cannot stand alone: hand it to a norm")
-        zero = torch.zeros((self.rows.shape[0], self.rows.shape[1]), dtype=torch.float32, device=self.rows.device)
+        zero = torch.zeros((self.rows.shape[0], self.rows.shape[1]), dtype=torch.float32, device=self.weight.device)
         return self.join(zero, None, 0.0, torch.empty_like(zero), store_residual=False)
 
 

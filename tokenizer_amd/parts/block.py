@@ -199,7 +199,7 @@ class _TokenInput:
         has none for these sizes."""
         block = self.block
         run = getattr(block.runtime.ops, "norm_side_norm", None)
-        if run is None or out.dtype != delta.rows.dtype:
+        if run is None or out.dtype != delta.rows.dtype or not isinstance(delta.rows, torch.Tensor):
             return None
         return run(residual, delta.rows, delta.weight, delta.eps, block.side_gate, block.side_proj, block.side_norm,
                    block.eps, block.side_table, self.token_ids, block.side_offset, block.side_dim, weight, eps, out, rows)
@@ -272,6 +272,11 @@ class PostNormBlock(Block):
             if part is None:
                 continue
             x = self._input(residual, delta)
-            out = part.forward(x, ctx, cache) if part is self.mixer else part.forward(x, ctx)
+            if part is self.mixer:
+                out = part.forward(x, ctx, cache)
+            else:
+                # (Norms over groups add a product's parts in their own kernel; the others would need one for the addition.)
+                in_parts = norm.groups > 1 and getattr(ops, "takes_pending_groups", False)
+                out = getattr(part, "forward_in_parts", part.forward)(x, ctx) if in_parts else part.forward(x, ctx)
             delta = NormedDelta(ops, out, weight, norm.eps, groups=norm.groups)
         return delta

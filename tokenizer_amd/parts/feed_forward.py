@@ -73,6 +73,11 @@ class GatedDense(FeedForward):
     def forward(self, x, ctx):
         return self._run(x, pending=False)
 
+    def forward_in_parts(self, x, ctx):
+        """As `forward`, but where the last product's K is cut over workgroups its parts are left for the next norm.  From
+        an inner width of 2,048 on: below it the cut of 65 to 256 rows is another one while a graph is recorded."""
+        return self._run(x, pending=self.w_down.shape[1] >= 2048)
+
     def _run(self, x, pending: bool):
         ops = self.runtime.ops
         if self.named:
