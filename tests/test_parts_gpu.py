@@ -135,6 +135,29 @@ def test_attention_mixer_alone(dtype, geometry):
         at += n
 
 
+@pytest.mark.parametrize("hidden", [100, 44])
+@pytest.mark.parametrize("lengths", [[9, 3], [37, 16], [65, 40]])
+def test_attention_mixer_of_a_width_that_is_no_multiple_of_eight(hidden, lengths):
+    """Heads that the projections with rotation and store take, rows that none of them does (the step runs through the
+    product that fills K up): few rows, a few dozen, more than 64."""
+    from tokenizer_amd.parts import MIXERS, LayerCache, MixerSpec, PositionSpec
+    n_q, n_kv, d, dtype = 4, 2, 32, torch.bfloat16
+    spec = MixerSpec("gqa_attention", hidden, n_q, n_kv, d, qkv_bias=True, position=PositionSpec("rope_half_split", d, 10000.0, 128))
+    mixer_cls, tensors = MIXERS.get("gqa_attention"), attention_tensors(n_q, n_kv, d, hidden, 10)
+    mixer = mixer_cls(spec, {k: (v.to(dtype) if v.dim() == 2 else v).cuda() for k, v in tensors.items()}, runtime(dtype))
+    manager, pools, ctx = context_for([mixer_cls.cache_need(spec)], lengths, dtype)
+    k_pages, v_pages = pools.layer_pages(0)
+    x = rand((sum(lengths), hidden), 20).to(dtype)
+    out = mixer.forward(x.cuda(), ctx, LayerCache(group=0, k_pages=k_pages, v_pages=v_pages)).float().cpu()
+    cos, sin = plain.rope_tables(10000.0, d, 128)
+    named = {f"a.{k}": v for k, v in tensors.items()}
+    at = 0
+    for n in lengths:
+        want = plain.self_attention(x[at:at + n].float(), named, "a", n_q, n_kv, d, cos, sin, list(range(n)), None)
+        close(out[at:at + n], want, dtype)
+        at += n
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows", [5, 130])
 def test_feed_forward_alone(dtype, rows):
