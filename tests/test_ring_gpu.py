@@ -170,6 +170,13 @@ def test_the_choice_of_kernel_does_not_change_the_product(ops, m, n, k, monkeypa
             assert float((got[fine].double() - want[fine].double()).abs().max()) <= limit * float(want[fine].double().abs().max())
 
 
+# The capped gate's three numbers may come as any sequence, with few rows and with many.
+@pytest.mark.parametrize("m", [9, 40, 300])
+def test_numbers_of_the_capped_gate_as_a_list(ops, m):
+    x, w = rand((m, 96), m), rand((64, 96), 2, 0.2)
+    assert torch.equal(ops.linear_silu_gate(x, w, act=[1.702, 2.0, 1.0]), ops.linear_silu_gate(x, w, act=(1.702, 2.0, 1.0)))
+
+
 def test_operands_that_are_refused(ops):
     x, w, out = rand((80, 96), 1), rand((64, 96), 2), torch.empty((80, 64), dtype=torch.bfloat16, device="cuda")
     call = lambda m, n, k, lda, ldc, parts=1, partial=None, xp=None: ops.lib.ta_gemm_ring(

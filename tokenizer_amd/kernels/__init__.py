@@ -1756,10 +1756,11 @@ class Ops:
         if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and self._gated_to_ring(m, inner, x.shape[1]):
             _need(x.is_cuda and weight.is_cuda and x.dim() == 2 and x.shape[1] == weight.shape[1], "linear shapes do not fit")
             _need(x.stride(1) == 1 and weight.is_contiguous(), "linear operands must have contiguous rows")
-            alpha, limit, shift = act if isinstance(act, tuple) else (0.0, 0.0, 0.0)
-            _need(not isinstance(act, str) or act in ("gelu_tanh", "relu"), f"unknown gated activation {act!r}")
+            named = act is None or isinstance(act, str)
+            _need(not named or act in (None, "gelu_tanh", "relu"), f"unknown gated activation {act!r}")
+            alpha, limit, shift = (0.0, 0.0, 0.0) if named else act
             status = self.lib.ta_gemm_ring_gated(_ptr(x), _ptr(weight), _ptr(out), m, inner, x.shape[1], x.stride(0),
-                                                 4 if isinstance(act, tuple) else {None: 1, "gelu_tanh": 2, "relu": 3}[act],
+                                                 {None: 1, "gelu_tanh": 2, "relu": 3}[act] if named else 4,
                                                  ctypes.c_float(alpha), ctypes.c_float(limit), ctypes.c_float(shift), -1,
                                                  self._stream())
             if status != -2:                  # -2: rows that are not aligned, matrices past 32-bit places
