@@ -56,6 +56,23 @@ def test_split_products_of_numbers_that_cannot_be_split(ops, odd, m, k):
     assert bool(((split.double() - want)[fine].abs() <= 2.0 ** -22 * size).all())
 
 
+# Whole rows of small numbers, of either operand, down to those that are no normal floats any more: against 64 bits relative to the row's
+# own sums, whose terms the other operand lifts back to ordinary sizes.  Float sums of K products: 2^-22 of the sum of their sizes is
+# some sixteen times a rounding; operands of which a bit was lost would miss it from 1e-35 on.
+@pytest.mark.parametrize("size", [1e-30, 1e-34, 1e-36, 1e-38, 1e-41])
+@pytest.mark.parametrize("m,n,k", [(70, 96, 200), (260, 140, 1024)])
+def test_split_products_of_small_numbers(ops, size, m, n, k):
+    x, w = rand((m, k), m), rand((n, k), n)
+    x[::2] *= size
+    w[1::2] *= size
+    x[::3] *= 1e16
+    w[::3] *= 1e16
+    split, _ = both_ways(ops, x, w)
+    want, terms = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    # (Below the smallest normal float there are only multiples of 2^-149: up to eight parts of K, each within half of one.)
+    assert bool(((split.double() - want).abs() <= 2.0 ** -22 * terms + 2.0 ** -146).all())
+
+
 def test_split_products_repeat_bit_for_bit(ops):
     x, w = rand((300, 896), 5), rand((1152, 896), 6)
     first = ops.linear(x, w)

@@ -165,12 +165,16 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 
 // The same products on the bfloat16 instructions, sixteen times as fast as the float ones, without losing anything of the operands: a float
 // is the sum of three bfloat16 numbers (its nearest one, that of the rest, that of what then is left: 8 + 8 + 8 bits and the signs), and
-// of the nine products of two such sums the six largest are summed, smallest first (a1 b3, a3 b1, a2 b2, a1 b2, a2 b1, a1 b1); the
-// three left out are at most 2^-26 of |a b| each.  Products of bfloat16 numbers are exact, the sums are floats, and an instruction rounds
-// a sum of sixteen products where the float one rounds after two: against 64 bits the relative error (2-norm) is 2.1e-7 to 7.7e-7
-// over 17 to 2,048 rows and K of 896 to 4,864, 10 to 20 % below the float instructions' at every size measured.
+// of the nine products of two such sums the six largest are summed, smallest first (a1 b3, a3 b1, a2 b2, a1 b2, a2 b1, a1 b1); of the
+// three left out a2 b3 and a3 b2 are at most 2^-25 of |a b| each, a3 b3 2^-34.  Products of bfloat16 numbers are exact, the sums are floats, and
+// an instruction rounds a sum of sixteen products where the float one rounds after two: against 64 bits the relative error (2-norm) is
+// 2.1e-7 to 7.7e-7 over 17 to 2,048 rows and K of 896 to 4,864, 10 to 20 % below the float instructions' at every size measured.
+// Operands are split times 2^24 and sums stored times 2^-48: every float, down to the smallest, then is a multiple of 2^-125, so that none of
+// the three numbers is too small for a bfloat16 (split as they are, operands below 2^-110 lose their last bits: rows of size 1e-36 were
+// off by 2.7e-5, of 1e-38 by 2.7e-3).  The multiplication costs 1 to 3 % (1,280 rows of 9,728 columns over 896 125 -> 128 us, of
+// 896 over 4,864 73.5 -> 76.5; 64 rows of 151,936 over 896 156 -> 159); ordinary operands' results are the same bits.
 // A sum that is no finite number sends its workgroup back over the tile with the float instructions, whose result takes its place:
-// infinities have no rest to split off, and numbers past the largest bfloat16 none either.
+// infinities have no rest to split off, and numbers past the largest bfloat16 (times 2^24: from 2^103 on, sums from 2^79) none either.
 // The splitting is done once a tile and step, on the way from registers to LDS: three planes of rows of 64 bytes, whose four pieces are
 // XOR-swizzled by a quarter of the row (by half of it the reads run at 0.9 of LDS's rate, by the row itself at half).  One buffer: three workgroups share a compute unit, so that one splits while another multiplies.
 // AHEAD steps' rows are on their way to registers.  Bound by the matrix cores (1,536 clocks a step of 32 at 128 x 128, six times the work of a
@@ -224,7 +228,9 @@ gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, 
   };
   const int put_at = row_in * ROW + (((piece >> 1) ^ ((row_in >> 2) & 3)) << 4) + (piece & 1) * 8;   // (rows 32 apart are swizzled alike)
   auto put = [&](const f32x4& v, int at) {
-    f32x4 rest = v;
+    f32x4 rest;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rest[e] = v[e] * 0x1p24f;
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       split_bf16x4 near;
@@ -292,8 +298,10 @@ gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, 
 #pragma unroll
     for (int j = 0; j < QN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
+      for (int e = 0; e < 16; ++e) {
         if (!(fabsf(acc[i][j][e]) < INFINITY)) odd |= 1ull << ((i * QN + j) * 16 + e);
+        acc[i][j][e] *= 0x1p-48f;
+      }
   f32_tile_store<BM, BN>(t, bias, C, M, N, ldc, partial, acc);
   if (!__syncthreads_or(odd != 0)) return;
   f32_tile_sums<BM, BN, 1>(t, A, W, M, N, K, lda, 1, lds.rows, acc);
