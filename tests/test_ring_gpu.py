@@ -62,6 +62,15 @@ def test_products_in_parts_of_every_tile(ops, tile, k, parts):
     assert close(out, want + bias.double(), k, False)
 
 
+# Parts are worth their trip to the norm where a whole K would be a long walk of few tiles, and not where the tiles fill the chip.
+def test_how_many_parts_a_product_is_cut_into(ops):
+    parts = ops.lib.ta_gemm_ring_parts
+    for m, n, k in ((700, 1536, 1536), (850, 1536, 1536), (600, 2048, 1536), (700, 2048, 2048), (700, 1024, 2816), (1024, 768, 3072)):
+        assert parts(m, n, k, 1) == 1, (m, n, k)
+    for m, n, k in ((64, 1536, 8960), (130, 1536, 1536), (300, 896, 4864), (512, 1536, 8960), (2048, 1536, 8960)):
+        assert parts(m, n, k, 1) > 1, (m, n, k)
+
+
 # (The two after the tiles: large tiles in front, small ones behind, as many columns in either.)
 @pytest.mark.parametrize("tile", range(1, len(TILES) + 2))
 @pytest.mark.parametrize("act", [None, "gelu_tanh", "relu", (1.702, 2.0, 1.0)])

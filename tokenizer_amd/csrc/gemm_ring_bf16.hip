@@ -183,10 +183,11 @@ qkv_ring_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, cons
 
 // The tiles there are, and what a product costs with each, in microseconds on a device of 256 compute units:
 //   start + rounds * (fixed + steps * step), rounds of workgroups over the compute units, steps of 64 of K,
-// but no less than the weights' trip from memory, and on top the result's (parts are written, and read by whoever adds them).
+// but no less than the weights' trip from memory, and on top the result's (parts are written, and read by whoever adds them: the norm
+// that follows, or a kernel of its own).
 // Fitted to 5,700 timed products (17 to 4,096 rows, the Qwen2.5 models' matrices at 0.5B, 1.5B and 7B sizes, one to ten parts, plain and
-// gated, weights from memory); the tile and parts with the lowest cost are on average 3 % slower than the fastest of all, 30 % at worst
-// (long K, fewer than 100 rows).
+// gated, weights from memory), the price of parts of more than 64 rows to 620 more of 24 matrices of widths of 512 to 5,504: the tile and parts
+// with the lowest cost are on average 1.5 % slower than the fastest of all, 20 % at worst.
 struct RingShape { int bm, bn; double start, fixed, step; };
 static const RingShape RING_SHAPES[] = {
   {64, 64, 2.06, 0.58, 0.232}, {64, 128, 2.37, 0.62, 0.376}, {64, 256, 0.99, 3.08, 0.627}, {128, 128, 0.39, 3.73, 0.513},
@@ -211,7 +212,9 @@ static RingPlan ring_plan(long M, long N, long K, bool gated, bool pending, int 
       // (Where the weights' trip is what counts, the cheaper tile reads the rows less often: 65 rows x 151,936 over 1,536 133 us in 64 x 256
       // tiles, 113 in 128 x 256 ones.)
       cost = cost < weights ? weights + 0.15 * cost : cost + 0.15 * weights;
-      cost += s == 1 ? M * N * 2 / 8e6 : s * (double)M * N * 4 / 4e6 + (pending ? 0.0 : 4.0);
+      if (s == 1) cost += M * N * 2 / 8e6;
+      else if (M <= 64) cost += s * (double)M * N / 1e6 + (pending ? 0.0 : 4.0);
+      else cost += s * (double)M * N / 0.8e6 + (pending ? 1.0 : 2.0);
       if (cost < best.cost) best = {shape, s, cost, 0};
     }
   }
