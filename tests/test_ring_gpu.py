@@ -71,6 +71,22 @@ def test_how_many_parts_a_product_is_cut_into(ops):
         assert parts(m, n, k, 1) > 1, (m, n, k)
 
 
+# Results of few tiles and long K go to the ring kernel, large results to the library; float results, which it does not give, never do.
+def test_which_products_of_many_rows_are_whose(ops):
+    def ring(m, n, k, dtype=torch.bfloat16, pending=False):
+        return ops._to_ring(m, n, k, k, dtype, pending)
+    for m, n, k in ((65, 512, 512), (512, 1536, 1536), (2048, 896, 896), (2048, 896, 4864), (400, 4096, 4096), (2048, 3584, 18944), (2048, 1536, 8960)):
+        assert ring(m, n, k, pending=True), (m, n, k)
+    for m, n, k in ((2048, 1536, 1536), (2048, 2560, 2560), (3000, 4096, 11008), (2600, 3584, 18944), (4096, 896, 896), (4096, 1152, 896)):
+        assert not ring(m, n, k, pending=True), (m, n, k)
+    for m, n, k in ((512, 1152, 896), (1024, 2048, 1536), (512, 1536, 8960), (2048, 1536, 8960)):
+        assert ring(m, n, k), (m, n, k)
+    for m, n, k in ((1600, 1536, 4480), (512, 4608, 3584), (300, 4096, 4096), (4096, 896, 896)):
+        assert not ring(m, n, k), (m, n, k)
+    assert ring(6000, 4096, 4096, torch.float32) and ring(4100, 32768, 1024, torch.float32)
+    assert not ring(512, 1536, 80) and not ring(512, 1534, 1536)
+
+
 # (The two after the tiles: large tiles in front, small ones behind, as many columns in either.)
 @pytest.mark.parametrize("tile", range(1, len(TILES) + 2))
 @pytest.mark.parametrize("act", [None, "gelu_tanh", "relu", (1.702, 2.0, 1.0)])
