@@ -87,6 +87,13 @@ def test_which_products_of_many_rows_are_whose(ops):
     assert not ring(512, 1536, 80) and not ring(512, 1534, 1536)
 
 
+def test_which_gated_products_are_whose(ops):
+    for m, inner, k in ((33, 4864, 896), (64, 8960, 1536), (65, 4864, 896), (512, 4864, 896), (2048, 8960, 1536), (2048, 18944, 3584), (400, 18944, 3584)):
+        assert ops._gated_to_ring(m, inner, k), (m, inner, k)
+    for m, inner, k in ((32, 4864, 896), (64, 2432, 896), (64, 8192, 2048), (64, 18944, 3584), (224, 18944, 3584), (300, 11008, 4096), (800, 11008, 4096)):
+        assert not ops._gated_to_ring(m, inner, k), (m, inner, k)
+
+
 # (The two after the tiles: large tiles in front, small ones behind, as many columns in either.)
 @pytest.mark.parametrize("tile", range(1, len(TILES) + 2))
 @pytest.mark.parametrize("act", [None, "gelu_tanh", "relu", (1.702, 2.0, 1.0)])

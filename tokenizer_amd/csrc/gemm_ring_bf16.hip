@@ -349,6 +349,19 @@ extern "C" int ta_gemm_ring_parts(int M, int N, int K, int pending) {
   return ring_plan(M, N, K, false, pending != 0, 1, RING_MOST_PARTS).parts;
 }
 
+// Whether the gated product of more than 64 rows (N columns of the result) is expected to be faster than the library's product and the
+// activation kernel: their multiplications at 1,330 TFLOP/s, part of the weights' trip, the sums' trip to memory and back, and 18 us for what
+// two launches cost.  Fitted to 314 products of 65 to 5,000 rows and matrices of 2 to 141 million elements: with the ring kernel wherever this
+// says so they take 0.836 of the other way's time (the faster of the two each time: 0.833), 10 of them 3 % more and the worst 11 %; with
+// it from 225 rows on, whatever the size, 0.840, 21 and 18 %.  (Us, library and activation | ring: 512 rows, inner 4,864 over 896 23.1 | 18.1;
+// 2,048 rows 59 | 45, 8,960 over 1,536 138 | 112, 18,944 over 3,584 557 | 468, 11,008 over 4,096 338 | 301; and the other way 300 rows, 11,008 over
+// 4,096 75 | 88, 800 rows 143 | 171, 300 rows, 13,824 over 5,120 104 | 119.)
+extern "C" int ta_gemm_ring_gated_pays(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K < 64) return 0;
+  const double other = 18.0 + 0.75 * 4e-9 * M * N * K + 0.4 * 4.0 * N * K / 5.2e6 + 1.5e-6 * M * N;
+  return ring_plan(M, N, K, true, false, 1, 1).cost <= other;
+}
+
 // out[M, N] = act(A Wg^T) * (A Wu^T), W = [Wg; Wu] of 2 N rows.  act: 1 silu, 2 gelu_tanh, 3 relu, 4 the capped gate of (alpha, limit, shift).
 // shape: a tile of RING_SHAPES, RING_TAILED for 128 x 256 and 64 x 128, + 1 for 256 x 256 and 128 x 128, or -1 for the cheapest.  -2: not these
 // operands.

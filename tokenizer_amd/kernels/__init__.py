@@ -155,7 +155,7 @@ class Ops:
                      "ta_sample_workspace_words", "ta_library_gemm_bf16", "ta_compute_units", "ta_read_stream",
                      "ta_embedding_streams", "ta_streams_step", "ta_token_shift", "ta_mlstm_scan", "ta_mlstm_chunked", "ta_head_norm_gate",
                      "ta_capped_gate", "ta_norm_add_rmsnorm", "ta_norm_rotate_store", "ta_differential_heads",
-                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
+                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_gated_pays", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
@@ -1796,19 +1796,26 @@ class Ops:
             return out
         return self.silu_gate(self.linear(x, weight), out, act=act)
 
-    RING_GATED_WEIGHT = 2 ** 26    # joined gate and up elements from which ...
-    RING_GATED_ROWS = 224          # ... the library's product and the activation kernel take up to so many rows
-    RING_GATED_FROM = 32           # the rows from which the ring kernel takes the smaller ones
+    RING_GATED_FROM = 32           # gated products of more rows than that: the ring kernel, up to 64 rows from an eighth to half of ...
+    RING_GATED_WEIGHT = 2 ** 26    # ... so many joined gate and up elements, up to ...
+    RING_GATED_ROWS = 224          # ... so many rows of fewer than them, and wherever else its launcher expects it to be the faster way
 
     def _gated_to_ring(self, m: int, inner: int, k: int) -> bool:
-        """Whether a gated bfloat16 product goes to the ring kernel, sums and activation in one.  Us, product and activation before
-        (the weight-streaming kernel up to 64 rows, the library above) | ring: 64 rows, inner 4,864 over 896 12.6 | 10.9, 512 rows
-        23.1 | 18.1, 2,048 rows 59 | 45; 512 rows, 8,960 over 1,536 43 | 42, 2,048 rows 138 | 112; 300 rows, 18,944 over 3,584 120 | 108,
-        512 rows 149 | 136, 2,048 rows 557 | 468, 4,096 rows 934 | 899, but 64 rows 62 | 70, 192 rows 83 | 91: large weights of few rows
-        are a stream that tiles of 128 columns do not share evenly.  32 rows, 4,864 over 896: 10.1 | 9.9, 17 rows 8.9 | 9.8."""
+        """Whether a gated bfloat16 product goes to the ring kernel, sums and activation in one.  Us, weight-streaming kernel or (of large
+        matrices) library and activation | ring: 64 rows, inner 4,864 over 896 12.6 | 10.9, 8,960 over 1,536 24.2 | 20.6, but 8,192 over 2,048
+        21.8 | 25.4, 6,912 over 2,560 24.5 | 29.6, 18,944 over 3,584 62 | 70, 130 rows 78 | 85: large weights of few rows are a stream that tiles
+        of 128 columns do not share evenly; and small ones, 33 and 64 rows, 2,432 over 896 7.0 | 9.4 and 9.0 | 10.1, 2,816 over 1,024 7.2 | 10.0 and
+        9.7 | 10.8, have too few of them.  32 rows, 4,864 over 896 10.1 | 9.9, 17 rows 8.9 | 9.8.  (More than 64 rows: figures at
+        `ta_gemm_ring_gated_pays`.)"""
         if not (self.use_ring and m > self.RING_GATED_FROM and k >= 64 and k % 32 == 0 and inner % 4 == 0):
             return False
-        return m > self.RING_GATED_ROWS or 2 * inner * k < self.RING_GATED_WEIGHT or not self.use_library_gemm
+        if not self.use_library_gemm:
+            return True
+        if m <= self.SKINNY_ROWS:
+            return self.RING_GATED_WEIGHT <= 16 * inner * k and 4 * inner * k < self.RING_GATED_WEIGHT
+        if m <= self.RING_GATED_ROWS and 2 * inner * k >= self.RING_GATED_WEIGHT:
+            return False
+        return bool(self.lib.ta_gemm_ring_gated_pays(m, inner, k))
 
     # ------------------------------------------------------- fused decode products
     FUSED_ROWS = 16
