@@ -210,8 +210,14 @@ static RingPlan ring_plan(long M, long N, long K, bool gated, bool pending, int 
       const double rounds = (double)((tiles * s + units - 1) / units), steps = (double)((K + s - 1) / s) / 64;
       double cost = t.start + rounds * (t.fixed + steps * t.step);
       // (Where the weights' trip is what counts, the cheaper tile reads the rows less often: 65 rows x 151,936 over 1,536 133 us in 64 x 256
-      // tiles, 113 in 128 x 256 ones.)
-      cost = cost < weights ? weights + 0.15 * cost : cost + 0.15 * weights;
+      // tiles, 113 in 128 x 256 ones.  Up to 64 rows of results so wide that the smallest tiles fill the chip twice read them next to never, and what
+      // counts is how many workgroups stream: rows of 4 KB and more of 131,072 and 64,000 columns over 2,048, one row 104 and 53.7 us in 64 x 64 tiles,
+      // 116 and 56.4 in 64 x 128, 125 and 60.9 in 64 x 256; 32,768 over 4,096 54, 63, 68; shorter ones are level or the other way, 50,256 over
+      // 1,600 34.7, 32.3, 31.0; and more than 32 rows are read again often enough: 64 of 152,064 over 3,584 247, 227, 234.)
+      const bool streams = M <= 64 && (N + 63) / 64 >= 2 * units && s == 1;
+      if (cost >= weights) cost += 0.15 * weights;
+      else if (streams) cost = weights * (K >= 2048 && t.bn > (M <= 32 ? 64 : 128) ? 1.02 : 1.0) + 0.05 * cost + (t.bn == 64 && M > 32 ? 0.02 * weights : 0.0);
+      else cost = weights + 0.15 * cost;
       if (s == 1) cost += M * N * 2 / 8e6;
       else if (M <= 64) cost += s * (double)M * N / 1e6 + (pending ? 0.0 : 4.0);
       else cost += s * (double)M * N / 0.8e6 + (pending ? 1.0 : 2.0);

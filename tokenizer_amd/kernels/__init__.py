@@ -1661,7 +1661,7 @@ class Ops:
         17 and 64 rows x 896 over 4,864 9.3 | 7.7 and 11.7 | 8.6, x 3,584 over 18,944 39.5 | 33.4 and 47.4 | 36.0, x 1,024 over 1,024
         6.4 | 6.8 and 7.9 | 7.5, but x 896 over 896 6.4 | 6.7 and 7.1 | 7.1), and the vocabulary's projection of any number (weight-streaming kernel up to 16 rows, tiled above | ring:
         151,936 over 896, 1, 8, 16, 64 rows 51.7 | 52.0, 55.4 | 52.7, 60.8 | 53.0, 78 | 65; over 1,536 87.1 | 85.0, 90.4 | 87.3, 101 | 90,
-        118 | 109; over 3,584 197 | 192, 196 | 190, 211 | 193, 248 | 218)."""
+        118 | 109; 152,064 over 3,584 199 | 194, 204 | 200, 214 | 208, 257 | 227; 131,072 over 2,048 99 | 105, 104 | 107, 113 | 109, 138 | 131)."""
         if not (self.use_ring and k >= 64 and k % 32 == 0 and n % 4 == 0 and m * lda < 2 ** 31 and n * k < 2 ** 31):
             return False
         if m <= self.SKINNY_ROWS:
