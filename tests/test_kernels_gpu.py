@@ -631,18 +631,22 @@ def test_linear_of_a_few_hundred_rows_with_k_cut(ops, ref, shape, monkeypatch):
     """65 to 256 rows (a portion of a prompt beside decoded tokens) and few output tiles: K is cut where the parts
     may stay for the next norm (long K: recorded or not; shorter K: when launched eagerly, where small products
     do not go to the library), or into four parts that the kernel adds itself.  The same product either way, the
-    same on every run; the parts, added, are the product too."""
+    same on every run; the parts, added, are the product too.  (In the tiled kernel, and wherever the product goes with
+    the ring kernel on, which takes those with a K of whole half steps.)"""
     m, n, k = shape
     x = rand((m, k), torch.bfloat16, 34)
     w = rand((n, k), torch.bfloat16, 35, 0.1)
     bias = rand((n,), torch.float32, 36)
     want = ref.linear(x, w, bias, out_dtype=torch.float64)
-    for capturing in (False, True):
+    for capturing, ring in ((False, False), (True, False), (False, True), (True, True)):
         monkeypatch.setattr(ops, "capturing", capturing)
+        monkeypatch.setattr(ops, "use_ring", ring)
         expect_parts = k >= 2048 or (not capturing and k >= 768)
         assert (ops._k_splits(m, n, k, True) > 1) == expect_parts
         assert (ops._k_splits(m, n, k, False) > 1) == (not capturing and k >= 2048 and m * n * k < ops.EAGER_LIBRARY_WORK)
         left = ops.linear(x, w, bias, pending=True)
+        if ring:
+            expect_parts = isinstance(left, PendingSum)
         assert isinstance(left, PendingSum) == expect_parts
         got = left.resolve() if expect_parts else left
         torch.testing.assert_close(got.double(), want, **linear_tol(torch.bfloat16, x, w))
@@ -681,9 +685,13 @@ def test_linear_with_k_cut_over_streaming_workgroups(ops, ref, shape):
 
 @pytest.mark.parametrize("shape", [(17, 1152, 896), (64, 896, 4864), (200, 264, 136), (2048, 1152, 896)])
 def test_linear_through_the_library_and_through_own_kernels(ops, ref, shape, monkeypatch):
-    """More than sixteen bfloat16 rows may go to the vendor's library, the float32 bias in its accumulator; the
-    package's own kernels give the same product.  Rows of the input may be strided."""
+    """More than sixteen bfloat16 rows may go to the vendor's library, the float32 bias in its accumulator (the two
+    shapes at the ends do here; the others are taken before it, by the kernel that cuts K and, small and launched eagerly,
+    by the tiled one); the package's own kernels give the same product, the ring kernel too.  Rows of the input may be
+    strided."""
     m, n, k = shape
+    calls, library = [], ops.lib.ta_library_gemm_bf16
+    monkeypatch.setattr(ops.lib, "ta_library_gemm_bf16", lambda *args: (calls.append(1), library(*args))[1])
     wide = rand((m, k + 24), torch.bfloat16, 27)
     x = wide[:, 8:8 + k]                                 # strided rows, 16-byte aligned
     w = rand((n, k), torch.bfloat16, 28, 0.1)
@@ -693,10 +701,17 @@ def test_linear_through_the_library_and_through_own_kernels(ops, ref, shape, mon
         want = ref.linear(x, w, b, out_dtype=torch.float64)
         monkeypatch.setattr(ops, "use_library_gemm", True)
         monkeypatch.setattr(ops, "LIBRARY_WEIGHT", 0)    # every product of more than sixteen rows
+        monkeypatch.setattr(ops, "use_ring", False)
+        calls.clear()
         through_library = ops.linear(x, w, b)
+        assert bool(calls) == (m in (17, 2048))
+        calls.clear()
         monkeypatch.setattr(ops, "use_library_gemm", False)
         own = ops.linear(x, w, b)
-        for got in (through_library, own):
+        monkeypatch.setattr(ops, "use_ring", True)
+        ring = ops.linear(x, w, b)
+        assert not calls
+        for got in (through_library, own, ring):
             torch.testing.assert_close(got.double(), want, **linear_tol(torch.bfloat16, x, w))
 
 
@@ -904,6 +919,7 @@ def test_weight_streaming_product_with_two_column_blocks(ops, ref, shape, monkey
     x, w = rand((m, k), torch.bfloat16, 31), rand((n, k), torch.bfloat16, 32, 0.05)
     bias = rand((n,), torch.float32, 33)
     monkeypatch.setattr(ops, "use_library_gemm", False)
+    monkeypatch.setattr(ops, "use_ring", False)
     want = ref.linear(x, w, bias, out_dtype=torch.float32)
     gated_want = ref.linear_silu_gate(x.float(), w.float(), None)
     results = []

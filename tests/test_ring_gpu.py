@@ -94,7 +94,8 @@ def test_which_gated_products_are_whose(ops):
         assert not ops._gated_to_ring(m, inner, k), (m, inner, k)
 
 
-# (The two after the tiles: large tiles in front, small ones behind, as many columns in either.)
+# (The two after the tiles: large tiles in front, small ones behind.  None, none, none and one strip of 128 columns is in front here, none and two
+# for the wider; the next test has more.)
 @pytest.mark.parametrize("tile", range(1, len(TILES) + 2))
 @pytest.mark.parametrize("act", [None, "gelu_tanh", "relu", (1.702, 2.0, 1.0)])
 def test_gated_products_of_every_tile(ops, tile, act):
@@ -119,6 +120,45 @@ def test_gated_products_of_every_tile(ops, tile, act):
         # The activation in float: 2^-20 of the product of its factors, beside the rounding of the result.
         slack = 2.0 ** -20 * float(gate.abs().max() * up.abs().max())
         assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 4e-5 * float(want.abs().max()) + slack).all())
+
+
+# More tiles of rows than go in a group (sixteen), a number that is no multiple of it, over several strips of columns and parts of K: every tile
+# of the result is somebody's.  Plain, in parts, gated; the gated product in large tiles and small ones behind with several strips of either.
+@pytest.mark.parametrize("tile", range(len(TILES) + 2))
+def test_products_of_more_tiles_of_rows_than_a_group_has(ops, tile):
+    bm, bn = (TILES + [(128, 256), (256, 256)])[tile]
+    m, n, k = 17 * bm + 3, 2 * bn + 100, 96
+    x, w = strided(m, k, k + 8, tile), rand((n, k), 3, 0.1)
+    if tile < len(TILES):
+        out = torch.full((m, n), float("nan"), device="cuda")
+        assert ops.lib.ta_gemm_ring(_ptr(x), _ptr(w), None, _ptr(out), None, m, n, k, k + 8, n, 1, 0, tile, ops._stream()) == 0
+        assert close(out, x.double() @ w.double().t(), k, False)
+        long, wide = rand((m, 288), 5), rand((n, 288), 6, 0.1)
+        partial = torch.full((3, m, n), float("nan"), device="cuda")
+        assert ops.lib.ta_gemm_ring(_ptr(long), _ptr(wide), None, None, _ptr(partial), m, n, 288, 288, n, 3, 1, tile, ops._stream()) == 0
+        assert close(partial.double().sum(0), long.double() @ wide.double().t(), 288, False)
+    if tile > 0:
+        inner = 1500 if tile >= len(TILES) else n // 8 * 4
+        w = rand((2 * inner, k), 4, 0.2)
+        gate, up = (x.double() @ half.double().t() for half in (w[:inner], w[inner:]))
+        out = torch.full((m, inner), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert ops.lib.ta_gemm_ring_gated(_ptr(x), _ptr(w), _ptr(out), m, inner, k, k + 8, 1, *map(ctypes.c_float, (0.0, 0.0, 0.0)), tile,
+                                          ops._stream()) == 0
+        want = gate * torch.sigmoid(gate) * up
+        slack = 2.0 ** -20 * float(gate.abs().max() * up.abs().max())
+        assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 4e-5 * float(want.abs().max()) + slack).all())
+
+
+# The gated product where the launcher's own choice is whole rounds of large tiles with the columns behind them in small ones.
+def test_gated_product_of_two_kinds_of_tiles_by_the_launchers_choice(ops):
+    m, inner, k = 2048, 4864, 896
+    x, w = rand((m, k), 1), rand((2 * inner, k), 2, 0.05)
+    got = ops.linear_silu_gate(x, w)
+    for rows in range(0, m, 512):
+        gate, up = (x[rows:rows + 512].double() @ half.double().t() for half in (w[:inner], w[inner:]))
+        want = gate * torch.sigmoid(gate) * up
+        slack = 2.0 ** -20 * float(gate.abs().max() * up.abs().max())
+        assert bool(((got[rows:rows + 512].double() - want).abs() <= 2.0 ** -8 * want.abs() + 4e-5 * float(want.abs().max()) + slack).all())
 
 
 # Heads of one pair of blocks, of two and of three, more columns than a tile and fewer; tokens that are stored nowhere, pages in any order.
@@ -155,6 +195,28 @@ def test_projections_with_rotation_and_store_of_every_tile(ops, tile, n_q, n_kv,
         slack = 8 * 2e-6 * k ** 0.5 * float(out.abs().max())
         for got, want in ((q, heads[:, :n_q].reshape(m, -1)), (k_pages, keys), (v_pages, values)):
             assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + slack).all())
+
+
+# The same of more tiles of rows than go in a group, over several strips of columns: against the product and the rotation one by one.
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_projections_of_more_tiles_of_rows_than_a_group_has(ops, tile):
+    n_q, n_kv, d, page_size, k = 9, 1, 64, 16, 96
+    m, n = 17 * TILES[tile][0] + 5, (n_q + 2 * n_kv) * d
+    x, w, bias = rand((m, k), tile), rand((n, k), d, 0.1), torch.randn(n, device="cuda")
+    positions, slots = torch.arange(m, dtype=torch.int32, device="cuda"), torch.randperm(m, device="cuda").int()
+    table, pages = torch.randn((m, d), device="cuda"), -(-m // page_size)
+    k_pages, v_pages = (torch.zeros(shape, dtype=torch.bfloat16, device="cuda") for shape in ((pages, n_kv, page_size, d), (pages, n_kv, d, page_size)))
+    q = torch.full((m, n_q * d), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert ops.lib.ta_gemm_ring_qkv(_ptr(x), k, _ptr(w), _ptr(bias), _ptr(q), _ptr(positions), _ptr(table), _ptr(slots), _ptr(k_pages),
+                                    _ptr(v_pages), m, k, n_q, n_kv, d, page_size, tile, ops._stream()) == 0
+    heads = (x.double() @ w.double().t() + bias.double()).view(m, -1, d)
+    cos, sin = (t[:, None] for t in table.double().split(d // 2, 1))
+    u, v = heads[..., :d // 2], heads[..., d // 2:]
+    turned = torch.cat([u * cos - v * sin, v * cos + u * sin], -1)
+    page, off = slots.long() // page_size, slots.long() % page_size
+    slack = 8 * 2e-6 * k ** 0.5 * float(heads.abs().max())
+    for got, want in ((q, turned[:, :n_q].reshape(m, -1)), (k_pages[page, 0, off], turned[:, n_q]), (v_pages[page, 0, :, off], heads[:, n_q + 1])):
+        assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + slack).all())
 
 
 # Through the entry point: a width that the ring kernel does not take comes back from the two kernels before it, keys and values stored alike.

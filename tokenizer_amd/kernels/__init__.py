@@ -1400,11 +1400,14 @@ class Ops:
             # rows of 500 keys of size 64 8.9 -> 6.7 us, of 128 14.3 -> 10.1; a single row of 2,000 keys among short ones would
             # take 23 us instead of 16, so longer ranges stay cut; tied values have workgroups of four waves only).
             split_keys = max(split_keys, 512, -(-4 * rows_of_keys * max_keys // self.target_workgroups))
-        elif max_keys <= 4 * self.min_split_keys and head_dim <= 128 and not keep_first and not tied_values and v_pages is not None:
+        elif (max_keys <= 4 * self.min_split_keys and head_dim <= 128 and not keep_first and not tied_values and v_pages is not None
+              and (head_dim <= 96 or max_keys <= 3 * self.min_split_keys or max_keys == self.PLAN_KEYS)):
             # Fewer rows, up to 512 keys: whole too, a workgroup of many waves for each and no merge.  (One row in parts | whole, 24, 150,
             # 300 and 500 keys of head size 64: 5.8 6.1 6.2 6.4 | 4.0 4.6 5.4 6.1 us; 96: 6.8 7.2 7.2 7.6 | 3.6 4.4 5.2 6.8; 128: 7.3 8.1 8.3
-            # 8.2 | 4.3 5.5 7.0 9.2, where a compute unit's intake of the last hundred keys costs what the merge did; 256: 11.1 12.8 12.9
-            # 13.0 | 6.7 10.0 13.1 18.1, so there in parts.  Of 513 to 1,024 keys, size 64, 600 and 1,000: 6.3 6.4 | 6.6 9.1.)
+            # 8.2 | 4.3 5.5 7.0 9.2; 256: 11.1 12.8 12.9 13.0 | 6.7 10.0 13.1 18.1, so there in parts.  Of 513 to 1,024 keys, size 64, 600 and
+            # 1,000: 6.3 6.4 | 6.6 9.1.)  At 128 the two meet at some 390 keys: from there to 512 a compute unit's intake of the last
+            # hundred costs 0.5 to 1.3 us more than the merge did, below 3.0 to 0.2 us are saved.  Where a window or a chunk sets the range it
+            # is known to be on the far side; a context is not, since a recorded step serves all of up to 512.
             split_keys = max(split_keys, max_keys)
         split_keys = -(-split_keys // 32) * 32
         # (Reach enough for the block of 32 that a window's or run's first key lies in: `max_keys` has it in its 32 more.  Counted
@@ -1505,8 +1508,9 @@ class Ops:
                pending: bool = False) -> "torch.Tensor | PendingSum":
         """out = x @ weight.T (+ bias).  x [M, K] (rows may be strided); weight [N, K]; bias float32 [N].
 
-        float32 operands run on the matrix cores' 32-bit instructions; bfloat16 operands on theirs, with
-        float accumulation and a bfloat16 or float32 result.  `pending=True` allows the result to come back
+        float32 operands keep all their bits: few rows, and rows that are not aligned, on the matrix cores' 32-bit or on vector
+        instructions, more than sixteen aligned rows as sums of three bfloat16 numbers each; bfloat16 operands run on the
+        bfloat16 instructions, with float accumulation and a bfloat16 or float32 result.  `pending=True` allows the result to come back
         as a `PendingSum` when K is cut over workgroups: whoever takes it next (the norm that follows) adds the
         parts in its own kernel and the addition's launch is saved.
         """
@@ -1599,10 +1603,10 @@ class Ops:
             else:
                 to_library = m > self.FUSED_ROWS and ((k >= 2048 and n <= 4096) or n * k >= self.LIBRARY_WEIGHT)
             if to_library and self.use_library_gemm and out_dtype == torch.bfloat16:
-                # Plain products of more than 64 rows go to the vendor's library (hipBLASLt, called from
-                # library_gemm.hip), as the reference's engine uses a library for its matrix products: on the
-                # device's own clock (launches recorded in a graph, weights cold) it is ahead of the tiled
-                # kernel of this package for nearly every shape of the 0.5B to 7B models.  So do products of 17
+                # Products of more than 64 rows that the ring kernel has not taken (large results, see `_to_ring`) go to the
+                # vendor's library (hipBLASLt, called from library_gemm.hip), as the reference's engine uses a library for its
+                # matrix products: on the device's own clock (launches recorded in a graph, weights cold) it is ahead of
+                # the tiled kernel of this package for nearly every shape of the 0.5B to 7B models.  So do products of 17
                 # to 64 rows with a big weight matrix (every tile of the weight-streaming kernel reads all the
                 # rows again, which costs more than the weights once there are more than sixteen of them), and
                 # those with a long K and few output columns that the kernels above did not take.  The float32 bias
@@ -1678,12 +1682,13 @@ class Ops:
         """Into how many parts the tiled kernel cuts K.  17 to 64 rows: more than one with a K so long, and so few
         output tiles of 64 x 64, that the library (which cuts K as well) falls behind.  65 to 256 rows (portions of
         prompts beside decoded tokens): few tiles again, far fewer than compute units, and a whole K for each is
-        a long walk (137 rows x 896 columns over a K of 4,864: 32 us in one piece).  Where the parts may be left
-        for the norm that follows (`pending`) and K is 2,048 or more, eight parts beat the library as well (the same
-        product: 10 us against 10 us; 137 x 1,536 over 8,960: 17 us against 23 us).  Launched eagerly, small
-        products do not go to the library at all (its launch costs the host more than they take): those are cut
-        whenever K allows, into parts for the next norm or, with a long K, into four that the kernel adds itself
-        (14 us)."""
+        a long walk; left to this kernel are the products that the ring kernel does not take, a K of no whole half steps
+        of 32 above all (and all of them where that kernel is switched off: 137 rows x 896 columns over a K of 4,864
+        32 us in one piece).  Where the parts may be left for the norm that follows (`pending`) and K is 2,048 or more,
+        eight parts beat the library as well (the same product: 10 us against 10 us; 137 x 1,536 over 8,960: 17 us
+        against 23 us).  Launched eagerly, small products do not go to the library at all (its launch costs the host
+        more than they take): those are cut whenever K allows, into parts for the next norm or, with a long K, into four
+        that the kernel adds itself (14 us)."""
         if not self.use_split_k or n % 4:
             return 1
         tiles = -(-m // 64) * -(-n // 64)
@@ -1750,7 +1755,8 @@ class Ops:
         """out = silu(x @ Wg.T) * (x @ Wu.T) for weight = [Wg; Wu] of shape [2I, K]; out [M, I].  `act`: another
         gated activation than silu (see `silu_gate`).
 
-        Few bfloat16 rows run in one kernel; otherwise the product and the gated activation are two."""
+        One kernel for few rows (of either type; bfloat16 up to 64) and for the bfloat16 rows that the ring kernel takes
+        (`_gated_to_ring`); otherwise the product and the gated activation are two."""
         _need(weight.dim() == 2 and weight.shape[0] % 2 == 0, "the joined gate and up matrix has an even row count")
         m, inner = x.shape[0], weight.shape[0] // 2
         if out is None:
