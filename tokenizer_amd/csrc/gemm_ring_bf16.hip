@@ -220,7 +220,7 @@ static RingPlan ring_plan(long M, long N, long K, bool gated, bool pending, int 
       else cost = weights + 0.15 * cost;
       if (s == 1) cost += M * N * 2 / 8e6;
       else if (M <= 64) cost += s * (double)M * N / 1e6 + (pending ? 0.0 : 4.0);
-      else cost += s * (double)M * N / 0.8e6 + (pending ? 1.0 : 2.0);
+      else cost += s * (double)M * N / 0.8e6 + (pending ? 1.0 : 3.0);
       if (cost < best.cost) best = {shape, s, cost, 0};
     }
   }

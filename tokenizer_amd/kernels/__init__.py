@@ -1644,23 +1644,27 @@ class Ops:
     skinny_column_blocks = 0   # blocks of sixteen output columns per workgroup of the weight-streaming kernel: 0 = its choice
 
     use_ring = True            # products of many rows in the ring kernel (gemm_ring_bf16.hip) where it is the faster one
-    RING_RESULT = 2 ** 21      # products of more than 64 rows: results of up to so many elements (of matrices of up to ...
-    RING_WEIGHT = 2 ** 23      # ... so many, where no parts may be left), or of a K from ...
-    RING_LONG = 448            # ... a 448th of them on (see `_to_ring`)
+    RING_RESULT = 2 ** 21      # products of more than 64 rows whose parts the next norm adds: results of up to so many elements, ...
+    RING_LONG = 448            # ... or of up to so many times K
+    RING_ROWS = 1024           # plain bfloat16 products: up to so many rows (twice as many of narrow results) ...
+    RING_WEIGHT = 2 ** 23      # ... of matrices of up to so many elements, or with a long K (see `_to_ring`)
 
     def _to_ring(self, m: int, n: int, k: int, lda: int, out_dtype: torch.dtype, pending: bool) -> bool:
         """Whether a bfloat16 product goes to the ring kernel.  More than 64 rows against the library's timed choice: where the result
         has few tiles, since the library leaves the chip idle there, or K is so long that parts of it pay; large results the library's tiles do
         faster.  Us, weights from memory, library | ring.  With parts left for the norm that follows, norm included: 512 rows x 1,536 over 8,960
         42.7 | 30.1, 256 x 3,584 over 18,944 120 | 55, 2,048 x 896 over 4,864 37.7 | 32.9, and the other way 1,600 x 1,536 over 1,536
-        21.1 | 22.4, 2,048 x 2,560 over 2,560 45.6 | 49.2, 3,000 x 4,096 over 11,008 228 | 274, 2,600 x 3,584 over 18,944 314 | 368.  Plain:
-        512 x 1,152 over 896 8.5 | 6.0, 1,024 x 2,048 over 1,536 12.8 | 11.1, 512 x 1,536 over 8,960 38 | 29, and 1,536 x 2,048 over 1,536 15.0 | 16.3,
-        512 x 4,608 over 3,584 29 | 33, 3,072 x 896 over 4,864 36 | 40, 400 x 3,584 over 7,168 47.8 | 38.1 and 800 54.2 | 58.8.  Of 27 matrices
-        of widths of 512 to 5,120 and 65 to 4,096 rows, 680 products with the norm: 0.888 of the library's time with every one in the ring
-        kernel, 136 of them more than 3 % slower; 0.881 and 17 by this rule (700 rows x 2,048 over 2,048 19.4 | 21.4, 1,450 x 1,024 over 2,816
-        22.3 | 25.7).  775 plain ones of up to 5,000 rows 0.875, 33 more than 3 % slower (512 x 2,560 over 2,560 17.5 | 21.0, 256 x 1,024
-        over 2,816 9.7 | 10.8).  Float results the library does not give: the tiled kernel | ring, 4,100 rows x 4,096 over 4,096 217 | 161,
-        65,536 over 1,280 1,232 | 810, 400 x 896 over 4,864 32.7 | 14.3.
+        21.1 | 22.4, 2,048 x 2,560 over 2,560 45.6 | 49.2, 3,000 x 4,096 over 11,008 228 | 274, 2,600 x 3,584 over 18,944 314 | 368.  Of 27
+        matrices of widths of 512 to 5,120 and 65 to 4,096 rows, 680 products with the norm: 0.888 of the library's time with every one in the
+        ring kernel, 136 of them more than 3 % slower; 0.881 and 17 by this rule (700 rows x 2,048 over 2,048 19.4 | 21.4, 1,450 x 1,024
+        over 2,816 22.3 | 25.7).
+        Plain: 512 x 1,152 over 896 8.5 | 6.0, 1,024 x 2,048 over 1,536 12.8 | 11.1, 512 x 1,536 over 8,960 38 | 29, 2,048 x 896 over 2,432
+        17.9 | 15.6, 400 x 3,584 over 7,168 47.8 | 38.1, and the other way 1,536 x 2,048 over 1,536 15.0 | 16.3, 512 x 4,608 over 3,584
+        29 | 33, 3,072 x 896 over 4,864 36 | 40, 800 x 3,584 over 7,168 54.2 | 58.8.  775 plain ones of up to 5,000 rows take 0.879 of the
+        library's time by this rule, 33 more than 3 % longer (512 x 2,560 over 2,560 17.5 | 21.0, 1,600 x 1,536 over 4,480 33.3 | 36.2; launched
+        eagerly, where the library has not timed its choice, narrow ones of some 2,000 rows are level or faster in the ring kernel).  Float
+        results the library does not give: the tiled kernel | ring, 4,100 rows x 4,096 over 4,096 217 | 161, 65,536 over 1,280 1,232 | 810,
+        400 x 896 over 4,864 32.7 | 14.3.
         Of 17 to 64 rows those whose parts are left (the weight-streaming and the tiled kernel | ring, with the norm:
         17 and 64 rows x 896 over 4,864 9.3 | 7.7 and 11.7 | 8.6, x 3,584 over 18,944 39.5 | 33.4 and 47.4 | 36.0, x 1,024 over 1,024
         6.4 | 6.8 and 7.9 | 7.5, but x 896 over 896 6.4 | 6.7 and 7.1 | 7.1), and the vocabulary's projection of any number (weight-streaming kernel up to 16 rows, tiled above | ring:
@@ -1674,9 +1678,11 @@ class Ops:
             return pending and m > self.FUSED_ROWS and n * k >= (2 ** 21 if m <= 32 else 2 ** 20)
         if out_dtype == torch.float32 or not self.use_library_gemm:
             return True
-        if m * n <= self.RING_RESULT and (pending or n * k <= self.RING_WEIGHT):
-            return True
-        return m * n <= self.RING_LONG * k and (pending or k >= 2 * n)
+        if pending:
+            return m * n <= self.RING_RESULT or m * n <= self.RING_LONG * k
+        if n <= 1536:
+            return m <= 2 * self.RING_ROWS
+        return m <= self.RING_ROWS and n * k <= self.RING_WEIGHT or k >= 2 * n and m <= 640 or k >= 4 * n and m <= 1700
 
     def _k_splits(self, m: int, n: int, k: int, pending: bool = False) -> int:
         """Into how many parts the tiled kernel cuts K.  17 to 64 rows: more than one with a K so long, and so few
