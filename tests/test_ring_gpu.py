@@ -264,6 +264,21 @@ def test_the_choice_of_kernel_does_not_change_the_product(ops, m, n, k, monkeypa
             assert float((got[fine].double() - want[fine].double()).abs().max()) <= limit * float(want[fine].double().abs().max())
 
 
+# Decode attention of few rows at head size 128: whole where a step may have any context up to 512, in parts where a window's range is known to lie
+# past 384 keys.
+def test_ranges_of_keys_that_are_whole(ops, monkeypatch):
+    seen, kernel = [], ops.lib.ta_decode_attention_bf16
+    monkeypatch.setattr(ops.lib, "ta_decode_attention_bf16", lambda *args: (seen.append(args[20]), kernel(*args))[1])
+    for d, window, context, whole in ((128, None, 500, True), (128, 300, 2000, True), (128, 400, 2000, False), (96, 400, 2000, True), (64, 400, 2000, True)):
+        n_q, n_kv, pages = 4, 2, 128
+        q = rand((2, (n_q + 2 * n_kv) * d), d)
+        keys, values = rand((pages, n_kv, 16, d), 1), rand((pages, n_kv, d, 16), 2)
+        table = torch.arange(128, dtype=torch.int32, device="cuda").expand(2, -1).contiguous()
+        positions, out = torch.full((2,), context - 1, dtype=torch.int32, device="cuda"), torch.empty((2, n_q * d), dtype=torch.bfloat16, device="cuda")
+        ops._decode_attention(q, out, keys, values, positions, None, table, n_q, n_kv, d, 16, window, d ** -0.5, context - 1, identity_entries=True)
+        assert (seen[-1] == 1) == whole, (d, window)
+
+
 # The capped gate's three numbers may come as any sequence, with few rows and with many.
 @pytest.mark.parametrize("m", [9, 40, 300])
 def test_numbers_of_the_capped_gate_as_a_list(ops, m):
