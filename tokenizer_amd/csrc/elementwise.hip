@@ -378,13 +378,14 @@ add_terms_rmsnorm_kernel(float* __restrict__ residual, SumTerms terms, const flo
 }
 
 // One more term that is a product still in parts: factor * scale[h] * the sum over `count` slabs [n_tokens, hidden] of floats,
-// `stride` floats apart, added in their order.
+// `stride` floats apart, added in their order; `rounded`: the sum is rounded to the output's type, as the whole product would be.
 struct SlabTerm {
   const float* slabs;
   const float* scale;
   float factor;
   int count;
   size_t stride;
+  int rounded;
 };
 
 // The same for rows of up to 4,096 elements (a multiple of 4), in pieces of four elements: everything a
@@ -447,6 +448,10 @@ add_terms_rmsnorm_vec_kernel(float* __restrict__ residual, SumTerms terms, const
         const float4 more = ld4(tail.slabs + (size_t)j * tail.stride + (size_t)r * hidden + min(h, hidden - 4));
         v.x += more.x; v.y += more.y; v.z += more.z; v.w += more.w;
       }
+      if (tail.rounded) {
+        v.x = bf16_bits_to_float(float_to_bf16_bits(v.x)); v.y = bf16_bits_to_float(float_to_bf16_bits(v.y));
+        v.z = bf16_bits_to_float(float_to_bf16_bits(v.z)); v.w = bf16_bits_to_float(float_to_bf16_bits(v.w));
+      }
       v.x *= tail.factor; v.y *= tail.factor; v.z *= tail.factor; v.w *= tail.factor;
       if (SCALED) { v.x *= tail_scale[c].x; v.y *= tail_scale[c].y; v.z *= tail_scale[c].z; v.w *= tail_scale[c].w; }
       sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
@@ -479,7 +484,7 @@ static int launch_terms_vec(void* residual, const SumTerms& terms, const void* w
                             const void* weight2, float eps2, void* out2, const void* rows, int n_rows, int hidden,
                             int store_residual, const SlabTerm& tail, int dtype, hipStream_t stream) {
   const uintptr_t piece = dtype == DT_F32 ? 15 : 7;
-  if (hidden % 4 || hidden > 4096 || out_stride % 4 || terms.count > 3 || (tail.slabs && !weight) ||
+  if (hidden % 4 || hidden > 4096 || out_stride % 4 || terms.count > 3 ||
       (((uintptr_t)out | (uintptr_t)out2) & piece) ||
       (((uintptr_t)residual | (uintptr_t)weight | (uintptr_t)weight2 | (uintptr_t)tail.slabs | (uintptr_t)tail.scale) & 15))
     return -2;
@@ -489,14 +494,15 @@ static int launch_terms_vec(void* residual, const SumTerms& terms, const void* w
     scaled += terms.scale[k] ? 1 : 0;
   }
   if (scaled != 0 && scaled != terms.count + (tail.slabs ? 1 : 0)) return -2;
-  if (tail.slabs && (dtype != DT_BF16 || terms.count != 1 || tail.count < 1)) return -2;
+  if (tail.slabs && (dtype != DT_BF16 || terms.count < 1 || terms.count > 2 || tail.count < 1)) return -2;
 #define GO(TT, CC, NN, SS, LL) add_terms_rmsnorm_vec_kernel<TT, CC, NN, SS, LL><<<n_rows, 256, 0, stream>>>((float*)residual, terms, \
     (const float*)weight, (TT*)out, (const int*)rows, hidden, eps, store_residual, out_stride, (const float*)weight2, eps2,          \
     (TT*)out2, tail)
 #define GO_CHUNKS(TT, NN, SS, LL) switch ((hidden + 1023) / 1024) { case 1: GO(TT, 1, NN, SS, LL); break; \
     case 2: GO(TT, 2, NN, SS, LL); break; case 3: GO(TT, 3, NN, SS, LL); break; default: GO(TT, 4, NN, SS, LL); break; }
 #define GO_SCALED(TT, NN, LL) if (scaled) GO_CHUNKS(TT, NN, true, LL) else GO_CHUNKS(TT, NN, false, LL)
-  if (tail.slabs) { GO_SCALED(bf16_t, 1, true) }
+  if (tail.slabs && terms.count == 1) { GO_SCALED(bf16_t, 1, true) }
+  else if (tail.slabs) { GO_SCALED(bf16_t, 2, true) }
   else if (dtype == DT_F32) {
     if (terms.count == 0) { GO_CHUNKS(float, 0, false, false) }
     else if (terms.count == 1) { GO_SCALED(float, 1, false) } else if (terms.count == 2) { GO_SCALED(float, 2, false) } else return -2;
@@ -525,7 +531,7 @@ extern "C" int ta_add_terms_rmsnorm(void* residual, int count, const void* rows0
   for (int k = 0; k < count; ++k)
     if (!terms.rows[k]) return -1;
   const int status = launch_terms_vec(residual, terms, weight, eps, out, out_stride, weight2, eps2, out2, rows, n_rows, hidden,
-                                      store_residual, SlabTerm{nullptr, nullptr, 0.f, 0, 0}, dtype, stream);
+                                      store_residual, SlabTerm{nullptr, nullptr, 0.f, 0, 0, 0}, dtype, stream);
   if (status != -2) return status;
 #define TERMS(TT, PP) add_terms_rmsnorm_kernel<TT, PP><<<n_rows, 256, 0, stream>>>((float*)residual, terms,     (const float*)weight, eps, (TT*)out, out_stride, (const float*)weight2, eps2, (TT*)out2, (const int*)rows, hidden, store_residual)
 #define TERMS_SIZES(TT) if (hidden <= 256) TERMS(TT, 1); else if (hidden <= 1024) TERMS(TT, 4); else if (hidden <= 2048) TERMS(TT, 8);                         else if (hidden <= 4096) TERMS(TT, 16); else TERMS(TT, 32)
@@ -535,17 +541,21 @@ extern "C" int ta_add_terms_rmsnorm(void* residual, int count, const void* rows0
   return LAUNCH_STATUS();
 }
 
-// One term of rows and one in parts (float slabs [n_slabs, n_tokens, hidden], `stride` floats apart) in bfloat16 mode.  Returns
-// -2 for operands without the vector form (the caller then adds the parts first).
-extern "C" int ta_add_slabs_rmsnorm(void* residual, const void* rows0, const void* scale0, float f0, const void* slabs,
-                                    const void* slab_scale, float slab_factor, int n_slabs, size_t stride, const void* weight,
-                                    float eps, void* out, const void* rows, int n_rows, int hidden, int store_residual,
-                                    hipStream_t stream) {
+// One or two terms of rows and, behind them, one in parts (float slabs [n_slabs, n_tokens, hidden], `stride` floats apart) in
+// bfloat16 mode; the outputs as ta_add_terms_rmsnorm's.  Returns -2 for operands without the vector form (the caller then adds the
+// parts first).
+extern "C" int ta_add_slabs_rmsnorm(void* residual, int count, const void* rows0, const void* rows1, const void* scale0,
+                                    const void* scale1, float f0, float f1, const void* slabs, const void* slab_scale,
+                                    float slab_factor, int n_slabs, size_t stride, int rounded, const void* weight, float eps, void* out,
+                                    int out_stride, const void* weight2, float eps2, void* out2, const void* rows, int n_rows,
+                                    int hidden, int store_residual, hipStream_t stream) {
   if (n_rows <= 0) return 0;
-  if (hidden <= 0 || !rows0 || !slabs || n_slabs < 1 || !weight) return -1;
-  const SumTerms terms = {{rows0, nullptr, nullptr, nullptr}, {(const float*)scale0, nullptr, nullptr, nullptr}, {f0, 0.f, 0.f, 0.f}, 1};
-  return launch_terms_vec(residual, terms, weight, eps, out, hidden, nullptr, 0.f, nullptr, rows, n_rows, hidden, store_residual,
-                          SlabTerm{(const float*)slabs, (const float*)slab_scale, slab_factor, n_slabs, stride}, DT_BF16, stream);
+  if (hidden <= 0 || out_stride < hidden || count < 1 || count > 2 || !rows0 || (count == 2 && !rows1) || !slabs || n_slabs < 1 ||
+      (out2 && !weight2)) return -1;
+  const SumTerms terms = {{rows0, rows1, nullptr, nullptr}, {(const float*)scale0, (const float*)scale1, nullptr, nullptr},
+                          {f0, f1, 0.f, 0.f}, count};
+  return launch_terms_vec(residual, terms, weight, eps, out, out_stride, weight2, eps2, out2, rows, n_rows, hidden, store_residual,
+                          SlabTerm{(const float*)slabs, (const float*)slab_scale, slab_factor, n_slabs, stride, rounded}, DT_BF16, stream);
 }
 
 extern "C" int ta_add_pair_rmsnorm(void* residual, const void* first, const void* second, const void* weight, void* out,
@@ -555,7 +565,7 @@ extern "C" int ta_add_pair_rmsnorm(void* residual, const void* first, const void
   if (hidden <= 0 || hidden > 256 * 32 || !first || !second) return -1;
   const SumTerms terms = {{first, second, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr}, {1.f, 1.f, 0.f, 0.f}, 2};
   const int status = launch_terms_vec(residual, terms, weight, eps, out, hidden, nullptr, 0.f, nullptr, rows, n_rows, hidden,
-                                      store_residual, SlabTerm{nullptr, nullptr, 0.f, 0, 0}, dtype, stream);
+                                      store_residual, SlabTerm{nullptr, nullptr, 0.f, 0, 0, 0}, dtype, stream);
   if (status != -2) return status;
 #define PAIR(TT, PP) add_pair_rmsnorm_kernel<TT, PP><<<n_rows, 256, 0, stream>>>((float*)residual, (const TT*)first, \
     (const TT*)second, (const float*)weight, (TT*)out, (const int*)rows, hidden, eps, store_residual)

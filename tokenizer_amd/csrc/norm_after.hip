@@ -81,14 +81,41 @@ __device__ __forceinline__ void na_st4(bf16_t* p, float4 v) {
 }
 __device__ __forceinline__ float na_sq4(float4 v) { return v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; }
 
+__device__ __forceinline__ float na_rounded(float v) { return bf16_bits_to_float(float_to_bf16_bits(v)); }
+
+// d += the slabs behind the first one of a product in parts, at a thread's pieces of a row (`row`: in the first slab): four asked for
+// at a time, added in their order.  `rounded`: the sum as the whole product in bfloat16 would be.
+template <int CHUNKS>
+__device__ __forceinline__ void na_add_slabs(float4 (&d)[CHUNKS], const float* row, int parts, size_t slab, int hidden, int rounded) {
+  for (int s0 = 1; s0 < parts; s0 += 4) {
+    float4 v[CHUNKS][4];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        v[c][j] = na_ld4(row + (size_t)min(s0 + j, parts - 1) * slab + min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4));
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (s0 + j < parts) { d[c].x += v[c][j].x; d[c].y += v[c][j].y; d[c].z += v[c][j].z; d[c].w += v[c][j].w; }
+  }
+  if (rounded) {
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+      d[c] = make_float4(na_rounded(d[c].x), na_rounded(d[c].y), na_rounded(d[c].z), na_rounded(d[c].w));
+  }
+}
+
 // The same for rows whose length is a multiple of 4, up to CHUNKS * 1,024 elements: a thread takes four consecutive
 // elements of each run of 1,024, so the rows and weights move sixteen bytes a load (eight for bfloat16); a thread
 // past the row's end asks for the row's last elements and does not use them, so that no load stands behind a condition.
-template <typename TD, typename TO, int CHUNKS, bool DELTA, bool POST, bool NEXT>
+// PARTS: delta is a product whose K was cut over workgroups, `parts` float slabs `slab` elements apart, added in their order.
+template <typename TD, typename TO, int CHUNKS, bool DELTA, bool POST, bool NEXT, bool PARTS = false>
 __global__ void __launch_bounds__(NA_THREADS)
 norm_add_rmsnorm_vec_kernel(float* __restrict__ residual, const TD* __restrict__ delta, const float* __restrict__ post_weight,
                             float post_eps, const float* __restrict__ weight, float eps, TO* __restrict__ out,
-                            const int* __restrict__ rows, int hidden, int store_residual) {
+                            const int* __restrict__ rows, int hidden, int store_residual, int parts, size_t slab, int rounded) {
   __shared__ float scratch[16];
   const int i = blockIdx.x;
   const int r = rows ? rows[i] : i;
@@ -103,7 +130,7 @@ norm_add_rmsnorm_vec_kernel(float* __restrict__ residual, const TD* __restrict__
     if (DELTA && POST) behind_w[c] = na_ld4(post_weight + h);
     if (NEXT) next_w[c] = na_ld4(weight + h);
   }
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  if constexpr (PARTS) na_add_slabs<CHUNKS>(d, del, parts, slab, hidden, rounded);
   if (DELTA) {
     float inv = 1.f;
     if (POST) {
@@ -142,7 +169,6 @@ norm_add_rmsnorm_vec_kernel(float* __restrict__ residual, const TD* __restrict__
                                           x[c].w * inv * next_w[c].w));
     else na_st4(dst + h, x[c]);
   }
-  (void)zero;
 }
 
 // Rows longer than a workgroup's registers hold: the same sums, with the row read again from memory for every pass.
@@ -438,36 +464,86 @@ norm_side_norm_vec_kernel(float* __restrict__ residual, const T* __restrict__ de
   }
 }
 
-// The same for few rows (no more than compute units) and token inputs of up to sixteen numbers, bfloat16: sixteen waves a
-// workgroup, so that everything a row needs of both small matrices is asked for at once, beside the row itself, and a row is
-// one trip to memory.  Wave j holds row j of the gate's matrix (its dot product is a wave's own), a thread the projection's
-// rows of its two elements of each run of 2,048.  Bound by the trip and the four sums over the workgroup behind it.
-// (1 to 64 rows of 1,536: 12.1 us in the kernel above, 7.0 here; of 896 9.8 and 6.8, of 3,584 18.8 and 9.6.  With more rows a workgroup would read both
-// matrices for each of them, or hold them and take row after row: 2,048 rows of 896 24.6 us above, 34.9 so.)
+// The same for token inputs of up to sixteen numbers, bfloat16, R rows a workgroup of sixteen waves: everything the rows need of both
+// small matrices is asked for at once, beside the rows themselves, and a workgroup is one trip to memory.  Wave j holds row j of the
+// gate's matrix (a row's dot product with it is a wave's own), a thread the projection's rows of its two elements of each run of
+// 2,048, for all R rows.  Few rows: one a workgroup, bound by the trip and the four sums over the workgroup behind it (three rows of
+// 1,536 6.6 us).  Many: both matrices are read once for R rows, where a workgroup a row pulls in some 100 KB for each of them; bound by
+// the rows' turns through LDS.  (The kernel above | this, us, 16 numbers a token: 300, 1,024 and 2,048 rows of 1,536 14.8 | 8.2, 22.3 | 12.3,
+// 39.7 | 21.0; of 896 10.8 | 7.7, 14.1 | 11.2, 23.7 | 18.8; of 3,584 22.8 | 12.4, 54 | 21, 91 | 42.)  PARTS: delta is a product whose
+// K was cut over workgroups, `parts` float slabs `slab` elements apart, added in their order and, `rounded`, rounded as the whole
+// product would be.
 #define NA_WIDE 1024
-template <int RUNS>
+
+// Sums over the workgroup's sixteen waves of R values a thread, as 1 / sqrt(sum / hidden + eps) in `inv`, for every thread.
+template <int R>
+__device__ __forceinline__ void na_row_rms(float (&v)[R], float (&inv)[R], float* scratch, float* inv_s, int hidden, float eps) {
+  if constexpr (R == 1) {
+    inv[0] = 1.0f / sqrtf(block_sum(v[0], scratch) / (float)hidden + eps);
+  } else {
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    // Half of the values change places with the lane `off` away at every step, until a lane holds one row's sum over its likes.
+    int off = WAVE / 2;
+#pragma unroll
+    for (int width = R; width > 1; width /= 2, off /= 2) {
+      const bool upper = lane & off;
+#pragma unroll
+      for (int i = 0; i < width / 2; ++i) {
+        const float send = upper ? v[i] : v[i + width / 2], keep = upper ? v[i + width / 2] : v[i];
+        v[i] = keep + __shfl_xor(send, off, WAVE);
+      }
+    }
+    for (; off > 0; off /= 2) v[0] += __shfl_xor(v[0], off, WAVE);
+    if (lane % (WAVE / R) == 0) scratch[lane / (WAVE / R) * 16 + wave] = v[0];
+    __syncthreads();
+    if (threadIdx.x < R * 16) {
+      float sum = scratch[threadIdx.x];
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) sum += __shfl_xor(sum, o, WAVE);
+      if ((threadIdx.x & 15) == 0) inv_s[threadIdx.x / 16] = 1.0f / sqrtf(sum / (float)hidden + eps);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < R; ++q) inv[q] = inv_s[q];
+  }
+}
+
+template <int RUNS, int R, bool PARTS>
 __global__ void __launch_bounds__(NA_WIDE)
-norm_side_norm_held_kernel(float* __restrict__ residual, const bf16_t* __restrict__ delta, const float* __restrict__ post_weight,
+norm_side_norm_held_kernel(float* __restrict__ residual, const void* __restrict__ delta, const float* __restrict__ post_weight,
                            float post_eps, const bf16_t* __restrict__ gate, const bf16_t* __restrict__ proj, int proj_stride,
                            const float* __restrict__ side_norm, float side_eps, const bf16_t* __restrict__ table, int table_width,
                            const int* __restrict__ token_ids, int offset, int dim, const float* __restrict__ weight, float eps,
-                           bf16_t* __restrict__ out, const int* __restrict__ rows, int hidden, int store_residual) {
-  __shared__ float scratch[16];
-  __shared__ __attribute__((aligned(16))) float x_s[RUNS * 2048];
-  __shared__ float g_s[16];
+                           bf16_t* __restrict__ out, const int* __restrict__ rows, int n_rows, int hidden, int store_residual,
+                           int parts, size_t slab, int rounded) {
+  __shared__ __attribute__((aligned(16))) float x_s[R][RUNS * 2048];
+  __shared__ __attribute__((aligned(16))) float g_s[R][16];
+  __shared__ float scratch[R * 16], inv_s[R], inv_t[R];
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
   const bool two = dim > 8;
-  const int r = rows ? rows[blockIdx.x] : blockIdx.x;
-  float* res = residual + (size_t)r * hidden;
-  float2 x[RUNS];
-  uint32_t d[RUNS];
+  int r[R];                                                  // (past the last row: the last row again, not stored)
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int i = min((int)blockIdx.x * R + q, n_rows - 1);
+    r[q] = rows ? rows[i] : i;
+  }
+  float2 x[R][RUNS], d[R][RUNS];
+  uint32_t raw[R][RUNS];
   float e = 0.f;
-  if (threadIdx.x < dim) e = ld(table + (size_t)token_ids[r] * table_width + offset + threadIdx.x);
+  if (threadIdx.x < R * 16 && (threadIdx.x & 15) < dim) {
+    const int i = min((int)blockIdx.x * R + (int)threadIdx.x / 16, n_rows - 1);
+    e = ld(table + (size_t)token_ids[rows ? rows[i] : i] * table_width + offset + (threadIdx.x & 15));
+  }
 #pragma unroll
   for (int c = 0; c < RUNS; ++c) {
     const int h = min(c * 2048 + (int)threadIdx.x * 2, hidden - 2);
-    x[c] = *reinterpret_cast<const float2*>(res + h);
-    d[c] = delta ? *reinterpret_cast<const uint32_t*>(delta + (size_t)r * hidden + h) : 0u;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const size_t at = (size_t)r[q] * hidden + h;
+      x[q][c] = *reinterpret_cast<const float2*>(residual + at);
+      if constexpr (PARTS) d[q][c] = *reinterpret_cast<const float2*>((const float*)delta + at);
+      else raw[q][c] = delta ? *reinterpret_cast<const uint32_t*>((const bf16_t*)delta + at) : 0u;
+    }
   }
   uint4 gate_row[RUNS * 4], proj_row[RUNS][2][2];
 #pragma unroll
@@ -488,87 +564,145 @@ norm_side_norm_held_kernel(float* __restrict__ residual, const bf16_t* __restric
     tail[c] = *reinterpret_cast<const float2*>(side_norm + h);
     next[c] = weight ? *reinterpret_cast<const float2*>(weight + h) : make_float2(1.f, 1.f);
   }
+  if constexpr (PARTS) {
+    constexpr int DEEP = R * RUNS <= 4 ? 4 : 2;              // slabs asked for at a time
+    for (int s0 = 1; s0 < parts; s0 += DEEP) {
+      float2 v[DEEP][R][RUNS];
+#pragma unroll
+      for (int j = 0; j < DEEP; ++j)
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+#pragma unroll
+          for (int c = 0; c < RUNS; ++c)
+            v[j][q][c] = *reinterpret_cast<const float2*>((const float*)delta + (size_t)min(s0 + j, parts - 1) * slab +
+                                                          (size_t)r[q] * hidden + min(c * 2048 + (int)threadIdx.x * 2, hidden - 2));
+#pragma unroll
+      for (int j = 0; j < DEEP; ++j)
+        if (s0 + j < parts) {
+#pragma unroll
+          for (int q = 0; q < R; ++q)
+#pragma unroll
+            for (int c = 0; c < RUNS; ++c) { d[q][c].x += v[j][q][c].x; d[q][c].y += v[j][q][c].y; }
+        }
+    }
+    if (rounded) {
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int c = 0; c < RUNS; ++c) d[q][c] = make_float2(na_rounded(d[q][c].x), na_rounded(d[q][c].y));
+    }
+  }
   auto low = [](uint32_t w) { return __uint_as_float(w << 16); };
   auto high = [](uint32_t w) { return __uint_as_float(w & 0xffff0000u); };
-  float sq = 0.f, inv = 1.f;
+  float sq[R], inv[R];
 #pragma unroll
-  for (int c = 0; c < RUNS; ++c) {
-    const float a = low(d[c]), b = high(d[c]);
-    if (c * 2048 + (int)threadIdx.x * 2 < hidden) sq += a * a + b * b;
-  }
-  if (delta && post_weight) inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)hidden + post_eps);
+  for (int q = 0; q < R; ++q) {
+    sq[q] = 0.f;
+    inv[q] = 1.f;
 #pragma unroll
-  for (int c = 0; c < RUNS; ++c) {
-    const int h = c * 2048 + (int)threadIdx.x * 2;
-    x[c].x += low(d[c]) * inv * behind[c].x;
-    x[c].y += high(d[c]) * inv * behind[c].y;
-    if (h < hidden) *reinterpret_cast<float2*>(x_s + h) = x[c];
+    for (int c = 0; c < RUNS; ++c) {
+      if constexpr (!PARTS) d[q][c] = make_float2(low(raw[q][c]), high(raw[q][c]));
+      if (c * 2048 + (int)threadIdx.x * 2 < hidden) sq[q] += d[q][c].x * d[q][c].x + d[q][c].y * d[q][c].y;
+    }
   }
+  if (delta && post_weight) na_row_rms<R>(sq, inv, scratch, inv_s, hidden, post_eps);
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+#pragma unroll
+    for (int c = 0; c < RUNS; ++c) {
+      const int h = c * 2048 + (int)threadIdx.x * 2;
+      x[q][c].x += d[q][c].x * inv[q] * behind[c].x;
+      x[q][c].y += d[q][c].y * inv[q] * behind[c].y;
+      if (h < hidden) *reinterpret_cast<float2*>(x_s[q] + h) = x[q][c];
+    }
   __syncthreads();
-  float z = 0.f;
   if (wave < dim) {
+    float z[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) z[q] = 0.f;
 #pragma unroll
     for (int c = 0; c < RUNS * 4; ++c) {
       const int at = c * 512 + lane * 8;
       if (at >= hidden) break;
-      const float4 a = *reinterpret_cast<const float4*>(x_s + at), b = *reinterpret_cast<const float4*>(x_s + at + 4);
       const uint4 w = gate_row[c];
-      z = fmaf(low(w.x), a.x, fmaf(high(w.x), a.y, fmaf(low(w.y), a.z, fmaf(high(w.y), a.w, z))));
-      z = fmaf(low(w.z), b.x, fmaf(high(w.z), b.y, fmaf(low(w.w), b.z, fmaf(high(w.w), b.w, z))));
-    }
-    z = wave_sum(z);
-    if (lane == 0) g_s[wave] = z;
-  }
-  __syncthreads();
-  if (threadIdx.x < 16) g_s[threadIdx.x] = threadIdx.x < dim ? na_gelu_tanh(g_s[threadIdx.x]) * e : 0.f;
-  __syncthreads();
-  float g[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) g[k] = g_s[k];
-  float2 y[RUNS];
-  sq = 0.f;
-#pragma unroll
-  for (int c = 0; c < RUNS; ++c) {
-    float s[2] = {0.f, 0.f};
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        if (p && !two) continue;
-        const uint32_t w[4] = {proj_row[c][q][p].x, proj_row[c][q][p].y, proj_row[c][q][p].z, proj_row[c][q][p].w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s[q] = fmaf(high(w[k]), g[8 * p + 2 * k + 1], fmaf(low(w[k]), g[8 * p + 2 * k], s[q]));
+      for (int q = 0; q < R; ++q) {
+        const float4 a = *reinterpret_cast<const float4*>(x_s[q] + at), b = *reinterpret_cast<const float4*>(x_s[q] + at + 4);
+        z[q] = fmaf(low(w.x), a.x, fmaf(high(w.x), a.y, fmaf(low(w.y), a.z, fmaf(high(w.y), a.w, z[q]))));
+        z[q] = fmaf(low(w.z), b.x, fmaf(high(w.z), b.y, fmaf(low(w.w), b.z, fmaf(high(w.w), b.w, z[q]))));
       }
-    y[c] = make_float2(s[0], s[1]);
-    if (c * 2048 + (int)threadIdx.x * 2 < hidden) sq += s[0] * s[0] + s[1] * s[1];
-  }
-  const float inv_y = 1.0f / sqrtf(block_sum(sq, scratch) / (float)hidden + side_eps);
-  sq = 0.f;
+    }
 #pragma unroll
-  for (int c = 0; c < RUNS; ++c) {
-    const int h = c * 2048 + (int)threadIdx.x * 2;
-    x[c].x += y[c].x * inv_y * tail[c].x;
-    x[c].y += y[c].y * inv_y * tail[c].y;
-    if (h < hidden) {
-      if (store_residual) *reinterpret_cast<float2*>(res + h) = x[c];
-      sq += x[c].x * x[c].x + x[c].y * x[c].y;
+    for (int q = 0; q < R; ++q) {
+      const float sum = wave_sum(z[q]);
+      if (lane == 0) g_s[q][wave] = sum;
     }
   }
-  inv = 1.f;
-  if (weight) inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)hidden + eps);
-  bf16_t* dst = out + (size_t)blockIdx.x * hidden;
+  __syncthreads();
+  if (threadIdx.x < R * 16) {
+    float* g = g_s[0] + threadIdx.x;
+    *g = (threadIdx.x & 15) < dim ? na_gelu_tanh(*g) * e : 0.f;
+  }
+  __syncthreads();
+  float2 y[R][RUNS];
 #pragma unroll
-  for (int c = 0; c < RUNS; ++c) {
-    const int h = c * 2048 + (int)threadIdx.x * 2;
-    if (h >= hidden) continue;
-    *reinterpret_cast<uint32_t*>(dst + h) = (uint32_t)float_to_bf16_bits(x[c].x * inv * next[c].x) |
-                                            ((uint32_t)float_to_bf16_bits(x[c].y * inv * next[c].y) << 16);
+  for (int q = 0; q < R; ++q) {
+    float g[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) g[k] = g_s[q][k];
+    sq[q] = 0.f;
+#pragma unroll
+    for (int c = 0; c < RUNS; ++c) {
+      float s[2] = {0.f, 0.f};
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          if (p && !two) continue;
+          const uint32_t w[4] = {proj_row[c][k2][p].x, proj_row[c][k2][p].y, proj_row[c][k2][p].z, proj_row[c][k2][p].w};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) s[k2] = fmaf(high(w[k]), g[8 * p + 2 * k + 1], fmaf(low(w[k]), g[8 * p + 2 * k], s[k2]));
+        }
+      y[q][c] = make_float2(s[0], s[1]);
+      if (c * 2048 + (int)threadIdx.x * 2 < hidden) sq[q] += s[0] * s[0] + s[1] * s[1];
+    }
+  }
+  na_row_rms<R>(sq, inv, scratch, inv_t, hidden, side_eps);
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    sq[q] = 0.f;
+    const bool live = (int)blockIdx.x * R + q < n_rows;
+#pragma unroll
+    for (int c = 0; c < RUNS; ++c) {
+      const int h = c * 2048 + (int)threadIdx.x * 2;
+      x[q][c].x += y[q][c].x * inv[q] * tail[c].x;
+      x[q][c].y += y[q][c].y * inv[q] * tail[c].y;
+      if (h < hidden) {
+        if (store_residual && live) *reinterpret_cast<float2*>(residual + (size_t)r[q] * hidden + h) = x[q][c];
+        sq[q] += x[q][c].x * x[q][c].x + x[q][c].y * x[q][c].y;
+      }
+    }
+    inv[q] = 1.f;
+  }
+  if (weight) na_row_rms<R>(sq, inv, scratch, inv_s, hidden, eps);
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int i = (int)blockIdx.x * R + q;
+    if (i >= n_rows) break;
+#pragma unroll
+    for (int c = 0; c < RUNS; ++c) {
+      const int h = c * 2048 + (int)threadIdx.x * 2;
+      if (h >= hidden) continue;
+      *reinterpret_cast<uint32_t*>(out + (size_t)i * hidden + h) =
+          (uint32_t)float_to_bf16_bits(x[q][c].x * inv[q] * next[c].x) | ((uint32_t)float_to_bf16_bits(x[q][c].y * inv[q] * next[c].y) << 16);
+    }
   }
 }
 
 // dtype: of delta, gate, proj, table and out.  Returns -2 for sizes the fused kernel does not take (rows longer than
-// a workgroup holds, a wider token input): the caller then runs the steps one by one.
-extern "C" int ta_norm_side_norm(void* residual, const void* delta, const void* post_weight, float post_eps, const void* gate,
+// a workgroup holds, a wider token input): the caller then runs the steps one by one.  parts > 0: delta is float [parts, slab_rows,
+// hidden], a product still in parts; -3: not in that form here (the caller adds the parts first).
+extern "C" int ta_norm_side_norm(void* residual, const void* delta, int parts, int slab_rows, int rounded, const void* post_weight, float post_eps, const void* gate,
                                  const void* proj, int proj_stride, const void* side_norm, float side_eps, const void* table,
                                  int table_width, const void* token_ids, int offset, int dim, const void* weight, float eps,
                                  void* out, const void* rows, int n_rows, int hidden, int store_residual, int dtype,
@@ -585,21 +719,33 @@ extern "C" int ta_norm_side_norm(void* residual, const void* delta, const void* 
         (float*)residual, (const TT*)delta, (const float*)post_weight, post_eps, (const TT*)gate, (const TT*)proj,      \
         proj_stride, (const float*)side_norm, side_eps, (const TT*)table, table_width, (const int*)token_ids, offset,   \
         dim, (const float*)weight, eps, (TT*)out, (const int*)rows, hidden, store_residual)
-    if (dtype != DT_F32 && dim <= 16 && n_rows <= compute_units()) {
-#define HELD_SIDE(RR)                                                                                                  \
-      norm_side_norm_held_kernel<RR><<<n_rows, NA_WIDE, 0, stream>>>(                                                  \
-          (float*)residual, (const bf16_t*)delta, (const float*)post_weight, post_eps, (const bf16_t*)gate,            \
-          (const bf16_t*)proj, proj_stride, (const float*)side_norm, side_eps, (const bf16_t*)table, table_width,      \
-          (const int*)token_ids, offset, dim, (const float*)weight, eps, (bf16_t*)out, (const int*)rows, hidden, store_residual)
-      if (hidden <= 2048) HELD_SIDE(1); else HELD_SIDE(2);
+    if (dtype != DT_F32 && dim <= 16) {
+      // As many rows a workgroup (while the registers hold them) as still give every compute unit one.
+      const size_t slab = (size_t)slab_rows * hidden;
+#define HELD_SIDE(UU, RR, PP)                                                                                          \
+      norm_side_norm_held_kernel<UU, RR, PP><<<(n_rows + RR - 1) / RR, NA_WIDE, 0, stream>>>(                          \
+          (float*)residual, delta, (const float*)post_weight, post_eps, (const bf16_t*)gate, (const bf16_t*)proj,      \
+          proj_stride, (const float*)side_norm, side_eps, (const bf16_t*)table, table_width, (const int*)token_ids,    \
+          offset, dim, (const float*)weight, eps, (bf16_t*)out, (const int*)rows, n_rows, hidden, store_residual, parts, slab, rounded)
+#define HELD_PARTS(UU, RR) do { if (parts) HELD_SIDE(UU, RR, true); else HELD_SIDE(UU, RR, false); } while (0)
+      const int units = compute_units();
+      if (hidden <= 2048) {
+        if (n_rows <= units) HELD_PARTS(1, 1); else if (n_rows <= 2 * units) HELD_PARTS(1, 2);
+        else if (n_rows <= 4 * units) HELD_PARTS(1, 4); else HELD_PARTS(1, 8);
+      } else {
+        if (n_rows <= units) HELD_PARTS(2, 1); else if (n_rows <= 2 * units) HELD_PARTS(2, 2); else HELD_PARTS(2, 4);
+      }
+#undef HELD_PARTS
 #undef HELD_SIDE
       return LAUNCH_STATUS();
     }
+    if (parts) return -3;
     if (dtype == DT_F32) { if (hidden <= 1024) SIDE(float, 1); else if (hidden <= 2048) SIDE(float, 2); else SIDE(float, 4); }
     else { if (hidden <= 1024) SIDE(bf16_t, 1); else if (hidden <= 2048) SIDE(bf16_t, 2); else SIDE(bf16_t, 4); }
 #undef SIDE
     return LAUNCH_STATUS();
   }
+  if (parts) return -3;
   if (dtype == DT_F32)
     norm_side_norm_kernel<float><<<n_rows, NA_THREADS, 0, stream>>>(
         (float*)residual, (const float*)delta, (const float*)post_weight, post_eps, (const float*)gate, (const float*)proj,
@@ -626,7 +772,7 @@ extern "C" int ta_norm_add_rmsnorm(void* residual, const void* delta, const void
 #define VEC3(TD, TO, CH, DD, PP, NN)                                                                                   \
     norm_add_rmsnorm_vec_kernel<TD, TO, CH, DD, PP, NN><<<n_rows, NA_THREADS, 0, stream>>>(                             \
         (float*)residual, (const TD*)delta, (const float*)post_weight, post_eps, (const float*)weight, eps, (TO*)out,   \
-        (const int*)rows, hidden, store_residual)
+        (const int*)rows, hidden, store_residual, 1, 0, 0)
 #define VEC2(TD, TO, CH)                                                                                               \
     do {                                                                                                               \
       if (delta && post_weight) { if (weight) VEC3(TD, TO, CH, true, true, true); else VEC3(TD, TO, CH, true, true, false); } \
@@ -696,7 +842,7 @@ __global__ void __launch_bounds__(NA_THREADS)
 group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ delta, const float* __restrict__ post_weight,
                           float post_eps, int post_groups, const float* __restrict__ weight, float eps, int groups,
                           TO* __restrict__ out, const int* __restrict__ rows, int hidden, int store_residual, int parts,
-                          size_t slab) {
+                          size_t slab, int rounded) {
   extern __shared__ float na_part[];
   float* inv = na_part + hidden / 4;
   const int i = blockIdx.x;
@@ -711,22 +857,7 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
     behind_w[c] = post_weight ? na_ld4(post_weight + h) : make_float4(1.f, 1.f, 1.f, 1.f);
     next_w[c] = weight ? na_ld4(weight + h) : make_float4(1.f, 1.f, 1.f, 1.f);
   }
-  if constexpr (PARTS) {                                     // (the other slabs, four asked for at a time, added in their order)
-    for (int s0 = 1; s0 < parts; s0 += 4) {
-      float4 v[CHUNKS][4];
-#pragma unroll
-      for (int c = 0; c < CHUNKS; ++c)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          v[c][j] = na_ld4(delta + (size_t)min(s0 + j, parts - 1) * slab + (size_t)r * hidden +
-                           min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4));
-#pragma unroll
-      for (int c = 0; c < CHUNKS; ++c)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (s0 + j < parts) { d[c].x += v[c][j].x; d[c].y += v[c][j].y; d[c].z += v[c][j].z; d[c].w += v[c][j].w; }
-    }
-  }
+  if constexpr (PARTS) na_add_slabs<CHUNKS>(d, delta + (size_t)r * hidden, parts, slab, hidden, rounded);
   if (post_weight) {
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
@@ -825,7 +956,7 @@ extern "C" int ta_group_norm_add(void* residual, const void* delta, const void* 
 #define GROUP_VEC(TD, TO, CH)                                                                                            \
     group_norm_add_vec_kernel<TD, TO, CH><<<n_rows, NA_THREADS, lds, stream>>>(                                           \
         (float*)residual, (const TD*)delta, (const float*)post_weight, post_eps, post_groups, (const float*)weight, eps,  \
-        groups, (TO*)out, (const int*)rows, hidden, store_residual, 1, 0)
+        groups, (TO*)out, (const int*)rows, hidden, store_residual, 1, 0, 0)
 #define GROUP_GO(TD, TO)                                                                                                 \
   do {                                                                                                                   \
     if (vec) {                                                                                                           \
@@ -845,22 +976,36 @@ extern "C" int ta_group_norm_add(void* residual, const void* delta, const void* 
   return LAUNCH_STATUS();
 }
 
-// The same with delta still in parts: `partial` float [parts, slab_rows, hidden], added in their order.  -2: rows that only the general
-// kernel takes, which reads them again for every pass (the caller adds the parts first).
-extern "C" int ta_group_norm_add_parts(void* residual, const void* partial, int parts, int slab_rows, const void* post_weight, float post_eps,
-                                       int post_groups, const void* weight, float eps, int groups, void* out, const void* rows,
-                                       int n_rows, int hidden, int store_residual, int out_dtype, hipStream_t stream) {
+// The same with delta still in parts: `partial` float [parts, slab_rows, hidden], added in their order; one group each: the norms
+// over whole rows.  -2: rows that only the general kernels take, which read them again for every pass (the caller adds the parts first).
+extern "C" int ta_norm_add_parts(void* residual, const void* partial, int parts, int slab_rows, int rounded, const void* post_weight, float post_eps,
+                                 int post_groups, const void* weight, float eps, int groups, void* out, const void* rows,
+                                 int n_rows, int hidden, int store_residual, int out_dtype, hipStream_t stream) {
   if (n_rows <= 0) return 0;
   if (hidden <= 0 || post_groups <= 0 || groups <= 0 || hidden % post_groups || hidden % groups || parts < 1 || !partial) return -1;
   const int most = post_groups > groups ? post_groups : groups;
   const bool aligned = (((uintptr_t)residual | (uintptr_t)partial | (uintptr_t)post_weight | (uintptr_t)weight | (uintptr_t)out) & 15) == 0;
   if (!aligned || hidden > 4096 || (hidden / post_groups) % 4 || (hidden / groups) % 4 || post_groups + groups > 12 * 1024) return -2;
   const size_t lds = sizeof(float) * ((size_t)hidden / 4 + most), slab = (size_t)slab_rows * hidden;
-#define GO(TO, CH) group_norm_add_vec_kernel<float, TO, CH, true><<<n_rows, NA_THREADS, lds, stream>>>( \
-    (float*)residual, (const float*)partial, (const float*)post_weight, post_eps, post_groups, (const float*)weight, eps, groups, \
-    (TO*)out, (const int*)rows, hidden, store_residual, parts, slab)
 #define LENGTHS(TO) \
   if (hidden <= 1024) GO(TO, 1); else if (hidden <= 2048) GO(TO, 2); else GO(TO, 4)
+  if (post_groups == 1 && groups == 1) {
+#define GO_FORM(TO, CH, PP, NN) norm_add_rmsnorm_vec_kernel<float, TO, CH, true, PP, NN, true><<<n_rows, NA_THREADS, 0, stream>>>( \
+    (float*)residual, (const float*)partial, (const float*)post_weight, post_eps, (const float*)weight, eps, (TO*)out, \
+    (const int*)rows, hidden, store_residual, parts, slab, rounded)
+#define GO(TO, CH)                                                                                     \
+    do {                                                                                               \
+      if (post_weight) { if (weight) GO_FORM(TO, CH, true, true); else GO_FORM(TO, CH, true, false); } \
+      else { if (weight) GO_FORM(TO, CH, false, true); else GO_FORM(TO, CH, false, false); }           \
+    } while (0)
+    if (out_dtype == DT_F32) { LENGTHS(float); } else { LENGTHS(bf16_t); }
+#undef GO
+#undef GO_FORM
+    return LAUNCH_STATUS();
+  }
+#define GO(TO, CH) group_norm_add_vec_kernel<float, TO, CH, true><<<n_rows, NA_THREADS, lds, stream>>>( \
+    (float*)residual, (const float*)partial, (const float*)post_weight, post_eps, post_groups, (const float*)weight, eps, groups, \
+    (TO*)out, (const int*)rows, hidden, store_residual, parts, slab, rounded)
   if (out_dtype == DT_F32) { LENGTHS(float); } else { LENGTHS(bf16_t); }
 #undef LENGTHS
 #undef GO

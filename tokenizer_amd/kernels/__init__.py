@@ -75,7 +75,10 @@ def _parts_of_k(k: int, splits: int, step: int) -> int:
 class PendingSum:
     """A product whose K was cut over workgroups, before its parts are added: float32 slabs [parts, M, N] and
     the bias that joins their sum.  `Ops.add_rmsnorm` takes it as the delta and adds the parts, the bias and the
-    residual and normalises in one kernel; `resolve()` adds the parts on their own and gives the product."""
+    residual and normalises in one kernel; `resolve()` adds the parts on their own and gives the product.  `rounded`: whoever
+    adds the parts in float rounds their sum to `dtype`, so that a row is the same whether its product was cut or not."""
+
+    rounded = False
 
     def __init__(self, ops: "Ops", partial: torch.Tensor, bias: torch.Tensor | None, dtype: torch.dtype):
         self.ops, self.partial, self.bias, self.dtype = ops, partial, bias, dtype
@@ -159,7 +162,7 @@ class Ops:
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
-                     "ta_rotation_table", "ta_head_norm_rotate_store", "ta_group_norm_add", "ta_group_norm_add_parts", "ta_relu_gate",
+                     "ta_rotation_table", "ta_head_norm_rotate_store", "ta_group_norm_add", "ta_norm_add_parts", "ta_relu_gate",
                      "ta_talking_attention_generic", "ta_talking_decode_bf16", "ta_talking_prefill_bf16",
                      "ta_talking_prefill_parts", "ta_retention_scan", "ta_retention_chunked", "ta_temper_store", "ta_add_slabs_rmsnorm", "ta_experts_few", "ta_experts_few_shared_parts",
                      "ta_fused_qk_temper",
@@ -471,7 +474,7 @@ class Ops:
         n_tokens, hidden = residual.shape
         n_rows = n_tokens if rows is None else rows.numel()
         if any(isinstance(term, PendingSum) for term, _, _ in terms):
-            done = self._add_slabs(residual, terms, weight, eps, out, rows, store_residual, weight2, out2)
+            done = self._add_slabs(residual, terms, weight, eps, out, rows, store_residual, weight2, eps2, out2)
             if done is not None:
                 return done
             terms = tuple((term.resolve() if isinstance(term, PendingSum) else term, factor, scale) for term, factor, scale in terms)
@@ -502,29 +505,37 @@ class Ops:
 
     takes_pending_terms = True      # `add_terms_rmsnorm` takes a product still in parts (`PendingSum`) as a term
 
-    def _add_slabs(self, residual, terms, weight, eps, out, rows, store_residual, weight2, out2) -> torch.Tensor | None:
-        """`add_terms_rmsnorm` of one term of rows and, behind it, a product still in parts, which the same kernel adds up;
-        None for other forms (the caller then adds the parts first)."""
-        if len(terms) != 2 or isinstance(terms[0][0], PendingSum) or weight is None or out2 is not None:
+    def _add_slabs(self, residual, terms, weight, eps, out, rows, store_residual, weight2, eps2, out2) -> torch.Tensor | None:
+        """`add_terms_rmsnorm` of one or two terms of rows and, behind them, a product still in parts, which the same kernel adds
+        up; None for other forms (the caller then adds the parts first)."""
+        if len(terms) not in (2, 3) or any(isinstance(term, PendingSum) for term, _, _ in terms[:-1]):
             return None
-        (first, factor, scale), (parts, slab_factor, slab_scale) = terms
+        plain, (parts, slab_factor, slab_scale) = terms[:-1], terms[-1]
         n_tokens, hidden = residual.shape
         n_rows = n_tokens if rows is None else rows.numel()
-        if (parts.bias is not None or hidden % 4 or hidden > 4096 or out.dtype != torch.bfloat16 or not out.is_contiguous()
-                or (scale is None) != (slab_scale is None)):
+        if (parts.bias is not None or hidden % 4 or hidden > 4096 or out.dtype != torch.bfloat16 or out.dim() != 2 or out.stride(1) != 1
+                or any((scale is None) != (slab_scale is None) for _, _, scale in plain)):
             return None
-        _dev(residual, first, scale, slab_scale, parts.partial, weight, out, rows)
-        _need(residual.dtype == torch.float32 and weight.dtype == torch.float32 and weight.numel() == hidden
-              and tuple(first.shape) == (n_tokens, hidden) == tuple(parts.shape) and first.dtype == out.dtype
-              and tuple(out.shape) == (n_rows, hidden) and parts.partial.dtype == torch.float32 and parts.partial.is_contiguous(),
-              "terms [T, H] in the output's dtype, a float32 residual stream and norm weight")
-        for each in (scale, slab_scale):
-            _need(each is None or (each.dtype == torch.float32 and each.numel() == hidden), "a term's scale is float32 [H]")
+        _dev(residual, slab_scale, parts.partial, weight, rows, weight2, out2)
+        _need(out.is_cuda and tuple(out.shape) == (n_rows, hidden) and out.stride(0) >= hidden, "norm output has the wrong shape")
+        _need(residual.dtype == torch.float32 and tuple(parts.shape) == (n_tokens, hidden) and parts.partial.dtype == torch.float32
+              and parts.partial.is_contiguous(), "terms [T, H] in the output's dtype and a float32 residual stream")
+        for term, _, scale in plain:
+            _dev(term, scale)
+            _need(tuple(term.shape) == (n_tokens, hidden) and term.dtype == out.dtype, "a term is [T, H] in the output's dtype")
+        for scale in [slab_scale] + [scale for _, _, scale in plain]:
+            _need(scale is None or (scale.dtype == torch.float32 and scale.numel() == hidden), "a term's scale is float32 [H]")
+        for w in (weight, weight2):
+            _need(w is None or (w.dtype == torch.float32 and w.numel() == hidden), "norm weight must be float32 [H]")
+        _need(out2 is None or (weight2 is not None and tuple(out2.shape) == (n_rows, hidden) and out2.dtype == out.dtype),
+              "the second output is [R, H] with a weight of its own")
         _need(rows is None or (rows.dtype == torch.int32 and not store_residual), "rows int32, and a subset stores nothing back")
+        (first, f0, scale0), (second, f1, scale1) = (tuple(plain) + ((None, 0.0, None),))[:2]
         status = self.lib.ta_add_slabs_rmsnorm(
-            _ptr(residual), _ptr(first), _ptr(scale), ctypes.c_float(float(factor)), _ptr(parts.partial), _ptr(slab_scale),
-            ctypes.c_float(float(slab_factor)), parts.partial.shape[0], ctypes.c_size_t(n_tokens * hidden), _ptr(weight),
-            ctypes.c_float(eps), _ptr(out), _ptr(rows), n_rows, hidden, int(bool(store_residual)), self._stream())
+            _ptr(residual), len(plain), _ptr(first), _ptr(second), _ptr(scale0), _ptr(scale1), ctypes.c_float(float(f0)),
+            ctypes.c_float(float(f1)), _ptr(parts.partial), _ptr(slab_scale), ctypes.c_float(float(slab_factor)),
+            parts.partial.shape[0], ctypes.c_size_t(n_tokens * hidden), int(parts.rounded), _ptr(weight), ctypes.c_float(eps), _ptr(out), out.stride(0),
+            _ptr(weight2), ctypes.c_float(eps2), _ptr(out2), _ptr(rows), n_rows, hidden, int(bool(store_residual)), self._stream())
         if status == -2:
             return None
         self._check(status, "add_slabs_rmsnorm")
@@ -650,11 +661,11 @@ class Ops:
         off; out = x / sqrt(mean(x^2) + eps) * weight, or x itself without `weight`.  `post_groups`, `groups`: the norm on
         delta (on x) is over so many equal runs of neighbours, each divided by its own root mean square.
 
-        residual float32 [T, H]; delta [T, H] float32 or bfloat16, or a product still in parts (`PendingSum`: norms over
-        groups add them in the same kernel); weights float32 [H]; rows int32 or None; out [rows, H] in delta's dtype or
+        residual float32 [T, H]; delta [T, H] float32 or bfloat16, or a product still in parts (`PendingSum`, added in the same
+        kernel); weights float32 [H]; rows int32 or None; out [rows, H] in delta's dtype or
         float32."""
         if isinstance(delta, PendingSum):
-            if (post_groups != 1 or groups != 1) and delta.bias is None:
+            if delta.bias is None:
                 n_rows, hidden = residual.shape[0] if rows is None else rows.numel(), residual.shape[1]
                 _dev(residual, delta.partial, post_weight, weight, out, rows)
                 _need(residual.dtype == torch.float32 and residual.is_contiguous(), "the residual stream is float32")
@@ -666,12 +677,13 @@ class Ops:
                 _need(rows is None or (rows.dtype == torch.int32 and not store_residual), "a row subset (int32) never stores the residual")
                 _need(post_groups > 0 and groups > 0 and hidden % post_groups == 0 and hidden % groups == 0,
                       "the groups are equal parts of the row")
-                status = self.lib.ta_group_norm_add_parts(
-                    _ptr(residual), _ptr(delta.partial), delta.partial.shape[0], residual.shape[0], _ptr(post_weight),
+                status = self.lib.ta_norm_add_parts(
+                    _ptr(residual), _ptr(delta.partial), delta.partial.shape[0], residual.shape[0],
+                    int(delta.rounded and delta.dtype == torch.bfloat16), _ptr(post_weight),
                     ctypes.c_float(post_eps), post_groups, _ptr(weight), ctypes.c_float(eps), groups, _ptr(out), _ptr(rows), n_rows,
                     hidden, int(store_residual), _code(out.dtype), self._stream())
                 if status != -2:              # -2: rows that only the general kernel takes
-                    self._check(status, "group_norm_add")
+                    self._check(status, "norm_add_parts")
                     return out
             delta = delta.resolve()
         _dev(residual, delta, post_weight, weight, out, rows)
@@ -708,15 +720,24 @@ class Ops:
         """`norm_add_rmsnorm` with a token input between the add and the last norm, in one kernel: with x the stream
         after the add, g = gelu_tanh(gate[:dim] x) * table[token, offset : offset + dim], y = proj[:, :dim] g,
         x += y / sqrt(mean(y^2) + side_eps) * side_norm (stored back unless `rows` selects a subset), out = x /
-        sqrt(mean(x^2) + eps) * weight.  gate [>= dim, H], proj [H, >= dim], table [V, W] and delta share out's dtype.
+        sqrt(mean(x^2) + eps) * weight.  gate [>= dim, H], proj [H, >= dim], table [V, W] and delta share out's dtype; delta may be
+        a product still in parts (`PendingSum`).
         Returns None for sizes the kernel does not take (rows of more than 4,096 elements, dim above 64)."""
+        parts, whole = 0, None
+        if isinstance(delta, PendingSum):
+            if delta.bias is not None or out.dtype != torch.bfloat16 or delta.dtype != out.dtype:
+                delta = delta.resolve()
+            else:
+                _need(delta.shape == tuple(residual.shape) and delta.partial.is_contiguous(), "delta must match the residual's shape")
+                parts, whole = delta.partial.shape[0], delta
+                delta = whole.partial
         _dev(residual, delta, post_weight, gate, proj, side_norm, table, token_ids, weight, out, rows)
         hidden = residual.shape[1]
         if hidden > 4096 or dim > 64:
             return None
         n_rows = residual.shape[0] if rows is None else rows.numel()
         _need(residual.dtype == torch.float32 and residual.is_contiguous(), "the residual stream is float32")
-        _need(delta.shape == residual.shape and delta.is_contiguous() and delta.dtype == out.dtype, "delta [T, H] of out's dtype")
+        _need(parts or (delta.shape == residual.shape and delta.is_contiguous() and delta.dtype == out.dtype), "delta [T, H] of out's dtype")
         _need(tuple(out.shape) == (n_rows, hidden) and out.is_contiguous(), "norm output shape")
         for vector in (post_weight, side_norm, weight):
             _need(vector is None or (vector.dtype == torch.float32 and vector.numel() == hidden), "norm weights are float32 [H]")
@@ -726,11 +747,14 @@ class Ops:
         _need(table.dim() == 2 and 0 <= offset and offset + dim <= table.shape[1], "the table's slice")
         _need(token_ids.dtype == torch.int32 and token_ids.numel() == residual.shape[0], "token ids are int32 [T]")
         _need(rows is None or rows.dtype == torch.int32, "rows are int32")
-        self._check(self.lib.ta_norm_side_norm(
-            _ptr(residual), _ptr(delta), _ptr(post_weight), ctypes.c_float(post_eps), _ptr(gate), _ptr(proj), proj.shape[1],
-            _ptr(side_norm), ctypes.c_float(side_eps), _ptr(table), table.shape[1], _ptr(token_ids), offset, dim, _ptr(weight),
-            ctypes.c_float(eps), _ptr(out), _ptr(rows), n_rows, hidden, int(rows is None), _code(out.dtype), self._stream()),
-            "norm_side_norm")
+        launch = lambda delta, parts: self.lib.ta_norm_side_norm(
+            _ptr(residual), _ptr(delta), parts, residual.shape[0], int(parts > 0 and whole.rounded), _ptr(post_weight), ctypes.c_float(post_eps), _ptr(gate), _ptr(proj),
+            proj.shape[1], _ptr(side_norm), ctypes.c_float(side_eps), _ptr(table), table.shape[1], _ptr(token_ids), offset, dim,
+            _ptr(weight), ctypes.c_float(eps), _ptr(out), _ptr(rows), n_rows, hidden, int(rows is None), _code(out.dtype), self._stream())
+        status = launch(delta, parts)
+        if status == -3:                      # sizes whose kernels take rows alone
+            status = launch(whole.resolve(), 0)
+        self._check(status, "norm_side_norm")
         return out
 
     def norm_rotate_store(self, qkv: torch.Tensor, bias: torch.Tensor | None, positions: torch.Tensor,
@@ -1500,7 +1524,7 @@ class Ops:
     talking_workgroups = 512      # what the single tokens' split of the keys aims at
 
     # --------------------------------------------------------------------- linear
-    takes_pending_groups = True   # `norm_add_rmsnorm` over groups takes a product still in parts as its delta
+    takes_pending_normed = True   # `norm_add_rmsnorm` and `norm_side_norm` take a product still in parts as their delta
     takes_pending = True      # `linear(pending=True)` and `add_rmsnorm` with a `PendingSum` exist here
 
     def linear(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,

@@ -225,17 +225,24 @@ class NormedDelta:
 
 class SumDelta:
     """What a layer whose two sub-layers read the same normalised rows hands on: their outputs `first` and `second`
-    [T, H] (compute dtype), still to be added to each other and to the stream, x + (first + second) in float32.  A norm
-    of the form x / sqrt(mean(x^2) + eps) * w takes it as its delta and does the two additions and the norm in one
-    kernel (`ops.add_pair_rmsnorm`); for anyone else `resolve()` gives the sum as a float32 tensor."""
+    [T, H] (compute dtype; `second` may be a product still in parts), still to be added to each other and to the stream,
+    x + (first + second) in float32.  A norm of the form x / sqrt(mean(x^2) + eps) * w takes it as its delta and does the
+    additions and the norm in one kernel (`join`); for anyone else `resolve()` gives the sum as a float32 tensor."""
 
     def __init__(self, ops, first: torch.Tensor, second: torch.Tensor):
         self.ops, self.first, self.second = ops, first, second
 
+    def join(self, residual: torch.Tensor, weight, eps: float, out: torch.Tensor, rows=None, store_residual: bool = True) -> torch.Tensor:
+        """The stream with both terms added (stored back unless told not to), normalised by `weight` (as it is where that is
+        None) into `out`."""
+        if hasattr(self.second, "partial"):
+            return self.ops.add_terms_rmsnorm(residual, ((self.first, 1.0, None), (self.second, 1.0, None)), weight, eps, out, rows,
+                                              store_residual=store_residual)
+        return self.ops.add_pair_rmsnorm(residual, self.first, self.second, weight, eps, out, rows, store_residual=store_residual)
+
     def resolve(self) -> torch.Tensor:
         zero = torch.zeros(self.first.shape, dtype=torch.float32, device=self.first.device)
-        rows = torch.empty(self.first.shape, dtype=self.first.dtype, device=self.first.device)
-        self.ops.add_pair_rmsnorm(zero, self.first, self.second, None, 0.0, rows)
+        self.join(zero, None, 0.0, torch.empty(self.first.shape, dtype=self.first.dtype, device=self.first.device))
         return zero
 
 
@@ -281,6 +288,13 @@ def as_tensor(delta):
     """The delta as a tensor: a product still in parts has them added now."""
     resolve = getattr(delta, "resolve", None)
     return resolve() if resolve is not None and not isinstance(delta, torch.Tensor) else delta
+
+
+def rounded_sum(delta):
+    """A sub-layer's output whose sum, if it is a product still in parts, is to be rounded as a whole product is."""
+    if hasattr(delta, "partial"):
+        delta.rounded = True
+    return delta
 
 
 def can_fuse_decode(ops, residual, dtype) -> bool:

@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .base import BLOCKS, Block, NormedDelta, Repeatable, ScaledSum, SumDelta, as_tensor, repeatable_of
+from .base import BLOCKS, Block, NormedDelta, Repeatable, ScaledSum, SumDelta, as_tensor, repeatable_of, rounded_sum
 from .spec import TensorSpec
 
 
@@ -57,7 +57,10 @@ class ParallelBlock(Block):
         mixed = self.mixer.forward(h, ctx, cache)
         if self.feed_forward is None:
             return mixed
-        return SumDelta(self.mixer.runtime.ops, mixed, self.feed_forward.forward(h, ctx))
+        ops = self.mixer.runtime.ops
+        # (A feed-forward that can leave its last product in parts may: the next norm adds them up in its kernel.)
+        run = getattr(self.feed_forward, "forward_pending", self.feed_forward.forward)
+        return SumDelta(ops, mixed, rounded_sum(run(h, ctx)))
 
 
 @BLOCKS.register("parallel_scaled")
@@ -115,12 +118,13 @@ class ScaledParallelBlock(Block):
         h1, h2 = self._normed(residual, delta)
         out = ScaledSum.of(ops, self.mixer.forward(h1, ctx, cache)).scaled_by(self.mixer_scale)
         if self.feed_forward is not None:
-            # (Behind one term of rows, a feed-forward that can leave its last product in parts may: the next norm adds
+            # (Behind one or two terms of rows, a feed-forward that can leave its last product in parts may: the next norm adds
             # them up in its kernel.)
             run = self.feed_forward.forward
-            if len(out.terms) == 1:
+            if len(out.terms) <= 2:
                 run = getattr(self.feed_forward, "forward_pending", run)
-            out = out.plus(ScaledSum.of(ops, run(h2, ctx)).scaled_by(self.ff_scale))
+            last = run(h2, ctx)
+            out = out.plus(ScaledSum.of(ops, last if len(out.terms) == 1 else rounded_sum(last)).scaled_by(self.ff_scale))
         return out
 
 
@@ -178,7 +182,10 @@ class SandwichNormBlock(Block):
             mixed = self.mixer.forward(self.mixer_norm.apply(residual, delta), ctx, cache)
             delta = NormedDelta(ops, mixed, self.after_mixer, self.eps)
         if self.feed_forward is not None:
-            out = self.feed_forward.forward(self.feed_forward_norm.apply(residual, delta), ctx)
+            run = self.feed_forward.forward                # (or with its last product left in parts for the norm behind it)
+            if getattr(ops, "takes_pending_normed", False):
+                run = getattr(self.feed_forward, "forward_in_parts", getattr(self.feed_forward, "forward_pending", run))
+            out = rounded_sum(run(self.feed_forward_norm.apply(residual, delta), ctx))
             delta = NormedDelta(ops, out, self.after_feed_forward, self.eps)
         if self.side_dim:
             if isinstance(delta, NormedDelta) and delta.side is None:
@@ -199,7 +206,7 @@ class _TokenInput:
         has none for these sizes."""
         block = self.block
         run = getattr(block.runtime.ops, "norm_side_norm", None)
-        if run is None or out.dtype != delta.rows.dtype or not isinstance(delta.rows, torch.Tensor):
+        if run is None or out.dtype != delta.rows.dtype:
             return None
         return run(residual, delta.rows, delta.weight, delta.eps, block.side_gate, block.side_proj, block.side_norm,
                    block.eps, block.side_table, self.token_ids, block.side_offset, block.side_dim, weight, eps, out, rows)
@@ -275,8 +282,8 @@ class PostNormBlock(Block):
             if part is self.mixer:
                 out = part.forward(x, ctx, cache)
             else:
-                # (Norms over groups add a product's parts in their own kernel; the others would need one for the addition.)
-                in_parts = norm.groups > 1 and getattr(ops, "takes_pending_groups", False)
+                # (Norms over groups add a product's parts in their own kernel.)
+                in_parts = norm.groups > 1 and getattr(ops, "takes_pending_normed", False)
                 out = getattr(part, "forward_in_parts", part.forward)(x, ctx) if in_parts else part.forward(x, ctx)
             delta = NormedDelta(ops, out, weight, norm.eps, groups=norm.groups)
         return delta

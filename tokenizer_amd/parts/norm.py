@@ -47,8 +47,7 @@ class RMSNorm(Norm):
         if self.groups != 1 and isinstance(delta, (SumDelta, ScaledSum)):
             delta = delta.resolve()
         if isinstance(delta, SumDelta):
-            return self.runtime.ops.add_pair_rmsnorm(residual, delta.first, delta.second, self.weight, self.eps, out, rows,
-                                                     store_residual=rows is None)
+            return delta.join(residual, self.weight, self.eps, out, rows, store_residual=rows is None)
         if isinstance(delta, ScaledSum):
             return self.runtime.ops.add_terms_rmsnorm(residual, delta.terms, self.weight, self.eps, out, rows,
                                                       store_residual=rows is None)
