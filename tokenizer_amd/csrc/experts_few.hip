@@ -3,23 +3,18 @@
 // the second product, whose results lie pick by pick (slab k holds every row's k-th pick), for whoever adds them up.
 // bfloat16 operands, float sums on the matrix cores (16x16x32), computed transposed, C^T = W x^T, as the weight-streaming
 // product does: sixteen weight rows are the M side, up to sixteen (row, pick) pairs of the expert the N side, the waves of a
-// workgroup take turns of 64 elements of K and add up through LDS.  An expert that every row uses besides (of an inner width of
+// workgroup take turns of 64 elements of K and add up through LDS.  Bound by the chosen matrices' way from memory: they are read line
+// by line (`lines_to_rows` in common.h) and past the caches, which no later workgroup asks them from.  (Sixteen rows' half lines a load |
+// whole lines | whole lines past the caches, us for both products: 2 of 8 experts of 9,472 over 3,584, four rows, 197 | 177 | 160
+// (6.4 TB/s); 2 of 8 of 2,240 and a shared one of 4,480 over 1,536, three rows, 42.3 | 37.3 | 34.4; half lines past the caches 215 and
+// 44.8: each line then comes twice.  Weights that are in the caches already, a model far smaller than them: level to 5 % slower.)  An expert that every row uses besides (of an inner width of
 // its own) is one further expert in both grids, whose pairs are the rows; its K in the second product is cut into parts about
 // as long as the others', each a slab of its own.
 #include "common.h"
 
-typedef __bf16 ef_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float ef_floatx4 __attribute__((ext_vector_type(4)));
 
 #define EF_MAX_PAIRS 256
-
-__device__ __forceinline__ ef_bf16x8 ef_load8(const bf16_t* p, bool ok) {
-  ef_bf16x8 z;
-  if (ok) return *reinterpret_cast<const ef_bf16x8*>(p);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) z[i] = (__bf16)0.0f;
-  return z;
-}
 
 // The pairs of this workgroup's expert, in rising order: every wave counts them for itself (the count is the same for all),
 // the first wave lists them in LDS.
@@ -41,33 +36,44 @@ __device__ __forceinline__ int ef_pairs_of(const int* __restrict__ chosen, int n
 // The expert that all rows use: `inner` 0 says that there is none.  Its matrices stand behind the others'; weights null: 1.
 struct EfShared { int inner; const float* weights; bf16_t* act; int parts, length; };   // K of `inner` in `parts` of `length`
 
-// acc[h] += sixteen rows of matrix h (row `wrow` + h * second of W, K elements `ldw` apart) times the lane's row of x, over this
-// wave's turns of K.
+// acc[h] += sixteen rows of matrix h (lane (col, g): `w_at[h][0]` is row col % 8 of them, `w_at[h][1]` row 8 + col % 8) times the
+// lane's row of x, over this wave's turns of K.
 template <int NW, int HALVES>
-__device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES], const bf16_t* x_at, bool x_ok, int K, int g, int wave,
+__device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], const bf16_t* x_at, bool x_ok, int K, int wave,
                                         ef_floatx4 (&acc)[HALVES]) {
-  constexpr int UN = HALVES == 2 ? 2 : 4;                    // turns asked for at once
+  // Turns asked for at once: four loads of weights a lane of two matrices (twice as many take registers that more waves a
+  // compute unit make better use of: twelve rows of the second example above 46.0 | 44.5 us), eight of one (four: 44.6).
+  constexpr int UN = HALVES == 2 ? 1 : 4;
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, piece = 2 * g + (col >> 3);
   const int turns = (K + 63) / 64;
+  const word4 zero = {0u, 0u, 0u, 0u};
   for (int first = wave; first < turns; first += UN * NW) {
-    ef_bf16x8 wf[UN][HALVES][2], xf[UN][2];
+    word4 wf[UN][HALVES][2], xf[UN][2];
 #pragma unroll
     for (int q = 0; q < UN; ++q) {
       const int turn = first + q * NW, at = min(turn, turns - 1) * 64;
+      const bool w_in = turn < turns && at + 8 * piece < K;
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const bool in = turn < turns && at + 32 * s + 8 * g < K;
+      for (int h = 0; h < HALVES; ++h)
 #pragma unroll
-        for (int h = 0; h < HALVES; ++h) wf[q][h][s] = ef_load8(w_at[h] + at + 32 * s, in);
-        xf[q][s] = ef_load8(x_at + at + 32 * s, in && x_ok);
+        for (int hh = 0; hh < 2; ++hh)
+          wf[q][h][hh] = w_in ? __builtin_nontemporal_load(reinterpret_cast<const word4*>(w_at[h][hh] + at + 8 * piece)) : zero;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {                          // what the weights are after the exchange: the bytes 2 g and 2 g + 1
+        const bool x_in = turn < turns && at + 16 * g + 8 * s < K;
+        xf[q][s] = x_in && x_ok ? *reinterpret_cast<const word4*>(x_at + at + 16 * g + 8 * s) : zero;
       }
     }
 #pragma unroll
     for (int q = 0; q < UN; ++q)
 #pragma unroll
-      for (int s = 0; s < 2; ++s)
+      for (int h = 0; h < HALVES; ++h) {
+        line_bf16x8 part[2];
+        lines_to_rows(wf[q][h][0], wf[q][h][1], col < 8, part[0], part[1]);
 #pragma unroll
-        for (int h = 0; h < HALVES; ++h)
-          acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[q][h][s], xf[q][s], acc[h], 0, 0, 0);
+        for (int s = 0; s < 2; ++s)
+          acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[s], __builtin_bit_cast(line_bf16x8, xf[q][s]), acc[h], 0, 0, 0);
+      }
   }
 }
 
@@ -100,18 +106,19 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
   }
   if (count == 0 || n0 >= inner) return;                     // nobody's expert, or past its width: the same for the whole workgroup
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = wave_index(), col = lane & 15, g = lane >> 4;
-  const bf16_t* w_at[HALVES];
+  const int lane = threadIdx.x & 63, wave = wave_index(), col = lane & 15;
+  const bf16_t* w_at[HALVES][2];
 #pragma unroll
   for (int h = 0; h < HALVES; ++h)
-    w_at[h] = first + ((size_t)h * inner + min(n0 + col, inner - 1)) * hidden + 8 * g;
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) w_at[h][hh] = first + ((size_t)h * inner + min(n0 + 8 * hh + (col & 7), inner - 1)) * hidden;
   for (int p0 = 0; p0 < count; p0 += 16) {
     const bool ok = p0 + col < count;
-    const bf16_t* x_at = x + (size_t)(list[min(p0 + col, count - 1)] / top) * x_stride + 8 * g;
+    const bf16_t* x_at = x + (size_t)(list[min(p0 + col, count - 1)] / top) * x_stride;
     ef_floatx4 acc[HALVES];
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) acc[h] = (ef_floatx4){0.f, 0.f, 0.f, 0.f};
-    ef_walk<NW, HALVES>(w_at, x_at, ok, hidden, g, wave, acc);
+    ef_walk<NW, HALVES>(w_at, x_at, ok, hidden, wave, acc);
     // A matrix instruction's result may be read eight wait states behind it at the earliest.  The compiler leaves them out in front
     // of the stores below where there is one matrix (the store is the second instruction behind the last sum; with many
     // workgroups some stored a sum that was not there yet), so they are here, twice over; with two matrices it has them.
@@ -182,13 +189,14 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
   }
   if (count == 0) return;
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = wave_index(), col = lane & 15, g = lane >> 4;
-  const bf16_t* const w_at[1] = {columns + (size_t)min(n0 + col, hidden - 1) * ldw + 8 * g};
+  const int lane = threadIdx.x & 63, wave = wave_index(), col = lane & 15;
+  const bf16_t* const w_at[1][2] = {{columns + (size_t)min(n0 + (col & 7), hidden - 1) * ldw,
+                                     columns + (size_t)min(n0 + 8 + (col & 7), hidden - 1) * ldw}};
   for (int p0 = 0; p0 < count; p0 += 16) {
     const bool ok = p0 + col < count;
-    const bf16_t* x_at = act + (size_t)list[min(p0 + col, count - 1)] * stride + 8 * g;
+    const bf16_t* x_at = act + (size_t)list[min(p0 + col, count - 1)] * stride;
     ef_floatx4 acc[1] = {(ef_floatx4){0.f, 0.f, 0.f, 0.f}};
-    ef_walk<NW, 1>(w_at, x_at, ok, inner, g, wave, acc);
+    ef_walk<NW, 1>(w_at, x_at, ok, inner, wave, acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave][r][lane] = acc[0][r];
     __syncthreads();

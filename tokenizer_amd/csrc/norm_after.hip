@@ -565,7 +565,7 @@ norm_side_norm_held_kernel(float* __restrict__ residual, const void* __restrict_
     next[c] = weight ? *reinterpret_cast<const float2*>(weight + h) : make_float2(1.f, 1.f);
   }
   if constexpr (PARTS) {
-    constexpr int DEEP = R * RUNS <= 4 ? 4 : 2;              // slabs asked for at a time
+    constexpr int DEEP = R * RUNS <= 2 ? 8 : R * RUNS <= 4 ? 4 : 2;              // slabs asked for at a time
     for (int s0 = 1; s0 < parts; s0 += DEEP) {
       float2 v[DEEP][R][RUNS];
 #pragma unroll
