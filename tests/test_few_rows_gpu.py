@@ -336,3 +336,43 @@ def test_norm_rotation_and_store_of_many_tokens_and_of_few(ops, n_q, n_k, n_v, d
                                   wq, wk, 1e-5)
         for mine, right in zip(got, want):
             torch.testing.assert_close(mine.cpu().float(), right.float(), rtol=bound, atol=1e-5)
+
+
+# Weights read by whole cache lines (a K of whole lines, more than a trip of them) against the plain product: rows on either side of
+# eight and up to sixteen, blocks of sixteen weight rows with only some of them there, K that leaves some waves a line less than
+# others, that is one trip of a wave's whole share and that is several, four to sixteen waves, and a K that is no multiple of a line.
+@pytest.mark.parametrize("rows", [1, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(24, 1088), (24, 1536), (4104, 1536), (20, 4160), (40, 5184), (16400, 640), (1540, 8256), (60, 3840), (40, 5192)])
+def test_weights_by_whole_lines(ops, rows, n, k):
+    x, w = rand_bf16((rows, k + 8), 7)[:, :k], (rand_bf16((2 * n, k), 8).float() * 0.05).to(torch.bfloat16)
+    bias = torch.randn(n, generator=torch.Generator().manual_seed(9)).cuda()
+    exact = x.double() @ w.double().t()
+    first, second = exact[:, :n], exact[:, n:]
+    gated = first / (1 + torch.exp(-first)) * second
+
+    def near(got, want):                       # float sums of K terms, and one rounding of the result to bfloat16 (2^-9)
+        assert float((got.double() - want).abs().max()) <= 2 ** -8 * max(1.0, float(want.abs().max()))
+
+    near(ops.linear(x, w[:n], bias), first + bias)
+    parts = ops.linear(x, w[:n], bias, pending=True)
+    near(parts if isinstance(parts, torch.Tensor) else parts.resolve(), first + bias)
+    near(ops.linear_silu_gate(x, w), gated)
+    near(ops.fused_norm_gated(x.contiguous(), None, 1e-6, w), gated)
+    residual = torch.randn(rows, n, generator=torch.Generator().manual_seed(10)).cuda()
+    want = residual.double() + first + bias
+    ops.linear_add(x.contiguous(), w[:n], bias, residual)
+    near(residual, want)
+
+
+@pytest.mark.parametrize("rows", [1, 16])
+@pytest.mark.parametrize("k", [2112, 3584])
+def test_qkv_by_whole_lines(ops, rows, k):
+    heads, kv, d, page = 3, 1, 32, 16
+    x, w = rand_bf16((rows, k), 11), (rand_bf16(((heads + 2 * kv) * d, k), 12).float() * 0.05).to(torch.bfloat16)
+    positions = torch.arange(rows, dtype=torch.int32, device="cuda")
+    k_pages = torch.zeros(1, kv, page, d, dtype=torch.bfloat16, device="cuda")
+    v_pages = torch.zeros(1, kv, d, page, dtype=torch.bfloat16, device="cuda")
+    q = ops.fused_norm_qkv_rope(x, None, 1e-6, w, None, positions, None, positions, k_pages, v_pages, heads, kv, d)
+    want = x.double() @ w.double().t()
+    got = torch.cat([q, k_pages[0, 0, :rows], v_pages[0, 0, :, :rows].t()], dim=1)
+    assert float((got.double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max())

@@ -70,7 +70,14 @@ __device__ __forceinline__ bf16x8 any8() {
 // epilogue then begin without any fetch of arguments (the bias, which only the epilogue needs, lies behind).  One pointer serves for the rows (bfloat16, or the float residual for the norm
 // prologue) and one for the result (bfloat16 rows, or the float residual that is added to), which never occur
 // together.  The rotation's own arguments lie behind; only wave 0, which writes the results, waits for them.
-template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES>
+//
+// LINES (K a multiple of 64): the weights come by whole cache lines (`lines_to_rows` in common.h), past the caches, which hold nothing
+// that comes again: a pair of steps is one line of each of a block's sixteen rows, u even its lower eight rows, u odd its upper
+// eight.  For walks of several trips; where all is asked for in one trip of four steps there is nothing to stream (896 columns level).
+// Us, sixteen rows' half lines a load | so, one input row and sixteen, weights from memory: gate/up 18,944 over 3,584 55.5 | 46.1
+// and 68.8 | 54.0, down 18,944 to 3,584 26.4 | 25.4 and 36.2 | 34.4, q/k/v of 3,584 13.8 | 11.3 and 16.1 | 12.3, gate/up 8,960 over 1,536
+// 17.8 | 17.0 and 22.6 | 18.1, down 8,960 to 1,536 11.2 | 9.7 and 15.2 | 14.2, down 4,864 to 896 6.4 | 5.8 and 9.2 | 8.7.
+template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES>
 __global__ void __launch_bounds__(NW * WAVE)
 fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const float* norm_weight,
                     int m, int n, int k, int rows, int lda, float eps, const float* bias,
@@ -121,13 +128,15 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
   const int n_limit = (EPI == EPI_GATED) ? p.n / 2 : p.n;
   const bf16_t* w0[PASSES];
   const bf16_t* w1[PASSES];
-  bool w_lane[PASSES];
+  bool w_lane[PASSES], w_upper[PASSES];                     // LINES: the lane's row of the lower eight, of the upper eight
+  const int piece = LINES ? 2 * g + (col >> 3) : g;
 #pragma unroll
   for (int ps = 0; ps < PASSES; ++ps) {
-    const int r = 16 * ps + col;
+    const int r = 16 * ps + (LINES ? col & 7 : col);
     w_lane[ps] = r < R && row0 + r < n_limit;
-    w0[ps] = p.w + (size_t)min(row0 + r, n_limit - 1) * K + 8 * g;
-    w1[ps] = p.w + (size_t)min(row1 + r, p.n - 1) * K + 8 * g;
+    w_upper[ps] = LINES && r + 8 < R && row0 + r + 8 < n_limit;
+    w0[ps] = p.w + (size_t)min(row0 + r, n_limit - 1) * K + 8 * piece;
+    w1[ps] = p.w + (size_t)min(row1 + r, p.n - 1) * K + 8 * piece;
   }
   const bool a_lane = col < M;
   const int a_m = min(col, M - 1);
@@ -160,8 +169,23 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
   // Step j of a wave's batch: steps come in pairs (128 contiguous bytes of a weight row, one cache line),
   // pair q of the batch starting at pair `base` is pair base + q * NW.
   auto step_of = [&](int base_pair, int u) { return (base_pair + (u >> 1) * NW) * 2 + (u & 1); };
+  const int pairs = (full_steps + 1) / 2;
   bf16x8 wf[HELD][UN][SETS];
   auto load_w = [&](int held, int ps, int base_pair) {
+    if constexpr (LINES) {
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        const int pair = base_pair + (u >> 1) * NW;
+        const int at = min(pair, pairs - 1) * 64 + (u & 1) * 8 * K;      // (the upper rows' place is only used by lanes that have one)
+        wf[held][u][0] = ONE ? any8() : fz8();
+        if (SETS == 2) wf[held][u][SETS - 1] = ONE ? any8() : fz8();
+        if ((u & 1 ? w_upper[ps] : w_lane[ps]) && (ONE || pair < pairs)) {
+          wf[held][u][0] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(w0[ps] + at));
+          if (SETS == 2) wf[held][u][SETS - 1] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(w1[ps] + at));
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       const int step = min(step_of(base_pair, u), max(full_steps - 1, 0));   // clamped loads are not used
@@ -180,13 +204,17 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
 #pragma unroll
     for (int ps = 1; ps < PASSES; ++ps) load_w(HELD - PASSES + ps, ps, wave);
   }
-  const bf16_t* ar = NORM ? nullptr : p.a + (size_t)a_m * p.lda + 8 * g;
+  // LINES: the lane's part of the rows for steps u and u + 1 of a pair is their sixteen bytes 2 g and 2 g + 1 of the line.
+  auto a_line = [&](int base_pair, int u) { return min(base_pair + (u >> 1) * NW, pairs - 1) * 64 + 8 * (u & 1); };
+  auto a_inside = [&](int base_pair, int u) { return base_pair + (u >> 1) * NW < pairs; };
+  constexpr int LANE_K = LINES ? 16 : 8;
+  const bf16_t* ar = NORM ? nullptr : p.a + (size_t)a_m * p.lda + LANE_K * g;
   bf16x8 af_one[ONE ? UN : 1];
   if (ONE && !NORM) {                                      // the rows' fragments as well
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       // (every lane: a row past the end repeats the last one and only feeds columns that are never stored)
-      af_one[u] = *reinterpret_cast<const bf16x8*>(ar + min(step_of(wave, u), max(full_steps - 1, 0)) * 32);
+      af_one[u] = *reinterpret_cast<const bf16x8*>(ar + (LINES ? a_line(wave, u) : min(step_of(wave, u), max(full_steps - 1, 0)) * 32));
     }
   }
 
@@ -279,7 +307,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
     }
     __syncthreads();
   }
-  const uint16_t* as_row = a_s + (size_t)a_m * lds_stride + 8 * g;
+  const uint16_t* as_row = a_s + (size_t)a_m * lds_stride + LANE_K * g;
   auto load_a = [&](int k) -> bf16x8 {
     if (NORM) return *reinterpret_cast<const bf16x8*>(as_row + k);
     return a_lane ? *reinterpret_cast<const bf16x8*>(ar + k) : fz8();
@@ -290,7 +318,60 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
     floatx4 acc[SETS];
 #pragma unroll
     for (int s = 0; s < SETS; ++s) acc[s] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    if constexpr (ONE) {
+    if constexpr (LINES) {
+      auto multiply = [&](const bf16x8 (&w)[UN][SETS], const bf16x8 (&af)[UN]) {
+#pragma unroll
+        for (int u = 0; u < UN; u += 2)
+#pragma unroll
+          for (int s = 0; s < SETS; ++s) {
+            bf16x8 b0, b1;
+            lines_to_rows(__builtin_bit_cast(word4, w[u][s]), __builtin_bit_cast(word4, w[u + 1][s]), col < 8, b0, b1);
+            acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, af[u], acc[s], 0, 0, 0);
+            acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, af[u + 1], acc[s], 0, 0, 0);
+          }
+      };
+      bf16x8 af[UN];
+      if constexpr (ONE) {
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+          af[u] = NORM ? load_a(a_line(wave, u)) : af_one[u];
+          if (!a_inside(wave, u)) af[u] = fz8();             // past the end of K: zeros, see below
+        }
+        multiply(wf[HELD - PASSES + ps], af);
+      } else {
+        // The next batch's weights, and rows that come from memory, are requested before the current one is multiplied (rows asked for with
+        // their own batch would wait in line behind the weights just asked for: down 18,944 to 3,584 33 us in place of 26).
+        bf16x8 next[UN];
+        auto ask_rows = [&](int pair) {
+#pragma unroll
+          for (int u = 0; u < UN; ++u) {
+            next[u] = fz8();
+            if (a_lane && a_inside(pair, u)) next[u] = *reinterpret_cast<const bf16x8*>(ar + a_line(pair, u));
+          }
+        };
+        if (!NORM) ask_rows(wave);
+        for (int pair = wave; pair < pairs; pair += (UN / 2) * NW) {
+          bf16x8 wc[UN][SETS];
+#pragma unroll
+          for (int u = 0; u < UN; ++u) {
+            wc[u][0] = wf[0][u][0];
+            if (SETS == 2) wc[u][SETS - 1] = wf[0][u][SETS - 1];
+            if (NORM) {
+              af[u] = load_a(a_line(pair, u));
+              if (!a_inside(pair, u)) af[u] = fz8();
+            } else {
+              af[u] = next[u];
+            }
+          }
+          if (pair + (UN / 2) * NW < pairs) {
+            load_w(0, ps, pair + (UN / 2) * NW);
+            if (!NORM) ask_rows(pair + (UN / 2) * NW);
+          }
+          multiply(wc, af);
+        }
+        if (ps + 1 < PASSES) load_w(0, ps + 1, wave);
+      }
+    } else if constexpr (ONE) {
 #pragma unroll
       for (int u = 0; u < UN; ++u) {
         // A step past the end of K is multiplied all the same, with zeros for the rows: no matrix instruction
@@ -324,7 +405,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
       }
       if (ps + 1 < PASSES) load_w(0, ps + 1, wave);          // the next block's first batch, before this one's sums
     }
-    if (K & 31) {                                            // tail of K (a multiple of 8): zero-filled; wave 0's
+    if (!LINES && (K & 31)) {                                            // tail of K (a multiple of 8): zero-filled; wave 0's
       const int k = full_steps * 32;
       const bool ok = wave == 0 && k + 8 * g < K;
       const bf16x8 af = ok ? load_a(k) : fz8();
@@ -405,14 +486,14 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
   }
 }
 
-template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES>
+template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES = false>
 static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
   size_t lds = NORM ? (size_t)args.m * (args.k + 8) * sizeof(uint16_t) : 0;
   if (lds > 48 * 1024) {
     // More dynamic LDS than the default limit: ask for it (the device has 160 KB per compute unit).
     if (lds > 140 * 1024) return -1;
     hipError_t err = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES>),
+        reinterpret_cast<const void*>(&fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return (int)err;
   }
@@ -420,7 +501,7 @@ static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
   const bool from_residual = args.residual_in != nullptr;
   if (from_residual != (args.norm_weight != nullptr) || (!from_residual && !args.a) || !args.w) return -1;
   if (EPI == EPI_RESIDUAL ? !args.residual_out : !args.out) return -1;
-  fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES><<<tiles, NW * WAVE, lds, stream>>>(
+  fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES><<<tiles, NW * WAVE, lds, stream>>>(
       args.w, from_residual ? (const void*)args.residual_in : (const void*)args.a,
       EPI == EPI_RESIDUAL ? (void*)args.residual_out : (void*)args.out, args.norm_weight, args.m, args.n,
       args.k, args.rows, args.lda, args.eps, args.bias, args.positions, args.cos_sin, args.slots, args.k_pages, args.v_pages,
@@ -433,6 +514,7 @@ static int launch_one(const FusedArgs& args, int tiles, hipStream_t stream) {
   // Steps of a wave: pairs of steps are dealt round-robin to the waves.
   const int pairs = (args.k / 32 + 1) / 2;
   const int steps_per_wave = 2 * ((pairs + NW - 1) / NW);
+  const bool whole = (args.k & 63) == 0;                     // K in whole cache lines
   if (steps_per_wave <= 4) return launch_kernel<NW, EPI, NORM, 4, true, PASSES>(args, tiles, stream);
   if constexpr (NORM && (EPI == EPI_ROPE_STORE || PASSES == 1)) {
     // Rows in LDS: only the weights take registers, and a wave's whole share of up to eight steps is one trip
@@ -440,6 +522,7 @@ static int launch_one(const FusedArgs& args, int tiles, hipStream_t stream) {
     // The gated product's matrix is several workgroups for every compute unit: it takes a whole share at once only
     // while two workgroups' registers fit a unit together, which is one block of rows and six steps (with two blocks
     // of rows 19.9 -> 22.3 us at 8,960 x 1,536, with eight steps 25.4 -> 31.3 us at 11,008 x 2,048).
+    if (EPI == EPI_GATED && whole && steps_per_wave <= 6) return launch_kernel<NW, EPI, NORM, 6, true, PASSES, true>(args, tiles, stream);
     if (steps_per_wave <= 6) return launch_kernel<NW, EPI, NORM, 6, true, PASSES>(args, tiles, stream);
     if constexpr (EPI == EPI_ROPE_STORE)
       if (steps_per_wave <= 8) return launch_kernel<NW, EPI, NORM, 8, true, PASSES>(args, tiles, stream);
@@ -447,8 +530,15 @@ static int launch_one(const FusedArgs& args, int tiles, hipStream_t stream) {
   if constexpr (!NORM && PASSES == 1) {
     // Rows from memory: one trip for a wave's whole share if it fits the registers (128 a lane at 16 waves).
     if (steps_per_wave <= 8) return launch_kernel<NW, EPI, NORM, 8, true, 1>(args, tiles, stream);
+    if (whole && steps_per_wave <= 10) return launch_kernel<NW, EPI, NORM, 10, true, 1, true>(args, tiles, stream);
     if (steps_per_wave <= 10) return launch_kernel<NW, EPI, NORM, 10, true, 1>(args, tiles, stream);
   }
+  if constexpr (EPI == EPI_RESIDUAL && PASSES == 1) {
+    // One set of weight rows leaves registers for three lines a trip; with more input rows the wider trip gains nothing.  Four steps |
+    // six, 8 rows: down 8,960 to 1,536 11.8 | 11.1 us (one row 11.3 | 9.7), 18,944 to 3,584 28.4 | 28.7; 16 rows 14.2 | 14.2, 34.4 | 35.2.
+    if (whole && args.m <= 8) return launch_kernel<NW, EPI, NORM, 6, false, PASSES, true>(args, tiles, stream);
+  }
+  if (whole) return launch_kernel<NW, EPI, NORM, 4, false, PASSES, true>(args, tiles, stream);
   return launch_kernel<NW, EPI, NORM, 4, false, PASSES>(args, tiles, stream);
 }
 

@@ -30,7 +30,7 @@ __device__ __forceinline__ void store1(float* p, float v) { *p = v; }
 __device__ __forceinline__ void store1(bf16_t* p, float v) { p->bits = float_to_bf16_bits(v); }
 
 // grid.x: tiles of 16 output columns (of N, or of N/2 with GATED).  NW waves per workgroup.
-// grid.y: parts of K of `k_chunk` elements (a multiple of 32) each: with more than one, a workgroup writes the
+// grid.y: parts of K of `k_chunk` elements (a multiple of 32, of 64 with LINES) each: with more than one, a workgroup writes the
 // float sums of its part into its slab of `partial` [parts, M, N] and `splitk_reduce` finishes the product.  That is
 // for few output tiles and a long K (the down projection of a decode batch): every compute unit gets a share.
 //
@@ -47,9 +47,9 @@ struct RopeStore {
 // NB: blocks of sixteen output columns per workgroup.  Every workgroup reads all the rows of A for its part of K;
 // with two blocks the rows are read half as often, which is what a product of many rows is bound by once the
 // rows outweigh a tile's weights (what comes over the fabric from the caches counts like what comes from memory).
-// LINES: the weights are read line by line (`lines_to_rows` in common.h), K walked in steps of 64; for products that
-// are one long stream over a big matrix.
-template <int MB, int NW, bool GATED, typename OutT, bool ROPE = false, int NB = 1, bool LINES = false>
+// LINES > 0: the weights are read line by line (`lines_to_rows` in common.h), K walked in steps of 64, LINES steps at a time, past the
+// caches (a stream that does not come again): for products that are one long stream over a big matrix.  WHOLE: K is a multiple of 64.
+template <int MB, int NW, bool GATED, typename OutT, bool ROPE = false, int NB = 1, int LINES = 0, bool WHOLE = false>
 __global__ void __launch_bounds__(NW * WAVE)
 skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf16_t* __restrict__ W,
                    OutT* __restrict__ C, int ldc, int M, int N, int K_all, float* __restrict__ partial,
@@ -102,7 +102,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
     for (int mb = 0; mb < MB; ++mb) acc[s][mb] = (floatx4){0.f, 0.f, 0.f, 0.f};
 
   constexpr int UN = (SETS * MB > 4) ? 2 : 4;
-  if constexpr (LINES) {
+  if constexpr (LINES > 0) {
     const int sub = col & 7, piece = 2 * g + (col >> 3);
     const bool low_lane = col < 8;
     const bf16_t* wl[SETS][2];
@@ -116,7 +116,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
           wl[h * NB + b][hh] = W + (size_t)wrow * K_all + k_lo + 8 * piece;
         }
     const int pairs = (K + 63) / 64;                        // lines of a row; the last may be short
-    constexpr int UP = UN / 2;
+    constexpr int UP = LINES;
     for (int first = wave; first < pairs; first += UP * NW) {
       word4 wf[UP][SETS][2];
       bf16x8 af[UP][MB][2];
@@ -125,18 +125,18 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
         const int pair = first + q * NW;
         const bool valid = pair < pairs;
         const int at = min(pair, pairs - 1) * 64;
-        const bool mine = valid && at + 8 * piece < K;        // this lane's sixteen bytes lie inside K
+        const bool mine = valid && (WHOLE || at + 8 * piece < K);        // this lane's sixteen bytes lie inside K
 #pragma unroll
         for (int s = 0; s < SETS; ++s)
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) {
             wf[q][s][hh] = (word4){0u, 0u, 0u, 0u};
-            if (mine) wf[q][s][hh] = *reinterpret_cast<const word4*>(wl[s][hh] + at);
+            if (mine) wf[q][s][hh] = __builtin_nontemporal_load(reinterpret_cast<const word4*>(wl[s][hh] + at));
           }
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {          // the rows' sixteen bytes 2 g and 2 g + 1 of the line: what the weights' are after the exchange
-          af[q][mb][0] = load8(a_row[mb] + at + 8 * g, valid && a_ok[mb] && at + 16 * g < K);
-          af[q][mb][1] = load8(a_row[mb] + at + 8 * g + 8, valid && a_ok[mb] && at + 16 * g + 8 < K);
+          af[q][mb][0] = load8(a_row[mb] + at + 8 * g, valid && a_ok[mb] && (WHOLE || at + 16 * g < K));
+          af[q][mb][1] = load8(a_row[mb] + at + 8 * g + 8, valid && a_ok[mb] && (WHOLE || at + 16 * g + 8 < K));
         }
       }
 #pragma unroll
@@ -293,19 +293,20 @@ static int column_blocks(int asked, int M, int n_out, int splits) {
 static int g_lines = 1;        // whether the long streams read their weights line by line (tests and measurements switch it)
 extern "C" void ta_skinny_lines(int on) { g_lines = on; }
 
-template <int MB, int NW, bool GATED, int NB = 1, bool LINES = false>
+template <int MB, int NW, bool GATED, int NB = 1, int LINES = 0, bool WHOLE = false>
 static int launch_skinny(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int M, int N,
                          int K, int out_dtype, hipStream_t stream, int splits = 1, void* partial = nullptr, int gate_act = 0) {
   const int n_out = GATED ? N / 2 : N;
-  const int k_chunk = splits > 1 ? ((K + splits - 1) / splits + 31) / 32 * 32 : K;
+  const int step = LINES > 0 ? 64 : 32;
+  const int k_chunk = splits > 1 ? ((K + splits - 1) / splits + step - 1) / step * step : K;
   if (splits > 1) splits = (K + k_chunk - 1) / k_chunk;          // no part without a step of its own
   const dim3 grid((n_out + 16 * NB - 1) / (16 * NB), splits);
   float* slabs = splits > 1 ? (float*)partial : nullptr;
   if (out_dtype == DT_F32)
-    skinny_gemm_kernel<MB, NW, GATED, float, false, NB, LINES><<<grid, NW * WAVE, 0, stream>>>(
+    skinny_gemm_kernel<MB, NW, GATED, float, false, NB, LINES, WHOLE><<<grid, NW * WAVE, 0, stream>>>(
         (const bf16_t*)A, lda, k_chunk, (const bf16_t*)W, (float*)C, ldc, M, N, K, slabs, (const float*)bias, RopeStore(), gate_act);
   else
-    skinny_gemm_kernel<MB, NW, GATED, bf16_t, false, NB, LINES><<<grid, NW * WAVE, 0, stream>>>(
+    skinny_gemm_kernel<MB, NW, GATED, bf16_t, false, NB, LINES, WHOLE><<<grid, NW * WAVE, 0, stream>>>(
         (const bf16_t*)A, lda, k_chunk, (const bf16_t*)W, (bf16_t*)C, ldc, M, N, K, slabs, (const float*)bias, RopeStore(), gate_act);
   int status = LAUNCH_STATUS();
   if (status == 0 && splits > 1 && C) status = launch_splitk_reduce(slabs, bias, C, M, N, ldc, splits, out_dtype, stream);
@@ -325,16 +326,36 @@ static int pick_waves(const void* A, int lda, const void* W, const void* bias, v
     if ((col_blocks == 0 || col_blocks == 4) && (N + 15) / 16 >= 4096 && K <= 8192) {
       // The one long stream of a decode step: its weights are read line by line (0.5B sizes, 8 rows: 61.7 -> 55.7 us;
       // 7B sizes: 229 -> 201 us, 16 rows 248 -> 211 us).
-      if (g_lines) return launch_skinny<1, 4, false, 4, true>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream);
+      if (g_lines && (K & 63) == 0) return launch_skinny<1, 4, false, 4, 2, true>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream);
+      if (g_lines) return launch_skinny<1, 4, false, 4, 2>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream);
       return launch_skinny<1, 4, false, 4>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream);
     }
   }
   // Few output tiles and a long K: more waves per tile, so that enough loads are in flight.
   const int tiles = ((GATED ? N / 2 : N) + 15) / 16;
   const int k_steps = (K + 31) / 32;
-  if (tiles >= 1024 || k_steps <= 8)
+  const int waves = tiles >= 1024 || k_steps <= 8 ? 4 : tiles >= 256 || k_steps <= 32 || MB * (GATED ? 2 : 1) > 2 ? 8 : 16;
+  if constexpr (MB == 1) {
+    // Whole lines where a wave's share of K is more than two of them: a shorter one is two trips at most and gains nothing (896 columns over
+    // 896 3.3 -> 3.4 us, gate/up 4,864 over 896 7.1 -> 7.4).  One line of both halves a trip when GATED (two: 43.4 | 45.9); else two with many
+    // tiles, more than eight rows or a share of at most four lines, one otherwise (the down product of 18,944 to 3,584, one row 24.1 | 27.6,
+    // sixteen 38.8 | 36.3).  Us before | so, weights from memory, one row and sixteen: gate/up 18,944 over 3,584 55.0 | 43.4 and 59.7 | 52.4, down
+    // 30.0 | 24.1 and 44.3 | 36.3, 18,944 over 3,584 27.1 | 23.5 and 41.4 | 34.4; gate/up 8,960 over 1,536 14.7 | 13.0 and 17.0 | 16.0, down
+    // 11.0 | 10.1 and 13.9 | 13.2, 8,960 over 1,536 level; down 4,864 to 896 8.7 | 7.8 and 11.7 | 11.3.
+    const int lines = K / 64;
+    if (g_lines && (K & 63) == 0 && lines > 2 * waves) {
+      const bool two = !GATED && (waves == 4 || M > 8 || lines <= 4 * waves);
+#define GO(NWV, L) return launch_skinny<1, NWV, GATED, 1, L, true>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act)
+      if (two) { if (waves == 4) GO(4, 2); if (waves == 8) GO(8, 2); GO(16, 2); }
+      if (waves == 4) GO(4, 1);
+      if (waves == 8) GO(8, 1);
+      GO(16, 1);
+#undef GO
+    }
+  }
+  if (waves == 4)
     return launch_skinny<MB, 4, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
-  if (tiles >= 256 || k_steps <= 32 || MB * (GATED ? 2 : 1) > 2)
+  if (waves == 8)
     return launch_skinny<MB, 8, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
   return launch_skinny<MB, 16, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
 }
@@ -358,7 +379,8 @@ extern "C" int ta_gemm_skinny_bf16(const void* A, int lda, const void* W, const 
 #undef GO
 }
 
-// The same product (not gated) with K cut into `splits` parts (at most; parts are multiples of 32) over the
+// The same product (not gated) with K cut into `splits` parts (at most; parts are multiples of 32, of 64 for up to sixteen rows and
+// K in whole lines, which are then read as such: 8 rows x 1,536 over 8,960 12.2 -> 11.7 us, one row 11.0 -> 10.2) over the
 // workgroups, the parts' float sums added afterwards in a fixed order.  partial: room for splits * M * N floats;
 // N % 4 == 0; M <= 64.  With C null (and more than one part after the rounding of the parts' length) the sums are
 // left in `partial` for a later kernel to add.
@@ -367,7 +389,9 @@ extern "C" int ta_gemm_skinny_bf16_splitk(const void* A, int lda, const void* W,
                                           int col_blocks, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || (K & 7) || (lda & 7) || (N & 3) || splits < 1 || (splits > 1 && !partial)) return -1;
-  if (!C && parts_of_k(K, splits, 32) < 2) return -1;
+  const bool whole = M <= 16 && (K & 63) == 0;
+  if (!C && parts_of_k(K, splits, whole ? 64 : 32) < 2) return -1;
+  if (whole) return launch_skinny<1, 8, false, 1, 1, true>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, splits, partial);
 #define GO(MBV, NBV) launch_skinny<MBV, 8, false, NBV>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, splits, partial)
   const bool two = column_blocks(col_blocks, M, N, parts_of_k(K, splits, 32)) == 2;
   switch ((M + 15) / 16) {

@@ -1599,7 +1599,7 @@ class Ops:
                 # 17 to 64 rows, a long K and few output columns (the down projection of a decode batch): the
                 # weight-streaming kernel with K cut over workgroups, so that every compute unit streams a share
                 # of the weights; the parts are added in a fixed order by a second small kernel.
-                parts = _parts_of_k(k, streaming_splits, 32)
+                parts = _parts_of_k(k, streaming_splits, 64 if m <= self.FUSED_ROWS and k % 64 == 0 else 32)
                 leave = pending and parts > 1
                 if out is None and not leave:
                     out = torch.empty((m, n), dtype=out_dtype, device=x.device)
@@ -1691,13 +1691,19 @@ class Ops:
         400 x 896 over 4,864 32.7 | 14.3.
         Of 17 to 64 rows those whose parts are left (the weight-streaming and the tiled kernel | ring, with the norm:
         17 and 64 rows x 896 over 4,864 9.3 | 7.7 and 11.7 | 8.6, x 3,584 over 18,944 39.5 | 33.4 and 47.4 | 36.0, x 1,024 over 1,024
-        6.4 | 6.8 and 7.9 | 7.5, but x 896 over 896 6.4 | 6.7 and 7.1 | 7.1), and the vocabulary's projection of any number (weight-streaming kernel up to 16 rows, tiled above | ring:
-        151,936 over 896, 1, 8, 16, 64 rows 51.7 | 52.0, 55.4 | 52.7, 60.8 | 53.0, 78 | 65; over 1,536 87.1 | 85.0, 90.4 | 87.3, 101 | 90,
-        118 | 109; 152,064 over 3,584 199 | 194, 204 | 200, 214 | 208, 257 | 227; 131,072 over 2,048 99 | 105, 104 | 107, 113 | 109, 138 | 131)."""
+        6.4 | 6.8 and 7.9 | 7.5, but x 896 over 896 6.4 | 6.7 and 7.1 | 7.1), and the vocabulary's projection of any number (tiled kernel | ring, 64 rows:
+        151,936 over 896 78 | 65, over 1,536 118 | 109, 152,064 over 3,584 257 | 227, 131,072 over 2,048 138 | 131) but for up to 16 rows against
+        whole lines of K below 4,096, which the weight-streaming kernel reads past the caches (it | ring, 1, 8, 16 rows: 151,936 over 896 43.3 |
+        50.0, 44.8 | 50.7, 51.1 | 51.3; over 1,536 71.5 | 79.7, 75.4 | 84.5, 84.4 | 87.4; 152,064 over 3,584 163 | 188, 168 | 190, 184 | 196;
+        131,072 over 2,048 82 | 97, 87 | 100, 98 | 101; 128,256 over 4,096 174 | 170, 175 | 175, 186 | 180), of small matrices up to 4
+        (1, 4, 8, 12 rows: 50,304 over 768 13.7 | 16.9, 15.0 | 17.0, 17.1 | 17.2, 19.3 | 17.4; 32,768 over 1,024 12.1 | 13.2, 12.9 | 13.2,
+        14.2 | 13.3, 15.9 | 13.4)."""
         if not (self.use_ring and k >= 64 and k % 32 == 0 and n % 4 == 0 and m * lda < 2 ** 31 and n * k < 2 ** 31):
             return False
         if m <= self.SKINNY_ROWS:
             if out_dtype == torch.float32 and n >= self.WIDE_OUTPUT:
+                if m <= self.FUSED_ROWS and k % 64 == 0 and k < 4096:
+                    return m > 4 and n * k < 2 ** 26
                 return k >= 1536 or m > 4
             return pending and m > self.FUSED_ROWS and n * k >= (2 ** 21 if m <= 32 else 2 ** 20)
         if out_dtype == torch.float32 or not self.use_library_gemm:
