@@ -376,3 +376,46 @@ def test_qkv_by_whole_lines(ops, rows, k):
     want = x.double() @ w.double().t()
     got = torch.cat([q, k_pages[0, 0, :rows], v_pages[0, 0, :, :rows].t()], dim=1)
     assert float((got.double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max())
+
+
+# The float32 products of few rows: a K of whole lines and not, that leaves a wave's last pair of units empty, whose parts are cut, weight
+# rows that end inside a tile, one to sixteen rows on both sides of the choice between matrix and vector instructions, and more workgroups
+# than compute units.
+@pytest.mark.parametrize("rows", [1, 2, 4, 5, 16])
+@pytest.mark.parametrize("n,k", [(24, 96), (20, 1056), (36, 4864), (4200, 2016), (40, 1004)])
+def test_float32_weights_by_whole_lines(ops, rows, n, k):
+    gen = torch.Generator().manual_seed(n + rows)
+    x, w = torch.randn(rows, k + 4, generator=gen).cuda()[:, :k], torch.randn(2 * n, k, generator=gen).cuda() * 0.05
+    bias = torch.randn(n, generator=gen).cuda()
+    exact = x.double() @ w.double().t()
+    first, second = exact[:, :n], exact[:, n:]
+
+    def near(got, want):                       # sums of K products of numbers around 0.05: K 2^-24 of their absolute sum at most, far less in fact
+        assert got.dtype == torch.float32 and float((got.double() - want).abs().max()) <= 1e-5 * max(1.0, float(want.abs().max()))
+
+    near(ops.linear(x, w[:n], bias), first + bias)
+    parts = ops.linear(x, w[:n], bias, pending=True)
+    near(parts if isinstance(parts, torch.Tensor) else parts.resolve(), first + bias)
+    near(ops.linear_silu_gate(x, w), first / (1 + torch.exp(-first)) * second)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 16])
+@pytest.mark.parametrize("heads,kv,d,k", [(3, 1, 32, 96), (14, 2, 64, 896), (2, 2, 96, 1000)])
+@pytest.mark.parametrize("rotate", [False, True])
+def test_float32_qkv_with_rotation_and_store(ops, rows, heads, kv, d, k, rotate):
+    gen = torch.Generator().manual_seed(d + rows)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).cuda()
+    x, w, bias = rand(rows, k), rand((heads + 2 * kv) * d, k) * 0.05, rand((heads + 2 * kv) * d)
+    positions = torch.randint(0, 40, (rows,), generator=gen, dtype=torch.int32).cuda()
+    slots = torch.randperm(48, generator=gen)[:rows].to(torch.int32).cuda()
+    slots[rows // 2] = -1                                     # this row's keys and values are not stored
+    table = rand(40, d) if rotate else None
+    pages = [(torch.full((3, kv, 16, d), 7.0, device="cuda"), torch.full((3, kv, d, 16), 7.0, device="cuda")) for _ in range(2)]
+    q = ops.fused_norm_qkv_rope(x, None, 0.0, w, bias, positions, table, slots, *pages[0], heads, kv, d)
+    qkv = (x.double() @ w.double().t() + bias).float()
+    ops.rope_store(qkv, None, positions, table, slots, *pages[1], heads, kv, d)
+    torch.testing.assert_close(q, qkv[:, :heads * d], rtol=1e-5, atol=2e-5)
+    for got, want in zip(*pages):
+        torch.testing.assert_close(got, want, rtol=1e-5, atol=2e-5)
+    silent = ops.fused_norm_qkv_rope(x, None, 0.0, w, bias, positions, table, None, *pages[0], heads, kv, d)
+    assert torch.equal(silent, q)

@@ -6,7 +6,7 @@
 //   more than 16 rows   tiles through LDS, K cut over workgroups where the tiles alone would leave compute units idle; where pieces of
 //                       sixteen bytes are aligned on the bfloat16 instructions, every operand split into three numbers of theirs
 //   up to 16 rows       one pass over the weights, sixteen weight rows a workgroup whose waves share K
-//   one or two rows (up to four of large matrices), and up to 16 whose pieces of sixteen bytes are not aligned    vector
+//   one or two rows (up to four of large wide matrices), and up to 16 whose pieces of sixteen bytes are not aligned    vector
 //                       multiply-adds, four weight rows a wave
 #include "splitk_reduce.h"
 
@@ -326,67 +326,128 @@ gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, 
 // matrix instruction's sum runs over the four g.  Four sums a lane (one for each float of a piece) keep the chains of
 // additions short; they and the eight waves' come together through LDS.  Bound by the weights' trip from memory: a wave
 // asks for its first two pairs of units at once and for the next pair before it multiplies the current one.
-// (Four rows at 0.5B sizes, the four products of a layer: 54 us with a wave on four weight rows and the gate's kernel, 41 with
-// this: gate/up with its gate 12.6, 896 columns over 4,864 8.5 in eight parts of K and 18.8 in one.)
-template <bool GATED>
+// (Half lines through the caches | whole lines past them, four rows: 896 columns over 4,864 in eight parts of K 8.7 | 7.1 us, over 896 in two
+// 5.6 | 4.4, 1,536 over 8,960 34 | 26; sixteen rows: gate/up of 17,920 over 1,536 45 | 30, of 37,888 over 3,584 182 | 128.)
+// LINES (K a multiple of 32): the weights come by whole cache lines, eight rows' a load (`lines_to_rows` in common.h), past the caches.
+// ROPE: the product is the joined q/k/v projection; a tile is eight elements of the first half of a head and the eight half a head further
+// on, which the half-split rotation pairs; bias, rotation and the store of keys and values into their pages follow in the epilogue.
+struct F32Store {
+  const int* positions; const float* cos_sin; const int* slots;
+  float* k_pages; float* v_pages;
+  int n_q, n_kv, d, page_size;
+};
+
+enum { ROWS_PLAIN = 0, ROWS_GATED = 1, ROWS_ROPE = 2 };
+
+template <int KIND, bool LINES>
 __global__ void __launch_bounds__(512)
 gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
                      float* __restrict__ C, int M, int N, int K, int lda, int ldc, int units_part,
-                     float* __restrict__ partial) {
+                     float* __restrict__ partial, const F32Store store = F32Store()) {
   constexpr int WAVES = 8, PAIR = 2;
+  constexpr bool HALVES = KIND != ROWS_PLAIN;               // eight weight rows here and eight a fixed way further on
   __shared__ float sums[WAVES][16][17];
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int row = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (GATED ? 8 : 16), half = N / 2;
-  const int n = GATED ? (row < 8 ? min(n0 + row, half - 1) : half + min(n0 + row - 8, half - 1)) : min(n0 + row, N - 1);
+  const int per_head = KIND == ROWS_ROPE ? store.d / 16 : 1;
+  const int head = KIND == ROWS_ROPE ? blockIdx.x / per_head : 0, first_in = KIND == ROWS_ROPE ? blockIdx.x % per_head * 8 : 0;
+  const int half = KIND == ROWS_ROPE ? store.d / 2 : N / 2;
+  const int n0 = KIND == ROWS_ROPE ? head * store.d + first_in : blockIdx.x * (HALVES ? 8 : 16);
+  const int limit = KIND == ROWS_GATED ? half : N;
+  // The weight row behind row i (0 .. 15) of the tile.
+  auto weight_row = [&](int i) {
+    return HALVES ? min(n0 + (i & 7), limit - 1) + (i < 8 ? 0 : half) : min(n0 + i, N - 1);
+  };
   const int units = (K + 31) / 32;
   const int u_begin = blockIdx.y * units_part, u_end = min(units, u_begin + units_part);
-  const float* w_row = W + (size_t)n * K;
   const float* a_row = A + (size_t)min(row, M - 1) * lda;
+  const float* w_row[2];
+  w_row[0] = W + (size_t)weight_row(LINES ? row & 7 : row) * K;
+  w_row[1] = LINES ? W + (size_t)weight_row(8 + (row & 7)) * K : w_row[0];
+  const int piece = 2 * g + (row >> 3);
   f32x4 w[2][PAIR][2], a[2][PAIR][2];
   auto ask = [&](int slot, int u0) {
 #pragma unroll
-    for (int p = 0; p < PAIR; ++p)
+    for (int p = 0; p < PAIR; ++p) {
+      const int u = u0 + p * WAVES;
+      if constexpr (LINES) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        // (K is a multiple of four: a piece is inside a row or past its end, where the row's first piece is read and
-        // multiplied by zeros.)
-        const int u = u0 + p * WAVES, k = u * 32 + 16 * h + 4 * g;
-        const bool in = u < u_end && k < K;
-        w[slot][p][h] = *reinterpret_cast<const f32x4*>(w_row + (in ? k : 0));
-        a[slot][p][h] = *reinterpret_cast<const f32x4*>(a_row + (in ? k : 0));
+        for (int h = 0; h < 2; ++h) w[slot][p][h] = a[slot][p][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (u < u_end) {                                     // (the same for the whole wave)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            w[slot][p][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w_row[h] + u * 32 + 4 * piece));
+#pragma unroll
+          for (int h = 0; h < 2; ++h) a[slot][p][h] = *reinterpret_cast<const f32x4*>(a_row + u * 32 + 8 * g + 4 * h);
+        }
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          // (K is a multiple of four: a piece is inside a row or past its end, where the row's first piece is read and
+          // multiplied by zeros.)
+          const int k = u * 32 + 16 * h + 4 * g;
+          const bool in = u < u_end && k < K;
+          w[slot][p][h] = *reinterpret_cast<const f32x4*>(w_row[0] + (in ? k : 0));
+          a[slot][p][h] = *reinterpret_cast<const f32x4*>(a_row + (in ? k : 0));
+        }
       }
+    }
   };
   f32x4 acc[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int first = u_begin + wave;
   ask(0, first);
+  // What the rotation needs hangs on the row's position: asked for behind the first weights.
+  const int m = threadIdx.x >> 4, at = threadIdx.x & 15;
+  float cosine = 1.f, sine = 0.f, bias1 = 0.f, bias2 = 0.f;
+  int slot_of = -1;
+  if (KIND == ROWS_ROPE && m < M && at < 8) {
+    if (head < store.n_q + store.n_kv && store.cos_sin) {
+      const float* cs = store.cos_sin + (size_t)store.positions[m] * store.d + first_in + at;
+      cosine = cs[0];
+      sine = cs[half];
+    }
+    if (bias) { bias1 = bias[n0 + at]; bias2 = bias[n0 + half + at]; }
+    if (store.slots) slot_of = store.slots[m];
+  }
   for (int u0 = first; u0 < u_end; u0 += 2 * PAIR * WAVES) {
 #pragma unroll
     for (int slot = 0; slot < 2; ++slot) {
       const int now = u0 + slot * PAIR * WAVES;
       ask(slot ^ 1, now + PAIR * WAVES);
 #pragma unroll
-      for (int p = 0; p < PAIR; ++p)
+      for (int p = 0; p < PAIR; ++p) {
+        if constexpr (LINES) {
+          // (Units past the end are zeros in both operands.)
+          line_bf16x8 b[2];
+          lines_to_rows(__builtin_bit_cast(word4, w[slot][p][0]), __builtin_bit_cast(word4, w[slot][p][1]), row < 8, b[0], b[1]);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int u = now + p * WAVES;
-          const bool in = u < u_end && u * 32 + 16 * h + 4 * g < K;
+          for (int h = 0; h < 2; ++h) {
+            const f32x4 wv = __builtin_bit_cast(f32x4, b[h]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            // (Both operands: the first piece of a row may hold an infinity, whose product with zero is no number.)
-            const float wv = in ? w[slot][p][h][e] : 0.f, av = in ? a[slot][p][h][e] : 0.f;
-            acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, av, acc[e], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[e], a[slot][p][h][e], acc[e], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int u = now + p * WAVES;
+            const bool in = u < u_end && u * 32 + 16 * h + 4 * g < K;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              // (Both operands: the first piece of a row may hold an infinity, whose product with zero is no number.)
+              const float wv = in ? w[slot][p][h][e] : 0.f, av = in ? a[slot][p][h][e] : 0.f;
+              acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, av, acc[e], 0, 0, 0);
+            }
           }
         }
+      }
     }
   }
   // A lane holds weight rows 4 g .. 4 g + 3 of A's row `row`.
 #pragma unroll
   for (int j = 0; j < 4; ++j) sums[wave][row][4 * g + j] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
   __syncthreads();
-  const int m = threadIdx.x >> 4, at = threadIdx.x & 15;
   if (m >= M) return;                                      // (threads from the sixteenth row on leave here too)
   auto total = [&](int place) {
     float t = 0.f;
@@ -394,7 +455,29 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     for (int v = 0; v < WAVES; ++v) t += sums[v][m][place];
     return t;
   };
-  if (GATED) {
+  if constexpr (KIND == ROWS_ROPE) {
+    if (at >= 8) return;
+    const float x1 = total(at) + bias1, x2 = total(at + 8) + bias2;
+    const float v1 = x1 * cosine - x2 * sine, v2 = x2 * cosine + x1 * sine;     // cosine 1 and sine 0 where nothing turns
+    const int i = first_in + at;
+    if (head < store.n_q) {
+      float* dst = C + (size_t)m * ldc + (size_t)head * store.d + i;
+      dst[0] = v1;
+      dst[half] = v2;
+      return;
+    }
+    if (slot_of < 0) return;                                // this row's keys and values are not stored
+    const int page = slot_of / store.page_size, off = slot_of % store.page_size;
+    if (head < store.n_q + store.n_kv) {
+      float* dst = store.k_pages + (((size_t)page * store.n_kv + (head - store.n_q)) * store.page_size + off) * store.d + i;
+      dst[0] = v1;
+      dst[half] = v2;
+    } else {
+      float* dst = store.v_pages + (((size_t)page * store.n_kv + (head - store.n_q - store.n_kv)) * store.d + i) * store.page_size + off;
+      dst[0] = v1;
+      dst[(size_t)half * store.page_size] = v2;
+    }
+  } else if (KIND == ROWS_GATED) {
     if (at < 8 && n0 + at < half) C[(size_t)m * ldc + n0 + at] = silu_f32(total(at)) * total(at + 8);
   } else if (n0 + at < N) {
     if (partial) partial[((size_t)blockIdx.y * M + m) * N + n0 + at] = total(at);
@@ -405,10 +488,11 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 // One or two rows, four of large matrices, and up to sixteen whose pieces of sixteen bytes do not lie on sixteen bytes (VEC false):
 // a wave takes four weight rows (GATED: two of W's first half and the two as far into its second, whose results meet in
 // silu(first) * second) and walks K sixteen bytes or an element a lane, every row of A against them.  With so little work for a
-// weight the matrix instructions gain nothing, and this way more of the weights are on their way at once: 9,728 columns over
-// 896, one row 8.7 us, 11.8 with the kernel above; 3,584 over 3,584 10.9 and 17.5; 896 over 4,864 11.6 and 19.4 (where K is cut
-// and the next norm adds the parts, the two together 13.9 and 11.9).
-template <int MR, bool VEC, bool GATED>
+// weight the matrix instructions gain nothing, and this way more of the weights are on their way at once (figures at `vector_rows`).
+// UN: pieces of 256 floats a wave asks for at once (past the caches).  Four where the workgroups are no more than the compute units, one
+// where they are more, which hide each other's trips (one row, one piece | four: 896 columns over 896 4.7 | 4.1, over 4,864 14.3 | 12.5,
+// 3,584 over 18,944 55.3 | 51.3, but 4,608 over 3,584 13.5 | 16.7, 151,936 over 896, three rows 84 | 98).
+template <int MR, bool VEC, bool GATED, int UN = 1>
 __global__ void __launch_bounds__(256)
 gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
                 float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
@@ -425,17 +509,27 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
   for (int r = 0; r < 4; ++r)
     w[r] = W + (size_t)(GATED ? (r < 2 ? 0 : half) + min(n0 + (r & 1), half - 1) : min(n0 + r, N - 1)) * K;
   if constexpr (VEC) {
-    for (int k = lane * 4; k < K; k += WAVE * 4) {
-      float4 wv[4];
+    for (int k0 = lane * 4; k0 < K; k0 += UN * WAVE * 4) {
+      f32x4 wv[UN][4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) wv[r] = *reinterpret_cast<const float4*>(w[r] + k);
+      for (int u = 0; u < UN; ++u)
 #pragma unroll
-      for (int m = 0; m < MR; ++m) {
-        if (m >= M) break;
-        const float4 a = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
+        for (int r = 0; r < 4; ++r) {
+          wv[u][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (k0 + u * WAVE * 4 < K) wv[u][r] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w[r] + k0 + u * WAVE * 4));
+        }
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          acc[r][m] = fmaf(a.x, wv[r].x, fmaf(a.y, wv[r].y, fmaf(a.z, wv[r].z, fmaf(a.w, wv[r].w, acc[r][m]))));
+      for (int u = 0; u < UN; ++u) {
+        const int k = k0 + u * WAVE * 4;
+        if (k >= K) break;
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+          if (m >= M) break;
+          const float4 a = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[r][m] = fmaf(a.x, wv[u][r][0], fmaf(a.y, wv[u][r][1], fmaf(a.z, wv[u][r][2], fmaf(a.w, wv[u][r][3], acc[r][m]))));
+        }
       }
     }
   } else {
@@ -475,13 +569,22 @@ static bool sixteen_bytes(const void* A, const void* W, int M, int K, int lda) {
   return K > 0 && K % 4 == 0 && (M <= 1 || lda % 4 == 0) && (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
 }
 
-// Whether up to sixteen aligned rows go to the vector kernel.  (us, matrix instructions | vector: two rows of 1,536 columns over
-// 8,960 34.0 | 21.7, of 2,048 over 1,024 6.6 | 6.6; four of 17,920 over 1,536 33.7 | 24.4, of 896 over 4,864 20.0 | 18.5, of 2,048
-// over 1,536 9.5 | 10.0, of 896 over 896 6.1 | 7.9; eight of 3,584 over 18,944 96.9 | 92.0, of 1,536 over 8,960 36.6 | 38.9.  With
-// K cut for the next norm, both kernels: two rows of 896 over 4,864 12.2 | 15.9, one of 3,584 over 18,944 80.9 | 67.9.)
+// Whether up to sixteen aligned rows go to the vector kernel.  K of whole lines, us, matrix instructions | vector: one row of 896 columns
+// over 896 5.1 | 4.1, over 4,864 14.5 | 12.5, 9,728 over 896 11.1 | 8.2, 3,584 over 18,944 50.2 | 51.3; two of 896 over 896 5.1 | 4.9, of
+// 1,536 over 8,960 24.8 | 24.6, of 3,584 over 18,944 51.1 | 55.4, of 9,728 over 896 11.0 | 8.7; four of 9,728 over 896 11.3 | 10.8, of 17,920
+// over 1,536 25.0 | 21.8, of 4,608 over 3,584 22 | 18, of 3,584 over 3,584 13.3 | 16.5; eight of 3,584 over 18,944 57 | 88.  With K cut for the
+// next norm, one row of 896 over 896 4.3 | 4.1, two 4.3 | 4.9, two of 3,584 over 18,944 51.9 | 55.5.
+// Other K: two rows of 1,536 columns over 8,960 34.0 | 21.7, four of 17,920 over 1,536 33.7 | 24.4, eight of 3,584 over 18,944
+// 96.9 | 92.0, of 1,536 over 8,960 36.6 | 38.9.
 static bool vector_rows(int M, int N, int K, bool pending) {
   if (pending && N % 4 == 0 && K >= 4096 && N <= 2048) return false;
-  return M <= 2 || (M <= 4 && (K >= 4096 || (long)N * K >= (8l << 20))) || (M <= 8 && K >= 16384 && !pending);
+  const bool large = (long)N * K >= (8l << 20), many = (N + 15) / 16 > compute_units();
+  if (K % 32 == 0) {
+    if (M == 1) return true;
+    if (pending && N % 4 == 0 && !many) return false;
+    return M == 2 ? !large || many : M <= 4 && large && many;
+  }
+  return M <= 2 || (M <= 4 && (K >= 4096 || large)) || (M <= 8 && K >= 16384 && !pending);
 }
 
 // The split kernel's microseconds for tiles of 64 and 128: start, a workgroup's fixed ones, and those of a step of 32 with one, two and three
@@ -554,8 +657,11 @@ extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void*
   float *c = (float*)C, *slabs = (float*)partial;
   const int k_part = parts > 1 ? ((K + parts - 1) / parts + 31) / 32 * 32 : K;
   if (tile == 16) {
-    gemm_f32_rows_kernel<false><<<dim3((N + 15) / 16, parts), 512, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc,
-                                                                               (k_part + 31) / 32, slabs);
+    const dim3 grid((N + 15) / 16, parts);
+    if (K % 32 == 0)
+      gemm_f32_rows_kernel<ROWS_PLAIN, true><<<grid, 512, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, (k_part + 31) / 32, slabs);
+    else
+      gemm_f32_rows_kernel<ROWS_PLAIN, false><<<grid, 512, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, (k_part + 31) / 32, slabs);
   } else if (tile) {
     const int m_tiles = (M + tile - 1) / tile, n_tiles = (N + tile - 1) / tile;
     dim3 grid((m_tiles * n_tiles + 7) / 8 * 8, parts);
@@ -572,8 +678,9 @@ extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void*
                                                              n_tiles, slabs);
   } else {
     const int blocks = (N + 15) / 16;
-#define GO(MR, VEC) gemv_f32_kernel<MR, VEC, false><<<blocks, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc)
-    if (aligned) { if (M <= 1) GO(1, true); else if (M <= 2) GO(2, true); else if (M <= 4) GO(4, true); else GO(8, true); }
+#define GO(MR, VEC, ...) gemv_f32_kernel<MR, VEC, false, ##__VA_ARGS__><<<blocks, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc)
+    if (aligned && blocks <= compute_units()) { if (M <= 1) GO(1, true, 4); else if (M <= 2) GO(2, true, 4); else if (M <= 4) GO(4, true, 4); else GO(8, true, 2); }
+    else if (aligned) { if (M <= 1) GO(1, true); else if (M <= 2) GO(2, true); else if (M <= 4) GO(4, true); else GO(8, true); }
     else if (M <= 1) GO(1, false); else if (M <= 2) GO(2, false); else if (M <= 4) GO(4, false);
     else if (M <= 8) GO(8, false); else GO(16, false);
 #undef GO
@@ -592,10 +699,33 @@ extern "C" int ta_gemm_f32_silu_gate(const void* A, const void* W, void* out, in
   if (M > 16 || !sixteen_bytes(A, W, M, K, lda)) return -2;
   const float *a = (const float*)A, *w = (const float*)W;
   const int blocks = (N / 2 + 7) / 8;
-#define GO(MR) gemv_f32_kernel<MR, true, true><<<blocks, 256, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc)
-  if (!vector_rows(M, N, K, false))
-    gemm_f32_rows_kernel<true><<<blocks, 512, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc, (K + 31) / 32, nullptr);
-  else if (M <= 1) GO(1); else if (M <= 2) GO(2); else if (M <= 4) GO(4); else GO(8);
+#define GO(MR) do { if (blocks <= compute_units()) gemv_f32_kernel<MR, true, true, 4><<<blocks, 256, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc); \
+                    else gemv_f32_kernel<MR, true, true><<<blocks, 256, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc); } while (0)
+  if (!vector_rows(M, N, K, false)) {
+    if (K % 32 == 0)
+      gemm_f32_rows_kernel<ROWS_GATED, true><<<blocks, 512, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc, (K + 31) / 32, nullptr);
+    else
+      gemm_f32_rows_kernel<ROWS_GATED, false><<<blocks, 512, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc, (K + 31) / 32, nullptr);
+  } else if (M <= 1) GO(1); else if (M <= 2) GO(2); else if (M <= 4) GO(4); else GO(8);
+#undef GO
+  return LAUNCH_STATUS();
+}
+
+// The joined q/k/v projection of up to sixteen rows with bias, rotation and the cache write in its epilogue (see F32Store): x [M, K] (row
+// stride lda), W [(n_q + 2 n_kv) d, K], d a multiple of 16, bias or null; queries go to q_out [M, n_q d]; cos_sin [positions, d] or null (no
+// rotation); slots int32 [M] or null (nothing is stored; a negative slot skips its row).  -2: rows without pieces of sixteen bytes.
+extern "C" int ta_gemm_f32_qkv_rope(const void* x, int lda, const void* W, const void* bias, void* q_out, const void* positions,
+                                    const void* cos_sin, const void* slots, void* k_pages, void* v_pages, int M, int K, int n_q,
+                                    int n_kv, int d, int page_size, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (M > 16 || d <= 0 || d % 16 || n_q <= 0 || n_kv <= 0 || page_size <= 0 || !positions || (slots && (!k_pages || !v_pages))) return -1;
+  if (!sixteen_bytes(x, W, M, K, lda)) return -2;
+  const F32Store store = {(const int*)positions, (const float*)cos_sin, (const int*)slots, (float*)k_pages, (float*)v_pages,
+                          n_q, n_kv, d, page_size};
+  const int heads = n_q + 2 * n_kv;
+#define GO(LINES) gemm_f32_rows_kernel<ROWS_ROPE, LINES><<<heads * (d / 16), 512, 0, stream>>>((const float*)x, (const float*)W, \
+      (const float*)bias, (float*)q_out, M, heads * d, K, lda, n_q * d, (K + 31) / 32, nullptr, store)
+  if (K % 32 == 0) GO(true); else GO(false);
 #undef GO
   return LAUNCH_STATUS();
 }

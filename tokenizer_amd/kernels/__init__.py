@@ -151,7 +151,7 @@ class Ops:
         for name in ("ta_embedding", "ta_add_rmsnorm", "ta_silu_gate", "ta_rope_store",
                      "ta_paged_attention_generic", "ta_decode_attention_bf16", "ta_prefill_attention_bf16",
                      "ta_prefill_attention_shared_plan", "ta_prefill_attention_key_splits",
-                     "ta_gemm_f32", "ta_gemm_f32_parts", "ta_gemm_f32_silu_gate", "ta_paged_attention_f32", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
+                     "ta_gemm_f32", "ta_gemm_f32_parts", "ta_gemm_f32_qkv_rope", "ta_gemm_f32_silu_gate", "ta_paged_attention_f32", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
                      "ta_gemm_skinny_bf16_splitk", "ta_gemm_skinny_qkv_rope", "ta_fused_norm_qkv_rope",
                      "ta_fused_norm_gated", "ta_fused_linear_residual", "ta_fused_qkv_rope", "ta_fused_gated",
                      "ta_splitk_reduce", "ta_splitk_add_rmsnorm", "ta_argmax", "ta_argmax_next_step", "ta_sample",
@@ -1887,17 +1887,22 @@ class Ops:
         """q, k, v = rmsnorm(residual) @ weight.T + bias; q and k rotated; k and v stored into their pages
         (when `slots` is given); returns q [M, n_q * d] in bfloat16 (more than 64 rows that the ring kernel does not take: q, k
         and v side by side, the query heads first).  residual float32 [M, K]; or, with
-        `norm_weight` None, `residual` holds the normalised rows in bfloat16 already."""
+        `norm_weight` None, `residual` holds the normalised rows in bfloat16 already, or up to sixteen of them in float32
+        against a float32 matrix (pages and result are float32 then)."""
         _dev(norm_weight, weight, bias, positions, cos_sin, slots, k_pages, v_pages)
         _need(residual.is_cuda and residual.dim() == 2, "the rows must live on the GPU")
         m, k = residual.shape
-        if norm_weight is None:
+        wide = norm_weight is None and residual.dtype == torch.float32 and m <= self.FUSED_ROWS
+        dtype = torch.float32 if wide else torch.bfloat16
+        if wide:
+            _need(residual.stride(1) == 1 and weight.is_contiguous(), "normalised rows and the matrix have contiguous rows")
+        elif norm_weight is None:
             _need(residual.dtype == torch.bfloat16 and residual.stride(1) == 1 and residual.stride(0) % 8 == 0
                   and residual.data_ptr() % 16 == 0, "normalised rows are bfloat16 with 16-byte aligned rows")
         else:
             _need(residual.dtype == torch.float32 and residual.is_contiguous() and norm_weight.dtype == torch.float32
                   and norm_weight.numel() == k, "the residual and the norm weight are float32")
-        _need(weight.dtype == torch.bfloat16 and tuple(weight.shape) == ((n_q + 2 * n_kv) * head_dim, k),
+        _need(weight.dtype == dtype and tuple(weight.shape) == ((n_q + 2 * n_kv) * head_dim, k),
               "the joined q/k/v matrix has the wrong shape")
         _need(k % 8 == 0 and head_dim % 32 == 0
               and (m <= self.FUSED_ROWS or norm_weight is None),
@@ -1910,13 +1915,20 @@ class Ops:
         page_size = 1
         if slots is not None:
             _need(slots.dtype == torch.int32 and slots.numel() == m, "slots must be int32 [M]")
-            _need(k_pages.dtype == torch.bfloat16 and v_pages.dtype == torch.bfloat16, "pages must be bfloat16")
+            _need(k_pages.dtype == dtype and v_pages.dtype == dtype, f"pages must be {dtype}")
             page_size = self._page_size(k_pages, v_pages, n_kv, head_dim)
-        q = torch.empty((m, n_q * head_dim), dtype=torch.bfloat16, device=residual.device)
+        q = torch.empty((m, n_q * head_dim), dtype=dtype, device=residual.device)
         tail = (_ptr(weight), _ptr(bias), _ptr(q), _ptr(positions), _ptr(cos_sin), _ptr(slots),
                 _ptr(k_pages if slots is not None else None), _ptr(v_pages if slots is not None else None),
                 m, k, n_q, n_kv, head_dim, page_size, self.fused_rows, self.fused_waves, self._stream())
-        if m > self.SKINNY_ROWS:
+        if wide:
+            status = self.lib.ta_gemm_f32_qkv_rope(_ptr(residual), residual.stride(0) if m > 1 else k, *tail[:-3], self._stream())
+            if status == -2:                  # rows without pieces of sixteen bytes
+                qkv = self.linear(residual, weight, bias)
+                self.rope_store(qkv, None, positions, cos_sin, slots, k_pages if slots is not None else None,
+                                v_pages if slots is not None else None, n_q, n_kv, head_dim)
+                return qkv
+        elif m > self.SKINNY_ROWS:
             # More than 64 rows: the ring kernel with the same epilogue.
             status = self.lib.ta_gemm_ring_qkv(_ptr(residual), residual.stride(0), *tail[:-3], -1, self._stream())
             if status == -2:                  # rows of no half steps of K, matrices past 32-bit places, a bias that is not aligned
@@ -1958,6 +1970,7 @@ class Ops:
             self._stream()), "fused_qk_temper")
         return q
 
+    ROPE_STORE_WEIGHT_F32 = 2 ** 23   # float32 matrices up to this many elements do so at up to four rows, any at five to sixteen
     ROPE_STORE_WEIGHT = 2 ** 22   # joined q/k/v matrices up to this many elements take the route below at 17-64 rows
 
     def can_rope_store(self, rows: int, dtype: torch.dtype, weight_elements: int = 0) -> bool:
@@ -1966,9 +1979,13 @@ class Ops:
         small (measured: 0.5B and 1.5B sizes); a big one is better off with the library's product and the
         rotation kernel.  More rows go to the ring kernel.  (Product and rotation | ring, us: 1,152 columns over 896, 65 rows
         9.4 | 6.7, 512 10.2 | 7.1, 2,048 18.0 | 14.8, 4,096 22.8 | 24.0; 2,048 over 1,536 10.8 | 8.1, 13.6 | 9.2, 26.6 | 20.3, 40.7 | 35.3;
-        4,608 over 3,584, 65 rows 22.4 | 18.2, 128 22.8 | 21.1, 300 28.6 | 29.4, 1,024 51.7 | 54.9, 4,096 140 | 164.)"""
-        if dtype != torch.bfloat16 or not self.use_fused_decode:
+        4,608 over 3,584, 65 rows 22.4 | 18.2, 128 22.8 | 21.1, 300 28.6 | 29.4, 1,024 51.7 | 54.9, 4,096 140 | 164.)
+        Float32: up to sixteen rows (product and rotation | one kernel, us: 1,152 columns over 896, 1, 4, 16 rows 6.1 | 5.5, 7.4 | 5.7, 8.3 | 6.4;
+        2,048 over 1,536 8.1 | 7.6, 9.6 | 7.9, 11.2 | 9.1; 4,608 over 3,584 15.8 | 21.3, 21.2 | 23.0, at 6 and 16 25.2 | 23.8 and 32.9 | 29.0)."""
+        if not self.use_fused_decode:
             return False
+        if dtype == torch.float32:
+            return 0 < rows <= self.FUSED_ROWS and (rows > 4 or weight_elements <= self.ROPE_STORE_WEIGHT_F32)
         if rows > self.SKINNY_ROWS:
             return self.use_ring and rows <= (self.RING_QKV_ROWS if weight_elements <= self.RING_WEIGHT else 2 * self.SKINNY_ROWS)
         return self.FUSED_ROWS < rows and weight_elements <= self.ROPE_STORE_WEIGHT
