@@ -582,9 +582,7 @@ class Ops:
         S <- diag(g) S; u = beta (v - S^T k); S <- S + k u^T; out = S^T q.  state float32 [slots, >= heads d dv] (an
         entry whose first position is 0 starts from zeros); out float32 [T, heads dv].
 
-        Steps with portions of many rows (more than `DELTA_PREPARE_ROWS` rows an entry on average) first make what does
-        not depend on the state for all tokens side by side (unit vectors, q . k, beta and the decays, which then stand in
-        `decay` in place of their pre-activations), so that the walk from token to token does nothing else."""
+        Steps with portions of many rows (see `DELTA_BLOCK_ROWS`) walk in blocks of eight tokens on the float matrix instructions; what does not depend on the state is made for all blocks side by side first."""
         _dev(fresh, decay, neg_rate, rows, state, cu_q, first_position, state_slots, out)
         n_tokens = fresh.shape[0]
         _need(heads > 0 and groups > 0 and heads % groups == 0 and 0 < d <= 256 and dv > 0, "heads of up to 256 key channels")
@@ -598,9 +596,12 @@ class Ops:
         n_entries = cu_q.numel() - 1
         _need(first_position.numel() == n_entries == state_slots.numel(), "one first position and slot per entry")
         prepared = None
-        if n_tokens > self.DELTA_PREPARE_ROWS * n_entries:
-            _need(decay.is_contiguous(), "the decays' rows are written in place")
-            prepared = torch.empty((n_tokens, 2 * groups * d + heads + groups), dtype=torch.float32, device=fresh.device)
+        record = heads * (25 * next(size for size in (16, 32, 64, 128, 256) if d <= size) + 128)
+        few, many = self.DELTA_BLOCK_ROWS
+        crowd = n_entries * heads * -(-dv // 16) * d >= 2 ** 17
+        if n_tokens > (few if crowd else many) * n_entries and (n_tokens // 8 + n_entries) * record <= self.DELTA_PREPARED:
+            _need(decay.is_contiguous(), "the decays have rows of their own")
+            prepared = torch.empty((n_tokens // 8 + n_entries, record), dtype=torch.float32, device=fresh.device)
         self._check(self.lib.ta_delta_scan(_ptr(fresh), fresh.shape[1], _ptr(decay), _ptr(neg_rate), _ptr(rows), rows.shape[1],
                                            beta_offset, _ptr(state), ctypes.c_long(state.shape[1]), _ptr(cu_q),
                                            _ptr(first_position), _ptr(state_slots), _ptr(out), _ptr(prepared), n_tokens,
@@ -608,7 +609,11 @@ class Ops:
                                            self._stream()), "delta_scan")
         return out
 
-    DELTA_PREPARE_ROWS = 4     # rows an entry (on average) above which the delta rule's inputs are prepared side by side
+    # Rows an entry (on average) above which the delta rule walks in blocks: where its columns of state fill the device, and where they do
+    # not.  (Token by token | in blocks, us: eight portions of five tokens, 28 heads of 128 36 | 32, eight of 256 72 | 44, 12 of 128 19 | 24,
+    # 14 of 64 16 | 22; of 12 tokens 42 | 38, 77 | 52, 22 | 28, 14 | 19; 64 of six, 14 heads of 64 35 | 31; 20 of 37 38 | 35.)
+    DELTA_BLOCK_ROWS = (4, 24)
+    DELTA_PREPARED = 2 ** 30   # the room their records may take: floats (87,000 tokens of 28 heads of 128)
 
     # ---------------------------------------------------- sigmoid router with groups, ungated experts
     def route_sigmoid(self, logits: torch.Tensor, correction: torch.Tensor, n_groups: int, keep_groups: int,
