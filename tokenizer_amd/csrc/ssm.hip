@@ -90,44 +90,53 @@ selective_scan_kernel(const T* __restrict__ x, int x_stride, const float* __rest
   // number of the stage's B and C rows.
   const int f_token = threadIdx.x / SS_CH, f_channel = c0 + threadIdx.x % SS_CH;
   constexpr int BC = (SS_STAGE * NP + 255) / 256;
-  float r_pre, r_x, r_z, r_b[BC], r_c[BC];
+  // (Every load is made, from a place inside, and its value is only looked at when it is put down: a load behind a condition, or one
+  // converted where it arrives, makes the wave wait for all that is under way, a trip to memory a stage.)
+  float r_pre;
+  T r_x, r_z, r_b[BC], r_c[BC];
   auto fetch = [&](int t0) {
-    const int t = t0 + f_token;
-    const bool there = t < hi && f_channel < channels;
-    r_pre = there ? pre[(size_t)t * channels + f_channel] : 0.f;
-    r_x = there ? ld(x + (size_t)t * x_stride + f_channel) : 0.f;
-    r_z = (there && MODE != SS_LOCAL) ? ld(z + (size_t)t * z_stride + z_off + f_channel) : 0.f;
+    const size_t t = min(t0 + f_token, hi - 1);
+    const int channel = min(f_channel, channels - 1);
+    r_pre = pre[t * channels + channel];
+    r_x = x[t * x_stride + channel];
+    if (MODE != SS_LOCAL) r_z = z[t * z_stride + z_off + channel];
 #pragma unroll
     for (int i = 0; i < BC; ++i) {
-      const int flat = threadIdx.x + i * 256, tt = flat / NP, j = flat % NP;
-      const bool ok = tt < SS_STAGE && t0 + tt < hi && j < n;
-      const T* row = low + (size_t)(ok ? t0 + tt : lo) * low_stride;
-      r_b[i] = ok ? ld(row + b_off + j) : 0.f;
-      r_c[i] = ok ? ld(row + c_off + j) : 0.f;
+      const int flat = threadIdx.x + i * 256, j = min(flat % NP, n - 1);
+      const T* row = low + (size_t)min(t0 + flat / NP % SS_STAGE, hi - 1) * low_stride;
+      r_b[i] = row[b_off + j];
+      if (MODE != SS_LOCAL) r_c[i] = row[c_off + j];
     }
   };
 
   // Where finished rows wait for the threads that write them out: sixteen tokens by sixteen channels.
   __shared__ float s_out[SS_STAGE][SS_CH];
-  auto write_out = [&](int t0) {                             // thread (token, channel) of the stage that lies in s_out
+  auto write_out = [&](int t0, float row) {                  // thread (token, channel) of a stage
     const int t = t0 + f_token;
-    if (t < hi && f_channel < channels) st(out + (size_t)t * channels + f_channel, s_out[f_token][threadIdx.x % SS_CH]);
+    if (t < hi && f_channel < channels) st(out + (size_t)t * channels + f_channel, row);
   };
 
   fetch(lo);
   for (int t0 = lo; t0 < hi; t0 += SS_STAGE) {
     __syncthreads();                                         // the stage before has been read, its rows lie in s_out
-    if (MODE != SS_LOCAL && t0 > lo) write_out(t0 - SS_STAGE);
+    const float done = MODE != SS_LOCAL && t0 > lo ? s_out[f_token][threadIdx.x % SS_CH] : 0.f;
     // (A token past the portion's end gets a step size of zero and zeros all round: it leaves the state as it is.)
-    s_dt[f_token][threadIdx.x % SS_CH] = t0 + f_token < hi ? ss_softplus(r_pre) : 0.f;
-    s_x[f_token][threadIdx.x % SS_CH] = r_x;
-    s_z[f_token][threadIdx.x % SS_CH] = r_z;
+    const bool there = t0 + f_token < hi && f_channel < channels;
+    s_dt[f_token][threadIdx.x % SS_CH] = there ? ss_softplus(r_pre) : 0.f;
+    s_x[f_token][threadIdx.x % SS_CH] = there ? ld(&r_x) : 0.f;
+    if (MODE != SS_LOCAL) s_z[f_token][threadIdx.x % SS_CH] = there ? ld(&r_z) : 0.f;
 #pragma unroll
     for (int i = 0; i < BC; ++i) {
-      const int flat = threadIdx.x + i * 256;
-      if (flat < SS_STAGE * NP) { s_b[flat / NP][flat % NP] = r_b[i]; s_c[flat / NP][flat % NP] = r_c[i]; }
+      const int flat = threadIdx.x + i * 256, tt = flat / NP, j = flat % NP;
+      const bool ok = t0 + tt < hi && j < n;
+      if (flat < SS_STAGE * NP) {
+        s_b[tt][j] = ok ? ld(&r_b[i]) : 0.f;
+        if (MODE != SS_LOCAL) s_c[tt][j] = ok ? ld(&r_c[i]) : 0.f;
+      }
     }
     __syncthreads();
+    // (The rows go out in front of the next loads: behind them, whoever waits for the loads would wait for the rows too.)
+    if (MODE != SS_LOCAL && t0 > lo) write_out(t0 - SS_STAGE, done);
     if (t0 + SS_STAGE < hi) fetch(t0 + SS_STAGE);            // under way while this stage is worked on
     float ys[SS_STAGE];
 #pragma unroll
@@ -139,7 +148,7 @@ selective_scan_kernel(const T* __restrict__ x, int x_stride, const float* __rest
       for (int r = 0; r < PER; ++r) {
         const int j = part + r * SS_LANES;
         S[r] = fmaf(__expf(step * a[r]), S[r], in * s_b[tt][j]);
-        y = fmaf(S[r], s_c[tt][j], y);
+        if (MODE != SS_LOCAL) y = fmaf(S[r], s_c[tt][j], y);
       }
       ys[tt] = y;
       if (MODE == SS_LOCAL) sum += step;
@@ -181,7 +190,7 @@ selective_scan_kernel(const T* __restrict__ x, int x_stride, const float* __rest
   }
   if (MODE != SS_LOCAL) {
     __syncthreads();
-    write_out(lo + (hi - lo - 1) / SS_STAGE * SS_STAGE);
+    write_out(lo + (hi - lo - 1) / SS_STAGE * SS_STAGE, s_out[f_token][threadIdx.x % SS_CH]);
   }
   if (!live) return;
   if (MODE == SS_LOCAL) {
