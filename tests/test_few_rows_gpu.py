@@ -419,3 +419,40 @@ def test_float32_qkv_with_rotation_and_store(ops, rows, heads, kv, d, k, rotate)
         torch.testing.assert_close(got, want, rtol=1e-5, atol=2e-5)
     silent = ops.fused_norm_qkv_rope(x, None, 0.0, w, bias, positions, table, None, *pages[0], heads, kv, d)
     assert torch.equal(silent, q)
+
+
+# The short convolution of steps of a token an entry: an entry of none, one of two (another has none), one that starts and one that goes on, rows
+# that only fill the batch up, two to four taps and (five: the kernels of long portions) more, three runs of channels past a workgroup's 256.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps", [2, 3, 4, 5])
+@pytest.mark.parametrize("biased", [False, True])
+def test_short_convolution_of_single_tokens(ops, dtype, taps, biased):
+    gen = torch.Generator().manual_seed(taps)
+    lengths, starts, widths, offsets, fill = [1, 0, 2, 1, 1], [0, 0, 7, 3, 0], (96, 200, 40), (4, 300, 104), 1
+    channels, n, keep = sum(widths), sum(lengths) + fill, taps - 1
+    rows = torch.randn(n, 512, generator=gen).to(dtype)
+    weights, bias = torch.randn(channels, taps, generator=gen), torch.randn(channels, generator=gen) if biased else None
+    state = torch.randn(8, 5 + keep * channels + 3, generator=gen)
+    slots = torch.randperm(8, generator=gen)[:len(lengths)]
+    entry = [e for e, count in enumerate(lengths) for _ in range(count)] + [-1] * fill
+    cu = [0]
+    for count in lengths:
+        cu.append(cu[-1] + count)
+    x = torch.cat([rows[:, o:o + w] for o, w in zip(offsets, widths)], dim=1).double()
+    want, behind = torch.zeros(n, channels, dtype=torch.float64), state.double().clone()
+    for e, s in enumerate(slots.tolist()):
+        kept = state[s, 5:5 + keep * channels].double().reshape(keep, channels) * (starts[e] > 0)
+        for t in range(cu[e], cu[e + 1]):
+            window = torch.cat([kept, x[t:t + 1]])
+            y = (weights.double() * window.t()).sum(1) + (bias.double() if biased else 0)
+            want[t] = y / (1 + torch.exp(-y))
+            kept = window[1:]
+        if lengths[e]:
+            behind[s, 5:5 + keep * channels] = kept.reshape(-1)
+    ints = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")
+    held, out = state.cuda(), torch.full((n, channels), 7.0, dtype=dtype, device="cuda")
+    ops.short_conv_silu(rows.cuda(), offsets, widths, weights.cuda(), held, 5, ints(cu), ints(starts), ints(slots.tolist()), ints(entry), out,
+                        **({"bias": bias.cuda()} if biased else {}))
+    rounding = 2 ** -8 if dtype == torch.bfloat16 else 1e-6   # the result's rounding; float sums of five terms
+    assert float((out.double().cpu() - want).abs().max()) <= rounding * max(1.0, float(want.abs().max()))
+    torch.testing.assert_close(held.double().cpu(), behind, rtol=0, atol=0)
