@@ -343,13 +343,25 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
 // keys: 12 heads of 128 9.1 -> 8.5 us, eight of 256 13.8 -> 11.8.)
 // A separate kernel on purpose: a last-arrival merge inside the first kernel needs device-wide fences,
 // which flush the L2 of every XCD and cost more than this launch.
-template <int LANES>
+// FIRST_TILES: the launch's workgroups are those of a prompt kernel's tiles in front (`tiled`) and of single tokens behind: one launch for
+// both kinds of a step that has both.
+struct MergeTiles { const float* part_o; const float* part_ml; int splits, blocks; };
+template <int LANES, bool FIRST_TILES = false>
 __global__ void __launch_bounds__(WAVE)
 decode_attention_merge(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                        const int* __restrict__ rows, bf16_t* __restrict__ out, int n_q, int d, int splits,
-                       const int* __restrict__ tiles, const int* __restrict__ cu_q) {
+                       const int* __restrict__ tiles, const int* __restrict__ cu_q, const MergeTiles tiled = MergeTiles()) {
   HELD(part_o, part_ml, rows, out, n_q, d, splits, tiles);   // (the words that are there when a wave starts)
-  const int item = blockIdx.x / n_q, head = blockIdx.x % n_q;
+  int block = blockIdx.x;
+  if constexpr (FIRST_TILES) {
+    if (block < tiled.blocks) {
+      part_o = tiled.part_o; part_ml = tiled.part_ml; splits = tiled.splits; rows = nullptr;
+    } else {
+      block -= tiled.blocks;
+      tiles = nullptr;
+    }
+  }
+  const int item = block / n_q, head = block % n_q;
   int t = rows ? scalar_int(rows + item) : item;
   if (t < 0) return;
   if (tiles) {
@@ -455,7 +467,7 @@ static int launch_decode(const void* q, int q_stride, void* out, const void* k_p
   else if (few) GO(NW, true, false, false); else GO(NW, false, false, false);
 #undef GO
   int status = LAUNCH_STATUS();
-  if (status == 0 && splits > 1) {
+  if (status == 0 && splits > 1 && out) {
     decode_attention_merge<D <= 64 ? 16 : D <= 128 ? 32 : 64><<<n_items * n_q, 64, 0, stream>>>(
                                                              (const float*)part_o, (const float*)part_ml, (const int*)rows, (bf16_t*)out, n_q, D, splits,
                                                              nullptr, nullptr);
@@ -477,7 +489,22 @@ extern "C" int ta_attention_merge_tiles(const void* part_o, const void* part_ml,
   return LAUNCH_STATUS();
 }
 
-// tied: the value pages hold what the key pages hold, and only the keys are read; vt_pages may then be null.
+// Both merges of a step that has prompt tiles and single tokens, whose kernels have left their parts (out null): one launch.
+extern "C" int ta_attention_merge_both(const void* tiles_o, const void* tiles_ml, const void* tiles, int n_tiles, const void* cu_q,
+                                       int tiles_splits, const void* part_o, const void* part_ml, const void* rows, int n_items,
+                                       int splits, void* out, int n_q, int d, hipStream_t stream) {
+  const long in_tiles = (long)n_tiles * 16 * n_q, blocks = in_tiles + (long)n_items * n_q;
+  if (n_tiles <= 0 || n_items <= 0 || blocks > 0x7fffffffL || d % 4 || tiles_splits < 1 || splits < 1) return -1;
+  const MergeTiles tiled = {(const float*)tiles_o, (const float*)tiles_ml, tiles_splits, (int)in_tiles};
+#define GO(LANES) decode_attention_merge<LANES, true><<<(unsigned)blocks, WAVE, 0, stream>>>((const float*)part_o, (const float*)part_ml, \
+      (const int*)rows, (bf16_t*)out, n_q, d, splits, (const int*)tiles, (const int*)cu_q, tiled)
+  if (d <= 64) GO(16); else if (d <= 128) GO(32); else GO(64);
+#undef GO
+  return LAUNCH_STATUS();
+}
+
+// tied: the value pages hold what the key pages hold, and only the keys are read; vt_pages may then be null.  out null with more than one
+// part: the parts are left where they are.
 // Returns -2 for a head size this kernel has no instance for (the caller then uses the generic kernel).
 extern "C" int ta_decode_attention_bf16(const void* q, int q_stride, void* out, const void* k_pages,
                                         const void* vt_pages, const void* rows, const void* positions,
@@ -487,7 +514,7 @@ extern "C" int ta_decode_attention_bf16(const void* q, int q_stride, void* out, 
                                         int chunk, const void* slopes, const void* sinks, int keep_first,
                                         int kept_splits, int n_v, float softcap, int tied, hipStream_t stream) {
   if (n_items <= 0) return 0;
-  if (n_kv <= 0 || n_q % n_kv || page_size % 16 || split_keys % 32 || splits < 1) return -1;
+  if (n_kv <= 0 || n_q % n_kv || page_size % 16 || split_keys % 32 || splits < 1 || (!out && splits < 2)) return -1;
   if (n_v <= 0) n_v = n_kv;
   if (n_kv % n_v || keep_first < 0 || kept_splits < 0 || kept_splits >= splits || (keep_first > 0) != (kept_splits > 0) ||
       (long)kept_splits * split_keys < keep_first || (keep_first > 0 && (window < 0 || chunk > 0)))

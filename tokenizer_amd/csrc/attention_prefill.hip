@@ -519,6 +519,7 @@ extern "C" int ta_prefill_attention_bf16(const void* q, int q_stride, void* out,
                                                         stream);
     if (status != -2) return status;
   }
+  if (!out) return -1;                                       // (only the kernel above leaves parts)
 #define CASE(DD, HG) case DD: return launch_prefill<DD, HG>(q, q_stride, out, k_pages, vt_pages, tiles, n_tiles, cu_q, \
     first_position, block_table, table_stride, n_q, n_kv, page_size, window, scale, max_keys, waves, extra, stream);
   switch (d) {

@@ -503,7 +503,7 @@ static int launch_shared(const void* q, int q_stride, void* out, const void* k_p
       window, scale * 1.4426950408889634f, key_splits, (float*)part_o, (float*)part_ml,
       (const float*)sinks);
   int status = LAUNCH_STATUS();
-  if (status == 0 && key_splits > 1)
+  if (status == 0 && key_splits > 1 && out)                  // (without, the parts are left where they are)
     status = ta_attention_merge_tiles(part_o, part_ml, tiles, n_tiles, cu_q, out, n_q, D, key_splits, stream);
   return status;
 }
@@ -590,6 +590,7 @@ extern "C" int ta_prefill_attention_shared_bf16(const void* q, int q_stride, voi
   if (n_tiles <= 0) return 0;
   const int heads_per_wave = shape % 10, key_groups = shape / 10 + 1;
   if (n_kv <= 0 || n_q % n_kv || page_size % 16 || heads_per_wave < 1 || heads_per_wave > 2 || key_groups > 2) return -1;
+  if (!out && key_splits < 2) return -1;
   if (key_splits < 1 || key_splits > 64 || (key_splits > 1 && (!part_o || !part_ml))) return -1;
 #define GO(DD, HG, KG) { if (tied) return launch_shared<DD, HG, KG, true>(q, q_stride, out, k_pages, vt_pages, tiles, n_tiles, cu_q, \
     first_position, block_table, table_stride, n_q, n_kv, page_size, window, scale, key_splits, part_o, part_ml, sinks, stream); \

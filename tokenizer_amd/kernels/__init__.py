@@ -158,7 +158,7 @@ class Ops:
                      "ta_sample_workspace_words", "ta_library_gemm_bf16", "ta_compute_units", "ta_read_stream",
                      "ta_embedding_streams", "ta_streams_step", "ta_token_shift", "ta_mlstm_scan", "ta_mlstm_chunked", "ta_head_norm_gate",
                      "ta_capped_gate", "ta_norm_add_rmsnorm", "ta_norm_rotate_store", "ta_differential_heads",
-                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_gated_pays", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
+                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_gated_pays", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_attention_merge_both", "ta_attention_merge_tiles", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
@@ -1319,14 +1319,26 @@ class Ops:
             if parts > 1:
                 part_o = torch.empty((n_tiles * 16, n_q, parts, head_dim), dtype=torch.float32, device=qkv.device)
                 part_ml = torch.empty((n_tiles * 16, n_q, parts, 2), dtype=torch.float32, device=qkv.device)
+            # Single tokens beside such tiles, their keys in parts too: both kernels leave their parts for one merge.
+            single = batch.decode_rows.numel()
+            held = {} if parts > 1 and single and not tied else None
             self._check(self.lib.ta_prefill_attention_bf16(
-                _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(k_pages), _ptr(v_pages), _ptr(batch.q_tiles),
+                _ptr(qkv), qkv.shape[1], _ptr(out if held is None else None), _ptr(k_pages), _ptr(v_pages), _ptr(batch.q_tiles),
                 n_tiles, _ptr(batch.cu_q), _ptr(batch.first_position), _ptr(block_table),
                 block_table.shape[1], n_q, n_kv, head_dim, page_size, choice[0], ctypes.c_float(scale), *choice[1:],
                 _ptr(part_o), _ptr(part_ml), 0 if chunk is None else int(chunk), _ptr(slopes), _ptr(sinks),
                 keep_first, value_heads, ctypes.c_float(softcap or 0.0), int(tied), self._stream()), "prefill_attention")
-            if batch.decode_rows.numel():
-                self._decode_attention(*args, rows=batch.decode_rows, **extras)
+            if single:
+                self._decode_attention(*args, rows=batch.decode_rows, held=held, **extras)
+            if held is not None:
+                if held:
+                    self._check(self.lib.ta_attention_merge_both(
+                        _ptr(part_o), _ptr(part_ml), _ptr(batch.q_tiles), n_tiles, _ptr(batch.cu_q), parts, *held["parts"],
+                        _ptr(batch.decode_rows), single, held["splits"], _ptr(out), n_q, head_dim, self._stream()), "paged_attention")
+                else:                          # (the single tokens' keys came in one part after all)
+                    self._check(self.lib.ta_attention_merge_tiles(
+                        _ptr(part_o), _ptr(part_ml), _ptr(batch.q_tiles), n_tiles, _ptr(batch.cu_q), _ptr(out), n_q, head_dim, parts,
+                        self._stream()), "paged_attention")
             return out
         if qkv.dtype == torch.float32 and self.use_fast_attention and self._attention_f32(
                 qkv, out, k_pages, v_pages, positions, entry_of_token, block_table, n_q, n_kv, head_dim, value_dim, page_size,
@@ -1399,9 +1411,9 @@ class Ops:
     def _decode_attention(self, qkv, out, k_pages, v_pages, positions, entry_of_token, block_table,
                           n_q, n_kv, head_dim, page_size, window, scale, max_position, rows=None,
                           identity_entries=False, chunk=None, slopes=None, sinks=None, keep_first=0, value_heads=None,
-                          softcap=None, tied_values=False):
+                          softcap=None, tied_values=False, held=None):
         """Matrix-core attention of single tokens with the key range split over workgroups (kept first keys behind a
-        window are further splits of their own)."""
+        window are further splits of their own).  `held` (a dict): where there are parts they are left, and said there."""
         n_items = qkv.shape[0] if rows is None else rows.numel()
         max_keys = (block_table.shape[1] * page_size) if max_position is None else max_position + 1
         # The split is planned for the context rounded up to a multiple of 512 keys: a step that replays a
@@ -1448,8 +1460,10 @@ class Ops:
         if splits > 1:
             part_o = torch.empty((n_items, n_q, splits, head_dim), dtype=torch.float32, device=qkv.device)
             part_ml = torch.empty((n_items, n_q, splits, 2), dtype=torch.float32, device=qkv.device)
+        if held is not None and splits > 1:
+            held.update(parts=(_ptr(part_o), _ptr(part_ml)), splits=splits, tensors=(part_o, part_ml))
         self._check(self.lib.ta_decode_attention_bf16(
-            _ptr(qkv), qkv.shape[1], _ptr(out), _ptr(k_pages), _ptr(v_pages), _ptr(rows), _ptr(positions),
+            _ptr(qkv), qkv.shape[1], _ptr(None if held else out), _ptr(k_pages), _ptr(v_pages), _ptr(rows), _ptr(positions),
             _ptr(None if identity_entries and rows is None else entry_of_token), _ptr(block_table),
             block_table.shape[1], _ptr(part_o), _ptr(part_ml), n_items,
             n_q, n_kv, head_dim, page_size, -1 if window is None else int(window), ctypes.c_float(scale),
