@@ -456,3 +456,20 @@ def test_short_convolution_of_single_tokens(ops, dtype, taps, biased):
     rounding = 2 ** -8 if dtype == torch.bfloat16 else 1e-6   # the result's rounding; float sums of five terms
     assert float((out.double().cpu() - want).abs().max()) <= rounding * max(1.0, float(want.abs().max()))
     torch.testing.assert_close(held.double().cpu(), behind, rtol=0, atol=0)
+
+
+# Products head by head with a gate a head and a gate a result: rows on either side of eight and of sixteen (the kernels of more rows, and the gate's
+# own), heads whose results end inside a workgroup's four, a K of several trips and of less than one.
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17])
+@pytest.mark.parametrize("heads,n,k", [(3, 10, 40), (14, 64, 136), (2, 33, 1032)])
+@pytest.mark.parametrize("each", [False, True])
+def test_head_products_with_gates(ops, rows, heads, n, k, each):
+    x, w = rand_bf16((rows, heads * k), 3), (rand_bf16((heads, n, k), 4).float() * 0.1).to(torch.bfloat16)
+    units = n if each else 1
+    gates = rand_bf16((rows, 5 + heads * units + 2), 5)
+    out = torch.full((rows, heads * n), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.head_linear(x, 0, k, w, out, 0, n, gate=(gates, 5, units))
+    product = torch.stack([x[:, h * k:(h + 1) * k].double() @ w[h].double().t() for h in range(heads)], dim=1)
+    factor = 1 / (1 + torch.exp(-gates[:, 5:5 + heads * units].double().reshape(rows, heads, units)))
+    want = (product * factor).reshape(rows, heads * n)
+    assert float((out.double() - want).abs().max()) <= 2 ** -7 * max(1.0, float(want.abs().max()))     # two roundings to bfloat16

@@ -158,7 +158,7 @@ class Ops:
                      "ta_sample_workspace_words", "ta_library_gemm_bf16", "ta_compute_units", "ta_read_stream",
                      "ta_embedding_streams", "ta_streams_step", "ta_token_shift", "ta_mlstm_scan", "ta_mlstm_chunked", "ta_head_norm_gate",
                      "ta_capped_gate", "ta_norm_add_rmsnorm", "ta_norm_rotate_store", "ta_differential_heads",
-                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_gated_pays", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_attention_merge_both", "ta_attention_merge_tiles", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
+                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_gated_pays", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_attention_merge_both", "ta_head_linear_gated", "ta_attention_merge_tiles", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
@@ -344,10 +344,14 @@ class Ops:
                                              _ptr(v_pages if slots is not None else None), page_size, _ptr(latent_q),
                                              n_tokens, int(neighbours), _code(rows.dtype), self._stream()), "latent_store")
 
+    gates_head_linear = True      # `head_linear(gate=...)` exists here
+
     def head_linear(self, x: torch.Tensor, x_offset: int, x_head_stride: int, weight: torch.Tensor, out: torch.Tensor,
-                    out_offset: int, out_head_stride: int) -> torch.Tensor:
+                    out_offset: int, out_head_stride: int, gate: tuple | None = None) -> torch.Tensor:
         """Products head by head: out[t, h out_head_stride + out_offset + n] = sum_k x[t, h x_head_stride + x_offset + k]
-        weight[h, n, k]; weight [heads, N, K]; float32 sums.  Other columns of `out` are left as they are."""
+        weight[h, n, k]; weight [heads, N, K]; float32 sums.  Other columns of `out` are left as they are.  `gate` (rows,
+        offset, units): `sigmoid_head_gate` of these rows on the whole of `out` afterwards, a gate a head (units 1) or for every
+        one of its N results (units N); out is [T, heads N] then, up to sixteen rows of it in the product's own kernel."""
         _dev(x, weight, out)
         _need(weight.dim() == 3 and x.dim() == 2 and out.dim() == 2 and x.dtype == weight.dtype == out.dtype,
               "x [T, .], weight [heads, N, K], out [T, .] of one dtype")
@@ -356,6 +360,22 @@ class Ops:
         _need(out.shape[0] == m and x_offset >= 0 and out_offset >= 0 and heads > 0
               and (heads - 1) * x_head_stride + x_offset + k <= x.shape[1]
               and (heads - 1) * out_head_stride + out_offset + n <= out.shape[1], "the heads do not fit the rows")
+        if gate is not None:
+            rows, offset, units = gate
+            _dev(rows)
+            _need(out_offset == 0 and out_head_stride == n and tuple(out.shape) == (m, heads * n) and units in (1, n),
+                  "gates belong to rows of whole heads")
+            _need(rows.dtype == out.dtype and rows.dim() == 2 and rows.shape[0] == m and rows.stride(1) == 1
+                  and 0 <= offset and offset + heads * units <= rows.shape[1], "the gates do not fit the rows")
+            if out.is_contiguous():
+                status = self.lib.ta_head_linear_gated(
+                    _ptr(x), x.shape[1], x_head_stride, x_offset, _ptr(weight), _ptr(out), out.shape[1], out_head_stride, out_offset,
+                    _ptr(rows[:, offset:]), rows.stride(0), units, int(units > 1), m, n, k, heads, _code(x.dtype), self._stream())
+                if status != -2:
+                    self._check(status, "head_linear")
+                    return out
+            self.head_linear(x, x_offset, x_head_stride, weight, out, out_offset, out_head_stride)
+            return self.sigmoid_head_gate(out, rows, offset, heads * units, n // units)
         self._check(self.lib.ta_head_linear(_ptr(x), x.shape[1], x_head_stride, x_offset, _ptr(weight), _ptr(out), out.shape[1],
                                             out_head_stride, out_offset, m, n, k, heads, _code(x.dtype), self._stream()),
                     "head_linear")

@@ -125,6 +125,10 @@ class LatentAttention(Mixer):
                             ctx.block_tables[cache.group], H, 1, D, self.window, self.scale, max_position=ctx.max_position,
                             batch=ctx, **self.more)
         out = torch.empty((n_tokens, H * self.dv), dtype=x.dtype, device=x.device)
+        units = 1 if self.spec.head_gate else self.dv if self.gated else 0
+        if units and getattr(ops, "gates_head_linear", False):
+            ops.head_linear(mixed, 0, D, self.w_uv, out, 0, self.dv, gate=(rows, self.offsets["g"], units))
+            return ops.linear(out, self.w_o)
         ops.head_linear(mixed, 0, D, self.w_uv, out, 0, self.dv)
         if self.spec.head_gate:
             ops.sigmoid_head_gate(out, rows, self.offsets["g"], H, self.dv)
