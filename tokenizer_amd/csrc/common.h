@@ -73,16 +73,31 @@ __device__ __forceinline__ int scalar_int(const int* p) {
   return *(constant_int)(p);
 }
 
+// The sum and the largest over a wave, in every lane: four rotations within the rows of sixteen lanes, which stay in registers, and two exchanges
+// between rows through the LDS crossbar.  (Six of those, one waiting for the other, were a third of a microsecond; a norm has two such sums
+// and more.  A lane that is not there counts for nothing.)
+#define WAVE_ROTATED(gone, v, n) \
+  __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(gone), __float_as_int(v), 0x120 | (n), 0xF, 0xF, false))
+__device__ __forceinline__ float lanes_sum16(float v) {
+  v += WAVE_ROTATED(0.f, v, 8);
+  v += WAVE_ROTATED(0.f, v, 4);
+  v += WAVE_ROTATED(0.f, v, 2);
+  return v + WAVE_ROTATED(0.f, v, 1);
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-  return v;
+  v = lanes_sum16(v);
+  v += __shfl_xor(v, 16, WAVE);
+  return v + __shfl_xor(v, 32, WAVE);
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, WAVE));
-  return v;
+  v = fmaxf(v, WAVE_ROTATED(v, v, 8));
+  v = fmaxf(v, WAVE_ROTATED(v, v, 4));
+  v = fmaxf(v, WAVE_ROTATED(v, v, 2));
+  v = fmaxf(v, WAVE_ROTATED(v, v, 1));
+  v = fmaxf(v, __shfl_xor(v, 16, WAVE));
+  return fmaxf(v, __shfl_xor(v, 32, WAVE));
 }
+#undef WAVE_ROTATED
 
 // Sum over a block of up to 1024 threads; every thread gets the result.  `scratch` holds 16 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
@@ -92,9 +107,7 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  float total = 0.f;
-  for (int w = 0; w < n_waves; ++w) total += scratch[w];
-  return total;
+  return lanes_sum16((lane & 15) < n_waves ? scratch[lane & 15] : 0.f);     // (every row of sixteen lanes adds up all the waves' sums)
 }
 
 // Sixteen rows of a matrix as a 16x16x32 matrix instruction wants them (lane (col, g): row col), read line by line.
