@@ -473,3 +473,27 @@ def test_head_products_with_gates(ops, rows, heads, n, k, each):
     factor = 1 / (1 + torch.exp(-gates[:, 5:5 + heads * units].double().reshape(rows, heads, units)))
     want = (product * factor).reshape(rows, heads * n)
     assert float((out.double() - want).abs().max()) <= 2 ** -7 * max(1.0, float(want.abs().max()))     # two roundings to bfloat16
+
+
+# Rows of pieces of eight, a thread a piece: a norm over the queries alone, over the keys alone and over neither, a bias, values narrower than keys, no rotation
+# and one of whole heads, tokens that store nothing, a wave of threads and just over the most (the general kernel).
+@pytest.mark.parametrize("n_q,n_k,n_v,d,dv,dims,norms,biased", [(4, 2, 1, 48, 16, 16, (True, False), True), (3, 1, 1, 32, 32, 0, (False, True), False),
+                                                                (24, 4, 2, 128, 128, 64, (True, True), False), (6, 6, 6, 64, 24, 64, (False, False), True),
+                                                                (62, 1, 1, 128, 128, 128, (True, True), True), (64, 33, 32, 64, 64, 32, (True, True), True)])
+def test_norm_rotation_and_store_by_pieces(ops, n_q, n_k, n_v, d, dv, dims, norms, biased):
+    gen = torch.Generator().manual_seed(d + n_q)
+    rand = lambda *shape: torch.rand(*shape, generator=gen) + 0.2
+    count, used = 7, (n_q + n_k) * d + n_v * dv
+    rows = torch.randn(count, used + 8, generator=gen).to(torch.bfloat16)
+    positions = torch.tensor([0, 1, 63, 64, 1000, 4095, 17], dtype=torch.int32)
+    slots = torch.tensor([3, -1, 47, 16, 0, 31, 5], dtype=torch.int32)
+    rates, wq, wk, bias = rand(dims // 2), rand(n_q * d) if norms[0] else None, rand(n_k * d) if norms[1] else None, rand(used + 8) if biased else None
+    pages = lambda device: (torch.zeros(3, n_k, 16, d, dtype=torch.bfloat16, device=device),
+                            torch.zeros(3, n_v, dv, 16, dtype=torch.bfloat16, device=device))
+    on = lambda t: None if t is None else t.cuda()
+    want, got = (rows.clone(), *pages("cpu")), (rows.cuda(), *pages("cuda"))
+    PlainOps(torch.float64).norm_rotate_store(want[0], bias, positions, rates if dims else None, dims, slots, *want[1:], n_q, n_k, n_v, d, dv, wq, wk, 1e-5)
+    ops.norm_rotate_store(got[0], on(bias), positions.cuda(), on(rates) if dims else None, dims, slots.cuda(), *got[1:], n_q, n_k, n_v, d, dv,
+                          on(wq), on(wk), 1e-5)
+    for mine, right in zip(got, want):                        # neighbours in bfloat16; angles of up to 4,095 in float32 (3e-4 of a radian)
+        torch.testing.assert_close(mine.cpu().float(), right.float(), rtol=2.0 ** -7, atol=4e-3)
