@@ -1,0 +1,84 @@
+"""In which order the products of few rows and the sums over a wave add up.  Reading the weights by whole cache lines, or a sum through
+other instructions, must leave the sums as they were: a product's bits decide a router's near ties, and with them whole rows of logits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BIG = 2.0 ** 30       # (in float32 a one that meets it before its negative does is lost)
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from tokenizer_amd.kernels import get_ops
+    return get_ops()
+
+
+def rand(shape, seed, scale=1.0):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(shape, generator=gen, device="cuda") * scale).bfloat16()
+
+
+def pattern(k, *places):
+    """Elements of K that add up to one if `places` (the big number, its negative, the one) meet in this order, else to zero."""
+    row = torch.zeros(k, dtype=torch.bfloat16, device="cuda")
+    for place, value in zip(places, (BIG, -BIG, 1.0)):
+        row[place] = value
+    return row
+
+
+# Columns and K by the launcher's sixteen, eight and four sums a tile, its lines a trip (1, 2, 3, 4 and 6), one workgroup a compute unit,
+# and columns that end inside a tile.
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n, k, gated", [(1000, 2240, False), (1000, 3584, False), (4200, 1344, False), (4200, 1984, False),
+                                         (4096, 4160, False), (16400, 704, False), (1000, 2240, True), (4200, 1344, True),
+                                         (4200, 1984, True), (4200, 2048, True), (16400, 704, True), (16400, 2048, True)])
+def test_product_by_whole_lines_has_the_bits_of_half_lines(ops, rows, n, k, gated):
+    x, w = rand((rows, k + 8), 1)[:, :k], rand((n * (2 if gated else 1), k), 2, 0.05)
+    bias = rand((n,), 3).float()
+    run = (lambda: ops.linear_silu_gate(x, w)) if gated else (lambda: ops.linear(x, w, bias, out_dtype=torch.float32))
+    got = run()
+    ops.lib.ta_skinny_lines(0)
+    try:
+        want = run()
+    finally:
+        ops.lib.ta_skinny_lines(1)
+    assert got.isfinite().all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows", [1, 16])
+@pytest.mark.parametrize("k", [896, 1536, 3584, 4864, 8960])
+def test_fused_products_add_32_elements_of_k_at_a_time(ops, rows, k):
+    x = torch.ones((rows, k), dtype=torch.bfloat16, device="cuda")
+    w = pattern(k, 0, 8, 33).repeat(80, 1)
+    residual = torch.zeros((rows, 80), device="cuda")
+    ops.linear_add(x, w, None, residual)
+    assert (residual == 1).all()
+    gated = ops.fused_norm_gated(x, None, 0.0, w)
+    want = torch.nn.functional.silu(torch.ones(1)).bfloat16().item()
+    assert ((gated.float() - want).abs() <= 2 ** -8).all()
+
+
+@pytest.mark.parametrize("rows", [1, 12])
+@pytest.mark.parametrize("hidden, inner", [(512, 64), (1536, 1088)])
+def test_experts_of_few_rows_add_32_elements_of_k_at_a_time(ops, rows, hidden, inner):
+    x = torch.ones((rows, hidden), dtype=torch.bfloat16, device="cuda")
+    first = pattern(hidden, 0, 8, 33).repeat(2 * inner, 1)                 # (two experts; relu squared of one is one)
+    second = torch.cat([pattern(inner, 0, 8, 33)] * 2).repeat(hidden, 1)
+    chosen = torch.zeros((rows, 1), dtype=torch.int32, device="cuda")
+    chosen[1::2] = 1
+    got = ops.experts_few(x, chosen, torch.ones((rows, 1), device="cuda"), 2, first, False, inner, second)
+    assert (got.partial == 1).all()
+
+
+@pytest.mark.parametrize("rows", [1, 8, 11])
+def test_sum_over_a_wave_starts_with_lanes_32_apart(ops, rows):
+    # A lane holds eight elements of K: lanes 0 and 32 meet first, lane 1's one afterwards.
+    heads, n, k = 3, 20, 512
+    x = torch.ones((rows, heads * k), dtype=torch.bfloat16, device="cuda")
+    w = pattern(k, 0, 256, 8).repeat(heads, n, 1)
+    out = torch.empty((rows, heads * n), dtype=torch.bfloat16, device="cuda")
+    ops.head_linear(x, 0, k, w, out, 0, n)
+    assert (out == 1).all()
+    gate = torch.zeros((rows, heads * n), dtype=torch.bfloat16, device="cuda")
+    ops.head_linear(x, 0, k, w, out, 0, n, gate=(gate, 0, n))
+    assert (out == 0.5).all()

@@ -73,50 +73,73 @@ __device__ __forceinline__ int scalar_int(const int* p) {
   return *(constant_int)(p);
 }
 
-// The sum and the largest over a wave, in every lane: four rotations within the rows of sixteen lanes, which stay in registers, and two exchanges
-// between rows through the LDS crossbar.  (Six of those, one waiting for the other, were a third of a microsecond; a norm has two such sums
-// and more.  A lane that is not there counts for nothing.)
-#define WAVE_ROTATED(gone, v, n) \
-  __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(gone), __float_as_int(v), 0x120 | (n), 0xF, 0xF, false))
-__device__ __forceinline__ float lanes_sum16(float v) {
-  v += WAVE_ROTATED(0.f, v, 8);
-  v += WAVE_ROTATED(0.f, v, 4);
-  v += WAVE_ROTATED(0.f, v, 2);
-  return v + WAVE_ROTATED(0.f, v, 1);
+// The sum and the largest over a wave whose 64 lanes are all active, in every lane, without LDS: lanes 32 and 16 apart change places
+// (`v_permlane32_swap`, `v_permlane16_swap`; both halves of a swap added are the same whichever came first), after which every row of
+// sixteen lanes holds the same numbers, and four rotations within a row add up what lies 8, 4, 2 and 1 apart.  That is, bit for bit, the
+// order of six exchanges between lanes 32, 16, .. 1 apart, which went through the LDS crossbar one behind the other, a third of a
+// microsecond a sum.  (Rows first and then across them is another order: a router's near tie that it tips moves a token's logits.)
+__device__ __forceinline__ void wave_across_rows(float v, float& a, float& b, bool by32) {
+  const uint32_t bits = __float_as_uint(v);
+  const auto got = by32 ? __builtin_amdgcn_permlane32_swap(bits, bits, false, false) : __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+  a = __uint_as_float(got[0]);
+  b = __uint_as_float(got[1]);
 }
+#define WAVE_ROTATED(v, n) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 | (n), 0xF, 0xF, false))
 __device__ __forceinline__ float wave_sum(float v) {
-  v = lanes_sum16(v);
-  v += __shfl_xor(v, 16, WAVE);
-  return v + __shfl_xor(v, 32, WAVE);
+  float a, b;
+  wave_across_rows(v, a, b, true);
+  wave_across_rows(a + b, a, b, false);
+  v = a + b;
+  v += WAVE_ROTATED(v, 8);
+  v += WAVE_ROTATED(v, 4);
+  v += WAVE_ROTATED(v, 2);
+  return v + WAVE_ROTATED(v, 1);
 }
 __device__ __forceinline__ float wave_max(float v) {
-  v = fmaxf(v, WAVE_ROTATED(v, v, 8));
-  v = fmaxf(v, WAVE_ROTATED(v, v, 4));
-  v = fmaxf(v, WAVE_ROTATED(v, v, 2));
-  v = fmaxf(v, WAVE_ROTATED(v, v, 1));
-  v = fmaxf(v, __shfl_xor(v, 16, WAVE));
-  return fmaxf(v, __shfl_xor(v, 32, WAVE));
+  float a, b;
+  wave_across_rows(v, a, b, true);
+  wave_across_rows(fmaxf(a, b), a, b, false);
+  v = fmaxf(a, b);
+  v = fmaxf(v, WAVE_ROTATED(v, 8));
+  v = fmaxf(v, WAVE_ROTATED(v, 4));
+  v = fmaxf(v, WAVE_ROTATED(v, 2));
+  return fmaxf(v, WAVE_ROTATED(v, 1));
 }
 #undef WAVE_ROTATED
 
-// Sum over a block of up to 1024 threads; every thread gets the result.  `scratch` holds 16 floats.
+// Sum over a block of up to 1024 threads, whole waves, added wave by wave in their order; every thread gets the result.  `scratch` holds 16
+// floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
   v = wave_sum(v);
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-  const int n_waves = (blockDim.x + WAVE - 1) / WAVE;
+  const int n_waves = blockDim.x / WAVE;
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  return lanes_sum16((lane & 15) < n_waves ? scratch[lane & 15] : 0.f);     // (every row of sixteen lanes adds up all the waves' sums)
+  // (All that may be needed is asked for at once: one after the other sixteen waves' sums are a trip to LDS each, 0.15 us a sum.)
+  float total = 0.f;
+  if (n_waves <= 4) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) total += w < n_waves ? scratch[w] : 0.f;
+  } else {
+    float part[16];
+#pragma unroll
+    for (int w = 0; w < 16; ++w) part[w] = scratch[w];
+#pragma unroll
+    for (int w = 0; w < 16; ++w) total += w < n_waves ? part[w] : 0.f;
+  }
+  return total;
 }
 
 // Sixteen rows of a matrix as a 16x16x32 matrix instruction wants them (lane (col, g): row col), read line by line.
 // The memory pipeline works a load off cache line by cache line, so a load that touches eight rows' whole lines of
 // 128 bytes streams far more than one that touches sixteen rows' half lines.  The rows are therefore read by two
-// loads, one for rows 0-7 (`lower`) and one for rows 8-15 (`upper`), in each of which lane (col, g) brings row
-// col % 8's sixteen bytes number 2 g + col / 8 of the line; `lines_to_rows` puts them right by one exchange between
-// lanes eight apart (a rotation within the row of sixteen lanes, no LDS): `first` = the sixteen bytes 2 g of row
-// col's line, `second` = the sixteen bytes 2 g + 1.  The other operand takes the same bytes of its rows.
+// loads, one for rows 0-7 (`lower`) and one for rows 8-15 (`upper`), in each of which lane (col, g) brings one of row
+// col % 8's eight pieces of sixteen bytes, lanes below eight and lanes above another; `lines_to_rows` puts them right by one exchange
+// between lanes eight apart (a rotation within the row of sixteen lanes, no LDS): `first` = row col's piece that the lower
+// lanes brought, `second` = the one that the upper lanes brought.  The other operand takes the same pieces of its rows.  With piece
+// g + 4 (col / 8) a line is two steps of 32 elements as half lines would be, and a sum the same to the last bit; with 2 g + col / 8
+// the two instructions take the even and the odd pieces.
 typedef uint32_t word4 __attribute__((ext_vector_type(4)));
 typedef __bf16 line_bf16x8 __attribute__((ext_vector_type(8)));
 

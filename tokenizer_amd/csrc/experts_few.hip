@@ -44,7 +44,7 @@ __device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], 
   // Turns asked for at once: four loads of weights a lane of two matrices (twice as many take registers that more waves a
   // compute unit make better use of: twelve rows of the second example above 46.0 | 44.5 us), eight of one (four: 44.6).
   constexpr int UN = HALVES == 2 ? 1 : 4;
-  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, piece = 2 * g + (col >> 3);
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, piece = g + 4 * (col >> 3);
   const int turns = (K + 63) / 64;
   const word4 zero = {0u, 0u, 0u, 0u};
   for (int first = wave; first < turns; first += UN * NW) {
@@ -59,9 +59,9 @@ __device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], 
         for (int hh = 0; hh < 2; ++hh)
           wf[q][h][hh] = w_in ? __builtin_nontemporal_load(reinterpret_cast<const word4*>(w_at[h][hh] + at + 8 * piece)) : zero;
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {                          // what the weights are after the exchange: the bytes 2 g and 2 g + 1
-        const bool x_in = turn < turns && at + 16 * g + 8 * s < K;
-        xf[q][s] = x_in && x_ok ? *reinterpret_cast<const word4*>(x_at + at + 16 * g + 8 * s) : zero;
+      for (int s = 0; s < 2; ++s) {                          // what the weights are after the exchange: the pieces g and 4 + g
+        const bool x_in = turn < turns && at + 32 * s + 8 * g < K;
+        xf[q][s] = x_in && x_ok ? *reinterpret_cast<const word4*>(x_at + at + 32 * s + 8 * g) : zero;
       }
     }
 #pragma unroll

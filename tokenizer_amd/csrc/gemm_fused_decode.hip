@@ -129,7 +129,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
   const bf16_t* w0[PASSES];
   const bf16_t* w1[PASSES];
   bool w_lane[PASSES], w_upper[PASSES];                     // LINES: the lane's row of the lower eight, of the upper eight
-  const int piece = LINES ? 2 * g + (col >> 3) : g;
+  const int piece = LINES ? g + 4 * (col >> 3) : g;
 #pragma unroll
   for (int ps = 0; ps < PASSES; ++ps) {
     const int r = 16 * ps + (LINES ? col & 7 : col);
@@ -204,11 +204,10 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
 #pragma unroll
     for (int ps = 1; ps < PASSES; ++ps) load_w(HELD - PASSES + ps, ps, wave);
   }
-  // LINES: the lane's part of the rows for steps u and u + 1 of a pair is their sixteen bytes 2 g and 2 g + 1 of the line.
-  auto a_line = [&](int base_pair, int u) { return min(base_pair + (u >> 1) * NW, pairs - 1) * 64 + 8 * (u & 1); };
+  // LINES: steps u and u + 1 of a pair, inside K or at its last line.
+  auto a_line = [&](int base_pair, int u) { return min(base_pair + (u >> 1) * NW, pairs - 1) * 64 + 32 * (u & 1); };
   auto a_inside = [&](int base_pair, int u) { return base_pair + (u >> 1) * NW < pairs; };
-  constexpr int LANE_K = LINES ? 16 : 8;
-  const bf16_t* ar = NORM ? nullptr : p.a + (size_t)a_m * p.lda + LANE_K * g;
+  const bf16_t* ar = NORM ? nullptr : p.a + (size_t)a_m * p.lda + 8 * g;
   bf16x8 af_one[ONE ? UN : 1];
   if (ONE && !NORM) {                                      // the rows' fragments as well
 #pragma unroll
@@ -307,7 +306,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
     }
     __syncthreads();
   }
-  const uint16_t* as_row = a_s + (size_t)a_m * lds_stride + LANE_K * g;
+  const uint16_t* as_row = a_s + (size_t)a_m * lds_stride + 8 * g;
   auto load_a = [&](int k) -> bf16x8 {
     if (NORM) return *reinterpret_cast<const bf16x8*>(as_row + k);
     return a_lane ? *reinterpret_cast<const bf16x8*>(ar + k) : fz8();

@@ -49,7 +49,9 @@ struct RopeStore {
 // rows outweigh a tile's weights (what comes over the fabric from the caches counts like what comes from memory).
 // LINES > 0: the weights are read line by line (`lines_to_rows` in common.h), K walked in steps of 64, LINES steps at a time, past the
 // caches (a stream that does not come again): for products that are one long stream over a big matrix.  WHOLE: K is a multiple of 64.
-template <int MB, int NW, bool GATED, typename OutT, bool ROPE = false, int NB = 1, int LINES = 0, bool WHOLE = false>
+// SUMS 2 (with WHOLE): a wave keeps the sums of two waves of half lines, a line's first 32 elements of K and its second, so that a
+// product has the same bits whichever way its weights come.
+template <int MB, int NW, bool GATED, typename OutT, bool ROPE = false, int NB = 1, int LINES = 0, bool WHOLE = false, int SUMS = 1>
 __global__ void __launch_bounds__(NW * WAVE)
 skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf16_t* __restrict__ W,
                    OutT* __restrict__ C, int ldc, int M, int N, int K_all, float* __restrict__ partial,
@@ -61,7 +63,8 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
   static_assert(!ROPE || NB == 1, "the rotation pairs rows within one block");
   constexpr int HALVES = GATED ? 2 : 1;                     // gate and up rows (or the two halves of a head)
   constexpr int SETS = HALVES * NB;                         // set h * NB + b: half h, column block b
-  __shared__ float red[NW][HALVES * MB * 4][WAVE];
+  static_assert(SUMS == 1 || (SUMS == 2 && LINES > 0 && WHOLE), "two sums a wave: whole lines, a sum for each half");
+  __shared__ float red[NW * SUMS][HALVES * MB * 4][WAVE];
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int col = lane & 15, g = lane >> 4;
   const int n_out = ROPE ? N : GATED ? N / 2 : N;
@@ -95,15 +98,19 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
     a_row[mb] = A + (size_t)min(m_base + mb * 16 + col, M - 1) * lda + k_lo + 8 * g;
   }
 
-  floatx4 acc[SETS][MB];
+  floatx4 sums[SUMS][SETS][MB];
+  floatx4 (&acc)[SETS][MB] = sums[0];
 #pragma unroll
-  for (int s = 0; s < SETS; ++s)
+  for (int i = 0; i < SUMS; ++i)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[s][mb] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < SETS; ++s)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) sums[i][s][mb] = (floatx4){0.f, 0.f, 0.f, 0.f};
 
   constexpr int UN = (SETS * MB > 4) ? 2 : 4;
   if constexpr (LINES > 0) {
-    const int sub = col & 7, piece = 2 * g + (col >> 3);
+    const int sub = col & 7, piece = SUMS == 2 ? g + 4 * (col >> 3) : 2 * g + (col >> 3);
+    const int a_first = SUMS == 2 ? 8 * g : 16 * g, a_apart = SUMS == 2 ? 32 : 8;    // the rows' elements of the line that meet the weights'
     const bool low_lane = col < 8;
     const bf16_t* wl[SETS][2];
 #pragma unroll
@@ -134,10 +141,12 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
             if (mine) wf[q][s][hh] = __builtin_nontemporal_load(reinterpret_cast<const word4*>(wl[s][hh] + at));
           }
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {          // the rows' sixteen bytes 2 g and 2 g + 1 of the line: what the weights' are after the exchange
-          af[q][mb][0] = load8(a_row[mb] + at + 8 * g, valid && a_ok[mb] && (WHOLE || at + 16 * g < K));
-          af[q][mb][1] = load8(a_row[mb] + at + 8 * g + 8, valid && a_ok[mb] && (WHOLE || at + 16 * g + 8 < K));
-        }
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh) {         // (`a_row` is 8 g on already)
+            const int place = at + a_first + hh * a_apart;
+            af[q][mb][hh] = load8(a_row[mb] + place - 8 * g, valid && a_ok[mb] && (WHOLE || place < K));
+          }
       }
 #pragma unroll
       for (int q = 0; q < UP; ++q) {
@@ -148,7 +157,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) {
             acc[s][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, af[q][mb][0], acc[s][mb], 0, 0, 0);
-            acc[s][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, af[q][mb][1], acc[s][mb], 0, 0, 0);
+            sums[SUMS - 1][s][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, af[q][mb][1], sums[SUMS - 1][s][mb], 0, 0, 0);
           }
         }
       }
@@ -200,11 +209,13 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
   const int n0 = n_first + 16 * b;
   if (b > 0) __syncthreads();                                   // the block before has been read
 #pragma unroll
-  for (int h = 0; h < HALVES; ++h)
+  for (int i = 0; i < SUMS; ++i)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int h = 0; h < HALVES; ++h)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][(h * MB + mb) * 4 + r][lane] = acc[h * NB + b][mb][r];
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave * SUMS + i][(h * MB + mb) * 4 + r][lane] = sums[i][h * NB + b][mb][r];
   __syncthreads();
   // Lane (col, g) of block mb holds C^T rows n0 + 4g + r (r = 0..3), column m = mb*16 + col.
   for (int item = threadIdx.x; item < MB * WAVE; item += NW * WAVE) {
@@ -217,7 +228,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
     for (int r = 0; r < 4; ++r) {
       float sum0 = 0.f, sum1 = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
+      for (int w = 0; w < NW * SUMS; ++w) {
         sum0 += red[w][mb * 4 + r][ln];
         if (GATED) sum1 += red[w][(MB + mb) * 4 + r][ln];
       }
@@ -290,10 +301,11 @@ static int column_blocks(int asked, int M, int n_out, int splits) {
   return (M > 32 && (long)((n_out + 31) / 32) * splits >= 128) ? 2 : 1;
 }
 
-static int g_lines = 1;        // whether the long streams read their weights line by line (tests and measurements switch it)
+// Whether products that are not cut over K read their weights line by line where that is the faster way (tests and measurements switch it).
+static int g_lines = 1;
 extern "C" void ta_skinny_lines(int on) { g_lines = on; }
 
-template <int MB, int NW, bool GATED, int NB = 1, int LINES = 0, bool WHOLE = false>
+template <int MB, int NW, bool GATED, int NB = 1, int LINES = 0, bool WHOLE = false, int SUMS = 1>
 static int launch_skinny(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int M, int N,
                          int K, int out_dtype, hipStream_t stream, int splits = 1, void* partial = nullptr, int gate_act = 0) {
   const int n_out = GATED ? N / 2 : N;
@@ -303,14 +315,30 @@ static int launch_skinny(const void* A, int lda, const void* W, const void* bias
   const dim3 grid((n_out + 16 * NB - 1) / (16 * NB), splits);
   float* slabs = splits > 1 ? (float*)partial : nullptr;
   if (out_dtype == DT_F32)
-    skinny_gemm_kernel<MB, NW, GATED, float, false, NB, LINES, WHOLE><<<grid, NW * WAVE, 0, stream>>>(
+    skinny_gemm_kernel<MB, NW, GATED, float, false, NB, LINES, WHOLE, SUMS><<<grid, NW * WAVE, 0, stream>>>(
         (const bf16_t*)A, lda, k_chunk, (const bf16_t*)W, (float*)C, ldc, M, N, K, slabs, (const float*)bias, RopeStore(), gate_act);
   else
-    skinny_gemm_kernel<MB, NW, GATED, bf16_t, false, NB, LINES, WHOLE><<<grid, NW * WAVE, 0, stream>>>(
+    skinny_gemm_kernel<MB, NW, GATED, bf16_t, false, NB, LINES, WHOLE, SUMS><<<grid, NW * WAVE, 0, stream>>>(
         (const bf16_t*)A, lda, k_chunk, (const bf16_t*)W, (bf16_t*)C, ldc, M, N, K, slabs, (const float*)bias, RopeStore(), gate_act);
   int status = LAUNCH_STATUS();
   if (status == 0 && splits > 1 && C) status = launch_splitk_reduce(slabs, bias, C, M, N, ldc, splits, out_dtype, stream);
   return status;
+}
+
+// Lines a wave with two sums asks for at once (`waves`: how many half lines would take).  The more rows, the fewer, since each brings as
+// much of its own per line; a share of K of six lines in one trip and one of seven or eight in two; a gated product's two matrices fill
+// a trip with one line, or two where rows are a multiple of 4 KB apart and a line of each is too much for the same memory channels.
+// (Us by lines a trip.  Sixteen sums: 3,584 over 18,944, one row, 1 to 4: 38.2, 29.4, 26.0, 26.2, eight 32.8, 29.5, 30.1, 32.7, sixteen 35.1, 36.2,
+// 37.7, 37.1; 3,584 over 3,584, one row 9.9, 8.1, 7.9, 7.5.  Eight: 4,608 over 3,584, one row 14.6, 11.3, 10.8, 11.2, sixteen 14.8, 15.3, 16.4, 16.1;
+// gate/up 8,960 over 1,536, eight rows, 1, 2 and 6: 15.0, 15.1, 14.2; 8,960 over 3,584, one row 26.4, 29.3, 28.6; 14,336 over 4,096
+// 47.2, 40.7, 42.3.  Four: 18,944 over 3,584, one row, 1 to 3: 26.4, 22.5, 25.1, sixteen 32.9, 36.0, 35.3; gate/up 42.5, 46.7, 44.6.)
+static int lines_a_trip(bool gated, int waves, int M, int K) {
+  const int share = (K / 64 + waves / 2 - 1) / (waves / 2);
+  if (waves == 8 && share <= 6 && (gated || M <= 8)) return 6;
+  if (M > 8) return 1;
+  if (gated) return waves == 16 || K % 2048 == 0 ? 2 : 1;
+  if (waves == 4 || M > 4) return 2;
+  return waves == 16 && (share == 7 || share == 8) ? 4 : 3;
 }
 
 template <int MB, bool GATED>
@@ -337,19 +365,26 @@ static int pick_waves(const void* A, int lda, const void* W, const void* bias, v
   const int waves = tiles >= 1024 || k_steps <= 8 ? 4 : tiles >= 256 || k_steps <= 32 || MB * (GATED ? 2 : 1) > 2 ? 8 : 16;
   if constexpr (MB == 1) {
     // Whole lines where a wave's share of K is more than two of them: a shorter one is two trips at most and gains nothing (896 columns over
-    // 896 3.3 -> 3.4 us, gate/up 4,864 over 896 7.1 -> 7.4).  One line of both halves a trip when GATED (two: 43.4 | 45.9); else two with many
-    // tiles, more than eight rows or a share of at most four lines, one otherwise (the down product of 18,944 to 3,584, one row 24.1 | 27.6,
-    // sixteen 38.8 | 36.3).  Us before | so, weights from memory, one row and sixteen: gate/up 18,944 over 3,584 55.0 | 43.4 and 59.7 | 52.4, down
-    // 30.0 | 24.1 and 44.3 | 36.3, 18,944 over 3,584 27.1 | 23.5 and 41.4 | 34.4; gate/up 8,960 over 1,536 14.7 | 13.0 and 17.0 | 16.0, down
-    // 11.0 | 10.1 and 13.9 | 13.2, 8,960 over 1,536 level; down 4,864 to 896 8.7 | 7.8 and 11.7 | 11.3.
+    // 896 3.3 -> 3.4 us, gate/up 4,864 over 896 7.1 -> 7.4).  Half as many waves with two sums each, so that the result is the one of half
+    // lines to the last bit.  With one workgroup a compute unit and eight sums, half lines' eight waves have more on their way: there only
+    // from five rows and 4,096 elements on (4,096 over 4,096, one and eight rows 9.2 and 9.4 us, whole lines 10.2 and 10.8; over 14,336
+    // 25.9 and 30.0, 28.1 and 28.8; gate/up 4,096 over 2,048 10.0 and 10.0, 10.6 and 10.9).  Lines a trip: few rows' own loads leave room
+    // for more of the weights' (see `lines_a_trip`).  Us half lines | so, weights from memory, one row and sixteen: gate/up 18,944 over 3,584
+    // 53.4 | 42.5 and 59.4 | 52.4, down 31.8 | 26.0 and 44.4 | 35.1, 18,944 over 3,584 28.2 | 22.5 and 41.2 | 32.9; 3,584 over 3,584 8.0 | 7.5
+    // and 9.5 | 9.1; gate/up 8,960 over 1,536 15.2 | 13.9 and 17.0 | 15.6, down 13.9 | 12.7 and 20.8 | 18.0; down 4,864 to 896 8.6 | 7.8 and
+    // 11.7 | 10.9; 768 over 3,072 6.2 | 6.0 and 8.0 | 7.9.  Weights that are in the last-level cache already (all of a model in less than its
+    // 256 MB) lose by it, one row and eight: 768 over 3,072 5.6 | 5.9 and 6.8 | 6.9, 896 over 4,864 7.8 | 7.8 and 9.3 | 9.4, 3,584 over
+    // 3,584 6.6 | 6.8 and 7.5 | 8.0; the kernel cannot know, and models of that size are the exception.
     const int lines = K / 64;
-    if (g_lines && (K & 63) == 0 && lines > 2 * waves) {
-      const bool two = !GATED && (waves == 4 || M > 8 || lines <= 4 * waves);
-#define GO(NWV, L) return launch_skinny<1, NWV, GATED, 1, L, true>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act)
-      if (two) { if (waves == 4) GO(4, 2); if (waves == 8) GO(8, 2); GO(16, 2); }
-      if (waves == 4) GO(4, 1);
-      if (waves == 8) GO(8, 1);
-      GO(16, 1);
+    if (g_lines && (K & 63) == 0 && lines > 2 * waves && (waves != 8 || tiles > compute_units() || (!GATED && M > 4 && K > 4096))) {
+      const int up = waves == 8 && tiles <= compute_units() ? 3 : lines_a_trip(GATED, waves, M, K);
+#define GO(NWV, L) return launch_skinny<1, NWV, GATED, 1, L, true, 2>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act)
+#define TRIPS(NWV) if (up == 1) GO(NWV, 1); if (up == 2) GO(NWV, 2); if constexpr (!GATED && NWV > 2) { if (up == 3) GO(NWV, 3); } \
+                   if constexpr (!GATED && NWV == 8) { if (up == 4) GO(NWV, 4); } if constexpr (NWV == 4) { if (up == 6) GO(NWV, 6); }
+      if (waves == 4) { TRIPS(2) }
+      if (waves == 8) { TRIPS(4) }
+      if (waves == 16) { TRIPS(8) }
+#undef TRIPS
 #undef GO
     }
   }
@@ -380,8 +415,8 @@ extern "C" int ta_gemm_skinny_bf16(const void* A, int lda, const void* W, const 
 }
 
 // The same product (not gated) with K cut into `splits` parts (at most; parts are multiples of 32, of 64 for up to sixteen rows and
-// K in whole lines, which are then read as such: 8 rows x 1,536 over 8,960 12.2 -> 11.7 us, one row 11.0 -> 10.2) over the
-// workgroups, the parts' float sums added afterwards in a fixed order.  partial: room for splits * M * N floats;
+// K in whole lines, which are then always read as such, one block of columns a workgroup, whatever `ta_skinny_lines` and `col_blocks`
+// say: 8 rows x 1,536 over 8,960 12.2 -> 11.7 us, one row 11.0 -> 10.2) over the workgroups, the parts' float sums added afterwards in a fixed order.  partial: room for splits * M * N floats;
 // N % 4 == 0; M <= 64.  With C null (and more than one part after the rounding of the parts' length) the sums are
 // left in `partial` for a later kernel to add.
 extern "C" int ta_gemm_skinny_bf16_splitk(const void* A, int lda, const void* W, const void* bias, void* C, int ldc,

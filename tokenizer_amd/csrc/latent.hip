@@ -188,23 +188,11 @@ head_linear_mfma_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride, i
 
 // Few rows (single tokens): a wave owns one output column of one head for up to HS_ROWS rows and reads the column's
 // row of W once, sixteen bytes a lane a trip, so that the head's matrix streams from memory once whatever the rows.
-// GATED: row m's results, rounded, times sigmoid(gate[m gate_row + h gate_head + n gate_unit]).  The sums over the wave run in registers (rotations
-// within sixteen lanes, then from row to row), and a lane a row stores: eight sums through the LDS crossbar and a lane's eight stores one behind
+// GATED: row m's results, rounded, times sigmoid(gate[m gate_row + h gate_head + n gate_unit]).  The sums over the wave run in registers
+// (`wave_sum`), and a lane a row stores: eight sums through the LDS crossbar and a lane's eight stores one behind
 // the other were half of the kernel, and the gate a kernel of its own (four rows, 14 heads of 64 over 128: 5.0 + 5.0 us where they were
 // profiled, 3.6 so).
 #define HS_ROWS 8
-__device__ __forceinline__ float hs_wave_sum(float x) {      // in every lane
-#define HS_DPP(code, rows) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), code, rows, 0xF, false))
-  x += HS_DPP(0x128, 0xF);
-  x += HS_DPP(0x124, 0xF);
-  x += HS_DPP(0x122, 0xF);
-  x += HS_DPP(0x121, 0xF);
-  x += HS_DPP(0x142, 0xA);                                   // lane 15 of a row into the next
-  x += HS_DPP(0x143, 0xC);                                   // lane 31 into the upper half
-#undef HS_DPP
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
-}
-
 template <bool GATED>
 __global__ void __launch_bounds__(256)
 head_linear_skinny_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride, int x_offset, const bf16_t* __restrict__ W,
@@ -236,7 +224,7 @@ head_linear_skinny_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride,
 #pragma unroll
   for (int i = 0; i < HS_ROWS; ++i) {
     if (m0 + i >= M) break;
-    const float total = hs_wave_sum(acc[i]);
+    const float total = wave_sum(acc[i]);
     if (lane == i) mine = total;
   }
   if (lane < HS_ROWS && m0 + lane < M) {
