@@ -82,3 +82,18 @@ def test_sum_over_a_wave_starts_with_lanes_32_apart(ops, rows):
     gate = torch.zeros((rows, heads * n), dtype=torch.bfloat16, device="cuda")
     ops.head_linear(x, 0, k, w, out, 0, n, gate=(gate, 0, n))
     assert (out == 0.5).all()
+
+
+@pytest.mark.parametrize("hidden, inner, shared", [(512, 1040, 0), (1000, 1040, 64), (2056, 520, 0)])
+def test_experts_of_one_row_and_of_many_have_the_same_bits(ops, hidden, inner, shared):
+    # Few workgroups ask for four turns of K at once, many for one: shares of K that end inside a trip, K that is no whole line.
+    experts, top = 8, 2
+    x = rand((16, hidden), 4)
+    first, second = rand((2 * (experts * inner + shared), hidden), 5, hidden ** -0.5), rand((hidden, experts * inner + shared), 6, inner ** -0.5)
+    gen = torch.Generator().manual_seed(7)
+    chosen = torch.stack([torch.randperm(experts, generator=gen)[:top] for _ in range(16)]).int().cuda()
+    weights = torch.rand((16, top), generator=gen).cuda()
+    run = lambda rows: ops.experts_few(x[:rows], chosen[:rows].contiguous(), weights[:rows].contiguous(), experts, first, True, inner,
+                                       second, shared=shared).partial
+    many, one = run(16), run(1)
+    assert many.isfinite().all() and torch.equal(many[:, :1], one)

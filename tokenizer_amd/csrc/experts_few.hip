@@ -37,13 +37,10 @@ __device__ __forceinline__ int ef_pairs_of(const int* __restrict__ chosen, int n
 struct EfShared { int inner; const float* weights; bf16_t* act; int parts, length; };   // K of `inner` in `parts` of `length`
 
 // acc[h] += sixteen rows of matrix h (lane (col, g): `w_at[h][0]` is row col % 8 of them, `w_at[h][1]` row 8 + col % 8) times the
-// lane's row of x, over this wave's turns of K.
-template <int NW, int HALVES>
+// lane's row of x, over this wave's turns of K, UN of which are asked for at once.
+template <int NW, int HALVES, int UN>
 __device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], const bf16_t* x_at, bool x_ok, int K, int wave,
                                         ef_floatx4 (&acc)[HALVES]) {
-  // Turns asked for at once: four loads of weights a lane of two matrices (twice as many take registers that more waves a
-  // compute unit make better use of: twelve rows of the second example above 46.0 | 44.5 us), eight of one (four: 44.6).
-  constexpr int UN = HALVES == 2 ? 1 : 4;
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, piece = g + 4 * (col >> 3);
   const int turns = (K + 63) / 64;
   const word4 zero = {0u, 0u, 0u, 0u};
@@ -81,7 +78,7 @@ __device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], 
 // W + e * HALVES * inner * hidden: [gate; up] of `inner` rows each (HALVES 2) or `up` alone (HALVES 1), rows of `hidden`.
 // act [n_rows * top, inner]: pair p's row.  HALVES 2: weigh_input ? silu(w g) * (w u) : w * silu(g) * u; HALVES 1: w * max(u, 0)^2.
 // Grid: (blocks of sixteen columns of inner, experts).
-template <int NW, int HALVES>
+template <int NW, int HALVES, int UN>
 __global__ void __launch_bounds__(NW * WAVE)
 experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __restrict__ chosen, const float* __restrict__ weights,
                       int n_pairs, int top, const bf16_t* __restrict__ W, int inner, int hidden, bf16_t* __restrict__ act,
@@ -118,7 +115,7 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
     ef_floatx4 acc[HALVES];
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) acc[h] = (ef_floatx4){0.f, 0.f, 0.f, 0.f};
-    ef_walk<NW, HALVES>(w_at, x_at, ok, hidden, wave, acc);
+    ef_walk<NW, HALVES, UN>(w_at, x_at, ok, hidden, wave, acc);
     // A matrix instruction's result may be read eight wait states behind it at the earliest.  The compiler leaves them out in front
     // of the stores below where there is one matrix (the store is the second instruction behind the last sum; with many
     // workgroups some stored a sum that was not there yet), so they are here, twice over; with two matrices it has them.
@@ -196,7 +193,7 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
     const bool ok = p0 + col < count;
     const bf16_t* x_at = act + (size_t)list[min(p0 + col, count - 1)] * stride;
     ef_floatx4 acc[1] = {(ef_floatx4){0.f, 0.f, 0.f, 0.f}};
-    ef_walk<NW, 1>(w_at, x_at, ok, inner, wave, acc);
+    ef_walk<NW, 1, 4>(w_at, x_at, ok, inner, wave, acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave][r][lane] = acc[0][r];
     __syncthreads();
@@ -248,12 +245,18 @@ extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, c
   if (n_experts + every.parts > 65535) return -2;            // (a grid's second dimension)
   const dim3 up(((inner > shared ? inner : shared) + 15) / 16, n_experts + (shared > 0)),
       down((hidden + 15) / 16, n_experts + every.parts);
-#define UP(NW, HH) experts_few_up_kernel<NW, HH><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
+#define UP(NW, HH, UN) experts_few_up_kernel<NW, HH, UN><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
     (const float*)weights, (int)pairs, top, (const bf16_t*)w_first, inner, hidden, (bf16_t*)act, weigh_input, every)
 #define DOWN(NW) experts_few_down_kernel<NW><<<down, NW * WAVE, 0, stream>>>((const bf16_t*)act, (const int*)chosen, (int)pairs, top, \
     n_rows, (const bf16_t*)w_second, ldw, inner, hidden, (float*)out, every)
-  if (halves == 2) { if (hidden <= 1024) UP(4, 2); else UP(8, 2); }
-  else { if (hidden <= 1024) UP(4, 1); else UP(8, 1); }
+  // Turns asked for at once.  One of two matrices, four loads of weights a lane (two take registers that more waves a compute unit make
+  // better use of: 5,504 over 2,048, four rows 52.5 | 55.0 us for both products), but four where the workgroups cannot be more than the
+  // compute units, however the rows choose, and none has another to hide its trips (one | four: 1,792 over 4,096, one row 33.6 | 24.8; 1,024
+  // over 1,024 10.9 | 9.4, two rows 11.4 | 9.8; 512 over 1,024, four rows 11.5 | 10.0).  Four of one matrix, eight loads.
+  const long busy = (pairs < n_experts ? pairs : n_experts) * ((inner + 15) / 16) + (shared + 15) / 16;
+  if (halves == 1) { if (hidden <= 1024) UP(4, 1, 4); else UP(8, 1, 4); }
+  else if (busy <= compute_units()) { if (hidden <= 1024) UP(4, 2, 4); else UP(8, 2, 4); }
+  else { if (hidden <= 1024) UP(4, 2, 1); else UP(8, 2, 1); }
   int status = LAUNCH_STATUS();
   if (status != 0) return status;
   if (inner <= 1024) DOWN(4); else DOWN(8);
