@@ -84,3 +84,39 @@ def test_blocks_of_eight_tokens(dtype, heads, groups, d, dv, strong):
     assert hit[cu[4] + 13, 1] and not hit[cu[4] + 14:cu[5], 1].any()
     error = lambda out: float((out[:cu[-1]] - want[:cu[-1]]).norm())
     assert error(results[0][0]) <= 2 * error(results[1][0])    # no less exact than the walk token by token (a factor for chance)
+
+
+def random_step(lengths, heads, groups, d, seed):
+    """A step's operands on the device, bfloat16, and a run of them that gives (out, state)."""
+    from tokenizer_amd.kernels import get_ops
+    ops, gen = get_ops(), torch.Generator().manual_seed(seed)
+    rand = lambda *shape: torch.randn(*shape, generator=gen)
+    T, cu = sum(lengths), [0]
+    for n in lengths:
+        cu.append(cu[-1] + n)
+    ints = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")
+    fresh, rows = rand(T, (2 * groups + heads) * d).bfloat16().cuda(), rand(T, heads).bfloat16().cuda()
+    z, rate, state = rand(T, heads * d).cuda(), -torch.rand(heads, generator=gen).cuda(), rand(len(lengths), heads * d * d).cuda() * 0.3
+    first, slots = ints([9 * (i % 2) for i in range(len(lengths))]), ints(list(range(len(lengths))))
+
+    def run(blocks=None, **more):
+        held, out = state.clone(), torch.zeros(T, heads * d, device="cuda")
+        kept = ops.DELTA_BLOCK_ROWS
+        ops.DELTA_BLOCK_ROWS = kept if blocks is None else (0, 0) if blocks else (1 << 30, 1 << 30)
+        try:
+            ops.delta_scan(fresh, z, rate, rows, 0, held, ints(cu), first, slots, out, heads, groups, d, d, 1e-6, **more)
+        finally:
+            ops.DELTA_BLOCK_ROWS = kept
+        return out, held
+    return run
+
+
+def test_a_long_portion_beside_single_tokens_walks_in_blocks():
+    from tokenizer_amd.parts.delta import portion_rows
+    lengths = [300] + [1] * 15
+    run = random_step(lengths, 4, 2, 64, 1)
+    same = lambda a, b: all(torch.equal(x, y) for x, y in zip(a, b))
+    scan, blocks = run(blocks=False), run(blocks=True)
+    assert not same(scan, blocks)
+    assert same(run(portion_rows=portion_rows(sum(lengths), len(lengths), 15)), blocks)
+    assert same(run(), scan)                                  # (who calls without: the average over all entries)

@@ -593,7 +593,8 @@ class Ops:
 
     def delta_scan(self, fresh: torch.Tensor, decay: torch.Tensor, neg_rate: torch.Tensor, rows: torch.Tensor, beta_offset: int,
                    state: torch.Tensor, cu_q: torch.Tensor, first_position: torch.Tensor, state_slots: torch.Tensor,
-                   out: torch.Tensor, heads: int, groups: int, d: int, dv: int, unit_eps: float) -> torch.Tensor:
+                   out: torch.Tensor, heads: int, groups: int, d: int, dv: int, unit_eps: float,
+                   portion_rows: int = 0) -> torch.Tensor:
         """The gated delta rule over every entry's rows, from and into the entries' state rows.
 
         fresh [T, 2 groups d + heads dv]: q, k (groups of d; head h reads group h // (heads / groups)) and v (heads of
@@ -602,7 +603,9 @@ class Ops:
         S <- diag(g) S; u = beta (v - S^T k); S <- S + k u^T; out = S^T q.  state float32 [slots, >= heads d dv] (an
         entry whose first position is 0 starts from zeros); out float32 [T, heads dv].
 
-        Steps with portions of many rows (see `DELTA_BLOCK_ROWS`) walk in blocks of eight tokens on the float matrix instructions; what does not depend on the state is made for all blocks side by side first."""
+        Steps with portions of many rows (see `DELTA_BLOCK_ROWS`) walk in blocks of eight tokens on the float matrix instructions; what
+        does not depend on the state is made for all blocks side by side first.  `portion_rows`: how many rows a portion of
+        several brings at least, where the caller knows (the average over all entries hides one among single tokens)."""
         _dev(fresh, decay, neg_rate, rows, state, cu_q, first_position, state_slots, out)
         n_tokens = fresh.shape[0]
         _need(heads > 0 and groups > 0 and heads % groups == 0 and 0 < d <= 256 and dv > 0, "heads of up to 256 key channels")
@@ -619,7 +622,8 @@ class Ops:
         record = heads * (25 * next(size for size in (16, 32, 64, 128, 256) if d <= size) + 128)
         few, many = self.DELTA_BLOCK_ROWS
         crowd = n_entries * heads * -(-dv // 16) * d >= 2 ** 17
-        if n_tokens > (few if crowd else many) * n_entries and (n_tokens // 8 + n_entries) * record <= self.DELTA_PREPARED:
+        long = n_tokens > (few if crowd else many) * n_entries or portion_rows > many
+        if long and (n_tokens // 8 + n_entries) * record <= self.DELTA_PREPARED:
             _need(decay.is_contiguous(), "the decays have rows of their own")
             prepared = torch.empty((n_tokens // 8 + n_entries, record), dtype=torch.float32, device=fresh.device)
         self._check(self.lib.ta_delta_scan(_ptr(fresh), fresh.shape[1], _ptr(decay), _ptr(neg_rate), _ptr(rows), rows.shape[1],
@@ -629,9 +633,11 @@ class Ops:
                                            self._stream()), "delta_scan")
         return out
 
+    delta_by_portion = True       # `delta_scan(portion_rows=...)` exists here
     # Rows an entry (on average) above which the delta rule walks in blocks: where its columns of state fill the device, and where they do
-    # not.  (Token by token | in blocks, us: eight portions of five tokens, 28 heads of 128 36 | 32, eight of 256 72 | 44, 12 of 128 19 | 24,
-    # 14 of 64 16 | 22; of 12 tokens 42 | 38, 77 | 52, 22 | 28, 14 | 19; 64 of six, 14 heads of 64 35 | 31; 20 of 37 38 | 35.)
+    # not, or one portion alone brings as many.  (Token by token | in blocks, us: eight portions of five tokens, 28 heads of 128 40 | 31,
+    # eight of 256 74 | 42, 12 of 128 20 | 23, 14 of 64 9 | 16; of 12 tokens 44 | 37, 78 | 51, 23 | 27, 10 | 19; of 24 66 | 43, 140 | 55, 34 | 30,
+    # 15 | 20; 64 of six, 14 heads of 64 35 | 30; 20 of 37 38 | 34.  One of 300 beside 15 single tokens 1,041 | 287, 2,496 | 357, 461 | 153, 172 | 55.)
     DELTA_BLOCK_ROWS = (4, 24)
     DELTA_PREPARED = 2 ** 30   # the room their records may take: floats (87,000 tokens of 28 heads of 128)
 

@@ -7,6 +7,13 @@ from .base import MIXERS, Mixer, Runtime
 from .spec import CacheNeed, MixerSpec, TensorSpec
 
 
+def portion_rows(n_tokens: int, n_entries: int, n_single: int) -> int:
+    """How many rows each portion of several brings on average, or more, in a step of `n_single` single tokens.  From the counts a
+    description is filled up to, so that a replayed step and the same one run eagerly choose alike: one of the portions counted at
+    least is there to do nothing (`filled_counts`)."""
+    return (n_tokens - n_single) // max(1, n_entries - n_single - 1)
+
+
 @MIXERS.register("gated_delta")
 class GatedDelta(Mixer):
     """With h the mixer's input, H = `n_heads`, G = `n_kv_heads` query/key heads of d, value heads of dv:
@@ -101,8 +108,11 @@ class GatedDelta(Mixer):
         decay = ops.linear(low_a, self.w_a2, self.dt_bias, out_dtype=torch.float32)       # the bias joins the float sum
         gate = ops.linear(low_g, self.w_g2)
         read = torch.empty((n_tokens, H * dv), dtype=torch.float32, device=x.device)
+        more = {}
+        if getattr(ops, "delta_by_portion", False):
+            more["portion_rows"] = portion_rows(n_tokens, ctx.n_entries, ctx.decode_rows.numel())
         ops.delta_scan(fresh, decay, self.neg_rate, rows, self.offsets["b"], cache.state, ctx.cu_q, ctx.first_position,
-                       ctx.state_slots, read, H, self.groups, d, dv, self.unit_eps)
+                       ctx.state_slots, read, H, self.groups, d, dv, self.unit_eps, **more)
         mixed = torch.empty((n_tokens, H * dv), dtype=x.dtype, device=x.device)
         ops.head_norm_gate(read, self.norm, gate, 0, self.eps, H, dv, mixed)
         return ops.linear(mixed, self.w_o)
