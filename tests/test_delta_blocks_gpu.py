@@ -99,14 +99,15 @@ def random_step(lengths, heads, groups, d, seed):
     z, rate, state = rand(T, heads * d).cuda(), -torch.rand(heads, generator=gen).cuda(), rand(len(lengths), heads * d * d).cuda() * 0.3
     first, slots = ints([9 * (i % 2) for i in range(len(lengths))]), ints(list(range(len(lengths))))
 
-    def run(blocks=None, **more):
+    def run(blocks=None, prepared=None, **more):
         held, out = state.clone(), torch.zeros(T, heads * d, device="cuda")
-        kept = ops.DELTA_BLOCK_ROWS
-        ops.DELTA_BLOCK_ROWS = kept if blocks is None else (0, 0) if blocks else (1 << 30, 1 << 30)
+        kept = ops.DELTA_BLOCK_ROWS, ops.DELTA_PREPARED
+        ops.DELTA_BLOCK_ROWS = kept[0] if blocks is None else (0, 0) if blocks else (1 << 30, 1 << 30)
+        ops.DELTA_PREPARED = kept[1] if prepared is None else prepared
         try:
             ops.delta_scan(fresh, z, rate, rows, 0, held, ints(cu), first, slots, out, heads, groups, d, d, 1e-6, **more)
         finally:
-            ops.DELTA_BLOCK_ROWS = kept
+            ops.DELTA_BLOCK_ROWS, ops.DELTA_PREPARED = kept
         return out, held
     return run
 
@@ -120,3 +121,14 @@ def test_a_long_portion_beside_single_tokens_walks_in_blocks():
     assert not same(scan, blocks)
     assert same(run(portion_rows=portion_rows(sum(lengths), len(lengths), 15)), blocks)
     assert same(run(), scan)                                  # (who calls without: the average over all entries)
+
+
+# Slices of one block a portion, of three (which end inside and at the end of a portion), and portions of less than one.
+@pytest.mark.parametrize("d", [16, 64, 200])
+@pytest.mark.parametrize("each", [1, 3])
+def test_blocks_slice_by_slice_are_the_same(d, each):
+    lengths = [53, 0, 24, 1, 8, 17]
+    run = random_step(lengths, 2, 1, d, d)
+    size = next(s for s in (16, 64, 256) if d <= s)
+    want, got = run(blocks=True), run(blocks=True, prepared=each * len(lengths) * 2 * (25 * size + 128))
+    assert all(torch.equal(x, y) for x, y in zip(got, want))

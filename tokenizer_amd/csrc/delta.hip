@@ -146,7 +146,8 @@ short_conv_step_kernel(const T* __restrict__ rows, int row_stride, ConvRuns runs
 // state behind the block is G_last S + sum_j e_j u_j, e_j = k_j times the decays behind j.  T and D T are lower triangular, a head's own and the
 // same for all columns of S.  Decays are only ever multiplied: nothing is divided by them.
 // This kernel makes all that does not depend on the state, for every block side by side: a wave a (block, head), a lane R rows of it.
-// A block's record (block number cu_q[e] / 8 + e + its number in the portion, which no two share) of 25 DP + 128 floats, DP = d filled up to a multiple
+// EACH 0: all blocks of all portions; else blocks FIRST .. FIRST + EACH - 1 of every portion, for steps whose records are more than their room.
+// A block's record (number cu_q[e] / 8 + e + its number in the portion, which no two share; else EACH e + its number among those) of 25 DP + 128 floats, DP = d filled up to a multiple
 // of 16 with zeros: [16 rows of DP: row 4 (a / 2) + a % 2 k G of token a, two further on its q G | e of token 2 g + s, row
 // 16 b + i: place (16 g + i) DP / 8 + 2 b + s | G_last | T and D T: place 2 (16 g + row) + s, row as above with T and D T for k G and q G, column
 // token 2 g + s].  Tokens past the end are zeros.
@@ -156,14 +157,22 @@ template <typename T, int R>
 __global__ void __launch_bounds__(4 * WAVE)
 delta_blocks_kernel(const T* __restrict__ fresh, int fresh_stride, const float* __restrict__ z, const float* __restrict__ neg_rate,
                     const T* __restrict__ beta_rows, int beta_stride, int beta_offset, float* __restrict__ prep,
-                    const int* __restrict__ cu_q, int n_entries, int heads, int groups, int d, int dp, float unit_eps) {
+                    const int* __restrict__ cu_q, int n_entries, int heads, int groups, int d, int dp, float unit_eps, int first,
+                    int each) {
   const int block = blockIdx.x, lane = threadIdx.x & (WAVE - 1), h = blockIdx.y * 4 + wave_index();
-  int from = 0;                                              // portions whose blocks' numbers begin at this one's or before
-  for (int i = lane; i < n_entries; i += WAVE) from += cu_q[i] / DL_BLOCK + i <= block ? 1 : 0;
+  int e, number;
+  if (each > 0) {
+    e = block / each;
+    number = first + block % each;
+  } else {
+    int from = 0;                                            // portions whose blocks' numbers begin at this one's or before
+    for (int i = lane; i < n_entries; i += WAVE) from += cu_q[i] / DL_BLOCK + i <= block ? 1 : 0;
 #pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) from += __shfl_xor(from, off, WAVE);
-  const int e = __builtin_amdgcn_readfirstlane(from) - 1;    // (the first portion's begin at 0)
-  const int lo = cu_q[e], t = lo + (block - lo / DL_BLOCK - e) * DL_BLOCK, count = min(DL_BLOCK, cu_q[e + 1] - t);
+    for (int off = WAVE / 2; off > 0; off >>= 1) from += __shfl_xor(from, off, WAVE);
+    e = __builtin_amdgcn_readfirstlane(from) - 1;            // (the first portion's begin at 0)
+    number = block - cu_q[e] / DL_BLOCK - e;
+  }
+  const int t = cu_q[e] + number * DL_BLOCK, count = min(DL_BLOCK, cu_q[e + 1] - t);
   if (count <= 0 || h >= heads) return;
   const float q_scale = 1.0f / sqrtf((float)d), rate = neg_rate[h];
   const int grp = h / (heads / groups);
@@ -270,23 +279,25 @@ delta_blocks_kernel(const T* __restrict__ fresh, int fresh_stride, const float* 
 // converted where it arrives makes the wave wait for all that is under way.  Per block DP / 4 instructions for (k G, q G) S, two for
 // (T, D T) y, DP / 2 for the state's update: at d = 64 26 of 32 clocks for eight tokens.  Bound by their chain: 0.9 us a block
 // where token by token eight took 1.6, a chain of some two dozen dependent instructions and two sums over lanes each.
-// (In a step with portions of 150 to 1,000 tokens, 14 heads of 64: token by token 199 us and 13 for what was prepared, so 115 and 25.  Both kernels
-// alone, token by token | so: one portion of 2,048 tokens 531 | 259, 12 heads of 128 818 | 450, eight of 256 2,790 | 1,050; 32 portions of 200
-// tokens 204 | 105, 12 heads of 128 618 | 210.)
+// (Both kernels, us: what had the same prepared token by token and then walked token by token | so.  One portion of 2,048 tokens, 14 heads of
+// 64 395 | 234, 12 of 128 539 | 391, eight of 256 2,167 | 1,058; portions of 150 to 1,000 tokens 198 | 136, 319 | 209, 1,878 | 541; 32 portions
+// of 200 tokens 169 | 105, 438 | 207, 3,078 | 546; one of 300 beside fifteen single tokens 120 | 53, 283 | 138, 2,204 | 343.)
 typedef float dl_x4 __attribute__((ext_vector_type(4)));
 template <typename T, int NB>
 __global__ void __launch_bounds__(4 * WAVE, 1)
 delta_walk_kernel(const T* __restrict__ fresh, int fresh_stride, const float* __restrict__ prep, float* __restrict__ state,
                   size_t state_stride, const int* __restrict__ cu_q, const int* __restrict__ first_position,
-                  const int* __restrict__ state_slots, float* __restrict__ out, int heads, int groups, int d, int dv) {
+                  const int* __restrict__ state_slots, float* __restrict__ out, int heads, int groups, int d, int dv, int first,
+                  int each) {
   constexpr int DP = 16 * NB, AHEAD = NB <= 8 ? 2 : 1;
   const int e = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & (WAVE - 1), col = lane & 15, g = lane >> 4;
   const int lo = cu_q[e], hi = cu_q[e + 1], first_col = ((int)blockIdx.z * 4 + wave_index()) * 16;
   if (hi <= lo || first_col >= dv) return;                   // (the same for the whole wave)
-  const int c = first_col + col, blocks = (hi - lo + DL_BLOCK - 1) / DL_BLOCK;
+  const int c = first_col + col, all = (hi - lo + DL_BLOCK - 1) / DL_BLOCK, blocks = each > 0 ? min(all, first + each) : all;
+  if (first >= blocks) return;                               // (its last block is behind it)
   const bool live = c < dv;
   float* mem = state + (size_t)state_slots[e] * state_stride + (size_t)h * d * dv;
-  const bool from_zero = first_position[e] == 0;
+  const bool from_zero = first == 0 && first_position[e] == 0;
   dl_x4 S[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -295,14 +306,14 @@ delta_walk_kernel(const T* __restrict__ fresh, int fresh_stride, const float* __
       const int j = 16 * b + 4 * g + r;
       S[b][r] = (!from_zero && live && j < d) ? mem[(size_t)j * dv + c] : 0.f;
     }
-  const float* mine = prep + ((size_t)(lo / DL_BLOCK + e) * heads + h) * DL_RECORD(DP);
+  const float* mine = prep + ((size_t)(each > 0 ? each * e : lo / DL_BLOCK + e) * heads + h) * DL_RECORD(DP);
   const size_t record = (size_t)heads * DL_RECORD(DP);
   const T* values = fresh + (size_t)2 * groups * d + (size_t)h * dv + min(c, dv - 1);
   typedef float dl_x2 __attribute__((ext_vector_type(2)));
   struct Block { dl_x4 rows[NB], decay[NB]; float back[NB][2]; dl_x2 number; T v[2]; };
   auto fetch = [&](Block& x, int asked) {
     const int n = min(asked, blocks - 1);
-    const float* at = mine + n * record;
+    const float* at = mine + (n - first) * record;
 #pragma unroll
     for (int b = 0; b < NB; ++b) x.rows[b] = *reinterpret_cast<const dl_x4*>(at + col * DP + 16 * b + 4 * g);
 #pragma unroll
@@ -326,8 +337,8 @@ delta_walk_kernel(const T* __restrict__ fresh, int fresh_stride, const float* __
   };
   Block next[AHEAD];
 #pragma unroll
-  for (int i = 0; i < AHEAD; ++i) fetch(next[i], i);
-  for (int from = 0; from < blocks; from += AHEAD)
+  for (int i = 0; i < AHEAD; ++i) fetch(next[i], first + i);
+  for (int from = first; from < blocks; from += AHEAD)
 #pragma unroll
   for (int turn = 0; turn < AHEAD; ++turn) {
     const int n = from + turn, t0 = lo + n * DL_BLOCK;
@@ -541,12 +552,14 @@ extern "C" int ta_short_conv_silu(const void* rows, int row_stride, int o0, int 
 }
 
 // fresh: rows of `fresh_stride` elements, [groups d (q) | groups d (k) | heads dv (v)]; z float [n_tokens, heads d];
-// neg_rate float [heads]; out float [n_tokens, heads dv].  prep: null, or room for n_tokens / 8 + n_entries records of heads (25 d' + 128) floats,
-// d' = d filled up to 16, 32, 64, 128 or 256: then the portions walk in blocks of eight tokens, whose share that does not depend on the
-// state is made for all of them side by side first, which is what steps with long portions want.
+// neg_rate float [heads]; out float [n_tokens, heads dv].  prep: null, or room for `records` (at least n_entries) records of heads
+// (25 d' + 128) floats, d' = d filled up to 16, 32, 64, 128 or 256: then the portions walk in blocks of eight tokens, whose share that does
+// not depend on the state is made for all of them side by side first, which is what steps with long portions want.  n_tokens / 8 +
+// n_entries records hold all blocks; with fewer the portions walk slice by slice, every portion's next records / n_entries blocks, and
+// the state is carried in memory.
 extern "C" int ta_delta_scan(const void* fresh, int fresh_stride, const void* z, const void* neg_rate, const void* beta_rows,
                              int beta_stride, int beta_offset, void* state, long state_stride, const void* cu_q,
-                             const void* first_position, const void* state_slots, void* out, void* prep, int n_tokens,
+                             const void* first_position, const void* state_slots, void* out, void* prep, int records, int n_tokens,
                              int n_entries, int heads, int groups, int d, int dv, float unit_eps, int dtype,
                              hipStream_t stream) {
   if (n_entries <= 0 || n_tokens <= 0) return 0;
@@ -559,17 +572,21 @@ extern "C" int ta_delta_scan(const void* fresh, int fresh_stride, const void* z,
   if (prep) {
     const int nb = per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : per <= 8 ? 8 : 16;
     const dim3 walks(n_entries, heads, (dv + 63) / 64);
-#define BLOCKS(TT, RR) delta_blocks_kernel<TT, RR><<<dim3(n_tokens / DL_BLOCK + n_entries, (heads + 3) / 4), 4 * WAVE, 0, stream>>>( \
+    const int all = n_tokens / DL_BLOCK + n_entries, each = records >= all ? 0 : records / n_entries;
+    if (each < 1 && records < all) return -1;
+#define BLOCKS(TT, RR) delta_blocks_kernel<TT, RR><<<dim3(each ? each * n_entries : all, (heads + 3) / 4), 4 * WAVE, 0, stream>>>( \
     (const TT*)fresh, fresh_stride, (const float*)z, (const float*)neg_rate, (const TT*)beta_rows, beta_stride, beta_offset,      \
-    (float*)prep, (const int*)cu_q, n_entries, heads, groups, d, 16 * nb, unit_eps)
+    (float*)prep, (const int*)cu_q, n_entries, heads, groups, d, 16 * nb, unit_eps, first, each)
 #define WALK(TT, NN) delta_walk_kernel<TT, NN><<<walks, 4 * WAVE, 0, stream>>>((const TT*)fresh, fresh_stride, (const float*)prep, \
     (float*)state, (size_t)state_stride, (const int*)cu_q, (const int*)first_position, (const int*)state_slots, (float*)out,     \
-    heads, groups, d, dv)
+    heads, groups, d, dv, first, each)
 #define BOTH(TT)                                                                                                              \
     if (nb <= 4) BLOCKS(TT, 1); else if (nb <= 8) BLOCKS(TT, 2); else BLOCKS(TT, 4);                                           \
     if (nb == 1) WALK(TT, 1); else if (nb == 2) WALK(TT, 2); else if (nb == 4) WALK(TT, 4); else if (nb == 8) WALK(TT, 8);     \
     else WALK(TT, 16)
-    if (dtype == DT_F32) { BOTH(float); } else { BOTH(bf16_t); }
+    for (int first = 0; first * DL_BLOCK < n_tokens; first += each ? each : all) {      // (no portion is longer than the step)
+      if (dtype == DT_F32) { BOTH(float); } else { BOTH(bf16_t); }
+    }
 #undef BOTH
 #undef WALK
 #undef BLOCKS

@@ -618,17 +618,17 @@ class Ops:
         _need(out.dtype == torch.float32 and tuple(out.shape) == (n_tokens, heads * dv), "out float32 [T, heads dv]")
         n_entries = cu_q.numel() - 1
         _need(first_position.numel() == n_entries == state_slots.numel(), "one first position and slot per entry")
-        prepared = None
-        record = heads * (25 * next(size for size in (16, 32, 64, 128, 256) if d <= size) + 128)
+        prepared, records = None, 0
         few, many = self.DELTA_BLOCK_ROWS
         crowd = n_entries * heads * -(-dv // 16) * d >= 2 ** 17
-        long = n_tokens > (few if crowd else many) * n_entries or portion_rows > many
-        if long and (n_tokens // 8 + n_entries) * record <= self.DELTA_PREPARED:
+        if n_tokens > (few if crowd else many) * n_entries or portion_rows > many:
             _need(decay.is_contiguous(), "the decays have rows of their own")
-            prepared = torch.empty((n_tokens // 8 + n_entries, record), dtype=torch.float32, device=fresh.device)
+            record = heads * (25 * next(size for size in (16, 32, 64, 128, 256) if d <= size) + 128)
+            records = min(n_tokens // 8 + n_entries, max(n_entries, self.DELTA_PREPARED // record))
+            prepared = torch.empty((records, record), dtype=torch.float32, device=fresh.device)
         self._check(self.lib.ta_delta_scan(_ptr(fresh), fresh.shape[1], _ptr(decay), _ptr(neg_rate), _ptr(rows), rows.shape[1],
                                            beta_offset, _ptr(state), ctypes.c_long(state.shape[1]), _ptr(cu_q),
-                                           _ptr(first_position), _ptr(state_slots), _ptr(out), _ptr(prepared), n_tokens,
+                                           _ptr(first_position), _ptr(state_slots), _ptr(out), _ptr(prepared), records, n_tokens,
                                            n_entries, heads, groups, d, dv, ctypes.c_float(unit_eps), _code(fresh.dtype),
                                            self._stream()), "delta_scan")
         return out
@@ -639,7 +639,8 @@ class Ops:
     # eight of 256 74 | 42, 12 of 128 20 | 23, 14 of 64 9 | 16; of 12 tokens 44 | 37, 78 | 51, 23 | 27, 10 | 19; of 24 66 | 43, 140 | 55, 34 | 30,
     # 15 | 20; 64 of six, 14 heads of 64 35 | 30; 20 of 37 38 | 34.  One of 300 beside 15 single tokens 1,041 | 287, 2,496 | 357, 461 | 153, 172 | 55.)
     DELTA_BLOCK_ROWS = (4, 24)
-    DELTA_PREPARED = 2 ** 30   # the room their records may take: floats (87,000 tokens of 28 heads of 128)
+    # The room their records may take, in floats: 11,500 tokens' of 28 heads of 128.  More walk slice by slice (see `ta_delta_scan`).
+    DELTA_PREPARED = 2 ** 27
 
     # ---------------------------------------------------- sigmoid router with groups, ungated experts
     def route_sigmoid(self, logits: torch.Tensor, correction: torch.Tensor, n_groups: int, keep_groups: int,
