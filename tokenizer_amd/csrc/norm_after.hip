@@ -565,7 +565,11 @@ norm_side_norm_held_kernel(float* __restrict__ residual, const void* __restrict_
     next[c] = weight ? *reinterpret_cast<const float2*>(weight + h) : make_float2(1.f, 1.f);
   }
   if constexpr (PARTS) {
-    constexpr int DEEP = R * RUNS <= 2 ? 8 : R * RUNS <= 4 ? 4 : 2;              // slabs asked for at a time
+    // Slabs asked for at a time.  With two runs both small matrices' rows take half of the registers: twice as many slabs would be put aside
+    // (rows of 3,584 in two parts, us, eight and four slabs of one row: 12.5 | 10.2, the parts added by a kernel of their own 11.1; four and
+    // two of two rows, 512 rows: 16.7 | 14.3, 17.2).  Four rows have some put aside either way and are ahead all the same (1,024 rows, two
+    // slabs and one: 25.5 | 28.0, 28.6; without parts 19.9, two rows a workgroup 23.6).
+    constexpr int DEEP = RUNS == 2 ? (R == 1 ? 4 : 2) : R <= 2 ? 8 : R <= 4 ? 4 : 2;
     for (int s0 = 1; s0 < parts; s0 += DEEP) {
       float2 v[DEEP][R][RUNS];
 #pragma unroll
