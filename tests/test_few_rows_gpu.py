@@ -421,14 +421,16 @@ def test_float32_qkv_with_rotation_and_store(ops, rows, heads, kv, d, k, rotate)
     assert torch.equal(silent, q)
 
 
-# The short convolution of steps of a token an entry: an entry of none, one of two (another has none), one that starts and one that goes on, rows
-# that only fill the batch up, two to four taps and (five: the kernels of long portions) more, three runs of channels past a workgroup's 256.
+# The short convolution of steps of a token an entry: entries of none, one of two, one that starts and one that goes on, a row that only fills the
+# batch up, two to four taps and (five: the kernels of long portions) more, three runs of channels past a workgroup's 256; as many rows as
+# entries (one kernel for all of it) and one row more (the two kernels of long portions).
+@pytest.mark.parametrize("lengths,starts", [([1, 0, 2, 0, 1, 1], [0, 0, 7, 5, 3, 0]), ([1, 0, 2, 1, 1], [0, 0, 7, 3, 0])])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("taps", [2, 3, 4, 5])
 @pytest.mark.parametrize("biased", [False, True])
-def test_short_convolution_of_single_tokens(ops, dtype, taps, biased):
+def test_short_convolution_of_single_tokens(ops, lengths, starts, dtype, taps, biased):
     gen = torch.Generator().manual_seed(taps)
-    lengths, starts, widths, offsets, fill = [1, 0, 2, 1, 1], [0, 0, 7, 3, 0], (96, 200, 40), (4, 300, 104), 1
+    widths, offsets, fill = (96, 200, 40), (4, 300, 104), 1
     channels, n, keep = sum(widths), sum(lengths) + fill, taps - 1
     rows = torch.randn(n, 512, generator=gen).to(dtype)
     weights, bias = torch.randn(channels, taps, generator=gen), torch.randn(channels, generator=gen) if biased else None
