@@ -147,8 +147,8 @@ short_conv_step_kernel(const T* __restrict__ rows, int row_stride, ConvRuns runs
 // same for all columns of S.  Decays are only ever multiplied: nothing is divided by them.
 // This kernel makes all that does not depend on the state, for every block side by side: a wave a (block, head), a lane R rows of it.
 // EACH 0: all blocks of all portions; else blocks FIRST .. FIRST + EACH - 1 of every portion, for steps whose records are more than their room.
-// A block's record (number cu_q[e] / 8 + e + its number in the portion, which no two share; else EACH e + its number among those) of 25 DP + 128 floats, DP = d filled up to a multiple
-// of 16 with zeros: [16 rows of DP: row 4 (a / 2) + a % 2 k G of token a, two further on its q G | e of token 2 g + s, row
+// A block's record (number cu_q[e] / 8 + e + its number in the portion, which no two share; else EACH e + its number among those) of
+// 25 DP + 128 floats, DP = d filled up to a multiple of 16 with zeros: [16 rows of DP: row 4 (a / 2) + a % 2 k G of token a, two further on its q G | e of token 2 g + s, row
 // 16 b + i: place (16 g + i) DP / 8 + 2 b + s | G_last | T and D T: place 2 (16 g + row) + s, row as above with T and D T for k G and q G, column
 // token 2 g + s].  Tokens past the end are zeros.
 #define DL_BLOCK 8
@@ -403,9 +403,9 @@ delta_walk_kernel(const T* __restrict__ fresh, int fresh_stride, const float* __
 template <typename T, int PER>
 __global__ void __launch_bounds__(4 * WAVE)
 delta_scan_kernel(const T* __restrict__ fresh, int fresh_stride, const float* __restrict__ z, const float* __restrict__ neg_rate,
-                  const T* __restrict__ beta_rows, int beta_stride, int beta_offset, float* __restrict__ state, size_t state_stride, const int* __restrict__ cu_q, const int* __restrict__ first_position,
-                  const int* __restrict__ state_slots, float* __restrict__ out, int heads, int groups, int d, int dv,
-                  float unit_eps) {
+                  const T* __restrict__ beta_rows, int beta_stride, int beta_offset, float* __restrict__ state, size_t state_stride,
+                  const int* __restrict__ cu_q, const int* __restrict__ first_position, const int* __restrict__ state_slots,
+                  float* __restrict__ out, int heads, int groups, int d, int dv, float unit_eps) {
   constexpr int DP = 16 * PER;                     // rows of S a workgroup's lanes cover (d filled up with zeros)
   constexpr int PIECES = (DL_GROUP * DP) / (4 * WAVE);       // (token, row) pairs a thread brings: PER
   __shared__ __attribute__((aligned(16))) float q_s[DL_GROUP][DP], k_s[DL_GROUP][DP], g_s[DL_GROUP][DP];

@@ -7,8 +7,10 @@
 // by line (`lines_to_rows` in common.h) and past the caches, which no later workgroup asks them from.  (Sixteen rows' half lines a load |
 // whole lines | whole lines past the caches, us for both products: 2 of 8 experts of 9,472 over 3,584, four rows, 197 | 177 | 160
 // (6.4 TB/s); 2 of 8 of 2,240 and a shared one of 4,480 over 1,536, three rows, 42.3 | 37.3 | 34.4; half lines past the caches 215 and
-// 44.8: each line then comes twice.  Weights that are in the caches already, a model far smaller than them: level to 5 % slower.)  An expert that every row uses besides (of an inner width of
-// its own) is one further expert in both grids, whose pairs are the rows; its K in the second product is cut into parts about
+// 44.8: each line then comes twice.  Weights that are in the last-level cache already, all of a model in less than its 256 MB, half lines | so,
+// one row, four and sixteen: 1,024 over 1,024 7.9 | 8.3, 11.3 | 11.7, 13.9 | 13.3; 3,648 over 896 14.8 | 14.0, 23.6 | 22.7, 32.4 | 32.4; 2,736
+// over 2,048 21.6 | 23.5, 31.9 | 30.6, 52.6 | 58.4.)  An expert that every row uses besides (of an inner width of its own) is one further
+// expert in both grids, whose pairs are the rows; its K in the second product is cut into parts about
 // as long as the others', each a slab of its own.
 #include "common.h"
 

@@ -327,7 +327,8 @@ gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, 
 // additions short; they and the eight waves' come together through LDS.  Bound by the weights' trip from memory: a wave
 // asks for its first two pairs of units at once and for the next pair before it multiplies the current one.
 // (Half lines through the caches | whole lines past them, four rows: 896 columns over 4,864 in eight parts of K 8.7 | 7.1 us, over 896 in two
-// 5.6 | 4.4, 1,536 over 8,960 34 | 26; sixteen rows: gate/up of 17,920 over 1,536 45 | 30, of 37,888 over 3,584 182 | 128.)
+// 5.6 | 4.4, 1,536 over 8,960 34 | 26; sixteen rows: gate/up of 17,920 over 1,536 45 | 30, of 37,888 over 3,584 182 | 128.  Weights that are in
+// the last-level cache already, all of a model in less than its 256 MB, four rows and sixteen: 768 columns over 3,072 12.0 | 10.5 and 14.3 | 13.3.)
 // LINES (K a multiple of 32): the weights come by whole cache lines, eight rows' a load (`lines_to_rows` in common.h), past the caches.
 // ROPE: the product is the joined q/k/v projection; a tile is eight elements of the first half of a head and the eight half a head further
 // on, which the half-split rotation pairs; bias, rotation and the store of keys and values into their pages follow in the epilogue.
@@ -491,7 +492,9 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 // weight the matrix instructions gain nothing, and this way more of the weights are on their way at once (figures at `vector_rows`).
 // UN: pieces of 256 floats a wave asks for at once (past the caches).  Four where the workgroups are no more than the compute units, one
 // where they are more, which hide each other's trips (one row, one piece | four: 896 columns over 896 4.7 | 4.1, over 4,864 14.3 | 12.5,
-// 3,584 over 18,944 55.3 | 51.3, but 4,608 over 3,584 13.5 | 16.7, 151,936 over 896, three rows 84 | 98).
+// 3,584 over 18,944 55.3 | 51.3, but 4,608 over 3,584 13.5 | 16.7, 151,936 over 896, three rows 84 | 98).  Past the caches, one row from memory
+// and from the last-level cache, us through them | past them: 768 columns over 3,072 9.7 | 8.3 and 6.9 | 8.0, over 768 4.0 | 3.4 and 3.3 | 3.4, 896
+// over 4,864 14.2 | 12.3 and 9.7 | 11.7: a model in less than the cache's 256 MB loses, which the kernel cannot know, and every other gains.
 template <int MR, bool VEC, bool GATED, int UN = 1>
 __global__ void __launch_bounds__(256)
 gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,

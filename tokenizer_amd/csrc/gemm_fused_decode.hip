@@ -67,8 +67,8 @@ __device__ __forceinline__ bf16x8 any8() {
 // The kernel takes its arguments one by one, those that every instance needs before its first load in the first
 // sixteen words of the argument block: the library is compiled so that these are in scalar registers when a wave
 // starts (`-amdgpu-kernarg-preload-count`; fourteen words in fact), and the products with the gated and the residual
-// epilogue then begin without any fetch of arguments (the bias, which only the epilogue needs, lies behind).  One pointer serves for the rows (bfloat16, or the float residual for the norm
-// prologue) and one for the result (bfloat16 rows, or the float residual that is added to), which never occur
+// epilogue then begin without any fetch of arguments (the bias, which only the epilogue needs, lies behind).  One
+// pointer serves for the rows (bfloat16, or the float residual for the norm prologue) and one for the result (bfloat16 rows, or the float residual that is added to), which never occur
 // together.  The rotation's own arguments lie behind; only wave 0, which writes the results, waits for them.
 //
 // LINES (K a multiple of 64): the weights come by whole cache lines (`lines_to_rows` in common.h), past the caches, which hold nothing
@@ -76,7 +76,9 @@ __device__ __forceinline__ bf16x8 any8() {
 // eight.  For walks of several trips; where all is asked for in one trip of four steps there is nothing to stream (896 columns level).
 // Us, sixteen rows' half lines a load | so, one input row and sixteen, weights from memory: gate/up 18,944 over 3,584 55.5 | 46.1
 // and 68.8 | 54.0, down 18,944 to 3,584 26.4 | 25.4 and 36.2 | 34.4, q/k/v of 3,584 13.8 | 11.3 and 16.1 | 12.3, gate/up 8,960 over 1,536
-// 17.8 | 17.0 and 22.6 | 18.1, down 8,960 to 1,536 11.2 | 9.7 and 15.2 | 14.2, down 4,864 to 896 6.4 | 5.8 and 9.2 | 8.7.
+// 17.8 | 17.0 and 22.6 | 18.1, down 8,960 to 1,536 11.2 | 9.7 and 15.2 | 14.2, down 4,864 to 896 6.4 | 5.8 and 9.2 | 8.7.  Weights that are in
+// the last-level cache already (all of a model in less than its 256 MB, the exception): gate/up 4,096 over 2,048 12.7 | 10.7 and 16.3 | 13.3,
+// 3,072 over 1,536 7.3 | 7.7 and 9.7 | 9.7, down 4,096 to 1,024 5.5 | 5.5 and 7.7 | 7.6, 8,192 to 2,048 8.9 | 9.6 and 14.2 | 13.7.
 template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES>
 __global__ void __launch_bounds__(NW * WAVE)
 fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const float* norm_weight,

@@ -416,9 +416,9 @@ extern "C" int ta_gemm_skinny_bf16(const void* A, int lda, const void* W, const 
 
 // The same product (not gated) with K cut into `splits` parts (at most; parts are multiples of 32, of 64 for up to sixteen rows and
 // K in whole lines, which are then always read as such, one block of columns a workgroup, whatever `ta_skinny_lines` and `col_blocks`
-// say: 8 rows x 1,536 over 8,960 12.2 -> 11.7 us, one row 11.0 -> 10.2) over the workgroups, the parts' float sums added afterwards in a fixed order.  partial: room for splits * M * N floats;
-// N % 4 == 0; M <= 64.  With C null (and more than one part after the rounding of the parts' length) the sums are
-// left in `partial` for a later kernel to add.
+// say: 8 rows x 1,536 over 8,960 12.2 -> 11.7 us, one row 11.0 -> 10.2) over the workgroups, the parts' float sums added afterwards in a
+// fixed order.  partial: room for splits * M * N floats; N % 4 == 0; M <= 64.  With C null (and more than one part after the rounding of
+// the parts' length) the sums are left in `partial` for a later kernel to add.
 extern "C" int ta_gemm_skinny_bf16_splitk(const void* A, int lda, const void* W, const void* bias, void* C, int ldc,
                                           void* partial, int M, int N, int K, int out_dtype, int splits,
                                           int col_blocks, hipStream_t stream) {

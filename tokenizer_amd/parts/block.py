@@ -119,7 +119,8 @@ class ScaledParallelBlock(Block):
         out = ScaledSum.of(ops, self.mixer.forward(h1, ctx, cache)).scaled_by(self.mixer_scale)
         if self.feed_forward is not None:
             # (Behind one or two terms of rows, a feed-forward that can leave its last product in parts may: the next norm adds
-            # them up in its kernel.)
+            # them up in its kernel.  Behind one the float sum is not rounded, on purpose: this layout has always kept it, and a
+            # router two layers on sees the difference.)
             run = self.feed_forward.forward
             if len(out.terms) <= 2:
                 run = getattr(self.feed_forward, "forward_pending", run)
