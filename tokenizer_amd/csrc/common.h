@@ -78,28 +78,54 @@ __device__ __forceinline__ int scalar_int(const int* p) {
 // sixteen lanes holds the same numbers, and four rotations within a row add up what lies 8, 4, 2 and 1 apart.  That is, bit for bit, the
 // order of six exchanges between lanes 32, 16, .. 1 apart, which went through the LDS crossbar one behind the other, a third of a
 // microsecond a sum.  (Rows first and then across them is another order: a router's near tie that it tips moves a token's logits.)
-__device__ __forceinline__ void wave_across_rows(float v, float& a, float& b, bool by32) {
-  const uint32_t bits = __float_as_uint(v);
-  const auto got = by32 ? __builtin_amdgcn_permlane32_swap(bits, bits, false, false) : __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+__device__ __forceinline__ void wave_swap32(float& a, float& b) {       // a's upper 32 lanes and b's lower 32 change places
+  const auto got = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(got[0]);
+  b = __uint_as_float(got[1]);
+}
+__device__ __forceinline__ void wave_swap16(float& a, float& b) {       // a's rows 1 and 3 of sixteen lanes and b's rows 0 and 2
+  const auto got = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   a = __uint_as_float(got[0]);
   b = __uint_as_float(got[1]);
 }
 #define WAVE_ROTATED(v, n) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 | (n), 0xF, 0xF, false))
-__device__ __forceinline__ float wave_sum(float v) {
-  float a, b;
-  wave_across_rows(v, a, b, true);
-  wave_across_rows(a + b, a, b, false);
-  v = a + b;
+__device__ __forceinline__ float wave_row_sum(float v) {
   v += WAVE_ROTATED(v, 8);
   v += WAVE_ROTATED(v, 4);
   v += WAVE_ROTATED(v, 2);
   return v + WAVE_ROTATED(v, 1);
 }
+__device__ __forceinline__ float wave_sum(float v) {
+  float b = v;
+  wave_swap32(v, b);
+  v += b;
+  b = v;
+  wave_swap16(v, b);
+  return wave_row_sum(v + b);
+}
+// Eight sums at once, each as `wave_sum` gives it: every exchange serves two.  Sum (lane & 1) + 2 ((lane >> 4) & 1) + 4 (lane >> 5).
+// (One by one by value: an array of which a lane picks an element is put into LDS, whose layout the kernel then asks the launch's packet
+// in host memory for, 13 us.)
+__device__ __forceinline__ float wave_pair32(float a, float b) {
+  wave_swap32(a, b);
+  return a + b;
+}
+__device__ __forceinline__ float wave_pair16(float a, float b) {
+  wave_swap16(a, b);
+  return wave_row_sum(a + b);
+}
+__device__ __forceinline__ float wave_sums8(const float (&v)[8], int lane) {
+  const float even = wave_pair16(wave_pair32(v[0], v[4]), wave_pair32(v[2], v[6]));
+  const float odd = wave_pair16(wave_pair32(v[1], v[5]), wave_pair32(v[3], v[7]));
+  return lane & 1 ? odd : even;
+}
 __device__ __forceinline__ float wave_max(float v) {
-  float a, b;
-  wave_across_rows(v, a, b, true);
-  wave_across_rows(fmaxf(a, b), a, b, false);
-  v = fmaxf(a, b);
+  float b = v;
+  wave_swap32(v, b);
+  v = fmaxf(v, b);
+  b = v;
+  wave_swap16(v, b);
+  v = fmaxf(v, b);
   v = fmaxf(v, WAVE_ROTATED(v, 8));
   v = fmaxf(v, WAVE_ROTATED(v, 4));
   v = fmaxf(v, WAVE_ROTATED(v, 2));

@@ -188,10 +188,10 @@ head_linear_mfma_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride, i
 
 // Few rows (single tokens): a wave owns one output column of one head for up to HS_ROWS rows and reads the column's
 // row of W once, sixteen bytes a lane a trip, so that the head's matrix streams from memory once whatever the rows.
-// GATED: row m's results, rounded, times sigmoid(gate[m gate_row + h gate_head + n gate_unit]).  The sums over the wave run in registers
-// (`wave_sum`), and a lane a row stores: eight sums through the LDS crossbar and a lane's eight stores one behind
-// the other were half of the kernel, and the gate a kernel of its own (four rows, 14 heads of 64 over 128: 5.0 + 5.0 us where they were
-// profiled, 3.6 so).
+// GATED: row m's results, rounded, times sigmoid(gate[m gate_row + h gate_head + n gate_unit]).  The eight sums over the wave share their
+// exchanges (`wave_sums8`), and a lane a row stores: eight sums through the LDS crossbar and a lane's eight stores one behind the other were
+// half of the kernel, and the gate a kernel of its own.  (Us, one, four and eight rows, 14 heads of 64 over 128: 2.4, 3.3 and 4.5 without the
+// gate; 2.3, 2.8 and 3.4 so, 2.6, 3.1 and 3.7 with it; each sum by itself 2.2, 2.9 and 3.7.)
 #define HS_ROWS 8
 template <bool GATED>
 __global__ void __launch_bounds__(256)
@@ -202,8 +202,9 @@ head_linear_skinny_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride,
   if (n >= N) return;
   const bf16_t* a = x + (size_t)h * x_stride + x_offset;
   const bf16_t* w = W + ((size_t)h * N + n) * K;
+  const int mine = m0 + (lane & 1) + 2 * ((lane >> 4) & 1) + 4 * (lane >> 5);         // the row whose sum ends in this lane
   bf16_t z = {0};
-  if (GATED) z = gate[(size_t)min(m0 + (lane & (HS_ROWS - 1)), M - 1) * gate_row + (size_t)h * gate_head + (size_t)n * gate_unit];
+  if (GATED) z = gate[(size_t)min(mine, M - 1) * gate_row + (size_t)h * gate_head + (size_t)n * gate_unit];
   float acc[HS_ROWS] = {};
   for (int k = lane * 8; k < K; k += 64 * 8) {
     const uint4 raw = *reinterpret_cast<const uint4*>(w + k);
@@ -220,16 +221,10 @@ head_linear_skinny_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride,
       }
     }
   }
-  float mine = 0.f;
-#pragma unroll
-  for (int i = 0; i < HS_ROWS; ++i) {
-    if (m0 + i >= M) break;
-    const float total = wave_sum(acc[i]);
-    if (lane == i) mine = total;
-  }
-  if (lane < HS_ROWS && m0 + lane < M) {
-    if (GATED) mine = bf16_bits_to_float(float_to_bf16_bits(mine)) / (1.0f + expf(-ld(&z)));
-    st(out + (size_t)(m0 + lane) * out_row + (size_t)h * out_stride + out_offset + n, mine);
+  float total = wave_sums8(acc, lane);
+  if ((lane & 15) < 2 && mine < M) {
+    if (GATED) total = bf16_bits_to_float(float_to_bf16_bits(total)) / (1.0f + expf(-ld(&z)));
+    st(out + (size_t)mine * out_row + (size_t)h * out_stride + out_offset + n, total);
   }
 }
 
