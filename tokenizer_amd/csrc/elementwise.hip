@@ -533,8 +533,10 @@ extern "C" int ta_add_terms_rmsnorm(void* residual, int count, const void* rows0
   const int status = launch_terms_vec(residual, terms, weight, eps, out, out_stride, weight2, eps2, out2, rows, n_rows, hidden,
                                       store_residual, SlabTerm{nullptr, nullptr, 0.f, 0, 0, 0}, dtype, stream);
   if (status != -2) return status;
-#define TERMS(TT, PP) add_terms_rmsnorm_kernel<TT, PP><<<n_rows, 256, 0, stream>>>((float*)residual, terms,     (const float*)weight, eps, (TT*)out, out_stride, (const float*)weight2, eps2, (TT*)out2, (const int*)rows, hidden, store_residual)
-#define TERMS_SIZES(TT) if (hidden <= 256) TERMS(TT, 1); else if (hidden <= 1024) TERMS(TT, 4); else if (hidden <= 2048) TERMS(TT, 8);                         else if (hidden <= 4096) TERMS(TT, 16); else TERMS(TT, 32)
+#define TERMS(TT, PP) add_terms_rmsnorm_kernel<TT, PP><<<n_rows, 256, 0, stream>>>((float*)residual, terms, (const float*)weight, eps, \
+    (TT*)out, out_stride, (const float*)weight2, eps2, (TT*)out2, (const int*)rows, hidden, store_residual)
+#define TERMS_SIZES(TT) if (hidden <= 256) TERMS(TT, 1); else if (hidden <= 1024) TERMS(TT, 4); else if (hidden <= 2048) TERMS(TT, 8); \
+                        else if (hidden <= 4096) TERMS(TT, 16); else TERMS(TT, 32)
   if (dtype == DT_F32) { TERMS_SIZES(float); } else { TERMS_SIZES(bf16_t); }
 #undef TERMS_SIZES
 #undef TERMS

@@ -151,20 +151,25 @@ class Ops:
         for name in ("ta_embedding", "ta_add_rmsnorm", "ta_silu_gate", "ta_rope_store",
                      "ta_paged_attention_generic", "ta_decode_attention_bf16", "ta_prefill_attention_bf16",
                      "ta_prefill_attention_shared_plan", "ta_prefill_attention_key_splits",
-                     "ta_gemm_f32", "ta_gemm_f32_parts", "ta_gemm_f32_qkv_rope", "ta_gemm_f32_silu_gate", "ta_paged_attention_f32", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
+                     "ta_gemm_f32", "ta_gemm_f32_parts", "ta_gemm_f32_qkv_rope", "ta_gemm_f32_silu_gate",
+                     "ta_paged_attention_f32", "ta_gemm_bf16", "ta_gemm_bf16_splitk", "ta_gemm_skinny_bf16",
                      "ta_gemm_skinny_bf16_splitk", "ta_gemm_skinny_qkv_rope", "ta_fused_norm_qkv_rope",
                      "ta_fused_norm_gated", "ta_fused_linear_residual", "ta_fused_qkv_rope", "ta_fused_gated",
                      "ta_splitk_reduce", "ta_splitk_add_rmsnorm", "ta_argmax", "ta_argmax_next_step", "ta_sample",
                      "ta_sample_workspace_words", "ta_library_gemm_bf16", "ta_compute_units", "ta_read_stream",
                      "ta_embedding_streams", "ta_streams_step", "ta_token_shift", "ta_mlstm_scan", "ta_mlstm_chunked", "ta_head_norm_gate",
                      "ta_capped_gate", "ta_norm_add_rmsnorm", "ta_norm_rotate_store", "ta_differential_heads",
-                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_gated_pays", "ta_gemm_ring_parts", "ta_gemm_ring_qkv", "ta_attention_merge_both", "ta_head_linear_gated", "ta_attention_merge_tiles", "ta_sigmoid_head_gate", "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows", "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
+                     "ta_gemm_ring", "ta_gemm_ring_gated", "ta_gemm_ring_gated_pays", "ta_gemm_ring_parts", "ta_gemm_ring_qkv",
+                     "ta_attention_merge_both", "ta_head_linear_gated", "ta_attention_merge_tiles", "ta_sigmoid_head_gate",
+                     "ta_route_top", "ta_expert_gate", "ta_side_gate", "ta_gelu_gate", "ta_norm_side_norm", "ta_route_rows",
+                     "ta_expert_slots", "ta_grouped_gemm_bf16", "ta_grouped_gemm_act", "ta_expert_combine",
                      "ta_add_pair_rmsnorm", "ta_latent_store", "ta_rotate_tails", "ta_head_linear", "ta_short_conv_silu",
                      "ta_delta_scan", "ta_route_sigmoid", "ta_route_rows_sigmoid", "ta_expert_act", "ta_relu2",
                      "ta_add_terms_rmsnorm", "ta_scale_cap", "ta_route_scores", "ta_selective_scan", "ta_route_rows_scores",
                      "ta_rotation_table", "ta_head_norm_rotate_store", "ta_group_norm_add", "ta_norm_add_parts", "ta_relu_gate",
                      "ta_talking_attention_generic", "ta_talking_decode_bf16", "ta_talking_prefill_bf16",
-                     "ta_talking_prefill_parts", "ta_retention_scan", "ta_retention_chunked", "ta_temper_store", "ta_add_slabs_rmsnorm", "ta_experts_few", "ta_experts_few_shared_parts",
+                     "ta_talking_prefill_parts", "ta_retention_scan", "ta_retention_chunked", "ta_temper_store",
+                     "ta_add_slabs_rmsnorm", "ta_experts_few", "ta_experts_few_shared_parts",
                      "ta_fused_qk_temper",
                      "ta_expert_gate_slots"):
             getattr(self.lib, name).restype = ctypes.c_int
@@ -780,7 +785,8 @@ class Ops:
         _need(token_ids.dtype == torch.int32 and token_ids.numel() == residual.shape[0], "token ids are int32 [T]")
         _need(rows is None or rows.dtype == torch.int32, "rows are int32")
         launch = lambda delta, parts: self.lib.ta_norm_side_norm(
-            _ptr(residual), _ptr(delta), parts, residual.shape[0], int(parts > 0 and whole.rounded), _ptr(post_weight), ctypes.c_float(post_eps), _ptr(gate), _ptr(proj),
+            _ptr(residual), _ptr(delta), parts, residual.shape[0], int(parts > 0 and whole.rounded), _ptr(post_weight),
+            ctypes.c_float(post_eps), _ptr(gate), _ptr(proj),
             proj.shape[1], _ptr(side_norm), ctypes.c_float(side_eps), _ptr(table), table.shape[1], _ptr(token_ids), offset, dim,
             _ptr(weight), ctypes.c_float(eps), _ptr(out), _ptr(rows), n_rows, hidden, int(rows is None), _code(out.dtype), self._stream())
         status = launch(delta, parts)
