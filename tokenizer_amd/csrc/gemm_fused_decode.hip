@@ -66,10 +66,19 @@ __device__ __forceinline__ bf16x8 any8() {
 //
 // The kernel takes its arguments one by one, those that every instance needs before its first load in the first
 // sixteen words of the argument block: the library is compiled so that these are in scalar registers when a wave
-// starts (`-amdgpu-kernarg-preload-count`; fourteen words in fact), and the products with the gated and the residual
-// epilogue then begin without any fetch of arguments (the bias, which only the epilogue needs, lies behind).  One
-// pointer serves for the rows (bfloat16, or the float residual for the norm prologue) and one for the result (bfloat16 rows, or the float residual that is added to), which never occur
-// together.  The rotation's own arguments lie behind; only wave 0, which writes the results, waits for them.
+// starts (`-amdgpu-kernarg-preload-count`; fourteen words in fact), and no instance begins with a fetch of arguments:
+// m, the rows a workgroup and the head size share a word (16 bits for the head size, which the launcher checks), the two numbers of heads another.
+// One pointer serves for the rows (bfloat16, or the float residual for the norm prologue) and one for the result (bfloat16 rows, or
+// the float residual that is added to), which never occur together.  The rest lies behind; only the waves of the epilogue wait for it,
+// with their weights under way.  Positions and slots come through the scalar unit there, so that the angles, which hang on the
+// position, are asked for without a wait among the vector loads (q/k/v of 896, one row, weights from memory: 4.4 -> 4.1 us).
+//
+// The epilogue is the tail that every launch waits for, and a wave's instructions one behind the other are its length: each of its
+// lanes has one output.  Wave v < ceil(M / 4) takes input rows 4 v .. 4 v + 3, sixteen lanes side by side the block's weight rows, so that a
+// store is one run of the result; a lane adds the NW partial sums of its output in the waves' order.  (Four outputs a lane of one wave,
+// four times the LDS reads, activations and stores behind each other, one row and eight: q/k/v of 896 5.0 -> 4.4 and 5.4 -> 5.0 us,
+// out 3.15 -> 2.8 and 3.5 -> 3.2, gate/up 4,864 over 896 6.8 -> 6.15 and 7.75 -> 7.15, down 5.6 -> 5.4 and 6.9 -> 6.7; a kernel that
+// does nothing is 1.65.)
 //
 // LINES (K a multiple of 64): the weights come by whole cache lines (`lines_to_rows` in common.h), past the caches, which hold nothing
 // that comes again: a pair of steps is one line of each of a block's sixteen rows, u even its lower eight rows, u odd its upper
@@ -81,12 +90,12 @@ __device__ __forceinline__ bf16x8 any8() {
 // 3,072 over 1,536 7.3 | 7.7 and 9.7 | 9.7, down 4,096 to 1,024 5.5 | 5.5 and 7.7 | 7.6, 8,192 to 2,048 8.9 | 9.6 and 14.2 | 13.7.
 template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES>
 __global__ void __launch_bounds__(NW * WAVE)
-fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const float* norm_weight,
-                    int m, int n, int k, int rows, int lda, float eps, const float* bias,
+fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weight, uint32_t m_rows_d, uint32_t heads,
+                    int n, int k, int lda, float eps, void* result, const float* bias,
                     const int* positions, const float* cos_sin, const int* slots, bf16_t* k_pages, bf16_t* v_pages,
-                    int n_q, int n_kv, int d, int page_size, float temper_coef, int temper_every) {
-  HELD(w, rows_in, result, norm_weight, m, n, k, rows, lda, eps);          // (the fourteen words that are there)
-  if constexpr (EPI == EPI_ROPE_STORE) HELD(n_q, n_kv, d, page_size);      // (where a tile's rows lie)
+                    int page_size, float temper_coef, int temper_every) {
+  HELD(w, rows_in, norm_weight, m_rows_d, heads, n, k, lda, eps, result);  // (the fourteen words that are there)
+  const int m = m_rows_d & 0xff, rows = (m_rows_d >> 8) & 0xff, d = m_rows_d >> 16, n_q = heads & 0xffff, n_kv = heads >> 16;
   FusedArgs p;
   // (Rows with a norm weight are the float residual; without one they are bfloat16, normalised already or plain.)
   p.a = norm_weight ? nullptr : (const bf16_t*)rows_in; p.lda = lda;
@@ -99,7 +108,8 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
   constexpr int SETS = (EPI == EPI_RESIDUAL) ? 1 : 2;
   constexpr int HELD = ONE ? PASSES : 1;                     // batches of weights held at once
   static_assert(EPI != EPI_ROPE_STORE || PASSES == 1, "the rotation pairs rows within one block");
-  __shared__ float red[NW][SETS * 4][WAVE];
+  constexpr int RS = WAVE + 4;                               // words between a lane's sums: the epilogue's reads touch every bank once
+  __shared__ float red[NW][SETS * 4][RS];
   extern __shared__ __attribute__((aligned(16))) uint16_t a_s[];   // NORM: the m normalised rows of K + 8 bfloat16
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int col = lane & 15, g = lane >> 4;
@@ -145,27 +155,10 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
   const int full_steps = K / 32;
   const int lds_stride = K + 8;
 
-  // The rotation's angles hang on the row's position: that chain starts before anything else is asked for (wave 0
-  // writes the results; lane (col, g) owns column m = col and rows 4g .. 4g+3 of each block).
-  float pre_cos[4] = {1.f, 1.f, 1.f, 1.f}, pre_sin[4] = {0.f, 0.f, 0.f, 0.f};
-  int pre_slot = -1;
-  if (EPI == EPI_ROPE_STORE && wave == 0) HELD(bias, positions, cos_sin, slots, k_pages, v_pages);
-  if (EPI == EPI_ROPE_STORE && wave == 0 && col < M && 4 * g < R) {
-    pre_slot = p.slots ? p.slots[col] : -1;
-    if (paired && p.cos_sin) {
-      const float* cs = p.cos_sin + (size_t)p.positions[col] * p.d + row0 % p.d + 4 * g;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pre_cos[r] = cs[r];
-        pre_sin[r] = cs[p.d / 2 + r];
-      }
-    } else if (temper_every > 0 && row0 < p.n_q * p.d) {      // the factor stands where a rotation's cosine would
-      const int steps = (p.positions[col] + 1) / temper_every;
-      const float factor = 1.f + temper_coef * logf((float)steps + 1.f);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pre_cos[r] = factor;
-    }
-  }
+  // The epilogue's lanes: weight row `er` of a block, input row `em`; `e_at` is where that output stands in a wave's part of `red`.
+  const int er = lane & 15, em = 4 * wave + (lane >> 4);
+  const bool e_wave = 4 * wave < M;
+  const int e_at = (er & 3) * RS + (er >> 2) * 16 + em;
 
   // Weight fragments come from HBM and take longest; the first batch is requested before the prologue.
   // Step j of a wave's batch: steps come in pairs (128 contiguous bytes of a weight row, one cache line),
@@ -220,31 +213,50 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
   }
 
   // What else the epilogue needs besides the sums is requested now as well, and not touched before the epilogue.
-  float pre_a[PASSES][4], pre_b[PASSES][4];                  // the old residual and the bias; or the two halves' bias
+  float pre_cos = 1.f, pre_sin = 0.f;
+  int pre_slot = -1;
+  if (EPI == EPI_ROPE_STORE && e_wave) {
+    HELD(bias, positions, cos_sin, slots, k_pages, v_pages);
+    const bool turned = p.cos_sin || temper_every > 0;
+    int position = 0;
 #pragma unroll
-  for (int ps = 0; ps < PASSES; ++ps)
+    for (int j = 0; j < 4; ++j) {
+      const int row = min(4 * wave + j, M - 1);
+      const int at = turned ? scalar_int(positions + row) : 0, slot = slots ? scalar_int(slots + row) : -1;
+      position = (lane >> 4) == j ? at : position;
+      pre_slot = (lane >> 4) == j ? slot : pre_slot;
+    }
+    if (em < M && er < R) {
+      if (paired && p.cos_sin) {
+        const float* cs = p.cos_sin + (size_t)position * p.d + row0 % p.d + er;
+        pre_cos = cs[0];
+        pre_sin = cs[p.d / 2];
+      } else if (temper_every > 0 && row0 < p.n_q * p.d) {    // the factor stands where a rotation's cosine would
+        pre_cos = 1.f + temper_coef * logf((float)((position + 1) / temper_every) + 1.f);
+      }
+    }
+  }
+  float pre_a[PASSES], pre_b[PASSES];                        // the old residual and the bias; or the two halves' bias
 #pragma unroll
-    for (int r = 0; r < 4; ++r) pre_a[ps][r] = pre_b[ps][r] = 0.f;
+  for (int ps = 0; ps < PASSES; ++ps) pre_a[ps] = pre_b[ps] = 0.f;
   // EPI_GATED with another activation than silu: its three numbers (alpha, limit, shift) lie where the rotation's table
   // would: g' = min(g, limit), u' = clamp(u, -limit, limit), g' sigmoid(alpha g') (u' + shift).
   float act_alpha = 1.f, act_limit = INFINITY, act_shift = 0.f;
   if (EPI == EPI_GATED && p.cos_sin) { act_alpha = p.cos_sin[0]; act_limit = p.cos_sin[1]; act_shift = p.cos_sin[2]; }
-  if (EPI == EPI_RESIDUAL && wave == 0) HELD(bias);
-  if (wave == 0 && col < M) {
+  if (EPI == EPI_RESIDUAL && e_wave) HELD(bias);
+  if (e_wave && em < M) {
     if (EPI == EPI_RESIDUAL) {
 #pragma unroll
-      for (int ps = 0; ps < PASSES; ++ps)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int local = 16 * ps + 4 * g + r, n = row0 + local;
-          if (local < R && n < p.n) {
-            pre_a[ps][r] = p.residual_out[(size_t)col * p.n + n];
-            if (p.bias) pre_b[ps][r] = p.bias[n];
-          }
+      for (int ps = 0; ps < PASSES; ++ps) {
+        const int local = 16 * ps + er, n = row0 + local;
+        if (local < R && n < p.n) {
+          pre_a[ps] = p.residual_out[(size_t)em * p.n + n];
+          if (p.bias) pre_b[ps] = p.bias[n];
         }
-    } else if (EPI == EPI_ROPE_STORE && 4 * g < R && p.bias) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) { pre_a[0][r] = p.bias[row0 + 4 * g + r]; pre_b[0][r] = p.bias[row1 + 4 * g + r]; }
+      }
+    } else if (EPI == EPI_ROPE_STORE && er < R && p.bias) {
+      pre_a[0] = p.bias[row0 + er];
+      pre_b[0] = p.bias[row1 + er];
     }
   }
 
@@ -414,73 +426,51 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, void* result, const fl
       if (SETS == 2)
         acc[SETS - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ok ? *reinterpret_cast<const bf16x8*>(w1[ps] + k) : fz8(), af, acc[SETS - 1], 0, 0, 0);
     }
-    if (ps > 0) __syncthreads();                             // wave 0 has read the block before
+    if (ps > 0) __syncthreads();                             // the block before has been read
 #pragma unroll
     for (int s = 0; s < SETS; ++s)
 #pragma unroll
       for (int r = 0; r < 4; ++r) red[wave][s * 4 + r][lane] = acc[s][r];
     __syncthreads();
-    // Lane (col, g) of wave 0: output column m = col, rows 4g .. 4g+3 of the block.
-    const int m = col;
-    if (wave == 0 && m < M && 16 * ps + 4 * g < R) {
-      float v0[4], v1[4];
+    const int local = 16 * ps + er;                          // the lane's row within the workgroup's
+    if (e_wave && em < M && local < R) {
+      float v0 = 0.f, v1 = 0.f;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-          s0 += red[w][r][lane];
-          if (SETS == 2) s1 += red[w][4 + r][lane];
-        }
-        v0[r] = s0;
-        v1[r] = s1;
+      for (int w = 0; w < NW; ++w) {
+        v0 += (&red[w][0][0])[e_at];
+        if (SETS == 2) v1 += (&red[w][(SETS - 1) * 4][0])[e_at];
       }
-      const int local = 16 * ps + 4 * g;                      // first of this lane's rows within the workgroup's
       if (EPI == EPI_RESIDUAL) {
         const int n = row0 + local;
-        float* dst = p.residual_out + (size_t)m * p.n + n;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (local + r < R && n + r < p.n) dst[r] = (pre_a[ps][r] + pre_b[ps][r]) + v0[r];   // old residual (+ bias) from the start
+        if (n < p.n) p.residual_out[(size_t)em * p.n + n] = (pre_a[ps] + pre_b[ps]) + v0;   // old residual (+ bias) from the start
       } else if (EPI == EPI_GATED) {
         const int n = row0 + local;
-        bf16_t* dst = p.out + (size_t)m * p.ldc + n;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (local + r < R && n + r < n_limit) {
-            if (p.cos_sin) {
-              const float gate = fminf(v0[r], act_limit), up = fminf(fmaxf(v1[r], -act_limit), act_limit);
-              st(dst + r, gate / (1.0f + __expf(-act_alpha * gate)) * (up + act_shift));
-            } else {
-              st(dst + r, v0[r] / (1.0f + __expf(-v0[r])) * v1[r]);
-            }
+        if (n < n_limit) {
+          bf16_t* dst = p.out + (size_t)em * p.ldc + n;
+          if (p.cos_sin) {
+            const float gate = fminf(v0, act_limit), up = fminf(fmaxf(v1, -act_limit), act_limit);
+            st(dst, gate / (1.0f + __expf(-act_alpha * gate)) * (up + act_shift));
+          } else {
+            st(dst, v0 / (1.0f + __expf(-v0)) * v1);
           }
+        }
       } else {
         const int d = p.d, half = d / 2;
         const int slot = pre_slot;
         const int page = slot >= 0 ? slot / p.page_size : 0, off = slot >= 0 ? slot % p.page_size : 0;
         if (paired) {
-          const int hd = row0 / d, i = row0 % d + 4 * g;            // element i (< half) of head hd, and i + half
-          float r1[4], r2[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float x1 = v0[r] + pre_a[0][r], x2 = v1[r] + pre_b[0][r];
-            r1[r] = x1 * pre_cos[r] - x2 * pre_sin[r];              // cos 1, sin 0 without a rotation
-            r2[r] = x2 * pre_cos[r] + x1 * pre_sin[r];
-          }
+          const int hd = row0 / d, i = row0 % d + er;               // element i (< half) of head hd, and i + half
+          const float x1 = v0 + pre_a[0], x2 = v1 + pre_b[0];
+          const float r1 = x1 * pre_cos - x2 * pre_sin;             // cos 1, sin 0 without a rotation
+          const float r2 = x2 * pre_cos + x1 * pre_sin;
           bf16_t* dst = nullptr;
-          if (hd < p.n_q) dst = p.out + (size_t)m * p.ldc + (size_t)hd * d + i;
+          if (hd < p.n_q) dst = p.out + (size_t)em * p.ldc + (size_t)hd * d + i;
           else if (slot >= 0) dst = p.k_pages + (((size_t)page * p.n_kv + (hd - p.n_q)) * p.page_size + off) * d + i;
-          if (dst) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) { st(dst + r, r1[r]); st(dst + half + r, r2[r]); }
-          }
+          if (dst) { st(dst, r1); st(dst + half, r2); }
         } else if (slot >= 0) {
-          const int e = row0 - (p.n_q + p.n_kv) * d + 4 * g;        // element of the joined value heads
+          const int e = row0 - (p.n_q + p.n_kv) * d + er;           // element of the joined value heads
           const int kvh = e / d, dd = e % d;
-          bf16_t* dst = p.v_pages + (((size_t)page * p.n_kv + kvh) * d + dd) * p.page_size + off;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) st(dst + (size_t)r * p.page_size, v0[r] + pre_a[0][r]);
+          st(p.v_pages + (((size_t)page * p.n_kv + kvh) * d + dd) * p.page_size + off, v0 + pre_a[0]);
         }
       }
     }
@@ -502,11 +492,12 @@ static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
   const bool from_residual = args.residual_in != nullptr;
   if (from_residual != (args.norm_weight != nullptr) || (!from_residual && !args.a) || !args.w) return -1;
   if (EPI == EPI_RESIDUAL ? !args.residual_out : !args.out) return -1;
+  if (args.d > 0xffff || args.n_q > 0xffff || args.n_kv > 0xffff) return -1;   // (what the packed arguments hold)
   fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES><<<tiles, NW * WAVE, lds, stream>>>(
-      args.w, from_residual ? (const void*)args.residual_in : (const void*)args.a,
-      EPI == EPI_RESIDUAL ? (void*)args.residual_out : (void*)args.out, args.norm_weight, args.m, args.n,
-      args.k, args.rows, args.lda, args.eps, args.bias, args.positions, args.cos_sin, args.slots, args.k_pages, args.v_pages,
-      args.n_q, args.n_kv, args.d, args.page_size, args.temper_coef, args.temper_every);
+      args.w, from_residual ? (const void*)args.residual_in : (const void*)args.a, args.norm_weight,
+      (uint32_t)args.m | (uint32_t)args.rows << 8 | (uint32_t)args.d << 16, (uint32_t)args.n_q | (uint32_t)args.n_kv << 16, args.n, args.k,
+      args.lda, args.eps, EPI == EPI_RESIDUAL ? (void*)args.residual_out : (void*)args.out, args.bias, args.positions, args.cos_sin,
+      args.slots, args.k_pages, args.v_pages, args.page_size, args.temper_coef, args.temper_every);
   return LAUNCH_STATUS();
 }
 
