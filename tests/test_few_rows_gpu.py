@@ -364,6 +364,22 @@ def test_weights_by_whole_lines(ops, rows, n, k):
     near(residual, want)
 
 
+# Rows that a wave brings through its own part of LDS: one load and as many as eight rows take, nine rows beside them (straight from
+# memory), a K of less than a wave's first line, with a last step of 32, with a tail of eight, and shares of 4, 8 and 10 steps; rows
+# with a stride of their own and what lies beyond K in them no number.
+@pytest.mark.parametrize("rows", [1, 2, 3, 5, 6, 8, 9])
+@pytest.mark.parametrize("n,k", [(20, 8), (20, 40), (896, 480), (896, 896), (100, 1352), (1536, 1536), (900, 4064), (896, 4864), (52, 5000)])
+def test_rows_staged_by_their_waves(ops, rows, n, k):
+    x = torch.full((rows, k + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    x[:, :k] = rand_bf16((rows, k), 21)
+    w = (rand_bf16((n, k), 22).float() * 0.05).to(torch.bfloat16)
+    bias, residual = torch.randn(n, device="cuda"), torch.randn(rows, n, device="cuda")
+    want = residual.double() + bias.double() + x[:, :k].double() @ w.double().t()
+    ops.linear_add(x[:, :k], w, bias, residual)
+    # (float sums of K terms of up to about 0.2: each of fewer than 2^13 roundings is of a partial sum no larger than about 32)
+    assert float((residual.double() - want).abs().max()) <= 1e-4
+
+
 @pytest.mark.parametrize("rows", [1, 16])
 @pytest.mark.parametrize("k", [2112, 3584])
 def test_qkv_by_whole_lines(ops, rows, k):

@@ -88,7 +88,14 @@ __device__ __forceinline__ bf16x8 any8() {
 // 17.8 | 17.0 and 22.6 | 18.1, down 8,960 to 1,536 11.2 | 9.7 and 15.2 | 14.2, down 4,864 to 896 6.4 | 5.8 and 9.2 | 8.7.  Weights that are in
 // the last-level cache already (all of a model in less than its 256 MB, the exception): gate/up 4,096 over 2,048 12.7 | 10.7 and 16.3 | 13.3,
 // 3,072 over 1,536 7.3 | 7.7 and 9.7 | 9.7, down 4,096 to 1,024 5.5 | 5.5 and 7.7 | 7.6, 8,192 to 2,048 8.9 | 9.6 and 14.2 | 13.7.
-template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES>
+//
+// STAGE (up to eight rows from memory, a share of K in one trip): a wave brings its lines of all rows in STAGE loads of sixteen
+// different bytes a lane and turns them into fragments through a part of LDS that is its own, without a barrier.  A fragment loaded
+// straight from memory is one of UN loads whose lanes mostly ask for the same bytes, and such a load holds up the memory pipeline
+// like any other: a workgroup's weights and rows, down 4,864 to 896, were 80 loads of the one and 160 of the other.  Us, direct |
+// staged, one row and eight: down 4,864 to 896 5.4 | 4.55 and 6.7 | 5.4, out 896 to 896 2.8 | 2.75 and 3.2 | 2.9 (weights alone 3.3 and 2.0).
+// With more than eight rows a staged share is as many loads as the fragments are.
+template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES, int STAGE>
 __global__ void __launch_bounds__(NW * WAVE)
 fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weight, uint32_t m_rows_d, uint32_t heads,
                     int n, int k, int lda, float eps, void* result, const float* bias,
@@ -110,7 +117,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   static_assert(EPI != EPI_ROPE_STORE || PASSES == 1, "the rotation pairs rows within one block");
   constexpr int RS = WAVE + 4;                               // words between a lane's sums: the epilogue's reads touch every bank once
   __shared__ float red[NW][SETS * 4][RS];
-  extern __shared__ __attribute__((aligned(16))) uint16_t a_s[];   // NORM: the m normalised rows of K + 8 bfloat16
+  extern __shared__ __attribute__((aligned(16))) uint16_t a_s[];   // NORM: the m normalised rows of K + 8 bfloat16; STAGE: the waves' pieces
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int col = lane & 15, g = lane >> 4;
   const int M = p.m, K = p.k, R = p.rows;
@@ -204,7 +211,18 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   auto a_inside = [&](int base_pair, int u) { return base_pair + (u >> 1) * NW < pairs; };
   const bf16_t* ar = NORM ? nullptr : p.a + (size_t)a_m * p.lda + 8 * g;
   bf16x8 af_one[ONE ? UN : 1];
-  if (ONE && !NORM) {                                      // the rows' fragments as well
+  // STAGE: piece i of the wave's M * PIECES pieces of sixteen bytes is piece i % PIECES of row i / PIECES.
+  constexpr int PIECES = UN * 4, ROW_BYTES = PIECES * 16 + 16;  // (sixteen bytes on, so that the rows of a fragment lie in different banks)
+  char* mine = reinterpret_cast<char*>(a_s) + (STAGE > 0 ? (size_t)wave * M * ROW_BYTES : 0);
+  word4 staged[STAGE > 0 ? STAGE : 1];
+  if constexpr (STAGE > 0) {
+#pragma unroll
+    for (int j = 0; j < STAGE; ++j) {
+      const int i = min(j * WAVE + lane, M * PIECES - 1), piece = i % PIECES;
+      const int k = min((wave + (piece >> 3) * NW) * 64 + 8 * (piece & 7), K - 8);   // (what lies past the end of K is not used)
+      staged[j] = *reinterpret_cast<const word4*>(p.a + (size_t)(i / PIECES) * p.lda + k);
+    }
+  } else if (ONE && !NORM) {                               // the rows' fragments as well
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       // (every lane: a row past the end repeats the last one and only feeds columns that are never stored)
@@ -319,6 +337,15 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
       }
     }
     __syncthreads();
+  }
+  if constexpr (STAGE > 0) {
+#pragma unroll
+    for (int j = 0; j < STAGE; ++j) {
+      const int i = min(j * WAVE + lane, M * PIECES - 1);
+      *reinterpret_cast<word4*>(mine + i / PIECES * ROW_BYTES + i % PIECES * 16) = staged[j];
+    }
+#pragma unroll
+    for (int u = 0; u < UN; ++u) af_one[u] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const word4*>(mine + a_m * ROW_BYTES + u * 64 + 16 * g));
   }
   const uint16_t* as_row = a_s + (size_t)a_m * lds_stride + 8 * g;
   auto load_a = [&](int k) -> bf16x8 {
@@ -477,14 +504,24 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   }
 }
 
-template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES = false>
+template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES = false, int STAGE = 0>
 static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
-  size_t lds = NORM ? (size_t)args.m * (args.k + 8) * sizeof(uint16_t) : 0;
+  if constexpr (ONE && !NORM && STAGE == 0) {
+    constexpr int MOST = UN / 2;                             // loads for eight rows of UN / 2 lines
+    const int loads = (args.m * UN * 4 + WAVE - 1) / WAVE;
+    if (args.m <= 8 && args.k >= 8) {
+      if (loads <= 1) return launch_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, 1>(args, tiles, stream);
+      if (loads <= 2) return launch_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, 2>(args, tiles, stream);
+      if (MOST > 2 && loads <= 3) return launch_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, MOST < 3 ? MOST : 3>(args, tiles, stream);
+      return launch_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, MOST>(args, tiles, stream);
+    }
+  }
+  size_t lds = NORM ? (size_t)args.m * (args.k + 8) * sizeof(uint16_t) : (size_t)(STAGE > 0 ? NW * args.m * (UN * 64 + 16) : 0);
   if (lds > 48 * 1024) {
     // More dynamic LDS than the default limit: ask for it (the device has 160 KB per compute unit).
     if (lds > 140 * 1024) return -1;
     hipError_t err = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES>),
+        reinterpret_cast<const void*>(&fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, STAGE>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) return (int)err;
   }
@@ -493,7 +530,7 @@ static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
   if (from_residual != (args.norm_weight != nullptr) || (!from_residual && !args.a) || !args.w) return -1;
   if (EPI == EPI_RESIDUAL ? !args.residual_out : !args.out) return -1;
   if (args.d > 0xffff || args.n_q > 0xffff || args.n_kv > 0xffff) return -1;   // (what the packed arguments hold)
-  fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES><<<tiles, NW * WAVE, lds, stream>>>(
+  fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, STAGE><<<tiles, NW * WAVE, lds, stream>>>(
       args.w, from_residual ? (const void*)args.residual_in : (const void*)args.a, args.norm_weight,
       (uint32_t)args.m | (uint32_t)args.rows << 8 | (uint32_t)args.d << 16, (uint32_t)args.n_q | (uint32_t)args.n_kv << 16, args.n, args.k,
       args.lda, args.eps, EPI == EPI_RESIDUAL ? (void*)args.residual_out : (void*)args.out, args.bias, args.positions, args.cos_sin,
