@@ -469,16 +469,16 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
       }
       if (EPI == EPI_RESIDUAL) {
         const int n = row0 + local;
-        if (n < p.n) p.residual_out[(size_t)em * p.n + n] = (pre_a[ps] + pre_b[ps]) + v0;   // old residual (+ bias) from the start
+        if (n < p.n) st_through(p.residual_out + (size_t)em * p.n + n, (pre_a[ps] + pre_b[ps]) + v0);   // old residual (+ bias) from the start
       } else if (EPI == EPI_GATED) {
         const int n = row0 + local;
         if (n < n_limit) {
           bf16_t* dst = p.out + (size_t)em * p.ldc + n;
           if (p.cos_sin) {
             const float gate = fminf(v0, act_limit), up = fminf(fmaxf(v1, -act_limit), act_limit);
-            st(dst, gate / (1.0f + __expf(-act_alpha * gate)) * (up + act_shift));
+            st_through(dst, gate / (1.0f + __expf(-act_alpha * gate)) * (up + act_shift));
           } else {
-            st(dst, v0 / (1.0f + __expf(-v0)) * v1);
+            st_through(dst, v0 / (1.0f + __expf(-v0)) * v1);
           }
         }
       } else {
@@ -493,11 +493,11 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
           bf16_t* dst = nullptr;
           if (hd < p.n_q) dst = p.out + (size_t)em * p.ldc + (size_t)hd * d + i;
           else if (slot >= 0) dst = p.k_pages + (((size_t)page * p.n_kv + (hd - p.n_q)) * p.page_size + off) * d + i;
-          if (dst) { st(dst, r1); st(dst + half, r2); }
+          if (dst) { st_through(dst, r1); st_through(dst + half, r2); }
         } else if (slot >= 0) {
           const int e = row0 - (p.n_q + p.n_kv) * d + er;           // element of the joined value heads
           const int kvh = e / d, dd = e % d;
-          st(p.v_pages + (((size_t)page * p.n_kv + kvh) * d + dd) * p.page_size + off, v0 + pre_a[0]);
+          st_through(p.v_pages + (((size_t)page * p.n_kv + kvh) * d + dd) * p.page_size + off, v0 + pre_a[0]);
         }
       }
     }
