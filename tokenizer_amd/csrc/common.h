@@ -35,6 +35,10 @@ __device__ __forceinline__ void st_through(float* p, float v) {
 __device__ __forceinline__ void st_through(bf16_t* p, float v) {
   __hip_atomic_store(&p->bits, float_to_bf16_bits(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void st_through(uint2* p, uint2 v) {          // (eight bytes, at a multiple of eight)
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v.x | (unsigned long long)v.y << 32, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // The index of a thread's wave within its workgroup, as a scalar: conditions built from it are uniform
 // branches.  Matrix instructions run whatever the lane mask says, so a matrix instruction must never sit
@@ -143,6 +147,29 @@ __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, WAVE_ROTATED(v, 4));
   v = fmaxf(v, WAVE_ROTATED(v, 2));
   return fmaxf(v, WAVE_ROTATED(v, 1));
+}
+// The largest of values that come again every N lanes (N a power of two up to sixteen).
+template <int N>
+__device__ __forceinline__ float wave_max_repeated(float v) {
+  if constexpr (N > 8) v = fmaxf(v, WAVE_ROTATED(v, 8));
+  if constexpr (N > 4) v = fmaxf(v, WAVE_ROTATED(v, 4));
+  if constexpr (N > 2) v = fmaxf(v, WAVE_ROTATED(v, 2));
+  if constexpr (N > 1) v = fmaxf(v, WAVE_ROTATED(v, 1));
+  return v;
+}
+// A lane's value added to, or the larger of it and, that of the lane SHIFT (16 or 32) away: two swapped registers hold the two in some
+// order.  What an exchange through the LDS crossbar gives, bit for bit, without its 0.05 us.
+template <int SHIFT>
+__device__ __forceinline__ float wave_add_across(float v) {
+  float b = v;
+  if constexpr (SHIFT == 16) wave_swap16(v, b); else wave_swap32(v, b);
+  return v + b;
+}
+template <int SHIFT>
+__device__ __forceinline__ float wave_max_across(float v) {
+  float b = v;
+  if constexpr (SHIFT == 16) wave_swap16(v, b); else wave_swap32(v, b);
+  return fmaxf(v, b);
 }
 #undef WAVE_ROTATED
 
