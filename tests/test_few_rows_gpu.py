@@ -380,6 +380,26 @@ def test_rows_staged_by_their_waves(ops, rows, n, k):
     assert float((residual.double() - want).abs().max()) <= 1e-4
 
 
+# Workgroups of four, seven, nine and sixteen weight rows with a last one that is not full; K below a step, with a tail, of one trip and
+# of several, by steps and by lines; rows that are staged in one load and in as many as eight rows take, and that come straight from
+# memory; rows of a longer stride with no numbers beyond K; the gate with few and with many columns.
+@pytest.mark.parametrize("rows", [1, 3, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(8, 8), (20, 40), (900, 904), (1544, 2112), (2060, 1536), (900, 4864), (1100, 6720), (4100, 904), (16400, 1536)])
+def test_products_of_few_rows_spread_over_the_device(ops, rows, n, k):
+    x = torch.full((rows, k + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    x[:, :k] = rand_bf16((rows, k), 31)
+    w = (rand_bf16((2 * n, k), 32).float() * 0.05).to(torch.bfloat16)
+    bias = torch.randn(n, device="cuda")
+    exact = x[:, :k].double() @ w.double().t()
+    got = ops.linear(x[:, :k], w[:n], bias, out_dtype=torch.float32)
+    # (float sums of K terms of up to about 0.2: each of fewer than 2^13 roundings is of a partial sum no larger than about 32)
+    assert float((got.double() - exact[:, :n] - bias.double()).abs().max()) <= 1e-4
+    gate = exact[:, :n]
+    want = gate / (1 + torch.exp(-gate)) * exact[:, n:]
+    got = ops.linear_silu_gate(x[:, :k], w)
+    assert float((got.double() - want).abs().max()) <= 2 ** -8 * max(1.0, float(want.abs().max()))     # (one rounding to bfloat16)
+
+
 @pytest.mark.parametrize("rows", [1, 16])
 @pytest.mark.parametrize("k", [2112, 3584])
 def test_qkv_by_whole_lines(ops, rows, k):

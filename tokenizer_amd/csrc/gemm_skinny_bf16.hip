@@ -294,6 +294,253 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
   }
 }
 
+// Up to sixteen rows: the same product with what a launch of that size is bound by taken out.
+// * A workgroup has R <= 16 weight rows, so that a small matrix is spread over all compute units (896 columns are 224 workgroups of
+//   four, not 56 of sixteen); lanes whose weight row is past R load nothing and only feed results that are never stored.  UPPER: R > 8 (LINES).
+// * The epilogue is the tail that the launch waits for: a lane has one output, which it adds up in the waves' order; wave v < ceil(M / 4)
+//   takes rows 4 v .. 4 v + 3, sixteen lanes the block's weight rows.  The bias is on its way beside the first weights.
+// * STAGE > 0 (up to eight rows): a wave brings a trip's share of the rows in STAGE loads of sixteen different bytes a lane and turns
+//   them into fragments through a part of LDS that is its own; a fragment straight from memory is a load that holds up the memory
+//   pipeline like any other though its lanes mostly ask for the same bytes.
+// Which wave takes which steps of K does not hang on any of this, nor does a result.
+// Us, weights from memory, sixteen rows a workgroup with four outputs a lane | so, one row, eight and sixteen: 896 over 896 3.5 | 3.0, 3.9 | 3.2
+// and 4.15 | 3.6; 896 over 4,864 8.1 | 5.7, 9.7 | 5.8 and 11.2 | 8.3; 1,536 over 1,536 4.5 | 3.6, 5.1 | 3.8 and 5.6 | 4.6; 1,536 over 8,960 12.6 | 9.3,
+// 15.5 | 9.4 and 18.3 | 14.2; 3,584 over 3,584 7.2 | 6.8, 8.5 | 7.5 and 9.4 | 8.7; 3,584 over 18,944 24.6 | 23.0, 30.1 | 25.0 and 35.7 | 33.8; gate/up
+// 4,864 over 896 7.3 | 6.4, 7.7 | 7.0 and 8.1 | 7.25, 8,960 over 1,536 14.9 | 12.7, 15.9 | 13.9 and 17.3 | 15.6.  (A kernel that does nothing: 1.65.)
+template <int NW, bool GATED, typename OutT, int LINES, bool WHOLE, int SUMS, bool UPPER, int STAGE>
+__global__ void __launch_bounds__(NW * WAVE)
+few_rows_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ bias,
+                     float* __restrict__ partial, int lda, int k_chunk, uint32_t m_rows, int N, int K_all, int gate_act,
+                     OutT* __restrict__ C, int ldc) {
+  HELD(A, W, bias, partial, lda, k_chunk, m_rows, N, K_all, gate_act);   // (the fourteen words that are there)
+  static_assert(SUMS == 1 || (SUMS == 2 && LINES > 0 && WHOLE), "two sums a wave: whole lines, a sum for each half");
+  constexpr int SETS = GATED ? 2 : 1, TRIP = LINES > 0 ? LINES : 4;      // lines, or steps of 32, a trip
+  constexpr int PIECES = TRIP * (LINES > 0 ? 8 : 4), ROW_BYTES = PIECES * 16 + 16;
+  __shared__ float red[NW * SUMS][SETS * 4][WAVE];
+  extern __shared__ __attribute__((aligned(16))) char rows_s[];
+  const int M = m_rows & 0xff, R = m_rows >> 8;
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int col = lane & 15, g = lane >> 4;
+  const int n_out = GATED ? N / 2 : N;
+  const int n_first = blockIdx.x * R;
+  const int k_lo = blockIdx.y * k_chunk;
+  const int K = min(K_all, k_lo + k_chunk) - k_lo;                // this workgroup's part of K
+  const bool a_ok = col < M;
+  const int a_m = min(col, M - 1);
+  const bf16_t* a_row = A + (size_t)a_m * lda + k_lo;
+  // The lane of the epilogue: weight row `er` of the block, row `em` (and, with two waves, the row eight further on).
+  const int er = lane & 15, em = 4 * wave + (lane >> 4), n = n_first + er;
+  const bool e_wave = 4 * wave < M;
+  float bias_here;
+  asm volatile("" : "=v"(bias_here));                             // (whatever it holds: only read where it was loaded)
+  const bool biased = bias && !partial;
+  if (e_wave && biased) bias_here = bias[min(n, n_out - 1)];
+  // STAGE: piece i of the M * PIECES of a trip is piece i % PIECES of row i / PIECES.
+  char* mine = rows_s + (STAGE > 0 ? (size_t)wave * M * ROW_BYTES : 0);
+  word4 staged[STAGE > 0 ? STAGE : 1];
+  int stage_k[STAGE > 0 ? STAGE : 1];
+  auto stage_ask = [&](int first) {                               // `first`: the wave's first line, or step, of the trip
+#pragma unroll
+    for (int j = 0; j < STAGE; ++j) {
+      const int i = min(j * WAVE + lane, M * PIECES - 1), piece = i % PIECES;
+      stage_k[j] = LINES > 0 ? (first + (piece >> 3) * NW) * 64 + 8 * (piece & 7) : (first + (piece >> 2) * NW) * 32 + 8 * (piece & 3);
+      staged[j] = *reinterpret_cast<const word4*>(A + (size_t)(i / PIECES) * lda + k_lo + min(stage_k[j], K - 8));
+    }
+  };
+  auto stage_put = [&]() {                                        // (past the end of K: zeros)
+#pragma unroll
+    for (int j = 0; j < STAGE; ++j) {
+      const int i = min(j * WAVE + lane, M * PIECES - 1);
+      if (stage_k[j] >= K) staged[j] = (word4){0u, 0u, 0u, 0u};
+      *reinterpret_cast<word4*>(mine + i / PIECES * ROW_BYTES + i % PIECES * 16) = staged[j];
+    }
+  };
+  auto fragment = [&](int byte) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const word4*>(mine + a_m * ROW_BYTES + byte)); };
+
+  floatx4 sums[SUMS][SETS];
+#pragma unroll
+  for (int i = 0; i < SUMS; ++i)
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) sums[i][s] = (floatx4){0.f, 0.f, 0.f, 0.f};
+
+  if constexpr (LINES > 0) {
+    constexpr int HH = UPPER ? 2 : 1;
+    const int sub = col & 7, piece = SUMS == 2 ? g + 4 * (col >> 3) : 2 * g + (col >> 3);
+    const int a_first = SUMS == 2 ? 8 * g : 16 * g, a_apart = SUMS == 2 ? 32 : 8;    // the rows' elements of the line that meet the weights'
+    const bf16_t* wl[SETS][HH];
+    bool w_ok[HH];
+#pragma unroll
+    for (int hh = 0; hh < HH; ++hh) {
+      w_ok[hh] = 8 * hh + sub < R && n_first + 8 * hh + sub < n_out;
+#pragma unroll
+      for (int s = 0; s < SETS; ++s)
+        wl[s][hh] = W + (size_t)(min(n_first + 8 * hh + sub, n_out - 1) + s * n_out) * K_all + k_lo + 8 * piece;
+    }
+    const int pairs = (K + 63) / 64;                        // lines of a row; the last may be short
+    for (int first = wave; first < pairs; first += LINES * NW) {
+      word4 wf[LINES][SETS][HH];
+      bf16x8 af[LINES][2];
+#pragma unroll
+      for (int q = 0; q < LINES; ++q) {
+        const int pair = first + q * NW;
+        const bool valid = pair < pairs;
+        const int at = min(pair, pairs - 1) * 64;
+        const bool inside = valid && (WHOLE || at + 8 * piece < K);      // this lane's sixteen bytes lie inside K
+#pragma unroll
+        for (int s = 0; s < SETS; ++s)
+#pragma unroll
+          for (int hh = 0; hh < HH; ++hh) {
+            wf[q][s][hh] = (word4){0u, 0u, 0u, 0u};
+            if (inside && w_ok[hh]) wf[q][s][hh] = __builtin_nontemporal_load(reinterpret_cast<const word4*>(wl[s][hh] + at));
+          }
+        if constexpr (STAGE == 0) {
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh) {
+            const int place = at + a_first + hh * a_apart;
+            af[q][hh] = load8(a_row + place, valid && a_ok && (WHOLE || place < K));
+          }
+        }
+      }
+      if constexpr (STAGE > 0) {
+        stage_ask(first);
+        stage_put();
+#pragma unroll
+        for (int q = 0; q < LINES; ++q)
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh) af[q][hh] = fragment(q * 128 + 2 * (a_first + hh * a_apart));
+      }
+#pragma unroll
+      for (int q = 0; q < LINES; ++q) {
+#pragma unroll
+        for (int s = 0; s < SETS; ++s) {
+          bf16x8 b0, b1;
+          lines_to_rows(wf[q][s][0], wf[q][s][HH - 1], col < 8, b0, b1);
+          sums[0][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, af[q][0], sums[0][s], 0, 0, 0);
+          sums[SUMS - 1][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, af[q][1], sums[SUMS - 1][s], 0, 0, 0);
+        }
+      }
+    }
+  } else {
+    const bool w_ok = col < R && n_first + col < n_out;
+    const bf16_t* wp[SETS];
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) wp[s] = W + (size_t)(min(n_first + col, n_out - 1) + s * n_out) * K_all + k_lo + 8 * g;
+    const int full_steps = K / 32;
+    // A wave's last trip may reach past the end of K: such steps load nothing and multiply zeros (no matrix instruction sits
+    // behind a condition).
+    for (int ks = wave; ks < full_steps; ks += TRIP * NW) {
+      bf16x8 wf[TRIP][SETS], af[TRIP];
+#pragma unroll
+      for (int u = 0; u < TRIP; ++u) {
+        const int step = ks + u * NW;
+        const bool valid = step < full_steps;
+        const int k = min(step, full_steps - 1) * 32;
+#pragma unroll
+        for (int s = 0; s < SETS; ++s) wf[u][s] = load8(wp[s] + k, valid && w_ok);
+        if constexpr (STAGE == 0) af[u] = load8(a_row + k + 8 * g, valid && a_ok);
+      }
+      if constexpr (STAGE > 0) {
+        stage_ask(ks);
+        stage_put();
+#pragma unroll
+        for (int u = 0; u < TRIP; ++u) {
+          af[u] = fragment(u * 64 + 16 * g);
+          if (ks + u * NW >= full_steps) af[u] = load8(nullptr, false);   // (the tail of K has weights of its own)
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < TRIP; ++u)
+#pragma unroll
+        for (int s = 0; s < SETS; ++s) sums[0][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][s], af[u], sums[0][s], 0, 0, 0);
+    }
+    if (K & 31) {
+      // The tail of K (a multiple of 8), zero-filled, is one wave's; the others multiply zeros, so that no matrix
+      // instruction sits behind a condition on the wave (it would run whatever a lane mask says).
+      const int k = full_steps * 32;
+      const bool k_ok = wave == full_steps % NW && k + 8 * g < K;
+      const bf16x8 af = load8(a_row + k + 8 * g, k_ok && a_ok);
+#pragma unroll
+      for (int s = 0; s < SETS; ++s)
+        sums[0][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(wp[s] + k, k_ok && w_ok), af, sums[0][s], 0, 0, 0);
+    }
+  }
+  // (A register's lanes are turned by four for every register before it, so that the epilogue's reads touch every bank once.)
+#pragma unroll
+  for (int i = 0; i < SUMS; ++i)
+#pragma unroll
+    for (int s = 0; s < SETS; ++s)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave * SUMS + i][s * 4 + r][(lane + 4 * r) & 63] = sums[i][s][r];
+  __syncthreads();
+  if (!e_wave || er >= R || n >= n_out) return;
+#pragma unroll
+  for (int at_m = 0; at_m < 16; at_m += 4 * NW) {
+    const int m = em + at_m;
+    if (m >= M) return;
+    const int at = (er & 3) * WAVE + (((er >> 2) * 16 + m + 4 * (er & 3)) & 63);
+    float v = 0.f, up = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW * SUMS; ++w) {
+      v += (&red[w][0][0])[at];
+      if (GATED) up += (&red[w][(SETS - 1) * 4][0])[at];
+    }
+    if (biased) v += bias_here;
+    // gate_act 1: the tanh form of GELU in place of silu; 2: max(z, 0).
+    if (GATED)
+      v = gate_act == 2 ? fmaxf(v, 0.f) * up
+          : gate_act == 1 ? 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v))) * up
+                          : v / (1.0f + __expf(-v)) * up;
+    if (partial) st_through(partial + ((size_t)blockIdx.y * M + m) * n_out + n, v);         // (never GATED)
+    else st_through(C + (size_t)m * ldc + n, v);
+  }
+}
+
+// Weight rows a workgroup: sixteen where their workgroups are as many as compute units, fewer (four at least) where they are not.
+static int few_rows_a_workgroup(int n_out, int splits) {
+  const int units = compute_units();
+  if ((long)((n_out + 15) / 16) * splits >= units) return 16;
+  const int rows = (int)(((long)n_out * splits + units - 1) / units);
+  return rows < 4 ? 4 : rows > 16 ? 16 : rows;
+}
+
+template <int NW, bool GATED, typename OutT, int LINES, bool WHOLE, int SUMS, bool UPPER, int STAGE>
+static int launch_few_kernel(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int M, int N, int K, int k_chunk,
+                             int rows, dim3 grid, float* slabs, int gate_act, hipStream_t stream) {
+  constexpr int PIECES = (LINES > 0 ? LINES * 8 : 16);
+  const size_t lds = STAGE > 0 ? (size_t)NW * M * (PIECES * 16 + 16) : 0;
+  auto kernel = few_rows_gemm_kernel<NW, GATED, OutT, LINES, WHOLE, SUMS, UPPER, STAGE>;
+  if (lds > 24 * 1024) {                                     // (beside up to 32 KB of its own)
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (err != hipSuccess) return (int)err;
+  }
+  kernel<<<grid, NW * WAVE, lds, stream>>>((const bf16_t*)A, (const bf16_t*)W, (const float*)bias, slabs, lda, k_chunk,
+                                           (uint32_t)M | (uint32_t)rows << 8, N, K, gate_act, (OutT*)C, ldc);
+  return LAUNCH_STATUS();
+}
+
+template <int NW, bool GATED, int LINES = 0, bool WHOLE = false, int SUMS = 1, bool UPPER = true>
+static int launch_few(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int M, int N, int K, int out_dtype,
+                      hipStream_t stream, int splits = 1, void* partial = nullptr, int gate_act = 0) {
+  const int n_out = GATED ? N / 2 : N;
+  const int step = LINES > 0 ? 64 : 32;
+  const int k_chunk = splits > 1 ? ((K + splits - 1) / splits + step - 1) / step * step : K;
+  if (splits > 1) splits = (K + k_chunk - 1) / k_chunk;          // no part without a step of its own
+  const int rows = few_rows_a_workgroup(n_out, splits);
+  if (!UPPER && rows > 8) return -1;
+  const dim3 grid((n_out + rows - 1) / rows, splits);
+  float* slabs = splits > 1 ? (float*)partial : nullptr;
+  constexpr int PIECES = (LINES > 0 ? LINES * 8 : 16), MOST = (8 * PIECES + WAVE - 1) / WAVE;
+  int status;
+#define RUN(T, ST) launch_few_kernel<NW, GATED, T, LINES, WHOLE, SUMS, UPPER, ST>(A, lda, W, bias, C, ldc, M, N, K, k_chunk, rows, grid, \
+                                                                                 slabs, gate_act, stream)
+#define PICK(T) status = M > 8 || K < 8 ? RUN(T, 0) : M * PIECES <= WAVE ? RUN(T, 1) : RUN(T, MOST)
+  if (out_dtype == DT_F32) PICK(float); else PICK(bf16_t);
+#undef PICK
+#undef RUN
+  if (status == 0 && splits > 1 && C) status = launch_splitk_reduce(slabs, bias, C, M, N, ldc, splits, out_dtype, stream);
+  return status;
+}
+
 // Column blocks per workgroup, by the launcher's choice (`asked` 0) or the caller's (1 or 2): two once there are
 // more than 32 rows and the workgroups still fill the device.
 static int column_blocks(int asked, int M, int n_out, int splits) {
@@ -378,21 +625,35 @@ static int pick_waves(const void* A, int lda, const void* W, const void* bias, v
     const int lines = K / 64;
     if (g_lines && (K & 63) == 0 && lines > 2 * waves && (waves != 8 || tiles > compute_units() || (!GATED && M > 4 && K > 4096))) {
       const int up = waves == 8 && tiles <= compute_units() ? 3 : lines_a_trip(GATED, waves, M, K);
-#define GO(NWV, L) return launch_skinny<1, NWV, GATED, 1, L, true, 2>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act)
+#define GO(NWV, L) return launch_few<NWV, GATED, L, true, 2>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act)
+#define HALF(L) return launch_few<8, false, L, true, 2, false>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act)
 #define TRIPS(NWV) if (up == 1) GO(NWV, 1); if (up == 2) GO(NWV, 2); if constexpr (!GATED && NWV > 2) { if (up == 3) GO(NWV, 3); } \
                    if constexpr (!GATED && NWV == 8) { if (up == 4) GO(NWV, 4); } if constexpr (NWV == 4) { if (up == 6) GO(NWV, 6); }
+      if constexpr (!GATED) {
+        // Up to eight weight rows a workgroup: a line of them is one load, so a trip has more lines.
+        if (waves == 16 && few_rows_a_workgroup(N, 1) <= 8) {
+          const int share = (lines + 7) / 8, trips = M > 8 ? (share + 3) / 4 : (share + 9) / 10, each = (share + trips - 1) / trips;
+          if (each <= 4) HALF(4);
+          if (each <= 6) HALF(6);
+          if (each <= 8) HALF(8);
+          HALF(10);
+        }
+      }
       if (waves == 4) { TRIPS(2) }
       if (waves == 8) { TRIPS(4) }
       if (waves == 16) { TRIPS(8) }
 #undef TRIPS
+#undef HALF
 #undef GO
     }
+    if (waves == 4) return launch_few<4, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
+    if (waves == 8) return launch_few<8, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
+    return launch_few<16, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
+  } else {
+    if (waves == 4) return launch_skinny<MB, 4, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
+    if (waves == 8) return launch_skinny<MB, 8, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
+    return launch_skinny<MB, 16, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
   }
-  if (waves == 4)
-    return launch_skinny<MB, 4, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
-  if (waves == 8)
-    return launch_skinny<MB, 8, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
-  return launch_skinny<MB, 16, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
 }
 
 // M <= 64; K, lda multiples of 8; pointers 16-byte aligned; with `gated` N is even and C is [M, N/2]
@@ -426,11 +687,11 @@ extern "C" int ta_gemm_skinny_bf16_splitk(const void* A, int lda, const void* W,
   if (M > 64 || (K & 7) || (lda & 7) || (N & 3) || splits < 1 || (splits > 1 && !partial)) return -1;
   const bool whole = M <= 16 && (K & 63) == 0;
   if (!C && parts_of_k(K, splits, whole ? 64 : 32) < 2) return -1;
-  if (whole) return launch_skinny<1, 8, false, 1, 1, true>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, splits, partial);
+  if (whole) return launch_few<8, false, 1, true>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, splits, partial);
 #define GO(MBV, NBV) launch_skinny<MBV, 8, false, NBV>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, splits, partial)
   const bool two = column_blocks(col_blocks, M, N, parts_of_k(K, splits, 32)) == 2;
   switch ((M + 15) / 16) {
-    case 1: return GO(1, 1);
+    case 1: return launch_few<8, false>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, splits, partial);
     case 2: return GO(2, 1);
     case 3: return two ? GO(3, 2) : GO(3, 1);
     default: return two ? GO(4, 2) : GO(4, 1);
