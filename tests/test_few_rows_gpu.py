@@ -380,6 +380,40 @@ def test_rows_staged_by_their_waves(ops, rows, n, k):
     assert float((residual.double() - want).abs().max()) <= 1e-4
 
 
+# Choices counted in registers (up to 64 experts) and searched for (more): ties, scores of minus infinity (with too few others to pick),
+# a logit that is no number, groups of one and of many; the logits form, whose kernels search, is the reference.
+@pytest.mark.parametrize("experts,groups,keep,top", [(8, 0, 0, 2), (8, 4, 2, 2), (8, 8, 3, 3), (1, 0, 0, 1), (64, 8, 2, 7), (60, 4, 1, 15), (64, 0, 0, 64), (72, 8, 2, 5)])
+@pytest.mark.parametrize("softmax", [False, True])
+def test_choice_counted_is_choice_searched(ops, experts, groups, keep, top, softmax):
+    rows, width = 5, 64
+    x, router = torch.zeros((rows, width), dtype=torch.bfloat16), torch.zeros((experts, width), dtype=torch.bfloat16)
+    x[:, :rows] = torch.eye(rows)
+    router[:, 0] = rand_bf16((experts,), 41).cpu()
+    router[:, 1] = torch.arange(experts) % 3                                    # ties
+    router[:, 2] = torch.where(torch.arange(experts) < 1, 1.0, -3e38)           # all but one weigh nothing
+    router[:, 3] = -torch.arange(experts) / 64
+    x[4, 0], router[0, 4] = 1.0, float("nan") if experts > 1 else 0.0           # (its product with every row that has it is no number)
+    x, router = x.cuda(), router.cuda()
+    logits = (x.cpu().double() @ torch.nan_to_num(router.cpu().double(), nan=0.0).t()).float().cuda()
+    finite = slice(0, 4)
+    for correction in (None, torch.randn(experts, generator=torch.Generator().manual_seed(42)).cuda().round(decimals=1)):
+        got = torch.full((rows, top), -1, dtype=torch.int32, device="cuda"), torch.full((rows, top), -1.0, device="cuda")
+        want = torch.full((rows, top), -1, dtype=torch.int32, device="cuda"), torch.full((rows, top), -1.0, device="cuda")
+        more = dict(softmax=softmax, group_max=False)
+        clean = torch.nan_to_num(router, nan=0.0)
+        assert ops.route_rows_scores(x[finite].contiguous(), clean, correction, experts, groups, keep, got[0][finite], got[1][finite], **more)
+        ops.route_scores(logits[finite].contiguous(), correction, experts, groups, keep, want[0][finite], want[1][finite], **more)
+        assert torch.equal(got[0][finite], want[0][finite])
+        assert torch.allclose(got[1][finite], want[1][finite], rtol=1e-6 * experts, atol=0, equal_nan=True)    # (sums in another order)
+        assert ops.route_rows_scores(x, router, correction, experts, groups, keep, *got, **more)               # a logit that is no number
+        assert bool(((got[0] >= 0) & (got[0] < experts)).all())
+    if not groups and experts <= 64:
+        assert ops.route_rows(x[finite].contiguous(), torch.nan_to_num(router, nan=0.0), got[0][finite], got[1][finite])
+        ops.route_top(logits[finite].contiguous(), want[0][finite], want[1][finite])
+        assert torch.equal(got[0][finite], want[0][finite])
+        assert torch.allclose(got[1][finite], want[1][finite], rtol=1e-6 * experts, atol=0, equal_nan=True)
+
+
 # Workgroups of four, seven, nine and sixteen weight rows with a last one that is not full; K below a step, with a tail, of one trip and
 # of several, by steps and by lines; rows that are staged in one load and in as many as eight rows take, and that come straight from
 # memory; rows of a longer stride with no numbers beyond K; the gate with few and with many columns.

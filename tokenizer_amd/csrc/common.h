@@ -32,6 +32,9 @@ __device__ __forceinline__ void st(bf16_t* p, float v) { p->bits = float_to_bf16
 __device__ __forceinline__ void st_through(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void st_through(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void st_through(bf16_t* p, float v) {
   __hip_atomic_store(&p->bits, float_to_bf16_bits(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -64,13 +64,12 @@ __device__ __forceinline__ uint4 rt_pack8(const float (&v)[8]) {
 template <typename T> struct RtVec;
 template <> struct RtVec<bf16_t> {
   static constexpr int N = 8;
-  __device__ static __forceinline__ void load(const bf16_t* p, float (&v)[8]) { rt_unpack8(*reinterpret_cast<const uint4*>(p), v); }
+  __device__ static __forceinline__ void unpack(const uint4 raw, float (&v)[8]) { rt_unpack8(raw, v); }
 };
 template <> struct RtVec<float> {
   static constexpr int N = 4;
-  __device__ static __forceinline__ void load(const float* p, float (&v)[4]) {
-    const float4 raw = *reinterpret_cast<const float4*>(p);
-    v[0] = raw.x; v[1] = raw.y; v[2] = raw.z; v[3] = raw.w;
+  __device__ static __forceinline__ void unpack(const uint4 raw, float (&v)[4]) {
+    v[0] = __uint_as_float(raw.x); v[1] = __uint_as_float(raw.y); v[2] = __uint_as_float(raw.z); v[3] = __uint_as_float(raw.w);
   }
 };
 
@@ -87,10 +86,14 @@ __device__ __forceinline__ void rt_row_sums(const T* __restrict__ row, const T* 
     for (int e = wave; e < count; e += WAVES) put(e, 0.f);
     return;
   }
-  float xv[PIECES][N], wv[PIECES][N];
-  auto ask = [&](const T* from, float (&v)[PIECES][N]) {
+  uint4 xv[PIECES], wv[PIECES];
+  auto ask = [&](const T* from, uint4 (&v)[PIECES]) {
 #pragma unroll
-    for (int p = 0; p < PIECES; ++p) RtVec<T>::load(from + min((p * WAVE + lane) * N, hidden - N), v[p]);
+    for (int p = 0; p < PIECES; ++p) v[p] = *reinterpret_cast<const uint4*>(from + min((p * WAVE + lane) * N, hidden - N));
+  };
+  auto inside = [&](int p, const uint4 raw, float (&v)[N]) {        // (nothing is past the end of pieces that are full)
+    const bool in = (p * WAVE + lane) * N < hidden;
+    RtVec<T>::unpack(make_uint4(in ? raw.x : 0u, in ? raw.y : 0u, in ? raw.z : 0u, in ? raw.w : 0u), v);
   };
   ask(row, xv);
   if (AHEAD) ask(router + (size_t)wave * hidden, wv);
@@ -99,19 +102,44 @@ __device__ __forceinline__ void rt_row_sums(const T* __restrict__ row, const T* 
     if (!AHEAD) ask(router + (size_t)e * hidden, wv);
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
-      const bool in = (p * WAVE + lane) * N < hidden;
+      float x[N], w[N];
+      inside(p, xv[p], x);
+      inside(p, wv[p], w);
 #pragma unroll
-      for (int k = 0; k < N; ++k) sum = fmaf(in ? wv[p][k] : 0.f, in ? xv[p][k] : 0.f, sum);
+      for (int k = 0; k < N; ++k) sum = fmaf(w[k], x[k], sum);
     }
     if (AHEAD && e + WAVES < count) ask(router + (size_t)(e + WAVES) * hidden, wv);
     put(e, wave_sum(sum));
   }
 }
 
+__device__ __forceinline__ float rt_lane(float v, int lane) {          // (`lane` the same for the whole wave)
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+
+// A lane's place among the wave's first `count` values, one a lane: how many are larger, or as large and of a lower lane.  For values
+// that are numbers that is the order in which a search for the largest one after the other finds them.
+__device__ __forceinline__ int rt_place(float mine, int lane, int count) {
+  int ahead = 0;
+  for (int o = 0; o < count; ++o) {
+    const float v = rt_lane(mine, o);
+    ahead += (v > mine || (v == mine && o < lane)) ? 1 : 0;
+  }
+  return ahead;
+}
+
+// The `top` first of those places: `value` of each, added up in their order.
+__device__ __forceinline__ float rt_sum_in_order(float value, int place, int top) {
+  float total = 0.f;
+  for (int k = 0; k < top; ++k) total += rt_lane(value, (int)__builtin_ctzll(__ballot(place == k)));
+  return total;
+}
+
 // The router's product and the choice in one kernel, a workgroup a token: x [n_tokens, hidden] (row stride lda) and
 // router [n_experts, hidden] of type T in pieces of sixteen bytes; wave w forms the logits of experts w, w + WAVES, ... as
 // float sums, wave 0 then picks as route_top_kernel does.  (Three rows of 1,536 and 8 experts: 5.5 us with four waves and loads
-// behind branches, 4.4 with a wave an expert.)
+// behind branches, 4.4 with a wave an expert; in a graph and with places
+// counted in place of searches through LDS 3.7 -> 2.6, four rows of 3,584 4.6 -> 3.4.)
 template <typename T, int PIECES, int WAVES>
 __global__ void __launch_bounds__(WAVES * WAVE)
 route_rows_kernel(const T* __restrict__ x, int lda, const T* __restrict__ router, int hidden, int n_experts, int top,
@@ -123,6 +151,20 @@ route_rows_kernel(const T* __restrict__ x, int lda, const T* __restrict__ router
                                 [&](int e, float sum) { if (lane == 0) logit_s[e] = sum; });
   __syncthreads();
   if (wave != 0) return;
+  if (n_experts <= WAVE) {
+    // An expert a lane: its place among them all is counted, not searched for (a search is twelve exchanges through LDS a pick).
+    const float z = lane < n_experts ? logit_s[lane] : -INFINITY;
+    if (__ballot(z != z) == 0) {                             // (what is no number has no place: those rows search)
+      const int place = lane < n_experts ? rt_place(z, lane, n_experts) : n_experts;
+      const float term = expf(z - rt_lane(z, (int)__builtin_ctzll(__ballot(place == 0))));
+      const float sum = rt_sum_in_order(term, place, top);
+      if (place < top) {
+        st_through(chosen + (size_t)t * top + place, lane);
+        st_through(weights + (size_t)t * top + place, term / sum);
+      }
+      return;
+    }
+  }
   float top_value = 0.f, total = 0.f, mine = 0.f, last_value = INFINITY;
   int last = -1;
   for (int k = 0; k < top; ++k) {
@@ -548,47 +590,92 @@ route_scores_kernel(const float* __restrict__ logits, int stride, const float* _
 // The router's product and the choice in one kernel, a token a workgroup (few rows: a decode step): as route_rows_kernel
 // forms the logits (float sums of the row with each expert's router row, the row kept in registers), then all
 // waves choose together and the first stores.  (Three rows of 896 and 8 experts in 4 groups: 6.8 us with four waves and loads
-// behind branches, 5.7 with a wave an expert.)
+// behind branches, 5.7 with a wave an expert; in a graph, with the correction on its
+// way beside the rows and places counted in registers, four rows of 896 5.05 -> 3.5, of 3,584 6.2 -> 4.5.)
+enum : uint32_t { RS_SOFTMAX = 0x100, RS_GROUP_MAX = 0x200, RS_RAW = 0x400 };     // beside `top`, which is 64 at most
 template <typename T, int PIECES, int WAVES>
 __global__ void __launch_bounds__(WAVES * WAVE)
 route_rows_sigmoid_kernel(const T* __restrict__ x, int lda, const T* __restrict__ router, const float* __restrict__ correction,
-                          int hidden, int n_experts, int n_groups, int keep, int top, int* __restrict__ chosen,
-                          float* __restrict__ weights, int softmax = 0, int group_max = 0, float* __restrict__ gate = nullptr,
-                          int raw = 0) {
+                          int hidden, int n_experts, uint32_t groups_keep, uint32_t top_kind, int* __restrict__ chosen,
+                          float* __restrict__ weights, float* __restrict__ gate) {
+  HELD(x, lda, router, correction, hidden, n_experts, groups_keep, top_kind, chosen);
   extern __shared__ float rs_scratch[];
   float* choice = rs_scratch;
   float* score = choice + n_experts;
   float* worth = score + n_experts;
+  const int n_groups = groups_keep & 0xffff, keep = groups_keep >> 16, top = top_kind & 0xff;
+  const bool softmax = top_kind & RS_SOFTMAX, group_max = top_kind & RS_GROUP_MAX, raw = top_kind & RS_RAW;
   const int t = blockIdx.x;
-  const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+  const int lane = threadIdx.x & (WAVE - 1), wave = wave_index();
+  const bool few = n_experts <= WAVE;
+  float correct = 0.f;                                       // (asked for beside the rows: behind the logits it is a trip of its own)
+  if (few && correction) correct = correction[min(lane, n_experts - 1)];
   // (With a gate, the router has one row more: the gate's, behind the experts'.)
   rt_row_sums<T, PIECES, WAVES, WAVES == 8>(x + (size_t)t * lda, router, hidden, n_experts + (gate ? 1 : 0), [&](int e, float sum) {
     if (lane != 0) return;
-    if (e == n_experts) {
-      gate[t] = 1.0f / (1.0f + expf(-sum));
-    } else if (softmax) {
-      score[e] = sum;                                        // the logit, until all of them are there
-    } else {
-      const float s = 1.0f / (1.0f + expf(-sum));
-      score[e] = s;
-      choice[e] = correction ? s + correction[e] : (n_groups > 0 ? s : sum);
-    }
+    if (e == n_experts) st_through(gate + t, 1.0f / (1.0f + expf(-sum)));
+    else score[e] = sum;                                     // the logit, until all of them are there
   });
   __syncthreads();
-  if (softmax) {                                             // every thread sums the few logits up for itself
-    float top_logit = -INFINITY, total = 0.f;
+  if (few) {
+    // An expert a lane, every score, worth and place in registers: searches for the largest are exchanges through LDS one behind
+    // the other.  Every step gives what the searches below give, in their order of sums.
+    const float z = lane < n_experts ? score[lane] : -INFINITY;
+    float s;
+    if (softmax) {
+      const float top_logit = wave_max(z), term = expf(z - top_logit);
+      float total = 0.f;
+      for (int e = 0; e < n_experts; ++e) total += rt_lane(term, e);
+      s = term / total;
+    } else {
+      s = 1.0f / (1.0f + expf(-z));
+    }
+    float pick = lane >= n_experts ? -INFINITY : correction ? s + correct : (n_groups > 0 ? s : z);
+    if (__ballot(pick != pick || z != z) == 0) {             // (what is no number has no place: those rows search)
+      if (n_groups > 0) {
+        const int per = n_experts / n_groups;
+        int group = 0;
+        for (int o = per; o < n_experts; o += per) group += lane >= o ? 1 : 0;
+        float first = -INFINITY, second = -INFINITY;
+        for (int o = 0, at = 0, g = 0; o < n_experts; ++o) {
+          const float v = rt_lane(pick, o);
+          const bool mine = g == group;
+          second = mine ? (v > first ? first : fmaxf(second, v)) : second;
+          first = mine ? fmaxf(first, v) : first;
+          if (++at == per) { at = 0; ++g; }
+        }
+        const float value = (per > 1 && !group_max) ? first + second : first;
+        int ahead = 0;
+        for (int g = 0; g < n_groups; ++g) {
+          const float v = rt_lane(value, g * per);
+          ahead += (v > value || (v == value && g < group)) ? 1 : 0;
+        }
+        if (ahead >= keep) pick = -INFINITY;
+      }
+      const int place = lane < n_experts ? rt_place(pick, lane, n_experts) : n_experts;
+      const float total = rt_sum_in_order(s, place, top);
+      if (wave == 0 && place < top) {
+        st_through(chosen + (size_t)t * top + place, lane);
+        st_through(weights + (size_t)t * top + place, raw ? s : s / (total + 1e-20f));
+      }
+      return;                                                // (all waves alike: the scores are the same for all)
+    }
+  }
+  // Every thread sums the few logits up for itself.
+  float top_logit = -INFINITY, total = 0.f;
+  if (softmax) {
     for (int e = 0; e < n_experts; ++e) top_logit = fmaxf(top_logit, score[e]);
     for (int e = 0; e < n_experts; ++e) total += expf(score[e] - top_logit);
-    __syncthreads();
-    for (int e = threadIdx.x; e < n_experts; e += WAVES * WAVE) {
-      const float z = score[e], s = expf(z - top_logit) / total;
-      score[e] = s;
-      choice[e] = correction ? s + correction[e] : (n_groups > 0 ? s : z);
-    }
-    __syncthreads();
   }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n_experts; e += WAVES * WAVE) {
+    const float z = score[e], s = softmax ? expf(z - top_logit) / total : 1.0f / (1.0f + expf(-z));
+    score[e] = s;
+    choice[e] = correction ? s + correction[e] : (n_groups > 0 ? s : z);
+  }
+  __syncthreads();
   rs_choose(choice, score, worth, lane, n_experts, n_groups, keep, top, wave == 0, chosen + (size_t)t * top,
-            weights + (size_t)t * top, group_max != 0, raw == 0);
+            weights + (size_t)t * top, group_max, !raw);
 }
 
 // up: [n_tokens, n_experts * inner]; out: [n_tokens, columns], columns >= n_experts * inner:
@@ -695,8 +782,9 @@ extern "C" int ta_route_rows_scores(const void* x, int lda, const void* router, 
     return -2;
   const size_t lds = (size_t)(2 * n_experts + n_groups) * sizeof(float);
 #define ROUTE(TT, PP, WW) route_rows_sigmoid_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, lds, stream>>>((const TT*)x, lda, \
-    (const TT*)router, (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights, softmax, \
-    group_max, (float*)gate, raw)
+    (const TT*)router, (const float*)correction, hidden, n_experts, (uint32_t)n_groups | (uint32_t)(n_groups > 0 ? keep : 0) << 16, \
+    (uint32_t)top | (softmax ? RS_SOFTMAX : 0u) | (group_max ? RS_GROUP_MAX : 0u) | (raw ? RS_RAW : 0u), (int*)chosen, (float*)weights, \
+    (float*)gate)
   RT_INSTANCES(ROUTE);
 #undef ROUTE
   return LAUNCH_STATUS();
@@ -715,7 +803,8 @@ extern "C" int ta_route_rows_sigmoid(const void* x, int lda, const void* router,
     return -2;
   const size_t lds = (size_t)(2 * n_experts + n_groups) * sizeof(float);
 #define ROUTE(TT, PP, WW) route_rows_sigmoid_kernel<TT, PP, WW><<<n_tokens, WW * WAVE, lds, stream>>>((const TT*)x, lda, \
-    (const TT*)router, (const float*)correction, hidden, n_experts, n_groups, keep, top, (int*)chosen, (float*)weights)
+    (const TT*)router, (const float*)correction, hidden, n_experts, (uint32_t)n_groups | (uint32_t)(n_groups > 0 ? keep : 0) << 16, \
+    (uint32_t)top, (int*)chosen, (float*)weights, nullptr)
   RT_INSTANCES(ROUTE);
 #undef ROUTE
   return LAUNCH_STATUS();
