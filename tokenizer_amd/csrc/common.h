@@ -93,6 +93,12 @@ __device__ __forceinline__ int scalar_int(const int* p) {
   return *(constant_int)(p);
 }
 
+// A float that is the same for the whole wave and that no kernel in flight writes, the same way.
+__device__ __forceinline__ float scalar_float(const float* p) {
+  typedef const float __attribute__((address_space(4))) * constant_float;
+  return *(constant_float)(p);
+}
+
 // The sum and the largest over a wave whose 64 lanes are all active, in every lane, without LDS: lanes 32 and 16 apart change places
 // (`v_permlane32_swap`, `v_permlane16_swap`; both halves of a swap added are the same whichever came first), after which every row of
 // sixteen lanes holds the same numbers, and four rotations within a row add up what lies 8, 4, 2 and 1 apart.  That is, bit for bit, the

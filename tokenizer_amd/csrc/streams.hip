@@ -170,6 +170,86 @@ streams_step_kernel(float* __restrict__ streams, const TY* __restrict__ y, const
   }
 }
 
+// The same for up to four streams of up to 1,024 columns and few rows, a thread a column.  Everything is asked for at the start: the
+// coefficients, the gain and the token's slot through the scalar unit (they are the same for a workgroup: sums take them from scalar
+// registers, nothing passes through LDS but the squares' sum), the rows as they come, looked at where they are used; a lane past
+// the last column has the last one's and stores nothing.  (Four rows of 896 in four streams, in a graph: 3.3 us with coefficients in LDS, loads
+// behind conditions and the gain behind the sum, 2.8 so.)
+template <typename TY, typename TO, bool SHIFT, int S>
+__global__ void __launch_bounds__(1024)
+streams_step_column_kernel(float* __restrict__ streams, const TY* __restrict__ y, const float* __restrict__ mix,
+                           const float* __restrict__ out_coef, const float* __restrict__ read, const float* __restrict__ gain,
+                           int width, float eps, const int* __restrict__ rows, const float* __restrict__ scale, TO* __restrict__ out,
+                           const float* __restrict__ mu, float* __restrict__ state, const int* __restrict__ entry_of_token,
+                           const int* __restrict__ state_slots, const int* __restrict__ positions) {
+  HELD(streams, y, mix, out_coef, read, gain, width, eps);
+  __shared__ float scratch[16];
+  const int i = blockIdx.x;
+  const int lane = threadIdx.x & (WAVE - 1), wave = wave_index(), n_waves = blockDim.x / WAVE;
+  const bool in = (int)threadIdx.x < width;
+  const int c = min((int)threadIdx.x, width - 1);
+  const int r = rows ? scalar_int(rows + i) : i;
+  float* x = streams + (size_t)r * S * width + c;
+  float old[S], m[S][S], write[S], take[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) old[s] = x[(size_t)s * width];
+  TY add_raw = {};
+  float scale_c = 1.f, before = 0.f, mu_c = 0.f;
+  if (y) add_raw = y[(size_t)r * width + c];
+  if (scale) scale_c = scale[c];
+  int slot = -1;
+  bool first = false;
+  if constexpr (SHIFT) {
+    mu_c = mu[c];
+    const int e = scalar_int(entry_of_token + r);
+    slot = e >= 0 ? scalar_int(state_slots + max(e, 0)) : -1;
+    first = scalar_int(positions + r) == 0;
+    before = state[(size_t)max(slot, 0) * width + c];        // (a row that only fills the batch up has slot 0's, which it does not use)
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s) take[s] = scalar_float(read + s);
+  if (y) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      write[s] = scalar_float(out_coef + s);
+#pragma unroll
+      for (int to = 0; to < S; ++to) m[s][to] = scalar_float(mix + s * S + to);
+    }
+  }
+  const float g = scalar_float(gain);
+  float u = 0.f;
+  if (!y) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) u = fmaf(take[s], old[s], u);
+  } else {
+    const float add = scale ? ld(&add_raw) * scale_c : ld(&add_raw) * 1.0f;
+#pragma unroll
+    for (int to = 0; to < S; ++to) {
+      float v = 0.f;
+#pragma unroll
+      for (int s = 0; s < S; ++s) v = fmaf(m[s][to], old[s], v);
+      v = fmaf(write[to], add, v);
+      if (!rows && in) x[(size_t)to * width] = v;            // (the same chiplet reads it again: it stays in its cache)
+      u = fmaf(take[to], v, u);
+    }
+  }
+  // (The waves' sums in the order of `block_sum`.)
+  const float mine = wave_sum(in ? u * u : 0.f);
+  if (lane == 0) scratch[wave] = mine;
+  __syncthreads();
+  float part[16], total = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) part[w] = scratch[w];
+#pragma unroll
+  for (int w = 0; w < 16; ++w) total += w < n_waves ? part[w] : 0.f;
+  float h = u * (1.0f / sqrtf(total / (float)width + eps) * g);
+  if (SHIFT && slot >= 0) {
+    if (in) state[(size_t)slot * width + c] = h;
+    h = fmaf((first ? 0.f : before) - h, mu_c, h);
+  }
+  if (in) st_through(out + (size_t)i * width + c, h);
+}
+
 // Token shift over a batch of portions: out[t] = h[t] + (before - h[t]) * mu, `before` = h[t - 1] inside a portion, the
 // request's state row for a portion's first token (zeros at position 0).  The block of a portion's first token also
 // leaves the portion's last row in the state: it alone touches that row, after it has read it.
@@ -231,6 +311,20 @@ extern "C" int ta_streams_step(void* streams, const void* y, const void* mix, co
   // 256 columns; many rows fill the device with workgroups of 256.
   int threads = 256;
   if (n_rows <= 2 * compute_units()) threads = width >= 1024 ? 1024 : (width + WAVE - 1) / WAVE * WAVE;
+  if (n_streams <= 4 && width <= threads) {
+#define GO(TY, TO) do { if (mu) GO_M(TY, TO, true); else GO_M(TY, TO, false); } while (0)
+#define GO_M(TY, TO, SH) do { if (n_streams == 4) GO_S(TY, TO, SH, 4); else if (n_streams == 3) GO_S(TY, TO, SH, 3); \
+                              else if (n_streams == 2) GO_S(TY, TO, SH, 2); else GO_S(TY, TO, SH, 1); } while (0)
+#define GO_S(TY, TO, SH, SS) streams_step_column_kernel<TY, TO, SH, SS><<<n_rows, threads, 0, stream>>>((float*)streams, (const TY*)y, (const float*)mix, \
+    (const float*)out_coef, (const float*)read, (const float*)gain, width, eps, (const int*)rows, (const float*)scale, (TO*)out, \
+    (const float*)mu, (float*)state, (const int*)entry_of_token, (const int*)state_slots, (const int*)positions)
+    if (y_dtype == DT_F32 && out_dtype != DT_F32) return -1;
+    if (y_dtype == DT_F32) GO(float, float); else if (out_dtype == DT_F32) GO(bf16_t, float); else GO(bf16_t, bf16_t);
+#undef GO_S
+#undef GO_M
+#undef GO
+    return LAUNCH_STATUS();
+  }
 #define GO(TY, TO) if (n_streams <= 4) GO_S(TY, TO, 4); else if (n_streams <= 8) GO_S(TY, TO, 8); else GO_S(TY, TO, 16)
 #define GO_S(TY, TO, SS) streams_step_kernel<TY, TO, SS><<<n_rows, threads, 0, stream>>>((float*)streams, (const TY*)y, (const float*)mix, \
     (const float*)out_coef, (const float*)scale, (const float*)read, (const float*)gain, eps, (TO*)out, (const int*)rows,   \
