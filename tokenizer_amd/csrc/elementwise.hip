@@ -398,7 +398,9 @@ __global__ void __launch_bounds__(256)
 add_terms_rmsnorm_vec_kernel(float* __restrict__ residual, SumTerms terms, const float* __restrict__ weight, T* __restrict__ out,
                              const int* __restrict__ rows, int hidden, float eps, int store_residual, int out_stride,
                              const float* __restrict__ weight2, float eps2, T* __restrict__ out2, SlabTerm tail) {
-  HELD(residual, weight, out, rows, hidden, eps, store_residual, out_stride, weight2, out2);
+  HELD(residual, weight, out, rows, hidden, eps, store_residual, out_stride, weight2, out2, terms.rows[0], terms.rows[1], terms.rows[2],
+       terms.rows[3], terms.factor[0], terms.factor[1], terms.factor[2], terms.factor[3], tail.slabs, tail.stride, tail.count, tail.factor,
+       tail.rounded);
   __shared__ float scratch[16];
   constexpr int FIRST = CHUNKS == 1 ? 8 : 4;                 // slabs asked for at the start
   const int i = blockIdx.x;

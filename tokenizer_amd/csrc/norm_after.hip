@@ -116,9 +116,10 @@ __global__ void __launch_bounds__(NA_THREADS)
 norm_add_rmsnorm_vec_kernel(float* __restrict__ residual, const TD* __restrict__ delta, const float* __restrict__ post_weight,
                             float post_eps, const float* __restrict__ weight, float eps, TO* __restrict__ out,
                             const int* __restrict__ rows, int hidden, int store_residual, int parts, size_t slab, int rounded) {
+  HELD(residual, delta, post_weight, post_eps, weight, eps, out, rows, hidden, store_residual, parts, slab, rounded);
   __shared__ float scratch[16];
   const int i = blockIdx.x;
-  const int r = rows ? rows[i] : i;
+  const int r = rows ? scalar_int(rows + i) : i;
   float* res = residual + (size_t)r * hidden;
   const TD* del = delta + (size_t)r * hidden;
   float4 x[CHUNKS], d[CHUNKS], behind_w[CHUNKS], next_w[CHUNKS];
@@ -516,6 +517,8 @@ norm_side_norm_held_kernel(float* __restrict__ residual, const void* __restrict_
                            const int* __restrict__ token_ids, int offset, int dim, const float* __restrict__ weight, float eps,
                            bf16_t* __restrict__ out, const int* __restrict__ rows, int n_rows, int hidden, int store_residual,
                            int parts, size_t slab, int rounded) {
+  HELD(residual, delta, post_weight, gate, proj, proj_stride, side_norm, table, table_width, token_ids, offset, dim, weight, out, rows,
+       n_rows, hidden, store_residual, parts, slab, rounded, post_eps, side_eps, eps);
   __shared__ __attribute__((aligned(16))) float x_s[R][RUNS * 2048];
   __shared__ __attribute__((aligned(16))) float g_s[R][16];
   __shared__ float scratch[R * 16], inv_s[R], inv_t[R];
@@ -525,7 +528,7 @@ norm_side_norm_held_kernel(float* __restrict__ residual, const void* __restrict_
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int i = min((int)blockIdx.x * R + q, n_rows - 1);
-    r[q] = rows ? rows[i] : i;
+    r[q] = rows ? scalar_int(rows + i) : i;
   }
   float2 x[R][RUNS], d[R][RUNS];
   uint32_t raw[R][RUNS];
@@ -827,7 +830,13 @@ __device__ __forceinline__ void na_group_rms(const float* part, float* inv, int 
   __syncthreads();
   for (int g = wave; g < groups; g += NA_THREADS / WAVE) {
     float sq = 0.f;
-    for (int i = lane; i < entries; i += WAVE) sq += part[(size_t)g * entries + i];
+    for (int i0 = 0; i0 < entries; i0 += 8 * WAVE) {         // (eight reads on their way at once, added in their order)
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = part[(size_t)g * entries + min(i0 + j * WAVE + lane, entries - 1)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sq += i0 + j * WAVE + lane < entries ? v[j] : 0.f;
+    }
     sq = wave_sum(sq);
     if (lane == 0) inv[g] = 1.0f / sqrtf(sq / (float)size + eps);
   }
@@ -847,19 +856,38 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
                           float post_eps, int post_groups, const float* __restrict__ weight, float eps, int groups,
                           TO* __restrict__ out, const int* __restrict__ rows, int hidden, int store_residual, int parts,
                           size_t slab, int rounded) {
+  HELD(residual, delta, post_weight, post_eps, post_groups, weight, eps, groups, out, rows, hidden, store_residual);
   extern __shared__ float na_part[];
   float* inv = na_part + hidden / 4;
   const int i = blockIdx.x;
-  const int r = rows ? rows[i] : i;
+  const int r = rows ? scalar_int(rows + i) : i;
   float* res = residual + (size_t)r * hidden;
+  // What a form has not is loaded from the row itself and not used: no load stands behind a condition, which would be a trip of its own.
+  const TD* del = delta ? delta + (size_t)r * hidden : reinterpret_cast<const TD*>(res);
+  const float* post_at = post_weight ? post_weight : res;
+  const float* next_at = weight ? weight : res;
   float4 x[CHUNKS], d[CHUNKS], behind_w[CHUNKS], next_w[CHUNKS];
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int h = min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4);
     x[c] = na_ld4(res + h);
-    d[c] = delta ? na_ld4(delta + (size_t)r * hidden + h) : make_float4(0.f, 0.f, 0.f, 0.f);
-    behind_w[c] = post_weight ? na_ld4(post_weight + h) : make_float4(1.f, 1.f, 1.f, 1.f);
-    next_w[c] = weight ? na_ld4(weight + h) : make_float4(1.f, 1.f, 1.f, 1.f);
+    if constexpr (PARTS) d[c] = na_ld4(del + h);
+    behind_w[c] = na_ld4(post_at + h);
+    next_w[c] = na_ld4(next_at + h);
+  }
+  // (The groups an element is in are worked out while the rows are on their way.)
+  int post_of[CHUNKS], next_of[CHUNKS];
+  const int post_size = hidden / post_groups, next_size = hidden / groups;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int h = min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4);
+    post_of[c] = h / post_size;
+    next_of[c] = h / next_size;
+    asm volatile("" : "+v"(post_of[c]), "+v"(next_of[c]));
+  }
+  if constexpr (!PARTS) {
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) d[c] = na_ld4(del + min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4));
   }
   if constexpr (PARTS) na_add_slabs<CHUNKS>(d, delta + (size_t)r * hidden, parts, slab, hidden, rounded);
   if (post_weight) {
@@ -874,9 +902,13 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
   for (int c = 0; c < CHUNKS; ++c) {
     const int h = (c * NA_THREADS + (int)threadIdx.x) * 4;
     if (h >= hidden) continue;
-    const float f = post_weight ? inv[h / (hidden / post_groups)] : 1.f;
-    x[c].x += d[c].x * f * behind_w[c].x; x[c].y += d[c].y * f * behind_w[c].y;
-    x[c].z += d[c].z * f * behind_w[c].z; x[c].w += d[c].w * f * behind_w[c].w;
+    if (post_weight) {
+      const float f = inv[post_of[c]];
+      x[c].x += d[c].x * f * behind_w[c].x; x[c].y += d[c].y * f * behind_w[c].y;
+      x[c].z += d[c].z * f * behind_w[c].z; x[c].w += d[c].w * f * behind_w[c].w;
+    } else if (PARTS || delta) {
+      x[c].x += d[c].x; x[c].y += d[c].y; x[c].z += d[c].z; x[c].w += d[c].w;
+    }
     if (store_residual) na_st4(res + h, x[c]);
   }
   if (weight) {
@@ -893,9 +925,13 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
   for (int c = 0; c < CHUNKS; ++c) {
     const int h = (c * NA_THREADS + (int)threadIdx.x) * 4;
     if (h >= hidden) continue;
-    const float f = weight ? inv[h / (hidden / groups)] : 1.f;
-    na_st4(dst + h, make_float4(x[c].x * f * next_w[c].x, x[c].y * f * next_w[c].y, x[c].z * f * next_w[c].z,
-                                x[c].w * f * next_w[c].w));
+    if (weight) {
+      const float f = inv[next_of[c]];
+      na_st4(dst + h, make_float4(x[c].x * f * next_w[c].x, x[c].y * f * next_w[c].y, x[c].z * f * next_w[c].z,
+                                  x[c].w * f * next_w[c].w));
+    } else {
+      na_st4(dst + h, x[c]);
+    }
   }
 }
 
