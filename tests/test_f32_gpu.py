@@ -50,6 +50,27 @@ def test_products(ops, ref, shape):
                                **linear_tol(torch.float32, x, w))
 
 
+# Few rows staged by their waves (three and four in one load, five and eight in two, nine not at all) and workgroups of four, seven and sixteen
+# weight rows with a last one that is not full; one unit, units for some of the waves, for two pairs of each, and many; the gate with
+# rows in LDS and without; rows of a longer stride with no numbers between them.
+@pytest.mark.parametrize("rows", [3, 4, 5, 8, 9])
+@pytest.mark.parametrize("n,k", [(20, 32), (100, 608), (900, 896), (1540, 1536), (2500, 4896)])
+def test_few_rows_spread_over_the_device(ops, ref, rows, n, k):
+    x = torch.full((rows, k + 4), float("nan"), device="cuda")
+    x[:, :k] = rand((rows, k), torch.float32, 71)
+    x, w, bias = x[:, :k], rand((n, k), torch.float32, 72, 0.1), rand((n,), torch.float32, 73)
+    want = ref.linear(x, w, bias, out_dtype=torch.float64)
+    torch.testing.assert_close(ops.linear(x, w, bias).double(), want, **linear_tol(torch.float32, x, w))
+    left = ops.linear(x, w, bias, pending=True)
+    left = left.resolve() if isinstance(left, PendingSum) else left
+    torch.testing.assert_close(left.double(), want, **linear_tol(torch.float32, x, w))
+    got, gate = ops.linear_silu_gate(x, w), want - bias.double()
+    exact = gate[:, :n // 2] / (1 + torch.exp(-gate[:, :n // 2])) * gate[:, n // 2:]
+    # (each factor is off by a product's bound, the other one is at most the largest sum)
+    bound = linear_tol(torch.float32, x, w)["atol"] * (2 + 2 * float(gate.abs().max()))
+    assert float((got.double() - exact).abs().max()) <= bound
+
+
 def test_a_product_of_infinities_keeps_them_to_their_row(ops):
     x, w = rand((4, 100), torch.float32, 64), rand((32, 100), torch.float32, 65)
     x[1, 0] = float("inf")

@@ -338,48 +338,69 @@ struct F32Store {
   int n_q, n_kv, d, page_size;
 };
 
+// PLAIN and ROPE take fewer rows a workgroup (`tile_rows` in all: down to four; of each half with ROPE: down to two) where sixteen (eight) are
+// fewer workgroups than compute units; lanes of rows past them load nothing and only feed sums that nobody reads.
+// STAGE > 0 (LINES, up to four rows for one and up to eight for two): a wave brings a pair of units of A's rows in STAGE loads of sixteen
+// different bytes a lane and turns them into fragments through a part of LDS of its own; a fragment straight from memory is a load
+// that holds up the memory pipeline like any other though its lanes mostly ask for the same bytes.
+// (Before all of this, a pair that is not there multiplied as zeros and positions fetched where they are used | so, us, weights from memory,
+// four rows and eight: q/k/v of 896 with rotation 5.7 | 4.9 and 5.9 | 5.3, 896 over 896 in two parts 4.4 | 3.5 and 4.5 | 3.6, 896 over 4,864 in eight
+// 7.4 | 6.3 and 7.7 | 7.0.)
 enum { ROWS_PLAIN = 0, ROWS_GATED = 1, ROWS_ROPE = 2 };
 
-template <int KIND, bool LINES>
+template <int KIND, bool LINES, int STAGE>
 __global__ void __launch_bounds__(512)
-gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int units_part,
-                     float* __restrict__ partial, const F32Store store = F32Store()) {
-  constexpr int WAVES = 8, PAIR = 2;
-  constexpr bool HALVES = KIND != ROWS_PLAIN;               // eight weight rows here and eight a fixed way further on
+gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, uint32_t m_rows_d, int N, int K, int lda, int units_part,
+                     const float* __restrict__ bias, float* __restrict__ partial, float* __restrict__ C, int ldc,
+                     const F32Store store = F32Store()) {
+  HELD(A, W, m_rows_d, N, K, lda, units_part, bias, partial);                // (the words that are there when a wave starts)
+  constexpr int WAVES = 8, PAIR = 2, ROW_BYTES = PAIR * 128 + 16;
+  constexpr bool HALVES = KIND != ROWS_PLAIN;               // weight rows here and as many a fixed way further on
+  static_assert(STAGE == 0 || LINES, "rows are staged line by line");
   __shared__ float sums[WAVES][16][17];
+  __shared__ __attribute__((aligned(16))) char rows_s[STAGE > 0 ? WAVES * 4 * STAGE * ROW_BYTES : 16];
+  const int M = m_rows_d & 0xff, tile_rows = (m_rows_d >> 8) & 0xff, d = m_rows_d >> 16;    // (d: ROPE)
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int row = lane & 15, g = lane >> 4;
-  const int per_head = KIND == ROWS_ROPE ? store.d / 16 : 1;
-  const int head = KIND == ROWS_ROPE ? blockIdx.x / per_head : 0, first_in = KIND == ROWS_ROPE ? blockIdx.x % per_head * 8 : 0;
-  const int half = KIND == ROWS_ROPE ? store.d / 2 : N / 2;
-  const int n0 = KIND == ROWS_ROPE ? head * store.d + first_in : blockIdx.x * (HALVES ? 8 : 16);
+  const int per_head = KIND == ROWS_ROPE ? d / 2 / tile_rows : 1;
+  const int head = KIND == ROWS_ROPE ? blockIdx.x / per_head : 0, first_in = KIND == ROWS_ROPE ? blockIdx.x % per_head * tile_rows : 0;
+  const int half = KIND == ROWS_ROPE ? d / 2 : N / 2;
+  const int n0 = KIND == ROWS_ROPE ? head * d + first_in : blockIdx.x * tile_rows;
   const int limit = KIND == ROWS_GATED ? half : N;
-  // The weight row behind row i (0 .. 15) of the tile.
+  // The weight row behind row i (0 .. 15) of the tile, and whether it is there.
   auto weight_row = [&](int i) {
     return HALVES ? min(n0 + (i & 7), limit - 1) + (i < 8 ? 0 : half) : min(n0 + i, N - 1);
   };
+  auto there = [&](int i) { return (HALVES ? i & 7 : i) < tile_rows; };
   const int units = (K + 31) / 32;
   const int u_begin = blockIdx.y * units_part, u_end = min(units, u_begin + units_part);
-  const float* a_row = A + (size_t)min(row, M - 1) * lda;
+  const int a_m = min(row, M - 1);
+  const float* a_row = A + (size_t)a_m * lda;
   const float* w_row[2];
+  bool w_ok[2];
   w_row[0] = W + (size_t)weight_row(LINES ? row & 7 : row) * K;
   w_row[1] = LINES ? W + (size_t)weight_row(8 + (row & 7)) * K : w_row[0];
+  w_ok[0] = there(LINES ? row & 7 : row);
+  w_ok[1] = LINES ? there(8 + (row & 7)) : w_ok[0];
   const int piece = 2 * g + (row >> 3);
-  f32x4 w[2][PAIR][2], a[2][PAIR][2];
+  char* mine = rows_s + (STAGE > 0 ? wave * M * ROW_BYTES : 0);
+  f32x4 w[2][PAIR][2], a[2][PAIR][2], staged[2][STAGE > 0 ? STAGE : 1];
   auto ask = [&](int slot, int u0) {
 #pragma unroll
     for (int p = 0; p < PAIR; ++p) {
       const int u = u0 + p * WAVES;
       if constexpr (LINES) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) w[slot][p][h] = a[slot][p][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int h = 0; h < 2; ++h) w[slot][p][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (STAGE == 0) a[slot][p][0] = a[slot][p][1] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (u < u_end) {                                     // (the same for the whole wave)
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            w[slot][p][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w_row[h] + u * 32 + 4 * piece));
+            if (w_ok[h]) w[slot][p][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w_row[h] + u * 32 + 4 * piece));
+          if constexpr (STAGE == 0) {
 #pragma unroll
-          for (int h = 0; h < 2; ++h) a[slot][p][h] = *reinterpret_cast<const f32x4*>(a_row + u * 32 + 8 * g + 4 * h);
+            for (int h = 0; h < 2; ++h) a[slot][p][h] = *reinterpret_cast<const f32x4*>(a_row + u * 32 + 8 * g + 4 * h);
+          }
         }
       } else {
 #pragma unroll
@@ -393,30 +414,66 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
         }
       }
     }
+    if (STAGE > 0 && u0 < u_end) {
+      // Piece i of the pair's M * 16 is piece i % 16 of row i / 16; a unit past the end is the last one again, put down as zeros.
+#pragma unroll
+      for (int j = 0; j < STAGE; ++j) {
+        const int i = min(j * WAVE + lane, M * 16 - 1), u = min(u0 + ((i & 15) >> 3) * WAVES, u_end - 1);
+        staged[slot][j] = *reinterpret_cast<const f32x4*>(A + (size_t)(i >> 4) * lda + u * 32 + 4 * (i & 7));
+      }
+    }
   };
   f32x4 acc[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int first = u_begin + wave;
   ask(0, first);
-  // What the rotation needs hangs on the row's position: asked for behind the first weights.
-  const int m = threadIdx.x >> 4, at = threadIdx.x & 15;
+  // What the epilogue needs is asked for behind the first weights, positions and slots through the scalar unit.
+  const int m = threadIdx.x >> 4, at = threadIdx.x & 15;    // its thread: row m, weight row `at`; wave v has rows 4 v .. 4 v + 3
   float cosine = 1.f, sine = 0.f, bias1 = 0.f, bias2 = 0.f;
   int slot_of = -1;
-  if (KIND == ROWS_ROPE && m < M && at < 8) {
-    if (head < store.n_q + store.n_kv && store.cos_sin) {
-      const float* cs = store.cos_sin + (size_t)store.positions[m] * store.d + first_in + at;
-      cosine = cs[0];
-      sine = cs[half];
+  if (4 * wave < M) {
+    HELD(C, ldc, store.positions, store.cos_sin, store.slots, store.k_pages, store.v_pages, store.n_q, store.n_kv, store.page_size);
+    if constexpr (KIND == ROWS_ROPE) {
+      const bool turned = head < store.n_q + store.n_kv && store.cos_sin;
+      int position = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int of = min(4 * wave + j, M - 1);
+        const int p = turned ? scalar_int(store.positions + of) : 0, s = store.slots ? scalar_int(store.slots + of) : -1;
+        position = (lane >> 4) == j ? p : position;
+        slot_of = (lane >> 4) == j ? s : slot_of;
+      }
+      if (m < M && at < tile_rows) {
+        if (turned) {
+          const float* cs = store.cos_sin + (size_t)position * d + first_in + at;
+          cosine = cs[0];
+          sine = cs[half];
+        }
+        if (bias) { bias1 = bias[n0 + at]; bias2 = bias[n0 + half + at]; }
+      }
+    } else if (KIND == ROWS_PLAIN && bias && !partial && m < M) {
+      bias1 = bias[min(n0 + at, N - 1)];
     }
-    if (bias) { bias1 = bias[n0 + at]; bias2 = bias[n0 + half + at]; }
-    if (store.slots) slot_of = store.slots[m];
   }
   for (int u0 = first; u0 < u_end; u0 += 2 * PAIR * WAVES) {
 #pragma unroll
     for (int slot = 0; slot < 2; ++slot) {
       const int now = u0 + slot * PAIR * WAVES;
+      if (now >= u_end) break;                               // (the same for the whole wave)
       ask(slot ^ 1, now + PAIR * WAVES);
+      if constexpr (STAGE > 0) {
+#pragma unroll
+        for (int j = 0; j < STAGE; ++j) {
+          const int i = min(j * WAVE + lane, M * 16 - 1);
+          if (now + ((i & 15) >> 3) * WAVES >= u_end) staged[slot][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          *reinterpret_cast<f32x4*>(mine + (i >> 4) * ROW_BYTES + (i & 15) * 16) = staged[slot][j];
+        }
+#pragma unroll
+        for (int p = 0; p < PAIR; ++p)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) a[slot][p][h] = *reinterpret_cast<const f32x4*>(mine + a_m * ROW_BYTES + p * 128 + 32 * g + 16 * h);
+      }
 #pragma unroll
       for (int p = 0; p < PAIR; ++p) {
         if constexpr (LINES) {
@@ -449,7 +506,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 #pragma unroll
   for (int j = 0; j < 4; ++j) sums[wave][row][4 * g + j] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
   __syncthreads();
-  if (m >= M) return;                                      // (threads from the sixteenth row on leave here too)
+  if (m >= M || at >= tile_rows) return;                   // (threads from the sixteenth row on leave here too)
   auto total = [&](int place) {
     float t = 0.f;
 #pragma unroll
@@ -457,33 +514,46 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
     return t;
   };
   if constexpr (KIND == ROWS_ROPE) {
-    if (at >= 8) return;
     const float x1 = total(at) + bias1, x2 = total(at + 8) + bias2;
     const float v1 = x1 * cosine - x2 * sine, v2 = x2 * cosine + x1 * sine;     // cosine 1 and sine 0 where nothing turns
     const int i = first_in + at;
     if (head < store.n_q) {
-      float* dst = C + (size_t)m * ldc + (size_t)head * store.d + i;
-      dst[0] = v1;
-      dst[half] = v2;
+      float* dst = C + (size_t)m * ldc + (size_t)head * d + i;
+      st_through(dst, v1);
+      st_through(dst + half, v2);
       return;
     }
     if (slot_of < 0) return;                                // this row's keys and values are not stored
     const int page = slot_of / store.page_size, off = slot_of % store.page_size;
     if (head < store.n_q + store.n_kv) {
-      float* dst = store.k_pages + (((size_t)page * store.n_kv + (head - store.n_q)) * store.page_size + off) * store.d + i;
-      dst[0] = v1;
-      dst[half] = v2;
+      float* dst = store.k_pages + (((size_t)page * store.n_kv + (head - store.n_q)) * store.page_size + off) * d + i;
+      st_through(dst, v1);
+      st_through(dst + half, v2);
     } else {
-      float* dst = store.v_pages + (((size_t)page * store.n_kv + (head - store.n_q - store.n_kv)) * store.d + i) * store.page_size + off;
-      dst[0] = v1;
-      dst[(size_t)half * store.page_size] = v2;
+      float* dst = store.v_pages + (((size_t)page * store.n_kv + (head - store.n_q - store.n_kv)) * d + i) * store.page_size + off;
+      st_through(dst, v1);
+      st_through(dst + (size_t)half * store.page_size, v2);
     }
   } else if (KIND == ROWS_GATED) {
-    if (at < 8 && n0 + at < half) C[(size_t)m * ldc + n0 + at] = silu_f32(total(at)) * total(at + 8);
+    if (n0 + at < half) st_through(C + (size_t)m * ldc + n0 + at, silu_f32(total(at)) * total(at + 8));
   } else if (n0 + at < N) {
-    if (partial) partial[((size_t)blockIdx.y * M + m) * N + n0 + at] = total(at);
-    else C[(size_t)m * ldc + n0 + at] = total(at) + (bias ? bias[n0 + at] : 0.f);
+    if (partial) st_through(partial + ((size_t)blockIdx.y * M + m) * N + n0 + at, total(at));
+    else st_through(C + (size_t)m * ldc + n0 + at, total(at) + bias1);
   }
+}
+
+// Launches the kernel above: `rows` weight rows a workgroup (of each half with GATED and ROPE), `d` the head size (ROPE).
+template <int KIND>
+static void launch_f32_rows(dim3 grid, const float* a, const float* w, const float* bias, float* c, int M, int N, int K, int lda, int ldc,
+                            int units_part, float* partial, int rows, int d, const F32Store& store, hipStream_t stream) {
+  const uint32_t packed = (uint32_t)M | (uint32_t)rows << 8 | (uint32_t)d << 16;
+#define GO(LINES, STAGE) gemm_f32_rows_kernel<KIND, LINES, STAGE><<<grid, 512, 0, stream>>>(a, w, packed, N, K, lda, units_part, bias, partial, c, \
+                                                                                            ldc, store)
+  if (K % 32) GO(false, 0);
+  else if (M <= 4) GO(true, 1);
+  else if (M <= 8) GO(true, 2);
+  else GO(true, 0);
+#undef GO
 }
 
 // One or two rows, four of large matrices, and up to sixteen whose pieces of sixteen bytes do not lie on sixteen bytes (VEC false):
@@ -495,13 +565,22 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, c
 // 3,584 over 18,944 55.3 | 51.3, but 4,608 over 3,584 13.5 | 16.7, 151,936 over 896, three rows 84 | 98).  Past the caches, one row from memory
 // and from the last-level cache, us through them | past them: 768 columns over 3,072 9.7 | 8.3 and 6.9 | 8.0, over 768 4.0 | 3.4 and 3.3 | 3.4, 896
 // over 4,864 14.2 | 12.3 and 9.7 | 11.7: a model in less than the cache's 256 MB loses, which the kernel cannot know, and every other gains.
-template <int MR, bool VEC, bool GATED, int UN = 1>
+// ROWS (VEC): the rows of A are brought into LDS once for the workgroup's four waves, which otherwise ask for all of them each.  The sums over
+// a wave are taken eight at a time, each where one lane stores it, the gate with it.  (Gate/up 4,864 over 896, four rows, each wave for itself
+// and one lane with all gates | so: 10.1 | 8.9 us, two rows 8.4 | 8.2; 35 MB of weights are 5.7.)
+template <int MR, bool VEC, bool GATED, int UN = 1, bool ROWS = false>
 __global__ void __launch_bounds__(256)
-gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-                float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = N / 2;
+gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int lda, const float* __restrict__ bias,
+                float* __restrict__ C, int ldc) {
+  HELD(A, W, M, N, K, lda, bias, C, ldc);
+  extern __shared__ __attribute__((aligned(16))) float rows_s[];
+  const int lane = threadIdx.x & 63, wave = wave_index(), half = N / 2;
   const int n0 = (blockIdx.x * 4 + wave) * (GATED ? 2 : 4);  // this wave's weight rows
-  if (n0 >= (GATED ? half : N)) return;
+  if (!ROWS && n0 >= (GATED ? half : N)) return;
+  // Which of eight sums ends in this lane (see `wave_sums8`), and the bias of its weight row.
+  const int s8 = (lane & 1) + 2 * ((lane >> 4) & 1) + 4 * (lane >> 5);
+  float bias_here = 0.f;
+  if (!GATED && bias) bias_here = bias[min(n0 + (s8 & 3), N - 1)];
   float acc[4][MR];
 #pragma unroll
   for (int r = 0; r < 4; ++r)
@@ -511,6 +590,14 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
 #pragma unroll
   for (int r = 0; r < 4; ++r)
     w[r] = W + (size_t)(GATED ? (r < 2 ? 0 : half) + min(n0 + (r & 1), half - 1) : min(n0 + r, N - 1)) * K;
+  if constexpr (ROWS) {
+    for (int i = threadIdx.x * 4; i < M * K; i += 256 * 4) {
+      const int m = i / K;
+      *reinterpret_cast<f32x4*>(rows_s + i) = *reinterpret_cast<const f32x4*>(A + (size_t)m * lda + (i - m * K));
+    }
+    __syncthreads();
+    if (n0 >= (GATED ? half : N)) return;
+  }
   if constexpr (VEC) {
     for (int k0 = lane * 4; k0 < K; k0 += UN * WAVE * 4) {
       f32x4 wv[UN][4];
@@ -528,7 +615,7 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
           if (m >= M) break;
-          const float4 a = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
+          const float4 a = *reinterpret_cast<const float4*>(ROWS ? rows_s + m * K + k : A + (size_t)m * lda + k);
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             acc[r][m] = fmaf(a.x, wv[u][r][0], fmaf(a.y, wv[u][r][1], fmaf(a.z, wv[u][r][2], fmaf(a.w, wv[u][r][3], acc[r][m]))));
@@ -549,20 +636,25 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, const 
       }
     }
   }
+  // Sum i of eight: PLAIN weight row i % 4 of row i / 4, GATED weight row i % 2 of row i / 2 of both halves.
+  constexpr int ROWS_IN_8 = GATED ? 4 : 2;
 #pragma unroll
-  for (int m = 0; m < MR; ++m) {
-    float total[4];
+  for (int m0 = 0; m0 < MR; m0 += ROWS_IN_8) {
+    if (m0 >= M) break;
+    float v[8], up[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) total[r] = wave_sum(acc[r][m]);
-    if (lane != 0 || m >= M) continue;
+    for (int i = 0; i < 8; ++i) {
+      const int m = m0 + i / (8 / ROWS_IN_8), r = i % (8 / ROWS_IN_8);
+      v[i] = m < MR ? acc[r][m < MR ? m : 0] : 0.f;
+      if (GATED) up[i] = m < MR ? acc[r + 2][m < MR ? m : 0] : 0.f;
+    }
+    const float total = wave_sums8(v, lane), second = GATED ? wave_sums8(up, lane) : 0.f;
+    const int m = m0 + s8 / (8 / ROWS_IN_8), n = n0 + s8 % (8 / ROWS_IN_8);
+    if ((lane & 15) > 1 || m >= M) continue;
     if constexpr (GATED) {
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-        if (n0 + r < half) C[(size_t)m * ldc + n0 + r] = silu_f32(total[r]) * total[r + 2];
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n0 + r < N) C[(size_t)m * ldc + n0 + r] = total[r] + (bias ? bias[n0 + r] : 0.f);
+      if (n < half) st_through(C + (size_t)m * ldc + n, silu_f32(total) * second);
+    } else if (n < N) {
+      st_through(C + (size_t)m * ldc + n, total + bias_here);
     }
   }
 }
@@ -660,11 +752,9 @@ extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void*
   float *c = (float*)C, *slabs = (float*)partial;
   const int k_part = parts > 1 ? ((K + parts - 1) / parts + 31) / 32 * 32 : K;
   if (tile == 16) {
-    const dim3 grid((N + 15) / 16, parts);
-    if (K % 32 == 0)
-      gemm_f32_rows_kernel<ROWS_PLAIN, true><<<grid, 512, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, (k_part + 31) / 32, slabs);
-    else
-      gemm_f32_rows_kernel<ROWS_PLAIN, false><<<grid, 512, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc, (k_part + 31) / 32, slabs);
+    const int units = compute_units(), even = (int)(((long)N * parts + units - 1) / units), rows = even < 4 ? 4 : even > 16 ? 16 : even;
+    launch_f32_rows<ROWS_PLAIN>(dim3((N + rows - 1) / rows, parts), a, w, b, c, M, N, K, lda, ldc, (k_part + 31) / 32, slabs, rows, 0,
+                                F32Store(), stream);
   } else if (tile) {
     const int m_tiles = (M + tile - 1) / tile, n_tiles = (N + tile - 1) / tile;
     dim3 grid((m_tiles * n_tiles + 7) / 8 * 8, parts);
@@ -681,7 +771,7 @@ extern "C" int ta_gemm_f32(const void* A, const void* W, const void* bias, void*
                                                              n_tiles, slabs);
   } else {
     const int blocks = (N + 15) / 16;
-#define GO(MR, VEC, ...) gemv_f32_kernel<MR, VEC, false, ##__VA_ARGS__><<<blocks, 256, 0, stream>>>(a, w, b, c, M, N, K, lda, ldc)
+#define GO(MR, VEC, ...) gemv_f32_kernel<MR, VEC, false, ##__VA_ARGS__><<<blocks, 256, 0, stream>>>(a, w, M, N, K, lda, b, c, ldc)
     if (aligned && blocks <= compute_units()) { if (M <= 1) GO(1, true, 4); else if (M <= 2) GO(2, true, 4); else if (M <= 4) GO(4, true, 4); else GO(8, true, 2); }
     else if (aligned) { if (M <= 1) GO(1, true); else if (M <= 2) GO(2, true); else if (M <= 4) GO(4, true); else GO(8, true); }
     else if (M <= 1) GO(1, false); else if (M <= 2) GO(2, false); else if (M <= 4) GO(4, false);
@@ -702,13 +792,13 @@ extern "C" int ta_gemm_f32_silu_gate(const void* A, const void* W, void* out, in
   if (M > 16 || !sixteen_bytes(A, W, M, K, lda)) return -2;
   const float *a = (const float*)A, *w = (const float*)W;
   const int blocks = (N / 2 + 7) / 8;
-#define GO(MR) do { if (blocks <= compute_units()) gemv_f32_kernel<MR, true, true, 4><<<blocks, 256, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc); \
-                    else gemv_f32_kernel<MR, true, true><<<blocks, 256, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc); } while (0)
+  const size_t rows_bytes = (size_t)M * K * sizeof(float);
+  const bool rows_fit = M > 1 && rows_bytes <= 20 * 1024;    // (eight workgroups a compute unit)
+#define GO(MR) do { if (blocks <= compute_units()) gemv_f32_kernel<MR, true, true, 4><<<blocks, 256, 0, stream>>>(a, w, M, N, K, lda, nullptr, (float*)out, ldc); \
+                    else if (rows_fit) gemv_f32_kernel<MR, true, true, 1, true><<<blocks, 256, rows_bytes, stream>>>(a, w, M, N, K, lda, nullptr, (float*)out, ldc); \
+                    else gemv_f32_kernel<MR, true, true><<<blocks, 256, 0, stream>>>(a, w, M, N, K, lda, nullptr, (float*)out, ldc); } while (0)
   if (!vector_rows(M, N, K, false)) {
-    if (K % 32 == 0)
-      gemm_f32_rows_kernel<ROWS_GATED, true><<<blocks, 512, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc, (K + 31) / 32, nullptr);
-    else
-      gemm_f32_rows_kernel<ROWS_GATED, false><<<blocks, 512, 0, stream>>>(a, w, nullptr, (float*)out, M, N, K, lda, ldc, (K + 31) / 32, nullptr);
+    launch_f32_rows<ROWS_GATED>(dim3(blocks), a, w, nullptr, (float*)out, M, N, K, lda, ldc, (K + 31) / 32, nullptr, 8, 0, F32Store(), stream);
   } else if (M <= 1) GO(1); else if (M <= 2) GO(2); else if (M <= 4) GO(4); else GO(8);
 #undef GO
   return LAUNCH_STATUS();
@@ -726,9 +816,10 @@ extern "C" int ta_gemm_f32_qkv_rope(const void* x, int lda, const void* W, const
   const F32Store store = {(const int*)positions, (const float*)cos_sin, (const int*)slots, (float*)k_pages, (float*)v_pages,
                           n_q, n_kv, d, page_size};
   const int heads = n_q + 2 * n_kv;
-#define GO(LINES) gemm_f32_rows_kernel<ROWS_ROPE, LINES><<<heads * (d / 16), 512, 0, stream>>>((const float*)x, (const float*)W, \
-      (const float*)bias, (float*)q_out, M, heads * d, K, lda, n_q * d, (K + 31) / 32, nullptr, store)
-  if (K % 32 == 0) GO(true); else GO(false);
-#undef GO
+  if (d > 0xffff) return -1;                                 // (what the kernel's packed arguments hold)
+  int rows = 8;                                              // of each half (d / 2 is a multiple of eight)
+  while (rows > 2 && heads * (d / 2 / rows) * 2 <= compute_units()) rows /= 2;
+  launch_f32_rows<ROWS_ROPE>(dim3(heads * (d / 2 / rows)), (const float*)x, (const float*)W, (const float*)bias, (float*)q_out, M, heads * d, K, lda,
+                             n_q * d, (K + 31) / 32, nullptr, rows, d, store, stream);
   return LAUNCH_STATUS();
 }
