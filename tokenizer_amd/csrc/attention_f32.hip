@@ -219,22 +219,50 @@ attention_f32_kernel(F32Args p) {
 __global__ void __launch_bounds__(WAVE)
 attention_f32_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ rows,
                            float* __restrict__ out, int n_q, int dv, int splits, const int* __restrict__ entry_of_token) {
-  const int item = blockIdx.x / n_q, head = blockIdx.x % n_q;
+  HELD(part_o, part_ml, rows, out, n_q, dv, splits, entry_of_token);
+  const int item = blockIdx.x / n_q, head = blockIdx.x % n_q, lane = threadIdx.x;
   const int row = rows ? scalar_int(rows + item) : item;
   if (row < 0 || scalar_int(entry_of_token + row) < 0) return;
   const size_t base = ((size_t)item * n_q + head) * splits;
   const float2* ml = reinterpret_cast<const float2*>(part_ml) + base;
+  float* dst = out + ((size_t)row * n_q + head) * dv;
+  if (splits <= WAVE) {
+    // A part a lane: maxima and sums, and the first parts' rows beside them, are one trip, each weight one exponential.
+    float2 stat = ml[min(lane, splits - 1)];
+    constexpr int AHEAD = 8;
+    float v[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) v[j] = part_o[(base + min(j, splits - 1)) * dv + min(lane, dv - 1)];
+    if (lane >= splits) stat = make_float2(-INFINITY, 0.f);
+    const float big = wave_max(stat.x), weight = lane < splits ? expf(stat.x - big) : 0.f;
+    const float denom = wave_sum(stat.y * weight);
+    for (int i0 = 0; i0 < dv; i0 += WAVE) {
+      const int i = min(i0 + lane, dv - 1);
+      float o = 0.f;
+      for (int s0 = 0; s0 < splits; s0 += AHEAD) {
+        if (i0 + s0 > 0) {
+#pragma unroll
+          for (int j = 0; j < AHEAD; ++j) v[j] = part_o[(base + min(s0 + j, splits - 1)) * dv + i];
+        }
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+          if (s0 + j < splits) o += v[j] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s0 + j));
+      }
+      if (i0 + lane < dv) st_through(dst + i, o / denom);
+    }
+    return;
+  }
   float big = -INFINITY;
-  for (int s = threadIdx.x; s < splits; s += WAVE) big = fmaxf(big, ml[s].x);
+  for (int s = lane; s < splits; s += WAVE) big = fmaxf(big, ml[s].x);
   big = wave_max(big);
   float denom = 0.f;
-  for (int s = threadIdx.x; s < splits; s += WAVE) denom += ml[s].y * expf(ml[s].x - big);
+  for (int s = lane; s < splits; s += WAVE) denom += ml[s].y * expf(ml[s].x - big);
   denom = wave_sum(denom);
-  for (int i = threadIdx.x; i < dv; i += WAVE) {
+  for (int i = lane; i < dv; i += WAVE) {
     float o = 0.f;
 #pragma unroll 8
     for (int s = 0; s < splits; ++s) o += part_o[(base + s) * dv + i] * expf(ml[s].x - big);
-    out[((size_t)row * n_q + head) * dv + i] = o / denom;
+    dst[i] = o / denom;
   }
 }
 
