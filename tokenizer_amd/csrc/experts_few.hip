@@ -39,15 +39,29 @@ __device__ __forceinline__ int ef_pairs_of(const int* __restrict__ chosen, int n
 struct EfShared { int inner; const float* weights; bf16_t* act; int parts, length; };   // K of `inner` in `parts` of `length`
 
 // acc[h] += sixteen rows of matrix h (lane (col, g): `w_at[h][0]` is row col % 8 of them, `w_at[h][1]` row 8 + col % 8) times the
-// lane's row of x, over this wave's turns of K, UN of which are asked for at once.
-template <int NW, int HALVES, int UN>
-__device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], const bf16_t* x_at, bool x_ok, int K, int wave,
-                                        ef_floatx4 (&acc)[HALVES]) {
+// rows of x that `row_at(i)` says for its `here` <= 16 pairs, over this wave's turns of K, UN of which are asked for at once.
+// SLOTS > 0 (here * UN * 8 pieces of sixteen bytes fill no more loads): the pairs' shares of a trip come in SLOTS loads of sixteen different
+// bytes a lane and become fragments through `stage`, LDS of the wave's own.  A chosen expert of a few rows has one or two pairs, and a
+// fragment straight from memory is two loads a turn, as many as a matrix has, whose lanes mostly ask for nothing of their own.
+#define EF_STAGE_ROWS(UN) ((UN) == 1 ? 8 : 16 / (UN))                 // pairs that are staged at most: SLOTS 1, with four turns 2 too
+#define EF_STAGE_BYTES(UN) (EF_STAGE_ROWS(UN) * ((UN) * 128 + 16))
+template <int NW, int HALVES, int UN, int SLOTS, typename RowAt>
+__device__ __forceinline__ void ef_walk_form(const bf16_t* const (&w_at)[HALVES][2], RowAt row_at, int here, int K, int wave, char* stage,
+                                             ef_floatx4 (&acc)[HALVES]) {
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, piece = g + 4 * (col >> 3);
   const int turns = (K + 63) / 64;
+  constexpr int PIECES = UN * 8, ROW_BYTES = PIECES * 16 + 16;
   const word4 zero = {0u, 0u, 0u, 0u};
+  const bf16_t* from[SLOTS > 0 ? SLOTS : 1];
+  if constexpr (SLOTS > 0) {
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j) from[j] = row_at(min(j * WAVE + lane, here * PIECES - 1) / PIECES);
+  } else {
+    from[0] = row_at(min(col, here - 1));
+  }
+  const bool x_ok = col < here;
   for (int first = wave; first < turns; first += UN * NW) {
-    word4 wf[UN][HALVES][2], xf[UN][2];
+    word4 wf[UN][HALVES][2], xf[UN][2], staged[SLOTS > 0 ? SLOTS : 1];
 #pragma unroll
     for (int q = 0; q < UN; ++q) {
       const int turn = first + q * NW, at = min(turn, turns - 1) * 64;
@@ -57,11 +71,30 @@ __device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], 
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh)
           wf[q][h][hh] = w_in ? __builtin_nontemporal_load(reinterpret_cast<const word4*>(w_at[h][hh] + at + 8 * piece)) : zero;
+      if constexpr (SLOTS == 0) {
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {                          // what the weights are after the exchange: the pieces g and 4 + g
-        const bool x_in = turn < turns && at + 32 * s + 8 * g < K;
-        xf[q][s] = x_in && x_ok ? *reinterpret_cast<const word4*>(x_at + at + 32 * s + 8 * g) : zero;
+        for (int s = 0; s < 2; ++s) {                        // what the weights are after the exchange: the pieces g and 4 + g
+          const bool x_in = turn < turns && at + 32 * s + 8 * g < K;
+          xf[q][s] = x_in && x_ok ? *reinterpret_cast<const word4*>(from[0] + at + 32 * s + 8 * g) : zero;
+        }
       }
+    }
+    if constexpr (SLOTS > 0) {
+#pragma unroll
+      for (int j = 0; j < SLOTS; ++j) {
+        const int i = min(j * WAVE + lane, here * PIECES - 1) % PIECES, k = (first + (i >> 3) * NW) * 64 + 8 * (i & 7);
+        staged[j] = *reinterpret_cast<const word4*>(from[j] + min(k, K - 8));
+      }
+#pragma unroll
+      for (int j = 0; j < SLOTS; ++j) {
+        const int i = min(j * WAVE + lane, here * PIECES - 1), k = (first + ((i % PIECES) >> 3) * NW) * 64 + 8 * (i & 7);
+        if (k >= K) staged[j] = zero;
+        *reinterpret_cast<word4*>(stage + i / PIECES * ROW_BYTES + i % PIECES * 16) = staged[j];
+      }
+#pragma unroll
+      for (int q = 0; q < UN; ++q)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) xf[q][s] = *reinterpret_cast<const word4*>(stage + min(col, here - 1) * ROW_BYTES + q * 128 + s * 64 + g * 16);
     }
 #pragma unroll
     for (int q = 0; q < UN; ++q)
@@ -75,19 +108,30 @@ __device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], 
       }
   }
 }
+template <int NW, int HALVES, int UN, bool STAGED, typename RowAt>
+__device__ __forceinline__ void ef_walk(const bf16_t* const (&w_at)[HALVES][2], RowAt row_at, int here, int K, int wave, char* stage,
+                                        ef_floatx4 (&acc)[HALVES]) {
+  static_assert(UN == 1 || UN == 4, "");
+  constexpr int ONE = 8 / UN;                                // pairs of one load
+  if (!STAGED) ef_walk_form<NW, HALVES, UN, 0>(w_at, row_at, here, K, wave, stage, acc);
+  else if (here <= ONE) ef_walk_form<NW, HALVES, UN, 1>(w_at, row_at, here, K, wave, stage, acc);
+  else if (UN == 4 && here <= 2 * ONE) ef_walk_form<NW, HALVES, UN, 2>(w_at, row_at, here, K, wave, stage, acc);
+  else ef_walk_form<NW, HALVES, UN, 0>(w_at, row_at, here, K, wave, stage, acc);
+}
 
 // x [n_rows, x_stride]; chosen int [n_rows * top], weights float [n_rows * top]; expert e's first matrix starts at
 // W + e * HALVES * inner * hidden: [gate; up] of `inner` rows each (HALVES 2) or `up` alone (HALVES 1), rows of `hidden`.
 // act [n_rows * top, inner]: pair p's row.  HALVES 2: weigh_input ? silu(w g) * (w u) : w * silu(g) * u; HALVES 1: w * max(u, 0)^2.
 // Grid: (blocks of sixteen columns of inner, experts).
-template <int NW, int HALVES, int UN>
+template <int NW, int HALVES, int UN, bool STAGED>
 __global__ void __launch_bounds__(NW * WAVE)
 experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __restrict__ chosen, const float* __restrict__ weights,
                       int n_pairs, int top, const bf16_t* __restrict__ W, int inner, int hidden, bf16_t* __restrict__ act,
                       int weigh_input, EfShared every) {
-  HELD(x, x_stride, chosen, weights, n_pairs, top, W, inner, hidden, act, weigh_input);
+  HELD(x, x_stride, chosen, weights, n_pairs, top, W, inner, hidden, act, weigh_input, every.inner, every.weights, every.act);
   __shared__ int list[EF_MAX_PAIRS];
   __shared__ float red[NW][HALVES * 4][WAVE];
+  __shared__ __attribute__((aligned(16))) char stage_s[STAGED ? NW * EF_STAGE_BYTES(UN) : 16];
   // (The shared expert's workgroups, the ones with the most rows, come first.)
   const bool shared = every.inner > 0 && blockIdx.y == 0;
   const int expert = blockIdx.y - (every.inner > 0 ? 1 : 0), n0 = blockIdx.x * 16;
@@ -112,12 +156,15 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) w_at[h][hh] = first + ((size_t)h * inner + min(n0 + 8 * hh + (col & 7), inner - 1)) * hidden;
   for (int p0 = 0; p0 < count; p0 += 16) {
-    const bool ok = p0 + col < count;
-    const bf16_t* x_at = x + (size_t)(list[min(p0 + col, count - 1)] / top) * x_stride;
+    const int here = min(count - p0, 16);
+    // The weight of the pair whose sum this thread stores, asked for beside the first rows.
+    float wgt = 1.f;
+    if (wave < 4 && weights) wgt = weights[list[p0 + min((int)threadIdx.x >> 4, here - 1)]];
     ef_floatx4 acc[HALVES];
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) acc[h] = (ef_floatx4){0.f, 0.f, 0.f, 0.f};
-    ef_walk<NW, HALVES, UN>(w_at, x_at, ok, hidden, wave, acc);
+    ef_walk<NW, HALVES, UN, STAGED>(w_at, [&](int i) { return x + (size_t)(list[p0 + i] / top) * x_stride; }, here, hidden, wave,
+                            stage_s + wave * EF_STAGE_BYTES(UN), acc);
     // A matrix instruction's result may be read eight wait states behind it at the earliest.  The compiler leaves them out in front
     // of the stores below where there is one matrix (the store is the second instruction behind the last sum; with many
     // workgroups some stored a sum that was not there yet), so they are here, twice over; with two matrices it has them.
@@ -142,7 +189,6 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
         v[h] = bf16_bits_to_float(float_to_bf16_bits(v[h]));
       }
       const int p = list[p0 + c];
-      const float wgt = weights ? weights[p] : 1.f;
       float value;
       if constexpr (HALVES == 2) {
         const float before = weigh_input ? wgt : 1.f, z = before * v[0];
@@ -153,7 +199,7 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
       }
       // (A pick that weighs nothing adds nothing, whatever its expert makes of the row: as the form over all experts has it.)
       if (!shared && wgt == 0.f) value = 0.f;
-      st(act + (size_t)p * inner + n0 + r, value);
+      st_through(act + (size_t)p * inner + n0 + r, value);
     }
     __syncthreads();                                         // the sums are read before the next sixteen pairs' are written
   }
@@ -165,9 +211,10 @@ template <int NW>
 __global__ void __launch_bounds__(NW * WAVE)
 experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ chosen, int n_pairs, int top, int n_rows,
                         const bf16_t* __restrict__ W, int ldw, int inner, int hidden, float* __restrict__ out, EfShared every) {
-  HELD(act, chosen, n_pairs, top, n_rows, W, ldw, inner, hidden, out);
+  HELD(act, chosen, n_pairs, top, n_rows, W, ldw, inner, hidden, out, every.parts, every.length, every.inner, every.act);
   __shared__ int list[EF_MAX_PAIRS];
   __shared__ float red[NW][4][WAVE];
+  __shared__ __attribute__((aligned(16))) char stage_s[NW * EF_STAGE_BYTES(4)];
   const int part = blockIdx.y;                               // below every.parts: a part of the shared expert's K
   const bool shared = part < every.parts;
   const int expert = part - every.parts, n0 = blockIdx.x * 16;
@@ -192,10 +239,9 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
   const bf16_t* const w_at[1][2] = {{columns + (size_t)min(n0 + (col & 7), hidden - 1) * ldw,
                                      columns + (size_t)min(n0 + 8 + (col & 7), hidden - 1) * ldw}};
   for (int p0 = 0; p0 < count; p0 += 16) {
-    const bool ok = p0 + col < count;
-    const bf16_t* x_at = act + (size_t)list[min(p0 + col, count - 1)] * stride;
+    const int here = min(count - p0, 16);
     ef_floatx4 acc[1] = {(ef_floatx4){0.f, 0.f, 0.f, 0.f}};
-    ef_walk<NW, 1, 4>(w_at, x_at, ok, inner, wave, acc);
+    ef_walk<NW, 1, 4, true>(w_at, [&](int i) { return act + (size_t)list[p0 + i] * stride; }, here, inner, wave, stage_s + wave * EF_STAGE_BYTES(4), acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave][r][lane] = acc[0][r];
     __syncthreads();
@@ -206,7 +252,7 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
 #pragma unroll
       for (int w = 0; w < NW; ++w) v += red[w][r & 3][(r >> 2) * 16 + c];
       const int p = list[p0 + c];
-      out[((size_t)(slab + p % top) * n_rows + p / top) * hidden + n0 + r] = v;
+      st_through(out + ((size_t)(slab + p % top) * n_rows + p / top) * hidden + n0 + r, v);
     }
     __syncthreads();
   }
@@ -247,7 +293,7 @@ extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, c
   if (n_experts + every.parts > 65535) return -2;            // (a grid's second dimension)
   const dim3 up(((inner > shared ? inner : shared) + 15) / 16, n_experts + (shared > 0)),
       down((hidden + 15) / 16, n_experts + every.parts);
-#define UP(NW, HH, UN) experts_few_up_kernel<NW, HH, UN><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
+#define UP(NW, HH, UN, ST) experts_few_up_kernel<NW, HH, UN, ST><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
     (const float*)weights, (int)pairs, top, (const bf16_t*)w_first, inner, hidden, (bf16_t*)act, weigh_input, every)
 #define DOWN(NW) experts_few_down_kernel<NW><<<down, NW * WAVE, 0, stream>>>((const bf16_t*)act, (const int*)chosen, (int)pairs, top, \
     n_rows, (const bf16_t*)w_second, ldw, inner, hidden, (float*)out, every)
@@ -256,9 +302,13 @@ extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, c
   // compute units, however the rows choose, and none has another to hide its trips (one | four: 1,792 over 4,096, one row 33.6 | 24.8; 1,024
   // over 1,024 10.9 | 9.4, two rows 11.4 | 9.8; 512 over 1,024, four rows 11.5 | 10.0).  Four of one matrix, eight loads.
   const long busy = (pairs < n_experts ? pairs : n_experts) * ((inner + 15) / 16) + (shared + 15) / 16;
-  if (halves == 1) { if (hidden <= 1024) UP(4, 1, 4); else UP(8, 1, 4); }
-  else if (busy <= compute_units()) { if (hidden <= 1024) UP(4, 2, 4); else UP(8, 2, 4); }
-  else { if (hidden <= 1024) UP(4, 2, 1); else UP(8, 2, 1); }
+  if (halves == 1) { if (hidden <= 1024) UP(4, 1, 4, true); else UP(8, 1, 4, true); }
+  else if (busy <= compute_units()) { if (hidden <= 1024) UP(4, 2, 4, true); else UP(8, 2, 4, true); }
+  // (The staged forms' registers leave a SIMD five waves in place of seven: they pay while an expert has few pairs.  Both products, two of 8
+  // experts, direct | staged: 1,536 and 2,240 beside 4,480, three rows 35.3 | 34.5, eight 41.7 | 41.9, sixteen 46.2 | 46.7; 3,584 and 9,472, four
+  // rows 188.4 | 185.0.)
+  else if (pairs <= 8) { if (hidden <= 1024) UP(4, 2, 1, true); else UP(8, 2, 1, true); }
+  else { if (hidden <= 1024) UP(4, 2, 1, false); else UP(8, 2, 1, false); }
   int status = LAUNCH_STATUS();
   if (status != 0) return status;
   if (inner <= 1024) DOWN(4); else DOWN(8);
