@@ -569,3 +569,39 @@ def test_norm_rotation_and_store_by_pieces(ops, n_q, n_k, n_v, d, dv, dims, norm
                           on(wq), on(wk), 1e-5)
     for mine, right in zip(got, want):                        # neighbours in bfloat16; angles of up to 4,095 in float32 (3e-4 of a radian)
         torch.testing.assert_close(mine.cpu().float(), right.float(), rtol=2.0 ** -7, atol=4e-3)
+
+
+# Two latents and a turned tail, a thread keeping one, two, four or eight of a latent's elements: latents on either side of each of those and longer than the
+# most that is kept, one of each far shorter than the other, a tail of none, of two, and of more pairs than threads, tokens that store nothing.
+@pytest.mark.parametrize("q_rank,kv_rank,rot", [(256, 1, 2), (257, 96, 0), (96, 513, 64), (1024, 1025, 16), (2049, 8, 600), (40, 2305, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("neighbours,values", [(False, True), (True, False)])
+def test_latents_kept_in_registers(ops, q_rank, kv_rank, rot, dtype, neighbours, values):
+    gen = torch.Generator().manual_seed(q_rank + kv_rank)
+    width, slots = kv_rank + rot, torch.tensor([3, -1, 47, 16, 0], dtype=torch.int32)
+    rows = torch.randn(5, 3 + q_rank + kv_rank + rot, generator=gen).to(dtype)
+    q_norm, kv_norm, rates = (torch.rand(n, generator=gen) + 0.2 for n in (q_rank, kv_rank, rot // 2))
+    positions = torch.tensor([0, 1, 63, 100, 17], dtype=torch.int32)
+    got_q = torch.full((5, q_rank), 7.0, dtype=dtype, device="cuda")
+    k_pages = torch.zeros(3, 1, 16, width, dtype=dtype, device="cuda")
+    v_pages = torch.zeros(3, 1, width, 16, dtype=dtype, device="cuda") if values else None
+    ops.latent_store(rows.cuda(), 3, q_rank, q_norm.cuda(), 3 + q_rank, kv_rank, kv_norm.cuda(), rot, rates.cuda() if rot else None, 1e-5,
+                     positions.cuda(), slots.cuda(), k_pages, v_pages, got_q, neighbours)
+    unit = lambda x, w: x / (x.square().mean(1, keepdim=True) + 1e-5).sqrt() * w.double()
+    x = rows.double()
+    want_q, kept = unit(x[:, 3:3 + q_rank], q_norm), unit(x[:, 3 + q_rank:3 + q_rank + kv_rank], kv_norm)
+    angles = (positions.float()[:, None] * rates[None, :]).double()       # the angle is a float product
+    tail, half = x[:, 3 + q_rank + kv_rank:], rot // 2
+    a, b = (tail[:, 0::2], tail[:, 1::2]) if neighbours else (tail[:, :half], tail[:, half:])
+    lo, hi = a * angles.cos() - b * angles.sin(), b * angles.cos() + a * angles.sin()
+    kept = torch.cat([kept, torch.stack([lo, hi], -1).flatten(1) if neighbours else torch.cat([lo, hi], 1)], 1)
+    want_k = torch.zeros(3 * 16, width, dtype=torch.float64)
+    for t, slot in enumerate(slots.tolist()):
+        if slot >= 0:
+            want_k[slot] = kept[t]
+    # A rounding to the type; in 32 bits sums of 2,305 squares and a root's and a quotient's roundings, 16 units of 2^-23 on values below 8.
+    tol = dict(rtol=2 ** -8, atol=1e-6) if dtype == torch.bfloat16 else dict(rtol=16 * 2 ** -23, atol=8 * 16 * 2 ** -23)
+    torch.testing.assert_close(got_q.double().cpu(), want_q, **tol)
+    torch.testing.assert_close(k_pages.double().cpu().reshape(48, width), want_k, **tol)
+    if values:
+        torch.testing.assert_close(v_pages.double().cpu()[:, 0].transpose(1, 2).reshape(48, width), want_k, **tol)

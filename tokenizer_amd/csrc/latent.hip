@@ -11,48 +11,85 @@
 // coordinates behind it in `rows` with coordinate i < rot / 2 and coordinate i + rot / 2 (neighbours: coordinates 2 i and
 // 2 i + 1) turned by the angle position * rates[i] (float).  It goes into key page [n_pages, 1, page_size, kv_rank + rot] at the token's slot and,
 // transposed inside a page, into value page [n_pages, 1, kv_rank + rot, page_size].  slots null or a negative slot:
-// nothing is stored; without value pages the row goes into its key page alone.  A workgroup a token.
-template <typename T>
+// nothing is stored; without value pages the row goes into its key page alone.
+// A workgroup a token and part (blockIdx.y: the queries' latent, the keys'); a thread keeps its PER elements in registers from their one
+// load on (what lies behind PER * LT_THREADS of a longer latent is read again), norm weights, position and rates are asked for beside them, and
+// the angles are the last wave's, which has the fewest elements.  (One workgroup for both parts one behind the other, each read twice | so, in a
+// graph: four rows of latents of 448 and 96 3.5 | 2.4 us, of 1,792 and 192 4.9 | 2.7, 2,000 rows of those 10.5 | 10.1.)
+template <typename T, int PER>
 __global__ void __launch_bounds__(LT_THREADS)
 latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, int q_rank, const float* __restrict__ q_norm,
                     int kv_offset, int kv_rank, const float* __restrict__ kv_norm, int rot, const float* __restrict__ rates,
                     float eps, const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ k_pages,
                     T* __restrict__ v_pages, int page_size, T* __restrict__ latent_q, int neighbours) {
+  HELD(rows, row_stride, q_offset, q_rank, q_norm, kv_offset, kv_rank, kv_norm, rot, rates, eps, positions, slots, k_pages, v_pages,
+       page_size, latent_q, neighbours);
   __shared__ float scratch[16];
   const int t = blockIdx.x;
+  const bool keys = blockIdx.y != 0;
+  const int slot = keys && slots ? scalar_int(slots + t) : -1;
+  if (keys && slot < 0) return;                               // (the same for every thread of the workgroup)
+  const int rank = keys ? kv_rank : q_rank;
   const T* row = rows + (size_t)t * row_stride;
+  const T* from = row + (keys ? kv_offset : q_offset);
+  const float* norm = keys ? kv_norm : q_norm;
+  T raw[PER];
+  float w[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = min(j * LT_THREADS + (int)threadIdx.x, rank - 1);
+    raw[j] = from[i];
+    w[j] = norm[i];
+  }
+  const int half = keys ? rot / 2 : 0, turn = (threadIdx.x + WAVE) % LT_THREADS;    // (the thread's pair of the tail: the last wave has the first)
+  const T* tail = row + kv_offset + kv_rank;
+  float rate = 0.f, position = 0.f;
+  T one_raw = {}, other_raw = {};
+  if (half > 0) {                                             // (the same for all)
+    const int i = min(turn, half - 1);
+    rate = rates[i];
+    one_raw = tail[neighbours ? 2 * i : i];
+    other_raw = tail[neighbours ? 2 * i + 1 : half + i];
+    position = (float)scalar_int(positions + t);
+  }
   float sq = 0.f;
-  for (int i = threadIdx.x; i < q_rank; i += LT_THREADS) { const float v = ld(row + q_offset + i); sq += v * v; }
-  const float inv_q = 1.0f / sqrtf(block_sum(sq, scratch) / (float)q_rank + eps);
-  for (int i = threadIdx.x; i < q_rank; i += LT_THREADS)
-    st(latent_q + (size_t)t * q_rank + i, ld(row + q_offset + i) * inv_q * q_norm[i]);
-  const int slot = slots ? slots[t] : -1;
-  if (slot < 0) return;                                       // (the same for every thread of the workgroup)
-  sq = 0.f;
-  for (int i = threadIdx.x; i < kv_rank; i += LT_THREADS) { const float v = ld(row + kv_offset + i); sq += v * v; }
-  const float inv_c = 1.0f / sqrtf(block_sum(sq, scratch) / (float)kv_rank + eps);
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const float v = ld(&raw[j]);
+    if (j * LT_THREADS + (int)threadIdx.x < rank) sq += v * v;
+  }
+  for (int i = PER * LT_THREADS + threadIdx.x; i < rank; i += LT_THREADS) { const float v = ld(from + i); sq += v * v; }
+  const float inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)rank + eps);
+  if (!keys) {
+    T* dst = latent_q + (size_t)t * q_rank;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int i = j * LT_THREADS + threadIdx.x;
+      if (i < rank) st(dst + i, ld(&raw[j]) * inv * w[j]);
+    }
+    for (int i = PER * LT_THREADS + threadIdx.x; i < rank; i += LT_THREADS) st(dst + i, ld(from + i) * inv * norm[i]);
+    return;
+  }
   const int page = slot / page_size, off = slot % page_size, width = kv_rank + rot;
   T* k_row = k_pages + ((size_t)page * page_size + off) * width;
   T* v_col = v_pages + (size_t)page * width * page_size + off;
-  for (int i = threadIdx.x; i < kv_rank; i += LT_THREADS) {
-    const float c = ld(row + kv_offset + i) * inv_c * kv_norm[i];
+  auto put = [&](int i, float c) {
     st(k_row + i, c);
     if (v_pages) st(v_col + (size_t)i * page_size, c);
+  };
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = j * LT_THREADS + threadIdx.x;
+    if (i < rank) put(i, ld(&raw[j]) * inv * w[j]);
   }
-  const int half = rot / 2;
-  const float position = (float)positions[t];
-  const T* tail = row + kv_offset + kv_rank;
-  for (int i = threadIdx.x; i < half; i += LT_THREADS) {
+  for (int i = PER * LT_THREADS + threadIdx.x; i < rank; i += LT_THREADS) put(i, ld(from + i) * inv * norm[i]);
+  for (int i = turn; i < half; i += LT_THREADS) {
+    if (i != turn) { rate = rates[i]; one_raw = tail[neighbours ? 2 * i : i]; other_raw = tail[neighbours ? 2 * i + 1 : half + i]; }
     float s, c;
-    sincosf(position * rates[i], &s, &c);
-    const int one = neighbours ? 2 * i : i, other = neighbours ? 2 * i + 1 : half + i;
-    const float a = ld(tail + one), b = ld(tail + other);
-    const float lo = a * c - b * s, hi = b * c + a * s;
-    st(k_row + kv_rank + one, lo);
-    st(k_row + kv_rank + other, hi);
-    if (!v_pages) continue;
-    st(v_col + (size_t)(kv_rank + one) * page_size, lo);
-    st(v_col + (size_t)(kv_rank + other) * page_size, hi);
+    sincosf(position * rate, &s, &c);
+    const float a = ld(&one_raw), b = ld(&other_raw);
+    put(kv_rank + (neighbours ? 2 * i : i), a * c - b * s);
+    put(kv_rank + (neighbours ? 2 * i + 1 : half + i), b * c + a * s);
   }
 }
 
@@ -192,12 +229,17 @@ head_linear_mfma_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride, i
 // exchanges (`wave_sums8`), and a lane a row stores: eight sums through the LDS crossbar and a lane's eight stores one behind the other were
 // half of the kernel, and the gate a kernel of its own.  (Us, one, four and eight rows, 14 heads of 64 over 128: 2.4, 3.3 and 4.5 without the
 // gate; 2.3, 2.8 and 3.4 so, 2.6, 3.1 and 3.7 with it; each sum by itself 2.2, 2.9 and 3.7.)
+// ROWS: the rows a wave asks for, all of them before the first is multiplied: one behind the other, behind a question whether there is a
+// further one, each was a trip.  One behind the other | so, one row, four and eight, 14 heads of 96 over 64: 2.6 | 2.0, 3.1 | 2.35 and
+// 3.8 | 2.7; 28 of 192 over 128, four rows 4.4 | 3.1, sixteen 7.1 | 5.5.  (The stores go through the chiplet's cache: a column's sixteen-bit
+// values lie apart, and each past the cache by itself cost 1.3 us.)
 #define HS_ROWS 8
-template <bool GATED>
+template <bool GATED, int ROWS>
 __global__ void __launch_bounds__(256)
 head_linear_skinny_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride, int x_offset, const bf16_t* __restrict__ W,
                           bf16_t* __restrict__ out, int out_row, int out_stride, int out_offset, int M, int N, int K,
                           const bf16_t* __restrict__ gate, int gate_row, int gate_head, int gate_unit) {
+  HELD(x, x_row, x_stride, x_offset, W, out, out_row, out_stride, out_offset, M, N, K, gate, gate_row, gate_head, gate_unit);
   const int h = blockIdx.z, lane = threadIdx.x & 63, n = blockIdx.x * 4 + wave_index(), m0 = blockIdx.y * HS_ROWS;
   if (n >= N) return;
   const bf16_t* a = x + (size_t)h * x_stride + x_offset;
@@ -208,12 +250,13 @@ head_linear_skinny_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride,
   float acc[HS_ROWS] = {};
   for (int k = lane * 8; k < K; k += 64 * 8) {
     const uint4 raw = *reinterpret_cast<const uint4*>(w + k);
+    uint4 xa[ROWS];                                          // (past the last row: the last one again, whose sum nobody stores)
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) xa[i] = *reinterpret_cast<const uint4*>(a + (size_t)min(m0 + i, M - 1) * x_row + k);
     const uint32_t ww[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
-    for (int i = 0; i < HS_ROWS; ++i) {
-      if (m0 + i >= M) break;
-      const uint4 xa = *reinterpret_cast<const uint4*>(a + (size_t)(m0 + i) * x_row + k);
-      const uint32_t xw[4] = {xa.x, xa.y, xa.z, xa.w};
+    for (int i = 0; i < ROWS; ++i) {
+      const uint32_t xw[4] = {xa[i].x, xa[i].y, xa[i].z, xa[i].w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         acc[i] = fmaf(__uint_as_float(ww[j] << 16), __uint_as_float(xw[j] << 16), acc[i]);
@@ -228,6 +271,18 @@ head_linear_skinny_kernel(const bf16_t* __restrict__ x, int x_row, int x_stride,
   }
 }
 
+template <bool GATED>
+static int launch_head_skinny(const void* x, int x_row, int x_stride, int x_offset, const void* W, void* out, int out_row, int out_stride,
+                              int out_offset, int M, int N, int K, int heads, const void* gate, int gate_row, int gate_head, int gate_unit,
+                              hipStream_t stream) {
+  const dim3 grid((N + 3) / 4, (M + HS_ROWS - 1) / HS_ROWS, heads);
+#define GO(ROWS) head_linear_skinny_kernel<GATED, ROWS><<<grid, 256, 0, stream>>>((const bf16_t*)x, x_row, x_stride, x_offset, (const bf16_t*)W, \
+    (bf16_t*)out, out_row, out_stride, out_offset, M, N, K, (const bf16_t*)gate, gate_row, gate_head, gate_unit)
+  if (M <= 1) GO(1); else if (M <= 2) GO(2); else if (M <= 4) GO(4); else GO(8);
+#undef GO
+  return LAUNCH_STATUS();
+}
+
 extern "C" int ta_latent_store(const void* rows, int row_stride, int q_offset, int q_rank, const void* q_norm, int kv_offset,
                                int kv_rank, const void* kv_norm, int rot, const void* rates, float eps, const void* positions,
                                const void* slots, void* k_pages, void* v_pages, int page_size, void* latent_q, int n_tokens,
@@ -235,11 +290,16 @@ extern "C" int ta_latent_store(const void* rows, int row_stride, int q_offset, i
   if (n_tokens <= 0) return 0;
   if (q_rank <= 0 || kv_rank <= 0 || rot < 0 || (rot & 1) || (rot > 0 && !rates) || (slots && (!k_pages || !kv_norm || page_size <= 0)))
     return -1;
-#define LS(TT) latent_store_kernel<TT><<<n_tokens, LT_THREADS, 0, stream>>>((const TT*)rows, row_stride, q_offset, q_rank, \
+  const int most = q_rank > kv_rank ? q_rank : kv_rank;
+  const dim3 grid(n_tokens, slots ? 2 : 1);
+#define LS_PER(TT, PER) latent_store_kernel<TT, PER><<<grid, LT_THREADS, 0, stream>>>((const TT*)rows, row_stride, q_offset, q_rank, \
     (const float*)q_norm, kv_offset, kv_rank, (const float*)kv_norm, rot, (const float*)rates, eps, (const int*)positions, \
     (const int*)slots, (TT*)k_pages, (TT*)v_pages, page_size, (TT*)latent_q, neighbours)
+#define LS(TT) do { if (most <= LT_THREADS) LS_PER(TT, 1); else if (most <= 2 * LT_THREADS) LS_PER(TT, 2); \
+                    else if (most <= 4 * LT_THREADS) LS_PER(TT, 4); else LS_PER(TT, 8); } while (0)
   if (dtype == DT_F32) LS(float); else LS(bf16_t);
 #undef LS
+#undef LS_PER
   return LAUNCH_STATUS();
 }
 
@@ -261,12 +321,9 @@ extern "C" int ta_head_linear(const void* x, int x_row, int x_stride, int x_offs
   if (K <= 0 || heads > 65535) return -1;
   if (dtype == DT_BF16 && K % 8 == 0 && x_row % 8 == 0 && x_stride % 8 == 0 && x_offset % 8 == 0 &&
       (((uintptr_t)x | (uintptr_t)W) & 15) == 0) {
-    if (M <= 2 * HS_ROWS) {
-      dim3 grid((N + 3) / 4, (M + HS_ROWS - 1) / HS_ROWS, heads);
-      head_linear_skinny_kernel<false><<<grid, 256, 0, stream>>>((const bf16_t*)x, x_row, x_stride, x_offset, (const bf16_t*)W,
-                                                                 (bf16_t*)out, out_row, out_stride, out_offset, M, N, K, nullptr, 0, 0, 0);
-      return LAUNCH_STATUS();
-    }
+    if (M <= 2 * HS_ROWS)
+      return launch_head_skinny<false>(x, x_row, x_stride, x_offset, W, out, out_row, out_stride, out_offset, M, N, K, heads, nullptr, 0, 0, 0,
+                                       stream);
     dim3 grid((N + 63) / 64, (M + 63) / 64, heads);
     if (grid.y > 65535) return -1;
     head_linear_mfma_kernel<<<grid, 256, 0, stream>>>((const bf16_t*)x, x_row, x_stride, x_offset, (const bf16_t*)W,
@@ -290,7 +347,6 @@ extern "C" int ta_head_linear_gated(const void* x, int x_row, int x_stride, int 
   if (M <= 0 || N <= 0 || heads <= 0) return 0;
   if (K <= 0 || heads > 65535 || !gate) return -1;
   if (dtype != DT_BF16 || M > 2 * HS_ROWS || K % 8 || x_row % 8 || x_stride % 8 || x_offset % 8 || (((uintptr_t)x | (uintptr_t)W) & 15)) return -2;
-  head_linear_skinny_kernel<true><<<dim3((N + 3) / 4, (M + HS_ROWS - 1) / HS_ROWS, heads), 256, 0, stream>>>((const bf16_t*)x, x_row, x_stride,
-      x_offset, (const bf16_t*)W, (bf16_t*)out, out_row, out_stride, out_offset, M, N, K, (const bf16_t*)gate, gate_row, gate_head, gate_unit);
-  return LAUNCH_STATUS();
+  return launch_head_skinny<true>(x, x_row, x_stride, x_offset, W, out, out_row, out_stride, out_offset, M, N, K, heads, gate, gate_row, gate_head,
+                                  gate_unit, stream);
 }
