@@ -605,3 +605,44 @@ def test_latents_kept_in_registers(ops, q_rank, kv_rank, rot, dtype, neighbours,
     torch.testing.assert_close(k_pages.double().cpu().reshape(48, width), want_k, **tol)
     if values:
         torch.testing.assert_close(v_pages.double().cpu()[:, 0].transpose(1, 2).reshape(48, width), want_k, **tol)
+
+
+# A matrix memory stepped a token at a time against the recurrence in 64 bits.  Widths on either side of the rows a thread holds and of the columns of a workgroup;
+# an entry that goes on, one that only fills the batch up, one that starts (in a state row full of NaN), state rows in another order.
+@pytest.mark.parametrize("heads,d,dv", [(1, 16, 16), (3, 33, 40), (2, 128, 256), (3, 72, 17), (1, 200, 3), (1, 256, 16)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_matrix_memory_of_single_tokens(ops, heads, d, dv, dtype):
+    gen = torch.Generator().manual_seed(d + dv)
+    slots, steps, cap = [2, 1, 0], 4, 15.0
+    keys, values = 2 * heads * d, heads * d * dv
+    state = torch.rand(3, values + heads * d + heads + 4, generator=gen)
+    state[0, :values + heads * d + heads] = float("nan")
+    held, ints = state.cuda(), lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    C, n, m = (state[[2, 0], a:b].double().reshape(2, heads, *shape) for a, b, shape in
+               ((0, values, (d, dv)), (values, values + heads * d, (d,)), (values + heads * d, values + heads * d + heads, ())))
+    C[1], n[1], m[1] = 0.0, 0.0, 0.0
+    # An exponent's argument (below 48) is rounded three times and a product twice a step; sums of d and of sixteen rows.
+    unit = (steps * (3 * 48 + 4) + d) * 2.0 ** -24
+    for i in range(steps):
+        x = torch.randn(2, keys + heads * dv + 5, generator=gen).to(dtype)
+        gates = 3 * torch.randn(2, 2 * heads + 1, generator=gen)
+        out = torch.full((2, heads * dv), 7.0, device="cuda")
+        ops.mlstm_scan(x.cuda(), gates.cuda(), held, ints([0, 1, 1, 2]), ints([7 + i, 0, i]), ints(slots), out, heads, d, dv, cap)
+        q, k = (x.double()[:, a:a + heads * d].reshape(2, heads, d) for a in (0, heads * d))
+        v, q = x.double()[:, keys:keys + heads * dv].reshape(2, heads, dv), q / d ** 0.5
+        g = cap * torch.tanh(gates.double() / cap)
+        gi, gf = g[:, :heads], torch.nn.functional.logsigmoid(g[:, heads:2 * heads])
+        after = torch.maximum(gf + m, gi)
+        keep, take = (gf + m - after).exp(), (gi - after).exp()
+        C = keep[..., None, None] * C + take[..., None, None] * k[..., :, None] * v[..., None, :]
+        n, m = keep[..., None] * n + take[..., None] * k, after
+        least = torch.maximum((n * q).sum(-1).abs(), (-m).exp()) + 1e-6
+        want = (C * q[..., None]).sum(-2) / least[..., None]
+        mags = [(a.abs().amax() * q.abs().sum(-1) / least)[..., None] for a in (C, n)]
+        slack = unit * (mags[0] + want.abs() * mags[1] + want.abs())
+        assert bool(((out.double().cpu().reshape(2, heads, dv) - want).abs() <= slack).all())
+    got = held[[2, 0]].double().cpu()
+    for a, want in ((0, C), (values, n), (values + heads * d, m)):
+        part = got[:, a:a + want[0].numel()].reshape(want.shape)
+        assert float((part - want).abs().max()) <= unit * max(1.0, float(want.abs().max()))
+    assert torch.equal(held[1].cpu(), state[1])
