@@ -25,10 +25,10 @@ __device__ __forceinline__ void st(bf16_t* p, float v) { p->bits = float_to_bf16
 
 // Stores past the caches of the chiplet that makes them (device scope): what a small kernel leaves is on its way to where the next
 // kernel's chiplets read it when the kernel ends, and the end has nothing to write back: 0.1 to 0.25 us of every launch that stores
-// a few KB (products of 896 columns, one row: q/k/v 3.83 -> 3.77 us, out 2.81 -> 2.63, gate/up 6.12 -> 6.01, down 4.59 -> 4.43, the four in
-// turn 17.5 -> 16.8).  For results of a few KB a chiplet whose lanes store side by side; a store of its own for every value of
-// a scattered result costs more this way than the write-back (four values a lane: q/k/v 4.6 -> 5.5).  Nontemporal stores do not do: of
-// single 16-bit values they cost 10 us.
+// a few KB (products of 896 columns, one row: out 2.81 -> 2.65 us, gate/up 6.12 -> 6.03, down 4.59 -> 4.44).  For results of a few KB a
+// chiplet whose lanes store side by side; a store of its own for every value of a scattered result costs more this way than the
+// write-back (four values a lane: q/k/v 4.6 -> 5.5; head products, whose 16-bit values lie apart, 1.3 us).  What the same chiplet reads
+// again soon stays in its cache by plain stores (streams).  Nontemporal stores do not do: of single 16-bit values they cost 10 us.
 __device__ __forceinline__ void st_through(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -49,9 +49,7 @@ struct RopeStore {
 // rows outweigh a tile's weights (what comes over the fabric from the caches counts like what comes from memory).
 // LINES > 0: the weights are read line by line (`lines_to_rows` in common.h), K walked in steps of 64, LINES steps at a time, past the
 // caches (a stream that does not come again): for products that are one long stream over a big matrix.  WHOLE: K is a multiple of 64.
-// SUMS 2 (with WHOLE): a wave keeps the sums of two waves of half lines, a line's first 32 elements of K and its second, so that a
-// product has the same bits whichever way its weights come.
-template <int MB, int NW, bool GATED, typename OutT, bool ROPE = false, int NB = 1, int LINES = 0, bool WHOLE = false, int SUMS = 1>
+template <int MB, int NW, bool GATED, typename OutT, bool ROPE = false, int NB = 1, int LINES = 0, bool WHOLE = false>
 __global__ void __launch_bounds__(NW * WAVE)
 skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf16_t* __restrict__ W,
                    OutT* __restrict__ C, int ldc, int M, int N, int K_all, float* __restrict__ partial,
@@ -63,8 +61,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
   static_assert(!ROPE || NB == 1, "the rotation pairs rows within one block");
   constexpr int HALVES = GATED ? 2 : 1;                     // gate and up rows (or the two halves of a head)
   constexpr int SETS = HALVES * NB;                         // set h * NB + b: half h, column block b
-  static_assert(SUMS == 1 || (SUMS == 2 && LINES > 0 && WHOLE), "two sums a wave: whole lines, a sum for each half");
-  __shared__ float red[NW * SUMS][HALVES * MB * 4][WAVE];
+  __shared__ float red[NW][HALVES * MB * 4][WAVE];
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int col = lane & 15, g = lane >> 4;
   const int n_out = ROPE ? N : GATED ? N / 2 : N;
@@ -98,19 +95,15 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
     a_row[mb] = A + (size_t)min(m_base + mb * 16 + col, M - 1) * lda + k_lo + 8 * g;
   }
 
-  floatx4 sums[SUMS][SETS][MB];
-  floatx4 (&acc)[SETS][MB] = sums[0];
+  floatx4 acc[SETS][MB];
 #pragma unroll
-  for (int i = 0; i < SUMS; ++i)
+  for (int s = 0; s < SETS; ++s)
 #pragma unroll
-    for (int s = 0; s < SETS; ++s)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) sums[i][s][mb] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    for (int mb = 0; mb < MB; ++mb) acc[s][mb] = (floatx4){0.f, 0.f, 0.f, 0.f};
 
   constexpr int UN = (SETS * MB > 4) ? 2 : 4;
   if constexpr (LINES > 0) {
-    const int sub = col & 7, piece = SUMS == 2 ? g + 4 * (col >> 3) : 2 * g + (col >> 3);
-    const int a_first = SUMS == 2 ? 8 * g : 16 * g, a_apart = SUMS == 2 ? 32 : 8;    // the rows' elements of the line that meet the weights'
+    const int sub = col & 7, piece = 2 * g + (col >> 3);
     const bool low_lane = col < 8;
     const bf16_t* wl[SETS][2];
 #pragma unroll
@@ -144,7 +137,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) {         // (`a_row` is 8 g on already)
-            const int place = at + a_first + hh * a_apart;
+            const int place = at + 16 * g + hh * 8;
             af[q][mb][hh] = load8(a_row[mb] + place - 8 * g, valid && a_ok[mb] && (WHOLE || place < K));
           }
       }
@@ -157,7 +150,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) {
             acc[s][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, af[q][mb][0], acc[s][mb], 0, 0, 0);
-            sums[SUMS - 1][s][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, af[q][mb][1], sums[SUMS - 1][s][mb], 0, 0, 0);
+            acc[s][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, af[q][mb][1], acc[s][mb], 0, 0, 0);
           }
         }
       }
@@ -209,13 +202,11 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
   const int n0 = n_first + 16 * b;
   if (b > 0) __syncthreads();                                   // the block before has been read
 #pragma unroll
-  for (int i = 0; i < SUMS; ++i)
+  for (int h = 0; h < HALVES; ++h)
 #pragma unroll
-    for (int h = 0; h < HALVES; ++h)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) red[wave * SUMS + i][(h * MB + mb) * 4 + r][lane] = sums[i][h * NB + b][mb][r];
+      for (int r = 0; r < 4; ++r) red[wave][(h * MB + mb) * 4 + r][lane] = acc[h * NB + b][mb][r];
   __syncthreads();
   // Lane (col, g) of block mb holds C^T rows n0 + 4g + r (r = 0..3), column m = mb*16 + col.
   for (int item = threadIdx.x; item < MB * WAVE; item += NW * WAVE) {
@@ -228,7 +219,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
     for (int r = 0; r < 4; ++r) {
       float sum0 = 0.f, sum1 = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW * SUMS; ++w) {
+      for (int w = 0; w < NW; ++w) {
         sum0 += red[w][mb * 4 + r][ln];
         if (GATED) sum1 += red[w][(MB + mb) * 4 + r][ln];
       }
@@ -552,7 +543,7 @@ static int column_blocks(int asked, int M, int n_out, int splits) {
 static int g_lines = 1;
 extern "C" void ta_skinny_lines(int on) { g_lines = on; }
 
-template <int MB, int NW, bool GATED, int NB = 1, int LINES = 0, bool WHOLE = false, int SUMS = 1>
+template <int MB, int NW, bool GATED, int NB = 1, int LINES = 0, bool WHOLE = false>
 static int launch_skinny(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int M, int N,
                          int K, int out_dtype, hipStream_t stream, int splits = 1, void* partial = nullptr, int gate_act = 0) {
   const int n_out = GATED ? N / 2 : N;
@@ -562,10 +553,10 @@ static int launch_skinny(const void* A, int lda, const void* W, const void* bias
   const dim3 grid((n_out + 16 * NB - 1) / (16 * NB), splits);
   float* slabs = splits > 1 ? (float*)partial : nullptr;
   if (out_dtype == DT_F32)
-    skinny_gemm_kernel<MB, NW, GATED, float, false, NB, LINES, WHOLE, SUMS><<<grid, NW * WAVE, 0, stream>>>(
+    skinny_gemm_kernel<MB, NW, GATED, float, false, NB, LINES, WHOLE><<<grid, NW * WAVE, 0, stream>>>(
         (const bf16_t*)A, lda, k_chunk, (const bf16_t*)W, (float*)C, ldc, M, N, K, slabs, (const float*)bias, RopeStore(), gate_act);
   else
-    skinny_gemm_kernel<MB, NW, GATED, bf16_t, false, NB, LINES, WHOLE, SUMS><<<grid, NW * WAVE, 0, stream>>>(
+    skinny_gemm_kernel<MB, NW, GATED, bf16_t, false, NB, LINES, WHOLE><<<grid, NW * WAVE, 0, stream>>>(
         (const bf16_t*)A, lda, k_chunk, (const bf16_t*)W, (bf16_t*)C, ldc, M, N, K, slabs, (const float*)bias, RopeStore(), gate_act);
   int status = LAUNCH_STATUS();
   if (status == 0 && splits > 1 && C) status = launch_splitk_reduce(slabs, bias, C, M, N, ldc, splits, out_dtype, stream);
