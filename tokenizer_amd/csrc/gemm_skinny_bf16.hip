@@ -293,6 +293,8 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
 // * STAGE > 0 (up to eight rows): a wave brings a trip's share of the rows in STAGE loads of sixteen different bytes a lane and turns
 //   them into fragments through a part of LDS that is its own; a fragment straight from memory is a load that holds up the memory
 //   pipeline like any other though its lanes mostly ask for the same bytes.
+// SUMS 2 (with whole lines): a wave keeps the sums of two waves of half lines, a line's first 32 elements of K and its second, so that a
+// product has the same bits whichever way its weights come.
 // Which wave takes which steps of K does not hang on any of this, nor does a result.
 // Us, weights from memory, sixteen rows a workgroup with four outputs a lane | so, one row, eight and sixteen: 896 over 896 3.5 | 3.0, 3.9 | 3.2
 // and 4.15 | 3.6; 896 over 4,864 8.1 | 5.7, 9.7 | 5.8 and 11.2 | 8.3; 1,536 over 1,536 4.5 | 3.6, 5.1 | 3.8 and 5.6 | 4.6; 1,536 over 8,960 12.6 | 9.3,
