@@ -1,5 +1,7 @@
 """In which order the products of few rows and the sums over a wave add up.  Reading the weights by whole cache lines, or a sum through
 other instructions, must leave the sums as they were: a product's bits decide a router's near ties, and with them whole rows of logits."""
+from ctypes import c_void_p
+
 import pytest
 import torch
 
@@ -97,3 +99,23 @@ def test_experts_of_one_row_and_of_many_have_the_same_bits(ops, hidden, inner, s
                                        second, shared=shared).partial
     many, one = run(16), run(1)
     assert many.isfinite().all() and torch.equal(many[:, :1], one)
+
+
+def test_merged_parts_join_their_neighbours_in_one_rounding(ops):
+    # Part 0 has x, part 1 -x under the same weight w = exp(-0.3): joined in one rounding, x w - round(x w) is what the rounding left, at most
+    # half a unit in the last place of a product below 4; joined after two roundings it is zero.  Part 2 has the largest maximum and the
+    # whole denominator, so that the result is the sum itself.
+    heads, splits = 3, 4
+    for d, single in ((32, True), (64, True), (96, False), (128, False)):
+        part_o = torch.zeros((16, heads, splits, d), device="cuda")
+        part_o[:, :, 0] = torch.rand((16, heads, d), generator=torch.Generator(device="cuda").manual_seed(d), device="cuda") + 1
+        part_o[:, :, 1] = -part_o[:, :, 0]
+        part_ml = torch.zeros((16, heads, splits, 2), device="cuda")
+        part_ml[:, :, :2, 0], part_ml[:, :, 3, 0], part_ml[:, :, 2, 1] = -0.3, -0.3, 1.0
+        ints = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+        tiles, cu_q = ints(0, 0), ints(0, 16)
+        out = torch.full((16, heads * d), 7.0, dtype=torch.bfloat16, device="cuda")
+        assert ops.lib.ta_attention_merge_tiles(*(c_void_p(t.data_ptr()) for t in (part_o, part_ml, tiles)), 1, c_void_p(cu_q.data_ptr()),
+                                                c_void_p(out.data_ptr()), heads, d, splits, ops._stream()) == 0
+        assert bool((out.abs() <= 2.0 ** -23).all())
+        assert float((out != 0).float().mean()) > 0.9 if single else not out.any()

@@ -430,13 +430,20 @@ decode_attention_merge(const float* __restrict__ part_o, const float* __restrict
     if constexpr (LANES <= 16) all_big = wave_max_across<16>(all_big);
     if constexpr (LANES <= 32) all_big = wave_max_across<32>(all_big);
     const float w = (big == -INFINITY) ? 0.f : __expf(big - all_big);
-    auto across = [](float x) {
-      if constexpr (LANES <= 16) x = wave_add_across<16>(x);
-      if constexpr (LANES <= 32) x = wave_add_across<32>(x);
-      return x;
+    // (Groups of sixteen lanes: a group's own product joins the neighbour's rounded one in one rounding, as `fmaf` says.  The second
+    // register of a swap of rows is the neighbour's in rows 0 and 2, which are those that group 0's sums come from.)
+    auto across = [w](float x) {
+      float sum = x * w;
+      if constexpr (LANES <= 16) {
+        float neighbour = sum;
+        wave_swap16(sum, neighbour);
+        sum = fmaf(x, w, neighbour);
+      }
+      if constexpr (LANES <= 32) sum = wave_add_across<32>(sum);
+      return sum;
     };
-    o.x = across(o.x * w); o.y = across(o.y * w); o.z = across(o.z * w); o.w = across(o.w * w);
-    denom = across(denom * w);
+    o.x = across(o.x); o.y = across(o.y); o.z = across(o.z); o.w = across(o.w);
+    denom = across(denom);
     if (grp == 0 && e < d) {
       const float inv = 1.0f / denom;
       bf16_t* dst = out + (size_t)t * n_q * d + (size_t)head * d + e;
