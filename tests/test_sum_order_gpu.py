@@ -119,3 +119,24 @@ def test_merged_parts_join_their_neighbours_in_one_rounding(ops):
                                                 c_void_p(out.data_ptr()), heads, d, splits, ops._stream()) == 0
         assert bool((out.abs() <= 2.0 ** -23).all())
         assert float((out != 0).float().mean()) > 0.9 if single else not out.any()
+
+
+@pytest.mark.parametrize("heads,d,dv", [(1, 16, 16), (3, 33, 40), (2, 128, 256), (1, 256, 17)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_matrix_memory_of_tokens_one_by_one_has_the_bits_of_a_walk(ops, heads, d, dv, dtype):
+    # Tokens a step each and all of them in one portion; one request from its start and one that goes on.
+    steps, cap, width = 6, 15.0, heads * (2 * d + dv)
+    gen = torch.Generator(device="cuda").manual_seed(d + dv)
+    x = torch.randn((2, steps, width), generator=gen, device="cuda").to(dtype)
+    gates = 3 * torch.randn((2, steps, 2 * heads), generator=gen, device="cuda")
+    start = torch.rand((2, heads * (d * dv + d + 1)), generator=gen, device="cuda")
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    walked, stepped = start.clone(), start.clone()
+    want, got = (torch.empty((2, steps, heads * dv), device="cuda") for _ in range(2))
+    ops.mlstm_scan(x.reshape(2 * steps, width), gates.reshape(2 * steps, -1), walked, ints(0, steps, 2 * steps), ints(0, 9), ints(1, 0),
+                   want.view(2 * steps, -1), heads, d, dv, cap)
+    for i in range(steps):
+        out = torch.empty((2, heads * dv), device="cuda")
+        ops.mlstm_scan(x[:, i].contiguous(), gates[:, i].contiguous(), stepped, ints(0, 1, 2), ints(i, 9 + i), ints(1, 0), out, heads, d, dv, cap)
+        got[:, i] = out
+    assert want.isfinite().all() and torch.equal(got, want) and torch.equal(stepped, walked)

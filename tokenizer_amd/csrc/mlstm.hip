@@ -58,7 +58,9 @@ mlstm_gates_kernel(const T* __restrict__ qkvg, int row_stride, const float* __re
     const T q_raw = x[(size_t)h * d + j], k_raw = x[(size_t)(heads + h) * d + j];
     const float n_raw = n_state[j], m_raw = *m_state;
     const float gi_raw = gates[(size_t)lo * gate_stride + h], gf_raw = gates[(size_t)lo * gate_stride + heads + h];
-    const float m = fresh ? 0.f : m_raw, gi = capped(gi_raw, cap), gf = log_sigmoid(capped(gf_raw, cap));
+    const float m = fresh ? 0.f : m_raw, gf = log_sigmoid(capped(gf_raw, cap));
+    float gi = capped(gi_raw, cap);
+    asm volatile("" : "+v"(gi));                             // (rounded here, as in the walk over a group: not one rounding with what is taken off it)
     const float m_new = fmaxf(gf + m, gi);
     const float keep = expf(gf + m - m_new), take = expf(gi - m_new), least = expf(-m_new);
     const float n = fmaf(keep, fresh || tid >= d ? 0.f : n_raw, take * (tid < d ? ld(&k_raw) : 0.f));
