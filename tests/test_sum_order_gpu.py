@@ -140,3 +140,29 @@ def test_matrix_memory_of_tokens_one_by_one_has_the_bits_of_a_walk(ops, heads, d
         ops.mlstm_scan(x[:, i].contiguous(), gates[:, i].contiguous(), stepped, ints(0, 1, 2), ints(i, 9 + i), ints(1, 0), out, heads, d, dv, cap)
         got[:, i] = out
     assert want.isfinite().all() and torch.equal(got, want) and torch.equal(stepped, walked)
+
+
+# Rows in LDS at eight waves by lines (K 2,112, or float rows), at four waves and by half lines, and rows straight from memory (16 of 4,096).
+@pytest.mark.parametrize("rows,k,waves,sine_first", [(1, 2112, 8, True), (16, 2112, 8, True), (1, 2112, 4, False), (3, 2120, 8, False),
+                                                     (8, 896, 8, False), (2, 1536, 8, False), (16, 4096, 8, True), (16, 4096, 4, False),
+                                                     (16, 4104, 8, False)])
+def test_rotation_rounds_the_products_it_did(ops, rows, k, waves, sine_first):
+    # Both elements of a pair are x (exact).  Sine s, cosine -s: the second result is what the rounding of one product left, its sign says
+    # of which; sine and cosine s: the first is x s - round(x s).  x has 8 bits, s 24, so that what is left is a bfloat16.
+    heads, kv, d = 2, 1, 64
+    x = rand((rows, k), 5)
+    w = torch.zeros(((heads + 2 * kv) * d, k), dtype=torch.bfloat16, device="cuda")
+    w[:, 0] = 1
+    s = torch.rand((1, d // 2), generator=torch.Generator(device="cuda").manual_seed(6), device="cuda") + 0.5
+    product = x[:, :1].double() * s.double()
+    left = (product - product.float().double()).float()       # x s - round(x s)
+    assert float((left != 0).float().mean()) > 0.5
+    positions = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    ops.fused_waves = waves
+    try:
+        run = lambda cosine: ops.fused_norm_qkv_rope(x, None, 0.0, w, None, positions, torch.cat([cosine, s], 1), None, None, None, heads, kv, d)
+        opposed, alike = (run(c).float().view(rows, heads, 2, d // 2) for c in (-s, s))
+    finally:
+        ops.fused_waves = 0
+    assert torch.equal(alike[:, :, 0], left[:, None].expand(-1, heads, -1))
+    assert torch.equal(opposed[:, :, 1], (-left if sine_first else left)[:, None].expand(-1, heads, -1))

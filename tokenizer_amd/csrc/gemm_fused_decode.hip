@@ -488,8 +488,10 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
         if (paired) {
           const int hd = row0 / d, i = row0 % d + er;               // element i (< half) of head hd, and i + half
           const float x1 = v0 + pre_a[0], x2 = v1 + pre_b[0];
-          const float r1 = x1 * pre_cos - x2 * pre_sin;             // cos 1, sin 0 without a rotation
-          const float r2 = x2 * pre_cos + x1 * pre_sin;
+          // cos 1, sin 0 without a rotation.  Which product is rounded before the other joins it is written down, so that it stays as it
+          // is when the code around it changes (the compiler joins either; its choice in the instances of eight waves by lines is the other).
+          const float r1 = fmaf(x1, pre_cos, -(x2 * pre_sin));
+          const float r2 = NW == 8 && LINES ? fmaf(x2, pre_cos, x1 * pre_sin) : fmaf(x1, pre_sin, x2 * pre_cos);
           bf16_t* dst = nullptr;
           if (hd < p.n_q) dst = p.out + (size_t)em * p.ldc + (size_t)hd * d + i;
           else if (slot >= 0) dst = p.k_pages + (((size_t)page * p.n_kv + (hd - p.n_q)) * p.page_size + off) * d + i;
