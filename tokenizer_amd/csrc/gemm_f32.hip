@@ -339,7 +339,8 @@ struct F32Store {
 };
 
 // PLAIN and ROPE take fewer rows a workgroup (`tile_rows` in all: down to four; of each half with ROPE: down to two) where sixteen (eight) are
-// fewer workgroups than compute units; lanes of rows past them load nothing and only feed sums that nobody reads.
+// fewer workgroups than compute units.  Rows of the sixteen past them repeat the last one (lanes that read by lines load nothing for
+// them): a matrix's places are all that is read, and what is made of them feeds sums that nobody reads.
 // STAGE > 0 (LINES, up to four rows for one and up to eight for two): a wave brings a pair of units of A's rows in STAGE loads of sixteen
 // different bytes a lane and turns them into fragments through a part of LDS of its own; a fragment straight from memory is a load
 // that holds up the memory pipeline like any other though its lanes mostly ask for the same bytes.
@@ -348,6 +349,32 @@ struct F32Store {
 // 7.4 | 6.3 and 7.7 | 7.0.)
 enum { ROWS_PLAIN = 0, ROWS_GATED = 1, ROWS_ROPE = 2 };
 
+// Where workgroup `block`'s weight rows lie in a matrix of n: row i (0 .. 15) of its tile, with two halves row i & 7 of the first or (i >= 8) of the second.
+template <int KIND>
+struct RowTile {
+  int head, first_in, n0, half, limit, rows;                // (head, first_in: ROPE, the head and the tile's place in its first half)
+  __host__ __device__ RowTile(int block, int n, int tile_rows, int d) : rows(tile_rows) {
+    const int per_head = KIND == ROWS_ROPE ? d / 2 / rows : 1;
+    head = KIND == ROWS_ROPE ? block / per_head : 0;
+    first_in = KIND == ROWS_ROPE ? block % per_head * rows : 0;
+    half = KIND == ROWS_ROPE ? d / 2 : n / 2;
+    n0 = KIND == ROWS_ROPE ? head * d + first_in : block * rows;
+    limit = KIND == ROWS_GATED ? half : n;
+  }
+  __host__ __device__ int place(int i) const { return KIND == ROWS_PLAIN ? i : i & 7; }
+  __host__ __device__ bool there(int i) const { return place(i) < rows; }
+  __host__ __device__ int row(int i) const {
+    const int at = n0 + (there(i) ? place(i) : rows - 1);
+    return (at < limit ? at : limit - 1) + (KIND != ROWS_PLAIN && i >= 8 ? half : 0);
+  }
+};
+
+// The row of the matrix that row i of a workgroup's tile is read from (`kind`: the enumeration above), as the kernel below has it.
+extern "C" int ta_gemm_f32_tile_row(int kind, int block, int n, int tile_rows, int d, int i) {
+  return kind == ROWS_ROPE ? RowTile<ROWS_ROPE>(block, n, tile_rows, d).row(i)
+         : kind == ROWS_GATED ? RowTile<ROWS_GATED>(block, n, tile_rows, d).row(i) : RowTile<ROWS_PLAIN>(block, n, tile_rows, d).row(i);
+}
+
 template <int KIND, bool LINES, int STAGE>
 __global__ void __launch_bounds__(512)
 gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, uint32_t m_rows_d, int N, int K, int lda, int units_part,
@@ -355,33 +382,24 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, u
                      const F32Store store = F32Store()) {
   HELD(A, W, m_rows_d, N, K, lda, units_part, bias, partial);                // (the words that are there when a wave starts)
   constexpr int WAVES = 8, PAIR = 2, ROW_BYTES = PAIR * 128 + 16;
-  constexpr bool HALVES = KIND != ROWS_PLAIN;               // weight rows here and as many a fixed way further on
   static_assert(STAGE == 0 || LINES, "rows are staged line by line");
   __shared__ float sums[WAVES][16][17];
   __shared__ __attribute__((aligned(16))) char rows_s[STAGE > 0 ? WAVES * 4 * STAGE * ROW_BYTES : 16];
   const int M = m_rows_d & 0xff, tile_rows = (m_rows_d >> 8) & 0xff, d = m_rows_d >> 16;    // (d: ROPE)
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int row = lane & 15, g = lane >> 4;
-  const int per_head = KIND == ROWS_ROPE ? d / 2 / tile_rows : 1;
-  const int head = KIND == ROWS_ROPE ? blockIdx.x / per_head : 0, first_in = KIND == ROWS_ROPE ? blockIdx.x % per_head * tile_rows : 0;
-  const int half = KIND == ROWS_ROPE ? d / 2 : N / 2;
-  const int n0 = KIND == ROWS_ROPE ? head * d + first_in : blockIdx.x * tile_rows;
-  const int limit = KIND == ROWS_GATED ? half : N;
-  // The weight row behind row i (0 .. 15) of the tile, and whether it is there.
-  auto weight_row = [&](int i) {
-    return HALVES ? min(n0 + (i & 7), limit - 1) + (i < 8 ? 0 : half) : min(n0 + i, N - 1);
-  };
-  auto there = [&](int i) { return (HALVES ? i & 7 : i) < tile_rows; };
+  const RowTile<KIND> tile(blockIdx.x, N, tile_rows, d);
+  const int head = tile.head, first_in = tile.first_in, half = tile.half, n0 = tile.n0;
   const int units = (K + 31) / 32;
   const int u_begin = blockIdx.y * units_part, u_end = min(units, u_begin + units_part);
   const int a_m = min(row, M - 1);
   const float* a_row = A + (size_t)a_m * lda;
   const float* w_row[2];
   bool w_ok[2];
-  w_row[0] = W + (size_t)weight_row(LINES ? row & 7 : row) * K;
-  w_row[1] = LINES ? W + (size_t)weight_row(8 + (row & 7)) * K : w_row[0];
-  w_ok[0] = there(LINES ? row & 7 : row);
-  w_ok[1] = LINES ? there(8 + (row & 7)) : w_ok[0];
+  w_row[0] = W + (size_t)tile.row(LINES ? row & 7 : row) * K;
+  w_row[1] = LINES ? W + (size_t)tile.row(8 + (row & 7)) * K : w_row[0];
+  w_ok[0] = tile.there(LINES ? row & 7 : row);
+  w_ok[1] = LINES ? tile.there(8 + (row & 7)) : w_ok[0];
   const int piece = 2 * g + (row >> 3);
   char* mine = rows_s + (STAGE > 0 ? wave * M * ROW_BYTES : 0);
   f32x4 w[2][PAIR][2], a[2][PAIR][2], staged[2][STAGE > 0 ? STAGE : 1];
