@@ -166,3 +166,26 @@ def test_rotation_rounds_the_products_it_did(ops, rows, k, waves, sine_first):
         ops.fused_waves = 0
     assert torch.equal(alike[:, :, 0], left[:, None].expand(-1, heads, -1))
     assert torch.equal(opposed[:, :, 1], (-left if sine_first else left)[:, None].expand(-1, heads, -1))
+
+
+# Rows of one, two and four pieces a thread, the product in parts and as it is, results of both types.
+@pytest.mark.parametrize("hidden,post_groups,groups", [(896, 2, 2), (1024, 1, 4), (1536, 2, 2), (4096, 8, 2)])
+@pytest.mark.parametrize("parts", [0, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_grouped_norm_joins_the_stream_in_one_rounding(ops, hidden, post_groups, groups, parts, dtype):
+    from tokenizer_amd.kernels import PendingSum
+    gen = torch.Generator(device="cuda").manual_seed(hidden + parts)
+    slabs = torch.randn((max(1, parts), 3, hidden), generator=gen, device="cuda")
+    delta = PendingSum(ops, slabs, None, dtype) if parts else slabs[0].to(dtype)
+    behind = 1 + 0.3 * torch.randn(hidden, generator=gen, device="cuda")
+
+    def stream_after(before, weight, normed=True):
+        kept, out = before.clone(), torch.empty((3, hidden), dtype=dtype, device="cuda")
+        ops.norm_add_rmsnorm(kept, delta, weight, 1e-5, torch.ones_like(behind) if normed else None, 1e-5, out, post_groups=post_groups, groups=groups)
+        return kept
+    nothing = torch.zeros((3, hidden), device="cuda")
+    factor = stream_after(nothing, torch.ones_like(behind))   # the product over its root mean square, rounded
+    rounded = stream_after(nothing, behind)
+    left = (factor.double() * behind.double() - rounded.double()).float()      # (exact: 48 bits without their first 24)
+    assert float((left != 0).float().mean()) > 0.9
+    assert torch.equal(stream_after(-rounded, behind), left) and torch.equal(stream_after(-rounded, behind, False), left)

@@ -904,8 +904,9 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
     if (h >= hidden) continue;
     if (post_weight) {
       const float f = inv[post_of[c]];
-      x[c].x += d[c].x * f * behind_w[c].x; x[c].y += d[c].y * f * behind_w[c].y;
-      x[c].z += d[c].z * f * behind_w[c].z; x[c].w += d[c].w * f * behind_w[c].w;
+      // (One rounding, written down: behind a sum that both branches share, the compiler rounds the product as well.)
+      x[c].x = fmaf(d[c].x * f, behind_w[c].x, x[c].x); x[c].y = fmaf(d[c].y * f, behind_w[c].y, x[c].y);
+      x[c].z = fmaf(d[c].z * f, behind_w[c].z, x[c].z); x[c].w = fmaf(d[c].w * f, behind_w[c].w, x[c].w);
     } else if (PARTS || delta) {
       x[c].x += d[c].x; x[c].y += d[c].y; x[c].z += d[c].z; x[c].w += d[c].w;
     }
