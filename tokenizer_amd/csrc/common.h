@@ -49,6 +49,14 @@ __device__ __forceinline__ void st_through(uint2* p, uint2 v) {          // (eig
 // from threadIdx) can end up as exactly that.
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// Between stores of a wave's lanes to LDS and reads of what other lanes of the same wave stored there, and between those reads and the next
+// stores to the place.  LDS serves a wave's instructions in their order, so nothing is waited for; the compiler, which looks at one lane
+// alone, must not move the one past the other.
+__device__ __forceinline__ void wave_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // HELD(a, b, ...): the listed kernel arguments are in scalar registers from this point on.  Left to itself the compiler
 // fetches each piece of the argument block where it is first used, with a wait each time; a kernel that lists its
 // arguments once, at its start, fetches them all in one trip.  (One statement for all of them: the fetches of a

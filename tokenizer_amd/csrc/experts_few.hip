@@ -91,10 +91,12 @@ __device__ __forceinline__ void ef_walk_form(const bf16_t* const (&w_at)[HALVES]
         if (k >= K) staged[j] = zero;
         *reinterpret_cast<word4*>(stage + i / PIECES * ROW_BYTES + i % PIECES * 16) = staged[j];
       }
+      wave_exchange();
 #pragma unroll
       for (int q = 0; q < UN; ++q)
 #pragma unroll
         for (int s = 0; s < 2; ++s) xf[q][s] = *reinterpret_cast<const word4*>(stage + min(col, here - 1) * ROW_BYTES + q * 128 + s * 64 + g * 16);
+      wave_exchange();                                       // (the next trip's pieces are stored behind these reads)
     }
 #pragma unroll
     for (int q = 0; q < UN; ++q)

@@ -487,10 +487,12 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, u
           if (now + ((i & 15) >> 3) * WAVES >= u_end) staged[slot][j] = f32x4{0.f, 0.f, 0.f, 0.f};
           *reinterpret_cast<f32x4*>(mine + (i >> 4) * ROW_BYTES + (i & 15) * 16) = staged[slot][j];
         }
+        wave_exchange();
 #pragma unroll
         for (int p = 0; p < PAIR; ++p)
 #pragma unroll
           for (int h = 0; h < 2; ++h) a[slot][p][h] = *reinterpret_cast<const f32x4*>(mine + a_m * ROW_BYTES + p * 128 + 32 * g + 16 * h);
+        wave_exchange();                                     // (the next pair's pieces are stored behind these reads)
       }
 #pragma unroll
       for (int p = 0; p < PAIR; ++p) {

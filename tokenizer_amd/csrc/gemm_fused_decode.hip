@@ -344,6 +344,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
       const int i = min(j * WAVE + lane, M * PIECES - 1);
       *reinterpret_cast<word4*>(mine + i / PIECES * ROW_BYTES + i % PIECES * 16) = staged[j];
     }
+    wave_exchange();
 #pragma unroll
     for (int u = 0; u < UN; ++u) af_one[u] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const word4*>(mine + a_m * ROW_BYTES + u * 64 + 16 * g));
   }

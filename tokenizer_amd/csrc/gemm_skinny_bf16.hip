@@ -347,6 +347,7 @@ few_rows_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
       if (stage_k[j] >= K) staged[j] = (word4){0u, 0u, 0u, 0u};
       *reinterpret_cast<word4*>(mine + i / PIECES * ROW_BYTES + i % PIECES * 16) = staged[j];
     }
+    wave_exchange();
   };
   auto fragment = [&](int byte) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const word4*>(mine + a_m * ROW_BYTES + byte)); };
 
@@ -401,6 +402,7 @@ few_rows_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
         for (int q = 0; q < LINES; ++q)
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) af[q][hh] = fragment(q * 128 + 2 * (a_first + hh * a_apart));
+        wave_exchange();                                    // (the next trip's pieces are stored behind these reads)
       }
 #pragma unroll
       for (int q = 0; q < LINES; ++q) {
@@ -440,6 +442,7 @@ few_rows_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
           af[u] = fragment(u * 64 + 16 * g);
           if (ks + u * NW >= full_steps) af[u] = load8(nullptr, false);   // (the tail of K has weights of its own)
         }
+        wave_exchange();
       }
 #pragma unroll
       for (int u = 0; u < TRIP; ++u)
