@@ -414,6 +414,31 @@ def test_choice_counted_is_choice_searched(ops, experts, groups, keep, top, soft
         assert torch.allclose(got[1][finite], want[1][finite], rtol=1e-6 * experts, atol=0, equal_nan=True)
 
 
+# Rows in LDS beside the waves' sums at what a launch has of it unasked, 64 KB: just below, above, and at the most that is taken.
+@pytest.mark.parametrize("rows,k", [(16, 1488), (16, 1520), (16, 1528), (12, 2040), (6, 4008), (6, 4096), (16, 3832)])
+@pytest.mark.parametrize("normed", [False, True])
+def test_fused_products_whose_rows_fill_local_memory(ops, rows, k, normed):
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    x, w, weight = rand(rows, k), (rand(256, k) * k ** -0.5).bfloat16(), 1 + 0.3 * rand(k)
+    if not normed:
+        x, weight = x.bfloat16(), None
+    unit = x.double() if weight is None else (x.double() / (x.double().square().mean(1, keepdim=True) + 1e-5).sqrt() * weight.double())
+    # bfloat16 has eight bits: a rounding is 2^-8 of its value at most, and one that falls to the other side 2^-7.  A result is rounded once; the
+    # normed rows before it, each |x| |w| of a sum by 2^-7; the K products are added in float (K units of 2^-24).
+    rows_in = unit.bfloat16().double()
+    product, mags = rows_in @ w.double().t(), rows_in.abs() @ w.double().t().abs()
+    slack = (2.0 ** -7 * normed + k * 2.0 ** -24) * mags
+    q = ops.fused_norm_qkv_rope(x, weight, 1e-5, w, None, torch.zeros(rows, dtype=torch.int32, device="cuda"), None, None, None, None, 2, 1, 64)
+    assert bool(((q.double() - product[:, :128]).abs() <= 2.0 ** -8 * product[:, :128].abs() + slack[:, :128]).all())
+    gated = ops.fused_norm_gated(x, weight, 1e-5, w)
+    gate, up = product.chunk(2, 1)
+    want = torch.nn.functional.silu(gate) * up
+    # (silu's slope is at most 1.1, silu(z) at most |z|; the exponential and the quotient are units of 2^-22.)
+    slack = 1.1 * slack[:, :128] * (up.abs() + slack[:, 128:]) + gate.abs() * slack[:, 128:] + (2.0 ** -8 + 2.0 ** -20) * want.abs()
+    assert bool(((gated.double() - want).abs() <= slack).all())
+
+
 # Workgroups of four, seven, nine and sixteen weight rows with a last one that is not full; K below a step, with a tail, of one trip and
 # of several, by steps and by lines; rows that are staged in one load and in as many as eight rows take, and that come straight from
 # memory; rows of a longer stride with no numbers beyond K; the gate with few and with many columns.

@@ -520,8 +520,9 @@ static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
     }
   }
   size_t lds = NORM ? (size_t)args.m * (args.k + 8) * sizeof(uint16_t) : (size_t)(STAGE > 0 ? NW * args.m * (UN * 64 + 16) : 0);
-  if (lds > 48 * 1024) {
-    // More dynamic LDS than the default limit: ask for it (the device has 160 KB per compute unit).
+  constexpr size_t SUMS_BYTES = NW * (EPI == EPI_RESIDUAL ? 1 : 2) * 4 * (WAVE + 4) * sizeof(float);   // (the kernel's own: `red`)
+  if (lds + SUMS_BYTES > 64 * 1024) {
+    // More LDS than a launch has unasked: ask for it (the device has 160 KB per compute unit).
     if (lds > 140 * 1024) return -1;
     hipError_t err = hipFuncSetAttribute(
         reinterpret_cast<const void*>(&fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, STAGE>),
