@@ -548,19 +548,22 @@ static int launch_one(const FusedArgs& args, int tiles, hipStream_t stream) {
   const int pairs = (args.k / 32 + 1) / 2;
   const int steps_per_wave = 2 * ((pairs + NW - 1) / NW);
   const bool whole = (args.k & 63) == 0;                     // K in whole cache lines
-  if (steps_per_wave <= 4) return launch_kernel<NW, EPI, NORM, 4, true, PASSES>(args, tiles, stream);
+  // (Rows straight from memory have a trip for all of a short share with the residual epilogue alone: the others' rows lie in LDS while K is short.)
+  if constexpr (NORM || EPI == EPI_RESIDUAL)
+    if (steps_per_wave <= 4) return launch_kernel<NW, EPI, NORM, 4, true, PASSES>(args, tiles, stream);
   if constexpr (NORM && (EPI == EPI_ROPE_STORE || PASSES == 1)) {
     // Rows in LDS: only the weights take registers, and a wave's whole share of up to eight steps is one trip
     // (rows of 1,025 to 2,048 elements at eight waves: two trips in the loop below; q/k/v at 1,536: 8.4 -> 7.5 us).
     // The gated product's matrix is several workgroups for every compute unit: it takes a whole share at once only
     // while two workgroups' registers fit a unit together, which is one block of rows and six steps (with two blocks
     // of rows 19.9 -> 22.3 us at 8,960 x 1,536, with eight steps 25.4 -> 31.3 us at 11,008 x 2,048).
-    if (EPI == EPI_GATED && whole && steps_per_wave <= 6) return launch_kernel<NW, EPI, NORM, 6, true, PASSES, true>(args, tiles, stream);
+    if constexpr (EPI == EPI_GATED)
+      if (whole && steps_per_wave <= 6) return launch_kernel<NW, EPI, NORM, 6, true, PASSES, true>(args, tiles, stream);
     if (steps_per_wave <= 6) return launch_kernel<NW, EPI, NORM, 6, true, PASSES>(args, tiles, stream);
     if constexpr (EPI == EPI_ROPE_STORE)
       if (steps_per_wave <= 8) return launch_kernel<NW, EPI, NORM, 8, true, PASSES>(args, tiles, stream);
   }
-  if constexpr (!NORM && PASSES == 1) {
+  if constexpr (!NORM && EPI == EPI_RESIDUAL && PASSES == 1) {
     // Rows from memory: one trip for a wave's whole share if it fits the registers (128 a lane at 16 waves).
     if (steps_per_wave <= 8) return launch_kernel<NW, EPI, NORM, 8, true, 1>(args, tiles, stream);
     if (whole && steps_per_wave <= 10) return launch_kernel<NW, EPI, NORM, 10, true, 1, true>(args, tiles, stream);

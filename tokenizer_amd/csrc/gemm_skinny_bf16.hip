@@ -30,7 +30,7 @@ __device__ __forceinline__ void store1(float* p, float v) { *p = v; }
 __device__ __forceinline__ void store1(bf16_t* p, float v) { p->bits = float_to_bf16_bits(v); }
 
 // grid.x: tiles of 16 output columns (of N, or of N/2 with GATED).  NW waves per workgroup.
-// grid.y: parts of K of `k_chunk` elements (a multiple of 32, of 64 with LINES) each: with more than one, a workgroup writes the
+// grid.y: parts of K of `k_chunk` elements (a multiple of 32; one part with LINES) each: with more than one, a workgroup writes the
 // float sums of its part into its slab of `partial` [parts, M, N] and `splitk_reduce` finishes the product.  That is
 // for few output tiles and a long K (the down projection of a decode batch): every compute unit gets a share.
 //
@@ -552,8 +552,7 @@ template <int MB, int NW, bool GATED, int NB = 1, int LINES = 0, bool WHOLE = fa
 static int launch_skinny(const void* A, int lda, const void* W, const void* bias, void* C, int ldc, int M, int N,
                          int K, int out_dtype, hipStream_t stream, int splits = 1, void* partial = nullptr, int gate_act = 0) {
   const int n_out = GATED ? N / 2 : N;
-  const int step = LINES > 0 ? 64 : 32;
-  const int k_chunk = splits > 1 ? ((K + splits - 1) / splits + step - 1) / step * step : K;
+  const int k_chunk = splits > 1 ? ((K + splits - 1) / splits + 31) / 32 * 32 : K;
   if (splits > 1) splits = (K + k_chunk - 1) / k_chunk;          // no part without a step of its own
   const dim3 grid((n_out + 16 * NB - 1) / (16 * NB), splits);
   float* slabs = splits > 1 ? (float*)partial : nullptr;
@@ -647,8 +646,9 @@ static int pick_waves(const void* A, int lda, const void* W, const void* bias, v
     return launch_few<16, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
   } else {
     if (waves == 4) return launch_skinny<MB, 4, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
-    if (waves == 8) return launch_skinny<MB, 8, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
-    return launch_skinny<MB, 16, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
+    if constexpr (MB * (GATED ? 2 : 1) <= 2)
+      if (waves == 16) return launch_skinny<MB, 16, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
+    return launch_skinny<MB, 8, GATED>(A, lda, W, bias, C, ldc, M, N, K, out_dtype, stream, 1, nullptr, gate_act);
   }
 }
 
