@@ -390,38 +390,54 @@ def test_rows_staged_by_their_waves(ops, rows, n, k):
     assert bool(((residual.double() - want).abs() <= slack).all())
 
 
-# Choices counted in registers (up to 64 experts) and searched for (more): ties, scores of minus infinity (with too few others to pick),
-# a logit that is no number, groups of one and of many; the logits form, whose kernels search, is the reference.
+# Choices counted in registers (up to 64 experts) and searched for (more): ties, logits and choice scores of minus infinity (with too few others to
+# pick), an infinite logit and one that is no number, groups of one and of many, worth their largest score or their two largest, weights
+# over their sum and as they are; the logits form, whose kernels search, is the reference.
 @pytest.mark.parametrize("experts,groups,keep,top", [(8, 0, 0, 2), (8, 4, 2, 2), (8, 8, 3, 3), (1, 0, 0, 1), (64, 8, 2, 7), (60, 4, 1, 15), (64, 0, 0, 64), (72, 8, 2, 5)])
 @pytest.mark.parametrize("softmax", [False, True])
-def test_choice_counted_is_choice_searched(ops, experts, groups, keep, top, softmax):
-    rows, width = 5, 64
+@pytest.mark.parametrize("group_max", [False, True])
+@pytest.mark.parametrize("renormalize", [False, True])
+def test_choice_counted_is_choice_searched(ops, experts, groups, keep, top, softmax, group_max, renormalize):
+    rows, width, inf = 5, 64, float("inf")
     x, router = torch.zeros((rows, width), dtype=torch.bfloat16), torch.zeros((experts, width), dtype=torch.bfloat16)
     x[:, :rows] = torch.eye(rows)
     router[:, 0] = rand_bf16((experts,), 41).cpu()
     router[:, 1] = torch.arange(experts) % 3                                    # ties
     router[:, 2] = torch.where(torch.arange(experts) < 1, 1.0, -3e38)           # all but one weigh nothing
     router[:, 3] = -torch.arange(experts) / 64
-    x[4, 0], router[0, 4] = 1.0, float("nan") if experts > 1 else 0.0           # (its product with every row that has it is no number)
-    x, router = x.cuda(), router.cuda()
-    logits = (x.cpu().double() @ torch.nan_to_num(router.cpu().double(), nan=0.0).t()).float().cuda()
-    finite = slice(0, 4)
-    for correction in (None, torch.randn(experts, generator=torch.Generator().manual_seed(42)).cuda().round(decimals=1)):
-        got = torch.full((rows, top), -1, dtype=torch.int32, device="cuda"), torch.full((rows, top), -1.0, device="cuda")
-        want = torch.full((rows, top), -1, dtype=torch.int32, device="cuda"), torch.full((rows, top), -1.0, device="cuda")
-        more = dict(softmax=softmax, group_max=False)
-        clean = torch.nan_to_num(router, nan=0.0)
-        assert ops.route_rows_scores(x[finite].contiguous(), clean, correction, experts, groups, keep, got[0][finite], got[1][finite], **more)
-        ops.route_scores(logits[finite].contiguous(), correction, experts, groups, keep, want[0][finite], want[1][finite], **more)
-        assert torch.equal(got[0][finite], want[0][finite])
-        assert torch.allclose(got[1][finite], want[1][finite], rtol=1e-6 * experts, atol=0, equal_nan=True)    # (sums in another order)
-        assert ops.route_rows_scores(x, router, correction, experts, groups, keep, *got, **more)               # a logit that is no number
-        assert bool(((got[0] >= 0) & (got[0] < experts)).all())
-    if not groups and experts <= 64:
-        assert ops.route_rows(x[finite].contiguous(), torch.nan_to_num(router, nan=0.0), got[0][finite], got[1][finite])
-        ops.route_top(logits[finite].contiguous(), want[0][finite], want[1][finite])
-        assert torch.equal(got[0][finite], want[0][finite])
-        assert torch.allclose(got[1][finite], want[1][finite], rtol=1e-6 * experts, atol=0, equal_nan=True)
+    router[:, 4] = torch.arange(experts) % 5 - 2
+    noted = torch.randn(experts, generator=torch.Generator().manual_seed(42)).round(decimals=1)
+    barred = torch.where(torch.arange(experts) % 4 == 1, noted, -inf)           # fewer than are picked are left
+    # A row of one in column 0 alone against logits of minus infinity but for one, an infinite one among others, and one that is no number.
+    single = torch.zeros((1, width), dtype=torch.bfloat16)
+    single[0, 0] = 1
+    columns = [torch.where(torch.arange(experts) == experts // 2, 1.0, -inf), router[:, 0].float(), router[:, 0].float()]
+    columns[1][experts - 1], columns[2][experts // 2] = inf, float("nan")
+    batches = [(x, router)]
+    for column in columns:
+        special = torch.zeros_like(router)
+        special[:, 0] = column
+        batches.append((single, special))
+    for rows_in, matrix in batches:
+        logits = (rows_in.float() @ matrix.float().t()) if len(rows_in) > 1 else matrix[:, 0].float()[None]      # (exact: one product a sum)
+        shape = (len(rows_in), top)
+
+        def chosen_by(route):
+            chosen, weights = torch.full(shape, -1, dtype=torch.int32, device="cuda"), torch.full(shape, 7.0, device="cuda")
+            assert route(chosen, weights) in (None, True)
+            return chosen, weights
+
+        def same(got, want):
+            assert bool((want[0] >= 0).all()) and torch.equal(got[0], want[0])
+            # (a weight is a quotient of terms of two roundings and sums of at most `experts` of them, in either order)
+            assert torch.allclose(got[1], want[1], rtol=2 * (experts + 4) * 2.0 ** -24, atol=0, equal_nan=True)
+        on = lambda t: None if t is None else t.contiguous().cuda()
+        for correction in (None, noted, barred):
+            more = dict(softmax=softmax, group_max=group_max, renormalize=renormalize)
+            same(chosen_by(lambda c, w: ops.route_rows_scores(on(rows_in), on(matrix), on(correction), experts, groups, keep, c, w, **more)),
+                 chosen_by(lambda c, w: ops.route_scores(on(logits), on(correction), experts, groups, keep, c, w, **more)))
+        if not groups:
+            same(chosen_by(lambda c, w: ops.route_rows(on(rows_in), on(matrix), c, w)), chosen_by(lambda c, w: ops.route_top(on(logits), c, w)))
 
 
 # Rows in LDS beside the waves' sums at what a launch has of it unasked, 64 KB: just below, above, and at the most that is taken.
