@@ -1,4 +1,6 @@
 """Kernels of steps of few rows alone, at the edges of the sizes they take."""
+import types
+
 import pytest
 import torch
 
@@ -696,3 +698,54 @@ def test_matrix_memory_of_single_tokens(ops, heads, d, dv, dtype):
         part = got[:, a:a + want[0].numel()].reshape(want.shape)
         assert float((part - want).abs().max()) <= unit * max(1.0, float(want.abs().max()))
     assert torch.equal(held[1].cpu(), state[1])
+
+
+# The streams' step with the token shift behind it, against 64 bits: one to four streams, columns of one wave and of sixteen, a last wave that is
+# partly empty, few rows and (at up to 256 columns) more than twice the compute units; a write pending and none.  Of five rows one only fills the
+# batch up (it takes no state and leaves none), one starts over a state row of NaN; entries and state rows lie in other orders.
+@pytest.mark.parametrize("streams", [1, 2, 3, 4])
+@pytest.mark.parametrize("width,rows", [(52, 5), (200, 700), (256, 5), (896, 10), (1000, 5), (1024, 15)])
+@pytest.mark.parametrize("written,out_dtype", [(None, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                               (torch.float32, torch.float32)])
+def test_streams_step_with_the_token_shift(ops, streams, width, rows, written, out_dtype):
+    gen = torch.Generator().manual_seed(width + streams)
+    rand = lambda *shape: torch.randn(*shape, generator=gen)
+    x, read, gain, mu, eps = rand(rows, streams, width), rand(streams), torch.tensor([1.7]), torch.rand(width, generator=gen), 1e-5
+    y, mix, coef, scale = rand(rows, width).to(written or torch.float32), rand(streams, streams), rand(streams), rand(width)
+    entry = torch.randperm(rows, generator=gen).int()
+    filler, fresh = torch.arange(rows) % 5 == 1, torch.arange(rows) % 5 == 2
+    entry[filler] = -1
+    slots = torch.randperm(rows + 3, generator=gen)[:rows].int()              # by entry
+    positions = torch.where(fresh, 0, 3 + torch.arange(rows)).int()
+    row_of = slots[entry.clamp(min=0).long()].long()                          # by row
+    state = rand(rows + 3, width)
+    state[row_of[fresh & ~filler]] = float("nan")
+    kept = state.clone()
+    ctx = types.SimpleNamespace(entry_of_token=entry.cuda(), state_slots=slots.cuda(), positions=positions.cuda())
+    held, on_state = x.cuda(), state.cuda()
+    write = types.SimpleNamespace(y=y.cuda(), mix=mix.cuda(), out=coef.cuda(), scale=scale.cuda()) if written else None
+    got = torch.empty((rows, width), dtype=out_dtype, device="cuda")
+    ops.streams_step(held, write, read.cuda(), gain.cuda(), eps, got, shift=(mu.cuda(), on_state, ctx))
+    new, mags = x.double(), x.double().abs()
+    if written:
+        add = scale.double() * y.double()
+        new = torch.einsum("tsw,sr->trw", new, mix.double()) + coef.double()[None, :, None] * add[:, None]
+        mags = torch.einsum("tsw,sr->trw", mags, mix.double().abs()) + coef.double().abs()[None, :, None] * add.abs()[:, None]
+    # A stream is a sum of at most five terms, the read one of four, each term rounded twice; the root mean square adds sums of sixty-four,
+    # of sixteen waves, a quotient and a root to what the squares are off by.
+    unit = 2.0 ** -24
+    assert bool(((held.double().cpu() - new).abs() <= 12 * unit * mags).all())
+    u, off = torch.einsum("tsw,s->tw", new, read.double()), 20 * unit * torch.einsum("tsw,s->tw", mags, read.double().abs())
+    rms = (u.square().mean(1, keepdim=True) + eps).sqrt()
+    h = u / rms * 1.7
+    off = 1.7 * off / rms + h.abs() * (off.norm(dim=1, keepdim=True) / u.norm(dim=1, keepdim=True) + 40 * unit)
+    live = ~filler
+    before = torch.where(fresh[:, None], 0.0, kept[row_of].double())
+    want = torch.where(live[:, None], h + (before - h) * mu.double(), h)
+    slack = 2 * off + 4 * unit * (h.abs() + before.nan_to_num().abs()) + (2.0 ** -8 * want.abs() if out_dtype == torch.bfloat16 else 0.0)
+    assert bool(((got.double().cpu() - want).abs() <= slack).all())
+    after = on_state.cpu()
+    assert bool(((after[row_of[live]].double() - h[live]).abs() <= off[live]).all())
+    untouched = torch.ones(rows + 3, dtype=torch.bool)
+    untouched[row_of[live]] = False
+    assert torch.equal(after[untouched], kept[untouched])
