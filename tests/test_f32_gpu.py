@@ -228,3 +228,34 @@ def test_attention_passes_over_a_description_of_other_tokens(ops, ref):
     want = run(ref)
     for batch in (make_batch(lengths, [1, 101, 2]), make_batch(lengths + [30], [1, 98, 2, 2])):    # other tokens, other entries
         torch.testing.assert_close(run(ops, batch), want, rtol=2e-5, atol=4e-6)
+
+
+# The merge of a single token's parts: 8, 16, 24, 48, 64 and (another walk) 80 of them, head sizes of a part of 64 coordinates, of a few and of four
+# times 64; rows whose contexts end in an early part; an infinite value among the last part's, which its coordinate alone has.
+@pytest.mark.parametrize("keys", [500, 900, 1500, 3000, 4000, 5000])
+@pytest.mark.parametrize("d", [32, 64, 100, 128, 192, 256])
+def test_merge_of_many_parts(ops, keys, d):
+    rows, heads, kv, page = 3, 4, 2, 16
+    gen = torch.Generator(device="cuda").manual_seed(keys + d)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    pages = -(-keys // page)
+    k, v = rand(rows * pages, kv, page, d), rand(rows * pages, kv, d, page)
+    last = [keys - 1, keys // 2, 70]
+    v[last[0] // page, 1, 5, last[0] % page] = float("inf")
+    q = rand(rows, (heads + 2 * kv) * d)
+    ints = lambda t: torch.tensor(t, dtype=torch.int32, device="cuda")
+    out = torch.empty((rows, heads * d), device="cuda")
+    ops.paged_attention(q, out, k, v, ints(last), ints([0, 1, 2]), ints(range(rows * pages)).view(rows, pages), heads, kv, d, None, d ** -0.5,
+                        max_position=keys - 1)
+    for r in range(rows):
+        n, mine = last[r] + 1, slice(r * pages, (r + 1) * pages)
+        keys_of = k[mine].transpose(1, 2).reshape(-1, kv, d)[:n].double().repeat_interleave(heads // kv, 1)
+        values = v[mine].permute(0, 3, 1, 2).reshape(-1, kv, d)[:n].double().repeat_interleave(heads // kv, 1)
+        query = q[r, :heads * d].view(heads, d).double() * d ** -0.5
+        weights = torch.softmax((keys_of * query).sum(-1), 0)[..., None]
+        want = (weights * values).sum(0)
+        # A weight is off by what its score is (d products, each sum rounded) and a few roundings more; sums of a wave's keys, of four waves and of the parts.
+        slack = (2 * (d + 8) * (keys_of * query).abs().sum(-1).max() + n / 4 + 100) * 2.0 ** -24 * (weights * values.abs()).sum(0)
+        got = out[r].view(heads, d).double()
+        assert bool((((got - want).abs() <= slack) | (got == want)).all())
+    assert int(torch.isinf(out).sum()) == heads // kv and not torch.isnan(out).any()

@@ -215,7 +215,12 @@ attention_f32_kernel(F32Args p) {
   if (!whole && threadIdx.x < 16) { p.part_ml[2 * item] = big; p.part_ml[2 * item + 1] = total; }
 }
 
-// out = the parts of a single token's keys under one maximum and sum; a wave a (token, head), a coordinate a lane.
+// out = the parts of a single token's keys under one maximum and sum; a wave a (token, head), COLS coordinates a lane, 64 apart.  Up to 64
+// parts: a part a lane brings maxima and sums and makes the weights, and beside them up to 64 numbers of a lane are on their way at once: one or
+// two trips to memory for what was one for every eight parts of every 64 coordinates.  (Attention and merge, us, eight parts of 64 coordinates
+// a trip behind two passes over the maxima | behind one | so: one row of 12 heads of 128 on two, 3,000 keys 14.0 | 15.8 | 10.7, of 32 of 256
+// on four 24.3 | 28.0 | 17.3; four rows of 28 of 128 on four, 1,500 keys 15.0 | 16.0 | 13.1, of 14 of 64 on two, 500 keys 8.0 | 8.0 | 7.5.)
+template <int COLS>
 __global__ void __launch_bounds__(WAVE)
 attention_f32_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ rows,
                            float* __restrict__ out, int n_q, int dv, int splits, const int* __restrict__ entry_of_token) {
@@ -227,29 +232,43 @@ attention_f32_merge_kernel(const float* __restrict__ part_o, const float* __rest
   const float2* ml = reinterpret_cast<const float2*>(part_ml) + base;
   float* dst = out + ((size_t)row * n_q + head) * dv;
   if (splits <= WAVE) {
-    // A part a lane: maxima and sums, and the first parts' rows beside them, are one trip, each weight one exponential.
+    constexpr int RUN = 8, RUNS = WAVE / RUN / COLS;         // parts that are asked for behind one question whether there are any
+    const float* from = part_o + base * dv;
     float2 stat = ml[min(lane, splits - 1)];
-    constexpr int AHEAD = 8;
-    float v[AHEAD];
+    float v[RUNS][RUN][COLS], o[COLS], weight = 0.f, denom = 0.f;
+    int at[COLS];
 #pragma unroll
-    for (int j = 0; j < AHEAD; ++j) v[j] = part_o[(base + min(j, splits - 1)) * dv + min(lane, dv - 1)];
-    if (lane >= splits) stat = make_float2(-INFINITY, 0.f);
-    const float big = wave_max(stat.x), weight = lane < splits ? expf(stat.x - big) : 0.f;
-    const float denom = wave_sum(stat.y * weight);
-    for (int i0 = 0; i0 < dv; i0 += WAVE) {
-      const int i = min(i0 + lane, dv - 1);
-      float o = 0.f;
-      for (int s0 = 0; s0 < splits; s0 += AHEAD) {
-        if (i0 + s0 > 0) {
+    for (int c = 0; c < COLS; ++c) { at[c] = min(lane + c * WAVE, dv - 1); o[c] = 0.f; }
+    for (int s0 = 0; s0 < splits; s0 += RUNS * RUN) {
 #pragma unroll
-          for (int j = 0; j < AHEAD; ++j) v[j] = part_o[(base + min(s0 + j, splits - 1)) * dv + i];
-        }
+      for (int r = 0; r < RUNS; ++r) {
+        if (s0 + r * RUN >= splits) break;
 #pragma unroll
-        for (int j = 0; j < AHEAD; ++j)
-          if (s0 + j < splits) o += v[j] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s0 + j));
+        for (int j = 0; j < RUN; ++j)
+#pragma unroll
+          for (int c = 0; c < COLS; ++c) v[r][j][c] = from[min(s0 + r * RUN + j, splits - 1) * dv + at[c]];
       }
-      if (i0 + lane < dv) st_through(dst + i, o / denom);
+      if (s0 == 0) {
+        if (lane >= splits) stat = make_float2(-INFINITY, 0.f);
+        const float big = wave_max(stat.x);
+        weight = lane < splits ? expf(stat.x - big) : 0.f;
+        denom = wave_sum(stat.y * weight);
+      }
+#pragma unroll
+      for (int r = 0; r < RUNS; ++r) {
+        if (s0 + r * RUN >= splits) break;
+#pragma unroll
+        for (int j = 0; j < RUN; ++j) {
+          const int s = s0 + r * RUN + j;
+          const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s));      // (0 past the last part)
+#pragma unroll
+          for (int c = 0; c < COLS; ++c) o[c] = fmaf(s < splits ? v[r][j][c] : 0.f, w, o[c]);
+        }
+      }
     }
+#pragma unroll
+    for (int c = 0; c < COLS; ++c)
+      if (lane + c * WAVE < dv) dst[lane + c * WAVE] = o[c] / denom;
     return;
   }
   float big = -INFINITY;
@@ -301,8 +320,10 @@ extern "C" int ta_paged_attention_f32(const void* q, int q_stride, void* out, co
 #undef GO
   int status = LAUNCH_STATUS();
   if (status == 0 && n_single > 0 && splits > 1) {
-    attention_f32_merge_kernel<<<n_single * n_q, WAVE, 0, stream>>>((const float*)part_o, (const float*)part_ml, (const int*)rows,
-                                                                    (float*)out, n_q, dv, splits, (const int*)entry_of_token);
+#define GO(COLS) attention_f32_merge_kernel<COLS><<<n_single * n_q, WAVE, 0, stream>>>((const float*)part_o, (const float*)part_ml, \
+      (const int*)rows, (float*)out, n_q, dv, splits, (const int*)entry_of_token)
+    if (dv <= 64) GO(1); else if (dv <= 128) GO(2); else GO(4);
+#undef GO
     status = LAUNCH_STATUS();
   }
   return status;
