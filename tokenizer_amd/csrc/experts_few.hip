@@ -201,7 +201,7 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
       }
       // (A pick that weighs nothing adds nothing, whatever its expert makes of the row: as the form over all experts has it.)
       if (!shared && wgt == 0.f) value = 0.f;
-      st_through(act + (size_t)p * inner + n0 + r, value);
+      st(act + (size_t)p * inner + n0 + r, value);
     }
     __syncthreads();                                         // the sums are read before the next sixteen pairs' are written
   }
@@ -254,7 +254,7 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
 #pragma unroll
       for (int w = 0; w < NW; ++w) v += red[w][r & 3][(r >> 2) * 16 + c];
       const int p = list[p0 + c];
-      st_through(out + ((size_t)(slab + p % top) * n_rows + p / top) * hidden + n0 + r, v);
+      out[((size_t)(slab + p % top) * n_rows + p / top) * hidden + n0 + r] = v;
     }
     __syncthreads();
   }
