@@ -24,11 +24,12 @@ __device__ __forceinline__ void st(float* p, float v) { *p = v; }
 __device__ __forceinline__ void st(bf16_t* p, float v) { p->bits = float_to_bf16_bits(v); }
 
 // Stores past the caches of the chiplet that makes them (device scope): what a small kernel leaves is on its way to where the next
-// kernel's chiplets read it when the kernel ends, and the end has nothing to write back: 0.1 to 0.25 us of every launch that stores
-// a few KB (products of 896 columns, one row: out 2.81 -> 2.65 us, gate/up 6.12 -> 6.03, down 4.59 -> 4.44).  For results of a few KB a
-// chiplet whose lanes store side by side; a store of its own for every value of a scattered result costs more this way than the
-// write-back (four values a lane: q/k/v 4.6 -> 5.5; head products, whose 16-bit values lie apart, 1.3 us).  What the same chiplet reads
-// again soon stays in its cache by plain stores (streams).  Nontemporal stores do not do: of single 16-bit values they cost 10 us.
+// kernel's chiplets read it when the kernel ends, and the end has nothing to write back.  It pays where few workgroups' lanes store floats side by
+// side: residual products (896 columns, one row: out 2.81 -> 2.65 us, down 4.59 -> 4.44; 270 of them, 64 to 30,000 columns, 0.97 of their time), less in
+// the gated ones beside them (gate/up 6.12 -> 6.03).  A store of its own for every value of a scattered result costs more this way than the
+// write-back (four values a lane: q/k/v 4.6 -> 5.5; head products, whose 16-bit values lie apart, 1.3 us; chosen experts, 176 of them, 1.01 of
+// their time), and products of few rows in bfloat16 and in 32 bits are level or 1 to 2 % slower by it: those store plainly.  What the same
+// chiplet reads again soon stays in its cache by plain stores (streams).  Nontemporal stores do not do: of single 16-bit values they cost 10 us.
 __device__ __forceinline__ void st_through(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

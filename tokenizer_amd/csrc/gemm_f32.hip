@@ -539,26 +539,26 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, u
     const int i = first_in + at;
     if (head < store.n_q) {
       float* dst = C + (size_t)m * ldc + (size_t)head * d + i;
-      st_through(dst, v1);
-      st_through(dst + half, v2);
+      st(dst, v1);
+      st(dst + half, v2);
       return;
     }
     if (slot_of < 0) return;                                // this row's keys and values are not stored
     const int page = slot_of / store.page_size, off = slot_of % store.page_size;
     if (head < store.n_q + store.n_kv) {
       float* dst = store.k_pages + (((size_t)page * store.n_kv + (head - store.n_q)) * store.page_size + off) * d + i;
-      st_through(dst, v1);
-      st_through(dst + half, v2);
+      st(dst, v1);
+      st(dst + half, v2);
     } else {
       float* dst = store.v_pages + (((size_t)page * store.n_kv + (head - store.n_q - store.n_kv)) * d + i) * store.page_size + off;
-      st_through(dst, v1);
-      st_through(dst + (size_t)half * store.page_size, v2);
+      st(dst, v1);
+      st(dst + (size_t)half * store.page_size, v2);
     }
   } else if (KIND == ROWS_GATED) {
-    if (n0 + at < half) st_through(C + (size_t)m * ldc + n0 + at, silu_f32(total(at)) * total(at + 8));
+    if (n0 + at < half) st(C + (size_t)m * ldc + n0 + at, silu_f32(total(at)) * total(at + 8));
   } else if (n0 + at < N) {
-    if (partial) st_through(partial + ((size_t)blockIdx.y * M + m) * N + n0 + at, total(at));
-    else st_through(C + (size_t)m * ldc + n0 + at, total(at) + bias1);
+    if (partial) st(partial + ((size_t)blockIdx.y * M + m) * N + n0 + at, total(at));
+    else st(C + (size_t)m * ldc + n0 + at, total(at) + bias1);
   }
 }
 
@@ -672,9 +672,9 @@ gemv_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, int M,
     const int m = m0 + s8 / (8 / ROWS_IN_8), n = n0 + s8 % (8 / ROWS_IN_8);
     if ((lane & 15) > 1 || m >= M) continue;
     if constexpr (GATED) {
-      if (n < half) st_through(C + (size_t)m * ldc + n, silu_f32(total) * second);
+      if (n < half) st(C + (size_t)m * ldc + n, silu_f32(total) * second);
     } else if (n < N) {
-      st_through(C + (size_t)m * ldc + n, total + bias_here);
+      st(C + (size_t)m * ldc + n, total + bias_here);
     }
   }
 }

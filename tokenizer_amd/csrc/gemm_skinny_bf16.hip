@@ -486,8 +486,8 @@ few_rows_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
       v = gate_act == 2 ? fmaxf(v, 0.f) * up
           : gate_act == 1 ? 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v))) * up
                           : v / (1.0f + __expf(-v)) * up;
-    if (partial) st_through(partial + ((size_t)blockIdx.y * M + m) * n_out + n, v);         // (never GATED)
-    else st_through(C + (size_t)m * ldc + n, v);
+    if (partial) st(partial + ((size_t)blockIdx.y * M + m) * n_out + n, v);         // (never GATED)
+    else st(C + (size_t)m * ldc + n, v);
   }
 }
 
