@@ -469,9 +469,11 @@ def test_fused_products_whose_rows_fill_local_memory(ops, rows, k, normed):
 
 # Workgroups of four, seven, nine and sixteen weight rows with a last one that is not full; K below a step, with a tail, of one trip and
 # of several, by steps and by lines; rows that are staged in one load and in as many as eight rows take, and that come straight from
-# memory; rows of a longer stride with no numbers beyond K; the gate with few and with many columns.
+# memory, at the last share of K that is staged and the first that is not; rows of a longer stride with no numbers beyond K; the gate with few
+# and with many columns.
 @pytest.mark.parametrize("rows", [1, 3, 5, 8, 9, 16])
-@pytest.mark.parametrize("n,k", [(8, 8), (20, 40), (900, 904), (1544, 2112), (2060, 1536), (900, 4864), (1100, 6720), (4100, 904), (16400, 1536)])
+@pytest.mark.parametrize("n,k", [(8, 8), (20, 40), (900, 904), (1544, 2112), (2060, 1536), (900, 4864), (1100, 6720), (4100, 904), (16400, 1536),
+                                 (300, 768), (300, 776), (300, 1032), (300, 2056), (4100, 1032), (16400, 392), (16400, 1000), (16400, 1064)])
 def test_products_of_few_rows_spread_over_the_device(ops, rows, n, k):
     x = torch.full((rows, k + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
     x[:, :k] = rand_bf16((rows, k), 31)

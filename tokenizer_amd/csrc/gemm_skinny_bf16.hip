@@ -529,7 +529,13 @@ static int launch_few(const void* A, int lda, const void* W, const void* bias, v
   int status;
 #define RUN(T, ST) launch_few_kernel<NW, GATED, T, LINES, WHOLE, SUMS, UPPER, ST>(A, lda, W, bias, C, ldc, M, N, K, k_chunk, rows, grid, \
                                                                                  slabs, gate_act, stream)
-#define PICK(T) status = M > 8 || K < 8 ? RUN(T, 0) : M * PIECES <= WAVE ? RUN(T, 1) : RUN(T, MOST)
+  // Rows straight from memory as well where a wave has up to three steps, whose fragments are hardly more loads than pieces and are there
+  // sooner, and, K not in whole lines, in walks of more than one trip (two over tens of thousands of columns), where a trip's pieces are
+  // asked for when the one before has been multiplied.  (Staged | direct, us: eight rows of 248 over 120 2.66 | 2.33, six of 200 over 232
+  // 2.69 | 2.34, three of 752 over 128 2.56 | 2.26; eight of 7,576 over 1,424 7.6 | 7.0, of 6,000 over 6,000 24.6 | 23.7, gate/up 5,176 over 2,272 15.3 | 14.3;
+  // six of 34,424 over 1,064 20.1 | 19.5, eight of 31,816 over 1,240 22.1 | 21.5.)
+  const bool direct = M > 8 || K < 8 || (LINES == 0 && ((NW <= 8 && k_chunk <= NW * 96) || k_chunk > NW * (NW == 4 ? 256 : 128)));
+#define PICK(T) status = direct ? RUN(T, 0) : M * PIECES <= WAVE ? RUN(T, 1) : RUN(T, MOST)
   if (out_dtype == DT_F32) PICK(float); else PICK(bf16_t);
 #undef PICK
 #undef RUN
