@@ -16,8 +16,8 @@
 // load on (what lies behind PER * LT_THREADS of a longer latent is read again), norm weights, position and rates are asked for beside them, and
 // the angles are the last wave's, which has the fewest elements.  (One workgroup for both parts one behind the other, each read twice | so, in a
 // graph: four rows of latents of 448 and 96 3.5 | 2.4 us, of 1,792 and 192 4.9 | 2.7, 2,000 rows of those 10.5 | 10.1.)
-template <typename T, int PER>
-__global__ void __launch_bounds__(LT_THREADS)
+template <typename T, int PER, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, int q_rank, const float* __restrict__ q_norm,
                     int kv_offset, int kv_rank, const float* __restrict__ kv_norm, int rot, const float* __restrict__ rates,
                     float eps, const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ k_pages,
@@ -37,11 +37,11 @@ latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, in
   float w[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int i = min(j * LT_THREADS + (int)threadIdx.x, rank - 1);
+    const int i = min(j * THREADS + (int)threadIdx.x, rank - 1);
     raw[j] = from[i];
     w[j] = norm[i];
   }
-  const int half = keys ? rot / 2 : 0, turn = (threadIdx.x + WAVE) % LT_THREADS;    // (the thread's pair of the tail: the last wave has the first)
+  const int half = keys ? rot / 2 : 0, turn = (threadIdx.x + WAVE) % THREADS;    // (the thread's pair of the tail: the last wave has the first)
   const T* tail = row + kv_offset + kv_rank;
   float rate = 0.f, position = 0.f;
   T one_raw = {}, other_raw = {};
@@ -56,18 +56,18 @@ latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, in
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const float v = ld(&raw[j]);
-    if (j * LT_THREADS + (int)threadIdx.x < rank) sq += v * v;
+    if (j * THREADS + (int)threadIdx.x < rank) sq += v * v;
   }
-  for (int i = PER * LT_THREADS + threadIdx.x; i < rank; i += LT_THREADS) { const float v = ld(from + i); sq += v * v; }
+  for (int i = PER * THREADS + threadIdx.x; i < rank; i += THREADS) { const float v = ld(from + i); sq += v * v; }
   const float inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)rank + eps);
   if (!keys) {
     T* dst = latent_q + (size_t)t * q_rank;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int i = j * LT_THREADS + threadIdx.x;
+      const int i = j * THREADS + threadIdx.x;
       if (i < rank) st(dst + i, ld(&raw[j]) * inv * w[j]);
     }
-    for (int i = PER * LT_THREADS + threadIdx.x; i < rank; i += LT_THREADS) st(dst + i, ld(from + i) * inv * norm[i]);
+    for (int i = PER * THREADS + threadIdx.x; i < rank; i += THREADS) st(dst + i, ld(from + i) * inv * norm[i]);
     return;
   }
   const int page = slot / page_size, off = slot % page_size, width = kv_rank + rot;
@@ -79,11 +79,11 @@ latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, in
   };
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int i = j * LT_THREADS + threadIdx.x;
+    const int i = j * THREADS + threadIdx.x;
     if (i < rank) put(i, ld(&raw[j]) * inv * w[j]);
   }
-  for (int i = PER * LT_THREADS + threadIdx.x; i < rank; i += LT_THREADS) put(i, ld(from + i) * inv * norm[i]);
-  for (int i = turn; i < half; i += LT_THREADS) {
+  for (int i = PER * THREADS + threadIdx.x; i < rank; i += THREADS) put(i, ld(from + i) * inv * norm[i]);
+  for (int i = turn; i < half; i += THREADS) {
     if (i != turn) { rate = rates[i]; one_raw = tail[neighbours ? 2 * i : i]; other_raw = tail[neighbours ? 2 * i + 1 : half + i]; }
     float s, c;
     sincosf(position * rate, &s, &c);
@@ -292,14 +292,16 @@ extern "C" int ta_latent_store(const void* rows, int row_stride, int q_offset, i
     return -1;
   const int most = q_rank > kv_rank ? q_rank : kv_rank;
   const dim3 grid(n_tokens, slots ? 2 : 1);
-#define LS_PER(TT, PER) latent_store_kernel<TT, PER><<<grid, LT_THREADS, 0, stream>>>((const TT*)rows, row_stride, q_offset, q_rank, \
-    (const float*)q_norm, kv_offset, kv_rank, (const float*)kv_norm, rot, (const float*)rates, eps, (const int*)positions, \
+  // (Short latents: no wave without an element of its own.  Two latents of 64, 2,000 rows, four waves a part | one: 5.5 | 3.6 us.)
+#define LS_GO(TT, PER, THREADS) latent_store_kernel<TT, PER, THREADS><<<grid, THREADS, 0, stream>>>((const TT*)rows, row_stride, \
+    q_offset, q_rank, (const float*)q_norm, kv_offset, kv_rank, (const float*)kv_norm, rot, (const float*)rates, eps, (const int*)positions, \
     (const int*)slots, (TT*)k_pages, (TT*)v_pages, page_size, (TT*)latent_q, neighbours)
-#define LS(TT) do { if (most <= LT_THREADS) LS_PER(TT, 1); else if (most <= 2 * LT_THREADS) LS_PER(TT, 2); \
-                    else if (most <= 4 * LT_THREADS) LS_PER(TT, 4); else LS_PER(TT, 8); } while (0)
+#define LS(TT) do { if (most <= 64) LS_GO(TT, 1, 64); else if (most <= 128) LS_GO(TT, 1, 128); else if (most <= LT_THREADS) LS_GO(TT, 1, LT_THREADS); \
+                    else if (most <= 2 * LT_THREADS) LS_GO(TT, 2, LT_THREADS); else if (most <= 4 * LT_THREADS) LS_GO(TT, 4, LT_THREADS); \
+                    else LS_GO(TT, 8, LT_THREADS); } while (0)
   if (dtype == DT_F32) LS(float); else LS(bf16_t);
 #undef LS
-#undef LS_PER
+#undef LS_GO
   return LAUNCH_STATUS();
 }
 
