@@ -65,13 +65,18 @@ norm_add_rmsnorm_kernel(float* __restrict__ residual, const TD* __restrict__ del
   }
 }
 
-// Four consecutive elements of a row as floats, and back.
-__device__ __forceinline__ float4 na_ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 na_ld4(const bf16_t* p) {
-  const uint2 raw = *reinterpret_cast<const uint2*>(p);
+// Four elements as they lie in memory, and as floats.
+template <typename T> struct NaRawOf { typedef float4 type; };
+template <> struct NaRawOf<bf16_t> { typedef uint2 type; };
+template <typename T> using NaRaw = typename NaRawOf<T>::type;
+__device__ __forceinline__ float4 na_of_raw(float4 raw) { return raw; }
+__device__ __forceinline__ float4 na_of_raw(uint2 raw) {
   return make_float4(bf16_bits_to_float(raw.x & 0xffffu), bf16_bits_to_float(raw.x >> 16),
                      bf16_bits_to_float(raw.y & 0xffffu), bf16_bits_to_float(raw.y >> 16));
 }
+// Four consecutive elements of a row as floats, and back.
+__device__ __forceinline__ float4 na_ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 na_ld4(const bf16_t* p) { return na_of_raw(*reinterpret_cast<const uint2*>(p)); }
 __device__ __forceinline__ void na_st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void na_st4(bf16_t* p, float4 v) {
   uint2 raw;
@@ -830,13 +835,7 @@ __device__ __forceinline__ void na_group_rms(const float* part, float* inv, int 
   __syncthreads();
   for (int g = wave; g < groups; g += NA_THREADS / WAVE) {
     float sq = 0.f;
-    for (int i0 = 0; i0 < entries; i0 += 8 * WAVE) {         // (eight reads on their way at once, added in their order)
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = part[(size_t)g * entries + min(i0 + j * WAVE + lane, entries - 1)];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sq += i0 + j * WAVE + lane < entries ? v[j] : 0.f;
-    }
+    for (int i = lane; i < entries; i += WAVE) sq += part[(size_t)g * entries + i];
     sq = wave_sum(sq);
     if (lane == 0) inv[g] = 1.0f / sqrtf(sq / (float)size + eps);
   }
@@ -850,7 +849,9 @@ __device__ __forceinline__ void na_group_rms(const float* part, float* inv, int 
 // for its loads, so the slabs are asked for four at a time before any of them is added.  What it saves is the kernel that added them
 // and a rounded copy of the product written and read again: eight layers of 1,536 with an inner width of 8,960, 8 requests from
 // prompts of 90 to 500 tokens through eight decoded ones, 7.73 ms with that kernel, 7.59 without.
-template <typename TD, typename TO, int CHUNKS, bool PARTS = false>
+// POST, NEXT: whether there is a weight behind the sub-layer and one in front of the next, so that every load stands at the start, chunk by
+// chunk, and none is made that the form has no use for; the groups an element is in are worked out while the rows are on their way.
+template <typename TD, typename TO, int CHUNKS, bool PARTS, bool POST, bool NEXT>
 __global__ void __launch_bounds__(NA_THREADS)
 group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ delta, const float* __restrict__ post_weight,
                           float post_eps, int post_groups, const float* __restrict__ weight, float eps, int groups,
@@ -862,35 +863,35 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
   const int i = blockIdx.x;
   const int r = rows ? scalar_int(rows + i) : i;
   float* res = residual + (size_t)r * hidden;
-  // What a form has not is loaded from the row itself and not used: no load stands behind a condition, which would be a trip of its own.
-  const TD* del = delta ? delta + (size_t)r * hidden : reinterpret_cast<const TD*>(res);
-  const float* post_at = post_weight ? post_weight : res;
-  const float* next_at = weight ? weight : res;
+  const bool added = PARTS || POST || delta;
+  const TD* del = added ? delta + (size_t)r * hidden : reinterpret_cast<const TD*>(res);     // (without a delta the row itself, not used)
   float4 x[CHUNKS], d[CHUNKS], behind_w[CHUNKS], next_w[CHUNKS];
+  NaRaw<TD> raw[CHUNKS];                                     // (bfloat16 becomes float where it is used: nothing waits in front)
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int h = min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4);
     x[c] = na_ld4(res + h);
-    if constexpr (PARTS) d[c] = na_ld4(del + h);
-    behind_w[c] = na_ld4(post_at + h);
-    next_w[c] = na_ld4(next_at + h);
+    raw[c] = *reinterpret_cast<const NaRaw<TD>*>(del + h);
+    if constexpr (POST) behind_w[c] = na_ld4(post_weight + h);
+    if constexpr (NEXT) next_w[c] = na_ld4(weight + h);
   }
-  // (The groups an element is in are worked out while the rows are on their way.)
   int post_of[CHUNKS], next_of[CHUNKS];
-  const int post_size = hidden / post_groups, next_size = hidden / groups;
+  const int post_size = POST ? hidden / post_groups : 1, next_size = NEXT ? hidden / groups : 1;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int h = min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4);
-    post_of[c] = h / post_size;
-    next_of[c] = h / next_size;
-    asm volatile("" : "+v"(post_of[c]), "+v"(next_of[c]));
+    const int h = (c * NA_THREADS + (int)threadIdx.x) * 4;
+    post_of[c] = next_of[c] = 0;
+    if (h < hidden) {
+      if constexpr (POST) post_of[c] = h / post_size;
+      if constexpr (NEXT) next_of[c] = h / next_size;
+    }
+    if constexpr (POST) asm volatile("" : "+v"(post_of[c]));
+    if constexpr (NEXT) asm volatile("" : "+v"(next_of[c]));
   }
-  if constexpr (!PARTS) {
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) d[c] = na_ld4(del + min((c * NA_THREADS + (int)threadIdx.x) * 4, hidden - 4));
-  }
+  for (int c = 0; c < CHUNKS; ++c) d[c] = na_of_raw(raw[c]);
   if constexpr (PARTS) na_add_slabs<CHUNKS>(d, delta + (size_t)r * hidden, parts, slab, hidden, rounded);
-  if (post_weight) {
+  if constexpr (POST) {
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
       const int e = c * NA_THREADS + threadIdx.x;
@@ -902,17 +903,17 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
   for (int c = 0; c < CHUNKS; ++c) {
     const int h = (c * NA_THREADS + (int)threadIdx.x) * 4;
     if (h >= hidden) continue;
-    if (post_weight) {
+    if constexpr (POST) {
       const float f = inv[post_of[c]];
       // (One rounding, written down: behind a sum that both branches share, the compiler rounds the product as well.)
       x[c].x = fmaf(d[c].x * f, behind_w[c].x, x[c].x); x[c].y = fmaf(d[c].y * f, behind_w[c].y, x[c].y);
       x[c].z = fmaf(d[c].z * f, behind_w[c].z, x[c].z); x[c].w = fmaf(d[c].w * f, behind_w[c].w, x[c].w);
-    } else if (PARTS || delta) {
+    } else if (added) {
       x[c].x += d[c].x; x[c].y += d[c].y; x[c].z += d[c].z; x[c].w += d[c].w;
     }
     if (store_residual) na_st4(res + h, x[c]);
   }
-  if (weight) {
+  if constexpr (NEXT) {
     __syncthreads();                                         // the first norm's factors have been read
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
@@ -926,7 +927,7 @@ group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ d
   for (int c = 0; c < CHUNKS; ++c) {
     const int h = (c * NA_THREADS + (int)threadIdx.x) * 4;
     if (h >= hidden) continue;
-    if (weight) {
+    if constexpr (NEXT) {
       const float f = inv[next_of[c]];
       na_st4(dst + h, make_float4(x[c].x * f * next_w[c].x, x[c].y * f * next_w[c].y, x[c].z * f * next_w[c].z,
                                   x[c].w * f * next_w[c].w));
@@ -994,10 +995,15 @@ extern "C" int ta_group_norm_add(void* residual, const void* delta, const void* 
   const bool aligned = (((uintptr_t)residual | (uintptr_t)delta | (uintptr_t)post_weight | (uintptr_t)weight | (uintptr_t)out) & 15) == 0;
   const bool vec = aligned && hidden <= 8192 && (hidden / post_groups) % 4 == 0 && (hidden / groups) % 4 == 0;
   const size_t lds = sizeof(float) * (vec ? (size_t)hidden / 4 + most : (size_t)post_groups + groups);
-#define GROUP_VEC(TD, TO, CH)                                                                                            \
-    group_norm_add_vec_kernel<TD, TO, CH><<<n_rows, NA_THREADS, lds, stream>>>(                                           \
+#define GROUP_FORM(TD, TO, CH, PP, NN)                                                                                   \
+    group_norm_add_vec_kernel<TD, TO, CH, false, PP, NN><<<n_rows, NA_THREADS, lds, stream>>>(                            \
         (float*)residual, (const TD*)delta, (const float*)post_weight, post_eps, post_groups, (const float*)weight, eps,  \
         groups, (TO*)out, (const int*)rows, hidden, store_residual, 1, 0, 0)
+#define GROUP_VEC(TD, TO, CH)                                                                                            \
+    do {                                                                                                                 \
+      if (post_weight) { if (weight) GROUP_FORM(TD, TO, CH, true, true); else GROUP_FORM(TD, TO, CH, true, false); }       \
+      else { if (weight) GROUP_FORM(TD, TO, CH, false, true); else GROUP_FORM(TD, TO, CH, false, false); }                 \
+    } while (0)
 #define GROUP_GO(TD, TO)                                                                                                 \
   do {                                                                                                                   \
     if (vec) {                                                                                                           \
@@ -1014,6 +1020,7 @@ extern "C" int ta_group_norm_add(void* residual, const void* delta, const void* 
   else return -1;
 #undef GROUP_GO
 #undef GROUP_VEC
+#undef GROUP_FORM
   return LAUNCH_STATUS();
 }
 
@@ -1044,11 +1051,17 @@ extern "C" int ta_norm_add_parts(void* residual, const void* partial, int parts,
 #undef GO_FORM
     return LAUNCH_STATUS();
   }
-#define GO(TO, CH) group_norm_add_vec_kernel<float, TO, CH, true><<<n_rows, NA_THREADS, lds, stream>>>( \
+#define GO_FORM(TO, CH, PP, NN) group_norm_add_vec_kernel<float, TO, CH, true, PP, NN><<<n_rows, NA_THREADS, lds, stream>>>( \
     (float*)residual, (const float*)partial, (const float*)post_weight, post_eps, post_groups, (const float*)weight, eps, groups, \
     (TO*)out, (const int*)rows, hidden, store_residual, parts, slab, rounded)
+#define GO(TO, CH)                                                                                     \
+    do {                                                                                               \
+      if (post_weight) { if (weight) GO_FORM(TO, CH, true, true); else GO_FORM(TO, CH, true, false); } \
+      else { if (weight) GO_FORM(TO, CH, false, true); else GO_FORM(TO, CH, false, false); }           \
+    } while (0)
   if (out_dtype == DT_F32) { LENGTHS(float); } else { LENGTHS(bf16_t); }
 #undef LENGTHS
 #undef GO
+#undef GO_FORM
   return LAUNCH_STATUS();
 }
