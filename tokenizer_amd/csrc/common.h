@@ -25,15 +25,13 @@ __device__ __forceinline__ void st(bf16_t* p, float v) { p->bits = float_to_bf16
 
 // Stores past the caches of the chiplet that makes them (device scope): what a small kernel leaves is on its way to where the next
 // kernel's chiplets read it when the kernel ends, and the end has nothing to write back.  It pays where few workgroups' lanes store floats side by
-// side: residual products (896 columns, one row: out 2.81 -> 2.65 us, down 4.59 -> 4.44; 270 of them, 64 to 30,000 columns, 0.97 of their time), less in
-// the gated ones beside them (gate/up 6.12 -> 6.03).  A store of its own for every value of a scattered result costs more this way than the
-// write-back (four values a lane: q/k/v 4.6 -> 5.5; head products, whose 16-bit values lie apart, 1.3 us; chosen experts, 176 of them, 1.01 of
-// their time), and products of few rows in bfloat16 and in 32 bits are level or 1 to 2 % slower by it: those store plainly.  What the same
-// chiplet reads again soon stays in its cache by plain stores (streams).  Nontemporal stores do not do: of single 16-bit values they cost 10 us.
+// side: residual products (896 columns, one row: out 2.81 -> 2.65 us, down 4.59 -> 4.44; 270 of them, 64 to 30,000 columns, 0.97 of their time),
+// decode attention (328 points, 1 to 16 rows, 1.005 of the time without, single ones 1.07), and by 1 % gated products of at most two workgroups a
+// compute unit.  A store of its own for every value of a scattered result costs more this way than the write-back (four values a lane: q/k/v
+// 4.6 -> 5.5; head products, whose 16-bit values lie apart, 1.3 us; chosen experts, 176 of them, 1.01 of their time), the streams' step and
+// the routers are 2 and 1 % slower by it, and products of few rows in bfloat16 and in 32 bits are level or 1 to 2 % slower: those store
+// plainly.  Nontemporal stores do not do: of single 16-bit values they cost 10 us.
 __device__ __forceinline__ void st_through(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_through(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void st_through(bf16_t* p, float v) {

@@ -159,8 +159,8 @@ route_rows_kernel(const T* __restrict__ x, int lda, const T* __restrict__ router
       const float term = expf(z - rt_lane(z, (int)__builtin_ctzll(__ballot(place == 0))));
       const float sum = rt_sum_in_order(term, place, top);
       if (place < top) {
-        st_through(chosen + (size_t)t * top + place, lane);
-        st_through(weights + (size_t)t * top + place, term / sum);
+        chosen[(size_t)t * top + place] = lane;
+        st(weights + (size_t)t * top + place, term / sum);
       }
       return;
     }
@@ -613,7 +613,7 @@ route_rows_sigmoid_kernel(const T* __restrict__ x, int lda, const T* __restrict_
   // (With a gate, the router has one row more: the gate's, behind the experts'.)
   rt_row_sums<T, PIECES, WAVES, WAVES == 8>(x + (size_t)t * lda, router, hidden, n_experts + (gate ? 1 : 0), [&](int e, float sum) {
     if (lane != 0) return;
-    if (e == n_experts) st_through(gate + t, 1.0f / (1.0f + expf(-sum)));
+    if (e == n_experts) st(gate + t, 1.0f / (1.0f + expf(-sum)));
     else score[e] = sum;                                     // the logit, until all of them are there
   });
   __syncthreads();
@@ -632,17 +632,23 @@ route_rows_sigmoid_kernel(const T* __restrict__ x, int lda, const T* __restrict_
     }
     float pick = lane >= n_experts ? -INFINITY : correction ? s + correct : (n_groups > 0 ? s : z);
     if (__ballot(pick != pick || z != z) == 0) {             // (what is no number has no place: those rows search)
+      if (wave != 0) return;                                 // (all waves alike: the scores are the same for all)
       if (n_groups > 0) {
         const int per = n_experts / n_groups;
         int group = 0;
         for (int o = per; o < n_experts; o += per) group += lane >= o ? 1 : 0;
+        // The two largest of the lane's group, from its own members alone, eight on their way at once.
         float first = -INFINITY, second = -INFINITY;
-        for (int o = 0, at = 0, g = 0; o < n_experts; ++o) {
-          const float v = rt_lane(pick, o);
-          const bool mine = g == group;
-          second = mine ? (v > first ? first : fmaxf(second, v)) : second;
-          first = mine ? fmaxf(first, v) : first;
-          if (++at == per) { at = 0; ++g; }
+        for (int j0 = 0; j0 < per; j0 += 8) {
+          float v[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = __shfl(pick, group * per + min(j0 + j, per - 1), WAVE);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            if (j0 + j >= per) v[j] = -INFINITY;
+            second = v[j] > first ? first : fmaxf(second, v[j]);
+            first = fmaxf(first, v[j]);
+          }
         }
         const float value = (per > 1 && !group_max) ? first + second : first;
         int ahead = 0;
@@ -654,11 +660,11 @@ route_rows_sigmoid_kernel(const T* __restrict__ x, int lda, const T* __restrict_
       }
       const int place = lane < n_experts ? rt_place(pick, lane, n_experts) : n_experts;
       const float total = rt_sum_in_order(s, place, top);
-      if (wave == 0 && place < top) {
-        st_through(chosen + (size_t)t * top + place, lane);
-        st_through(weights + (size_t)t * top + place, raw ? s : s / (total + 1e-20f));
+      if (place < top) {
+        chosen[(size_t)t * top + place] = lane;
+        st(weights + (size_t)t * top + place, raw ? s : s / (total + 1e-20f));
       }
-      return;                                                // (all waves alike: the scores are the same for all)
+      return;
     }
   }
   // Every thread sums the few logits up for itself.
