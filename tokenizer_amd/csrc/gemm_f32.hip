@@ -479,7 +479,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, u
     for (int slot = 0; slot < 2; ++slot) {
       const int now = u0 + slot * PAIR * WAVES;
       if (now >= u_end) break;                               // (the same for the whole wave)
-      ask(slot ^ 1, now + PAIR * WAVES);
+      if (LINES || now + PAIR * WAVES < u_end) ask(slot ^ 1, now + PAIR * WAVES);
       if constexpr (STAGE > 0) {
 #pragma unroll
         for (int j = 0; j < STAGE; ++j) {
