@@ -467,6 +467,25 @@ def test_fused_products_whose_rows_fill_local_memory(ops, rows, k, normed):
     assert bool(((gated.double() - want).abs() <= slack).all())
 
 
+# Gated products of as many workgroups as pass their results by the chiplet's caches at most, and of more, in one block of rows and in two; silu and the
+# capped activation.
+@pytest.mark.parametrize("rows", [1, 8, 9])
+@pytest.mark.parametrize("inner", [8192, 8200, 17000])
+@pytest.mark.parametrize("capped", [False, True])
+def test_gated_products_of_many_columns(ops, rows, inner, capped):
+    x, w, k = rand_bf16((rows, 64), 33), rand_bf16((2 * inner, 64), 34), 64
+    gate, up = (x.double() @ w.double().t()).chunk(2, 1)
+    off_gate, off_up = (k * 2.0 ** -24 * x.double().abs() @ w.double().t().abs()).chunk(2, 1)      # K products added in float
+    act = torch.tensor([1.7, 7.0, 1.0], device="cuda") if capped else None
+    if capped:
+        gate, up = gate.clamp(max=7.0), up.clamp(-7.0, 7.0) + 1
+    alpha = 1.7 if capped else 1.0
+    want = gate * torch.sigmoid(alpha * gate) * up
+    # z sigmoid(alpha z) has a slope of at most 1.1; the exponential's argument is below 128 and rounded twice, the rest are units of 2^-22.
+    slack = 1.1 * off_gate * (up.abs() + off_up) + gate.abs() * off_up + (2.0 ** -8 + 2.0 ** -15) * want.abs()
+    assert bool(((ops.fused_norm_gated(x, None, 0.0, w, act).double() - want).abs() <= slack).all())
+
+
 # Workgroups of four, seven, nine and sixteen weight rows with a last one that is not full; K below a step, with a tail, of one trip and
 # of several, by steps and by lines; rows that are staged in one load and in as many as eight rows take, and that come straight from
 # memory, at the last share of K that is staged and the first that is not; rows of a longer stride with no numbers beyond K; the gate with few

@@ -115,8 +115,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   constexpr int SETS = (EPI == EPI_RESIDUAL) ? 1 : 2;
   constexpr int HELD = ONE ? PASSES : 1;                     // batches of weights held at once
   static_assert(EPI != EPI_ROPE_STORE || PASSES == 1, "the rotation pairs rows within one block");
-  constexpr int RS = WAVE + 4;                               // words between a lane's sums: the epilogue's reads touch every bank once
-  __shared__ float red[NW][SETS * 4][RS];
+  __shared__ float red[NW][SETS * 4][WAVE];                  // a register's lanes turned by four for every register before it in its set
   extern __shared__ __attribute__((aligned(16))) uint16_t a_s[];   // NORM: the m normalised rows of K + 8 bfloat16; STAGE: the waves' pieces
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int col = lane & 15, g = lane >> 4;
@@ -165,7 +164,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   // The epilogue's lanes: weight row `er` of a block, input row `em`; `e_at` is where that output stands in a wave's part of `red`.
   const int er = lane & 15, em = 4 * wave + (lane >> 4);
   const bool e_wave = 4 * wave < M;
-  const int e_at = (er & 3) * RS + (er >> 2) * 16 + em;
+  const int e_at = (er & 3) * WAVE + (((er >> 2) * 16 + em + 4 * (er & 3)) & 63);   // (turned, so that the reads touch every bank once)
 
   // Weight fragments come from HBM and take longest; the first batch is requested before the prologue.
   // Step j of a wave's batch: steps come in pairs (128 contiguous bytes of a weight row, one cache line),
@@ -458,7 +457,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
 #pragma unroll
     for (int s = 0; s < SETS; ++s)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][s * 4 + r][lane] = acc[s][r];
+      for (int r = 0; r < 4; ++r) red[wave][s * 4 + r][(lane + 4 * r) & 63] = acc[s][r];
     __syncthreads();
     const int local = 16 * ps + er;                          // the lane's row within the workgroup's
     if (e_wave && em < M && local < R) {
@@ -477,10 +476,11 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
           bf16_t* dst = p.out + (size_t)em * p.ldc + n;
           if (p.cos_sin) {
             const float gate = fminf(v0, act_limit), up = fminf(fmaxf(v1, -act_limit), act_limit);
-            st_through(dst, gate / (1.0f + __expf(-act_alpha * gate)) * (up + act_shift));
+            v0 = gate / (1.0f + __expf(-act_alpha * gate)) * (up + act_shift);
           } else {
-            st_through(dst, v0 / (1.0f + __expf(-v0)) * v1);
+            v0 = v0 / (1.0f + __expf(-v0)) * v1;
           }
+          if (heads) st_through(dst, v0); else st(dst, v0);        // (the word says which, see the launcher)
         }
       } else {
         const int d = p.d, half = d / 2;
@@ -520,7 +520,7 @@ static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
     }
   }
   size_t lds = NORM ? (size_t)args.m * (args.k + 8) * sizeof(uint16_t) : (size_t)(STAGE > 0 ? NW * args.m * (UN * 64 + 16) : 0);
-  constexpr size_t SUMS_BYTES = NW * (EPI == EPI_RESIDUAL ? 1 : 2) * 4 * (WAVE + 4) * sizeof(float);   // (the kernel's own: `red`)
+  constexpr size_t SUMS_BYTES = NW * (EPI == EPI_RESIDUAL ? 1 : 2) * 4 * WAVE * sizeof(float);   // (the kernel's own: `red`)
   if (lds + SUMS_BYTES > 64 * 1024) {
     // More LDS than a launch has unasked: ask for it (the device has 160 KB per compute unit).
     if (lds > 140 * 1024) return -1;
@@ -534,9 +534,13 @@ static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
   if (from_residual != (args.norm_weight != nullptr) || (!from_residual && !args.a) || !args.w) return -1;
   if (EPI == EPI_RESIDUAL ? !args.residual_out : !args.out) return -1;
   if (args.d > 0xffff || args.n_q > 0xffff || args.n_kv > 0xffff) return -1;   // (what the packed arguments hold)
+  // Gated results go past the chiplet's caches while two workgroups a compute unit are all there are: with more, the first ones' are written back
+  // under the others' way (8,960 over 1,536, 747 workgroups: 17.9 us past them, 17.3 plainly, eight rows 16.0 and 14.9; 4,864 over 896, 487
+  // workgroups: 6.05 and 6.19).
+  const bool through = tiles <= 2 * compute_units();
   fused_decode_kernel<NW, EPI, NORM, UN, ONE, PASSES, LINES, STAGE><<<tiles, NW * WAVE, lds, stream>>>(
       args.w, from_residual ? (const void*)args.residual_in : (const void*)args.a, args.norm_weight,
-      (uint32_t)args.m | (uint32_t)args.rows << 8 | (uint32_t)args.d << 16, (uint32_t)args.n_q | (uint32_t)args.n_kv << 16, args.n, args.k,
+      (uint32_t)args.m | (uint32_t)args.rows << 8 | (uint32_t)args.d << 16, EPI == EPI_GATED ? (uint32_t)through : (uint32_t)args.n_q | (uint32_t)args.n_kv << 16, args.n, args.k,
       args.lda, args.eps, EPI == EPI_RESIDUAL ? (void*)args.residual_out : (void*)args.out, args.bias, args.positions, args.cos_sin,
       args.slots, args.k_pages, args.v_pages, args.page_size, args.temper_coef, args.temper_every);
   return LAUNCH_STATUS();
