@@ -680,6 +680,31 @@ def test_latents_kept_in_registers(ops, q_rank, kv_rank, rot, dtype, neighbours,
         torch.testing.assert_close(v_pages.double().cpu()[:, 0].transpose(1, 2).reshape(48, width), want_k, **tol)
 
 
+# Many rows, whose two latents share a workgroup where one is short, and the same rows a few at a time, which have one each: latents of one wave and of
+# four, and longer, either of them the short one, tails of none and of more pairs than the keys' waves have threads, tokens that store nothing.
+@pytest.mark.parametrize("q_rank,kv_rank,rot", [(64, 64, 0), (192, 64, 64), (100, 600, 32), (256, 129, 2), (1030, 40, 300), (2100, 128, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_latents_of_many_rows_have_the_bits_of_few(ops, q_rank, kv_rank, rot, dtype):
+    gen = torch.Generator().manual_seed(q_rank + rot)
+    n, width, few = 2 * ops.compute_units + 7, kv_rank + rot, 61
+    rows, norms = torch.randn(n, q_rank + kv_rank + rot, generator=gen).to(dtype).cuda(), [torch.rand(r, generator=gen).cuda() for r in (q_rank, kv_rank)]
+    rates, positions = torch.rand(rot // 2, generator=gen).cuda(), torch.randint(0, 4000, (n,), generator=gen, dtype=torch.int32).cuda()
+    slots = torch.randperm(n, generator=gen).int()
+    slots[::9] = -1
+    slots, results = slots.cuda(), []
+    for step in (n, few):
+        q = torch.full((n, q_rank), 7.0, dtype=dtype, device="cuda")
+        k_pages = torch.full((-(-n // 16), 1, 16, width), 7.0, dtype=dtype, device="cuda")
+        v_pages = torch.full((-(-n // 16), 1, width, 16), 7.0, dtype=dtype, device="cuda")
+        for i in range(0, n, step):
+            at = slice(i, i + step)
+            ops.latent_store(rows[at], 0, q_rank, norms[0], q_rank, kv_rank, norms[1], rot, rates if rot else None, 1e-5, positions[at], slots[at],
+                             k_pages, v_pages, q[at])
+        results.append((q, k_pages, v_pages))
+    for many, one in zip(*results):
+        assert many.isfinite().all() and torch.equal(many, one)
+
+
 # A matrix memory stepped a token at a time against the recurrence in 64 bits.  Widths on either side of the rows a thread holds and of the columns of a workgroup;
 # an entry that goes on, one that only fills the batch up, one that starts (in a state row full of NaN), state rows in another order.
 @pytest.mark.parametrize("heads,d,dv", [(1, 16, 16), (3, 33, 40), (2, 128, 256), (3, 72, 17), (1, 200, 3), (1, 256, 16)])

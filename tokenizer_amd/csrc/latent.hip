@@ -12,24 +12,27 @@
 // 2 i + 1) turned by the angle position * rates[i] (float).  It goes into key page [n_pages, 1, page_size, kv_rank + rot] at the token's slot and,
 // transposed inside a page, into value page [n_pages, 1, kv_rank + rot, page_size].  slots null or a negative slot:
 // nothing is stored; without value pages the row goes into its key page alone.
-// A workgroup a token and part (blockIdx.y: the queries' latent, the keys'); a thread keeps its PER elements in registers from their one
-// load on (what lies behind PER * LT_THREADS of a longer latent is read again), norm weights, position and rates are asked for beside them, and
-// the angles are the last wave's, which has the fewest elements.  (One workgroup for both parts one behind the other, each read twice | so, in a
-// graph: four rows of latents of 448 and 96 3.5 | 2.4 us, of 1,792 and 192 4.9 | 2.7, 2,000 rows of those 10.5 | 10.1.)
-template <typename T, int PER, int THREADS>
-__global__ void __launch_bounds__(THREADS)
+// A workgroup a token and part (blockIdx.y: the queries' latent, the keys'), or with BOTH a workgroup a token, whose first `q_threads` threads
+// have the queries' latent and the others the keys'; a part is as many waves as it has elements for, four at most.  A thread keeps its
+// PER elements in registers from their one load on (what lies behind PER * LT_THREADS of a longer latent is read again), norm weights,
+// position and rates are asked for beside them, and the angles are the last wave's, which has the fewest elements.  (One workgroup for
+// both parts one behind the other, each read twice | so, in a graph: four rows of latents of 448 and 96 3.5 | 2.4 us, of 1,792 and 192
+// 4.9 | 2.7.)
+template <typename T, int PER, bool BOTH>
+__global__ void __launch_bounds__(2 * LT_THREADS)
 latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, int q_rank, const float* __restrict__ q_norm,
                     int kv_offset, int kv_rank, const float* __restrict__ kv_norm, int rot, const float* __restrict__ rates,
                     float eps, const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ k_pages,
-                    T* __restrict__ v_pages, int page_size, T* __restrict__ latent_q, int neighbours) {
+                    T* __restrict__ v_pages, int page_size, T* __restrict__ latent_q, int neighbours, int q_threads) {
   HELD(rows, row_stride, q_offset, q_rank, q_norm, kv_offset, kv_rank, kv_norm, rot, rates, eps, positions, slots, k_pages, v_pages,
-       page_size, latent_q, neighbours);
-  __shared__ float scratch[16];
-  const int t = blockIdx.x;
-  const bool keys = blockIdx.y != 0;
-  const int slot = keys && slots ? scalar_int(slots + t) : -1;
-  if (keys && slot < 0) return;                               // (the same for every thread of the workgroup)
-  const int rank = keys ? kv_rank : q_rank;
+       page_size, latent_q, neighbours, q_threads);
+  __shared__ float scratch[2 * LT_THREADS / WAVE];
+  const int t = blockIdx.x, wave = wave_index();
+  const bool keys = BOTH ? wave >= q_threads / WAVE : blockIdx.y != 0;
+  const int slot = keys ? scalar_int(slots + t) : -1;         // (without slots there is no such part)
+  if (!BOTH && keys && slot < 0) return;                      // (the same for every thread of the workgroup)
+  const int before = BOTH && keys ? q_threads : 0;            // the part's first thread
+  const int rank = keys ? kv_rank : q_rank, tid = threadIdx.x - before, threads = (BOTH && !keys ? q_threads : blockDim.x) - before;
   const T* row = rows + (size_t)t * row_stride;
   const T* from = row + (keys ? kv_offset : q_offset);
   const float* norm = keys ? kv_norm : q_norm;
@@ -37,15 +40,15 @@ latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, in
   float w[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int i = min(j * THREADS + (int)threadIdx.x, rank - 1);
+    const int i = min(j * LT_THREADS + tid, rank - 1);
     raw[j] = from[i];
     w[j] = norm[i];
   }
-  const int half = keys ? rot / 2 : 0, turn = (threadIdx.x + WAVE) % THREADS;    // (the thread's pair of the tail: the last wave has the first)
+  const int half = keys ? rot / 2 : 0, turn = tid + WAVE < threads ? tid + WAVE : tid + WAVE - threads;    // (the thread's pair of the tail)
   const T* tail = row + kv_offset + kv_rank;
   float rate = 0.f, position = 0.f;
   T one_raw = {}, other_raw = {};
-  if (half > 0) {                                             // (the same for all)
+  if (half > 0) {                                             // (the same for the wave)
     const int i = min(turn, half - 1);
     rate = rates[i];
     one_raw = tail[neighbours ? 2 * i : i];
@@ -56,18 +59,25 @@ latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, in
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const float v = ld(&raw[j]);
-    if (j * THREADS + (int)threadIdx.x < rank) sq += v * v;
+    if (j * LT_THREADS + tid < rank) sq += v * v;
   }
-  for (int i = PER * THREADS + threadIdx.x; i < rank; i += THREADS) { const float v = ld(from + i); sq += v * v; }
-  const float inv = 1.0f / sqrtf(block_sum(sq, scratch) / (float)rank + eps);
+  for (int i = PER * LT_THREADS + tid; i < rank; i += LT_THREADS) { const float v = ld(from + i); sq += v * v; }
+  sq = wave_sum(sq);
+  if ((threadIdx.x & (WAVE - 1)) == 0) scratch[wave] = sq;
+  __syncthreads();
+  if (BOTH && keys && slot < 0) return;                       // (the same for the wave)
+  float total = 0.f;                                          // (added wave by wave in their order)
+#pragma unroll
+  for (int j = 0; j < LT_THREADS / WAVE; ++j) total += j < threads / WAVE ? scratch[before / WAVE + j] : 0.f;
+  const float inv = 1.0f / sqrtf(total / (float)rank + eps);
   if (!keys) {
     T* dst = latent_q + (size_t)t * q_rank;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int i = j * THREADS + threadIdx.x;
+      const int i = j * LT_THREADS + tid;
       if (i < rank) st(dst + i, ld(&raw[j]) * inv * w[j]);
     }
-    for (int i = PER * THREADS + threadIdx.x; i < rank; i += THREADS) st(dst + i, ld(from + i) * inv * norm[i]);
+    for (int i = PER * LT_THREADS + tid; i < rank; i += LT_THREADS) st(dst + i, ld(from + i) * inv * norm[i]);
     return;
   }
   const int page = slot / page_size, off = slot % page_size, width = kv_rank + rot;
@@ -79,11 +89,11 @@ latent_store_kernel(const T* __restrict__ rows, int row_stride, int q_offset, in
   };
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int i = j * THREADS + threadIdx.x;
+    const int i = j * LT_THREADS + tid;
     if (i < rank) put(i, ld(&raw[j]) * inv * w[j]);
   }
-  for (int i = PER * THREADS + threadIdx.x; i < rank; i += THREADS) put(i, ld(from + i) * inv * norm[i]);
-  for (int i = turn; i < half; i += THREADS) {
+  for (int i = PER * LT_THREADS + tid; i < rank; i += LT_THREADS) put(i, ld(from + i) * inv * norm[i]);
+  for (int i = turn; i < half; i += threads) {
     if (i != turn) { rate = rates[i]; one_raw = tail[neighbours ? 2 * i : i]; other_raw = tail[neighbours ? 2 * i + 1 : half + i]; }
     float s, c;
     sincosf(position * rate, &s, &c);
@@ -291,16 +301,23 @@ extern "C" int ta_latent_store(const void* rows, int row_stride, int q_offset, i
   if (q_rank <= 0 || kv_rank <= 0 || rot < 0 || (rot & 1) || (rot > 0 && !rates) || (slots && (!k_pages || !kv_norm || page_size <= 0)))
     return -1;
   const int most = q_rank > kv_rank ? q_rank : kv_rank;
-  const dim3 grid(n_tokens, slots ? 2 : 1);
-  // (Short latents: no wave without an element of its own.  Two latents of 64, 2,000 rows, four waves a part | one: 5.5 | 3.6 us.)
-#define LS_GO(TT, PER, THREADS) latent_store_kernel<TT, PER, THREADS><<<grid, THREADS, 0, stream>>>((const TT*)rows, row_stride, \
+  auto threads_of = [](int rank) { return rank >= LT_THREADS ? LT_THREADS : (rank + WAVE - 1) / WAVE * WAVE; };
+  const int q_threads = threads_of(q_rank), k_threads = threads_of(kv_rank);
+  // Many rows whose parts are of different lengths, or short: both in a workgroup, so that none is there for waves without an element.
+  // (2,000 rows in bfloat16, latents of 192 and 64, a workgroup a part | one for both: 5.55 | 4.15 us, 64 and 192 6.3 | 5.2, 768 and 64
+  // 6.35 | 5.6, but 1,536 and 192 8.3 | 9.0; four rows 2.4 to 3.0 | 0.1 to 0.3 more.)
+  const bool both = slots && n_tokens >= 2 * compute_units() && (q_threads < LT_THREADS || k_threads <= LT_THREADS / 2);
+  const int threads = both ? q_threads + k_threads : slots && k_threads > q_threads ? k_threads : q_threads;
+  const dim3 grid(n_tokens, slots && !both ? 2 : 1);
+#define LS_GO(TT, PER, BOTH) latent_store_kernel<TT, PER, BOTH><<<grid, threads, 0, stream>>>((const TT*)rows, row_stride, \
     q_offset, q_rank, (const float*)q_norm, kv_offset, kv_rank, (const float*)kv_norm, rot, (const float*)rates, eps, (const int*)positions, \
-    (const int*)slots, (TT*)k_pages, (TT*)v_pages, page_size, (TT*)latent_q, neighbours)
-#define LS(TT) do { if (most <= 64) LS_GO(TT, 1, 64); else if (most <= 128) LS_GO(TT, 1, 128); else if (most <= LT_THREADS) LS_GO(TT, 1, LT_THREADS); \
-                    else if (most <= 2 * LT_THREADS) LS_GO(TT, 2, LT_THREADS); else if (most <= 4 * LT_THREADS) LS_GO(TT, 4, LT_THREADS); \
-                    else LS_GO(TT, 8, LT_THREADS); } while (0)
+    (const int*)slots, (TT*)k_pages, (TT*)v_pages, page_size, (TT*)latent_q, neighbours, q_threads)
+#define LS_PER(TT, PER) do { if (both) LS_GO(TT, PER, true); else LS_GO(TT, PER, false); } while (0)
+#define LS(TT) do { if (most <= LT_THREADS) LS_PER(TT, 1); else if (most <= 2 * LT_THREADS) LS_PER(TT, 2); \
+                    else if (most <= 4 * LT_THREADS) LS_PER(TT, 4); else LS_PER(TT, 8); } while (0)
   if (dtype == DT_F32) LS(float); else LS(bf16_t);
 #undef LS
+#undef LS_PER
 #undef LS_GO
   return LAUNCH_STATUS();
 }
