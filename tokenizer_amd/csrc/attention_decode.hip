@@ -77,6 +77,9 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   const int col = lane & 15, g = lane >> 4;
   const int heads_here = min(16, group - hb * 16);
   const int head = kvh * group + hb * 16 + col;          // valid when col < heads_here
+  // (The lane's head's sink, asked for here: behind the sums, where it is used, it is a trip of its own.)
+  float sink_of = 0.f;
+  if (sinks) sink_of = sinks[kvh * group + hb * 16 + min(col, heads_here - 1)];
   // entry_of_token null: every request has one token in the batch, request e is row e (one dependent load fewer).
   const int* table = block_table + (size_t)(entry_of_token ? scalar_int(entry_of_token + t) : t) * table_stride;
   // Without a window the split's first key does not hang on the position, so the pages of the wave's first block
@@ -316,7 +319,7 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
     float big = wave_max_repeated<DEC_WAVES>(mine);
     float denom = 0.f;
     if (sinks && split == 0) {
-      const float sink = sinks[hg];
+      const float sink = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sink_of), h));
       big = fmaxf(big, sink);
       denom = __expf(sink - big);
     }
