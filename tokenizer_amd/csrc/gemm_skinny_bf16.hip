@@ -303,15 +303,15 @@ skinny_gemm_kernel(const bf16_t* __restrict__ A, int lda, int k_chunk, const bf1
 template <int NW, bool GATED, typename OutT, int LINES, bool WHOLE, int SUMS, bool UPPER, int STAGE>
 __global__ void __launch_bounds__(NW * WAVE)
 few_rows_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ bias,
-                     float* __restrict__ partial, int lda, int k_chunk, uint32_t m_rows, int N, int K_all, int gate_act,
-                     OutT* __restrict__ C, int ldc) {
-  HELD(A, W, bias, partial, lda, k_chunk, m_rows, N, K_all, gate_act);   // (the fourteen words that are there)
+                     float* __restrict__ partial, int lda, int k_chunk, uint32_t m_rows_act, int N, int K_all, int ldc,
+                     OutT* __restrict__ C) {
+  HELD(A, W, bias, partial, lda, k_chunk, m_rows_act, N, K_all, ldc);    // (the fourteen words that are there)
   static_assert(SUMS == 1 || (SUMS == 2 && LINES > 0 && WHOLE), "two sums a wave: whole lines, a sum for each half");
   constexpr int SETS = GATED ? 2 : 1, TRIP = LINES > 0 ? LINES : 4;      // lines, or steps of 32, a trip
   constexpr int PIECES = TRIP * (LINES > 0 ? 8 : 4), ROW_BYTES = PIECES * 16 + 16;
   __shared__ float red[NW * SUMS][SETS * 4][WAVE];
   extern __shared__ __attribute__((aligned(16))) char rows_s[];
-  const int M = m_rows & 0xff, R = m_rows >> 8;
+  const int M = m_rows_act & 0xff, R = (m_rows_act >> 8) & 0xff, gate_act = m_rows_act >> 16;
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int col = lane & 15, g = lane >> 4;
   const int n_out = GATED ? N / 2 : N;
@@ -510,7 +510,7 @@ static int launch_few_kernel(const void* A, int lda, const void* W, const void* 
     if (err != hipSuccess) return (int)err;
   }
   kernel<<<grid, NW * WAVE, lds, stream>>>((const bf16_t*)A, (const bf16_t*)W, (const float*)bias, slabs, lda, k_chunk,
-                                           (uint32_t)M | (uint32_t)rows << 8, N, K, gate_act, (OutT*)C, ldc);
+                                           (uint32_t)M | (uint32_t)rows << 8 | (uint32_t)gate_act << 16, N, K, ldc, (OutT*)C);
   return LAUNCH_STATUS();
 }
 
