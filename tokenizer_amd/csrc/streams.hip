@@ -199,15 +199,10 @@ streams_step_column_kernel(float* __restrict__ streams, const TY* __restrict__ y
   if (scale) scale_c = scale[c];
   int slot = -1;
   bool first = false;
-  if constexpr (SHIFT) {
-    mu_c = mu[c];
-    const int e = scalar_int(entry_of_token + r);
-    slot = e >= 0 ? scalar_int(state_slots + max(e, 0)) : -1;
-    first = scalar_int(positions + r) == 0;
-    before = state[(size_t)max(slot, 0) * width + c];        // (a row that only fills the batch up has slot 0's, which it does not use)
-  }
+  // (What hangs on nothing comes before the chain from the token's entry to its state row.)
 #pragma unroll
   for (int s = 0; s < S; ++s) take[s] = scalar_float(read + s);
+  const float g = scalar_float(gain);
   if (y) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -216,7 +211,13 @@ streams_step_column_kernel(float* __restrict__ streams, const TY* __restrict__ y
       for (int to = 0; to < S; ++to) m[s][to] = scalar_float(mix + s * S + to);
     }
   }
-  const float g = scalar_float(gain);
+  if constexpr (SHIFT) {
+    mu_c = mu[c];
+    const int e = scalar_int(entry_of_token + r);
+    first = scalar_int(positions + r) == 0;
+    slot = e >= 0 ? scalar_int(state_slots + max(e, 0)) : -1;
+    before = state[(size_t)max(slot, 0) * width + c];        // (a row that only fills the batch up has slot 0's, which it does not use)
+  }
   float u = 0.f;
   if (!y) {
 #pragma unroll
@@ -247,7 +248,7 @@ streams_step_column_kernel(float* __restrict__ streams, const TY* __restrict__ y
     if (in) state[(size_t)slot * width + c] = h;
     h = fmaf((first ? 0.f : before) - h, mu_c, h);
   }
-  if (in) st_through(out + (size_t)i * width + c, h);
+  if (in) st(out + (size_t)i * width + c, h);
 }
 
 // Token shift over a batch of portions: out[t] = h[t] + (before - h[t]) * mu, `before` = h[t - 1] inside a portion, the
