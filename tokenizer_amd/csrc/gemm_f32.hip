@@ -375,7 +375,9 @@ extern "C" int ta_gemm_f32_tile_row(int kind, int block, int n, int tile_rows, i
          : kind == ROWS_GATED ? RowTile<ROWS_GATED>(block, n, tile_rows, d).row(i) : RowTile<ROWS_PLAIN>(block, n, tile_rows, d).row(i);
 }
 
-template <int KIND, bool LINES, int STAGE>
+// FULL: the tile has all of its rows (always with GATED), so that no load of weights stands behind a question of its lane's (151,936 columns over 896,
+// sixteen rows 129 -> 126 us).
+template <int KIND, bool LINES, int STAGE, bool FULL>
 __global__ void __launch_bounds__(512)
 gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, uint32_t m_rows_d, int N, int K, int lda, int units_part,
                      const float* __restrict__ bias, float* __restrict__ partial, float* __restrict__ C, int ldc,
@@ -414,7 +416,7 @@ gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W, u
         if (u < u_end) {                                     // (the same for the whole wave)
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            if (w_ok[h]) w[slot][p][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w_row[h] + u * 32 + 4 * piece));
+            if (FULL || w_ok[h]) w[slot][p][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w_row[h] + u * 32 + 4 * piece));
           if constexpr (STAGE == 0) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) a[slot][p][h] = *reinterpret_cast<const f32x4*>(a_row + u * 32 + 8 * g + 4 * h);
@@ -567,13 +569,16 @@ template <int KIND>
 static void launch_f32_rows(dim3 grid, const float* a, const float* w, const float* bias, float* c, int M, int N, int K, int lda, int ldc,
                             int units_part, float* partial, int rows, int d, const F32Store& store, hipStream_t stream) {
   const uint32_t packed = (uint32_t)M | (uint32_t)rows << 8 | (uint32_t)d << 16;
-#define GO(LINES, STAGE) gemm_f32_rows_kernel<KIND, LINES, STAGE><<<grid, 512, 0, stream>>>(a, w, packed, N, K, lda, units_part, bias, partial, c, \
-                                                                                            ldc, store)
-  if (K % 32) GO(false, 0);
+#define GO_FORM(LINES, STAGE, FULL) gemm_f32_rows_kernel<KIND, LINES, STAGE, FULL><<<grid, 512, 0, stream>>>(a, w, packed, N, K, lda, units_part, \
+                                                                                                           bias, partial, c, ldc, store)
+#define GO(LINES, STAGE) do { if (KIND == ROWS_GATED || rows == (KIND == ROWS_PLAIN ? 16 : 8)) GO_FORM(LINES, STAGE, true); \
+                              else GO_FORM(LINES, STAGE, KIND == ROWS_GATED); } while (0)
+  if (K % 32) GO_FORM(false, 0, false);
   else if (M <= 4) GO(true, 1);
   else if (M <= 8) GO(true, 2);
   else GO(true, 0);
 #undef GO
+#undef GO_FORM
 }
 
 // One or two rows, four of large matrices, and up to sixteen whose pieces of sixteen bytes do not lie on sixteen bytes (VEC false):
