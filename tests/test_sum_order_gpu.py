@@ -86,7 +86,7 @@ def test_sum_over_a_wave_starts_with_lanes_32_apart(ops, rows):
     assert (out == 0.5).all()
 
 
-@pytest.mark.parametrize("hidden, inner, shared", [(512, 1040, 0), (1000, 1040, 64), (2056, 520, 0)])
+@pytest.mark.parametrize("hidden, inner, shared", [(512, 1040, 0), (1000, 1040, 64), (2056, 520, 0), (520, 512, 0), (512, 520, 40)])
 def test_experts_of_one_row_and_of_many_have_the_same_bits(ops, hidden, inner, shared):
     # Few workgroups ask for four turns of K at once, many for one: shares of K that end inside a trip, K that is no whole line.
     experts, top = 8, 2

@@ -209,14 +209,14 @@ experts_few_up_kernel(const bf16_t* __restrict__ x, int x_stride, const int* __r
 
 // out [top, n_rows, hidden] float: out[p % top, p / top] = act[p] times expert chosen[p]'s second matrix, which is columns
 // e * inner .. of W [hidden, ldw].  Grid: (blocks of sixteen output columns, experts).
-template <int NW>
+template <int NW, bool STAGED>
 __global__ void __launch_bounds__(NW * WAVE)
 experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ chosen, int n_pairs, int top, int n_rows,
                         const bf16_t* __restrict__ W, int ldw, int inner, int hidden, float* __restrict__ out, EfShared every) {
   HELD(act, chosen, n_pairs, top, n_rows, W, ldw, inner, hidden, out, every.parts, every.length, every.inner, every.act);
   __shared__ int list[EF_MAX_PAIRS];
   __shared__ float red[NW][4][WAVE];
-  __shared__ __attribute__((aligned(16))) char stage_s[NW * EF_STAGE_BYTES(4)];
+  __shared__ __attribute__((aligned(16))) char stage_s[STAGED ? NW * EF_STAGE_BYTES(4) : 16];
   const int part = blockIdx.y;                               // below every.parts: a part of the shared expert's K
   const bool shared = part < every.parts;
   const int expert = part - every.parts, n0 = blockIdx.x * 16;
@@ -243,7 +243,7 @@ experts_few_down_kernel(const bf16_t* __restrict__ act, const int* __restrict__ 
   for (int p0 = 0; p0 < count; p0 += 16) {
     const int here = min(count - p0, 16);
     ef_floatx4 acc[1] = {(ef_floatx4){0.f, 0.f, 0.f, 0.f}};
-    ef_walk<NW, 1, 4, true>(w_at, [&](int i) { return act + (size_t)list[p0 + i] * stride; }, here, inner, wave, stage_s + wave * EF_STAGE_BYTES(4), acc);
+    ef_walk<NW, 1, 4, STAGED>(w_at, [&](int i) { return act + (size_t)list[p0 + i] * stride; }, here, inner, wave, stage_s + wave * EF_STAGE_BYTES(4), acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave][r][lane] = acc[0][r];
     __syncthreads();
@@ -297,23 +297,28 @@ extern "C" int ta_experts_few(const void* x, int x_stride, const void* chosen, c
       down((hidden + 15) / 16, n_experts + every.parts);
 #define UP(NW, HH, UN, ST) experts_few_up_kernel<NW, HH, UN, ST><<<up, NW * WAVE, 0, stream>>>((const bf16_t*)x, x_stride, (const int*)chosen, \
     (const float*)weights, (int)pairs, top, (const bf16_t*)w_first, inner, hidden, (bf16_t*)act, weigh_input, every)
-#define DOWN(NW) experts_few_down_kernel<NW><<<down, NW * WAVE, 0, stream>>>((const bf16_t*)act, (const int*)chosen, (int)pairs, top, \
+#define DOWN(NW, ST) experts_few_down_kernel<NW, ST><<<down, NW * WAVE, 0, stream>>>((const bf16_t*)act, (const int*)chosen, (int)pairs, top, \
     n_rows, (const bf16_t*)w_second, ldw, inner, hidden, (float*)out, every)
   // Turns asked for at once.  One of two matrices, four loads of weights a lane (two take registers that more waves a compute unit make
   // better use of: 5,504 over 2,048, four rows 52.5 | 55.0 us for both products), but four where the workgroups cannot be more than the
   // compute units, however the rows choose, and none has another to hide its trips (one | four: 1,792 over 4,096, one row 33.6 | 24.8; 1,024
   // over 1,024 10.9 | 9.4, two rows 11.4 | 9.8; 512 over 1,024, four rows 11.5 | 10.0).  Four of one matrix, eight loads.
   const long busy = (pairs < n_experts ? pairs : n_experts) * ((inner + 15) / 16) + (shared + 15) / 16;
-  if (halves == 1) { if (hidden <= 1024) UP(4, 1, 4, true); else UP(8, 1, 4, true); }
-  else if (busy <= compute_units()) { if (hidden <= 1024) UP(4, 2, 4, true); else UP(8, 2, 4, true); }
-  // (The staged forms' registers leave a SIMD five waves in place of seven: they pay while an expert has few pairs.  Both products, two of 8
+  // Rows are staged where a wave has more than two turns of K: with fewer most of a trip's pieces are none (512 over 512, two of 8 experts, one row
+  // 6.8 | 7.05 us both products, sixteen 8.3 | 8.5).
+#define FOUR(HH) do { if (hidden <= 512) UP(4, HH, 4, false); else if (hidden <= 1024) UP(4, HH, 4, true); else UP(8, HH, 4, true); } while (0)
+  if (halves == 1) FOUR(1);
+  else if (busy <= compute_units()) FOUR(2);
+  // (The staged forms' registers leave a SIMD five waves in place of seven: they pay while an expert has few pairs and long rows.  Both products, two of 8
   // experts, direct | staged: 1,536 and 2,240 beside 4,480, three rows 35.3 | 34.5, eight 41.7 | 41.9, sixteen 46.2 | 46.7; 3,584 and 9,472, four
-  // rows 188.4 | 185.0.)
-  else if (pairs <= 8) { if (hidden <= 1024) UP(4, 2, 1, true); else UP(8, 2, 1, true); }
-  else { if (hidden <= 1024) UP(4, 2, 1, false); else UP(8, 2, 1, false); }
+  // rows 188.4 | 185.0; but 1,024 and 3,584, two rows 20.2 | 21.0.)
+  else if (hidden <= 1024) UP(4, 2, 1, false);
+  else if (pairs <= 8) UP(8, 2, 1, true);
+  else UP(8, 2, 1, false);
   int status = LAUNCH_STATUS();
   if (status != 0) return status;
-  if (inner <= 1024) DOWN(4); else DOWN(8);
+  if (inner <= 512) DOWN(4, false); else if (inner <= 1024) DOWN(4, true); else DOWN(8, true);
+#undef FOUR
 #undef UP
 #undef DOWN
   return LAUNCH_STATUS();
