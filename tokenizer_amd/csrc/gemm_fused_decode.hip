@@ -49,6 +49,9 @@ __device__ __forceinline__ bf16x8 any8() {
   return v;
 }
 
+// Words between a wave's sums of one register and of the next.
+__host__ __device__ constexpr int fused_sum_words(int epi, bool one) { return epi == EPI_RESIDUAL || one ? WAVE + 4 : WAVE; }
+
 // A workgroup owns `p.rows` weight rows (output columns), in PASSES blocks of up to sixteen: the M side of the
 // MFMA.  Lanes whose weight row or input row only feeds results that are never stored load nothing: a
 // load costs the memory pipeline by its active lanes.  So a small matrix is spread thinly over many
@@ -67,7 +70,8 @@ __device__ __forceinline__ bf16x8 any8() {
 // The kernel takes its arguments one by one, those that every instance needs before its first load in the first
 // sixteen words of the argument block: the library is compiled so that these are in scalar registers when a wave
 // starts (`-amdgpu-kernarg-preload-count`; fourteen words in fact), and no instance begins with a fetch of arguments:
-// m, the rows a workgroup and the head size share a word (16 bits for the head size, which the launcher checks), the two numbers of heads another.
+// m, the rows a workgroup and the head size share a word (16 bits for the head size, which the launcher checks), the two numbers of heads another (with the
+// gated epilogue: whether its results go past the chiplet's caches).
 // One pointer serves for the rows (bfloat16, or the float residual for the norm prologue) and one for the result (bfloat16 rows, or
 // the float residual that is added to), which never occur together.  The rest lies behind; only the waves of the epilogue wait for it,
 // with their weights under way.  Positions and slots come through the scalar unit there, so that the angles, which hang on the
@@ -115,7 +119,11 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   constexpr int SETS = (EPI == EPI_RESIDUAL) ? 1 : 2;
   constexpr int HELD = ONE ? PASSES : 1;                     // batches of weights held at once
   static_assert(EPI != EPI_ROPE_STORE || PASSES == 1, "the rotation pairs rows within one block");
-  __shared__ float red[NW][SETS * 4][WAVE];                  // a register's lanes turned by four for every register before it in its set
+  // (The epilogue's reads touch every bank once: four words stand between a wave's registers.  Where long rows lie in LDS beside two sets, that
+  // kilobyte can be a workgroup less on a compute unit, nine rows of 3,584 60.4 -> 69.7 us, and a register's lanes are turned by four for every
+  // register before it instead, which costs short launches 0.02 to 0.1 us.)
+  constexpr int RS = fused_sum_words(EPI, ONE), TURN = RS == WAVE ? 4 : 0;
+  __shared__ float red[NW][SETS * 4][RS];
   extern __shared__ __attribute__((aligned(16))) uint16_t a_s[];   // NORM: the m normalised rows of K + 8 bfloat16; STAGE: the waves' pieces
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int col = lane & 15, g = lane >> 4;
@@ -164,7 +172,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   // The epilogue's lanes: weight row `er` of a block, input row `em`; `e_at` is where that output stands in a wave's part of `red`.
   const int er = lane & 15, em = 4 * wave + (lane >> 4);
   const bool e_wave = 4 * wave < M;
-  const int e_at = (er & 3) * WAVE + (((er >> 2) * 16 + em + 4 * (er & 3)) & 63);   // (turned, so that the reads touch every bank once)
+  const int e_at = (er & 3) * RS + (((er >> 2) * 16 + em + TURN * (er & 3)) & 63);
 
   // Weight fragments come from HBM and take longest; the first batch is requested before the prologue.
   // Step j of a wave's batch: steps come in pairs (128 contiguous bytes of a weight row, one cache line),
@@ -457,7 +465,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
 #pragma unroll
     for (int s = 0; s < SETS; ++s)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][s * 4 + r][(lane + 4 * r) & 63] = acc[s][r];
+      for (int r = 0; r < 4; ++r) red[wave][s * 4 + r][(lane + TURN * r) & 63] = acc[s][r];
     __syncthreads();
     const int local = 16 * ps + er;                          // the lane's row within the workgroup's
     if (e_wave && em < M && local < R) {
@@ -520,7 +528,7 @@ static int launch_kernel(const FusedArgs& args, int tiles, hipStream_t stream) {
     }
   }
   size_t lds = NORM ? (size_t)args.m * (args.k + 8) * sizeof(uint16_t) : (size_t)(STAGE > 0 ? NW * args.m * (UN * 64 + 16) : 0);
-  constexpr size_t SUMS_BYTES = NW * (EPI == EPI_RESIDUAL ? 1 : 2) * 4 * WAVE * sizeof(float);   // (the kernel's own: `red`)
+  constexpr size_t SUMS_BYTES = NW * (EPI == EPI_RESIDUAL ? 1 : 2) * 4 * fused_sum_words(EPI, ONE) * sizeof(float);   // (the kernel's own: `red`)
   if (lds + SUMS_BYTES > 64 * 1024) {
     // More LDS than a launch has unasked: ask for it (the device has 160 KB per compute unit).
     if (lds > 140 * 1024) return -1;
