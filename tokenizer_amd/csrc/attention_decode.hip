@@ -77,9 +77,6 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   const int col = lane & 15, g = lane >> 4;
   const int heads_here = min(16, group - hb * 16);
   const int head = kvh * group + hb * 16 + col;          // valid when col < heads_here
-  // (The lane's head's sink, asked for here: behind the sums, where it is used, it is a trip of its own.)
-  float sink_of = 0.f;
-  if (sinks) sink_of = sinks[kvh * group + hb * 16 + min(col, heads_here - 1)];
   // entry_of_token null: every request has one token in the batch, request e is row e (one dependent load fewer).
   const int* table = block_table + (size_t)(entry_of_token ? scalar_int(entry_of_token + t) : t) * table_stride;
   // Without a window the split's first key does not hang on the position, so the pages of the wave's first block
@@ -300,6 +297,10 @@ decode_attention_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   }
   // Sum of the lane groups' partial denominators (the maximum is already common to them).
   l = wave_add_across<32>(wave_add_across<16>(l));
+  // (The lane's head's sink, on its way while the waves meet: asked for behind them it is a trip of its own, and at the start, before the keys, it cost
+  // kernels without sinks 0.1 us.)
+  float sink_of = 0.f;
+  if (sinks) sink_of = sinks[kvh * group + hb * 16 + min(col, heads_here - 1)];
   if (TIED) __syncthreads();                                // (no wave reads its keys any more)
 #pragma unroll
   for (int db = 0; db < DB; ++db)
