@@ -850,7 +850,8 @@ __device__ __forceinline__ void na_group_rms(const float* part, float* inv, int 
 // and a rounded copy of the product written and read again: eight layers of 1,536 with an inner width of 8,960, 8 requests from
 // prompts of 90 to 500 tokens through eight decoded ones, 7.73 ms with that kernel, 7.59 without.
 // POST, NEXT: whether there is a weight behind the sub-layer and one in front of the next, so that every load stands at the start, chunk by
-// chunk, and none is made that the form has no use for; the groups an element is in are worked out while the rows are on their way.
+// chunk, and none is made that the form has no use for; the groups an element is in are worked out while the rows are on their way.  (600 rows of
+// 3,584 in 32 bits without a weight 5.5 us, 6.8 with loads that are not used; 6.1 with one form whose loads stand in blocks of their own.)
 template <typename TD, typename TO, int CHUNKS, bool PARTS, bool POST, bool NEXT>
 __global__ void __launch_bounds__(NA_THREADS)
 group_norm_add_vec_kernel(float* __restrict__ residual, const TD* __restrict__ delta, const float* __restrict__ post_weight,
