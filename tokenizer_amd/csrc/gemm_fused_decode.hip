@@ -99,8 +99,13 @@ __host__ __device__ constexpr int fused_sum_words(int epi, bool one) { return ep
 // like any other: a workgroup's weights and rows, down 4,864 to 896, were 80 loads of the one and 160 of the other.  Us, direct |
 // staged, one row and eight: down 4,864 to 896 5.4 | 4.55 and 6.7 | 5.4, out 896 to 896 2.8 | 2.75 and 3.2 | 2.9 (weights alone 3.3 and 2.0).
 // With more than eight rows a staged share is as many loads as the fragments are.
+//
+// An instance's code begins on a page of its own, so that none of up to 4 KB lies across a page's end and where it lies in the cache of instructions
+// does not hang on the instances in front of it: out of 896 over 896, eight rows, had come to lie across one when others were taken out, and took 3.0 us
+// for the 2.77 that the same instructions take elsewhere (eight chat turns 13.75 ms, so 13.66; on 8 KB, where all instances' starts share
+// their places in that cache, 13.79).
 template <int NW, int EPI, bool NORM, int UN, bool ONE, int PASSES, bool LINES, int STAGE>
-__global__ void __launch_bounds__(NW * WAVE)
+__global__ void __launch_bounds__(NW * WAVE) __attribute__((aligned(4096)))
 fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weight, uint32_t m_rows_d, uint32_t heads,
                     int n, int k, int lda, float eps, void* result, const float* bias,
                     const int* positions, const float* cos_sin, const int* slots, bf16_t* k_pages, bf16_t* v_pages,
@@ -172,7 +177,7 @@ fused_decode_kernel(const bf16_t* w, const void* rows_in, const float* norm_weig
   // The epilogue's lanes: weight row `er` of a block, input row `em`; `e_at` is where that output stands in a wave's part of `red`.
   const int er = lane & 15, em = 4 * wave + (lane >> 4);
   const bool e_wave = 4 * wave < M;
-  const int e_at = (er & 3) * RS + (((er >> 2) * 16 + em + TURN * (er & 3)) & 63);
+  const int e_lane = (er >> 2) * 16 + em, e_at = (er & 3) * RS + (TURN ? (e_lane + TURN * (er & 3)) & 63 : e_lane);
 
   // Weight fragments come from HBM and take longest; the first batch is requested before the prologue.
   // Step j of a wave's batch: steps come in pairs (128 contiguous bytes of a weight row, one cache line),
