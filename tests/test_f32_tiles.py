@@ -50,3 +50,9 @@ def test_rows_of_a_plain_matrix(row_of, n, rows):
             assert 0 <= got < n and (i >= rows or got == min(block * rows + i, n - 1))
             seen.add(got)
     assert seen == set(range(n))
+
+
+@pytest.mark.parametrize("kind, block, n, rows, d, i", [(ROPE, 0, 576, 0, 96, 0), (ROPE, 0, 576, 8, 0, 0), (PLAIN, 0, 0, 16, 0, 0),
+                                                        (GATED, -1, 8, 8, 0, 0), (PLAIN, 0, 8, 16, 0, 16)])
+def test_what_is_no_tile(row_of, kind, block, n, rows, d, i):
+    assert row_of(kind, block, n, rows, d, i) == -1

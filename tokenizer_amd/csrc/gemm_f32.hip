@@ -369,8 +369,9 @@ struct RowTile {
   }
 };
 
-// The row of the matrix that row i of a workgroup's tile is read from (`kind`: the enumeration above), as the kernel below has it.
+// The row of the matrix that row i of a workgroup's tile is read from (`kind`: the enumeration above), as the kernel below has it; -1 for what is no tile.
 extern "C" int ta_gemm_f32_tile_row(int kind, int block, int n, int tile_rows, int d, int i) {
+  if (n <= 0 || tile_rows <= 0 || tile_rows > 16 || i < 0 || i > 15 || block < 0 || (kind == ROWS_ROPE && d / 2 < tile_rows)) return -1;
   return kind == ROWS_ROPE ? RowTile<ROWS_ROPE>(block, n, tile_rows, d).row(i)
          : kind == ROWS_GATED ? RowTile<ROWS_GATED>(block, n, tile_rows, d).row(i) : RowTile<ROWS_PLAIN>(block, n, tile_rows, d).row(i);
 }
